@@ -89,8 +89,8 @@ const char *spy_hip_error_string(int code);
  * to fp16; additionally (Q4_K|Q6_K, F32) -> Q8_0 activations, which the reference lacks.
  * `scratch` holds the converted activations (the reference allocates it in get_control_header,
  * mat.cpp:61-68); query its size with spy_hip_op_matmul_scratch_size.  While the host's summation
- * order is on (spy_hip_set_exact_order) that size also covers fp16 copies of both operands, from which
- * the prompt-sized Q4_0 / Q8_0 MatMul of that order runs fastest; a buffer that holds only the
+ * order is on (spy_hip_set_exact_order) that size also covers the fp16 operands from which the MatMul
+ * of several rows runs fastest in that order; a buffer that holds only the
  * activations (rows * row size of the converted type) is accepted too and gives the same results.
  * One contiguous f32 row against a plain quantized matrix (the weight products of a single-token pass) is
  * quantized inside the launch that multiplies it and leaves `scratch` untouched, in either summation order. */

@@ -19,6 +19,11 @@ int spy_exact_matvec(hipStream_t st, int t0, const void *w, const float *x, floa
 int spy_exact_dots(hipStream_t st, int t0, const spy_hip_tensor *w, const uint8_t *xm, int64_t x_row, int64_t ne11, const spy_hip_tensor *dst, int x_own_quants,
                    void *pack, size_t pack_bytes);
 size_t spy_exact_pack_bytes(int64_t ne01, int64_t ne00, int64_t ne11);
+// exact_gemm.hip: several activation rows in the host's order from activations packed once
+size_t spy_xgemm_pack_bytes(int64_t T, int64_t K);
+bool spy_xgemm_ok(int wtype, const void *w, const float *dst, int64_t M, int64_t K, int64_t T, int64_t d_row);
+int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, int64_t K, void *pack);
+int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
 
 struct tdesc {              // a tensor as the kernels see it
     uint8_t *p;
@@ -658,7 +663,9 @@ extern "C" size_t spy_hip_op_matmul_scratch_size(const spy_hip_tensor *w, const 
     const size_t act = matmul_act_bytes(w, x);
     if (!act || !spy_exact_on() || x->type != SPY_HIP_F32 || (w->type != SPY_HIP_Q4_0 && w->type != SPY_HIP_Q8_0) || w->ne[2] != 1 || w->ne[3] != 1) return act;
     const size_t pk = spy_exact_pack_bytes(w->ne[1], w->ne[0], x->ne[1]);
-    return pk ? ((act + 255) & ~(size_t)255) + pk : act;
+    const size_t xp = x->ne[1] >= 2 ? spy_xgemm_pack_bytes(x->ne[1], x->ne[0]) : 0;
+    const size_t need = pk ? ((act + 255) & ~(size_t)255) + pk : act;
+    return need > xp ? need : xp;
 }
 
 int spy_own_matvec_q4_0(hipStream_t st, const void *w, const float *x, float *out, int M, int K);      // engine_q*.hip: the one-row-per-wave kernel without a residual
@@ -714,7 +721,21 @@ static int matmul_impl(void *stream, const spy_hip_tensor *w, const spy_hip_tens
                                       : own_matvec(st, t0, w->data, (const float *)x->data, (float *)dst->data, ne01, ne00);
         if (rc != SPY_HIP_EUNSUPPORTED) return rc;
     }
-    // the host's order with 2 .. 15 rows (a short prompt): the same launch once per row -- the lane kernels below take 44 us per row
+    // the host's order, several rows: the kernels of exact_gemm.hip where they take the matrix and the scratch buffer holds the packed
+    // activations (SPY_HIP_EXACT_TILED=u / 0, SPY_HIP_EXACT_SERIAL: tests of the other kernels)
+    if (quant && t1 == SPY_HIP_F32 && ne11 >= 2 && ne12 == 1 && ne13 == 1 && skip_past < 0 && klimit_past < 0 && spy_exact_on() && x->nb[0] == 4 && x->nb[1] % 16 == 0 &&
+        ((uintptr_t)x->data & 15) == 0 && dst->nb[1] % 16 == 0 && w->nb[0] == spy_type_size(t0) && w->nb[1] == spy_row_size(t0, ne00) &&
+        spy_xgemm_ok(t0, w->data, (const float *)dst->data, ne01, ne00, ne11, dst->nb[1] / 4)) {
+        const char *tiled = getenv("SPY_HIP_EXACT_TILED");
+        const size_t need = spy_xgemm_pack_bytes(ne11, ne00);
+        if (scratch && ((uintptr_t)scratch & 15) == 0 && scratch_bytes >= need && !(tiled && (*tiled == '0' || *tiled == 'u')) && !getenv("SPY_HIP_EXACT_SERIAL")) {
+            const void *wp = w->data;
+            float *dp = (float *)dst->data;
+            const int rc = spy_xgemm_pack(st, (const float *)x->data, x->nb[1], ne11, ne00, scratch);
+            return rc ? rc : spy_xgemm(st, t0, 1, &wp, &dp, ne01, ne00, ne11, dst->nb[1] / 4, nullptr, scratch);
+        }
+    }
+    // ... without that room 2 .. 15 rows (a short prompt) run the single-row launch once per row -- the lane kernels below take 44 us per row
     // of a 4096 x 4096 matrix, this one 5; from 16 rows on the tiled kernel
     if (quant && t1 == SPY_HIP_F32 && ne11 >= 2 && ne11 <= 15 && ne12 == 1 && ne13 == 1 && skip_past < 0 && klimit_past < 0 && spy_exact_on() &&
         x->nb[0] == 4 && x->nb[1] % 16 == 0 && dst->nb[1] % 4 == 0 && w->nb[0] == spy_type_size(t0) && w->nb[1] == spy_row_size(t0, ne00)) {

@@ -91,6 +91,27 @@ def test_single_row_matmul_takes_the_two_phase_kernel(hip, oracle, wtype, M, K, 
             assert (scratch.download(np.uint8) == 0xEE).all(), "the single-row route does not use the scratch buffer"
 
 
+@pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0])
+@pytest.mark.parametrize("M,K,T", [(4, 256, 2), (20, 512, 3), (4096, 256, 15), (100, 1024, 16), (36, 4096, 17), (12288, 256, 33), (4100, 512, 48), (8192, 256, 100), (4096, 768, 257)])
+def test_packed_activation_matmul_bits(hip, oracle, wtype, M, K, T):
+    """Two rows and more against whole super-block rows: the kernels that unpack a weight once per wave (exact_gemm.hip), in every tile
+    the dispatch has, with partial tiles on both sides, the shortest contraction and scales down to fp16 subnormals."""
+    from tests.gpu_util import dev, dev_empty, call
+    rng = np.random.default_rng(11 * wtype + M + K + T)
+    w = O.quantize(oracle, (rng.standard_normal((M, K)) * 0.02).astype(np.float32), wtype)
+    x = (rng.standard_normal((T, K // 32, 32)) * 2.0 ** rng.integers(-18, 6, (T, K // 32, 1))).reshape(T, K).astype(np.float32)
+    x[0, 32:64] = 0.0
+    want = O.matmul(oracle, w, wtype, M, K, x, nthread=8)
+    tw, tx = hip.tensor(dev(w), wtype, [K, M]), hip.tensor(dev(x), hip.F32, [K, T])
+    L = hip.load()
+    need = L.spy_hip_op_matmul_scratch_size(B(tw), B(tx))
+    scratch, dd = dev_empty(need, 0xEE), dev_empty(T * M * 4 + 64, 0xFF)
+    call(L.spy_hip_op_matmul, None, B(tw), B(tx), B(hip.tensor(dd, hip.F32, [M, T])), scratch.ptr, need)
+    got = dd.download(np.float32)
+    _same_bits(got[:T * M].reshape(T, M), want, "packed-activation matmul type %d %dx%d T %d" % (wtype, M, K, T))
+    assert (got[T * M:].view(np.uint32) == 0xFFFFFFFF).all(), "nothing is written beyond the outputs"
+
+
 @pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0, O.Q4_K, O.Q6_K])
 @pytest.mark.parametrize("M,K,T", [(96, 4096, 16), (200, 512, 70), (64, 128, 64), (64, 256, 64), (132, 11008, 33), (4096, 4096, 130)])
 def test_tiled_matmul_bits(hip, oracle, wtype, M, K, T, monkeypatch):

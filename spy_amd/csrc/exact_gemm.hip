@@ -20,6 +20,7 @@
 #include "common.cuh"
 
 #include <type_traits>
+#include <utility>
 
 namespace {
 
@@ -29,9 +30,9 @@ typedef float xt_v16f __attribute__((ext_vector_type(16)));
 
 // Layout of packed activations, per group of 16 rows and stage of four Q8_0 blocks: XT_XB bytes of quants
 //   [block][word pair g][row][word of the pair][4 x fp16: elements 0, 2, 1, 3 of the word]
-// and one record of scales [block][row], XT_XD bytes: fp16 in the lower half of a dword
+// and one record of XT_XD bytes: scales [block][row], fp16 in the lower half of a dword, then the sums of the quants [block][row], fp32
 #define XT_XB 4096
-#define XT_XD 256
+#define XT_XD 512
 
 // 16 (4) bytes per lane from base + off to LDS bytes lds .. in lane order; base and lds are uniform over the wave.  Written as
 // instructions so that the compiler does not wait for them at the next LDS read; xt_wait_vm says when they have to be there.
@@ -75,7 +76,7 @@ template <int WT, int AS, int RG, int C, int NXS, int P, int NWC, int OCC>
 __global__ __launch_bounds__(64 * AS * RG, OCC) void xt_kernel(xt_args a) {
     constexpr int NT = 64 * AS * RG, ROWS = 16 * RG;
     constexpr int CU = xt_w<WT>::CU, UW = ROWS * CU, NI = (UW + NT - 1) / NT, NXI = C * 256 / NT;
-    constexpr int XB = C * (XT_XB + XT_XD), WB = (UW + 63) / 64 * 1024;
+    constexpr int XB = C * (XT_XB + 256), WB = (UW + 63) / 64 * 1024;
     static_assert(NXI * NT == C * 256 && AS * RG >= C && NXS > P && NWC * 2 > P, "one request per thread and group, one wave per group's scales, slots for what is on its way");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -100,7 +101,7 @@ __global__ __launch_bounds__(64 * AS * RG, OCC) void xt_kernel(xt_args a) {
     const bool spare = wave * 64 + (NI - 1) * NT >= UW;
     const uint32_t lds_spare = __builtin_amdgcn_readfirstlane(lds0 + NXS * XB + NWC * WB);
     const uint32_t l16 = lane * 16, l4 = lane * 4;
-    const uint32_t ldsx = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024), ldsd = __builtin_amdgcn_readfirstlane(lds0 + C * XT_XB + min(wave, C - 1) * XT_XD),
+    const uint32_t ldsx = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024), ldsd = __builtin_amdgcn_readfirstlane(lds0 + C * XT_XB + min(wave, C - 1) * 256),
                    ldsw = __builtin_amdgcn_readfirstlane(lds0 + NXS * XB + wave * 1024);
     int is = 0;                                    // next stage to request; past the last one it is requested again (same count of requests, slot unused)
     auto issue_x = [&]() {
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(64 * AS * RG, OCC) void xt_kernel(xt_args a) {
         uint32_t dx = *(const uint32_t *)sd, dxn = 0;
         xv[0] = rd(0);
         xv[1] = rd(1);
-        if (C > 1) dxn = *(const uint32_t *)(sd + XT_XD);
+        if (C > 1) dxn = *(const uint32_t *)(sd + 256);
         D[0] = xt_mfma(dw, 0u, dx, 0u);
         p[0] = xt_mfma(wa[0], wb[0], xv[0].x, xv[0].y);
 #pragma unroll
@@ -192,7 +193,7 @@ __global__ __launch_bounds__(64 * AS * RG, OCC) void xt_kernel(xt_args a) {
                 const int c1 = (j + 1) / NW, i1 = (j + 1) % NW;
                 if (i1 == 0) {
                     D[c1 & 1] = xt_mfma(dw, 0u, dxn, 0u);
-                    if (c1 + 1 < C) dxn = *(const uint32_t *)(sd + (c1 + 1) * XT_XD);
+                    if (c1 + 1 < C) dxn = *(const uint32_t *)(sd + (c1 + 1) * 256);
                 }
                 p[(j + 1) & 1] = xt_mfma(wa[i1], wb[i1], xv[(j + 1) % 3].x, xv[(j + 1) % 3].y);
             }
@@ -289,15 +290,343 @@ __global__ __launch_bounds__(256) void xt_pack_kernel(const uint8_t *__restrict_
     for (int i = 0; i < 4; i++) { qv[i] = qv[i] < -128 ? -128 : (qv[i] > 127 ? 127 : qv[i]); h[i] = __builtin_bit_cast(uint16_t, (_Float16)(float)qv[i]); }
     uint8_t *o = xq + ((int64_t)cg * nst + (b >> 2)) * XT_XB + (b & 3) * 1024 + (e >> 1) * 256 + c * 16 + (e & 1) * 8;
     *(uint2 *)o = make_uint2(h[0] | (h[2] << 16), h[1] | (h[3] << 16));
-    if (e == 0) *(uint32_t *)(xd + ((int64_t)cg * nst + (b >> 2)) * XT_XD + (b & 3) * 64 + c * 4) = f2h(d);
+    int sum = (qv[0] + qv[1]) + (qv[2] + qv[3]);
+    sum += __shfl_xor(sum, 1, SPY_WAVE);
+    sum += __shfl_xor(sum, 2, SPY_WAVE);
+    sum += __shfl_xor(sum, 4, SPY_WAVE);
+    if (e == 0) {
+        uint32_t *rec = (uint32_t *)(xd + ((int64_t)cg * nst + (b >> 2)) * XT_XD + (b & 3) * 64 + c * 4);
+        rec[0] = f2h(d);
+        rec[64] = __float_as_uint((float)sum);
+    }
 }
 
 template <int WT, int AS, int RG, int C, int NXS, int P, int NWC, int OCC>
 int xt_launch(hipStream_t st, xt_args a, int nmat) {
-    constexpr size_t ring = NXS * C * (XT_XB + XT_XD) + NWC * ((16 * RG * xt_w<WT>::CU + 63) / 64) * 1024 + 1024, ex = (size_t)RG * (AS - 1) * C * (32 / AS) * 256, lds = ring > ex ? ring : ex;
+    constexpr size_t ring = NXS * C * (XT_XB + 256) + NWC * ((16 * RG * xt_w<WT>::CU + 63) / 64) * 1024 + 1024, ex = (size_t)RG * (AS - 1) * C * (32 / AS) * 256, lds = ring > ex ? ring : ex;
     static_assert(lds <= 64 * 1024, "no raised LDS limit");
     a.tiles = (a.M + 16 * RG - 1) / (16 * RG);
     xt_kernel<WT, AS, RG, C, NXS, P, NWC, OCC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * AS * RG), lds, st>>>(a);
+    return SPY_LAUNCH_RC();
+}
+
+// ---- Q4_K / Q6_K ------------------------------------------------------------------------------------------------------------------------
+// These dots keep ONE accumulator per output and add one term per sub-block of 32 elements (the order this project defines; exact_order.hip):
+//   Q4_K:  acc = fma(d_x, d * float(sc * isum) - dmin * float(m * bsum), acc)       Q6_K:  acc = fma(d_x * d, float(sc0 * isum0 + sc1 * isum1), acc)
+// so the integer sums of a whole sub-block come from v_mfma_f32_16x16x32_f16 -- lane (q, r): elements 8q .. 8q + 7 of row r -- and the vector units
+// have 16 (Q4_K) or 8 (Q6_K) instructions per 16 x 16 tile and sub-block where the tile kernel of exact_order.hip had 64 and 56:
+//   * small integers are fp16 subnormals as they are (the bit pattern n is n * 2^-24): unpacking a pair of nibbles is one AND.  The factor
+//     2^24 goes into the weights' scale; every product and sum below is still exact.
+//   * d * sc, dmin * m and d_w * d_x have at most 22 significant bits: they are exact in fp32, so (d * sc) * isum rounds once, as d * (sc * isum) does.
+//   * Q6_K: q - 32 = l + 16 (h - 2) with the low four and the high two bits, and sc * l, 16 * sc * (h - 2) are exact in fp16: the scales of the
+//     two halves of a sub-block ride on the operands, and two matrix instructions leave sc0 * isum0 + sc1 * isum1 (below 2^24).
+// A wave takes 16 weight rows, which it reads straight into registers one super-block ahead, and C groups of 16 activation rows.
+// 4096 x 4096 x 2048, quantization and packing included: Q4_K 374 -> 162 us, Q6_K 346 -> 169; 77 rows 89 -> 28 and 89 -> 37.  The vector units bound both:
+// 592 (Q4_K: 512 of them the terms) and 484 (Q6_K) instructions per super-block of 16 rows x 4 groups, 4 cycles each.
+typedef _Float16 xk_h8 __attribute__((ext_vector_type(8)));
+typedef float xk_v4f __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ xk_v4f xk_mfma(const uint4 &a, const uint4 &b, const xk_v4f &c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(xk_h8, a), __builtin_bit_cast(xk_h8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ uint32_t xk_pk_mul(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(xt_h2, a) * __builtin_bit_cast(xt_h2, b));
+}
+__device__ __forceinline__ uint32_t xk_pk_fma(uint32_t a, uint32_t b, uint32_t c) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(xt_h2, a), __builtin_bit_cast(xt_h2, b), __builtin_bit_cast(xt_h2, c)));
+}
+typedef uint32_t xk_u2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t xk_u4 __attribute__((ext_vector_type(4), aligned(2)));
+
+// the raw super-block of a lane's weight row: its quants and the row's scales
+template <int WT> struct xk_raw;
+template <> struct xk_raw<SPY_HIP_Q4_K> { uint2 qs[4]; uint4 head; };
+template <> struct xk_raw<SPY_HIP_Q6_K> { uint2 ql[4], qh[2]; uint4 sc; uint32_t d; };
+
+template <int WT>
+__device__ __forceinline__ xk_raw<WT> xk_load(const uint8_t *row, int sb, int q) {
+    xk_raw<WT> t;
+    if constexpr (WT == SPY_HIP_Q4_K) {
+        const uint8_t *p = row + (int64_t)sb * 144;
+        t.head = *(const uint4 *)p;
+#pragma unroll
+        for (int k = 0; k < 4; k++) t.qs[k] = *(const uint2 *)(p + 16 + 32 * k + 8 * q);
+    } else {                                                         // super-blocks of 210 bytes: two-byte alignment
+        const uint8_t *p = row + (int64_t)sb * 210;
+#pragma unroll
+        for (int k = 0; k < 4; k++) t.ql[k] = __builtin_bit_cast(uint2, *(const xk_u2 *)(p + 32 * k + 8 * q));
+#pragma unroll
+        for (int k = 0; k < 2; k++) t.qh[k] = __builtin_bit_cast(uint2, *(const xk_u2 *)(p + 128 + 32 * k + 8 * q));
+        t.sc = __builtin_bit_cast(uint4, *(const xk_u4 *)(p + 192));
+        t.d = *(const uint16_t *)(p + 208);
+    }
+    return t;
+}
+__device__ __forceinline__ float xk_half(uint32_t h) { return h == 0xFFFFu ? 0.0f : h2f((uint16_t)h); }      // conversion.h:39-41
+// The scales of a super-block into the wave's table: lane (q, r) prepares those of row r, sub-blocks 2q and 2q + 1.
+// Q4_K: [sub-block][d * sc | dmin * m][row]; Q6_K: [row] d
+template <int WT>
+__device__ __forceinline__ void xk_put_scales(const xk_raw<WT> &w, float *tab, int q, int r) {
+    if constexpr (WT == SPY_HIP_Q4_K) {
+        const float d = xk_half(w.head.x & 0xFFFFu), dmin = xk_half(w.head.x >> 16);
+        const int s16 = 16 * (q & 1);
+        const uint32_t t0 = w.head.y >> s16, t1 = w.head.z >> s16, t2 = w.head.w >> s16;      // bytes 2q, 2q + 1 (mod 4) of scales[0..3], [4..7], [8..11]
+        const bool hi = q >= 2;                                                               // get_scale_min_k4 for sub-blocks 4 .. 7
+        const uint32_t sc = hi ? (t2 & 0x0F0Fu) | ((t0 >> 2) & 0x3030u) : t0 & 0x3F3Fu, mm = hi ? ((t2 >> 4) & 0x0F0Fu) | ((t1 >> 2) & 0x3030u) : t1 & 0x3F3Fu;
+        float *o = tab + 2 * q * 32 + r;
+        o[0] = (d * 16777216.0f) * (float)(sc & 0xFFu);                 // low nibbles: n * 2^-24
+        o[16] = dmin * (float)(mm & 0xFFu);
+        o[32] = (d * 1048576.0f) * (float)((sc >> 8) & 0xFFu);          // high nibbles stay where they are: n * 2^-20
+        o[48] = dmin * (float)((mm >> 8) & 0xFFu);
+    } else if (q == 0) tab[r] = xk_half(w.d) * 16777216.0f;
+    __builtin_amdgcn_wave_barrier();                                    // other lanes of the wave read them
+    asm volatile("" ::: "memory");
+}
+// operand(s) of sub-block t of the super-block
+template <int WT, int t>
+__device__ __forceinline__ void xk_unpack(const xk_raw<WT> &w, int q, uint4 (&o)[WT == SPY_HIP_Q4_K ? 1 : 2]) {
+    if constexpr (WT == SPY_HIP_Q4_K) {
+        const uint2 v = w.qs[t >> 1];
+        constexpr uint32_t m = t & 1 ? 0x00F000F0u : 0x000F000Fu;
+        o[0] = make_uint4(v.x & m, (v.x >> 8) & m, v.y & m, (v.y >> 8) & m);
+    } else {
+        constexpr int n = t >> 2, grp = t & 3;
+        const uint2 l = w.ql[2 * n + (grp & 1)], h = w.qh[n];
+        const uint32_t scw = t < 2 ? w.sc.x : t < 4 ? w.sc.y : t < 6 ? w.sc.z : w.sc.w;
+        const int sci = (int)(int8_t)(scw >> (16 * (t & 1) + 8 * (q >> 1)));                        // the scale of this lane's half of the sub-block
+        const xt_h2 s2 = {(_Float16)(short)sci, (_Float16)(short)sci};
+        constexpr uint32_t up[4] = {0x4C004C00u, 0x44004400u, 0x3C003C00u, 0x34003400u};            // 16 / 4^grp: the high pair of bits is taken where it stands
+        const uint32_t s = __builtin_bit_cast(uint32_t, s2), sl = grp >> 1 ? xk_pk_mul(s, 0x2C002C00u) : s, sh = xk_pk_mul(s, up[grp]), sm = xk_pk_mul(s, 0x80208020u);
+        constexpr uint32_t ml = grp >> 1 ? 0x00F000F0u : 0x000F000Fu, mh = 0x00030003u << (2 * grp);
+        uint32_t lo[4], hh[4];
+        const uint32_t w2[2] = {l.x, l.y}, h2[2] = {h.x, h.y};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            lo[i] = xk_pk_mul((w2[i >> 1] >> (8 * (i & 1))) & ml, sl);
+            hh[i] = xk_pk_fma((h2[i >> 1] >> (8 * (i & 1))) & mh, sh, sm);
+        }
+        o[0] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        o[1] = make_uint4(hh[0], hh[1], hh[2], hh[3]);
+    }
+}
+
+template <int WT, int RG, int C, int OCC>
+__global__ __launch_bounds__(64 * RG, OCC) void xk_kernel(xt_args a) {
+    constexpr bool K4 = WT == SPY_HIP_Q4_K;
+    constexpr int NT = 64 * RG, ROWS = 16 * RG, NXI = C * 256 / NT, C2 = (C + 1) / 2;
+    constexpr int XB = C * XT_XB + C2 * 1024;
+    constexpr int NXS = 2;                         // stage s is worked on, stage s + 1 is on its way
+    static_assert(NXI * NT == C * 256 && RG >= C2, "one request per thread and group, one wave per two groups' records");
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, r = lane & 15;
+    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS, cg0 = (int)blockIdx.y * C;
+    const int nst = a.nst, ncg = a.ncg, M = a.M;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
+    // activation stages into the ring, as in xt_kernel; one request brings the records of two groups
+    const uint8_t *bx[NXI], *bd;
+#pragma unroll
+    for (int i = 0; i < NXI; i++) bx[i] = a.xq + (int64_t)min(cg0 + (i * NT + wave * 64) / 256, ncg - 1) * nst * XT_XB + (i * NT + wave * 64) % 256 * 16;
+    const int dc0 = min(cg0 + 2 * min(wave, C2 - 1), ncg - 1), dc1 = min(dc0 + 1, ncg - 1);
+    bd = a.xd + (int64_t)dc0 * nst * XT_XD;
+    const uint32_t l16 = lane * 16, ld = (lane & 31) * 16 + (lane >> 5) * (uint32_t)((dc1 - dc0) * nst * XT_XD);
+    const uint32_t ldsx = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024), ldsd = __builtin_amdgcn_readfirstlane(lds0 + C * XT_XB + min(wave, C2 - 1) * 1024);
+    int is = 0;
+    auto issue_x = [&]() {
+        const uint32_t o = (is & (NXS - 1)) * XB;
+        const int adv = is + 1 < nst ? 1 : 0;
+#pragma unroll
+        for (int i = 0; i < NXI; i++) { xt_dma16(bx[i], l16, ldsx + o + i * NT * 16); bx[i] += adv * XT_XB; }
+        xt_dma16(bd, ld, ldsd + o);
+        bd += adv * XT_XD;
+        is++;
+    };
+    const uint8_t *wr = a.w[mat] + (int64_t)min(m0 + wave * 16 + r, M - 1) * a.w_row;
+    xk_raw<WT> cur = xk_load<WT>(wr, 0, q);
+    issue_x();
+
+    float acc[C][4];                               // rows 4q .. 4q + 3 of the wave's 16, activation row r of the group
+#pragma unroll
+    for (int c = 0; c < C; c++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) acc[c][v] = 0.0f;
+    float *tab = (float *)(smem + NXS * XB) + wave * (K4 ? 256 : 16);      // the wave's scales: Q4_K [sub-block][d * sc, dmin * m][row], Q6_K [row] d
+    const xk_v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto compute = [&](int s, auto par_c) {
+        constexpr int par = decltype(par_c)::value;
+        const uint8_t *sx = smem + (s & (NXS - 1)) * XB + q * 256 + r * 16, *sd = smem + (s & (NXS - 1)) * XB + C * XT_XB + r * 4;
+        // steps (sub-block, activation group): operands of step j + 2 read and the matrix instruction of step j + 1 issued before the vector work of step j
+        constexpr int NJ = 4 * C;
+        uint4 w[2][K4 ? 1 : 2], xv[3];
+        uint32_t dx[3];
+        float bs[3];
+        xk_v4f p[2], dsc[2], dm[2];
+        auto rd = [&](int j) {
+            const int b = j / C, c = j % C;
+            xv[j % 3] = *(const uint4 *)(sx + c * XT_XB + b * 1024);
+            dx[j % 3] = *(const uint32_t *)(sd + c * XT_XD + b * 64);
+            if constexpr (K4) bs[j % 3] = *(const float *)(sd + c * XT_XD + 256 + b * 64);
+        };
+        auto weights = [&](auto b_c) {
+            constexpr int b = decltype(b_c)::value;
+            xk_unpack<WT, 4 * par + b>(cur, q, w[b & 1]);
+            if constexpr (K4) {
+                dsc[b & 1] = *(const xk_v4f *)(tab + (4 * par + b) * 32 + 4 * q);
+                dm[b & 1] = *(const xk_v4f *)(tab + (4 * par + b) * 32 + 16 + 4 * q);
+            }
+        };
+        auto mm = [&](int j) {
+            const int b = j / C;
+            p[j & 1] = xk_mfma(w[b & 1][0], xv[j % 3], zero);
+            if constexpr (!K4) p[j & 1] = xk_mfma(w[b & 1][1], xv[j % 3], p[j & 1]);
+        };
+        if constexpr (!K4) dsc[0] = *(const xk_v4f *)(tab + 4 * q);
+        rd(0);
+        rd(1);
+        weights(std::integral_constant<int, 0>{});
+        mm(0);
+        auto step = [&](auto j_c) {
+            constexpr int j = decltype(j_c)::value, b = j / C, c = j % C;
+            if constexpr (j + 2 < NJ) rd(j + 2);
+            if constexpr (j + 1 < NJ) {
+                if constexpr ((j + 1) % C == 0) weights(std::integral_constant<int, (j + 1) / C>{});
+                mm(j + 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const float x = h2f((uint16_t)dx[j % 3]);
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                if constexpr (K4) {
+                    const float pos = dsc[b & 1][v] * p[j & 1][v], neg = dm[b & 1][v] * bs[j % 3];
+                    acc[c][v] = fmaf(x, pos - neg, acc[c][v]);
+                } else acc[c][v] = fmaf(x * dsc[0][v], p[j & 1][v], acc[c][v]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        [&]<int... J>(std::integer_sequence<int, J...>) { (step(std::integral_constant<int, J>{}), ...); }(std::make_integer_sequence<int, NJ>{});
+    };
+    auto ready = [&]() {
+        xt_wait_vm<0>();
+        __builtin_amdgcn_s_barrier();
+    };
+    for (int s = 0; s < nst; s += 2) {
+        ready();
+        xk_put_scales<WT>(cur, tab, q, r);         // the compiler's own wait for the super-block stands here, where nothing is on its way
+        const xk_raw<WT> nxt = xk_load<WT>(wr, min(s / 2 + 1, nst / 2 - 1), q);
+        issue_x();
+        compute(s, std::integral_constant<int, 0>{});
+        ready();
+        issue_x();
+        compute(s + 1, std::integral_constant<int, 1>{});
+        cur = nxt;
+    }
+    xt_wait_vm<0>();
+    const int row = m0 + wave * 16 + 4 * q;
+    float *dst = a.dst[mat];
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int t = (cg0 + c) * 16 + r;
+        if (t < a.T && row + 3 < M) {
+            const int64_t at = (int64_t)t * a.d_row + row;
+            float4 o = make_float4(acc[c][0], acc[c][1], acc[c][2], acc[c][3]);
+            if (a.resid) { const float4 z = *(const float4 *)(a.resid + at); o.x += z.x; o.y += z.y; o.z += z.z; o.w += z.w; }
+            *(float4 *)(dst + at) = o;
+        }
+    }
+}
+// The same dots for few activation rows: a workgroup takes one 16 x 16 tile and its four waves take every fourth super-block.  What is serial is only
+// the fma per sub-block; the terms are independent, so each round the waves leave the terms of four super-blocks in LDS and then every wave
+// walks a quarter of the outputs through their 32 fmas.  (16 rows of a 4096 x 4096 Q4_K matrix: 20 us as a chain in one wave, 10 here.)
+template <int WT>
+__global__ __launch_bounds__(256, 3) void xks_kernel(xt_args a) {
+    constexpr bool K4 = WT == SPY_HIP_Q4_K;
+    __shared__ __align__(16) float s_t[32][4][64];                  // [sub-block of the round][row 4q + v][lane]
+    __shared__ __align__(16) float s_tab[4][K4 ? 256 : 16];
+    __shared__ float s_x[32][16], s_d[4][16];                       // d_x of the round's sub-blocks; Q6_K: d of its super-blocks
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, r = lane & 15;
+    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * 16, cg = (int)blockIdx.y, nsb = a.nst / 2;
+    const uint8_t *wr = a.w[mat] + (int64_t)min(m0 + r, a.M - 1) * a.w_row;
+    const uint8_t *xq = a.xq + (int64_t)cg * a.nst * XT_XB + q * 256 + r * 16, *xd = a.xd + (int64_t)cg * a.nst * XT_XD;
+    xk_raw<WT> cur = xk_load<WT>(wr, min(wave, nsb - 1), q), nxt;
+    uint4 xv[8], xn[8];
+    uint32_t dx[2], dn[2];
+    float bs[K4 ? 8 : 1], bn[K4 ? 8 : 1];
+    auto fetch = [&](int sb, uint4 (&v)[8], uint32_t (&d)[2], float (&b)[K4 ? 8 : 1]) {
+        const uint8_t *p = xq + (int64_t)sb * 2 * XT_XB, *e = xd + (int64_t)sb * 2 * XT_XD;
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = *(const uint4 *)(p + k * 1024);
+#pragma unroll
+        for (int k = 0; k < 2; k++) d[k] = *(const uint32_t *)(e + k * XT_XD + lane * 4);            // lane (q, r): block q of the stage, activation row r
+        if constexpr (K4) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) b[k] = *(const float *)(e + (k >> 2) * XT_XD + 256 + (k & 3) * 64 + r * 4);
+        }
+    };
+    fetch(min(wave, nsb - 1), xv, dx, bs);
+    float *tab = s_tab[wave];
+    const int v_ = wave;                           // the row 4q + v_ of the tile whose outputs this wave walks
+    float acc = 0.0f;
+    const xk_v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = 0; s0 < nsb; s0 += 4) {
+        const int sb = s0 + wave;
+        xk_put_scales<WT>(cur, tab, q, r);
+        if (s0 + 4 < nsb) { nxt = xk_load<WT>(wr, min(sb + 4, nsb - 1), q); fetch(min(sb + 4, nsb - 1), xn, dn, bn); }
+        if (s0) __syncthreads();                   // the terms of the round before have been walked
+#pragma unroll
+        for (int k = 0; k < 2; k++) s_x[wave * 8 + 4 * k + q][r] = h2f((uint16_t)dx[k]);
+        if (!K4 && q == 0) s_d[wave][r] = tab[r];
+        auto term = [&](auto t_c) {
+            constexpr int t = decltype(t_c)::value;
+            uint4 w[K4 ? 1 : 2];
+            xk_unpack<WT, t>(cur, q, w);
+            xk_v4f p = xk_mfma(w[0], xv[t], zero);
+            if constexpr (!K4) p = xk_mfma(w[1], xv[t], p);
+            if constexpr (K4) {
+                const xk_v4f dsc = *(const xk_v4f *)(tab + t * 32 + 4 * q), dm = *(const xk_v4f *)(tab + t * 32 + 16 + 4 * q);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const float pos = dsc[v] * p[v], neg = dm[v] * bs[t];
+                    p[v] = pos - neg;
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) s_t[wave * 8 + t][v][lane] = p[v];
+        };
+        [&]<int... J>(std::integer_sequence<int, J...>) { (term(std::integral_constant<int, J>{}), ...); }(std::make_integer_sequence<int, 8>{});
+        __syncthreads();
+        const int nb = min(4, nsb - s0) * 8;
+#pragma unroll 8
+        for (int b = 0; b < nb; b++) {
+            float x = s_x[b][r];
+            if constexpr (!K4) x = x * s_d[b >> 3][4 * q + v_];
+            acc = fmaf(x, s_t[b][v_][lane], acc);
+        }
+        cur = nxt;
+#pragma unroll
+        for (int k = 0; k < 8; k++) xv[k] = xn[k];
+        dx[0] = dn[0]; dx[1] = dn[1];
+        if constexpr (K4) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) bs[k] = bn[k];
+        }
+    }
+    const int row = m0 + 4 * q + v_, t = cg * 16 + r;
+    if (t < a.T && row < a.M) {
+        const int64_t at = (int64_t)t * a.d_row + row;
+        a.dst[mat][at] = a.resid ? acc + a.resid[at] : acc;
+    }
+}
+template <int WT, int RG, int C, int OCC>
+int xk_launch(hipStream_t st, xt_args a, int nmat) {
+    constexpr size_t lds = 2 * (C * XT_XB + (C + 1) / 2 * 1024) + RG * 1024;
+    if (lds > 64 * 1024) { const int rc = spy_raise_lds_limit((const void *)xk_kernel<WT, RG, C, OCC>, lds); if (rc) return rc; }
+    a.tiles = (a.M + 16 * RG - 1) / (16 * RG);
+    xk_kernel<WT, RG, C, OCC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * RG), lds, st>>>(a);
+    return SPY_LAUNCH_RC();
+}
+template <int WT>
+int xks_launch(hipStream_t st, xt_args a, int nmat) {
+    a.tiles = (a.M + 15) / 16;
+    xks_kernel<WT><<<dim3((unsigned)(a.tiles * nmat), (unsigned)a.ncg), dim3(256), 0, st>>>(a);
     return SPY_LAUNCH_RC();
 }
 
@@ -310,18 +639,41 @@ int xt_num_cu() {
     return n;
 }
 
-// Which tile: a workgroup of four waves puts one wave on each SIMD, and n workgroups per compute unit take about lat + (n - 1) * inc (in
-// tenths of a microsecond for K = 4096, measured for n = 1 .. 16): small tiles have the shorter chain, large ones unpack a weight for
-// more activation rows.
+// Which tile.  n workgroups per compute unit take about lat + (n - 1) * inc: figures in tenths of a microsecond for K = 4096, measured for
+// n = 1 .. 16 (whole workgroups count while they are few; everything scales with K).  Small tiles have the shorter chain, large ones unpack a
+// weight for more activation rows.
+struct xt_cost { int rows, groups, lat, inc; };
+int xt_pick(const xt_args &a, int nmat, const xt_cost *c, int n) {
+    const int64_t cu = xt_num_cu();
+    int best = 0;
+    int64_t least = 0;
+    for (int i = 0; i < n; i++) {
+        const int64_t wgs = (int64_t)((a.M + c[i].rows - 1) / c[i].rows) * nmat * ((a.ncg + c[i].groups - 1) / c[i].groups);
+        const int64_t t = c[i].lat + (wgs <= 6 * cu ? (wgs + cu - 1) / cu * 10 - 10 : 10 * wgs / cu - 10) * c[i].inc / 10;
+        if (!i || t < least) { best = i; least = t; }
+    }
+    return best;
+}
 template <int WT>
 int xt_dispatch(hipStream_t st, const xt_args &a, int nmat) {
-    const int64_t cu = xt_num_cu(), r16 = (int64_t)((a.M + 15) / 16) * nmat, r32 = (int64_t)((a.M + 31) / 32) * nmat;
-    auto cost = [&](int64_t wgs, int64_t lat, int64_t inc) { return lat + (wgs <= 6 * cu ? (wgs + cu - 1) / cu - 1 : (10 * wgs / cu - 10) / 10) * inc; };
-    const int64_t k0 = cost(r16 * a.ncg, 86, 43), k1 = cost(r32 * a.ncg, 103, 56), k2 = cost(r32 * ((a.ncg + 1) / 2), 173, 96), k4 = cost(r32 * ((a.ncg + 3) / 4), 288, 165);
-    if (k4 <= k0 && k4 <= k1 && k4 <= k2) return xt_launch<WT, 2, 2, 4, 2, 1, 2, 3>(st, a, nmat);
-    if (k2 <= k0 && k2 <= k1) return xt_launch<WT, 2, 2, 2, 4, 2, 2, 3>(st, a, nmat);
-    if (k1 <= k0) return xt_launch<WT, 2, 2, 1, 4, 2, 2, 3>(st, a, nmat);
-    return xt_launch<WT, 4, 1, 1, 8, 6, 4, 2>(st, a, nmat);
+    static const xt_cost c[4] = {{16, 1, 86, 43}, {32, 1, 103, 56}, {32, 2, 173, 96}, {32, 4, 288, 165}};
+    switch (xt_pick(a, nmat, c, 4)) {
+    case 0: return xt_launch<WT, 4, 1, 1, 8, 6, 4, 2>(st, a, nmat);
+    case 1: return xt_launch<WT, 2, 2, 1, 4, 2, 2, 3>(st, a, nmat);
+    case 2: return xt_launch<WT, 2, 2, 2, 4, 2, 2, 3>(st, a, nmat);
+    default: return xt_launch<WT, 2, 2, 4, 2, 1, 2, 3>(st, a, nmat);
+    }
+}
+template <int WT>
+int xk_dispatch(hipStream_t st, const xt_args &a, int nmat) {
+    static const xt_cost k4[4] = {{16, 1, 94, 43}, {64, 2, 230, 132}, {64, 4, 360, 205}, {128, 8, 900, 660}},
+                         k6[4] = {{16, 1, 110, 56}, {64, 2, 330, 210}, {64, 4, 440, 260}, {128, 8, 940, 690}};
+    switch (xt_pick(a, nmat, WT == SPY_HIP_Q4_K ? k4 : k6, 4)) {
+    case 0: return xks_launch<WT>(st, a, nmat);
+    case 1: return xk_launch<WT, 4, 2, 4>(st, a, nmat);
+    case 2: return xk_launch<WT, 4, 4, 4>(st, a, nmat);
+    default: return xk_launch<WT, 8, 8, 4>(st, a, nmat);
+    }
 }
 
 }   // namespace
@@ -334,7 +686,7 @@ size_t spy_xgemm_pack_bytes(int64_t T, int64_t K) {
 }
 // shapes and alignments the kernels take: whole chunks, 16-byte-aligned weight rows, four outputs stored together
 bool spy_xgemm_ok(int wtype, const void *w, const float *dst, int64_t M, int64_t K, int64_t T, int64_t d_row) {
-    return (wtype == SPY_HIP_Q4_0 || wtype == SPY_HIP_Q8_0) && T >= 2 && T < (1 << 20) && K > 0 && K % 256 == 0 && K <= (1 << 20) && M > 0 && M % 4 == 0 && M < (1 << 24) &&
+    return (wtype == SPY_HIP_Q4_0 || wtype == SPY_HIP_Q8_0 || wtype == SPY_HIP_Q4_K || wtype == SPY_HIP_Q6_K) && T >= 2 && T < (1 << 20) && K > 0 && K % 256 == 0 && K <= (1 << 20) && M > 0 && M % 4 == 0 && M < (1 << 24) &&
            ((uintptr_t)w & 15) == 0 && ((uintptr_t)dst & 15) == 0 && d_row % 4 == 0;
 }
 int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, int64_t K, void *pack) {
@@ -356,5 +708,10 @@ int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *
     a.resid = resid; a.w_row = spy_row_size(wtype, K); a.d_row = d_row;
     a.M = (int)M; a.nst = (int)(K / 128); a.ncg = (int)((T + 15) / 16); a.T = (int)T;
     a.xq = (const uint8_t *)pack; a.xd = a.xq + (int64_t)a.ncg * a.nst * XT_XB;
-    return wtype == SPY_HIP_Q4_0 ? xt_dispatch<SPY_HIP_Q4_0>(st, a, nmat) : xt_dispatch<SPY_HIP_Q8_0>(st, a, nmat);
+    switch (wtype) {
+    case SPY_HIP_Q4_0: return xt_dispatch<SPY_HIP_Q4_0>(st, a, nmat);
+    case SPY_HIP_Q8_0: return xt_dispatch<SPY_HIP_Q8_0>(st, a, nmat);
+    case SPY_HIP_Q4_K: return xk_dispatch<SPY_HIP_Q4_K>(st, a, nmat);
+    default: return xk_dispatch<SPY_HIP_Q6_K>(st, a, nmat);
+    }
 }

@@ -661,9 +661,9 @@ static size_t matmul_act_bytes(const spy_hip_tensor *w, const spy_hip_tensor *x)
 // MatMul runs from (a call with less than this, but the activations' part, runs the kernel that unpacks per tile: same results)
 extern "C" size_t spy_hip_op_matmul_scratch_size(const spy_hip_tensor *w, const spy_hip_tensor *x) {
     const size_t act = matmul_act_bytes(w, x);
-    if (!act || !spy_exact_on() || x->type != SPY_HIP_F32 || (w->type != SPY_HIP_Q4_0 && w->type != SPY_HIP_Q8_0) || w->ne[2] != 1 || w->ne[3] != 1) return act;
-    const size_t pk = spy_exact_pack_bytes(w->ne[1], w->ne[0], x->ne[1]);
-    const size_t xp = x->ne[1] >= 2 ? spy_xgemm_pack_bytes(x->ne[1], x->ne[0]) : 0;
+    if (!act || !spy_exact_on() || x->type != SPY_HIP_F32 || mid_type(w->type, x->type) != SPY_HIP_Q8_0 || w->ne[2] != 1 || w->ne[3] != 1) return act;
+    const size_t pk = w->type == SPY_HIP_Q4_0 || w->type == SPY_HIP_Q8_0 ? spy_exact_pack_bytes(w->ne[1], w->ne[0], x->ne[1]) : 0;
+    const size_t xp = x->ne[1] >= 3 ? spy_xgemm_pack_bytes(x->ne[1], x->ne[0]) : 0;
     const size_t need = pk ? ((act + 255) & ~(size_t)255) + pk : act;
     return need > xp ? need : xp;
 }
@@ -721,9 +721,9 @@ static int matmul_impl(void *stream, const spy_hip_tensor *w, const spy_hip_tens
                                       : own_matvec(st, t0, w->data, (const float *)x->data, (float *)dst->data, ne01, ne00);
         if (rc != SPY_HIP_EUNSUPPORTED) return rc;
     }
-    // the host's order, several rows: the kernels of exact_gemm.hip where they take the matrix and the scratch buffer holds the packed
-    // activations (SPY_HIP_EXACT_TILED=u / 0, SPY_HIP_EXACT_SERIAL: tests of the other kernels)
-    if (quant && t1 == SPY_HIP_F32 && ne11 >= 2 && ne12 == 1 && ne13 == 1 && skip_past < 0 && klimit_past < 0 && spy_exact_on() && x->nb[0] == 4 && x->nb[1] % 16 == 0 &&
+    // the host's order, three rows and more (two single-row launches take less): the kernels of exact_gemm.hip where they take the matrix and
+    // the scratch buffer holds the packed activations (SPY_HIP_EXACT_TILED=u / 0, SPY_HIP_EXACT_SERIAL: tests of the other kernels)
+    if (quant && t1 == SPY_HIP_F32 && ne11 >= 3 && ne12 == 1 && ne13 == 1 && skip_past < 0 && klimit_past < 0 && spy_exact_on() && x->nb[0] == 4 && x->nb[1] % 16 == 0 &&
         ((uintptr_t)x->data & 15) == 0 && dst->nb[1] % 16 == 0 && w->nb[0] == spy_type_size(t0) && w->nb[1] == spy_row_size(t0, ne00) &&
         spy_xgemm_ok(t0, w->data, (const float *)dst->data, ne01, ne00, ne11, dst->nb[1] / 4)) {
         const char *tiled = getenv("SPY_HIP_EXACT_TILED");

@@ -91,16 +91,25 @@ def test_single_row_matmul_takes_the_two_phase_kernel(hip, oracle, wtype, M, K, 
             assert (scratch.download(np.uint8) == 0xEE).all(), "the single-row route does not use the scratch buffer"
 
 
-@pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0])
-@pytest.mark.parametrize("M,K,T", [(4, 256, 2), (20, 512, 3), (4096, 256, 15), (100, 1024, 16), (36, 4096, 17), (12288, 256, 33), (4100, 512, 48), (8192, 256, 100), (4096, 768, 257)])
+@pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0, O.Q4_K, O.Q6_K])
+@pytest.mark.parametrize("M,K,T", [(4, 256, 3), (20, 512, 4), (4096, 256, 15), (100, 1280, 16), (36, 4096, 17), (12288, 256, 33), (4100, 512, 48), (8192, 256, 100), (4096, 768, 257), (8192, 256, 1025)])
 def test_packed_activation_matmul_bits(hip, oracle, wtype, M, K, T):
-    """Two rows and more against whole super-block rows: the kernels that unpack a weight once per wave (exact_gemm.hip), in every tile
+    """Three rows and more against rows of whole super-blocks: the kernels that unpack a weight once per wave (exact_gemm.hip), in every tile
     the dispatch has, with partial tiles on both sides, the shortest contraction and scales down to fp16 subnormals."""
     from tests.gpu_util import dev, dev_empty, call
     rng = np.random.default_rng(11 * wtype + M + K + T)
     w = O.quantize(oracle, (rng.standard_normal((M, K)) * 0.02).astype(np.float32), wtype)
     x = (rng.standard_normal((T, K // 32, 32)) * 2.0 ** rng.integers(-18, 6, (T, K // 32, 1))).reshape(T, K).astype(np.float32)
     x[0, 32:64] = 0.0
+    if wtype in (O.Q4_K, O.Q6_K):                                        # every quant, scale and minimum byte there is, on the first rows
+        wb = w.reshape(M, -1)
+        bs = 144 if wtype == O.Q4_K else 210
+        rnd = rng.integers(0, 256, (min(M, 64), wb.shape[1] // bs, bs)).astype(np.uint8)
+        scale = slice(0, 4) if wtype == O.Q4_K else slice(208, 210)      # the fp16 scales stay
+        rnd[:, :, scale] = wb[:rnd.shape[0]].reshape(rnd.shape)[:, :, scale]
+        wb[:rnd.shape[0]] = rnd.reshape(rnd.shape[0], -1)
+        w = wb.reshape(w.shape)
+        x[1, :32] = np.sign(x[1, :32])                                   # activation quants of +-127: the largest sums
     want = O.matmul(oracle, w, wtype, M, K, x, nthread=8)
     tw, tx = hip.tensor(dev(w), wtype, [K, M]), hip.tensor(dev(x), hip.F32, [K, T])
     L = hip.load()

@@ -364,7 +364,12 @@ int spy_softmax_row_ok(int64_t ne0);                                            
 int64_t spy_exact_prompt_attn_row(int64_t n_kv);                                                                             // exact_prompt.hip
 size_t spy_exact_pack_bytes(int64_t ne01, int64_t ne00, int64_t ne11);                                                           // exact_order.hip
 size_t spy_xgemm_pack_bytes(int64_t T, int64_t K);                                                                              // exact_gemm.hip
-int spy_exact_prompt_attn(hipStream_t st, const float *q, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, float *out, const float *lut,
+bool spy_xgemm_ok(int wtype, const void *w, const float *dst, int64_t M, int64_t K, int64_t T, int64_t d_row);
+int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, int64_t K, void *pack);
+int spy_xgemm_norm_pack(hipStream_t st, const float *x, const float *w, float eps, int64_t T, int64_t K, void *pack);
+int spy_xgemm_silu_pack(hipStream_t st, const float *gate, const float *up, const float *lut, int64_t T, int64_t F, void *pack);
+int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
+int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, float *out, const float *lut,
                           int T, int H, int P, int64_t C, int n_total, float scale);                                        // exact_prompt.hip
 
 // KQ mask of a pass over tokens P .. P + T - 1 (llama.cpp:248-263): row i allows the cached positions j <= P + i
@@ -382,6 +387,88 @@ static bool exact_attn_ok(const spy_hip_llama *m) {
     const char *e = getenv("SPY_HIP_EXACT_PROMPT_ATTN");
     return m->hd == 128 && m->desc.n_ctx % 32 == 0 && m->desc.n_ctx <= 8192 && m->lut && !(e && e[0] == '0');
 }
+static int ops_workspace(spy_hip_llama *m, hipStream_t st, size_t bytes) {
+    if (bytes <= m->ops_bytes) return 0;
+    if (m->ops_buf) { HIP_TRY(hipStreamSynchronize(st)); HIP_TRY(hipFree(m->ops_buf)); m->ops_buf = nullptr; m->ops_bytes = 0; }
+    HIP_TRY(hipMalloc((void **)&m->ops_buf, bytes));
+    m->ops_bytes = bytes;
+    return 0;
+}
+
+// A prompt pass in the host's order with what lies between two MatMuls in the kernels around them, 13 launches per layer instead of 42:
+// norm and activation end in the next MatMul's packed activations (quantized once for wq | wk | wv and for gate | up, which are one launch
+// each where their types allow), Rope stores q as fp16 and k into its cache rows, the residual additions are the products' epilogues.  Each
+// step is the arithmetic of the operator it replaces, so the bits are those of forward_ops with the exact order on.
+static bool exact_fused_ok(const spy_hip_llama *m, int T) {
+    const spy_hip_llama_desc &c = m->desc;
+    if (!m->exact_ok || !m->rope_tab || T < 2 || c.n_embd % 256 || c.n_ff % 256 || c.n_embd > 8192 || ((uintptr_t)c.out_norm & 15) || !exact_attn_ok(m)) return false;
+    if (getenv("SPY_HIP_EXACT_TILED") || getenv("SPY_HIP_EXACT_SERIAL")) return false;          // tests of the operator kernels
+    for (const spy_hip_llama_layer &L : m->layers) {
+        const void *w[9] = {L.wq, L.wk, L.wv, L.wo, L.w_gate, L.w_up, L.w_down, L.attn_norm, L.ffn_norm};
+        for (const void *p : w) if ((uintptr_t)p & 15) return false;
+        if (L.t_wq != L.t_wk || L.t_gate != L.t_up) return false;
+    }
+    return true;
+}
+static int forward_exact(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_host, int T, int P, float *logits_host, int head, int n_total) {
+    const spy_hip_llama_desc &c = m->desc;
+    const int64_t d = c.n_embd, F = c.n_ff, C = c.n_ctx, H = c.n_head, hd = m->hd, V = c.n_vocab;
+    size_t off = 0;
+    auto take = [&](size_t bytes) { size_t o = off; off += (bytes + 255) & ~(size_t)255; return o; };
+    const size_t sp = (size_t)spy_exact_prompt_attn_row((int64_t)P + T) * T * H;
+    const size_t o_x = take(d * T * 4), o_t1 = take(d * T * 4), o_q = take(d * T * 4), o_k = take(d * T * 4), o_v = take(d * T * 4), o_o2 = take(d * T * 4), o_q16 = take(d * T * 2),
+                 o_up = take(F * T * 4), o_gate = take(F * T * 4), o_S = take(sp * 4), o_P = take(sp * 2), o_ids = take(T * 4), o_xn = take(d * 4),
+                 o_logits = take(head == HEAD_ALL ? V * T * 4 : V * 4), o_pack = take(spy_xgemm_pack_bytes(T, F > d ? F : d));
+    RC_TRY(ops_workspace(m, st, off));
+    uint8_t *B = m->ops_buf;
+    float *x = (float *)(B + o_x), *t1 = (float *)(B + o_t1), *q = (float *)(B + o_q), *k = (float *)(B + o_k), *v = (float *)(B + o_v), *o2 = (float *)(B + o_o2),
+          *up = (float *)(B + o_up), *gate = (float *)(B + o_gate), *lg = (float *)(B + o_logits), *xn = (float *)(B + o_xn);
+    uint16_t *q16 = (uint16_t *)(B + o_q16);
+    int32_t *ids = (int32_t *)(B + o_ids);
+    void *pack = B + o_pack;
+    const float scale = 1.0f / sqrtf((float)hd);
+    HIP_TRY(hipMemcpyAsync(ids, tokens_host, (size_t)T * 4, hipMemcpyHostToDevice, st));
+    spy_hip_tensor t_ids = T2(SPY_HIP_I32, ids, T, 1), t_x = T2(SPY_HIP_F32, x, d, T);
+    t_ids.dim = 1;
+    { spy_hip_tensor te = T2(c.t_tok_embd, (void *)c.tok_embd, d, V); RC_TRY(spy_hip_op_get_row(st, &te, &t_ids, &t_x)); }
+    for (int il = 0; il < c.n_layer; il++) {
+        const spy_hip_llama_layer &L = m->layers[il];
+        RC_TRY(spy_xgemm_norm_pack(st, x, L.attn_norm, c.eps, T, d, pack));
+        const void *w3[3] = {L.wq, L.wk, L.wv};
+        float *d3[3] = {q, k, v};
+        const int together = L.t_wv == L.t_wq ? 3 : 2;
+        RC_TRY(spy_xgemm(st, L.t_wq, together, w3, d3, d, d, T, d, nullptr, pack));
+        if (together == 2) RC_TRY(spy_xgemm(st, L.t_wv, 1, w3 + 2, d3 + 2, d, d, T, d, nullptr, pack));
+        RC_TRY(spy_rope_store_launch(st, q, k, m->rope_tab + (size_t)P * hd, q16, m->k_cache[il] + d * P, T, (int)H, (int)hd));
+        RC_TRY(spy_vt_store_launch(st, v, m->v_cache[il] + P, T, (int)d, C));
+        RC_TRY(spy_exact_prompt_attn(st, q16, true, m->k_cache[il], m->v_cache[il], (float *)(B + o_S), (uint16_t *)(B + o_P), o2, m->lut, T, (int)H, P, C, n_total, scale));
+        RC_TRY(spy_xgemm_pack(st, o2, 4 * d, T, d, pack));
+        RC_TRY(spy_xgemm(st, L.t_wo, 1, &L.wo, &t1, d, d, T, d, x, pack));                     // KQV_linear + Add
+        RC_TRY(spy_xgemm_norm_pack(st, t1, L.ffn_norm, c.eps, T, d, pack));
+        const void *w2[2] = {L.w_up, L.w_gate};
+        float *d2[2] = {up, gate};
+        RC_TRY(spy_xgemm(st, L.t_up, 2, w2, d2, F, d, T, F, nullptr, pack));
+        RC_TRY(spy_xgemm_silu_pack(st, gate, up, m->lut, T, F, pack));
+        RC_TRY(spy_xgemm(st, L.t_down, 1, &L.w_down, &x, d, F, T, d, t1, pack));              // ffn_down + Add
+    }
+    if (head == HEAD_ALL) {
+        RC_TRY(spy_xgemm_norm_pack(st, x, c.out_norm, c.eps, T, d, pack));
+        if (spy_xgemm_ok(c.t_out, c.w_out, lg, V, d, T, V)) RC_TRY(spy_xgemm(st, c.t_out, 1, &c.w_out, &lg, V, d, T, V, nullptr, pack));
+        else return SPY_HIP_EUNSUPPORTED;
+        if (logits_host) HIP_TRY(hipMemcpyAsync(logits_host, lg, (size_t)V * T * 4, hipMemcpyDeviceToHost, st));
+    } else if (head == HEAD_LAST) {
+        spy_hip_tensor t_nw = T2(SPY_HIP_F32, (void *)c.out_norm, d, 1), t_x1 = T2(SPY_HIP_F32, x + (size_t)(T - 1) * d, d, 1), t_xn1 = T2(SPY_HIP_F32, xn, d, 1), t_l1 = T2(SPY_HIP_F32, lg, V, 1),
+                       tw = T2(c.t_out, (void *)c.w_out, d, V);
+        t_nw.dim = 1;
+        RC_TRY(spy_hip_op_norm_rms(st, &t_x1, &t_xn1, c.eps));
+        RC_TRY(spy_hip_op_binary(st, 2, &t_xn1, &t_nw, &t_xn1));
+        RC_TRY(spy_hip_op_matmul(st, &tw, &t_xn1, &t_l1, pack, spy_xgemm_pack_bytes(T, d)));
+        if (logits_host) HIP_TRY(hipMemcpyAsync(logits_host, lg, (size_t)V * 4, hipMemcpyDeviceToHost, st));
+    }
+    HIP_TRY(hipStreamSynchronize(st));
+    return 0;
+}
+
 static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_host, int T, int P, float *logits_host, int head, int n_total) {
     const spy_hip_llama_desc &c = m->desc;
     const int64_t d = c.n_embd, F = c.n_ff, C = c.n_ctx, H = c.n_head, hd = m->hd, V = c.n_vocab, n_kv = (int64_t)P + T;
@@ -416,11 +503,7 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
     const size_t xpack = exact && T >= 2 ? spy_xgemm_pack_bytes(T, F > d ? F : d) : 0;
     const size_t o_scr = take(std::max((act_q8 > act_f16 ? act_q8 : act_f16) + 256 + pack, xpack));
     const size_t scr_bytes = off - o_scr;
-    if (off > m->ops_bytes) {
-        if (m->ops_buf) { HIP_TRY(hipStreamSynchronize(st)); HIP_TRY(hipFree(m->ops_buf)); m->ops_buf = nullptr; m->ops_bytes = 0; }
-        HIP_TRY(hipMalloc((void **)&m->ops_buf, off));
-        m->ops_bytes = off;
-    }
+    RC_TRY(ops_workspace(m, st, off));
     uint8_t *B = m->ops_buf;
     float *x = (float *)(B + o_x), *xn = (float *)(B + o_xn), *q = (float *)(B + o_q), *k = (float *)(B + o_k), *v = (float *)(B + o_v),
           *o = (float *)(B + o_o), *o2 = (float *)(B + o_o2), *t1 = (float *)(B + o_t1), *up = (float *)(B + o_up), *gate = (float *)(B + o_gate),
@@ -493,7 +576,7 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
             RC_TRY(spy_prompt_attn_launch(st, (const uint16_t *)xn, (const uint16_t *)m->k_cache[il], (const uint16_t *)m->v_cache[il], o2,
                                           T, (int)H, (int)hd, P, C, scale));
         } else if (xattn) {
-            RC_TRY(spy_exact_prompt_attn(st, q, (const uint16_t *)m->k_cache[il], (const uint16_t *)m->v_cache[il], S, (uint16_t *)Pm, o2, m->lut,
+            RC_TRY(spy_exact_prompt_attn(st, q, false, (const uint16_t *)m->k_cache[il], (const uint16_t *)m->v_cache[il], S, (uint16_t *)Pm, o2, m->lut,
                                          T, (int)H, P, C, n_total, scale));
         } else {
         spy_hip_tensor t_kall = T3s(SPY_HIP_F16, m->k_cache[il], hd, n_kv, H, 2, 2 * d, 2 * hd);
@@ -597,12 +680,14 @@ static int forward_any(spy_hip_llama *m, void *stream, const int32_t *tokens_hos
     // the 8-lane part and the scalar tail of the KQV dots and between the groups of four of the softmax sum)
     // ... unless the attention kernels that take the length of the whole row as a number are in use
     const int CH = exact && !exact_attn_ok(m) ? n_token : ch_req >= 16 ? ch_req : SPY_PREFILL_CHUNK;
+    const bool fused = exact && exact_fused_ok(m, n_token) && (m->desc.n_vocab % 4 == 0 && ((uintptr_t)m->desc.w_out & 15) == 0);
     for (int t0 = 0; t0 < n_token; t0 += CH) {
         const int tc = n_token - t0 < CH ? n_token - t0 : CH;
         // logits nobody asked for are not computed: no buffer -> no head; last_only -> the head runs on the last row of the last chunk
         const int head = !logits_host ? HEAD_NONE : !last_only ? HEAD_ALL : (t0 + tc == n_token ? HEAD_LAST : HEAD_NONE);
         float *dst = !logits_host ? nullptr : last_only ? logits_host : logits_host + (size_t)t0 * m->desc.n_vocab;
-        RC_TRY(forward_ops(m, st, tokens_host + t0, tc, n_past + t0, dst, head, n_past + n_token));
+        if (fused && tc >= 2) RC_TRY(forward_exact(m, st, tokens_host + t0, tc, n_past + t0, dst, head, n_past + n_token));
+        else RC_TRY(forward_ops(m, st, tokens_host + t0, tc, n_past + t0, dst, head, n_past + n_token));
     }
     return 0;
 }

@@ -301,6 +301,105 @@ __global__ __launch_bounds__(256) void xt_pack_kernel(const uint8_t *__restrict_
     }
 }
 
+// ---- producers: the operators in front of a MatMul, ending in its packed activations, in the host's order ---------------------------------
+// Two words (eight elements) per lane, four lanes per block: quantize and store.  xq, xd: the bases of the lane's block for activation row 0 of the group
+__device__ __forceinline__ void xt_store8(const float (&y)[8], int sub, uint8_t *xq, uint8_t *xd, int row) {
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(y[i]));
+    amax = fmaxf(amax, __shfl_xor(amax, 1, SPY_WAVE));
+    amax = fmaxf(amax, __shfl_xor(amax, 2, SPY_WAVE));
+    const float d = amax / 127.0f, id = (amax != 0.0f) ? 127.0f / amax : 0.0f;
+    int sum = 0;
+    uint32_t h[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        int q = (int)rintf(y[i] * id);
+        q = q < -128 ? -128 : (q > 127 ? 127 : q);
+        sum += q;
+        h[i] = __builtin_bit_cast(uint16_t, (_Float16)(float)q);
+    }
+    sum += __shfl_xor(sum, 1, SPY_WAVE);
+    sum += __shfl_xor(sum, 2, SPY_WAVE);
+    *(uint4 *)(xq + sub * 256 + row * 16) = make_uint4(h[0] | (h[2] << 16), h[1] | (h[3] << 16), h[4] | (h[6] << 16), h[5] | (h[7] << 16));
+    if (sub == 0) {
+        *(uint32_t *)(xd + row * 4) = f2h(d);
+        *(float *)(xd + 256 + row * 4) = (float)sum;
+    }
+}
+
+// NormRMS (non-linear.cpp:194-223) -> Mul by the norm weights -> packed activations; one wave per row.  The sum of squares is the host's
+// std::transform_reduce: groups of four, (x0^2 + x1^2) + (x2^2 + x3^2), added to one running sum.  That chain (K / 4 additions of 4.3 ns)
+// is the length of the kernel; rows past T of the last group are written as zeros.
+#define XT_NORM_WAVES 4
+template <int NV>        // K <= 512 * NV
+__global__ __launch_bounds__(64 * XT_NORM_WAVES) void xt_norm_pack_kernel(const float *__restrict__ x, const float *__restrict__ w, float eps, int K, int T, int nst,
+                                                                          uint8_t *__restrict__ xq, uint8_t *__restrict__ xd) {
+    extern __shared__ __attribute__((aligned(16))) float s_grp[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = (int)blockIdx.x * XT_NORM_WAVES + wave;
+    const int cg = t >> 4, row = t & 15, n8 = K / 8;
+    float *g = s_grp + wave * (K / 4 + 64);
+    const float4 *xr = (const float4 *)(x + (int64_t)min(t, T - 1) * K);
+    float4 v[NV][2];
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = min(j * 64 + lane, n8 - 1);
+        v[j][0] = xr[2 * i]; v[j][1] = xr[2 * i + 1];
+        if (j * 64 + lane < n8) {
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const float4 z = v[j][k];
+                const float a0 = z.x * z.x, a1 = z.y * z.y, a2 = z.z * z.z, a3 = z.w * z.w, v1 = a0 + a1, v2 = a2 + a3;
+                g[2 * i + k] = v1 + v2;
+            }
+        }
+    }
+    __builtin_amdgcn_wave_barrier();               // the other lanes of the wave read them
+    asm volatile("" ::: "memory");
+    float sum = 0.0f;
+    {   // four group sums per read, requested two reads (eight additions) ahead; K / 4 is a multiple of 64
+        const float4 *p = (const float4 *)g;
+        float4 a = p[0], b = p[1];
+        for (int i = 0; i < K / 16; i += 2) {
+            const float4 c = p[i + 2], e = p[i + 3];                 // up to 8 floats past the row's sums: not added
+            sum = sum + a.x; sum = sum + a.y; sum = sum + a.z; sum = sum + a.w;
+            sum = sum + b.x; sum = sum + b.y; sum = sum + b.z; sum = sum + b.w;
+            a = c; b = e;
+        }
+    }
+    const float mean = sum / (float)K, scale = 1.0f / sqrtf(mean + eps);
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = j * 64 + lane;
+        if (i < n8) {                                                // n8 is a multiple of 32: the four lanes of a block stay together
+            const float4 w0 = ((const float4 *)w)[2 * i], w1 = ((const float4 *)w)[2 * i + 1], v0 = v[j][0], v1 = v[j][1];
+            float y[8] = {(v0.x * scale) * w0.x, (v0.y * scale) * w0.y, (v0.z * scale) * w0.z, (v0.w * scale) * w0.w,
+                          (v1.x * scale) * w1.x, (v1.y * scale) * w1.y, (v1.z * scale) * w1.z, (v1.w * scale) * w1.w};
+            if (t >= T) {
+#pragma unroll
+                for (int k = 0; k < 8; k++) y[k] = 0.0f;
+            }
+            const int b = i >> 2;
+            xt_store8(y, i & 3, xq + ((int64_t)cg * nst + (b >> 2)) * XT_XB + (b & 3) * 1024, xd + ((int64_t)cg * nst + (b >> 2)) * XT_XD + (b & 3) * 64, row);
+        }
+    }
+}
+
+// Silu by the host's table -> Mul (up * silu(gate)) -> packed activations (non-linear.cpp:11-14,57-77); a workgroup takes 16 rows and four blocks
+__global__ __launch_bounds__(256) void xt_silu_pack_kernel(const float *__restrict__ gate, const float *__restrict__ up, const float *__restrict__ lut, int F, int T, int nst,
+                                                           uint8_t *__restrict__ xq, uint8_t *__restrict__ xd) {
+    const int tid = threadIdx.x, sub = tid & 3, bl = (tid >> 2) & 3, row = tid >> 4, b = (int)blockIdx.x * 4 + bl, cg = blockIdx.y, t = cg * 16 + row;
+    float y[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    if (t < T) {
+        const int64_t at = (int64_t)t * F + b * 32 + sub * 8;
+        const float4 g0 = *(const float4 *)(gate + at), g1 = *(const float4 *)(gate + at + 4), u0 = *(const float4 *)(up + at), u1 = *(const float4 *)(up + at + 4);
+        const float ga[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w}, ua[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+#pragma unroll
+        for (int k = 0; k < 8; k++) y[k] = ua[k] * lut[65536 + f2h(ga[k])];
+    }
+    xt_store8(y, sub, xq + ((int64_t)cg * nst + blockIdx.x) * XT_XB + bl * 1024, xd + ((int64_t)cg * nst + blockIdx.x) * XT_XD + bl * 64, row);
+}
+
 template <int WT, int AS, int RG, int C, int NXS, int P, int NWC, int OCC>
 int xt_launch(hipStream_t st, xt_args a, int nmat) {
     constexpr size_t ring = NXS * C * (XT_XB + 256) + NWC * ((16 * RG * xt_w<WT>::CU + 63) / 64) * 1024 + 1024, ex = (size_t)RG * (AS - 1) * C * (32 / AS) * 256, lds = ring > ex ? ring : ex;
@@ -694,6 +793,25 @@ int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, 
     const int nst = (int)(K / 128), ncg = (int)((T + 15) / 16);
     uint8_t *xq = (uint8_t *)pack, *xd = xq + (int64_t)ncg * nst * XT_XB;
     xt_pack_kernel<<<dim3((unsigned)(K / 64), (unsigned)ncg), dim3(256), 0, st>>>((const uint8_t *)x, x_stride, (int)T, nst, xq, xd);
+    return SPY_LAUNCH_RC();
+}
+// x [T][K] f32 -> NormRMS * w -> packed activations
+int spy_xgemm_norm_pack(hipStream_t st, const float *x, const float *w, float eps, int64_t T, int64_t K, void *pack) {
+    if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)pack & 15) || !spy_xgemm_pack_bytes(T, K) || (T + 15) / 16 > 65535 || K > 8192) return SPY_HIP_EINVAL;
+    const int nst = (int)(K / 128), ncg = (int)((T + 15) / 16);
+    uint8_t *xq = (uint8_t *)pack, *xd = xq + (int64_t)ncg * nst * XT_XB;
+    const dim3 grid((unsigned)(ncg * 16 / XT_NORM_WAVES));
+    const size_t lds = (size_t)XT_NORM_WAVES * (K / 4 + 64) * 4;
+    if (K <= 4096) xt_norm_pack_kernel<8><<<grid, dim3(64 * XT_NORM_WAVES), lds, st>>>(x, w, eps, (int)K, (int)T, nst, xq, xd);
+    else xt_norm_pack_kernel<16><<<grid, dim3(64 * XT_NORM_WAVES), lds, st>>>(x, w, eps, (int)K, (int)T, nst, xq, xd);
+    return SPY_LAUNCH_RC();
+}
+// gate, up [T][F] f32 -> up * silu(gate) -> packed activations; lut: the host's tables (spy_exact_luts)
+int spy_xgemm_silu_pack(hipStream_t st, const float *gate, const float *up, const float *lut, int64_t T, int64_t F, void *pack) {
+    if (((uintptr_t)gate & 15) || ((uintptr_t)up & 15) || ((uintptr_t)pack & 15) || !spy_xgemm_pack_bytes(T, F) || (T + 15) / 16 > 65535) return SPY_HIP_EINVAL;
+    const int nst = (int)(F / 128), ncg = (int)((T + 15) / 16);
+    uint8_t *xq = (uint8_t *)pack, *xd = xq + (int64_t)ncg * nst * XT_XB;
+    xt_silu_pack_kernel<<<dim3((unsigned)nst, (unsigned)ncg), dim3(256), 0, st>>>(gate, up, lut, (int)F, (int)T, nst, xq, xd);
     return SPY_LAUNCH_RC();
 }
 // nmat (1 .. 3) matrices of the same type and shape times the packed activations; resid (one matrix only): added to the result

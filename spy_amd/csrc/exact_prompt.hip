@@ -105,7 +105,8 @@ __device__ __forceinline__ void xp_dot128_pair(const uint32_t (&qa)[64], const u
     sb = tail_b + reduce(sum_b);
 }
 
-__global__ __launch_bounds__(256, 2) void xp_scores_kernel(const float *__restrict__ q, const uint16_t *__restrict__ kc, float *__restrict__ S,
+template <bool F16Q>     // q: f32 [T][H * 128] as Rope leaves it, or already rounded to fp16 and laid out [H][T][128]
+__global__ __launch_bounds__(256, 2) void xp_scores_kernel(const void *__restrict__ q, const uint16_t *__restrict__ kc, float *__restrict__ S,
                                                            int T, int H, int P, int64_t s_row) {
     __shared__ float s_tile[XP_QT][65];
     __shared__ __align__(16) uint4 s_k[64][16];                  // 64 key rows of 256 bytes
@@ -120,9 +121,17 @@ __global__ __launch_bounds__(256, 2) void xp_scores_kernel(const float *__restri
     const int kv_end = min(P + min(t0 + XP_QT - 1, T - 1) + 1, ((int)blockIdx.z + 1) * XP_KSEG);       // cached positions that some row of the tile may see, within this segment
     if ((int)blockIdx.z * XP_KSEG >= kv_end) return;
     uint32_t qa[64], qb[64];
-    {
-        const float4 *qp = (const float4 *)(q + (int64_t)min(t0 + lane, T - 1) * d + (int64_t)h * 128);
-        const float4 *qp2 = (const float4 *)(q + (int64_t)min(t0 + 64 + lane, T - 1) * d + (int64_t)h * 128);
+    if constexpr (F16Q) {
+        const uint4 *qp = (const uint4 *)((const uint16_t *)q + ((int64_t)h * T + min(t0 + lane, T - 1)) * 128), *qp2 = (const uint4 *)((const uint16_t *)q + ((int64_t)h * T + min(t0 + 64 + lane, T - 1)) * 128);
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const uint4 f = qp[i], f2 = qp2[i];
+            qa[4 * i] = f.x; qa[4 * i + 1] = f.y; qa[4 * i + 2] = f.z; qa[4 * i + 3] = f.w;
+            qb[4 * i] = f2.x; qb[4 * i + 1] = f2.y; qb[4 * i + 2] = f2.z; qb[4 * i + 3] = f2.w;
+        }
+    } else {
+        const float4 *qp = (const float4 *)((const float *)q + (int64_t)min(t0 + lane, T - 1) * d + (int64_t)h * 128);
+        const float4 *qp2 = (const float4 *)((const float *)q + (int64_t)min(t0 + 64 + lane, T - 1) * d + (int64_t)h * 128);
 #pragma unroll
         for (int i = 0; i < 32; i++) {
             const float4 f = qp[i], f2 = qp2[i];
@@ -402,17 +411,19 @@ __global__ __launch_bounds__(256, 2) void xp_pv_kernel(const uint16_t *__restric
 
 }   // namespace
 
-// q: fp32 [T][H][128] after Rope; kc: fp16 [position][H][128]; vt: fp16 [H * 128][C]; out: fp32 [T][H][128];
+// q: after Rope, fp32 [T][H][128], or (q_f16) fp16 [H][T][128]; kc: fp16 [position][H][128]; vt: fp16 [H * 128][C]; out: fp32 [T][H][128];
 // S: H * T * s_row floats and P16: H * T * s_row halves of scratch, s_row = spy_exact_prompt_attn_row(P + T)
 int64_t spy_exact_prompt_attn_row(int64_t n_kv) { return (n_kv + 127) & ~(int64_t)127; }
 
-int spy_exact_prompt_attn(hipStream_t st, const float *q, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, float *out, const float *lut,
+int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, float *out, const float *lut,
                           int T, int H, int P, int64_t C, int n_total, float scale) {
     if (T <= 0 || H <= 0 || H > 65535 || P < 0 || (int64_t)P + T > C || n_total < P + T || n_total > C || C % 32) return SPY_HIP_EINVAL;
     if ((int64_t)P + T > 1024 * XP_SM_R) return SPY_HIP_EUNSUPPORTED;      // the softmax kernel keeps a row in the registers of 256 threads
     if (((uintptr_t)q & 15) || ((uintptr_t)kc & 15) || ((uintptr_t)S & 15) || ((uintptr_t)P16 & 7) || ((uintptr_t)out & 15)) return SPY_HIP_EINVAL;
     const int64_t s_row = spy_exact_prompt_attn_row((int64_t)P + T);
-    xp_scores_kernel<<<dim3((unsigned)H, (unsigned)((T + XP_QT - 1) / XP_QT), (unsigned)((P + T + XP_KSEG - 1) / XP_KSEG)), dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row);
+    const dim3 sgrid((unsigned)H, (unsigned)((T + XP_QT - 1) / XP_QT), (unsigned)((P + T + XP_KSEG - 1) / XP_KSEG));
+    if (q_f16) xp_scores_kernel<true><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row);
+    else xp_scores_kernel<false><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row);
     if (hipGetLastError() != hipSuccess) return SPY_HIP_EINVAL;
     xp_softmax_kernel<<<dim3((unsigned)T, (unsigned)H), dim3(256), 0, st>>>(S, P16, lut, T, P, s_row, n_total, scale);
     if (hipGetLastError() != hipSuccess) return SPY_HIP_EINVAL;
@@ -439,5 +450,5 @@ extern "C" int spy_hip_prompt_attention_exact(void *stream, const float *q, cons
     if (rc) return rc;
     float *S = (float *)scratch;
     uint16_t *P16 = (uint16_t *)((uint8_t *)scratch + need / 6 * 4);
-    return spy_exact_prompt_attn((hipStream_t)stream, q, (const uint16_t *)k_cache, (const uint16_t *)v_cache, S, P16, out, lut, T, H, past, n_ctx, n_total, scale);
+    return spy_exact_prompt_attn((hipStream_t)stream, q, false, (const uint16_t *)k_cache, (const uint16_t *)v_cache, S, P16, out, lut, T, H, past, n_ctx, n_total, scale);
 }

@@ -328,24 +328,27 @@ __device__ __forceinline__ void xt_store8(const float (&y)[8], int sub, uint8_t 
     }
 }
 
-// NormRMS (non-linear.cpp:194-223) -> Mul by the norm weights -> packed activations; one wave per row.  The sum of squares is the host's
-// std::transform_reduce: groups of four, (x0^2 + x1^2) + (x2^2 + x3^2), added to one running sum.  That chain (K / 4 additions of 4.3 ns)
-// is the length of the kernel; rows past T of the last group are written as zeros.
-#define XT_NORM_WAVES 4
-template <int NV>        // K <= 512 * NV
-__global__ __launch_bounds__(64 * XT_NORM_WAVES) void xt_norm_pack_kernel(const float *__restrict__ x, const float *__restrict__ w, float eps, int K, int T, int nst,
-                                                                          uint8_t *__restrict__ xq, uint8_t *__restrict__ xd) {
-    extern __shared__ __attribute__((aligned(16))) float s_grp[];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = (int)blockIdx.x * XT_NORM_WAVES + wave;
-    const int cg = t >> 4, row = t & 15, n8 = K / 8;
-    float *g = s_grp + wave * (K / 4 + 64);
+// NormRMS (non-linear.cpp:194-223) -> Mul by the norm weights -> packed activations; one workgroup per row.  The sum of squares is the host's
+// std::transform_reduce: groups of four, (x0^2 + x1^2) + (x2^2 + x3^2), added to one running sum, which one wave walks; that chain (K / 4
+// additions of 4.3 ns) is most of the kernel.  Rows past T of the last group are written as zeros.
+template <int NV>        // K <= 2048 * NV
+__global__ __launch_bounds__(256) void xt_norm_pack_kernel(const float *__restrict__ x, const float *__restrict__ w, float eps, int K, int T, int nst,
+                                                           uint8_t *__restrict__ xq, uint8_t *__restrict__ xd) {
+    __shared__ __align__(16) float g[512 * NV + 32];
+    __shared__ float s_sum;
+    const int tid = threadIdx.x, t = blockIdx.x, cg = t >> 4, row = t & 15, n8 = K / 8;
     const float4 *xr = (const float4 *)(x + (int64_t)min(t, T - 1) * K);
-    float4 v[NV][2];
+    float4 v[NV][2], wv[NV][2];
 #pragma unroll
     for (int j = 0; j < NV; j++) {
-        const int i = min(j * 64 + lane, n8 - 1);
+        const int i = min(j * 256 + tid, n8 - 1);
         v[j][0] = xr[2 * i]; v[j][1] = xr[2 * i + 1];
-        if (j * 64 + lane < n8) {
+    }
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = min(j * 256 + tid, n8 - 1);
+        wv[j][0] = ((const float4 *)w)[2 * i]; wv[j][1] = ((const float4 *)w)[2 * i + 1];
+        if (j * 256 + tid < n8) {
 #pragma unroll
             for (int k = 0; k < 2; k++) {
                 const float4 z = v[j][k];
@@ -354,25 +357,34 @@ __global__ __launch_bounds__(64 * XT_NORM_WAVES) void xt_norm_pack_kernel(const 
             }
         }
     }
-    __builtin_amdgcn_wave_barrier();               // the other lanes of the wave read them
-    asm volatile("" ::: "memory");
-    float sum = 0.0f;
-    {   // four group sums per read, requested two reads (eight additions) ahead; K / 4 is a multiple of 64
+    __syncthreads();
+    if (tid < 64) {      // eight group sums per step, requested three steps (24 additions, about the latency of an LDS read) ahead; K / 4 is a multiple of 32
         const float4 *p = (const float4 *)g;
-        float4 a = p[0], b = p[1];
-        for (int i = 0; i < K / 16; i += 2) {
-            const float4 c = p[i + 2], e = p[i + 3];                 // up to 8 floats past the row's sums: not added
-            sum = sum + a.x; sum = sum + a.y; sum = sum + a.z; sum = sum + a.w;
-            sum = sum + b.x; sum = sum + b.y; sum = sum + b.z; sum = sum + b.w;
-            a = c; b = e;
+        float4 r[4][2];
+        float sum = 0.0f;
+        auto ld = [&](int k, int i) { r[k][0] = p[2 * i]; r[k][1] = p[2 * i + 1]; };                   // up to 24 floats past the row's sums: not added
+#pragma unroll
+        for (int k = 0; k < 3; k++) ld(k, k);
+        for (int i = 0; i < K / 32; i += 4) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                ld((k + 3) & 3, i + k + 3);
+                __builtin_amdgcn_sched_barrier(0);
+                const float4 a = r[k][0], c = r[k][1];
+                sum = sum + a.x; sum = sum + a.y; sum = sum + a.z; sum = sum + a.w;
+                sum = sum + c.x; sum = sum + c.y; sum = sum + c.z; sum = sum + c.w;
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
+        if (tid == 0) s_sum = sum;
     }
-    const float mean = sum / (float)K, scale = 1.0f / sqrtf(mean + eps);
+    __syncthreads();
+    const float mean = s_sum / (float)K, scale = 1.0f / sqrtf(mean + eps);
 #pragma unroll
     for (int j = 0; j < NV; j++) {
-        const int i = j * 64 + lane;
+        const int i = j * 256 + tid;
         if (i < n8) {                                                // n8 is a multiple of 32: the four lanes of a block stay together
-            const float4 w0 = ((const float4 *)w)[2 * i], w1 = ((const float4 *)w)[2 * i + 1], v0 = v[j][0], v1 = v[j][1];
+            const float4 w0 = wv[j][0], w1 = wv[j][1], v0 = v[j][0], v1 = v[j][1];
             float y[8] = {(v0.x * scale) * w0.x, (v0.y * scale) * w0.y, (v0.z * scale) * w0.z, (v0.w * scale) * w0.w,
                           (v1.x * scale) * w1.x, (v1.y * scale) * w1.y, (v1.z * scale) * w1.z, (v1.w * scale) * w1.w};
             if (t >= T) {
@@ -800,10 +812,8 @@ int spy_xgemm_norm_pack(hipStream_t st, const float *x, const float *w, float ep
     if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)pack & 15) || !spy_xgemm_pack_bytes(T, K) || (T + 15) / 16 > 65535 || K > 8192) return SPY_HIP_EINVAL;
     const int nst = (int)(K / 128), ncg = (int)((T + 15) / 16);
     uint8_t *xq = (uint8_t *)pack, *xd = xq + (int64_t)ncg * nst * XT_XB;
-    const dim3 grid((unsigned)(ncg * 16 / XT_NORM_WAVES));
-    const size_t lds = (size_t)XT_NORM_WAVES * (K / 4 + 64) * 4;
-    if (K <= 4096) xt_norm_pack_kernel<8><<<grid, dim3(64 * XT_NORM_WAVES), lds, st>>>(x, w, eps, (int)K, (int)T, nst, xq, xd);
-    else xt_norm_pack_kernel<16><<<grid, dim3(64 * XT_NORM_WAVES), lds, st>>>(x, w, eps, (int)K, (int)T, nst, xq, xd);
+    if (K <= 4096) xt_norm_pack_kernel<2><<<dim3((unsigned)(ncg * 16)), dim3(256), 0, st>>>(x, w, eps, (int)K, (int)T, nst, xq, xd);
+    else xt_norm_pack_kernel<4><<<dim3((unsigned)(ncg * 16)), dim3(256), 0, st>>>(x, w, eps, (int)K, (int)T, nst, xq, xd);
     return SPY_LAUNCH_RC();
 }
 // gate, up [T][F] f32 -> up * silu(gate) -> packed activations; lut: the host's tables (spy_exact_luts)

@@ -49,9 +49,9 @@ __device__ __forceinline__ float xp_fma_hi(uint32_t a, uint32_t b, float c) {
 }
 
 // One key row (in LDS, 16 x 16 bytes) against the two query rows of a lane; the row is taken in its four chunks of 32 elements
-// so that only one chunk of it is in registers at a time.  A: the first query row takes part (else its score is not needed).
-template <bool A>
-__device__ __forceinline__ void xp_dot128_pair(const uint32_t (&qa)[64], const uint32_t (&qb)[64], const uint4 *kr, float &sa, float &sb) {
+// so that only one chunk of it is in registers at a time.  A, B: the first / second query row takes part (else its score is not needed).
+template <bool A, bool B, int NB>
+__device__ __forceinline__ void xp_dot128_pair(const uint32_t (&qa)[64], const uint32_t (&qb)[NB], const uint4 *kr, float &sa, float &sb) {
     float sum_a[32], sum_b[32];
     // chunks of 32 elements while i + 32 < 128: accumulator l takes elements l, 32 + l, 64 + l
 #pragma unroll
@@ -69,8 +69,10 @@ __device__ __forceinline__ void xp_dot128_pair(const uint32_t (&qa)[64], const u
                     sum_a[l] = xp_fma_lo(kw[i], qa[qi], c == 0 ? 0.0f : sum_a[l]);
                     sum_a[l + 1] = xp_fma_hi(kw[i], qa[qi], c == 0 ? 0.0f : sum_a[l + 1]);
                 }
-                sum_b[l] = xp_fma_lo(kw[i], qb[qi], c == 0 ? 0.0f : sum_b[l]);
-                sum_b[l + 1] = xp_fma_hi(kw[i], qb[qi], c == 0 ? 0.0f : sum_b[l + 1]);
+                if (B) {
+                    sum_b[l] = xp_fma_lo(kw[i], qb[qi], c == 0 ? 0.0f : sum_b[l]);
+                    sum_b[l + 1] = xp_fma_hi(kw[i], qb[qi], c == 0 ? 0.0f : sum_b[l + 1]);
+                }
             }
         }
     }
@@ -87,8 +89,7 @@ __device__ __forceinline__ void xp_dot128_pair(const uint32_t (&qa)[64], const u
             for (int i = 0; i < 4; i++) {
                 const int qi = 48 + 4 * v + i;
                 if (A) { tail_a = xp_fma_lo(kw[i], qa[qi], tail_a); tail_a = xp_fma_hi(kw[i], qa[qi], tail_a); }
-                tail_b = xp_fma_lo(kw[i], qb[qi], tail_b);
-                tail_b = xp_fma_hi(kw[i], qb[qi], tail_b);
+                if (B) { tail_b = xp_fma_lo(kw[i], qb[qi], tail_b); tail_b = xp_fma_hi(kw[i], qb[qi], tail_b); }
             }
         }
     }
@@ -102,32 +103,34 @@ __device__ __forceinline__ void xp_dot128_pair(const uint32_t (&qa)[64], const u
         return (u0 + u1) + (u2 + u3);
     };
     if (A) sa = tail_a + reduce(sum_a);
-    sb = tail_b + reduce(sum_b);
+    if (B) sb = tail_b + reduce(sum_b);
 }
 
-template <bool F16Q>     // q: f32 [T][H * 128] as Rope leaves it, or already rounded to fp16 and laid out [H][T][128]
+// ONE: 64 query rows per workgroup, one per lane (short passes: twice the waves per SIMD, half the granularity)
+template <bool F16Q, bool ONE>     // q: f32 [T][H * 128] as Rope leaves it, or already rounded to fp16 and laid out [H][T][128]
 __global__ __launch_bounds__(256, 2) void xp_scores_kernel(const void *__restrict__ q, const uint16_t *__restrict__ kc, float *__restrict__ S,
-                                                           int T, int H, int P, int64_t s_row) {
-    __shared__ float s_tile[XP_QT][65];
+                                                           int T, int H, int P, int64_t s_row, int kseg) {
+    constexpr int QT = ONE ? 64 : XP_QT;
+    __shared__ float s_tile[QT][65];
     __shared__ __align__(16) uint4 s_k[64][16];                  // 64 key rows of 256 bytes
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // The head is the fastest-running index of the grid: consecutive workgroups go to the eight XCDs in turn, and with the query tile
     // there an XCD would get tiles k and k + 8 of 16 only -- under the causal mask 24 to 10 units of work (68 % of the compute units
     // busy over the launch).  With the head there every XCD gets the same mix of tiles, and the key rows of its heads stay in its L2.
-    const int t0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * XP_QT, h = blockIdx.x;      // the longest rows first
+    const int t0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * QT, h = blockIdx.x;      // the longest rows first
     const int64_t d = (int64_t)H * 128;
-    // the cached positions are dealt out in segments of XP_KSEG over blockIdx.z, so that the workgroups are of similar length
+    // the cached positions are dealt out in segments of kseg (a multiple of 64) over blockIdx.z, so that the workgroups are of similar length
     // (one workgroup per 128 query rows would make the longest rows the critical path of the launch)
-    const int kv_end = min(P + min(t0 + XP_QT - 1, T - 1) + 1, ((int)blockIdx.z + 1) * XP_KSEG);       // cached positions that some row of the tile may see, within this segment
-    if ((int)blockIdx.z * XP_KSEG >= kv_end) return;
-    uint32_t qa[64], qb[64];
+    const int kv_end = min(P + min(t0 + QT - 1, T - 1) + 1, ((int)blockIdx.z + 1) * kseg);       // cached positions that some row of the tile may see, within this segment
+    if ((int)blockIdx.z * kseg >= kv_end) return;
+    uint32_t qa[64], qb[ONE ? 1 : 64];
     if constexpr (F16Q) {
         const uint4 *qp = (const uint4 *)((const uint16_t *)q + ((int64_t)h * T + min(t0 + lane, T - 1)) * 128), *qp2 = (const uint4 *)((const uint16_t *)q + ((int64_t)h * T + min(t0 + 64 + lane, T - 1)) * 128);
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const uint4 f = qp[i], f2 = qp2[i];
             qa[4 * i] = f.x; qa[4 * i + 1] = f.y; qa[4 * i + 2] = f.z; qa[4 * i + 3] = f.w;
-            qb[4 * i] = f2.x; qb[4 * i + 1] = f2.y; qb[4 * i + 2] = f2.z; qb[4 * i + 3] = f2.w;
+            if constexpr (!ONE) { qb[4 * i] = f2.x; qb[4 * i + 1] = f2.y; qb[4 * i + 2] = f2.z; qb[4 * i + 3] = f2.w; }
         }
     } else {
         const float4 *qp = (const float4 *)((const float *)q + (int64_t)min(t0 + lane, T - 1) * d + (int64_t)h * 128);
@@ -137,8 +140,10 @@ __global__ __launch_bounds__(256, 2) void xp_scores_kernel(const void *__restric
             const float4 f = qp[i], f2 = qp2[i];
             qa[2 * i] = __builtin_bit_cast(uint32_t, xp_pack(f.x, f.y));
             qa[2 * i + 1] = __builtin_bit_cast(uint32_t, xp_pack(f.z, f.w));
-            qb[2 * i] = __builtin_bit_cast(uint32_t, xp_pack(f2.x, f2.y));
-            qb[2 * i + 1] = __builtin_bit_cast(uint32_t, xp_pack(f2.z, f2.w));
+            if constexpr (!ONE) {
+                qb[2 * i] = __builtin_bit_cast(uint32_t, xp_pack(f2.x, f2.y));
+                qb[2 * i + 1] = __builtin_bit_cast(uint32_t, xp_pack(f2.z, f2.w));
+            }
         }
     }
     const int kv_end_a = P + min(t0 + 63, T - 1) + 1;            // cached positions that some row of the tile's first half may see
@@ -148,7 +153,7 @@ __global__ __launch_bounds__(256, 2) void xp_scores_kernel(const void *__restric
 #define XP_FETCH_K(kv_first) do { \
         const uint4 *src_ = (const uint4 *)(kc + (int64_t)min((kv_first) + st_row, kv_end - 1) * d + (int64_t)h * 128) + st_q; \
         kst0 = src_[0]; kst1 = src_[1]; kst2 = src_[2]; kst3 = src_[3]; } while (0)
-    for (int kv0 = (int)blockIdx.z * XP_KSEG; kv0 < kv_end; kv0 += 64) {
+    for (int kv0 = (int)blockIdx.z * kseg; kv0 < kv_end; kv0 += 64) {
         // (no key tile travelling in registers during the dots: with 2 x 64 registers of q values and 2 x 32 accumulators there is
         // no room for it; the second workgroup of the compute unit covers the wait)
         XP_FETCH_K(kv0);
@@ -160,21 +165,23 @@ __global__ __launch_bounds__(256, 2) void xp_scores_kernel(const void *__restric
             const int kvl = wave * 16 + j;
             float sa = 0.0f, sb = 0.0f;
             if (kv0 + kvl < kv_end) {
-                if (first_half) xp_dot128_pair<true>(qa, qb, s_k[kvl], sa, sb);
-                else xp_dot128_pair<false>(qa, qb, s_k[kvl], sa, sb);
+                if constexpr (ONE) xp_dot128_pair<true, false, 64>(qa, qa, s_k[kvl], sa, sb);
+                else if (first_half) xp_dot128_pair<true, true, 64>(qa, qb, s_k[kvl], sa, sb);
+                else xp_dot128_pair<false, true, 64>(qa, qb, s_k[kvl], sa, sb);
             }
             s_tile[lane][kvl] = sa;
-            s_tile[64 + lane][kvl] = sb;
+            if constexpr (!ONE) s_tile[64 + lane][kvl] = sb;
         }
         __syncthreads();
         {
-            const int row = threadIdx.x >> 1, seg = threadIdx.x & 1;
+            constexpr int W = ONE ? 16 : 32;                      // scores per thread
+            const int row = threadIdx.x / (64 / W), seg = threadIdx.x % (64 / W);
             if (t0 + row < T && (row >= 64 || first_half)) {
-                float4 *out = (float4 *)(S + ((int64_t)h * T + t0 + row) * s_row + kv0 + seg * 32);
+                float4 *out = (float4 *)(S + ((int64_t)h * T + t0 + row) * s_row + kv0 + seg * W);
 #pragma unroll
-                for (int i = 0; i < 8; i++)
-                    out[i] = make_float4(s_tile[row][seg * 32 + 4 * i], s_tile[row][seg * 32 + 4 * i + 1], s_tile[row][seg * 32 + 4 * i + 2],
-                                         s_tile[row][seg * 32 + 4 * i + 3]);
+                for (int i = 0; i < W / 4; i++)
+                    out[i] = make_float4(s_tile[row][seg * W + 4 * i], s_tile[row][seg * W + 4 * i + 1], s_tile[row][seg * W + 4 * i + 2],
+                                         s_tile[row][seg * W + 4 * i + 3]);
             }
         }
         // the next tile's key rows go into s_k at the top of the loop: every wave is past its reads of s_k once it has passed the
@@ -421,9 +428,17 @@ int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint1
     if ((int64_t)P + T > 1024 * XP_SM_R) return SPY_HIP_EUNSUPPORTED;      // the softmax kernel keeps a row in the registers of 256 threads
     if (((uintptr_t)q & 15) || ((uintptr_t)kc & 15) || ((uintptr_t)S & 15) || ((uintptr_t)P16 & 7) || ((uintptr_t)out & 15)) return SPY_HIP_EINVAL;
     const int64_t s_row = spy_exact_prompt_attn_row((int64_t)P + T);
-    const dim3 sgrid((unsigned)H, (unsigned)((T + XP_QT - 1) / XP_QT), (unsigned)((P + T + XP_KSEG - 1) / XP_KSEG));
-    if (q_f16) xp_scores_kernel<true><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row);
-    else xp_scores_kernel<false><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row);
+    // segments of the cached positions: 512 long where that fills the chip, down to one key tile for short passes (77 tokens on 1000 cached ones
+    // gave 96 workgroups: 114 us; one per 64 positions and 64 query rows 29)
+    const bool one = T <= 256;
+    const int tiles = (T + (one ? 64 : XP_QT) - 1) / (one ? 64 : XP_QT);
+    int kseg = XP_KSEG;
+    while (kseg > 64 && (int64_t)H * tiles * ((P + T + kseg - 1) / kseg) < 1024) kseg >>= 1;
+    const dim3 sgrid((unsigned)H, (unsigned)tiles, (unsigned)((P + T + kseg - 1) / kseg));
+    if (q_f16 && one) xp_scores_kernel<true, true><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
+    else if (q_f16) xp_scores_kernel<true, false><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
+    else if (one) xp_scores_kernel<false, true><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
+    else xp_scores_kernel<false, false><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
     if (hipGetLastError() != hipSuccess) return SPY_HIP_EINVAL;
     xp_softmax_kernel<<<dim3((unsigned)T, (unsigned)H), dim3(256), 0, st>>>(S, P16, lut, T, P, s_row, n_total, scale);
     if (hipGetLastError() != hipSuccess) return SPY_HIP_EINVAL;

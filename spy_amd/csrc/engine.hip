@@ -349,6 +349,7 @@ static spy_hip_tensor T3s(int type, void *p, int64_t e0, int64_t e1, int64_t e2,
 
 int spy_matmul_causal(void *stream, const spy_hip_tensor *w, const spy_hip_tensor *x, const spy_hip_tensor *dst, void *scratch, size_t scratch_bytes,
                       int which, int past);                                                                                  // ops.hip
+int spy_matmul_own(void *stream, const spy_hip_tensor *w, const spy_hip_tensor *x, const spy_hip_tensor *dst, void *scratch, size_t scratch_bytes);   // ops.hip
 int spy_norm_mul_q8_launch(hipStream_t st, const float *x, int64_t x_stride, const float *w, float eps, void *y, int64_t nrow, int64_t K);   // prompt_fused.hip
 int spy_silu_mul_q8_launch(hipStream_t st, const float *gate, const float *up, void *y, int64_t nrow, int64_t F);                           // prompt_fused.hip
 int spy_rope_table_launch(hipStream_t st, float *table, int past, int T, int hd, float freq_base, float freq_scale, float mscale);       // prompt_fused.hip
@@ -536,7 +537,7 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
     const float scale = 1.0f / sqrtf((float)hd);
     auto mm = [&](const void *w, int wt, int64_t K, int64_t M, spy_hip_tensor *xin, spy_hip_tensor *out) {
         spy_hip_tensor tw = T2(wt, (void *)w, K, M);
-        return spy_hip_op_matmul(st, &tw, xin, out, scr, scr_bytes);
+        return exact ? spy_hip_op_matmul(st, &tw, xin, out, scr, scr_bytes) : spy_matmul_own(st, &tw, xin, out, scr, scr_bytes);
     };
     float *rope_tab = (float *)(B + o_rt);
     if (fuse_act) RC_TRY(spy_rope_table_launch(st, rope_tab, P, T, (int)hd, rp.freq_base, rp.freq_scale, rp.attention_factor));

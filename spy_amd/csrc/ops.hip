@@ -657,13 +657,21 @@ static size_t matmul_act_bytes(const spy_hip_tensor *w, const spy_hip_tensor *x)
     if (x->ne[0] % spy_block_size(tm) != 0) return 0;
     return (size_t)(spy_t_nrow(x) * spy_row_size(tm, x->ne[0]));
 }
+// Whether exact_gemm.hip runs a MatMul.  In the host's order: three activation rows and more (two single-row launches take less).  In this backend's own
+// order K-quants from eight rows: their sums are sub-block by sub-block as well, and the row kernels (2 us per row of a 4096 x 4096 matrix) and the
+// 128 x 128 tiles take longer at any number of rows: 4096 x 4096 Q4_K 16 rows 32 -> 12 us, 128 rows 52 -> 29, 1000 rows 128 -> 104; Q6_K 35 -> 14,
+// 69 -> 39, 195 -> 110 (at six rows of 11008 columns they are still 10 % slower). 
+static bool xgemm_rows(int wtype, int64_t T) {
+    if (spy_exact_on()) return T >= 3;
+    return (wtype == SPY_HIP_Q4_K || wtype == SPY_HIP_Q6_K) && T >= 8;
+}
 // ... plus, while the exact summation order is on, room for the fp16 copies of both operands that its prompt-sized Q4_0 / Q8_0
 // MatMul runs from (a call with less than this, but the activations' part, runs the kernel that unpacks per tile: same results)
 extern "C" size_t spy_hip_op_matmul_scratch_size(const spy_hip_tensor *w, const spy_hip_tensor *x) {
     const size_t act = matmul_act_bytes(w, x);
-    if (!act || !spy_exact_on() || x->type != SPY_HIP_F32 || mid_type(w->type, x->type) != SPY_HIP_Q8_0 || w->ne[2] != 1 || w->ne[3] != 1) return act;
-    const size_t pk = w->type == SPY_HIP_Q4_0 || w->type == SPY_HIP_Q8_0 ? spy_exact_pack_bytes(w->ne[1], w->ne[0], x->ne[1]) : 0;
-    const size_t xp = x->ne[1] >= 3 ? spy_xgemm_pack_bytes(x->ne[1], x->ne[0]) : 0;
+    if (!act || x->type != SPY_HIP_F32 || mid_type(w->type, x->type) != SPY_HIP_Q8_0 || w->ne[2] != 1 || w->ne[3] != 1) return act;
+    const size_t pk = spy_exact_on() && (w->type == SPY_HIP_Q4_0 || w->type == SPY_HIP_Q8_0) ? spy_exact_pack_bytes(w->ne[1], w->ne[0], x->ne[1]) : 0;
+    const size_t xp = xgemm_rows(w->type, x->ne[1]) ? spy_xgemm_pack_bytes(x->ne[1], x->ne[0]) : 0;
     const size_t need = pk ? ((act + 255) & ~(size_t)255) + pk : act;
     return need > xp ? need : xp;
 }
@@ -683,7 +691,12 @@ static int own_matvec(hipStream_t st, int t0, const void *w, const float *x, flo
     }
 }
 static int matmul_impl(void *stream, const spy_hip_tensor *w, const spy_hip_tensor *x, const spy_hip_tensor *dst, void *scratch, size_t scratch_bytes,
-                       int skip_past, int klimit_past);
+                       int skip_past, int klimit_past, bool own_kernels = false);
+// MatMul by the kernels of this backend's own order whatever the number of rows: the token loop's passes in that order, whose results do not depend on
+// how long a prompt is
+int spy_matmul_own(void *stream, const spy_hip_tensor *w, const spy_hip_tensor *x, const spy_hip_tensor *dst, void *scratch, size_t scratch_bytes) {
+    return matmul_impl(stream, w, x, dst, scratch, scratch_bytes, -1, -1, true);
+}
 extern "C" int spy_hip_op_matmul(void *stream, const spy_hip_tensor *w, const spy_hip_tensor *x, const spy_hip_tensor *dst,
                                  void *scratch, size_t scratch_bytes) {
     return matmul_impl(stream, w, x, dst, scratch, scratch_bytes, -1, -1);
@@ -698,7 +711,7 @@ int spy_matmul_causal(void *stream, const spy_hip_tensor *w, const spy_hip_tenso
     return matmul_impl(stream, w, x, dst, scratch, scratch_bytes, which == 0 ? past : -1, which == 1 ? past : -1);
 }
 static int matmul_impl(void *stream, const spy_hip_tensor *w, const spy_hip_tensor *x, const spy_hip_tensor *dst, void *scratch, size_t scratch_bytes,
-                       int skip_past, int klimit_past) {
+                       int skip_past, int klimit_past, bool own_kernels) {
     SPY_CHECK_ARG(w && x && dst && w->data && x->data && dst->data);
     const int t0 = w->type, t1 = x->type, tm = mid_type(t0, t1);
     if (dst->type != SPY_HIP_F32) return SPY_HIP_EUNSUPPORTED;
@@ -721,9 +734,9 @@ static int matmul_impl(void *stream, const spy_hip_tensor *w, const spy_hip_tens
                                       : own_matvec(st, t0, w->data, (const float *)x->data, (float *)dst->data, ne01, ne00);
         if (rc != SPY_HIP_EUNSUPPORTED) return rc;
     }
-    // the host's order, three rows and more (two single-row launches take less): the kernels of exact_gemm.hip where they take the matrix and
-    // the scratch buffer holds the packed activations (SPY_HIP_EXACT_TILED=u / 0, SPY_HIP_EXACT_SERIAL: tests of the other kernels)
-    if (quant && t1 == SPY_HIP_F32 && ne11 >= 3 && ne12 == 1 && ne13 == 1 && skip_past < 0 && klimit_past < 0 && spy_exact_on() && x->nb[0] == 4 && x->nb[1] % 16 == 0 &&
+    // several rows: the kernels of exact_gemm.hip where they take the matrix and the scratch buffer holds the packed activations
+    // (SPY_HIP_EXACT_TILED=u / 0, SPY_HIP_EXACT_SERIAL: tests of the other kernels)
+    if (quant && t1 == SPY_HIP_F32 && xgemm_rows(t0, ne11) && !own_kernels && ne12 == 1 && ne13 == 1 && skip_past < 0 && klimit_past < 0 && x->nb[0] == 4 && x->nb[1] % 16 == 0 &&
         ((uintptr_t)x->data & 15) == 0 && dst->nb[1] % 16 == 0 && w->nb[0] == spy_type_size(t0) && w->nb[1] == spy_row_size(t0, ne00) &&
         spy_xgemm_ok(t0, w->data, (const float *)dst->data, ne01, ne00, ne11, dst->nb[1] / 4)) {
         const char *tiled = getenv("SPY_HIP_EXACT_TILED");

@@ -151,3 +151,27 @@ def test_op_matmul_prompt_sizes(hip, oracle):
     sc2 = dev_empty(need, 0)
     call(L.spy_hip_op_matmul, None, B(tv), B(tP), B(tO), sc2.ptr, need)
     assert_close(dO.download(np.float32).reshape(O_want.shape), O_want, "KQV T=40", tol=1e-5)
+
+
+@pytest.mark.parametrize("wtype,M,K,T", [(O.Q4_K, 36, 512, 8), (O.Q4_K, 4100, 256, 130), (O.Q6_K, 36, 512, 9), (O.Q6_K, 4100, 256, 130)])
+def test_matmul_operator_takes_the_packed_activation_kernels(hip, oracle, wtype, M, K, T, monkeypatch):
+    """MatMul in this backend's own order from packed activations, with partial tiles on both sides: within fp32 rounding of the oracle."""
+    from tests.gpu_util import dev, dev_empty, call, assert_close
+    L = hip.load()
+    monkeypatch.delenv("SPY_HIP_GEMM", raising=False)
+    prev = L.spy_hip_set_exact_order(0)
+    try:
+        rng = np.random.default_rng(wtype + M + K + T)
+        w = O.quantize(oracle, (rng.standard_normal((M, K)) * 0.02).astype(np.float32), wtype)
+        x = rng.standard_normal((T, K)).astype(np.float32)
+        x[:, : K // 2] *= 3.0
+        want = O.matmul(oracle, w, wtype, M, K, x, nthread=8)
+        tw, tx, dout = hip.tensor(dev(w), wtype, [K, M]), hip.tensor(dev(x), hip.F32, [K, T]), dev_empty(T * M * 4 + 64, 0xFF)
+        need = L.spy_hip_op_matmul_scratch_size(B(tw), B(tx))
+        scratch = dev_empty(need, 0xEE)
+        call(L.spy_hip_op_matmul, None, B(tw), B(tx), B(hip.tensor(dout, hip.F32, [M, T])), scratch.ptr, need)
+        got = dout.download(np.float32)
+        assert (got[T * M:].view(np.uint32) == 0xFFFFFFFF).all(), "nothing is written beyond the outputs"
+        assert_close(got[:T * M].reshape(T, M), want, "own-order matmul type %d %dx%d T=%d" % (wtype, M, K, T), tol=1e-5)
+    finally:
+        L.spy_hip_set_exact_order(prev)

@@ -367,8 +367,10 @@ size_t spy_exact_pack_bytes(int64_t ne01, int64_t ne00, int64_t ne11);          
 size_t spy_xgemm_pack_bytes(int64_t T, int64_t K);                                                                              // exact_gemm.hip
 bool spy_xgemm_ok(int wtype, const void *w, const float *dst, int64_t M, int64_t K, int64_t T, int64_t d_row);
 int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, int64_t K, void *pack);
-int spy_xgemm_norm_pack(hipStream_t st, const float *x, const float *w, float eps, int64_t T, int64_t K, void *pack);
+int spy_xgemm_norm_pack(hipStream_t st, bool own, const float *x, const float *w, float eps, int64_t T, int64_t K, void *pack);
 int spy_xgemm_silu_pack(hipStream_t st, const float *gate, const float *up, const float *lut, int64_t T, int64_t F, void *pack);
+int spy_xgemm_own(hipStream_t st, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
+bool spy_gemm_unsplit_shape(int64_t M, int64_t T);                                                                               // gemm.hip
 int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
 int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, float *out, const float *lut,
                           int T, int H, int P, int64_t C, int n_total, float scale);                                        // exact_prompt.hip
@@ -434,7 +436,7 @@ static int forward_exact(spy_hip_llama *m, hipStream_t st, const int32_t *tokens
     { spy_hip_tensor te = T2(c.t_tok_embd, (void *)c.tok_embd, d, V); RC_TRY(spy_hip_op_get_row(st, &te, &t_ids, &t_x)); }
     for (int il = 0; il < c.n_layer; il++) {
         const spy_hip_llama_layer &L = m->layers[il];
-        RC_TRY(spy_xgemm_norm_pack(st, x, L.attn_norm, c.eps, T, d, pack));
+        RC_TRY(spy_xgemm_norm_pack(st, false, x, L.attn_norm, c.eps, T, d, pack));
         const void *w3[3] = {L.wq, L.wk, L.wv};
         float *d3[3] = {q, k, v};
         const int together = L.t_wv == L.t_wq ? 3 : 2;
@@ -445,7 +447,7 @@ static int forward_exact(spy_hip_llama *m, hipStream_t st, const int32_t *tokens
         RC_TRY(spy_exact_prompt_attn(st, q16, true, m->k_cache[il], m->v_cache[il], (float *)(B + o_S), (uint16_t *)(B + o_P), o2, m->lut, T, (int)H, P, C, n_total, scale));
         RC_TRY(spy_xgemm_pack(st, o2, 4 * d, T, d, pack));
         RC_TRY(spy_xgemm(st, L.t_wo, 1, &L.wo, &t1, d, d, T, d, x, pack));                     // KQV_linear + Add
-        RC_TRY(spy_xgemm_norm_pack(st, t1, L.ffn_norm, c.eps, T, d, pack));
+        RC_TRY(spy_xgemm_norm_pack(st, false, t1, L.ffn_norm, c.eps, T, d, pack));
         const void *w2[2] = {L.w_up, L.w_gate};
         float *d2[2] = {up, gate};
         RC_TRY(spy_xgemm(st, L.t_up, 2, w2, d2, F, d, T, F, nullptr, pack));
@@ -453,7 +455,7 @@ static int forward_exact(spy_hip_llama *m, hipStream_t st, const int32_t *tokens
         RC_TRY(spy_xgemm(st, L.t_down, 1, &L.w_down, &x, d, F, T, d, t1, pack));              // ffn_down + Add
     }
     if (head == HEAD_ALL) {
-        RC_TRY(spy_xgemm_norm_pack(st, x, c.out_norm, c.eps, T, d, pack));
+        RC_TRY(spy_xgemm_norm_pack(st, false, x, c.out_norm, c.eps, T, d, pack));
         if (spy_xgemm_ok(c.t_out, c.w_out, lg, V, d, T, V)) RC_TRY(spy_xgemm(st, c.t_out, 1, &c.w_out, &lg, V, d, T, V, nullptr, pack));
         else return SPY_HIP_EUNSUPPORTED;
         if (logits_host) HIP_TRY(hipMemcpyAsync(logits_host, lg, (size_t)V * T * 4, hipMemcpyDeviceToHost, st));
@@ -502,7 +504,11 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
         for (auto &sh : shapes) { const size_t b = spy_exact_pack_bytes(sh[0], sh[1], T); pack = b > pack ? b : pack; }
     }
     const size_t xpack = exact && T >= 2 ? spy_xgemm_pack_bytes(T, F > d ? F : d) : 0;
-    const size_t o_scr = take(std::max((act_q8 > act_f16 ? act_q8 : act_f16) + 256 + pack, xpack));
+    // own order, Q4_0 weights: where a product is large enough for gemm.hip not to split K, it runs from packed activations instead
+    // (exact_gemm.hip: same bits, tiles that fill the chip better, wq | wk | wv in one launch)
+    auto x_ok = [&](int t, const void *w, int64_t M, int64_t K) { return fuse_act && t == SPY_HIP_Q4_0 && d <= 8192 && K % 256 == 0 && spy_gemm_unsplit_shape(M, T) && spy_xgemm_ok(t, w, nullptr, M, K, T, M); };
+    const bool any_x = fuse_act && (spy_gemm_unsplit_shape(d, T) || spy_gemm_unsplit_shape(F, T));
+    const size_t o_scr = take(std::max((act_q8 > act_f16 ? act_q8 : act_f16) + 256 + pack, std::max(xpack, any_x ? spy_xgemm_pack_bytes(T, F > d ? F : d) : 0)));
     const size_t scr_bytes = off - o_scr;
     RC_TRY(ops_workspace(m, st, off));
     uint8_t *B = m->ops_buf;
@@ -544,7 +550,12 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
     for (int il = 0; il < c.n_layer; il++) {
         const spy_hip_llama_layer &L = m->layers[il];
         spy_hip_tensor t_nw = T2(SPY_HIP_F32, (void *)L.attn_norm, d, 1); t_nw.dim = 1;
-        if (fuse_act) {           // NormRMS -> Mul -> Q8_0 in one kernel, quantized once for the three MatMuls
+        if (((uintptr_t)L.attn_norm & 15) == 0 && x_ok(L.t_wq, L.wq, d, d) && x_ok(L.t_wk, L.wk, d, d) && x_ok(L.t_wv, L.wv, d, d)) {
+            const void *w3[3] = {L.wq, L.wk, L.wv};
+            float *d3[3] = {q, k, v};
+            RC_TRY(spy_xgemm_norm_pack(st, true, x, L.attn_norm, c.eps, T, d, scr));
+            RC_TRY(spy_xgemm_own(st, 3, w3, d3, d, d, T, d, nullptr, scr));
+        } else if (fuse_act) {    // NormRMS -> Mul -> Q8_0 in one kernel, quantized once for the three MatMuls
             RC_TRY(spy_norm_mul_q8_launch(st, x, 4 * d, (const float *)L.attn_norm, c.eps, scr, T, d));
             RC_TRY(spy_hip_gemm_q8_0act(st, L.t_wq, L.wq, scr, q, d, d, T, d));
             RC_TRY(spy_hip_gemm_q8_0act(st, L.t_wk, L.wk, scr, k, d, d, T, d));
@@ -603,18 +614,36 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
             RC_TRY(spy_hip_op_contiguous(st, &t_Op, &t_o2c));
         }
         }
-        RC_TRY(mm(L.wo, L.t_wo, d, d, &t_o2, &t_t1));
-        RC_TRY(spy_hip_op_binary(st, 0, &t_t1, &t_x, &t_t1));
+        if (x_ok(L.t_wo, L.wo, d, d)) {
+            RC_TRY(spy_xgemm_pack(st, o2, 4 * d, T, d, scr));
+            RC_TRY(spy_xgemm_own(st, 1, &L.wo, &t1, d, d, T, d, x, scr));
+        } else {
+            RC_TRY(mm(L.wo, L.t_wo, d, d, &t_o2, &t_t1));
+            RC_TRY(spy_hip_op_binary(st, 0, &t_t1, &t_x, &t_t1));
+        }
         t_nw.data = (void *)L.ffn_norm;
+        const bool x_down = x_ok(L.t_down, L.w_down, d, F);
         if (fuse_act) {
-            RC_TRY(spy_norm_mul_q8_launch(st, t1, 4 * d, (const float *)L.ffn_norm, c.eps, scr, T, d));
-            if (L.t_up == L.t_gate) RC_TRY(spy_gemm_q8act_pair(st, L.t_up, L.w_up, L.w_gate, scr, up, gate, F, d, T, F));   // one grid for both
-            else {
-                RC_TRY(spy_hip_gemm_q8_0act(st, L.t_up, L.w_up, scr, up, F, d, T, F));
-                RC_TRY(spy_hip_gemm_q8_0act(st, L.t_gate, L.w_gate, scr, gate, F, d, T, F));
+            if (((uintptr_t)L.ffn_norm & 15) == 0 && x_ok(L.t_up, L.w_up, F, d) && x_ok(L.t_gate, L.w_gate, F, d)) {
+                const void *w2[2] = {L.w_up, L.w_gate};
+                float *d2[2] = {up, gate};
+                RC_TRY(spy_xgemm_norm_pack(st, true, t1, L.ffn_norm, c.eps, T, d, scr));
+                RC_TRY(spy_xgemm_own(st, 2, w2, d2, F, d, T, F, nullptr, scr));
+            } else {
+                RC_TRY(spy_norm_mul_q8_launch(st, t1, 4 * d, (const float *)L.ffn_norm, c.eps, scr, T, d));
+                if (L.t_up == L.t_gate) RC_TRY(spy_gemm_q8act_pair(st, L.t_up, L.w_up, L.w_gate, scr, up, gate, F, d, T, F));   // one grid for both
+                else {
+                    RC_TRY(spy_hip_gemm_q8_0act(st, L.t_up, L.w_up, scr, up, F, d, T, F));
+                    RC_TRY(spy_hip_gemm_q8_0act(st, L.t_gate, L.w_gate, scr, gate, F, d, T, F));
+                }
             }
-            RC_TRY(spy_silu_mul_q8_launch(st, gate, up, scr, T, F));        // Silu -> Mul -> Q8_0
-            RC_TRY(spy_hip_gemm_q8_0act(st, L.t_down, L.w_down, scr, o, d, F, T, d));
+            if (x_down) {
+                RC_TRY(spy_xgemm_silu_pack(st, gate, up, nullptr, T, F, scr));
+                RC_TRY(spy_xgemm_own(st, 1, &L.w_down, &x, d, F, T, d, t1, scr));
+            } else {
+                RC_TRY(spy_silu_mul_q8_launch(st, gate, up, scr, T, F));        // Silu -> Mul -> Q8_0
+                RC_TRY(spy_hip_gemm_q8_0act(st, L.t_down, L.w_down, scr, o, d, F, T, d));
+            }
         } else {
             RC_TRY(spy_hip_op_norm_rms(st, &t_t1, &t_xn, c.eps));
             RC_TRY(spy_hip_op_binary(st, 2, &t_xn, &t_nw, &t_xn));
@@ -624,7 +653,7 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
             RC_TRY(spy_hip_op_binary(st, 2, &t_up, &t_gate, &t_par));
             RC_TRY(mm(L.w_down, L.t_down, F, d, &t_par, &t_od));
         }
-        RC_TRY(spy_hip_op_binary(st, 0, &t_t1, &t_od, &t_x));
+        if (!x_down) RC_TRY(spy_hip_op_binary(st, 0, &t_t1, &t_od, &t_x));
     }
     if (head == HEAD_ALL) {
         spy_hip_tensor t_nw = T2(SPY_HIP_F32, (void *)c.out_norm, d, 1); t_nw.dim = 1;

@@ -330,8 +330,9 @@ __device__ __forceinline__ void xt_store8(const float (&y)[8], int sub, uint8_t 
 
 // NormRMS (non-linear.cpp:194-223) -> Mul by the norm weights -> packed activations; one workgroup per row.  The sum of squares is the host's
 // std::transform_reduce: groups of four, (x0^2 + x1^2) + (x2^2 + x3^2), added to one running sum, which one wave walks; that chain (K / 4
-// additions of 4.3 ns) is most of the kernel.  Rows past T of the last group are written as zeros.
-template <int NV>        // K <= 2048 * NV
+// additions of 4.3 ns) is most of the kernel.  Rows past T of the last group are written as zeros.  OWN: the sum in this backend's own order, by the thread
+// pattern of norm_rms_kernel.
+template <int NV, bool OWN>        // K <= 2048 * NV
 __global__ __launch_bounds__(256) void xt_norm_pack_kernel(const float *__restrict__ x, const float *__restrict__ w, float eps, int K, int T, int nst,
                                                            uint8_t *__restrict__ xq, uint8_t *__restrict__ xd) {
     __shared__ __align__(16) float g[512 * NV + 32];
@@ -348,7 +349,7 @@ __global__ __launch_bounds__(256) void xt_norm_pack_kernel(const float *__restri
     for (int j = 0; j < NV; j++) {
         const int i = min(j * 256 + tid, n8 - 1);
         wv[j][0] = ((const float4 *)w)[2 * i]; wv[j][1] = ((const float4 *)w)[2 * i + 1];
-        if (j * 256 + tid < n8) {
+        if (!OWN && j * 256 + tid < n8) {
 #pragma unroll
             for (int k = 0; k < 2; k++) {
                 const float4 z = v[j][k];
@@ -357,8 +358,16 @@ __global__ __launch_bounds__(256) void xt_norm_pack_kernel(const float *__restri
             }
         }
     }
+    if (OWN) {
+        float acc = 0.0f;
+        for (int i = tid; i < K; i += 256) { const float e = ((const float *)xr)[i]; acc = fmaf(e, e, acc); }
+        acc = wave_sum(acc);
+        if ((tid & 63) == 0) g[tid >> 6] = acc;
+    }
     __syncthreads();
-    if (tid < 64) {      // eight group sums per step, requested three steps (24 additions, about the latency of an LDS read) ahead; K / 4 is a multiple of 32
+    if (OWN) {
+        if (tid == 0) s_sum = (g[0] + g[1]) + (g[2] + g[3]);
+    } else if (tid < 64) {      // eight group sums per step, requested three steps (24 additions, about the latency of an LDS read) ahead; K / 4 is a multiple of 32
         const float4 *p = (const float4 *)g;
         float4 r[4][2];
         float sum = 0.0f;
@@ -397,7 +406,8 @@ __global__ __launch_bounds__(256) void xt_norm_pack_kernel(const float *__restri
     }
 }
 
-// Silu by the host's table -> Mul (up * silu(gate)) -> packed activations (non-linear.cpp:11-14,57-77); a workgroup takes 16 rows and four blocks
+// Silu by the host's table (lut == nullptr: of this backend, v / (1 + exp(-v)) of the fp16-rounded argument) -> Mul (up * silu(gate)) -> packed
+// activations (non-linear.cpp:11-14,57-77); a workgroup takes 16 rows and four blocks
 __global__ __launch_bounds__(256) void xt_silu_pack_kernel(const float *__restrict__ gate, const float *__restrict__ up, const float *__restrict__ lut, int F, int T, int nst,
                                                            uint8_t *__restrict__ xq, uint8_t *__restrict__ xd) {
     const int tid = threadIdx.x, sub = tid & 3, bl = (tid >> 2) & 3, row = tid >> 4, b = (int)blockIdx.x * 4 + bl, cg = blockIdx.y, t = cg * 16 + row;
@@ -407,7 +417,12 @@ __global__ __launch_bounds__(256) void xt_silu_pack_kernel(const float *__restri
         const float4 g0 = *(const float4 *)(gate + at), g1 = *(const float4 *)(gate + at + 4), u0 = *(const float4 *)(up + at), u1 = *(const float4 *)(up + at + 4);
         const float ga[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w}, ua[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
 #pragma unroll
-        for (int k = 0; k < 8; k++) y[k] = ua[k] * lut[65536 + f2h(ga[k])];
+        for (int k = 0; k < 8; k++) {
+            float sl;
+            if (lut) sl = lut[65536 + f2h(ga[k])];
+            else { const float v = h2f(f2h(ga[k])); sl = v / (1.0f + expf(-v)); }
+            y[k] = ua[k] * sl;
+        }
     }
     xt_store8(y, sub, xq + ((int64_t)cg * nst + blockIdx.x) * XT_XB + bl * 1024, xd + ((int64_t)cg * nst + blockIdx.x) * XT_XD + bl * 64, row);
 }
@@ -726,6 +741,174 @@ __global__ __launch_bounds__(256, 3) void xks_kernel(xt_args a) {
         a.dst[mat][at] = a.resid ? acc + a.resid[at] : acc;
     }
 }
+// ---- Q4_0 in this backend's own order: ONE accumulator per output, acc = fma(d_w * d_x, float(block dot), acc) block after block -----
+// (the arithmetic and the bits of gemm_q8act_kernel in gemm.hip).  The block dot of a 16 x 16 tile is one v_mfma_f32_16x16x32_f16, a float and exact,
+// and the scale products of four blocks are one 16x16x4_4b as above: 24 matrix-core cycles and four fmas (16 cycles) per tile and block, where
+// the int8 form takes a 35-cycle instruction, a 32-cycle one and two vector instructions per output of a 32 x 32 tile.
+// Matrix and vector cycles of these instructions add up here (counters: both together 70 % of the time with two or three waves per SIMD), which is
+// why the cycles above are what counts; and the tiles fill the chip better than 128 x 128 ones.  Packing included, Q4_0, 4096 x 4096: 385 rows 66 -> 46 us,
+// 512 rows 68 -> 48, 600 rows 96 -> 64, 1000 rows 94 -> 75, 2048 rows 118 -> 117; 4096 x 11008: 512 rows 164 -> 112, 1000 rows 228 -> 184;
+// 22016 x 4096: 77 rows 85 -> 62, 320 rows 152 -> 131, 1000 rows 314 -> 302.
+// A wave takes RW groups of 16 weight rows and C groups of activation rows, so that an activation operand read from LDS serves RW instructions.
+// Weights: lane (q, r) reads blocks 2q and 2q + 1 of row r and chunk (contiguous over the four lanes of a row), and 4 x 4 exchanges between the
+// lane blocks (v_permlane16_swap, v_permlane32_swap) leave words q and 4 + q of every block in lane block q.
+struct xo_raw { uint32_t w[9]; };
+__device__ __forceinline__ void xo_transpose(uint32_t (&r)[4]) {
+    auto s16 = [](uint32_t &a, uint32_t &b) { auto v = __builtin_amdgcn_permlane16_swap(a, b, false, false); a = v[0]; b = v[1]; };
+    auto s32 = [](uint32_t &a, uint32_t &b) { auto v = __builtin_amdgcn_permlane32_swap(a, b, false, false); a = v[0]; b = v[1]; };
+    s16(r[0], r[1]); s16(r[2], r[3]);
+    s32(r[0], r[2]); s32(r[1], r[3]);
+}
+template <int RW, int WV, int C, int OCC>
+__global__ __launch_bounds__(64 * WV, OCC) void xo_kernel(xt_args a) {
+    constexpr int NT = 64 * WV, ROWS = 16 * RW * WV, NXI = C * 256 / NT, C2 = (C + 1) / 2, XB = C * XT_XB + C2 * 1024, NDW = 9, CB = xt_w<SPY_HIP_Q4_0>::CB;
+    static_assert(NXI * NT == C * 256 && WV >= C2, "one request per thread and group, one wave per two groups' records");
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, r = lane & 15;
+    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS, cg0 = (int)blockIdx.y * C;
+    const int nst = a.nst, ncg = a.ncg, M = a.M;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
+    const uint8_t *bx[NXI], *bd;
+#pragma unroll
+    for (int i = 0; i < NXI; i++) bx[i] = a.xq + (int64_t)min(cg0 + (i * NT + wave * 64) / 256, ncg - 1) * nst * XT_XB + (i * NT + wave * 64) % 256 * 16;
+    const int dc0 = min(cg0 + 2 * min(wave, C2 - 1), ncg - 1), dc1 = min(dc0 + 1, ncg - 1);
+    bd = a.xd + (int64_t)dc0 * nst * XT_XD;
+    const uint32_t l16 = lane * 16, ld = (lane & 31) * 16 + (lane >> 5) * (uint32_t)((dc1 - dc0) * nst * XT_XD);
+    const uint32_t ldsx = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024), ldsd = __builtin_amdgcn_readfirstlane(lds0 + C * XT_XB + min(wave, C2 - 1) * 1024);
+    int is = 0;
+    auto issue_x = [&]() {
+        const uint32_t o = (is & 1) * XB;
+        const int adv = is + 1 < nst ? 1 : 0;
+#pragma unroll
+        for (int i = 0; i < NXI; i++) { xt_dma16(bx[i], l16, ldsx + o + i * NT * 16); bx[i] += adv * XT_XB; }
+        xt_dma16(bd, ld, ldsd + o);
+        bd += adv * XT_XD;
+        is++;
+    };
+    const uint8_t *wr[RW];
+#pragma unroll
+    for (int w = 0; w < RW; w++) wr[w] = a.w[mat] + (int64_t)min(m0 + (wave * RW + w) * 16 + r, M - 1) * a.w_row + q * (NDW * 4);
+    auto load_w = [&](xo_raw (&t)[RW], int chunk) {
+#pragma unroll
+        for (int w = 0; w < RW; w++) __builtin_memcpy(t[w].w, __builtin_assume_aligned(wr[w] + (int64_t)chunk * CB, 4), NDW * 4);
+    };
+    xo_raw cur[RW];
+    load_w(cur, 0);
+    issue_x();
+    float acc[RW][C][4];
+#pragma unroll
+    for (int w = 0; w < RW; w++)
+#pragma unroll
+        for (int c = 0; c < C; c++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) acc[w][c][v] = 0.0f;
+    uint32_t wd[RW][2][4], dd[RW];                 // [row group][even, odd blocks][block of that kind]; the lane's two scales
+    auto spread = [&]() {
+#pragma unroll
+        for (int w = 0; w < RW; w++) {
+            const uint32_t *v = cur[w].w;
+            dd[w] = (v[0] & 0xFFFFu) | (v[4] & 0xFFFF0000u);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                wd[w][0][k] = __builtin_amdgcn_alignbit(v[k + 1], v[k], 16);
+                wd[w][1][k] = v[5 + k];
+            }
+            xo_transpose(wd[w][0]);
+            xo_transpose(wd[w][1]);
+        }
+    };
+    const uint32_t c64 = 0x64006400u;
+    const xk_v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto compute = [&](int s, auto par_c) {
+        constexpr int par = decltype(par_c)::value;
+        const uint8_t *sx = smem + (s & 1) * XB + (q >> 1) * 256 + r * 16 + (q & 1) * 8, *sd = smem + (s & 1) * XB + C * XT_XB + lane * 4;
+        uint4 w[RW][4];                            // operands of the stage's four blocks: words q and 4 + q, elements 0, 2, 1, 3 each
+        uint32_t dw[RW];
+#pragma unroll
+        for (int g = 0; g < RW; g++) {
+            // lane (kb, r): the scale of block 4 par + kb, which lane block 2 par + kb / 2 holds
+            const uint32_t d2 = (uint32_t)__builtin_amdgcn_ds_bpermute(((2 * par + (q >> 1)) * 16 + r) * 4, (int)dd[g]);
+            dw[g] = (q & 1) ? d2 >> 16 : d2 & 0xFFFFu;
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const uint32_t v = wd[g][b & 1][2 * par + (b >> 1)], u = v >> 8;
+                w[g][b] = make_uint4(xt_sub(xt_and_or(v, 0x000F000Fu, c64), 0x64086408u), xt_sub(xt_and_or(u, 0x000F000Fu, c64), 0x64086408u),
+                                     xk_pk_fma(xt_and_or(v, 0x00F000F0u, c64), 0x2C002C00u, 0xD480D480u), xk_pk_fma(xt_and_or(u, 0x00F000F0u, c64), 0x2C002C00u, 0xD480D480u));   // (1024 + 16 n) / 16 - 72
+            }
+        }
+        constexpr int NJ = 4 * C;                  // steps (activation group, block)
+        uint4 xv[3];
+        uint32_t dx[2];
+        xk_v4f p[2][RW];
+        xt_v16f D[RW];
+        auto rd = [&](int j) {
+            const uint8_t *o = sx + (j >> 2) * XT_XB + (j & 3) * 1024;
+            const uint2 l = *(const uint2 *)o, h = *(const uint2 *)(o + 512);
+            xv[j % 3] = make_uint4(l.x, l.y, h.x, h.y);
+        };
+        dx[0] = *(const uint32_t *)sd;
+        rd(0);
+        rd(1);
+#pragma unroll
+        for (int g = 0; g < RW; g++) p[0][g] = xk_mfma(w[g][0], xv[0], zero);
+#pragma unroll
+        for (int g = 0; g < RW; g++) D[g] = xt_mfma(dw[g], 0u, dx[0], 0u);
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const int c = j >> 2, b = j & 3;
+            if (j + 2 < NJ) rd(j + 2);
+            if (b == 1 && c + 1 < C) dx[(c + 1) & 1] = *(const uint32_t *)(sd + (c + 1) * XT_XD);
+            // one matrix instruction, then the four fmas that run beside it
+#pragma unroll
+            for (int g = 0; g < RW; g++) {
+                if (j + 1 < NJ) p[(j + 1) & 1][g] = xk_mfma(w[g][(j + 1) & 3], xv[(j + 1) % 3], zero);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[g][c][v] = fmaf(D[g][4 * b + v], p[j & 1][g][v], acc[g][c][v]);
+                if (b == 3 && c + 1 < C) D[g] = xt_mfma(dw[g], 0u, dx[(c + 1) & 1], 0u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    auto ready = [&]() {
+        xt_wait_vm<0>();
+        __builtin_amdgcn_s_barrier();
+    };
+    for (int s = 0; s < nst; s += 2) {
+        ready();
+        spread();                                  // the compiler's own wait for the chunk stands here, where nothing is on its way
+        load_w(cur, min(s / 2 + 1, nst / 2 - 1));
+        issue_x();
+        compute(s, std::integral_constant<int, 0>{});
+        ready();
+        issue_x();
+        compute(s + 1, std::integral_constant<int, 1>{});
+    }
+    xt_wait_vm<0>();
+    float *dst = a.dst[mat];
+#pragma unroll
+    for (int g = 0; g < RW; g++) {
+        const int row = m0 + (wave * RW + g) * 16 + 4 * q;
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            const int t = (cg0 + c) * 16 + r;
+            if (t < a.T && row + 3 < M) {
+                const int64_t at = (int64_t)t * a.d_row + row;
+                float4 o = make_float4(acc[g][c][0], acc[g][c][1], acc[g][c][2], acc[g][c][3]);
+                if (a.resid) { const float4 z = *(const float4 *)(a.resid + at); o.x += z.x; o.y += z.y; o.z += z.z; o.w += z.w; }
+                *(float4 *)(dst + at) = o;
+            }
+        }
+    }
+}
+template <int RW, int WV, int C, int OCC>
+int xo_launch(hipStream_t st, xt_args a, int nmat) {
+    constexpr size_t lds = 2 * (C * XT_XB + (C + 1) / 2 * 1024);
+    if (lds > 64 * 1024) { const int rc = spy_raise_lds_limit((const void *)xo_kernel<RW, WV, C, OCC>, lds); if (rc) return rc; }
+    a.tiles = (a.M + 16 * RW * WV - 1) / (16 * RW * WV);
+    xo_kernel<RW, WV, C, OCC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * WV), lds, st>>>(a);
+    return SPY_LAUNCH_RC();
+}
 template <int WT, int RG, int C, int OCC>
 int xk_launch(hipStream_t st, xt_args a, int nmat) {
     constexpr size_t lds = 2 * (C * XT_XB + (C + 1) / 2 * 1024) + RG * 1024;
@@ -787,6 +970,16 @@ int xk_dispatch(hipStream_t st, const xt_args &a, int nmat) {
     }
 }
 
+int xo_dispatch(hipStream_t st, const xt_args &a, int nmat) {
+    // as in xt_dispatch: measured with one workgroup per CU and with the chip full
+    static const xt_cost c4[3] = {{64, 4, 290, 155}, {128, 4, 400, 275}, {128, 8, 600, 490}};
+    switch (xt_pick(a, nmat, c4, 3)) {
+    case 0: return xo_launch<1, 4, 4, 3>(st, a, nmat);
+    case 1: return xo_launch<2, 4, 4, 3>(st, a, nmat);
+    default: return xo_launch<2, 4, 8, 2>(st, a, nmat);
+    }
+}
+
 }   // namespace
 
 // ---- what exact_order.hip and the engine call -----------------------------------------------------------------------------------------
@@ -807,16 +1000,19 @@ int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, 
     xt_pack_kernel<<<dim3((unsigned)(K / 64), (unsigned)ncg), dim3(256), 0, st>>>((const uint8_t *)x, x_stride, (int)T, nst, xq, xd);
     return SPY_LAUNCH_RC();
 }
-// x [T][K] f32 -> NormRMS * w -> packed activations
-int spy_xgemm_norm_pack(hipStream_t st, const float *x, const float *w, float eps, int64_t T, int64_t K, void *pack) {
+// x [T][K] f32 -> NormRMS * w -> packed activations; own: sum of squares in this backend's own order
+int spy_xgemm_norm_pack(hipStream_t st, bool own, const float *x, const float *w, float eps, int64_t T, int64_t K, void *pack) {
     if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)pack & 15) || !spy_xgemm_pack_bytes(T, K) || (T + 15) / 16 > 65535 || K > 8192) return SPY_HIP_EINVAL;
     const int nst = (int)(K / 128), ncg = (int)((T + 15) / 16);
     uint8_t *xq = (uint8_t *)pack, *xd = xq + (int64_t)ncg * nst * XT_XB;
-    if (K <= 4096) xt_norm_pack_kernel<2><<<dim3((unsigned)(ncg * 16)), dim3(256), 0, st>>>(x, w, eps, (int)K, (int)T, nst, xq, xd);
-    else xt_norm_pack_kernel<4><<<dim3((unsigned)(ncg * 16)), dim3(256), 0, st>>>(x, w, eps, (int)K, (int)T, nst, xq, xd);
+    const dim3 grid((unsigned)(ncg * 16));
+    if (own && K <= 4096) xt_norm_pack_kernel<2, true><<<grid, dim3(256), 0, st>>>(x, w, eps, (int)K, (int)T, nst, xq, xd);
+    else if (own) xt_norm_pack_kernel<4, true><<<grid, dim3(256), 0, st>>>(x, w, eps, (int)K, (int)T, nst, xq, xd);
+    else if (K <= 4096) xt_norm_pack_kernel<2, false><<<grid, dim3(256), 0, st>>>(x, w, eps, (int)K, (int)T, nst, xq, xd);
+    else xt_norm_pack_kernel<4, false><<<grid, dim3(256), 0, st>>>(x, w, eps, (int)K, (int)T, nst, xq, xd);
     return SPY_LAUNCH_RC();
 }
-// gate, up [T][F] f32 -> up * silu(gate) -> packed activations; lut: the host's tables (spy_exact_luts)
+// gate, up [T][F] f32 -> up * silu(gate) -> packed activations; lut: the host's tables (spy_exact_luts), or null
 int spy_xgemm_silu_pack(hipStream_t st, const float *gate, const float *up, const float *lut, int64_t T, int64_t F, void *pack) {
     if (((uintptr_t)gate & 15) || ((uintptr_t)up & 15) || ((uintptr_t)pack & 15) || !spy_xgemm_pack_bytes(T, F) || (T + 15) / 16 > 65535) return SPY_HIP_EINVAL;
     const int nst = (int)(F / 128), ncg = (int)((T + 15) / 16);
@@ -824,10 +1020,9 @@ int spy_xgemm_silu_pack(hipStream_t st, const float *gate, const float *up, cons
     xt_silu_pack_kernel<<<dim3((unsigned)nst, (unsigned)ncg), dim3(256), 0, st>>>(gate, up, lut, (int)F, (int)T, nst, xq, xd);
     return SPY_LAUNCH_RC();
 }
-// nmat (1 .. 3) matrices of the same type and shape times the packed activations; resid (one matrix only): added to the result
-int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack) {
+static int xt_fill(xt_args &a, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack) {
     if (nmat < 1 || nmat > 3 || (resid && nmat != 1) || ((uintptr_t)resid & 15) || ((uintptr_t)pack & 15)) return SPY_HIP_EINVAL;
-    xt_args a = {};
+    a = {};
     for (int i = 0; i < nmat; i++) {
         if (!spy_xgemm_ok(wtype, w[i], dst[i], M, K, T, d_row)) return SPY_HIP_EINVAL;
         a.w[i] = (const uint8_t *)w[i];
@@ -836,10 +1031,23 @@ int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *
     a.resid = resid; a.w_row = spy_row_size(wtype, K); a.d_row = d_row;
     a.M = (int)M; a.nst = (int)(K / 128); a.ncg = (int)((T + 15) / 16); a.T = (int)T;
     a.xq = (const uint8_t *)pack; a.xd = a.xq + (int64_t)a.ncg * a.nst * XT_XB;
+    return 0;
+}
+// nmat (1 .. 3) matrices of the same type and shape times the packed activations; resid (one matrix only): added to the result
+int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack) {
+    xt_args a;
+    const int rc = xt_fill(a, wtype, nmat, w, dst, M, K, T, d_row, resid, pack);
+    if (rc) return rc;
     switch (wtype) {
     case SPY_HIP_Q4_0: return xt_dispatch<SPY_HIP_Q4_0>(st, a, nmat);
     case SPY_HIP_Q8_0: return xt_dispatch<SPY_HIP_Q8_0>(st, a, nmat);
     case SPY_HIP_Q4_K: return xk_dispatch<SPY_HIP_Q4_K>(st, a, nmat);
     default: return xk_dispatch<SPY_HIP_Q6_K>(st, a, nmat);
     }
+}
+// the same in this backend's own order; Q4_0 (Q8_0 unpacks more per block: 3 % slower than the tile kernel of gemm.hip at 22016 rows)
+int spy_xgemm_own(hipStream_t st, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack) {
+    xt_args a;
+    const int rc = xt_fill(a, SPY_HIP_Q4_0, nmat, w, dst, M, K, T, d_row, resid, pack);
+    return rc ? rc : xo_dispatch(st, a, nmat);
 }

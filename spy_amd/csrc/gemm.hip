@@ -30,6 +30,7 @@ typedef int v2i __attribute__((ext_vector_type(2)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 #define GEMM_TILE 128
+#define GEMM_SKINNY_WANT 512      // workgroups of the 32-row kernel: two per compute unit
 #define GEMM_SKINNY_MAX_TILES 160 // the 32-row kernel is used up to 64 activation rows and wherever the 128 x 128 tiling would give at most this many workgroups (measured crossover)
 #define GEMM_KQ_SMALL_MAX_TILES 768 // Q4_K / Q6_K: the 64 x 64 tiling is used where it gives at most this many workgroups (3 per CU: all resident at once)
 #define GEMM_ROWB 80             // bytes per LDS row: 64 payload + 16 pad
@@ -388,7 +389,7 @@ static int launch_gemm_skinny(hipStream_t st, const void *w, const void *xq, flo
     // Token sub-tiles per workgroup (the other waves split K): as many as still leave two workgroups per compute unit.  A wave
     // advances one chunk of K per memory round trip, so with few workgroups (4096 rows x 128 tokens: 128) the launch is a chain
     // of K / 256 round trips on half of the compute units; splitting K four ways instead gives 512 workgroups a quarter as long.
-    const int64_t rows = (M + 31) / 32, want = 512;
+    const int64_t rows = (M + 31) / 32, want = GEMM_SKINNY_WANT;
     if (T <= 32) return launch_gemm_skinny_ntw<WT, 1>(st, w, xq, dst, M, K, T, dst_stride);
     if (T > 64 && rows * ((T + 127) / 128) >= want) return launch_gemm_skinny_ntw<WT, 4>(st, w, xq, dst, M, K, T, dst_stride);
     if (T <= 64 || rows * ((T + 63) / 64) >= want) return launch_gemm_skinny_ntw<WT, 2>(st, w, xq, dst, M, K, T, dst_stride);
@@ -653,6 +654,11 @@ extern "C" int spy_hip_gemm_q8_0act(void *stream, int wtype, const void *w_dev, 
     return SPY_LAUNCH_RC();
 }
 
+// Shapes at which spy_hip_gemm_q8_0act adds every output's blocks in one sequence, without slices of K (the tile kernel, or four token sub-tiles per
+// workgroup of the 32-row kernel): the own-order kernel of exact_gemm.hip gives the same bits there
+bool spy_gemm_unsplit_shape(int64_t M, int64_t T) {
+    return T > 64 && (M + 31) / 32 * ((T + 127) / 128) >= GEMM_SKINNY_WANT && !getenv("SPY_HIP_GEMM");
+}
 // Two weight matrices of the same type and shape against the same activations (gate and up of a layer): one grid
 // where the 128 x 128 tile kernel applies, else two launches.  Same results as two calls of spy_hip_gemm_q8_0act.
 int spy_gemm_q8act_pair(hipStream_t st, int wtype, const void *w1, const void *w2, const void *xq, float *dst1, float *dst2,

@@ -23,6 +23,7 @@ size_t spy_exact_pack_bytes(int64_t ne01, int64_t ne00, int64_t ne11);
 size_t spy_xgemm_pack_bytes(int64_t T, int64_t K);
 bool spy_xgemm_ok(int wtype, const void *w, const float *dst, int64_t M, int64_t K, int64_t T, int64_t d_row);
 int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, int64_t K, void *pack);
+int spy_xgemm_own(hipStream_t st, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
 int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
 
 struct tdesc {              // a tensor as the kernels see it
@@ -660,10 +661,12 @@ static size_t matmul_act_bytes(const spy_hip_tensor *w, const spy_hip_tensor *x)
 // Whether exact_gemm.hip runs a MatMul.  In the host's order: three activation rows and more (two single-row launches take less).  In this backend's own
 // order K-quants from eight rows: their sums are sub-block by sub-block as well, and the row kernels (2 us per row of a 4096 x 4096 matrix) and the
 // 128 x 128 tiles take longer at any number of rows: 4096 x 4096 Q4_K 16 rows 32 -> 12 us, 128 rows 52 -> 29, 1000 rows 128 -> 104; Q6_K 35 -> 14,
-// 69 -> 39, 195 -> 110 (at six rows of 11008 columns they are still 10 % slower). 
-static bool xgemm_rows(int wtype, int64_t T) {
+// 69 -> 39, 195 -> 110 (at six rows of 11008 columns they are still 10 % slower).  Q4_0 in the own order where the kernels of gemm.hip would not
+// split K (more than 64 rows and enough tiles), with the same bits.
+bool spy_gemm_unsplit_shape(int64_t M, int64_t T);                 // gemm.hip
+static bool xgemm_rows(int wtype, int64_t M, int64_t T) {
     if (spy_exact_on()) return T >= 3;
-    return (wtype == SPY_HIP_Q4_K || wtype == SPY_HIP_Q6_K) && T >= 8;
+    return wtype == SPY_HIP_Q4_K || wtype == SPY_HIP_Q6_K ? T >= 8 : wtype == SPY_HIP_Q4_0 && spy_gemm_unsplit_shape(M, T);
 }
 // ... plus, while the exact summation order is on, room for the fp16 copies of both operands that its prompt-sized Q4_0 / Q8_0
 // MatMul runs from (a call with less than this, but the activations' part, runs the kernel that unpacks per tile: same results)
@@ -671,7 +674,7 @@ extern "C" size_t spy_hip_op_matmul_scratch_size(const spy_hip_tensor *w, const 
     const size_t act = matmul_act_bytes(w, x);
     if (!act || x->type != SPY_HIP_F32 || mid_type(w->type, x->type) != SPY_HIP_Q8_0 || w->ne[2] != 1 || w->ne[3] != 1) return act;
     const size_t pk = spy_exact_on() && (w->type == SPY_HIP_Q4_0 || w->type == SPY_HIP_Q8_0) ? spy_exact_pack_bytes(w->ne[1], w->ne[0], x->ne[1]) : 0;
-    const size_t xp = xgemm_rows(w->type, x->ne[1]) ? spy_xgemm_pack_bytes(x->ne[1], x->ne[0]) : 0;
+    const size_t xp = xgemm_rows(w->type, w->ne[1], x->ne[1]) ? spy_xgemm_pack_bytes(x->ne[1], x->ne[0]) : 0;
     const size_t need = pk ? ((act + 255) & ~(size_t)255) + pk : act;
     return need > xp ? need : xp;
 }
@@ -736,7 +739,7 @@ static int matmul_impl(void *stream, const spy_hip_tensor *w, const spy_hip_tens
     }
     // several rows: the kernels of exact_gemm.hip where they take the matrix and the scratch buffer holds the packed activations
     // (SPY_HIP_EXACT_TILED=u / 0, SPY_HIP_EXACT_SERIAL: tests of the other kernels)
-    if (quant && t1 == SPY_HIP_F32 && xgemm_rows(t0, ne11) && !own_kernels && ne12 == 1 && ne13 == 1 && skip_past < 0 && klimit_past < 0 && x->nb[0] == 4 && x->nb[1] % 16 == 0 &&
+    if (quant && t1 == SPY_HIP_F32 && xgemm_rows(t0, ne01, ne11) && !own_kernels && ne12 == 1 && ne13 == 1 && skip_past < 0 && klimit_past < 0 && x->nb[0] == 4 && x->nb[1] % 16 == 0 &&
         ((uintptr_t)x->data & 15) == 0 && dst->nb[1] % 16 == 0 && w->nb[0] == spy_type_size(t0) && w->nb[1] == spy_row_size(t0, ne00) &&
         spy_xgemm_ok(t0, w->data, (const float *)dst->data, ne01, ne00, ne11, dst->nb[1] / 4)) {
         const char *tiled = getenv("SPY_HIP_EXACT_TILED");
@@ -745,6 +748,7 @@ static int matmul_impl(void *stream, const spy_hip_tensor *w, const spy_hip_tens
             const void *wp = w->data;
             float *dp = (float *)dst->data;
             const int rc = spy_xgemm_pack(st, (const float *)x->data, x->nb[1], ne11, ne00, scratch);
+            if (!rc && !spy_exact_on() && t0 == SPY_HIP_Q4_0) return spy_xgemm_own(st, 1, &wp, &dp, ne01, ne00, ne11, dst->nb[1] / 4, nullptr, scratch);
             return rc ? rc : spy_xgemm(st, t0, 1, &wp, &dp, ne01, ne00, ne11, dst->nb[1] / 4, nullptr, scratch);
         }
     }

@@ -153,9 +153,11 @@ def test_op_matmul_prompt_sizes(hip, oracle):
     assert_close(dO.download(np.float32).reshape(O_want.shape), O_want, "KQV T=40", tol=1e-5)
 
 
-@pytest.mark.parametrize("wtype,M,K,T", [(O.Q4_K, 36, 512, 8), (O.Q4_K, 4100, 256, 130), (O.Q6_K, 36, 512, 9), (O.Q6_K, 4100, 256, 130)])
+@pytest.mark.parametrize("wtype,M,K,T", [(O.Q4_0, 16356, 256, 65), (O.Q4_0, 8164, 512, 129), (O.Q4_0, 4068, 768, 400), (O.Q4_0, 2020, 256, 1025), (O.Q4_0, 11008, 4096, 130),
+                                         (O.Q4_K, 36, 512, 8), (O.Q4_K, 4100, 256, 130), (O.Q6_K, 36, 512, 9), (O.Q6_K, 4100, 256, 130)])
 def test_matmul_operator_takes_the_packed_activation_kernels(hip, oracle, wtype, M, K, T, monkeypatch):
-    """MatMul in this backend's own order from packed activations, with partial tiles on both sides: within fp32 rounding of the oracle."""
+    """MatMul in this backend's own order from packed activations, with partial tiles on both sides: within fp32 rounding of the oracle,
+    and for Q4_0 the bits of the tile kernel, which adds an output's blocks in the same sequence."""
     from tests.gpu_util import dev, dev_empty, call, assert_close
     L = hip.load()
     monkeypatch.delenv("SPY_HIP_GEMM", raising=False)
@@ -173,5 +175,32 @@ def test_matmul_operator_takes_the_packed_activation_kernels(hip, oracle, wtype,
         got = dout.download(np.float32)
         assert (got[T * M:].view(np.uint32) == 0xFFFFFFFF).all(), "nothing is written beyond the outputs"
         assert_close(got[:T * M].reshape(T, M), want, "own-order matmul type %d %dx%d T=%d" % (wtype, M, K, T), tol=1e-5)
+        if wtype == O.Q4_0:
+            monkeypatch.setenv("SPY_HIP_GEMM", "tile")
+            call(L.spy_hip_op_matmul, None, B(tw), B(tx), B(hip.tensor(dout, hip.F32, [M, T])), scratch.ptr, need)
+            assert np.array_equal(dout.download(np.float32).view(np.uint32), got.view(np.uint32)), "the same bits as the tile kernel"
     finally:
         L.spy_hip_set_exact_order(prev)
+
+
+@pytest.mark.parametrize("n_prompt", [129, 400])
+def test_own_order_prompt_from_packed_activations(hip, n_prompt, monkeypatch):
+    """One layer of the 7B shape in this backend's own order: norm, activation and residual steps around the packed-activation MatMuls (from 129 tokens
+    gate | up, from 385 all of them) give the bits of the separate steps around the tile kernel."""
+    from spy_amd import model as M
+    cfg = M.Config.llama2_7b(n_ctx=512, wtype=O.Q4_0)
+    cfg.n_layer = 1
+    tensors = M.synth_model(cfg, seed=8)
+    prompt = np.random.default_rng(1).integers(0, cfg.n_vocab, n_prompt).astype(np.int32)
+    got = {}
+    for forced in (None, "tile"):
+        if forced: monkeypatch.setenv("SPY_HIP_GEMM", forced)
+        else: monkeypatch.delenv("SPY_HIP_GEMM", raising=False)
+        eng = M.Engine(cfg, tensors)
+        eng.set_order(0)
+        got[forced] = eng.forward_last(prompt, 0)
+        eng.close()
+    if n_prompt > 384:
+        assert np.array_equal(got[None].view(np.uint32), got["tile"].view(np.uint32))
+    else:                       # q, k, v, wo and down in slices of K without the switch
+        assert np.linalg.norm(got[None] - got["tile"]) <= 3e-2 * np.linalg.norm(got["tile"])

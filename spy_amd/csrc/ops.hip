@@ -54,22 +54,37 @@ static unsigned grid_for(int64_t n, int per) { return (unsigned)((n + per - 1) /
 // ---------------------------------------------------------------------------------------------
 // NormRMS (non-linear.cpp:194-223): y = x * (1 / sqrt(sum(x^2)/n + eps)); one workgroup per row.
 // ---------------------------------------------------------------------------------------------
+// Thread t adds elements t, t + 256, ... in this order.  ROW: rows of up to 4096 elements stay in registers between the two passes, all of their loads
+// on the way together (a single row of 4096 is one memory latency: 7.8 -> 3.4 us; the loop loads an element per latency, twice).
+template <bool ROW>
 __global__ __launch_bounds__(256) void norm_rms_kernel(tdesc x, tdesc y, float eps) {
     __shared__ float s_part[4];
     const int64_t r = blockIdx.x;
     const int64_t ne0 = y.ne[0], ne1 = y.ne[1], ne2 = y.ne[2];
-    const int64_t i3 = r / (ne1 * ne2), i2 = r % (ne1 * ne2) / ne1, i1 = r % ne1;
+    int64_t i1 = r, i2 = 0, i3 = 0;
+    if (r >= ne1) { i3 = r / (ne1 * ne2); i2 = r % (ne1 * ne2) / ne1; i1 = r % ne1; }
     const float *s = (const float *)at(x, 0, i1, i2, i3);
     float *d = (float *)at(y, 0, i1, i2, i3);
     float acc = 0.0f;
-    for (int64_t i = threadIdx.x; i < ne0; i += 256) { const float v = s[i]; acc = fmaf(v, v, acc); }
+    [[maybe_unused]] float v[16];
+    if constexpr (ROW) {
+#pragma unroll
+        for (int j = 0; j < 16; j++) v[j] = s[min((int)threadIdx.x + 256 * j, (int)ne0 - 1)];
+#pragma unroll
+        for (int j = 0; j < 16; j++) if ((int)threadIdx.x + 256 * j < (int)ne0) acc = fmaf(v[j], v[j], acc);
+    } else
+        for (int64_t i = threadIdx.x; i < ne0; i += 256) { const float e = s[i]; acc = fmaf(e, e, acc); }
     acc = wave_sum(acc);
     if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = acc;
     __syncthreads();
     const float sum = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
     const float mean = sum / (float)ne0;
     const float scale = 1.0f / sqrtf(mean + eps);
-    for (int64_t i = threadIdx.x; i < ne0; i += 256) d[i] = s[i] * scale;
+    if constexpr (ROW) {
+#pragma unroll
+        for (int j = 0; j < 16; j++) if ((int)threadIdx.x + 256 * j < (int)ne0) d[threadIdx.x + 256 * j] = v[j] * scale;
+    } else
+        for (int64_t i = threadIdx.x; i < ne0; i += 256) d[i] = s[i] * scale;
 }
 
 extern "C" int spy_hip_op_norm_rms(void *stream, const spy_hip_tensor *x, const spy_hip_tensor *dst, float eps) {
@@ -79,7 +94,8 @@ extern "C" int spy_hip_op_norm_rms(void *stream, const spy_hip_tensor *x, const 
     const int64_t nrow = spy_t_nrow(dst);
     CHECK_GRID(nrow, 1);
     if (spy_exact_on()) return spy_exact_norm_rms((hipStream_t)stream, x, dst, eps);
-    norm_rms_kernel<<<dim3((unsigned)nrow), dim3(256), 0, (hipStream_t)stream>>>(mk(x), mk(dst), eps);
+    if (dst->ne[0] <= 4096) norm_rms_kernel<true><<<dim3((unsigned)nrow), dim3(256), 0, (hipStream_t)stream>>>(mk(x), mk(dst), eps);
+    else norm_rms_kernel<false><<<dim3((unsigned)nrow), dim3(256), 0, (hipStream_t)stream>>>(mk(x), mk(dst), eps);
     return SPY_LAUNCH_RC();
 }
 
@@ -273,7 +289,7 @@ __global__ __launch_bounds__(256) void softmax_kernel(tdesc x, tdesc mask, bool 
 // The same arithmetic with the row kept in LDS between the passes (one read of the scores, one write of the
 // probabilities) for rows of up to SOFTMAX_LDS_ROW elements; the additions of the sum happen in the same order
 // as above (thread stride 256, then the same tree), so both kernels give the same bits.  Masked elements
-// (mask = -inf, scale > 0) are not read: (s - inf) * scale = -inf whatever the finite score.  F16OUT stores the
+// (mask = -inf, scale > 0) do not matter: (s - inf) * scale = -inf whatever the finite score.  F16OUT stores the
 // probabilities rounded to fp16, which is what the KQV product does to them first anyway (mat.cpp:37).
 #define SOFTMAX_LDS_ROW 16384
 template <bool F16OUT>
@@ -291,12 +307,23 @@ __global__ __launch_bounds__(256) void softmax_row_kernel(tdesc x, tdesc mask, b
     const int nv = causal_past >= 0 ? (int)min((int64_t)ne0, causal_past + i1 + 1) : ne0;
     const float *mk_ = (has_mask && causal_past < 0) ? (const float *)at(mask, 0, i1, 0, 0) : nullptr;
     float mx = -INFINITY;
-    for (int i = threadIdx.x; i < nv; i += 256) {
-        float t;
-        if (mk_) { const float mv = mk_[i]; t = (mv == -INFINITY) ? -INFINITY : (s[i] + mv) * scale; }
-        else t = s[i] * scale;
-        s_row[i] = t;
-        mx = fmaxf(mx, t);
+    for (int base = threadIdx.x; base < nv; base += 1024) {         // four loads of a thread on the way together
+        float sv[4], mv[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int i = min(base + 256 * u, nv - 1);
+            sv[u] = s[i];
+            if (mk_) mv[u] = mk_[i];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (base + 256 * u < nv) {
+                float t;
+                if (mk_) t = (mv[u] == -INFINITY) ? -INFINITY : (sv[u] + mv[u]) * scale;
+                else t = sv[u] * scale;
+                s_row[base + 256 * u] = t;
+                mx = fmaxf(mx, t);
+            }
     }
     mx = block_reduce_256(mx, true, s_part);
     float sum = 0.0f;
@@ -377,17 +404,18 @@ __global__ __launch_bounds__(64) void rope_kernel(tdesc x, const int32_t *pos, i
     const int64_t i1 = blockIdx.x, i2 = blockIdx.y, i3 = blockIdx.z;
     const int32_t pi = *(const int32_t *)((const uint8_t *)pos + i2 * pos_stride);
     const float p = (float)pi;
-    const int64_t npair = y.ne[0] / 2;
+    const int npair = (int)(y.ne[0] / 2);
     const float ne0f = (float)y.ne[0];
-    for (int64_t k = threadIdx.x; k < npair; k += 64) {
-        float theta = p;
-        for (int64_t j = 0; j < k; j++) theta *= theta_scale;
-        float ang = freq_scale * theta;
-        if (ramp_on) ang = ang * (1 - ramp_mix) + theta * ramp_mix;
-        const float c = cosf(ang) * mscale, s = sinf(ang) * mscale;
+    for (int k = threadIdx.x; k < npair; k += 64) {
         const float *sp = (const float *)at(x, 2 * k, i1, i2, i3);
         float *dp = (float *)at(y, 2 * k, i1, i2, i3);
         const float x0 = sp[0], x1 = sp[1];
+        float theta = p;
+#pragma unroll 8
+        for (int j = 0; j < k; j++) theta *= theta_scale;
+        float ang = freq_scale * theta;
+        if (ramp_on) ang = ang * (1 - ramp_mix) + theta * ramp_mix;
+        const float c = cosf(ang) * mscale, s = sinf(ang) * mscale;
         if (xpos_base != 0.0f) {
             float zeta = powf(((float)(2 * k) + 0.4f * ne0f) / (1.4f * ne0f), p / xpos_base);
             if (xpos_down) zeta = 1.0f / zeta;
@@ -460,20 +488,23 @@ extern "C" int spy_hip_op_rope(void *stream, const spy_hip_tensor *x, const spy_
 // flat source counter unravelled in the destination's dimensions (:164-171).
 // conv: 0 raw 4-byte copy, 1 f32 -> f16, 2 f16 -> f32, 3 raw 2-byte copy.
 // ---------------------------------------------------------------------------------------------
+// element index -> coordinates; I = uint32_t where the tensor has fewer than 2^32 elements (a 64-bit division takes about ten times as long)
+template <class I> static __device__ __forceinline__ void unravel(I g, const tdesc &t, int64_t (&i)[4]) {
+    const I n0 = (I)t.ne[0], n1 = (I)t.ne[1], n2 = (I)t.ne[2];
+    const I r = g / n0, r2 = r / n1, r3 = r2 / n2;
+    i[0] = (int64_t)(g - r * n0); i[1] = (int64_t)(r - r2 * n1); i[2] = (int64_t)(r2 - r3 * n2); i[3] = (int64_t)r3;
+}
+template <class I>
 __global__ __launch_bounds__(256) void dup_kernel(tdesc s, tdesc d, int mode, int conv, int64_t total) {
     const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (g >= total) return;
-    const int64_t i00 = g % s.ne[0], r = g / s.ne[0];
-    const int64_t i01 = r % s.ne[1], i02 = r / s.ne[1] % s.ne[2], i03 = r / (s.ne[1] * s.ne[2]);
-    const uint8_t *sp = at(s, i00, i01, i02, i03);
+    int64_t i[4];
+    unravel((I)g, s, i);
+    const uint8_t *sp = at(s, i[0], i[1], i[2], i[3]);
     uint8_t *dp;
-    if (mode == 0) dp = at(d, i00, i01, i02, i03);
+    if (mode == 0) dp = at(d, i[0], i[1], i[2], i[3]);
     else if (mode == 1) dp = d.p + g * d.nb[0];
-    else {
-        const int64_t i0 = g % d.ne[0], i1 = g / d.ne[0] % d.ne[1];
-        const int64_t i2 = g % (d.ne[2] * d.ne[1] * d.ne[0]) / (d.ne[1] * d.ne[0]), i3 = g / (d.ne[2] * d.ne[1] * d.ne[0]);
-        dp = at(d, i0, i1, i2, i3);
-    }
+    else { unravel((I)g, d, i); dp = at(d, i[0], i[1], i[2], i[3]); }
     switch (conv) {
     case 0: *(uint32_t *)dp = *(const uint32_t *)sp; break;
     case 1: *(uint16_t *)dp = f2h(*(const float *)sp); break;
@@ -506,17 +537,19 @@ extern "C" int spy_hip_op_dup(void *stream, const spy_hip_tensor *src, const spy
     }
     const int64_t total = spy_t_nelem(src);
     CHECK_GRID(total, 256);
-    dup_kernel<<<dim3(grid_for(total, 256)), dim3(256), 0, (hipStream_t)stream>>>(mk(src), mk(dst), mode, conv, total);
+    if (total < (1ll << 32)) dup_kernel<uint32_t><<<dim3(grid_for(total, 256)), dim3(256), 0, (hipStream_t)stream>>>(mk(src), mk(dst), mode, conv, total);
+    else dup_kernel<uint64_t><<<dim3(grid_for(total, 256)), dim3(256), 0, (hipStream_t)stream>>>(mk(src), mk(dst), mode, conv, total);
     return SPY_LAUNCH_RC();
 }
 
 // Contiguous (view.cpp:285-321): dst (contiguous, src's dims) [i0..i3] = src[i0..i3]
+template <class I>
 __global__ __launch_bounds__(256) void contiguous_kernel(tdesc s, float *d, int64_t total) {
     const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (g >= total) return;
-    const int64_t i0 = g % s.ne[0], r = g / s.ne[0];
-    const int64_t i1 = r % s.ne[1], i2 = r / s.ne[1] % s.ne[2], i3 = r / (s.ne[1] * s.ne[2]);
-    d[g] = *(const float *)at(s, i0, i1, i2, i3);
+    int64_t i[4];
+    unravel((I)g, s, i);
+    d[g] = *(const float *)at(s, i[0], i[1], i[2], i[3]);
 }
 
 extern "C" int spy_hip_op_contiguous(void *stream, const spy_hip_tensor *src, const spy_hip_tensor *dst) {
@@ -525,7 +558,8 @@ extern "C" int spy_hip_op_contiguous(void *stream, const spy_hip_tensor *src, co
     SPY_CHECK_ARG(same_ne(src, dst) && spy_t_contiguous(dst));
     const int64_t total = spy_t_nelem(src);
     CHECK_GRID(total, 256);
-    contiguous_kernel<<<dim3(grid_for(total, 256)), dim3(256), 0, (hipStream_t)stream>>>(mk(src), (float *)dst->data, total);
+    if (total < (1ll << 32)) contiguous_kernel<uint32_t><<<dim3(grid_for(total, 256)), dim3(256), 0, (hipStream_t)stream>>>(mk(src), (float *)dst->data, total);
+    else contiguous_kernel<uint64_t><<<dim3(grid_for(total, 256)), dim3(256), 0, (hipStream_t)stream>>>(mk(src), (float *)dst->data, total);
     return SPY_LAUNCH_RC();
 }
 
@@ -544,9 +578,26 @@ __global__ __launch_bounds__(256) void get_row_kernel(tdesc table, bool q8, cons
     const int64_t ne00 = table.ne[0];
     if (!q8) { for (int64_t i = threadIdx.x; i < ne00; i += 256) dp[i] = ((const float *)sp)[i]; }
     else {
-        for (int64_t i = threadIdx.x; i < ne00; i += 256) {
-            const blk_q8_0 *b = (const blk_q8_0 *)sp + (i >> 5);
-            dp[i] = (float)b->qs[i & 31] * h2f(b->d);
+        // four quants per load and four loads of a thread on the way together: a row of 4096 is one memory latency (10.2 -> 4 us for one row)
+        for (int64_t base = threadIdx.x; base < ne00 / 4; base += 1024) {
+            uint32_t q[4];
+            uint16_t e[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int64_t i = min(base + 256 * u, ne00 / 4 - 1);
+                const blk_q8_0 *b = (const blk_q8_0 *)sp + (i >> 3);
+                const uint16_t *w = (const uint16_t *)(b->qs + (i & 7) * 4);
+                e[u] = b->d;
+                q[u] = w[0] | ((uint32_t)w[1] << 16);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (base + 256 * u < ne00 / 4) {
+                    const float d = h2f(e[u]);
+                    float *o = dp + 4 * (base + 256 * u);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) o[k] = (float)(int8_t)(q[u] >> (8 * k)) * d;
+                }
         }
     }
 }
@@ -601,20 +652,52 @@ extern "C" int spy_hip_argmax(void *stream, const float *logits, int64_t n, int3
 // ---------------------------------------------------------------------------------------------
 // MatMul (mat.cpp:32-146)
 // ---------------------------------------------------------------------------------------------
-// fp16 weight rows x fp16 activation rows (Dot<FP16,FP16>, vec_dot.h:117-146): one wave per
-// output element, lanes stride along the contraction.  w and dst strided, xh contiguous.
-__global__ __launch_bounds__(256) void matmul_f16_kernel(tdesc w, const uint16_t *__restrict__ xh, tdesc d, int64_t ne11, int64_t total) {
-    const int64_t o = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (o >= total) return;
-    const int lane = threadIdx.x & 63;
-    const int64_t ne00 = w.ne[0], ne01 = w.ne[1], ne02 = w.ne[2];
-    const int64_t i01 = o % ne01, i11 = o / ne01 % ne11, i02 = o / (ne01 * ne11) % ne02, i03 = o / (ne01 * ne11 * ne02);
-    const uint16_t *wr = (const uint16_t *)at(w, 0, i01, i02, i03);
-    const uint16_t *xr = xh + ((i03 * ne02 + i02) * ne11 + i11) * ne00;
-    float acc = 0.0f;
-    for (int64_t k = lane; k < ne00; k += 64) acc = fmaf(h2f(wr[k]), h2f(xr[k]), acc);
-    acc = wave_sum(acc);
-    if (lane == 0) *(float *)at(d, i01, i11, i02, i03) = acc;
+// fp16 weight rows x activation rows (Dot<FP16,FP16>, vec_dot.h:117-146): one wave per R output elements along i01, lanes stride along the contraction.
+// grid (i01 in fours of R, i11, i02 + ne02 * i03).  XF32: the activations are f32 and are rounded to fp16 here (mat.cpp:37,95-128), else contiguous fp16.
+// A single token's attention products (4096 x 128 and 128 x n_kv outputs) are launch and latency: R outputs share the activations and have their loads
+// on the way together, nothing is divided per output (64-bit divisions took longer than the products), and no launch converts the
+// activations: 8.7 + 2.5 -> 4.9 us each at 513 cached tokens and 32 heads.
+template <bool XF32, int R>
+__global__ __launch_bounds__(256) void matmul_f16_kernel(tdesc w, const uint8_t *__restrict__ x, int64_t x_nb1, int64_t x_nb2, int64_t x_nb3, tdesc d, int y0, int z0) {
+    const int i01 = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * R, ne01 = (int)w.ne[1];
+    if (i01 >= ne01) return;
+    const int lane = threadIdx.x & 63, i11 = y0 + (int)blockIdx.y, ne00 = (int)w.ne[0], ne02 = (int)w.ne[2];
+    int i02 = z0 + (int)blockIdx.z, i03 = 0;
+    if (i02 >= ne02) { i03 = i02 / ne02; i02 -= i03 * ne02; }
+    const uint16_t *wr[R];
+#pragma unroll
+    for (int j = 0; j < R; j++) wr[j] = (const uint16_t *)at(w, 0, min(i01 + j, ne01 - 1), i02, i03);
+    const uint8_t *xr = x + i11 * x_nb1 + i02 * x_nb2 + i03 * x_nb3;
+    float acc[R];
+#pragma unroll
+    for (int j = 0; j < R; j++) acc[j] = 0.0f;
+    auto get = [&](int k) { return XF32 ? h2f(f2h(((const float *)xr)[k])) : h2f(((const uint16_t *)xr)[k]); };
+    int k = lane;
+    for (; k + 192 < ne00; k += 256) {
+        float xv[4];
+        uint16_t wv[4][R];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            xv[u] = get(k + 64 * u);
+#pragma unroll
+            for (int j = 0; j < R; j++) wv[u][j] = wr[j][k + 64 * u];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int j = 0; j < R; j++) acc[j] = fmaf(h2f(wv[u][j]), xv[u], acc[j]);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        if (k + 64 * u < ne00) {
+            const float xv = get(k + 64 * u);
+#pragma unroll
+            for (int j = 0; j < R; j++) acc[j] = fmaf(h2f(wr[j][k + 64 * u]), xv, acc[j]);
+        }
+    float out = 0.0f;
+#pragma unroll
+    for (int j = 0; j < R; j++) { const float t = wave_sum(acc[j]); if (lane == j) out = t; }
+    if (lane < R && i01 + lane < ne01) *(float *)at(d, i01 + lane, i11, i02, i03) = out;
 }
 
 int spy_gemm_f16_launch(hipStream_t st, const void *A, int64_t a_nb1, int64_t a_nb2, const uint16_t *B, void *dst, int64_t d_nb1, int64_t d_nb2,
@@ -692,6 +775,24 @@ static int own_matvec(hipStream_t st, int t0, const void *w, const float *x, flo
     case SPY_HIP_Q6_K: return spy_own_matvec_q6_k(st, w, x, out, (int)M, (int)K);
     default: return SPY_HIP_EUNSUPPORTED;
     }
+}
+// R: as many outputs per wave as still give every compute unit two workgroups
+template <bool XF32>
+static int matmul_f16_launch(hipStream_t st, const spy_hip_tensor *w, const uint8_t *x, int64_t x_nb1, int64_t x_nb2, int64_t x_nb3, const spy_hip_tensor *dst) {
+    const int64_t ne11 = dst->ne[1], nz = w->ne[2] * w->ne[3];
+    SPY_CHECK_ARG(w->ne[0] > 0 && w->ne[0] < (1ll << 30) && w->ne[1] > 0 && w->ne[1] < (1ll << 30) && ne11 > 0 && ne11 < (1ll << 31) && nz > 0 && nz < (1ll << 31));
+    const int64_t wgs = w->ne[1] * ne11 * nz / 4;
+    const int R = wgs >= 8 * 512 ? 8 : wgs >= 4 * 256 ? 4 : 1;
+    for (int64_t z = 0; z < nz; z += 65535)
+        for (int64_t y = 0; y < ne11; y += 65535) {
+            const dim3 grid((unsigned)((w->ne[1] + 4 * R - 1) / (4 * R)), (unsigned)(ne11 - y < 65535 ? ne11 - y : 65535), (unsigned)(nz - z < 65535 ? nz - z : 65535));
+            if (R == 8) matmul_f16_kernel<XF32, 8><<<grid, dim3(256), 0, st>>>(mk(w), x, x_nb1, x_nb2, x_nb3, mk(dst), (int)y, (int)z);
+            else if (R == 4) matmul_f16_kernel<XF32, 4><<<grid, dim3(256), 0, st>>>(mk(w), x, x_nb1, x_nb2, x_nb3, mk(dst), (int)y, (int)z);
+            else matmul_f16_kernel<XF32, 1><<<grid, dim3(256), 0, st>>>(mk(w), x, x_nb1, x_nb2, x_nb3, mk(dst), (int)y, (int)z);
+            const int rc = SPY_LAUNCH_RC();
+            if (rc) return rc;
+        }
+    return 0;
 }
 static int matmul_impl(void *stream, const spy_hip_tensor *w, const spy_hip_tensor *x, const spy_hip_tensor *dst, void *scratch, size_t scratch_bytes,
                        int skip_past, int klimit_past, bool own_kernels = false);
@@ -771,6 +872,10 @@ static int matmul_impl(void *stream, const spy_hip_tensor *w, const spy_hip_tens
         const size_t need = (size_t)(spy_t_nrow(x) * mid_row);
         if (!scratch || scratch_bytes < need) return SPY_HIP_ENOSPACE;
         SPY_CHECK_ARG(x->nb[0] == 4);
+        // few activation rows against fp16 rows in this backend's own order: converted where they are read
+        if (tm == SPY_HIP_F16 && ne11 < 16 && !(spy_exact_on() && skip_past < 0 && klimit_past < 0) && w->nb[0] == 2 && x->nb[1] % 4 == 0 && x->nb[2] % 4 == 0 &&
+            x->nb[3] % 4 == 0 && ((uintptr_t)x->data & 3) == 0)
+            return matmul_f16_launch<true>(st, w, (const uint8_t *)x->data, x->nb[1], x->nb[2], x->nb[3], dst);
         if (tm == SPY_HIP_F16 && ne12 * ne13 > 1 && ne12 * ne13 <= 65535 && ne10 % 4 == 0 && x->nb[1] % 16 == 0 && x->nb[2] % 16 == 0 &&
             x->nb[3] % 16 == 0 && ((uintptr_t)x->data & 15) == 0 && ne10 * ne11 / 4 < (1ll << 31) * 256) {
             // all batches (heads) in one launch
@@ -831,10 +936,7 @@ static int matmul_impl(void *stream, const spy_hip_tensor *w, const spy_hip_tens
         }
         return 0;
     }
-    const int64_t total = ne01 * ne11 * ne02 * ne03;
-    CHECK_GRID(total, 4);
-    matmul_f16_kernel<<<dim3(grid_for(total, 4)), dim3(256), 0, st>>>(mk(w), (const uint16_t *)xm, mk(dst), ne11, total);
-    return SPY_LAUNCH_RC();
+    return matmul_f16_launch<false>(st, w, xm, 2 * ne10, 2 * ne10 * ne11, 2 * ne10 * ne11 * ne12, dst);
 }
 
 // ---- MatMul for callers that cannot allocate ---------------------------------------------------------

@@ -204,3 +204,29 @@ def test_own_order_prompt_from_packed_activations(hip, n_prompt, monkeypatch):
         assert np.array_equal(got[None].view(np.uint32), got["tile"].view(np.uint32))
     else:                       # q, k, v, wo and down in slices of K without the switch
         assert np.linalg.norm(got[None] - got["tile"]) <= 3e-2 * np.linalg.norm(got["tile"])
+
+
+@pytest.mark.parametrize("M,K,T,batch", [(1, 2, 1, 1), (5, 63, 2, 3), (130, 513, 1, 32), (600, 128, 1, 32), (33, 300, 15, 9), (1027, 257, 3, 8)])
+@pytest.mark.parametrize("x_type", ["f32", "f16"])
+def test_fp16_rows_against_few_activation_rows(hip, M, K, T, batch, x_type):
+    """The attention products of few tokens in this backend's own order, one, four or eight outputs per wave, activations rounded to fp16 where they are
+    read (f32) or given as fp16, with remainders on every side."""
+    from tests.gpu_util import dev, dev_empty, call, assert_close
+    L = hip.load()
+    prev = L.spy_hip_set_exact_order(0)
+    try:
+        rng = np.random.default_rng(M + K + T)
+        w = rng.standard_normal((batch, M, K)).astype(np.float16)
+        x = rng.standard_normal((batch, T, K)).astype(np.float32)
+        xh = x.astype(np.float16)
+        want = np.matmul(xh.astype(np.float64), w.astype(np.float64).transpose(0, 2, 1))
+        dx = dev(x) if x_type == "f32" else dev(xh.view(np.uint16))
+        tw, tx = hip.tensor(dev(w.view(np.uint16)), hip.F16, [K, M, batch]), hip.tensor(dx, hip.F32 if x_type == "f32" else hip.F16, [K, T, batch])
+        need = L.spy_hip_op_matmul_scratch_size(B(tw), B(tx))
+        scratch, out = dev_empty(max(need, 16), 0xEE), dev_empty(batch * T * M * 4 + 64, 0xFF)
+        call(L.spy_hip_op_matmul, None, B(tw), B(tx), B(hip.tensor(out, hip.F32, [M, T, batch])), scratch.ptr, need)
+        got = out.download(np.float32)
+        assert (got[batch * T * M:].view(np.uint32) == 0xFFFFFFFF).all(), "nothing is written beyond the outputs"
+        assert_close(got[:batch * T * M].reshape(batch, T, M), want, "fp16 rows %dx%d T=%d x %d" % (M, K, T, batch), tol=1e-5)
+    finally:
+        L.spy_hip_set_exact_order(prev)

@@ -63,6 +63,13 @@ int spy_hip_alloc(void **ptr, size_t bytes);
 int spy_hip_free(void *ptr);
 int spy_hip_upload(void *dst_dev, const void *src_host, size_t bytes, void *stream);
 int spy_hip_download(void *dst_host, const void *src_dev, size_t bytes, void *stream);
+/* Pinned host memory, and transfers between it and device memory that are only queued on `stream` (16-byte aligned pointers for
+ * the kernel that moves small ones; the host side must stay unchanged until the stream has passed them).  download_pinned also
+ * hands out and clears the device's error flag (spy_hip_take_error) at this point of the stream: *flag_out, in pinned memory too. */
+int spy_hip_host_alloc(void **ptr, size_t bytes);
+int spy_hip_host_free(void *ptr);
+int spy_hip_upload_pinned(void *dst, const void *src, size_t bytes, void *stream);
+int spy_hip_download_pinned(void *dst, const void *src, size_t bytes, int *flag_out, void *stream);
 int spy_hip_fill_u8(void *dst_dev, int value, size_t bytes, void *stream);   /* fill kernel, graph-safe */
 int spy_hip_sync(void *stream);                      /* NULL: whole device */
 int spy_hip_stream_create(void **stream);

@@ -67,6 +67,10 @@ SIGNATURES = {
     "spy_hip_free": (_i32, [_vp]),
     "spy_hip_upload": (_i32, [_vp, _vp, _sz, _vp]),
     "spy_hip_download": (_i32, [_vp, _vp, _sz, _vp]),
+    "spy_hip_host_alloc": (_i32, [C.POINTER(_vp), _sz]),
+    "spy_hip_host_free": (_i32, [_vp]),
+    "spy_hip_upload_pinned": (_i32, [_vp, _vp, _sz, _vp]),
+    "spy_hip_download_pinned": (_i32, [_vp, _vp, _sz, _vp, _vp]),
     "spy_hip_fill_u8": (_i32, [_vp, _i32, _sz, _vp]),
     "spy_hip_sync": (_i32, [_vp]),
     "spy_hip_stream_create": (_i32, [C.POINTER(_vp)]),

@@ -23,12 +23,6 @@
 #define XG_THREADS 1024
 #define XG_WAVES 16
 #define XG_NBS 128                         // blocks per K slab (= 64 lanes x one block pair)
-#ifndef XG_PSUM
-#define XG_PSUM 1                          // gate|up: the running sum of the norm through xg_exact_sum (0: one chain, as in the other kernels)
-#endif
-#ifndef XG_DEPTH
-#define XG_DEPTH 3                         // rows per wave requested ahead of their use
-#endif
 
 template <int WT> struct xg_traits { static constexpr int NCH = (WT == SPY_HIP_Q4_0 || WT == SPY_HIP_Q8_0) ? 8 : 1; };
 // floats of LDS per row slot: NCH rows of partials (+4: bank skew between the rows) and the row of scale products (+4: skew between slots)
@@ -91,155 +85,115 @@ static __device__ __forceinline__ float xg_serial_sum(const float *s, int n, flo
     return init;
 }
 
-// ---- the same running sum, for NON-NEGATIVE terms, mostly in parallel and still bit for bit -----------------------------
+// ---- the same running sum of up to 1024 M NON-NEGATIVE terms by ONE wave, mostly in parallel and still bit for bit -----------------
 // While the running sum s stays inside one binade [2^e, 2^(e+1)) it is an integer multiple S of ulp = 2^(e-23), and adding a term
-// g >= 0 with round-to-nearest-even is integer arithmetic: with f = g / ulp (exact: a power-of-two scaling),
+// g >= 0 with round-to-nearest-even is integer arithmetic: with f = g / ulp,
 //     RNE(S + f) = S + floor(f) + r,   r = 1 if frac(f) > 1/2, 0 if < 1/2, and for frac(f) = 1/2 the parity of S + floor(f).
-// So a term is a map from the parity of the incoming S to an increment, (inc_even, inc_odd), maps compose associatively
-// (C[p] = A[p] + B[(p + A[p]) & 1]), and 64 consecutive terms reduce to one pair in four DPP steps and three scalar ones.  The
-// sum is non-decreasing, so if the chunk's first and last value lie in binade e, every value between does.  Wave c reduces
-// chunk c (terms 64 c .. 64 c + 63) against the binade that an approximate prefix sum predicts; then one wave walks the chunks:
-// where the exact running sum has the predicted exponent and bits(s) + increment keeps it (the integer addition on the float's
-// bits IS s + increment * ulp), the chunk is one addition; otherwise (the sum crosses a power of two inside the chunk, the first
-// chunk, a wrong prediction) the chunk's 64 terms are added one by one as above.  Nothing is approximated in what is kept: the
-// prediction only selects which chunks take the short way.
-struct xg_psum_lds { float cs[32]; int t0[32], t1[32], eb[32]; };
-// g[j]: term 1024 j + tid of the n <= 1024 NG terms (0 beyond n), all of them also at s_g in LDS (written before the call,
-// 16-byte aligned, readable 40 floats beyond n).  Every thread of the 1024 calls; the sum is returned by wave 0 only (wave-uniform).
-// `others` runs in the other waves once their part is done, i.e. while wave 0 walks.
-template <int NG, class Others>
-static __device__ __forceinline__ float xg_exact_sum(const float (&g)[NG], int n, const float *s_g, xg_psum_lds *L, float init, Others others, long long *dbg = nullptr) {
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nchunk = (n + 63) >> 6;
-    // sum over the wave through DPP only (no LDS permutes), read from lane 63; the order of these additions does not matter:
-    // they only predict binades
-    auto total = [](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wave_total_lane63(v)), 63)); };
+// So a run of terms is a map from the parity of the incoming S to an increment, (inc_even, inc_odd), and maps compose associatively
+// (C[p] = A[p] + B[(p + A[p]) & 1]).  The sum is non-decreasing: if its first and last value lie in binade e, every value between does.
+// Lane c has the 16 M terms from 16 M c on.
+// Padded layout of the terms: 16 floats every 20 (80 bytes: the lanes' 128-bit reads spread over the banks); zeros up to the next multiple of 16 M.
+static __device__ __forceinline__ int xg_seg_at(int i) { return i + (i >> 4) * 4; }
+// Every lane adds its terms to two candidate values of the running sum, neighbours (even and odd) near an approximate prefix sum: by the rule above
+// the differences are the increments for ANY incoming sum of that binade, as long as it stays there.  Runs of segments in one binade are composed by a
+// segmented scan, and the walk takes a run in one addition; what remains are the segments in which the sum crosses a power of two (about one per
+// doubling), added term by term.  Where the prefix sum named the wrong binade (the exact sum has another exponent before or after the run), the
+// run is added term by term as well: nothing that is kept is approximate.  1024 terms: 2 us (chain of single additions: 4.4).
+template <int M>
+static __device__ __forceinline__ float xg_segment_sum(const float *s_g, int n) {
+    if (n <= 0) return 0.0f;
+    const int lane = threadIdx.x & 63, nseg = (n + 16 * M - 1) / (16 * M);
+    float4 v[4 * M];
+    auto term4 = [&](int c, int u) { return *(const float4 *)(s_g + c * (20 * M) + (u >> 2) * 20 + 4 * (u & 3)); };
 #pragma unroll
-    for (int j = 0; j < NG; j++) {
-        const float cs = total(g[j]);
-        if (lane == 0) L->cs[wave + 16 * j] = cs;
+    for (int u = 0; u < 4 * M; u++) v[u] = term4(min(lane, nseg - 1), u);
+    float cs = 0.0f;
+#pragma unroll
+    for (int u = 0; u < 4 * M; u++) cs += (v[u].x + v[u].y) + (v[u].z + v[u].w);
+    float incl = cs;                                     // inclusive prefix over the lanes (an approximation: its rounding does not matter)
+#define XG_DPP_F(x, CTRL, ROWS) __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, ROWS, 0xF, true))
+    incl += XG_DPP_F(incl, 0x111, 0xF); incl += XG_DPP_F(incl, 0x112, 0xF); incl += XG_DPP_F(incl, 0x114, 0xF); incl += XG_DPP_F(incl, 0x118, 0xF);
+    incl += XG_DPP_F(incl, 0x142, 0xA); incl += XG_DPP_F(incl, 0x143, 0xC);
+#undef XG_DPP_F
+    // (bound_ctrl: lanes outside the row mask and before the row's start get 0)
+    const int before = __float_as_int(__int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(incl), 0x138, 0xF, 0xF, true)));       // wave_shr:1
+    const int be = before & ~1, bo = before | 1, eb = be >> 23;
+    float se = __int_as_float(be), so = __int_as_float(bo);
+#pragma unroll
+    for (int u = 0; u < 4 * M; u++) {
+        se += v[u].x; so += v[u].x; se += v[u].y; so += v[u].y; se += v[u].z; so += v[u].z; se += v[u].w; so += v[u].w;
     }
-    XSTAMP(dbg, 8);
-    __syncthreads();                                     // chunk sums and (by the caller) the terms are in LDS
-    XSTAMP(dbg, 9);
+    const int ee = __float_as_int(se), eo = __float_as_int(so);
+    const bool ok = eb >= 1 && eb < 254 && (ee >> 23) == eb && (eo >> 23) == eb;
+    int t0 = ee - be, t1 = eo - bo;
+    const int pe = __builtin_amdgcn_update_dpp(-1, ok ? eb : -1, 0x138, 0xF, 0xF, false);      // binade of the segment before, -1: none
+    const bool head = !ok || pe != eb;
+    int f = head ? 1 : 0;
+#define XG_STEP(CTRL, ROWS) { const int p0 = __builtin_amdgcn_update_dpp(0, t0, CTRL, ROWS, 0xF, false), p1 = __builtin_amdgcn_update_dpp(0, t1, CTRL, ROWS, 0xF, false), \
+                                        pf = __builtin_amdgcn_update_dpp(1, f, CTRL, ROWS, 0xF, false), has = __builtin_amdgcn_update_dpp(0, 1, CTRL, ROWS, 0xF, false); \
+                              const int c0 = p0 + ((p0 & 1) ? t1 : t0), c1 = p1 + ((p1 & 1) ? t0 : t1); \
+                              if (has && !f) { t0 = c0; t1 = c1; f = pf; } }
+    XG_STEP(0x111, 0xF) XG_STEP(0x112, 0xF) XG_STEP(0x114, 0xF) XG_STEP(0x118, 0xF) XG_STEP(0x142, 0xA) XG_STEP(0x143, 0xC)
+#undef XG_STEP
+    const unsigned long long in = nseg >= 64 ? ~0ull : (1ull << nseg) - 1, heads = __ballot(head) & in, slow = __ballot(!ok) & in;
+    auto next = [&](unsigned long long m, int from) -> int { const unsigned long long x = from < 64 ? m >> from << from : 0ull; return x ? __builtin_ctzll(x) : nseg; };
+    float4 w[4 * M];
+    auto request = [&](int c) {
 #pragma unroll
-    for (int j = 0; j < NG; j++) {
-        const int c = wave + 16 * j;
-        if (c < nchunk) {
-            const float before = total(lane < c ? L->cs[lane & 31] : 0.0f) + init, after = before + L->cs[c];
-            const int eb = (__float_as_int(before) >> 23) & 0xFF;
-            const float f = ldexpf(g[j], 150 - eb);      // g / ulp
-            const bool fits = f < 16777216.0f;           // false for a NaN too
-            const int fl = fits ? (int)f : 0;
-            const float frac = f - (float)fl;
-            const int up = frac > 0.5f ? 1 : 0, tie = frac == 0.5f ? 1 : 0;
-            int a0 = fl + (up | (tie & fl & 1)), a1 = fl + (up | (tie & ~fl & 1));    // incoming S even / odd: a tie rounds to the even neighbour
-            // within each row of 16 lanes: lane l takes over the terms of lane l + d (row_shl), earlier terms first; lanes
-            // that reach beyond their row compute values nobody uses
-#define XG_PS_STEP(CTRL) { const int b0 = __builtin_amdgcn_update_dpp(0, a0, CTRL, 0xF, 0xF, true), b1 = __builtin_amdgcn_update_dpp(0, a1, CTRL, 0xF, 0xF, true); \
-                           a0 = a0 + ((a0 & 1) ? b1 : b0); a1 = a1 + ((a1 & 1) ? b0 : b1); }   /* incoming odd: the parity after the first part is (1 + a1) & 1 */
-            XG_PS_STEP(0x101) XG_PS_STEP(0x102) XG_PS_STEP(0x104) XG_PS_STEP(0x108)
-#undef XG_PS_STEP
-            // the four rows in order, as scalars
-            int t0 = __builtin_amdgcn_readlane(a0, 0), t1 = __builtin_amdgcn_readlane(a1, 0);
-#pragma unroll
-            for (int r = 1; r < 4; r++) {
-                const int b0 = __builtin_amdgcn_readlane(a0, 16 * r), b1 = __builtin_amdgcn_readlane(a1, 16 * r);
-                t0 = t0 + ((t0 & 1) ? b1 : b0);
-                t1 = t1 + ((t1 & 1) ? b0 : b1);
-            }
-            const bool ok = __all(fits) && c > 0 && eb >= 1 && eb < 254 && ((__float_as_int(after) >> 23) & 0xFF) == eb;
-            if (lane == 0) { L->t0[c] = t0; L->t1[c] = t1; L->eb[c] = ok ? eb : -1; }
+        for (int u = 0; u < 4 * M; u++) w[u] = term4(c, u);
+    };
+    int have = next(slow, 0);                            // the next segment to be added term by term is requested ahead
+    if (have < nseg) request(have);
+    int bits = 0, c = 0;
+    while (c < nseg) {
+        int to = c + 1;
+        if (!((slow >> c) & 1)) {
+            const int x = next(heads, c + 1), e = __builtin_amdgcn_readlane(eb, c);
+            const int nb = bits + ((bits & 1) ? __builtin_amdgcn_readlane(t1, x - 1) : __builtin_amdgcn_readlane(t0, x - 1));
+            if ((bits >> 23) == e && (nb >> 23) == e) { bits = nb; c = x; continue; }
+            to = x;                                      // the prefix sum named the wrong binade: the whole run term by term
         }
+        float s = __int_as_float(bits);
+        for (; c < to; c++) {
+            if (c != have) request(c);
+#pragma unroll
+            for (int u = 0; u < 4 * M; u++) { s = s + w[u].x; s = s + w[u].y; s = s + w[u].z; s = s + w[u].w; }
+            have = next(slow, c + 1);
+            if (have < nseg) request(have);
+        }
+        bits = __builtin_amdgcn_readfirstlane(__float_as_int(s));
     }
-    XSTAMP(dbg, 10);
-    __syncthreads();
-    XSTAMP(dbg, 11);
-    float s = init;
-    if (wave == 0) {
-        const int vt0 = L->t0[lane & 31], vt1 = L->t1[lane & 31], veb = L->eb[lane & 31];
-        // the terms of the chunks predicted to need the long way are requested ahead: the first such chunk now, the next one
-        // when the current one is taken up (a chunk that fails without having been predicted pays the LDS latency)
-        const unsigned long long slowmask = __ballot(lane < nchunk && veb < 0);
-        auto next_slow = [&](int from) -> int { const unsigned long long m = from < 64 ? (slowmask >> from) << from : 0ull; return m ? __builtin_ctzll(m) : -1; };
-        // (its first 32 terms; the other 32 are requested when the chunk is taken up and arrive behind the first 32 additions)
-        float4 v[8], w[8];
-        auto request = [&](int c) {
-#pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = *(const float4 *)(s_g + 64 * c + 4 * u);
-        };
-        int pre = next_slow(0);
-        if (pre >= 0) request(pre);
-        int bits = __builtin_amdgcn_readfirstlane(__float_as_int(s));             // the running sum as a scalar
-        [[maybe_unused]] int nfall = 0;
-        for (int c = 0; c < nchunk; c++) {
-            const int eb = __builtin_amdgcn_readlane(veb, c), t = (bits & 1) ? __builtin_amdgcn_readlane(vt1, c) : __builtin_amdgcn_readlane(vt0, c);
-            const int nb = bits + t;
-            if (eb == (bits >> 23) && (nb >> 23) == eb && t >= 0) { bits = nb; continue; }
-            s = __int_as_float(bits);
-            nfall++;
-            if (n - 64 * c >= 64) {                      // a whole chunk one by one
-                if (c != pre) request(c);
-#pragma unroll
-                for (int u = 0; u < 8; u++) w[u] = *(const float4 *)(s_g + 64 * c + 32 + 4 * u);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int u = 0; u < 8; u++) { s = s + v[u].x; s = s + v[u].y; s = s + v[u].z; s = s + v[u].w; }
-                __builtin_amdgcn_sched_barrier(0);
-                if (c == pre) { pre = next_slow(c + 1); if (pre >= 0) request(pre); }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int u = 0; u < 8; u++) { s = s + w[u].x; s = s + w[u].y; s = s + w[u].z; s = s + w[u].w; }
-            } else s = xg_serial_sum(s_g + 64 * c, n - 64 * c, s);
-            bits = __builtin_amdgcn_readfirstlane(__float_as_int(s));
-        }
-        s = __int_as_float(bits);
-        XSTAMP(dbg, 12);
-#ifdef XDBG_STAMPS
-        if (dbg && blockIdx.x == 0 && threadIdx.x == 0) dbg[13] = nfall;
-#endif
-    } else others();
-    return s;
+    return __int_as_float(bits);
 }
 
 // ---- activations: f32 vector -> (RMSNorm * weight ->) Q8_0 in LDS, sums in the host order --------------------------
 // NormRMS (non-linear.cpp:194-223): sum = std::transform_reduce(x, x) = groups of four ((x0^2 + x1^2) + (x2^2 + x3^2))
 // added to one running sum in order; scale = 1 / sqrt(sum / n + eps); y = x * scale; then the Mul node: y * w.
-// The 1024 threads form the group sums (one float4 each per 4096 elements), lane 0 of wave 0 adds them.
-template <int NITK, bool NORM, bool PSUM = false, class Issue>
+// The 1024 threads form the group sums (one float4 each per 4096 elements), wave 0 adds them (xg_segment_sum).
+template <int NITK, bool NORM, class Issue>
 static __device__ __forceinline__ void xg_stage(const float4 (&xv)[NITK], const float4 (&wv)[NORM ? NITK : 1], int K, float eps,
                                                 int8_t *s_q, int2 *s_meta, float *s_grp, float *s_sum, Issue issue_rows) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     float scale = 1.0f;
     if constexpr (NORM) {
-        float grp[NITK];
 #pragma unroll
         for (int j = 0; j < NITK; j++) {
             const int i = tid + j * XG_THREADS;
-            grp[j] = 0.0f;
             if (i < K / 4) {
                 const float4 v = xv[j];
                 const float a0 = v.x * v.x, a1 = v.y * v.y, a2 = v.z * v.z, a3 = v.w * v.w;
                 const float v1 = a0 + a1, v2 = a2 + a3;
-                grp[j] = v1 + v2;
-                s_grp[i] = grp[j];
-            }
+                s_grp[xg_seg_at(i)] = v1 + v2;
+            } else if (i < (K / 4 + 16 * NITK - 1) / (16 * NITK) * (16 * NITK)) s_grp[xg_seg_at(i)] = 0.0f;
         }
-        // The weight rows are requested only after the group sums (and the scan of the sum): a wave that asks for several rows sits
-        // in the issue stage until the memory queue has room, and a request made earlier would hold up the barriers for every wave.
-        // Wave 0 walks the sum first.
-        if constexpr (NITK <= 2 && PSUM) {
-            xg_psum_lds *L = (xg_psum_lds *)(s_grp + ((K / 4 + 3) & ~3) + 64);
-            const float tot = xg_exact_sum<NITK>(grp, K / 4, s_grp, L, 0.0f, issue_rows);
-            if (wave == 0) { if (lane == 0) *s_sum = tot; issue_rows(); }
-        } else {
-            __syncthreads();
-            if (wave == 0) {
-                const float init = xg_serial_sum(s_grp, K / 4, 0.0f);
-                if (lane == 0) *s_sum = init;
-            }
-            issue_rows();
+        // The weight rows are requested only after the group sums: a wave that asks for several rows sits in the issue stage until the memory
+        // queue has room, and a request made earlier would hold up the barriers for every wave.  Wave 0 walks the sum first.
+        __syncthreads();
+        if (wave == 0) {
+            const float tot = xg_segment_sum<NITK>(s_grp, K / 4);
+            if (lane == 0) *s_sum = tot;
         }
+        issue_rows();
         __syncthreads();
         const float mean = *s_sum / (float)K;
         scale = 1.0f / sqrtf(mean + eps);
@@ -462,14 +416,12 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(xg_args a) {
         xv[j] = ((const float4 *)a.x_in)[i];
         if constexpr (NORM) wv[j] = ((const float4 *)a.normw)[i];
     }
-    // rows requested ahead of their use: all of the wave's rows where their registers allow (Q4_0 rows, up to 6), so
-    // that the weights stream in while the serial sum of the norm is walked; XG_DEPTH otherwise
-    // The sum of the norm in chunks (xg_exact_sum) pays where the wait that follows it is short: gate|up with three rows requested
-    // ahead (17.1 against 18.5 us; with all six requested the waves sit in the issue stage for longer than the serial walk takes, and
-    // the chunked sum gains nothing: 19.6).  It lost in the other kernels with a norm (qkv 13.2 against 12.7 at any depth, head 22.0
-    // against 20.6).
-    constexpr bool PSUM = XG_PSUM && EPI == EPI_GATEUP;
-    constexpr int DEPTH = (!PSUM && NROW <= 6 && wt_traits<WT>::PAIR_DW * NITK <= 9) ? NROW : (XG_DEPTH < NROW ? XG_DEPTH : NROW);
+    // Rows requested ahead of their use.  A wave waits in the issue stage while the memory queue is full, i.e. while the stream runs, and the barriers
+    // of the norm wait for every wave: 2 rows of each of 16 waves (73 KB of Q4_0, 3.3 us of the stream) about cover the norm's sum.  qkv with 2 of 3
+    // rows 11.1 us (all 3: 11.9), head with 2 24.4 us (3: 25.1), gate|up with 3 of 6 15.8 us (2: 16.1; 4: 16.9).
+    // gate|up asks for its first row (37 KB, which the queue takes at once) right behind the activations: 15.5 us; with less to
+    // stream after the norm the other kernels lose by it (qkv 11.9).
+    constexpr int DEPTH = EPI == EPI_GATEUP ? (NROW < 3 ? NROW : 3) : NROW < 2 ? NROW : 2, PRE = EPI == EPI_GATEUP ? 1 : 0;
     constexpr int RING = NROW < DEPTH + 1 ? NROW : DEPTH + 1;
     wtile<WT, NITK> t[RING];
     wtile<WTV, NITK> tv;
@@ -480,15 +432,19 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(xg_args a) {
     auto issue_first = [&]() {
         if constexpr (!NORM) __builtin_amdgcn_s_barrier();      // x of every wave ahead of every wave's rows in the compute unit's memory queue
 #pragma unroll
-        for (int r = 0; r < NROW; r++) if (r < DEPTH) issue(r);
+        for (int r = 0; r < NROW; r++) if (r < DEPTH && r >= PRE) issue(r);
     };
+    if constexpr (PRE > 0) {
+        __builtin_amdgcn_s_barrier();
+        issue(0);
+    }
 
     // 3. stage the activations (the first rows are requested inside: after the group sums of the norm, or at once)
     int8_t *s_q = (int8_t *)smem;
     int2 *s_meta = (int2 *)(smem + staged_q_bytes(K));
     float *s_part = (float *)(smem + ((staged_bytes(K) + 15) & ~(size_t)15));      // row slots; the group sums of the norm use the same bytes before
     XSTAMP(a.dbg, 16);
-    xg_stage<NITK, NORM, PSUM>(xv, wv, K, a.eps, s_q, s_meta, s_part, &s_sum, issue_first);
+    xg_stage<NITK, NORM>(xv, wv, K, a.eps, s_q, s_meta, s_part, &s_sum, issue_first);
     XSTAMP(a.dbg, 17);
     if (a.q8_dump && blockIdx.x == 0) xg_dump_q8(s_q, s_meta, K, a.q8_dump);
     staged_act act; act.q = s_q; act.meta = s_meta;
@@ -692,9 +648,6 @@ __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_stat
 // last 1..32 elements, by the lane of accumulator 0).
 #define XP_THREADS 1024
 #define XP_NP 10                           // 16-byte pieces per lane of a V^T row: n_ctx <= 5120
-#ifndef XP_PSUM
-#define XP_PSUM 0                          // the softmax sum through xg_exact_sum: 4.1 instead of 4.9 us for the sum, but the V^T rows are then requested later and the kernel takes 15.2 instead of 14.0 us
-#endif
 #define XP_NS 5                            // scores per thread: n_ctx <= 5120
 static inline int xattn_pv_vstride(int n_ctx) { return ((n_ctx + 63) / 64) * 64 + 32; }        // halfs between rows in LDS: = 64 bytes mod 128, the two rows of a wave on different banks
 static inline size_t xattn_pv_lds(int n_ctx) {
@@ -755,7 +708,7 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
             s_grp[g] = grp[u];
         }
     }
-    if (!XP_PSUM) __syncthreads();
+    __syncthreads();
     XSTAMP(dbg, 3);
     // The V^T rows are requested now, by every wave but the one that walks the sum (a wave that asks for its whole row sits in the
     // issue stage until the memory queue has room, i.e. for most of the row's transfer time): the rows arrive while the sum is walked.
@@ -770,15 +723,7 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
         vb6 = *(const uint4 *)(vp + (size_t)min(6 * 64 + lane, last_piece) * 8); vb7 = *(const uint4 *)(vp + (size_t)min(7 * 64 + lane, last_piece) * 8);
         vb8 = *(const uint4 *)(vp + (size_t)min(8 * 64 + lane, last_piece) * 8); vb9 = *(const uint4 *)(vp + (size_t)min(9 * 64 + lane, last_piece) * 8);
     };
-    if (XP_PSUM) {
-        xg_psum_lds *L = (xg_psum_lds *)(s_grp + ((n_ctx / 4 + 3) & ~3) + 64);
-        float init = xg_exact_sum<2>(grp, ngrp, s_grp, L, 0.0f, load_row, dbg);
-        if (wave == 0) {
-            for (int j = ngrp * 4; j < n_kv; j++) init = init + s_e[j];
-            if (lane == 0) s_sum = init;
-            load_row();
-        }
-    } else if (wave != 0) load_row();
+    if (wave != 0) load_row();
     else {
         float init = xg_serial_sum(s_grp, ngrp, 0.0f);
         for (int j = ngrp * 4; j < n_kv; j++) init = init + s_e[j];

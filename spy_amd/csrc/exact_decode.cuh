@@ -545,6 +545,7 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(xg_args a) {
 // accumulators sum[j][l] over the chunks i = 0, 32, 64 (i + 32 < n), the reduction tree of FP16::block_reduce, then the
 // scalar tail over elements 96..127 (a product of two fp16 values is exact in fp32, so `tail += a * b` is the fma it is
 // written as here), result = tail + simd.  Stored: t = dot * scale (mask 0, then * scale: non-linear.cpp:141-150).
+typedef uint32_t xp_u4 __attribute__((ext_vector_type(4)));
 #define XS_THREADS 1024
 #define XS_TOK 18
 #define XS_NLD 9                                        // pieces per thread requested together: 1024 x 9 x 16 bytes = 18 tokens of 32 heads
@@ -563,48 +564,56 @@ __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_stat
     uint4 *s_k = (uint4 *)smem;                         // [XS_TOK][n_head][16 chunks of 16 bytes], chunk index rotated per key against bank conflicts
     uint4 *s_qh = s_k + XS_TOK * n_head * 16;           // [n_head][16]
     const int per_tok = n_head * 16;                    // 16-byte pieces per token
-    // the pieces in flight: named registers (an indexed array that lives across the rounds ends up in scratch memory)
-    uint4 k0, k1, k2, k3, k4, k5, k6, k7, k8;
-    static_assert(XS_NLD == 9, "nine named registers");
-#define XS_EACH(X) X(0, k0) X(1, k1) X(2, k2) X(3, k3) X(4, k4) X(5, k5) X(6, k6) X(7, k7) X(8, k8)
-    auto request = [&](int t0, int npiece, int c0) {
-#define XS_REQ(u, r) { const int c = min(c0 + u * XS_THREADS + tid, npiece - 1); const int tt = c / per_tok, rem = c - tt * per_tok; \
-                       r = *(const uint4 *)(kc + (size_t)(t0 + tt) * d + rem * 8); }
-        XS_EACH(XS_REQ)
-#undef XS_REQ
+    // the pieces in flight
+    xp_u4 kr[XS_NLD];
+    // piece u of a thread: token and place in it; the quotient by multiplication with 2^32 / per_tok rounded up, exact for the few thousand pieces there are
+    const uint32_t inv = 0xFFFFFFFFu / (uint32_t)per_tok + 1u;
+    auto pieces = [&](auto f) {
+        int c0 = tid;
+        asm volatile("" : "+v"(c0));                     // worked out again each time: kept over the dots they would not fit the registers
+#pragma unroll
+        for (int u = 0; u < XS_NLD; u++) {
+            const int c = c0 + u * XS_THREADS, tt = (int)__umulhi((uint32_t)c, inv);
+            f(u, tt, c - tt * per_tok);
+        }
     };
-    auto lay = [&](int npiece, int c0) {
-#define XS_LAY(u, r) { const int c = c0 + u * XS_THREADS + tid; \
-                       if (c < npiece) { const int tt = c / per_tok, rem = c - tt * per_tok, hh = rem >> 4, ch = rem & 15; \
-                                         s_k[(tt * n_head + hh) * 16 + ((ch + tt + 8 * (hh & 1)) & 15)] = r; } }
-        XS_EACH(XS_LAY)
-#undef XS_LAY
+    auto request = [&](int t0, int nt, int tb) {
+        pieces([&](int u, int tt, int rem) {
+            if (u < 5 || tb * per_tok + 5 * XS_THREADS < nt * per_tok) kr[u] = *(const xp_u4 *)(kc + (size_t)(t0 + min(tb + tt, nt - 1)) * d + rem * 8);
+        });
     };
-#undef XS_EACH
-    request(t_begin, min(XS_TOK, t_end - t_begin) * per_tok, 0);
-    for (int c = tid; c < per_tok; c += XS_THREADS) s_qh[c] = *(const uint4 *)(q16 + c * 8);
-    for (int t0 = t_begin; t0 < t_end; t0 += XS_TOK) {
-        const int nt = min(XS_TOK, t_end - t0), npiece = nt * per_tok;
-        if (t0 != t_begin) __syncthreads();             // the previous round's keys have been read
-        lay(npiece, 0);                                 // the first batch of the round was requested a round ahead
-        for (int c0 = XS_NLD * XS_THREADS; c0 < npiece; c0 += XS_NLD * XS_THREADS) { request(t0, npiece, c0); lay(npiece, c0); }
-        if (t0 + XS_TOK < t_end) request(t0 + XS_TOK, min(XS_TOK, t_end - t0 - XS_TOK) * per_tok, 0);
-        __syncthreads();
-        for (int key = tid; key < nt * n_head; key += XS_THREADS) {
+    // a workgroup with few keys: at most four pieces per thread, four threads per key
+    const int nt_all = t_end - t_begin;
+    const bool few = nt_all * n_head * 4 <= XS_THREADS && nt_all <= XS_TOK;
+    auto lay = [&](int nt, int tb) {
+        pieces([&](int u, int tt, int rem) {
+            const int t = tb + tt, hh = rem >> 4, ch = rem & 15;
+            if (t < nt) *(xp_u4 *)&s_k[(t * n_head + hh) * 16 + ((ch + t + 8 * (hh & 1)) & 15)] = kr[u];
+        });
+    };
+    // SP = 1: one thread walks a key; 4, where the workgroup's keys leave threads for it: four adjacent threads, thread `part` with the accumulators of
+    // j = part (one thread alone takes 1.6 us for its 128 elements).  No form between them: the kernels of a layer together fill the 64 KB
+    // instruction cache, and what does not fit costs every kernel 0.5 to 1 us.
+    auto dots = [&](auto sp, int t0, int nt) {
+        constexpr int SP = decltype(sp)::value, NJ = 4 / SP;
+        for (int base = 0; base < nt * n_head * SP; base += XS_THREADS) {
+            const int w = base + tid, key = w / SP, part = w % SP;
+            if (key >= nt * n_head) break;
             const int hh = key / nt, tt = key - hh * nt;
             const uint4 *kp = s_k + (tt * n_head + hh) * 16, *qp = s_qh + hh * 16;
             const int rot = tt + 8 * (hh & 1);
-            float sum[4][8];
+            float sum[NJ][8];
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int j = 0; j < NJ; j++)
 #pragma unroll
                 for (int l = 0; l < 8; l++) sum[j][l] = 0.0f;
 #pragma unroll
             for (int i = 0; i < 3; i++) {                // chunks of 32 elements = 4 x 16 bytes
                 __builtin_amdgcn_sched_barrier(0);      // one chunk's LDS reads at a time: the next round's keys occupy registers meanwhile
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const uint4 kv = kp[(4 * i + j + rot) & 15], qv = qp[4 * i + j];
+                for (int j = 0; j < NJ; j++) {
+                    const int jj = part + j * SP;
+                    const uint4 kv = kp[(4 * i + jj + rot) & 15], qv = qp[4 * i + jj];
                     const uint32_t kw[4] = {kv.x, kv.y, kv.z, kv.w}, qw[4] = {qv.x, qv.y, qv.z, qv.w};
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
@@ -614,10 +623,16 @@ __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_stat
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
+            auto other = [](float v, auto ctrl) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xF, 0xF, true)); };
+            // sum[0] += sum[2], sum[1] += sum[3]; sum[0] += sum[1]
 #pragma unroll
-            for (int l = 0; l < 8; l++) { sum[0][l] += sum[2][l]; sum[1][l] += sum[3][l]; }
-#pragma unroll
-            for (int l = 0; l < 8; l++) sum[0][l] += sum[1][l];
+            for (int l = 0; l < 8; l++) {
+                if constexpr (SP == 1) { sum[0][l] += sum[2][l]; sum[1][l] += sum[3][l]; sum[0][l] += sum[1][l]; }
+                else {
+                    sum[0][l] += other(sum[0][l], std::integral_constant<int, 0x4E>{});        // quad_perm [2, 3, 0, 1]
+                    sum[0][l] += other(sum[0][l], std::integral_constant<int, 0xB1>{});             // quad_perm [1, 0, 3, 2]
+                }
+            }
             const float u0 = sum[0][0] + sum[0][4], u1 = sum[0][1] + sum[0][5], u2 = sum[0][2] + sum[0][6], u3 = sum[0][3] + sum[0][7];
             const float v0 = u0 + u1, v1 = u2 + u3;
             const float simd = v0 + v1;
@@ -632,8 +647,30 @@ __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_stat
                     tail = fmaf(h2f((uint16_t)(kw[e] >> 16)), h2f((uint16_t)(qw[e] >> 16)), tail);
                 }
             }
-            scores[(size_t)hh * n_ctx + t0 + tt] = (tail + simd) * scale;
+            if (part == 0) scores[(size_t)hh * n_ctx + t0 + tt] = (tail + simd) * scale;
         }
+    };
+    constexpr int TB = XS_NLD * XS_THREADS;              // pieces per request of the workgroup
+    if (few) pieces([&](int u, int tt, int rem) { if (u < 4 && u * XS_THREADS < nt_all * per_tok) kr[u] = *(const xp_u4 *)(kc + (size_t)(t_begin + min(tt, nt_all - 1)) * d + rem * 8); });
+    else request(t_begin, min(XS_TOK, nt_all), 0);
+    for (int c = tid; c < per_tok; c += XS_THREADS) s_qh[c] = *(const uint4 *)(q16 + c * 8);
+    if (few) {
+        pieces([&](int u, int tt, int rem) {
+            const int hh = rem >> 4, ch = rem & 15;
+            if (u < 4 && tt < nt_all) *(xp_u4 *)&s_k[(tt * n_head + hh) * 16 + ((ch + tt + 8 * (hh & 1)) & 15)] = kr[u];
+        });
+        __syncthreads();
+        dots(std::integral_constant<int, 4>{}, t_begin, nt_all);
+        return;
+    }
+    for (int t0 = t_begin; t0 < t_end; t0 += XS_TOK) {
+        const int nt = min(XS_TOK, t_end - t0);
+        if (t0 != t_begin) __syncthreads();             // the previous round's keys have been read
+        lay(nt, 0);                                     // the first batch of the round was requested a round ahead
+        for (int tb = TB / per_tok; tb < nt; tb += TB / per_tok) { request(t0, nt, tb); lay(nt, tb); }
+        if (t0 + XS_TOK < t_end) request(t0 + XS_TOK, min(XS_TOK, t_end - t0 - XS_TOK), 0);
+        __syncthreads();
+        dots(std::integral_constant<int, 1>{}, t0, nt);
     }
 }
 
@@ -652,7 +689,7 @@ __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_stat
 static inline int xattn_pv_vstride(int n_ctx) { return ((n_ctx + 63) / 64) * 64 + 32; }        // halfs between rows in LDS: = 64 bytes mod 128, the two rows of a wave on different banks
 static inline size_t xattn_pv_lds(int n_ctx) {
     const size_t p_bytes = (size_t)((n_ctx + 32 + 7) & ~7) * 2, v_bytes = (size_t)16 * xattn_pv_vstride(n_ctx) * 2 + 1024;      // + the walk's read-ahead
-    const size_t soft = (size_t)n_ctx * 4 + (size_t)((n_ctx / 4 + 3) & ~3) * 4;                  // t / e and the group sums live where the rows go later
+    const size_t soft = (size_t)n_ctx * 4 + (size_t)(n_ctx / 4 + 31) / 32 * 160;                  // t / e and the group sums live where the rows go later
     return p_bytes + (v_bytes > soft ? v_bytes : soft);
 }
 template <int DUMMY>
@@ -664,7 +701,7 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
     XSTAMP(dbg, 0);
     const int n_kv = (st ? st->pos : pos_imm) + 1;
     const int hd_ = blockIdx.x >> 3, dgrp = blockIdx.x & 7;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int VS = ((n_ctx + 63) / 64) * 64 + 32;
     uint16_t *s_p = (uint16_t *)smem;                                 // n_ctx + 32 halfs: the probabilities as fp16
     uint8_t *region = smem + (size_t)((n_ctx + 32 + 7) & ~7) * 2;
@@ -677,6 +714,17 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
     float sreg[XP_NS];
 #pragma unroll
     for (int u = 0; u < XP_NS; u++) sreg[u] = srow[min(tid + u * XP_THREADS, n_ctx - 1)];
+    // The V^T rows: nothing beyond the last cached token is asked for.  Rows of up to 1024 tokens are on their way beside the scores; the
+    // pieces of longer ones would stand before the table gathers in the memory queue (4096 tokens 13.9 -> 14.1 us with four of eight ahead).
+    // vc is not a restrict pointer on purpose: the loads must stay where they are written.
+    xp_u4 vb[XP_NP];
+    const int last_piece = (n_kv - 1) >> 3;
+    auto load_row = [&]() {
+#pragma unroll
+        for (int i = 0; i < XP_NP; i++) if (i * 64 <= last_piece) vb[i] = *(const xp_u4 *)(vrow + (size_t)min(i * 64 + lane, last_piece) * 8);
+    };
+    const bool early = n_kv <= 1024;
+    if (early) load_row();
     float mx = -INFINITY;
 #pragma unroll
     for (int u = 0; u < XP_NS; u++) if (tid + u * XP_THREADS < n_kv) mx = fmaxf(mx, sreg[u]);
@@ -687,48 +735,35 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
 #pragma unroll
     for (int w = 1; w < 16; w++) mx = fmaxf(mx, s_red[w]);
     XSTAMP(dbg, 1);
-    // exponentials from the table
+    // exponentials from the table (a gather of 64 entries takes 64 cycles: only where there are scores)
 #pragma unroll
-    for (int u = 0; u < XP_NS; u++) sreg[u] = lut[f2h(sreg[u] - mx)];
+    for (int u = 0; u < XP_NS; u++) if (wave * 64 + u * XP_THREADS < n_kv) sreg[u] = lut[f2h(sreg[u] - mx)];
 #pragma unroll
     for (int u = 0; u < XP_NS; u++) { const int j = tid + u * XP_THREADS; if (j < n_kv) s_e[j] = sreg[u]; }
     __syncthreads();
     XSTAMP(dbg, 2);
     const int ngrp = n_kv / 4;
-    float grp[2];
     static_assert(XP_NS * XP_THREADS / 4 <= 2 * XP_THREADS, "two group sums per thread");
 #pragma unroll
     for (int u = 0; u < 2; u++) {
         const int g = tid + u * XP_THREADS;
-        grp[u] = 0.0f;
         if (g < ngrp) {
             const float4 v = *(const float4 *)(s_e + 4 * g);
             const float v1 = v.x + v.y, v2 = v.z + v.w;
-            grp[u] = v1 + v2;
-            s_grp[g] = grp[u];
+            s_grp[xg_seg_at(g)] = v1 + v2;
         }
     }
+    if (tid < 32) for (int g = ngrp + tid; g < ((ngrp + 31) & ~31); g += 32) s_grp[xg_seg_at(g)] = 0.0f;
     __syncthreads();
     XSTAMP(dbg, 3);
-    // The V^T rows are requested now, by every wave but the one that walks the sum (a wave that asks for its whole row sits in the
-    // issue stage until the memory queue has room, i.e. for most of the row's transfer time): the rows arrive while the sum is walked.
-    // vc is not a restrict pointer on purpose: the loads must stay between the two barriers around them.
-    uint4 vb0, vb1, vb2, vb3, vb4, vb5, vb6, vb7, vb8, vb9;
-    const int last_piece = (n_kv - 1) >> 3;
-    auto load_row = [&]() {
-        const uint16_t *vp = vrow;
-        vb0 = *(const uint4 *)(vp + (size_t)min(0 * 64 + lane, last_piece) * 8); vb1 = *(const uint4 *)(vp + (size_t)min(1 * 64 + lane, last_piece) * 8);
-        vb2 = *(const uint4 *)(vp + (size_t)min(2 * 64 + lane, last_piece) * 8); vb3 = *(const uint4 *)(vp + (size_t)min(3 * 64 + lane, last_piece) * 8);
-        vb4 = *(const uint4 *)(vp + (size_t)min(4 * 64 + lane, last_piece) * 8); vb5 = *(const uint4 *)(vp + (size_t)min(5 * 64 + lane, last_piece) * 8);
-        vb6 = *(const uint4 *)(vp + (size_t)min(6 * 64 + lane, last_piece) * 8); vb7 = *(const uint4 *)(vp + (size_t)min(7 * 64 + lane, last_piece) * 8);
-        vb8 = *(const uint4 *)(vp + (size_t)min(8 * 64 + lane, last_piece) * 8); vb9 = *(const uint4 *)(vp + (size_t)min(9 * 64 + lane, last_piece) * 8);
-    };
-    if (wave != 0) load_row();
+    // Longer rows are requested now, by every wave but the one that walks the sum (a wave that asks for its whole row sits in the issue stage
+    // until the memory queue has room, i.e. for most of the row's transfer time): they arrive while the sum is walked.
+    if (wave != 0) { if (!early) load_row(); }
     else {
-        float init = xg_serial_sum(s_grp, ngrp, 0.0f);
+        float init = xg_segment_sum<2>(s_grp, ngrp);
         for (int j = ngrp * 4; j < n_kv; j++) init = init + s_e[j];
         if (lane == 0) s_sum = init;
-        load_row();
+        if (!early) load_row();
     }
     __syncthreads();
     XSTAMP(dbg, 4);
@@ -738,16 +773,8 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
     // ---- the rows into LDS (s_e / s_grp are dead: every thread passed the barrier after the sum) ----
     {
         uint16_t *dst = s_v + (size_t)wave * VS + lane * 8;
-        if (0 * 64 + lane <= last_piece) *(uint4 *)(dst + 0 * 512) = vb0;
-        if (1 * 64 + lane <= last_piece) *(uint4 *)(dst + 1 * 512) = vb1;
-        if (2 * 64 + lane <= last_piece) *(uint4 *)(dst + 2 * 512) = vb2;
-        if (3 * 64 + lane <= last_piece) *(uint4 *)(dst + 3 * 512) = vb3;
-        if (4 * 64 + lane <= last_piece) *(uint4 *)(dst + 4 * 512) = vb4;
-        if (5 * 64 + lane <= last_piece) *(uint4 *)(dst + 5 * 512) = vb5;
-        if (6 * 64 + lane <= last_piece) *(uint4 *)(dst + 6 * 512) = vb6;
-        if (7 * 64 + lane <= last_piece) *(uint4 *)(dst + 7 * 512) = vb7;
-        if (8 * 64 + lane <= last_piece) *(uint4 *)(dst + 8 * 512) = vb8;
-        if (9 * 64 + lane <= last_piece) *(uint4 *)(dst + 9 * 512) = vb9;
+#pragma unroll
+        for (int i = 0; i < XP_NP; i++) if (i * 64 + lane <= last_piece) *(xp_u4 *)(dst + i * 512) = vb[i];
     }
     __syncthreads();
     XSTAMP(dbg, 5);
@@ -760,7 +787,10 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
         const _Float16 *vr = (const _Float16 *)s_v + (size_t)r16 * VS + cl, *pr = (const _Float16 *)s_p + cl;
         float acc = 0.0f;
         const int ntail = n_kv - 32 * nfull;                          // 1 .. 32
-        const float tprod = cl < ntail ? (float)vr[32 * nfull] * (float)pr[32 * nfull] : 0.0f;
+        // operands of the scalar tail, requested ahead of the walk (the 32 lanes of a row read the same addresses)
+        xp_u4 tv[4], tq[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) { tv[u] = *(const xp_u4 *)(vr - cl + 32 * nfull + 8 * u); tq[u] = *(const xp_u4 *)(pr - cl + 32 * nfull + 8 * u); }
         _Float16 va[8], pa[8], vb[8], pb[8];
         auto ld = [&](_Float16 (&v)[8], _Float16 (&q)[8], int i) {   // up to 16 chunks beyond nfull are read and not used: the next row, or the slack after the last
 #pragma unroll
@@ -787,21 +817,21 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
         }
         for (; i < nfull; i++) acc = fmaf((float)vr[32 * i], (float)pr[32 * i], acc);
         XSTAMP(dbg, 6);
-        acc += __shfl_xor(acc, 16, SPY_WAVE);         // sum[0] += sum[2], sum[1] += sum[3]
-        acc += __shfl_xor(acc, 8, SPY_WAVE);          // sum[0] += sum[1]
-        acc += __shfl_xor(acc, 4, SPY_WAVE);          // t_l = sum[0][l] + sum[0][l + 4]
-        acc += __shfl_xor(acc, 1, SPY_WAVE);          // t_0 + t_1, t_2 + t_3
-        acc += __shfl_xor(acc, 2, SPY_WAVE);          // (t_0 + t_1) + (t_2 + t_3)
-        // the scalar tail: elements 32 nfull .. n_kv - 1, one after the other.  A product of two fp16 values is exact in fp32, so
-        // `tail = fma(v, p, tail)` is `tail + v * p` with the product formed beforehand: lane cl forms the product of element
-        // 32 nfull + cl (operands read before the walk above), the 32 products are fetched with wave permutes that do not depend
-        // on each other, and what remains serial is one addition per element.
-        float tp[32];
-#pragma unroll
-        for (int e = 0; e < 32; e++) tp[e] = __shfl(tprod, (lane & 32) + e, SPY_WAVE);
+        // sum[0] += sum[2], sum[1] += sum[3] (lane ^ 16); sum[0] += sum[1] (^ 8); t_l = sum[0][l] + sum[0][l + 4] (^ 4); t_0 + t_1, t_2 + t_3 (^ 1);
+        // (t_0 + t_1) + (t_2 + t_3) (^ 2); inside a row of 16 as rotations where the values are periodic already
+        const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc), __float_as_uint(acc), false, false);
+        acc = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+#define XP_ADD(CTRL) acc += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc), CTRL, 0xF, 0xF, true));
+        XP_ADD(0x128) XP_ADD(0x124) XP_ADD(0xB1) XP_ADD(0x4E)
+#undef XP_ADD
+        // the scalar tail: elements 32 nfull .. n_kv - 1, one after the other (a product of two fp16 values is exact in fp32: the fma is
+        // `tail + v * p`)
         float tail = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 32; e++) if (e < ntail) tail = tail + tp[e];
+        for (int e = 0; e < 32; e++) {
+            const uint32_t wv = tv[e >> 3][(e >> 1) & 3], wq = tq[e >> 3][(e >> 1) & 3];
+            if (e < ntail) tail = fmaf(h2f((uint16_t)(e & 1 ? wv >> 16 : wv & 0xFFFFu)), h2f((uint16_t)(e & 1 ? wq >> 16 : wq & 0xFFFFu)), tail);
+        }
         if (cl == 0) attn_out[hd_ * 128 + dgrp * 16 + r16] = tail + acc;
         XSTAMP(dbg, 7);
     }

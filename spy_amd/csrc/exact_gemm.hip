@@ -72,8 +72,8 @@ struct xt_args {
 
 // AS: waves that share the accumulators of a tile (2 or 4); RG: groups of 16 weight rows per workgroup; C: groups of 16 activation rows per
 // wave; NXS, NWC: LDS slots for stages and chunks (powers of two); P: stages requested ahead
-template <int WT, int AS, int RG, int C, int NXS, int P, int NWC, int OCC>
-__global__ __launch_bounds__(64 * AS * RG, OCC) void xt_kernel(xt_args a) {
+template <int WT, int AS, int RG, int C, int NXS, int P, int NWC>
+__device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
     constexpr int NT = 64 * AS * RG, ROWS = 16 * RG;
     constexpr int CU = xt_w<WT>::CU, UW = ROWS * CU, NI = (UW + NT - 1) / NT, NXI = C * 256 / NT;
     constexpr int XB = C * (XT_XB + 256), WB = (UW + 63) / 64 * 1024;
@@ -81,7 +81,7 @@ __global__ __launch_bounds__(64 * AS * RG, OCC) void xt_kernel(xt_args a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = wave % AS, rg = wave / AS, q = lane >> 4, r = lane & 15;
-    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS, cg0 = (int)blockIdx.y * C;
+    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS;
     const int nst = a.nst, ncg = a.ncg, M = a.M;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
 
@@ -272,6 +272,17 @@ __global__ __launch_bounds__(64 * AS * RG, OCC) void xt_kernel(xt_args a) {
     }
 }
 
+template <int WT, int AS, int RG, int C, int NXS, int P, int NWC, int OCC>
+__global__ __launch_bounds__(64 * AS * RG, OCC) void xt_kernel(xt_args a) { xt_tile<WT, AS, RG, C, NXS, P, NWC>(a, (int)blockIdx.y * C); }
+// Tiles of four activation groups and, behind them in the grid, one of the R groups that remain: the sums of groups that do not exist cost as much
+// as those of groups that do (22016 x 4096 Q4_0: 77 rows 98 -> 85 us, 140 rows 161 -> 135, 200 rows 224 -> 188, 900 rows 831 -> 796)
+template <int WT, int R>
+__global__ __launch_bounds__(256, 3) void xt_mixed_kernel(xt_args a) {
+    const int full = a.ncg / 4;
+    if ((int)blockIdx.y < full) xt_tile<WT, 2, 2, 4, 2, 1, 2>(a, (int)blockIdx.y * 4);
+    else xt_tile<WT, 2, 2, R, R < 3 ? 4 : 2, R < 3 ? 2 : 1, 2>(a, full * 4);
+}
+
 // f32 rows -> packed activations: Quantizator<FP32,Q8_0>::transform (vec_convert.h:178-261), as quantize_q8_0_kernel, the quants as fp16.
 // Rows past T become zeros.  8 lanes per block; a workgroup takes 16 rows and two blocks.
 __global__ __launch_bounds__(256) void xt_pack_kernel(const uint8_t *__restrict__ x, int64_t x_stride, int T, int nst, uint8_t *__restrict__ xq, uint8_t *__restrict__ xd) {
@@ -427,12 +438,22 @@ __global__ __launch_bounds__(256) void xt_silu_pack_kernel(const float *__restri
     xt_store8(y, sub, xq + ((int64_t)cg * nst + blockIdx.x) * XT_XB + bl * 1024, xd + ((int64_t)cg * nst + blockIdx.x) * XT_XD + bl * 64, row);
 }
 
-template <int WT, int AS, int RG, int C, int NXS, int P, int NWC, int OCC>
-int xt_launch(hipStream_t st, xt_args a, int nmat) {
+template <int WT, int AS, int RG, int C, int NXS, int NWC> constexpr size_t xt_lds() {
     constexpr size_t ring = NXS * C * (XT_XB + 256) + NWC * ((16 * RG * xt_w<WT>::CU + 63) / 64) * 1024 + 1024, ex = (size_t)RG * (AS - 1) * C * (32 / AS) * 256, lds = ring > ex ? ring : ex;
     static_assert(lds <= 64 * 1024, "no raised LDS limit");
+    return lds;
+}
+template <int WT, int AS, int RG, int C, int NXS, int P, int NWC, int OCC>
+int xt_launch(hipStream_t st, xt_args a, int nmat) {
     a.tiles = (a.M + 16 * RG - 1) / (16 * RG);
-    xt_kernel<WT, AS, RG, C, NXS, P, NWC, OCC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * AS * RG), lds, st>>>(a);
+    xt_kernel<WT, AS, RG, C, NXS, P, NWC, OCC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * AS * RG), xt_lds<WT, AS, RG, C, NXS, NWC>(), st>>>(a);
+    return SPY_LAUNCH_RC();
+}
+template <int WT, int R>
+int xt_launch_mixed(hipStream_t st, xt_args a, int nmat) {
+    a.tiles = (a.M + 31) / 32;
+    constexpr size_t l4 = xt_lds<WT, 2, 2, 4, 2, 2>(), lr = xt_lds<WT, 2, 2, R, R < 3 ? 4 : 2, 2>();
+    xt_mixed_kernel<WT, R><<<dim3((unsigned)(a.tiles * nmat), (unsigned)(a.ncg / 4 + 1)), dim3(256), l4 > lr ? l4 : lr, st>>>(a);
     return SPY_LAUNCH_RC();
 }
 
@@ -936,26 +957,31 @@ int xt_num_cu() {
 // Which tile.  n workgroups per compute unit take about lat + (n - 1) * inc: figures in tenths of a microsecond for K = 4096, measured for
 // n = 1 .. 16 (whole workgroups count while they are few; everything scales with K).  Small tiles have the shorter chain, large ones unpack a
 // weight for more activation rows.
-struct xt_cost { int rows, groups, lat, inc; };
+// rest: what a workgroup of the ncg % groups groups that remain takes, 0 if it is a whole one.
+struct xt_cost { int rows, groups, lat, inc, rest = 0; };
 int xt_pick(const xt_args &a, int nmat, const xt_cost *c, int n) {
     const int64_t cu = xt_num_cu();
     int best = 0;
     int64_t least = 0;
     for (int i = 0; i < n; i++) {
-        const int64_t wgs = (int64_t)((a.M + c[i].rows - 1) / c[i].rows) * nmat * ((a.ncg + c[i].groups - 1) / c[i].groups);
-        const int64_t t = c[i].lat + (wgs <= 6 * cu ? (wgs + cu - 1) / cu * 10 - 10 : 10 * wgs / cu - 10) * c[i].inc / 10;
+        const int64_t tiles = (int64_t)((a.M + c[i].rows - 1) / c[i].rows) * nmat, wgs = tiles * (c[i].rest ? a.ncg / c[i].groups : (a.ncg + c[i].groups - 1) / c[i].groups);
+        const int64_t t = c[i].lat + (wgs <= 6 * cu && !c[i].rest ? (wgs + cu - 1) / cu * 10 - 10 : 10 * wgs / cu - 10) * c[i].inc / 10 + tiles * c[i].rest / cu;
         if (!i || t < least) { best = i; least = t; }
     }
     return best;
 }
 template <int WT>
 int xt_dispatch(hipStream_t st, const xt_args &a, int nmat) {
-    static const xt_cost c[4] = {{16, 1, 86, 43}, {32, 1, 103, 56}, {32, 2, 173, 96}, {32, 4, 288, 165}};
-    switch (xt_pick(a, nmat, c, 4)) {
+    // the last one: tiles of four groups and one of what remains, where something remains
+    static const int of_rest[4] = {0, 60, 100, 132};
+    const int rest = a.ncg > 4 ? a.ncg % 4 : 0;
+    const xt_cost c[5] = {{16, 1, 86, 43}, {32, 1, 103, 56}, {32, 2, 173, 96}, {32, 4, 288, 165}, {32, 4, 288, 165, of_rest[rest]}};
+    switch (xt_pick(a, nmat, c, rest ? 5 : 4)) {
     case 0: return xt_launch<WT, 4, 1, 1, 8, 6, 4, 2>(st, a, nmat);
     case 1: return xt_launch<WT, 2, 2, 1, 4, 2, 2, 3>(st, a, nmat);
     case 2: return xt_launch<WT, 2, 2, 2, 4, 2, 2, 3>(st, a, nmat);
-    default: return xt_launch<WT, 2, 2, 4, 2, 1, 2, 3>(st, a, nmat);
+    case 3: return xt_launch<WT, 2, 2, 4, 2, 1, 2, 3>(st, a, nmat);
+    default: return rest == 1 ? xt_launch_mixed<WT, 1>(st, a, nmat) : rest == 2 ? xt_launch_mixed<WT, 2>(st, a, nmat) : xt_launch_mixed<WT, 3>(st, a, nmat);
     }
 }
 template <int WT>

@@ -18,6 +18,7 @@
 // Measured against what these kernels replaced (operands packed as fp16 once per call, 64 x 64 tiles), packing included:
 // 4096 x 4096 Q4_0: 16 rows 80 -> 15 us, 77 rows 104 -> 28, 512 rows 137 -> 88, 2048 rows 400 -> 313; 8 rows (one launch per row) 36 -> 15.
 #include "common.cuh"
+#include "exact_sum.cuh"
 
 #include <type_traits>
 #include <utility>
@@ -340,13 +341,12 @@ __device__ __forceinline__ void xt_store8(const float (&y)[8], int sub, uint8_t 
 }
 
 // NormRMS (non-linear.cpp:194-223) -> Mul by the norm weights -> packed activations; one workgroup per row.  The sum of squares is the host's
-// std::transform_reduce: groups of four, (x0^2 + x1^2) + (x2^2 + x3^2), added to one running sum, which one wave walks; that chain (K / 4
-// additions of 4.3 ns) is most of the kernel.  Rows past T of the last group are written as zeros.  OWN: the sum in this backend's own order, by the thread
-// pattern of norm_rms_kernel.
+// std::transform_reduce: groups of four, (x0^2 + x1^2) + (x2^2 + x3^2), added to one running sum (xg_segment_sum).  Rows past T of the last
+// group are written as zeros.  OWN: the sum in this backend's own order, by the thread pattern of norm_rms_kernel, from a copy of the row in LDS.
 template <int NV, bool OWN>        // K <= 2048 * NV
 __global__ __launch_bounds__(256) void xt_norm_pack_kernel(const float *__restrict__ x, const float *__restrict__ w, float eps, int K, int T, int nst,
                                                            uint8_t *__restrict__ xq, uint8_t *__restrict__ xd) {
-    __shared__ __align__(16) float g[512 * NV + 32];
+    __shared__ __align__(16) float g[OWN ? 2048 * NV : 640 * NV];      // OWN: the row; else the group sums as xg_segment_sum reads them
     __shared__ float s_sum;
     const int tid = threadIdx.x, t = blockIdx.x, cg = t >> 4, row = t & 15, n8 = K / 8;
     const float4 *xr = (const float4 *)(x + (int64_t)min(t, T - 1) * K);
@@ -360,42 +360,29 @@ __global__ __launch_bounds__(256) void xt_norm_pack_kernel(const float *__restri
     for (int j = 0; j < NV; j++) {
         const int i = min(j * 256 + tid, n8 - 1);
         wv[j][0] = ((const float4 *)w)[2 * i]; wv[j][1] = ((const float4 *)w)[2 * i + 1];
-        if (!OWN && j * 256 + tid < n8) {
+        if (j * 256 + tid < n8) {
 #pragma unroll
             for (int k = 0; k < 2; k++) {
                 const float4 z = v[j][k];
-                const float a0 = z.x * z.x, a1 = z.y * z.y, a2 = z.z * z.z, a3 = z.w * z.w, v1 = a0 + a1, v2 = a2 + a3;
-                g[2 * i + k] = v1 + v2;
+                if constexpr (OWN) ((float4 *)g)[2 * i + k] = z;
+                else {
+                    const float a0 = z.x * z.x, a1 = z.y * z.y, a2 = z.z * z.z, a3 = z.w * z.w, v1 = a0 + a1, v2 = a2 + a3;
+                    g[xg_seg_at(2 * i + k)] = v1 + v2;               // K / 4 is a multiple of 64: no segment is left open
+                }
             }
         }
-    }
-    if (OWN) {
-        float acc = 0.0f;
-        for (int i = tid; i < K; i += 256) { const float e = ((const float *)xr)[i]; acc = fmaf(e, e, acc); }
-        acc = wave_sum(acc);
-        if ((tid & 63) == 0) g[tid >> 6] = acc;
     }
     __syncthreads();
-    if (OWN) {
-        if (tid == 0) s_sum = (g[0] + g[1]) + (g[2] + g[3]);
-    } else if (tid < 64) {      // eight group sums per step, requested three steps (24 additions, about the latency of an LDS read) ahead; K / 4 is a multiple of 32
-        const float4 *p = (const float4 *)g;
-        float4 r[4][2];
-        float sum = 0.0f;
-        auto ld = [&](int k, int i) { r[k][0] = p[2 * i]; r[k][1] = p[2 * i + 1]; };                   // up to 24 floats past the row's sums: not added
-#pragma unroll
-        for (int k = 0; k < 3; k++) ld(k, k);
-        for (int i = 0; i < K / 32; i += 4) {
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                ld((k + 3) & 3, i + k + 3);
-                __builtin_amdgcn_sched_barrier(0);
-                const float4 a = r[k][0], c = r[k][1];
-                sum = sum + a.x; sum = sum + a.y; sum = sum + a.z; sum = sum + a.w;
-                sum = sum + c.x; sum = sum + c.y; sum = sum + c.z; sum = sum + c.w;
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
+    if constexpr (OWN) {
+        __shared__ float part[4];
+        float acc = 0.0f;
+        for (int i = tid; i < K; i += 256) acc = fmaf(g[i], g[i], acc);
+        acc = wave_sum(acc);
+        if ((tid & 63) == 0) part[tid >> 6] = acc;
+        __syncthreads();
+        if (tid == 0) s_sum = (part[0] + part[1]) + (part[2] + part[3]);
+    } else if (tid < 64) {
+        const float sum = xg_segment_sum<NV / 2>(g, K / 4);
         if (tid == 0) s_sum = sum;
     }
     __syncthreads();

@@ -13,6 +13,7 @@
 // Values that cannot occur are not looked after: the fp16 caches are written by this library's float -> half
 // conversion, which never produces the pattern 0xFFFF that the host's conversion table maps to 0 (conversion.h:39-41).
 #include "common.cuh"
+#include "exact_sum.cuh"
 
 namespace {
 
@@ -191,85 +192,104 @@ __global__ __launch_bounds__(256, 2) void xp_scores_kernel(const void *__restric
 }
 
 // ---------------------------------------------------------------- softmax
-// One workgroup per (head, query row); L = the positions the row may see.  A thread keeps its share of the row in registers
-// (groups of four consecutive elements, the unit of the host's sum), so the row is read once and written once.  The
-// probabilities leave as fp16 (the first step of the KQV MatMul, mat.cpp:37), followed by zeros up to the end of the 32-row
-// tile's last chunk, which the product kernel reads.
-#define XP_SM_R 8          // groups per thread: rows of up to 8192 positions
-__global__ __launch_bounds__(256) void xp_softmax_kernel(const float *__restrict__ S, uint16_t *__restrict__ P16, const float *__restrict__ lut, int T, int P,
-                                                         int64_t s_row, int n_total, float scale) {
-    __shared__ __align__(16) float s_grp[256 * XP_SM_R];
-    __shared__ float s_part[4], s_rem[4];
-    __shared__ float s_out;
-    const int t = blockIdx.x, h = blockIdx.y;
-    const float4 *s4 = (const float4 *)(S + ((int64_t)h * T + t) * s_row);
-    uint16_t *p = P16 + ((int64_t)h * T + t) * s_row;
-    const int L = P + t + 1, ng_row = (L + 3) / 4;       // groups that hold an element of the row
-    float v[XP_SM_R][4];
-    float mx = -INFINITY;
+// One wave per (head, query row), NW waves per resident workgroup, rows dealt out in turn (the longest first); L = the positions the row may see.  A
+// lane keeps its share of the row in registers (groups of four consecutive elements, the unit of the host's sum), so the row is read once
+// and written once.  The probabilities leave as fp16 (the first step of the KQV MatMul, mat.cpp:37), followed by zeros up to the end of the
+// 32-row tile's last chunk, which the product kernel reads.
+// The exponentials: a gather of 64 table entries from memory takes about 64 cycles of the compute unit, so the part of the table that is not zero lies in
+// LDS: arguments are <= 0 (or NaN), and exp is 0 from -104 on.  The sum of a row goes through xg_segment_sum: 2 us instead of a chain of up to
+// 1024 additions.  2048 rows of 2049 .. 4096 positions and 32 heads (1.2 GB): 462 -> 306 us; 2048 rows of 1 .. 2048: 193 -> 152.
+#define XP_LUT 0x5680      // fp16 -104.0 without its sign
+#define XP_SM_R 32         // groups per lane: rows of up to 8192 positions
+template <int R, int NW>
+__global__ __launch_bounds__(64 * NW) void xp_softmax_kernel(const float *__restrict__ S, uint16_t *__restrict__ P16, const float *__restrict__ lut, int T, int H, int P,
+                                                             int64_t s_row, int n_total, float scale) {
+    extern __shared__ __align__(16) float s_mem[];               // table, then per wave 64 R padded group sums and 4 floats
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float *s_grp = s_mem + XP_LUT + 4 + wave * (80 * R + 4), *s_rem = s_grp + 80 * R;
+    for (int i = threadIdx.x; i <= XP_LUT / 4; i += 64 * NW) ((float4 *)s_mem)[i] = ((const float4 *)(lut + 0x8000))[i];
+    __syncthreads();
+    const int rows = T * H;
+    for (int id = (int)blockIdx.x * NW + wave; id < rows; id += (int)gridDim.x * NW) {
+        const int t = T - 1 - id / H, h = id % H;
+        const float4 *s4 = (const float4 *)(S + ((int64_t)h * T + t) * s_row);
+        const int L = P + t + 1, ng_row = (L + 3) / 4;           // groups that hold an element of the row
+        float4 v[R];
+        float mx = -INFINITY;
+        // blocks of 64 groups: whole ones, and the one in which the row ends (elements past L: -inf, which leaves 0)
 #pragma unroll
-    for (int r = 0; r < XP_SM_R; r++) {
-        const int g = threadIdx.x + 256 * r;
-        if (g < ng_row) {
-            const float4 f = s4[g];
-            const float e[4] = {f.x, f.y, f.z, f.w};
+        for (int r = 0; r < R; r++) if (64 * r < ng_row) v[r] = s4[min(lane + 64 * r, ng_row - 1)];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                float x = e[k] + 0.0f;                   // + the mask value of an allowed position
-                x = x * scale;
-                v[r][k] = x;
-                if (4 * g + k < L) mx = fmaxf(mx, x);
+        for (int r = 0; r < R; r++)
+            if (64 * r < ng_row) {
+                float e[4] = {v[r].x * scale, v[r].y * scale, v[r].z * scale, v[r].w * scale};      // (+ the mask value 0 of an allowed position: nothing but the sign of a zero)
+                if (256 * (r + 1) > L) {
+#pragma unroll
+                    for (int k = 0; k < 4; k++) e[k] = 4 * (lane + 64 * r) + k < L ? e[k] : -INFINITY;
+                }
+                mx = fmaxf(fmaxf(fmaxf(mx, e[0]), fmaxf(e[1], e[2])), e[3]);
+                v[r] = make_float4(e[0], e[1], e[2], e[3]);
             }
-        }
-    }
-    mx = wave_max(mx);
-    if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(s_part[0], s_part[1]), fmaxf(s_part[2], s_part[3]));
-    // std::reduce in libstdc++: groups of four as init + ((a0 + a1) + (a2 + a3)) over the first n_total / 4 * 4 elements, the rest one
-    // by one; groups and elements past L are zeros and leave the sum as it is
-    const int ng_sum = min(n_total / 4, ng_row);
+        mx = wave_max(mx);
+        // std::reduce in libstdc++: groups of four as init + ((a0 + a1) + (a2 + a3)) over the first n_total / 4 * 4 elements, the rest one
+        // by one; groups and elements past L are zeros and leave the sum as it is
+        const int ng_sum = min(n_total / 4, ng_row);
+        if ((ng_sum & 31) && lane < 32) s_grp[xg_seg_at((ng_sum & ~31) + lane)] = 0.0f;       // an open last segment
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int r = 0; r < XP_SM_R; r++) {
-        const int g = threadIdx.x + 256 * r;
-        if (g < ng_row) {
+        for (int r = 0; r < R; r++)
+            if (64 * r < ng_row) {
+                float e[4] = {v[r].x, v[r].y, v[r].z, v[r].w};
+                uint32_t hx[4];
 #pragma unroll
-            for (int k = 0; k < 4; k++) v[r][k] = 4 * g + k < L ? lut[f2h(v[r][k] - mx)] : 0.0f;
-            const float v1 = v[r][0] + v[r][1], v2 = v[r][2] + v[r][3];
-            if (g < ng_sum) s_grp[g] = v1 + v2;
-            else {                                       // the group that n_total cuts short: its elements are added one by one
+                for (int k = 0; k < 4; k++) hx[k] = f2h(mx - e[k]);          // the argument without its sign
 #pragma unroll
-                for (int k = 0; k < 4; k++) s_rem[k] = v[r][k];
+                for (int k = 0; k < 4; k++) e[k] = s_mem[min(hx[k], (uint32_t)XP_LUT)];      // entry XP_LUT: 0, exp of everything below
+                if (__any(max(max(hx[0], hx[1]), max(hx[2], hx[3])) > 0x7C00u)) {            // a NaN somewhere
+                    const float w[4] = {v[r].x, v[r].y, v[r].z, v[r].w};
+#pragma unroll
+                    for (int k = 0; k < 4; k++) if (hx[k] > 0x7C00u && 4 * (lane + 64 * r) + k < L) e[k] = lut[f2h(w[k] - mx)];
+                }
+                v[r] = make_float4(e[0], e[1], e[2], e[3]);
+                const int g = lane + 64 * r;
+                const float v1 = e[0] + e[1], v2 = e[2] + e[3];
+                if (g < ng_sum) s_grp[xg_seg_at(g)] = v1 + v2;
+                if (g == ng_sum) { s_rem[0] = e[0]; s_rem[1] = e[1]; s_rem[2] = e[2]; s_rem[3] = e[3]; }      // the group that n_total cuts short: its elements are added one by one
             }
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float init = 0.0f;
-        int g = 0;
-        for (; g + 4 <= ng_sum; g += 4) {
-            const float4 a = *(const float4 *)&s_grp[g];
-            init = init + a.x; init = init + a.y; init = init + a.z; init = init + a.w;
-        }
-        for (; g < ng_sum; g++) init = init + s_grp[g];
-        for (int i = n_total / 4 * 4; i < min(n_total, L); i++) init = init + s_rem[i & 3];
-        s_out = init;
-    }
-    __syncthreads();
-    const float inv = 1.0f / s_out;
-    const int zend = (int)min((int64_t)((P + (t | 31) + 1 + 31) & ~31), s_row);       // a multiple of 32
-    uint2 *p4 = (uint2 *)p;
+        __builtin_amdgcn_wave_barrier();
+        float sum = xg_segment_sum<(R + 15) / 16>(s_grp, ng_sum);
+        for (int i = n_total / 4 * 4; i < min(n_total, L); i++) sum = sum + s_rem[i & 3];
+        const float inv = 1.0f / sum;
+        uint2 *p4 = (uint2 *)(P16 + ((int64_t)h * T + t) * s_row);
+        const int zend = (int)min((int64_t)((P + (t | 31) + 1 + 31) & ~31), s_row);       // a multiple of 32
 #pragma unroll
-    for (int r = 0; r < XP_SM_R; r++) {
-        const int g = threadIdx.x + 256 * r;
-        if (g < ng_row) {
-            uint16_t o[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) o[k] = 4 * g + k < L ? f2h(v[r][k] * inv) : (uint16_t)0;
-            p4[g] = make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
-        }
+        for (int r = 0; r < R; r++)
+            if (64 * r < ng_row) {
+                const int g = lane + 64 * r;
+                if (g < ng_row)                                  // elements past L are zeros
+                    p4[g] = make_uint2((uint32_t)f2h(v[r].x * inv) | ((uint32_t)f2h(v[r].y * inv) << 16), (uint32_t)f2h(v[r].z * inv) | ((uint32_t)f2h(v[r].w * inv) << 16));
+            }
+        for (int g = ng_row + lane; g < zend / 4; g += 64) p4[g] = make_uint2(0, 0);
+        __builtin_amdgcn_wave_barrier();
     }
-    for (int g = ng_row + threadIdx.x; g < zend / 4; g += 256) p4[g] = make_uint2(0, 0);
+}
+int xp_num_cu() {
+    static int n = 0;                              // the same value whoever writes it
+    if (!n) {
+        int dev = 0, v = 0;
+        n = hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0 ? v : 256;
+    }
+    return n;
+}
+template <int R, int NW>
+int xp_softmax_launch(hipStream_t st, const float *S, uint16_t *P16, const float *lut, int T, int H, int P, int64_t s_row, int n_total, float scale, int ncu) {
+    constexpr size_t lds = (XP_LUT + 4 + NW * (80 * R + 4)) * 4;
+    static_assert(lds <= 160 * 1024, "");
+    const int rc = spy_raise_lds_limit((const void *)xp_softmax_kernel<R, NW>, lds);
+    if (rc) return rc;
+    const int64_t need = ((int64_t)T * H + NW - 1) / NW;
+    xp_softmax_kernel<R, NW><<<dim3((unsigned)(need < ncu ? need : ncu)), dim3(64 * NW), lds, st>>>(S, P16, lut, T, H, P, s_row, n_total, scale);
+    return SPY_LAUNCH_RC();
 }
 
 // ---------------------------------------------------------------- product with V^T
@@ -425,7 +445,7 @@ int64_t spy_exact_prompt_attn_row(int64_t n_kv) { return (n_kv + 127) & ~(int64_
 int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, float *out, const float *lut,
                           int T, int H, int P, int64_t C, int n_total, float scale) {
     if (T <= 0 || H <= 0 || H > 65535 || P < 0 || (int64_t)P + T > C || n_total < P + T || n_total > C || C % 32) return SPY_HIP_EINVAL;
-    if ((int64_t)P + T > 1024 * XP_SM_R) return SPY_HIP_EUNSUPPORTED;      // the softmax kernel keeps a row in the registers of 256 threads
+    if ((int64_t)P + T > 256 * XP_SM_R) return SPY_HIP_EUNSUPPORTED;      // the softmax kernel keeps a row in the registers of a wave
     if (((uintptr_t)q & 15) || ((uintptr_t)kc & 15) || ((uintptr_t)S & 15) || ((uintptr_t)P16 & 7) || ((uintptr_t)out & 15)) return SPY_HIP_EINVAL;
     const int64_t s_row = spy_exact_prompt_attn_row((int64_t)P + T);
     // segments of the cached positions: 512 long where that fills the chip, down to one key tile for short passes (77 tokens on 1000 cached ones
@@ -440,8 +460,10 @@ int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint1
     else if (one) xp_scores_kernel<false, true><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
     else xp_scores_kernel<false, false><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
     if (hipGetLastError() != hipSuccess) return SPY_HIP_EINVAL;
-    xp_softmax_kernel<<<dim3((unsigned)T, (unsigned)H), dim3(256), 0, st>>>(S, P16, lut, T, P, s_row, n_total, scale);
-    if (hipGetLastError() != hipSuccess) return SPY_HIP_EINVAL;
+    const int ncu = xp_num_cu(), rc = (int64_t)P + T <= 4096 ? xp_softmax_launch<16, 12>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
+                                         : (int64_t)P + T <= 6144 ? xp_softmax_launch<24, 8>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
+                                                                  : xp_softmax_launch<32, 4>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu);
+    if (rc) return rc;
     xp_pv_kernel<<<dim3((unsigned)H, 4, (unsigned)((T + XP_PT - 1) / XP_PT)), dim3(256), 0, st>>>(P16, vt, out, T, H, P, s_row, C, n_total);
     return SPY_LAUNCH_RC();
 }

@@ -260,6 +260,41 @@ def test_exact_prompt_attention_bits(hip, oracle, H_, past, T, n_ctx, cuts):
     assert L.spy_hip_prompt_attention_exact(None, dq.ptr, dk.ptr, dv.ptr, out.ptr, T, H_, hd, past, n_ctx, n_kv, scale, sc.ptr, 1024) == hip.ENOSPACE
 
 
+@pytest.mark.parametrize("H_,past,T,n_ctx,spread", [
+    (2, 4032, 64, 4096, 1.0),                 # the longest row of sixteen groups per lane, 1024 group sums
+    (1, 5000, 40, 5056, 1.0), (1, 6130, 30, 6176, 1.0), (1, 8170, 22, 8192, 1.0),      # the wider forms and their edges (6144, 8192)
+    (32, 100, 120, 256, 1.0),                 # more rows than waves
+    (4, 10, 70, 96, 60.0),                    # scores more than 104 below the largest: exp is 0
+    (2, 10, 70, 96, 3000.0),                    # one position takes all
+])
+def test_exact_prompt_softmax_forms(hip, oracle, H_, past, T, n_ctx, spread):
+    """The softmax of the causal attention kernels at the edges of its row lengths and of its table of exponentials."""
+    from tests.gpu_util import dev, dev_empty, call
+    hd, n_kv = 128, past + T
+    d = H_ * hd
+    rng = np.random.default_rng(T + past)
+    scale = float(1.0 / np.sqrt(hd))
+    q = (rng.standard_normal((T, H_, hd)) * spread).astype(np.float32)
+    kc, vc = np.zeros((n_ctx, d), np.float16), np.zeros((d, n_ctx), np.float16)
+    kc[:n_kv] = rng.standard_normal((n_kv, d)).astype(np.float16)
+    vc[:, :n_kv] = rng.standard_normal((d, n_kv)).astype(np.float16)
+    mask = np.where(np.arange(n_ctx)[None, :] <= (np.arange(T)[:, None] + past), 0.0, -np.inf).astype(np.float32)
+    S_o, P_o = np.zeros((H_, T, n_kv), np.float32), np.zeros((H_, T, n_kv), np.float32)
+    O_o = np.zeros((H_, T, hd), np.float32)
+    assert oracle.spy_o_matmul(B(O.tensor(kc.view(np.uint16), O.F16, [hd, n_kv, H_], nb=[2, 2 * d, 2 * hd])),
+                               B(O.tensor(q, O.F32, [hd, T, H_], nb=[4, 4 * d, 4 * hd])), B(O.tensor(S_o, O.F32, [n_kv, T, H_])), 8) == 0
+    assert oracle.spy_o_softmax(B(O.tensor(S_o, O.F32, [n_kv, T, H_])), B(O.tensor(mask, O.I32, [n_ctx, T])), B(O.tensor(P_o, O.F32, [n_kv, T, H_])), scale) == 0
+    assert oracle.spy_o_matmul(B(O.tensor(vc.view(np.uint16), O.F16, [n_kv, hd, H_], nb=[2, 2 * n_ctx, 2 * n_ctx * hd])),
+                               B(O.tensor(P_o, O.F32, [n_kv, T, H_])), B(O.tensor(O_o, O.F32, [hd, T, H_])), 8) == 0
+    want = np.ascontiguousarray(O_o.transpose(1, 0, 2)).reshape(T, d)
+    L = hip.load()
+    need = L.spy_hip_prompt_attention_exact_scratch_size(T, H_, past)
+    sc, out = dev_empty(need, 0xFF), dev_empty(T * d * 4, 0xFF)
+    dq, dk, dv = dev(q), dev(kc.view(np.uint16)), dev(vc.view(np.uint16))
+    call(L.spy_hip_prompt_attention_exact, None, dq.ptr, dk.ptr, dv.ptr, out.ptr, T, H_, hd, past, n_ctx, n_kv, scale, sc.ptr, need)
+    _same_bits(out.download(np.float32).reshape(T, d), want, "attention H %d past %d T %d spread %g" % (H_, past, T, spread))
+
+
 def test_norm_softmax_silu_rope_bits(hip, oracle):
     from tests.gpu_util import dev, dev_empty, call
     L = hip.load()

@@ -277,39 +277,41 @@ template <int WT, int NIT> struct wtile { uint32_t w[NIT][wt_traits<WT>::PAIR_DW
 // wait for "all but the N youngest" loads when those N are issued unconditionally.  Lanes whose
 // pair index lies beyond the row re-read the last pair (a cache hit that dot_tile ignores).
 template <int WT, int LPR, int NIT>
-static __device__ __forceinline__ void load_tile(wtile<WT, NIT> &t, const uint8_t *__restrict__ rowp, int npair, int l) {
+static __device__ __forceinline__ void load_slab(wtile<WT, NIT> &t, const uint8_t *__restrict__ rowp, int npair, int l, int it) {
     constexpr int DW = wt_traits<WT>::PAIR_DW;
+    const int p = min(it * LPR + l, npair - 1);
+    if constexpr (WT == SPY_HIP_Q4_K) {
+        static_assert(WT != SPY_HIP_Q4_K || LPR == 64, "K-quant tiles use 64 lanes per row");
+        const uint8_t *sb = rowp + (size_t)(p >> 2) * 144;
+        const uint4 hdr = *(const uint4 *)sb, q0 = *(const uint4 *)(sb + 16 + 32 * (p & 3)), q1 = *(const uint4 *)(sb + 32 + 32 * (p & 3));
+        t.w[it][0] = hdr.x; t.w[it][1] = hdr.y; t.w[it][2] = hdr.z; t.w[it][3] = hdr.w;
+        t.w[it][4] = q0.x; t.w[it][5] = q0.y; t.w[it][6] = q0.z; t.w[it][7] = q0.w;
+        t.w[it][8] = q1.x; t.w[it][9] = q1.y; t.w[it][10] = q1.z; t.w[it][11] = q1.w;
+    } else if constexpr (WT == SPY_HIP_Q6_K) {
+        static_assert(WT != SPY_HIP_Q6_K || LPR == 64, "K-quant tiles use 64 lanes per row");
+        // lane (n = half of the super-block, e = 16-element slice): ql[64n + 16e ..], ql[64n + 32 + 16e ..], qh[32n + 16e ..], scales[8n ..]
+        const int j = p & 3, n = j >> 1, e = j & 1;
+        const uint8_t *sb = rowp + (size_t)(p >> 2) * 210;
+        uint4 ca, cb, ch; uint2 cs;
+        __builtin_memcpy(&ca, __builtin_assume_aligned(sb + 64 * n + 16 * e, 2), 16);
+        __builtin_memcpy(&cb, __builtin_assume_aligned(sb + 64 * n + 32 + 16 * e, 2), 16);
+        __builtin_memcpy(&ch, __builtin_assume_aligned(sb + 128 + 32 * n + 16 * e, 2), 16);
+        __builtin_memcpy(&cs, __builtin_assume_aligned(sb + 192 + 8 * n, 2), 8);
+        t.w[it][0] = ca.x; t.w[it][1] = ca.y; t.w[it][2] = ca.z; t.w[it][3] = ca.w;
+        t.w[it][4] = cb.x; t.w[it][5] = cb.y; t.w[it][6] = cb.z; t.w[it][7] = cb.w;
+        t.w[it][8] = ch.x; t.w[it][9] = ch.y; t.w[it][10] = ch.z; t.w[it][11] = ch.w;
+        t.w[it][12] = cs.x; t.w[it][13] = cs.y;
+        t.w[it][14] = *(const uint16_t *)(sb + 208);
+    } else {
+        const uint32_t *wp = (const uint32_t *)rowp + (size_t)p * DW;
 #pragma unroll
-    for (int it = 0; it < NIT; it++) {
-        const int p = min(it * LPR + l, npair - 1);
-        if constexpr (WT == SPY_HIP_Q4_K) {
-            static_assert(WT != SPY_HIP_Q4_K || LPR == 64, "K-quant tiles use 64 lanes per row");
-            const uint8_t *sb = rowp + (size_t)(p >> 2) * 144;
-            const uint4 hdr = *(const uint4 *)sb, q0 = *(const uint4 *)(sb + 16 + 32 * (p & 3)), q1 = *(const uint4 *)(sb + 32 + 32 * (p & 3));
-            t.w[it][0] = hdr.x; t.w[it][1] = hdr.y; t.w[it][2] = hdr.z; t.w[it][3] = hdr.w;
-            t.w[it][4] = q0.x; t.w[it][5] = q0.y; t.w[it][6] = q0.z; t.w[it][7] = q0.w;
-            t.w[it][8] = q1.x; t.w[it][9] = q1.y; t.w[it][10] = q1.z; t.w[it][11] = q1.w;
-        } else if constexpr (WT == SPY_HIP_Q6_K) {
-            static_assert(WT != SPY_HIP_Q6_K || LPR == 64, "K-quant tiles use 64 lanes per row");
-            // lane (n = half of the super-block, e = 16-element slice): ql[64n + 16e ..], ql[64n + 32 + 16e ..], qh[32n + 16e ..], scales[8n ..]
-            const int j = p & 3, n = j >> 1, e = j & 1;
-            const uint8_t *sb = rowp + (size_t)(p >> 2) * 210;
-            uint4 ca, cb, ch; uint2 cs;
-            __builtin_memcpy(&ca, __builtin_assume_aligned(sb + 64 * n + 16 * e, 2), 16);
-            __builtin_memcpy(&cb, __builtin_assume_aligned(sb + 64 * n + 32 + 16 * e, 2), 16);
-            __builtin_memcpy(&ch, __builtin_assume_aligned(sb + 128 + 32 * n + 16 * e, 2), 16);
-            __builtin_memcpy(&cs, __builtin_assume_aligned(sb + 192 + 8 * n, 2), 8);
-            t.w[it][0] = ca.x; t.w[it][1] = ca.y; t.w[it][2] = ca.z; t.w[it][3] = ca.w;
-            t.w[it][4] = cb.x; t.w[it][5] = cb.y; t.w[it][6] = cb.z; t.w[it][7] = cb.w;
-            t.w[it][8] = ch.x; t.w[it][9] = ch.y; t.w[it][10] = ch.z; t.w[it][11] = ch.w;
-            t.w[it][12] = cs.x; t.w[it][13] = cs.y;
-            t.w[it][14] = *(const uint16_t *)(sb + 208);
-        } else {
-            const uint32_t *wp = (const uint32_t *)rowp + (size_t)p * DW;
-#pragma unroll
-            for (int i = 0; i < DW; i++) t.w[it][i] = wp[i];
-        }
+        for (int i = 0; i < DW; i++) t.w[it][i] = wp[i];
     }
+}
+template <int WT, int LPR, int NIT>
+static __device__ __forceinline__ void load_tile(wtile<WT, NIT> &t, const uint8_t *__restrict__ rowp, int npair, int l) {
+#pragma unroll
+    for (int it = 0; it < NIT; it++) load_slab<WT, LPR, NIT>(t, rowp, npair, l, it);
 }
 
 static __device__ __forceinline__ int dot_q4_dwords(const uint32_t n0, const uint32_t n1, const uint32_t n2, const uint32_t n3,

@@ -640,16 +640,18 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
 #pragma unroll
     for (int u = 0; u < XP_NS; u++) sreg[u] = srow[min(tid + u * XP_THREADS, n_ctx - 1)];
     // The V^T rows: nothing beyond the last cached token is asked for.  Rows of up to 1024 tokens are on their way beside the scores; the
-    // pieces of longer ones would stand before the table gathers in the memory queue (4096 tokens 13.9 -> 14.1 us with four of eight ahead).
+    // pieces of longer ones would stand before the table gathers in the memory queue (4096 tokens 13.9 -> 14.1 us with four of eight ahead).  From 3072
+    // tokens on, two pieces of a row follow right behind the gathers (4096 tokens 13.8 -> 12.7 us, 3000 11.65 -> 11.55; 2500 10.6 -> 11.2:
+    // there the stream is shorter than what the wait for their issue costs).
     // vc is not a restrict pointer on purpose: the loads must stay where they are written.
     xp_u4 vb[XP_NP];
     const int last_piece = (n_kv - 1) >> 3;
-    auto load_row = [&]() {
+    auto load_row = [&](int from, int to) {
 #pragma unroll
-        for (int i = 0; i < XP_NP; i++) if (i * 64 <= last_piece) vb[i] = *(const xp_u4 *)(vrow + (size_t)min(i * 64 + lane, last_piece) * 8);
+        for (int i = 0; i < XP_NP; i++) if (i >= from && i < to && i * 64 <= last_piece) vb[i] = *(const xp_u4 *)(vrow + (size_t)min(i * 64 + lane, last_piece) * 8);
     };
-    const bool early = n_kv <= 1024;
-    if (early) load_row();
+    const bool early = n_kv <= 1024, ahead = n_kv > 3072;
+    if (early) load_row(0, 2);
     float mx = -INFINITY;
 #pragma unroll
     for (int u = 0; u < XP_NS; u++) if (tid + u * XP_THREADS < n_kv) mx = fmaxf(mx, sreg[u]);
@@ -663,6 +665,7 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
     // exponentials from the table (a gather of 64 entries takes 64 cycles: only where there are scores)
 #pragma unroll
     for (int u = 0; u < XP_NS; u++) if (wave * 64 + u * XP_THREADS < n_kv) sreg[u] = lut[f2h(sreg[u] - mx)];
+    if (ahead) load_row(0, 2);
 #pragma unroll
     for (int u = 0; u < XP_NS; u++) { const int j = tid + u * XP_THREADS; if (j < n_kv) s_e[j] = sreg[u]; }
     __syncthreads();
@@ -683,12 +686,16 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
     XSTAMP(dbg, 3);
     // Longer rows are requested now, by every wave but the one that walks the sum (a wave that asks for its whole row sits in the issue stage
     // until the memory queue has room, i.e. for most of the row's transfer time): they arrive while the sum is walked.
-    if (wave != 0) { if (!early) load_row(); }
+    auto rest = [&]() {
+        if (!early && !ahead) load_row(0, 2);
+        if (!early) load_row(2, XP_NP);
+    };
+    if (wave != 0) rest();
     else {
         float init = xg_segment_sum<2>(s_grp, ngrp);
         for (int j = ngrp * 4; j < n_kv; j++) init = init + s_e[j];
         if (lane == 0) s_sum = init;
-        if (!early) load_row();
+        rest();
     }
     __syncthreads();
     XSTAMP(dbg, 4);

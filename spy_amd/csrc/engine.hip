@@ -369,7 +369,7 @@ bool spy_xgemm_ok(int wtype, const void *w, const float *dst, int64_t M, int64_t
 int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, int64_t K, void *pack);
 int spy_xgemm_norm_pack(hipStream_t st, bool own, const float *x, const float *w, float eps, int64_t T, int64_t K, void *pack);
 int spy_xgemm_silu_pack(hipStream_t st, const float *gate, const float *up, const float *lut, int64_t T, int64_t F, void *pack);
-int spy_xgemm_own(hipStream_t st, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
+int spy_xgemm_own(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
 bool spy_gemm_unsplit_shape(int64_t M, int64_t T);                                                                               // gemm.hip
 int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
 int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, float *out, const float *lut,
@@ -554,7 +554,7 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
             const void *w3[3] = {L.wq, L.wk, L.wv};
             float *d3[3] = {q, k, v};
             RC_TRY(spy_xgemm_norm_pack(st, true, x, L.attn_norm, c.eps, T, d, scr));
-            RC_TRY(spy_xgemm_own(st, 3, w3, d3, d, d, T, d, nullptr, scr));
+            RC_TRY(spy_xgemm_own(st, L.t_wq, 3, w3, d3, d, d, T, d, nullptr, scr));
         } else if (fuse_act) {    // NormRMS -> Mul -> Q8_0 in one kernel, quantized once for the three MatMuls
             RC_TRY(spy_norm_mul_q8_launch(st, x, 4 * d, (const float *)L.attn_norm, c.eps, scr, T, d));
             RC_TRY(spy_hip_gemm_q8_0act(st, L.t_wq, L.wq, scr, q, d, d, T, d));
@@ -616,7 +616,7 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
         }
         if (x_ok(L.t_wo, L.wo, d, d)) {
             RC_TRY(spy_xgemm_pack(st, o2, 4 * d, T, d, scr));
-            RC_TRY(spy_xgemm_own(st, 1, &L.wo, &t1, d, d, T, d, x, scr));
+            RC_TRY(spy_xgemm_own(st, L.t_wo, 1, &L.wo, &t1, d, d, T, d, x, scr));
         } else {
             RC_TRY(mm(L.wo, L.t_wo, d, d, &t_o2, &t_t1));
             RC_TRY(spy_hip_op_binary(st, 0, &t_t1, &t_x, &t_t1));
@@ -628,7 +628,7 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
                 const void *w2[2] = {L.w_up, L.w_gate};
                 float *d2[2] = {up, gate};
                 RC_TRY(spy_xgemm_norm_pack(st, true, t1, L.ffn_norm, c.eps, T, d, scr));
-                RC_TRY(spy_xgemm_own(st, 2, w2, d2, F, d, T, F, nullptr, scr));
+                RC_TRY(spy_xgemm_own(st, L.t_up, 2, w2, d2, F, d, T, F, nullptr, scr));
             } else {
                 RC_TRY(spy_norm_mul_q8_launch(st, t1, 4 * d, (const float *)L.ffn_norm, c.eps, scr, T, d));
                 if (L.t_up == L.t_gate) RC_TRY(spy_gemm_q8act_pair(st, L.t_up, L.w_up, L.w_gate, scr, up, gate, F, d, T, F));   // one grid for both
@@ -639,7 +639,7 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
             }
             if (x_down) {
                 RC_TRY(spy_xgemm_silu_pack(st, gate, up, nullptr, T, F, scr));
-                RC_TRY(spy_xgemm_own(st, 1, &L.w_down, &x, d, F, T, d, t1, scr));
+                RC_TRY(spy_xgemm_own(st, L.t_down, 1, &L.w_down, &x, d, F, T, d, t1, scr));
             } else {
                 RC_TRY(spy_silu_mul_q8_launch(st, gate, up, scr, T, F));        // Silu -> Mul -> Q8_0
                 RC_TRY(spy_hip_gemm_q8_0act(st, L.t_down, L.w_down, scr, o, d, F, T, d));

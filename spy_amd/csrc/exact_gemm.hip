@@ -516,6 +516,24 @@ __device__ __forceinline__ void xk_put_scales(const xk_raw<WT> &w, float *tab, i
     __builtin_amdgcn_wave_barrier();                                    // other lanes of the wave read them
     asm volatile("" ::: "memory");
 }
+// Q4_K in the own order: [sub-block][row] sc as a pair of fp16 (times 2^10 / 2^6: the product with a nibble is n * sc * 2^-14), [sub-block][row] m, [row] d * 2^14, [row] -dmin
+__device__ __forceinline__ void xk_put_scales_own(const xk_raw<SPY_HIP_Q4_K> &w, float *tab, int q, int r) {
+    const int s16 = 16 * (q & 1);
+    const uint32_t t0 = w.head.y >> s16, t1 = w.head.z >> s16, t2 = w.head.w >> s16;
+    const bool hi = q >= 2;
+    const uint32_t sc = hi ? (t2 & 0x0F0Fu) | ((t0 >> 2) & 0x3030u) : t0 & 0x3F3Fu, mm = hi ? ((t2 >> 4) & 0x0F0Fu) | ((t1 >> 2) & 0x3030u) : t1 & 0x3F3Fu;
+    const _Float16 s0 = (_Float16)(float)((sc & 0xFFu) << 10), s1 = (_Float16)(float)((sc >> 8 & 0xFFu) << 6);
+    const xt_h2 p0 = {s0, s0}, p1 = {s1, s1};
+    uint32_t *o = (uint32_t *)tab + 2 * q * 16 + r;
+    o[0] = __builtin_bit_cast(uint32_t, p0);
+    o[16] = __builtin_bit_cast(uint32_t, p1);
+    tab[128 + 2 * q * 16 + r] = (float)(mm & 0xFFu);
+    tab[128 + (2 * q + 1) * 16 + r] = (float)((mm >> 8) & 0xFFu);
+    if (q == 0) tab[256 + r] = xk_half(w.head.x & 0xFFFFu) * 16384.0f;
+    if (q == 1) tab[272 + r] = -xk_half(w.head.x >> 16);
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+}
 // operand(s) of sub-block t of the super-block
 template <int WT, int t>
 __device__ __forceinline__ void xk_unpack(const xk_raw<WT> &w, int q, uint4 (&o)[WT == SPY_HIP_Q4_K ? 1 : 2]) {
@@ -544,7 +562,12 @@ __device__ __forceinline__ void xk_unpack(const xk_raw<WT> &w, int q, uint4 (&o)
     }
 }
 
-template <int WT, int RG, int C, int OCC>
+// OWN: this backend's own order.  The terms of a super-block are added before its d and dmin are applied:
+//   acc = acc + d * (sum d_x * (sc * isum)) - dmin * (sum m * (d_x * bsum))
+// with sc on the weights' operand and the second sum, a contraction over sub-blocks, on v_mfma_f32_16x16x4_f32: 5 vector instructions per tile and
+// sub-block instead of 17 (Q4_K) and 9 (Q6_K).  4096 x 4096 x 1000, packing included: Q4_K 105 -> 87 us, Q6_K 112 -> 97; 22016 x 4096 x 1000: 557 -> 401
+// and 588 -> 449 (the 128 x 128 tiles of gemm.hip: 424 and 755).
+template <int WT, bool OWN, int RG, int C, int OCC>
 __global__ __launch_bounds__(64 * RG, OCC) void xk_kernel(xt_args a) {
     constexpr bool K4 = WT == SPY_HIP_Q4_K;
     constexpr int NT = 64 * RG, ROWS = 16 * RG, NXI = C * 256 / NT, C2 = (C + 1) / 2;
@@ -583,7 +606,9 @@ __global__ __launch_bounds__(64 * RG, OCC) void xk_kernel(xt_args a) {
     for (int c = 0; c < C; c++)
 #pragma unroll
         for (int v = 0; v < 4; v++) acc[c][v] = 0.0f;
-    float *tab = (float *)(smem + NXS * XB) + wave * (K4 ? 256 : 16);      // the wave's scales: Q4_K [sub-block][d * sc, dmin * m][row], Q6_K [row] d
+    float A[OWN ? C : 1][4];
+    xk_v4f Bm[OWN && K4 ? C : 1];
+    float *tab = (float *)(smem + NXS * XB) + wave * (K4 ? (OWN ? 288 : 256) : 16);      // the wave's scales: Q4_K [sub-block][d * sc, dmin * m][row], Q6_K [row] d
     const xk_v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
     auto compute = [&](int s, auto par_c) {
         constexpr int par = decltype(par_c)::value;
@@ -598,12 +623,16 @@ __global__ __launch_bounds__(64 * RG, OCC) void xk_kernel(xt_args a) {
             const int b = j / C, c = j % C;
             xv[j % 3] = *(const uint4 *)(sx + c * XT_XB + b * 1024);
             dx[j % 3] = *(const uint32_t *)(sd + c * XT_XD + b * 64);
-            if constexpr (K4) bs[j % 3] = *(const float *)(sd + c * XT_XD + 256 + b * 64);
+            if constexpr (K4 && !OWN) bs[j % 3] = *(const float *)(sd + c * XT_XD + 256 + b * 64);
         };
         auto weights = [&](auto b_c) {
             constexpr int b = decltype(b_c)::value;
             xk_unpack<WT, 4 * par + b>(cur, q, w[b & 1]);
-            if constexpr (K4) {
+            if constexpr (K4 && OWN) {
+                const uint32_t sc = ((const uint32_t *)tab)[(4 * par + b) * 16 + r];
+                uint4 &o = w[b & 1][0];
+                o = make_uint4(xk_pk_mul(o.x, sc), xk_pk_mul(o.y, sc), xk_pk_mul(o.z, sc), xk_pk_mul(o.w, sc));
+            } else if constexpr (K4) {
                 dsc[b & 1] = *(const xk_v4f *)(tab + (4 * par + b) * 32 + 4 * q);
                 dm[b & 1] = *(const xk_v4f *)(tab + (4 * par + b) * 32 + 16 + 4 * q);
             }
@@ -613,7 +642,7 @@ __global__ __launch_bounds__(64 * RG, OCC) void xk_kernel(xt_args a) {
             p[j & 1] = xk_mfma(w[b & 1][0], xv[j % 3], zero);
             if constexpr (!K4) p[j & 1] = xk_mfma(w[b & 1][1], xv[j % 3], p[j & 1]);
         };
-        if constexpr (!K4) dsc[0] = *(const xk_v4f *)(tab + 4 * q);
+        if constexpr (!K4 && !OWN) dsc[0] = *(const xk_v4f *)(tab + 4 * q);
         rd(0);
         rd(1);
         weights(std::integral_constant<int, 0>{});
@@ -629,7 +658,8 @@ __global__ __launch_bounds__(64 * RG, OCC) void xk_kernel(xt_args a) {
             const float x = h2f((uint16_t)dx[j % 3]);
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                if constexpr (K4) {
+                if constexpr (OWN) A[c][v] = par == 0 && b == 0 ? x * p[j & 1][v] : fmaf(x, p[j & 1][v], A[c][v]);
+                else if constexpr (K4) {
                     const float pos = dsc[b & 1][v] * p[j & 1][v], neg = dm[b & 1][v] * bs[j % 3];
                     acc[c][v] = fmaf(x, pos - neg, acc[c][v]);
                 } else acc[c][v] = fmaf(x * dsc[0][v], p[j & 1][v], acc[c][v]);
@@ -637,6 +667,27 @@ __global__ __launch_bounds__(64 * RG, OCC) void xk_kernel(xt_args a) {
             __builtin_amdgcn_sched_barrier(0);
         };
         [&]<int... J>(std::integer_sequence<int, J...>) { (step(std::integral_constant<int, J>{}), ...); }(std::make_integer_sequence<int, NJ>{});
+        if constexpr (OWN && K4) {                 // lane (q, r): sub-block q of the stage, row r of either side
+            const float m = tab[128 + (4 * par + q) * 16 + r];
+            const uint8_t *sq = sd + q * 64;
+#pragma unroll
+            for (int c = 0; c < C; c++) {
+                const float xb = h2f((uint16_t)*(const uint32_t *)(sq + c * XT_XD)) * *(const float *)(sq + c * XT_XD + 256);
+                Bm[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(m, xb, par == 0 ? zero : Bm[c], 0, 0, 0);
+            }
+        }
+        if constexpr (OWN && par == 1) {
+            const xk_v4f d = *(const xk_v4f *)(tab + (K4 ? 256 : 0) + 4 * q);
+            xk_v4f dmin = zero;
+            if constexpr (K4) dmin = *(const xk_v4f *)(tab + 272 + 4 * q);
+#pragma unroll
+            for (int c = 0; c < C; c++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    acc[c][v] = fmaf(d[v], A[c][v], acc[c][v]);
+                    if constexpr (K4) acc[c][v] = fmaf(dmin[v], Bm[c][v], acc[c][v]);
+                }
+        }
     };
     auto ready = [&]() {
         xt_wait_vm<0>();
@@ -644,7 +695,8 @@ __global__ __launch_bounds__(64 * RG, OCC) void xk_kernel(xt_args a) {
     };
     for (int s = 0; s < nst; s += 2) {
         ready();
-        xk_put_scales<WT>(cur, tab, q, r);         // the compiler's own wait for the super-block stands here, where nothing is on its way
+        if constexpr (OWN && K4) xk_put_scales_own(cur, tab, q, r);
+        else xk_put_scales<WT>(cur, tab, q, r);         // the compiler's own wait for the super-block stands here, where nothing is on its way
         const xk_raw<WT> nxt = xk_load<WT>(wr, min(s / 2 + 1, nst / 2 - 1), q);
         issue_x();
         compute(s, std::integral_constant<int, 0>{});
@@ -917,12 +969,12 @@ int xo_launch(hipStream_t st, xt_args a, int nmat) {
     xo_kernel<RW, WV, C, OCC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * WV), lds, st>>>(a);
     return SPY_LAUNCH_RC();
 }
-template <int WT, int RG, int C, int OCC>
+template <int WT, bool OWN, int RG, int C, int OCC>
 int xk_launch(hipStream_t st, xt_args a, int nmat) {
-    constexpr size_t lds = 2 * (C * XT_XB + (C + 1) / 2 * 1024) + RG * 1024;
-    if (lds > 64 * 1024) { const int rc = spy_raise_lds_limit((const void *)xk_kernel<WT, RG, C, OCC>, lds); if (rc) return rc; }
+    constexpr size_t lds = 2 * (C * XT_XB + (C + 1) / 2 * 1024) + RG * (OWN ? 1152 : 1024);
+    if (lds > 64 * 1024) { const int rc = spy_raise_lds_limit((const void *)xk_kernel<WT, OWN, RG, C, OCC>, lds); if (rc) return rc; }
     a.tiles = (a.M + 16 * RG - 1) / (16 * RG);
-    xk_kernel<WT, RG, C, OCC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * RG), lds, st>>>(a);
+    xk_kernel<WT, OWN, RG, C, OCC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * RG), lds, st>>>(a);
     return SPY_LAUNCH_RC();
 }
 template <int WT>
@@ -977,9 +1029,24 @@ int xk_dispatch(hipStream_t st, const xt_args &a, int nmat) {
                          k6[4] = {{16, 1, 110, 56}, {64, 2, 330, 210}, {64, 4, 440, 260}, {128, 8, 940, 690}};
     switch (xt_pick(a, nmat, WT == SPY_HIP_Q4_K ? k4 : k6, 4)) {
     case 0: return xks_launch<WT>(st, a, nmat);
-    case 1: return xk_launch<WT, 4, 2, 4>(st, a, nmat);
-    case 2: return xk_launch<WT, 4, 4, 4>(st, a, nmat);
-    default: return xk_launch<WT, 8, 8, 4>(st, a, nmat);
+    case 1: return xk_launch<WT, false, 4, 2, 4>(st, a, nmat);
+    case 2: return xk_launch<WT, false, 4, 4, 4>(st, a, nmat);
+    default: return xk_launch<WT, false, 8, 8, 4>(st, a, nmat);
+    }
+}
+
+// the own order of the K-quants; as in xt_dispatch
+template <int WT>
+int xko_dispatch(hipStream_t st, const xt_args &a, int nmat) {
+    static const xt_cost k4[6] = {{16, 1, 94, 43}, {32, 2, 235, 74}, {64, 2, 250, 128}, {32, 4, 330, 128}, {64, 4, 355, 185}, {64, 8, 560, 355}},
+                         k6[6] = {{16, 1, 110, 56}, {32, 2, 230, 110}, {64, 2, 310, 196}, {32, 4, 315, 161}, {64, 4, 390, 254}, {64, 8, 560, 396}};
+    switch (xt_pick(a, nmat, WT == SPY_HIP_Q4_K ? k4 : k6, 6)) {
+    case 0: return xks_launch<WT>(st, a, nmat);
+    case 1: return xk_launch<WT, true, 2, 2, 4>(st, a, nmat);
+    case 2: return xk_launch<WT, true, 4, 2, 4>(st, a, nmat);
+    case 3: return xk_launch<WT, true, 2, 4, 3>(st, a, nmat);
+    case 4: return xk_launch<WT, true, 4, 4, 4>(st, a, nmat);
+    default: return xk_launch<WT, true, 4, 8, 2>(st, a, nmat);
     }
 }
 
@@ -1058,9 +1125,10 @@ int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *
     default: return xk_dispatch<SPY_HIP_Q6_K>(st, a, nmat);
     }
 }
-// the same in this backend's own order; Q4_0 (Q8_0 unpacks more per block: 3 % slower than the tile kernel of gemm.hip at 22016 rows)
-int spy_xgemm_own(hipStream_t st, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack) {
+// the same in this backend's own order; Q4_0, Q4_K, Q6_K (Q8_0 unpacks more per block than Q4_0: 3 % slower than the tile kernel of gemm.hip at 22016 rows)
+int spy_xgemm_own(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack) {
     xt_args a;
-    const int rc = xt_fill(a, SPY_HIP_Q4_0, nmat, w, dst, M, K, T, d_row, resid, pack);
-    return rc ? rc : xo_dispatch(st, a, nmat);
+    const int rc = xt_fill(a, wtype, nmat, w, dst, M, K, T, d_row, resid, pack);
+    if (rc) return rc;
+    return wtype == SPY_HIP_Q4_0 ? xo_dispatch(st, a, nmat) : wtype == SPY_HIP_Q4_K ? xko_dispatch<SPY_HIP_Q4_K>(st, a, nmat) : wtype == SPY_HIP_Q6_K ? xko_dispatch<SPY_HIP_Q6_K>(st, a, nmat) : SPY_HIP_EINVAL;
 }

@@ -23,7 +23,7 @@ size_t spy_exact_pack_bytes(int64_t ne01, int64_t ne00, int64_t ne11);
 size_t spy_xgemm_pack_bytes(int64_t T, int64_t K);
 bool spy_xgemm_ok(int wtype, const void *w, const float *dst, int64_t M, int64_t K, int64_t T, int64_t d_row);
 int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, int64_t K, void *pack);
-int spy_xgemm_own(hipStream_t st, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
+int spy_xgemm_own(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
 int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
 
 struct tdesc {              // a tensor as the kernels see it
@@ -742,10 +742,10 @@ static size_t matmul_act_bytes(const spy_hip_tensor *w, const spy_hip_tensor *x)
     return (size_t)(spy_t_nrow(x) * spy_row_size(tm, x->ne[0]));
 }
 // Whether exact_gemm.hip runs a MatMul.  In the host's order: three activation rows and more (two single-row launches take less).  In this backend's own
-// order K-quants from eight rows: their sums are sub-block by sub-block as well, and the row kernels (2 us per row of a 4096 x 4096 matrix) and the
-// 128 x 128 tiles take longer at any number of rows: 4096 x 4096 Q4_K 16 rows 32 -> 12 us, 128 rows 52 -> 29, 1000 rows 128 -> 104; Q6_K 35 -> 14,
-// 69 -> 39, 195 -> 110 (at six rows of 11008 columns they are still 10 % slower).  Q4_0 in the own order where the kernels of gemm.hip would not
-// split K (more than 64 rows and enough tiles), with the same bits.
+// order K-quants from eight rows (at six rows of 11008 columns the row kernels are still 10 % faster): those take 2 us per row of a 4096 x 4096
+// matrix, and the 128 x 128 tiles as long or longer at any number of rows: 4096 x 4096 Q4_K 16 rows 33 -> 13 us, 128 rows 52 -> 30, 1000 rows
+// 128 -> 87; Q6_K 35 -> 14, 69 -> 38, 195 -> 98.  Q4_0 in the own order where the kernels of gemm.hip would not split K (more than 64 rows and
+// enough tiles), with the same bits.
 bool spy_gemm_unsplit_shape(int64_t M, int64_t T);                 // gemm.hip
 static bool xgemm_rows(int wtype, int64_t M, int64_t T) {
     if (spy_exact_on()) return T >= 3;
@@ -849,7 +849,7 @@ static int matmul_impl(void *stream, const spy_hip_tensor *w, const spy_hip_tens
             const void *wp = w->data;
             float *dp = (float *)dst->data;
             const int rc = spy_xgemm_pack(st, (const float *)x->data, x->nb[1], ne11, ne00, scratch);
-            if (!rc && !spy_exact_on() && t0 == SPY_HIP_Q4_0) return spy_xgemm_own(st, 1, &wp, &dp, ne01, ne00, ne11, dst->nb[1] / 4, nullptr, scratch);
+            if (!rc && !spy_exact_on()) return spy_xgemm_own(st, t0, 1, &wp, &dp, ne01, ne00, ne11, dst->nb[1] / 4, nullptr, scratch);
             return rc ? rc : spy_xgemm(st, t0, 1, &wp, &dp, ne01, ne00, ne11, dst->nb[1] / 4, nullptr, scratch);
         }
     }

@@ -154,7 +154,7 @@ def test_op_matmul_prompt_sizes(hip, oracle):
 
 
 @pytest.mark.parametrize("wtype,M,K,T", [(O.Q4_0, 16356, 256, 65), (O.Q4_0, 8164, 512, 129), (O.Q4_0, 4068, 768, 400), (O.Q4_0, 2020, 256, 1025), (O.Q4_0, 11008, 4096, 130),
-                                         (O.Q4_K, 36, 512, 8), (O.Q4_K, 4100, 256, 130), (O.Q6_K, 36, 512, 9), (O.Q6_K, 4100, 256, 130)])
+                                         (O.Q4_K, 36, 512, 8), (O.Q4_K, 4100, 256, 130), (O.Q4_K, 12300, 256, 70), (O.Q4_K, 8200, 512, 650), (O.Q4_K, 11012, 256, 40), (O.Q6_K, 36, 512, 9), (O.Q6_K, 4100, 256, 130), (O.Q6_K, 12300, 256, 70), (O.Q6_K, 8200, 512, 650)])
 def test_matmul_operator_takes_the_packed_activation_kernels(hip, oracle, wtype, M, K, T, monkeypatch):
     """MatMul in this backend's own order from packed activations, with partial tiles on both sides: within fp32 rounding of the oracle,
     and for Q4_0 the bits of the tile kernel, which adds an output's blocks in the same sequence."""

@@ -93,6 +93,7 @@ extern "C" int spy_hip_op_norm_rms(void *stream, const spy_hip_tensor *x, const 
     SPY_CHECK_ARG(same_ne(x, dst) && x->nb[0] == 4 && dst->nb[0] == 4);
     const int64_t nrow = spy_t_nrow(dst);
     CHECK_GRID(nrow, 1);
+    if (dst->ne[0] <= 0) return 0;                                           // rows without elements: nothing to write, and no last element for ROW to repeat
     if (spy_exact_on()) return spy_exact_norm_rms((hipStream_t)stream, x, dst, eps);
     if (dst->ne[0] <= 4096) norm_rms_kernel<true><<<dim3((unsigned)nrow), dim3(256), 0, (hipStream_t)stream>>>(mk(x), mk(dst), eps);
     else norm_rms_kernel<false><<<dim3((unsigned)nrow), dim3(256), 0, (hipStream_t)stream>>>(mk(x), mk(dst), eps);

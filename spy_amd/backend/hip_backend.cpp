@@ -163,7 +163,11 @@ const void *HIPBackend::device_view(DataNode *node, bool is_output) {
         if (bytes <= kCompareLimit && s.uploaded_valid && s.uploaded_bytes == bytes && std::memcmp(s.uploaded, t.data_ptr, bytes) == 0) return s.dev;
         s.uploaded_valid = false;
         if (bytes > kCompareLimit) return spy_hip_upload(s.dev, t.data_ptr, bytes, stream_) == 0 ? s.dev : nullptr;
-        if (s.queued == syncs_) { spy_hip_sync(stream_); ++syncs_; }                                 // the last upload may still be reading the pinned bytes
+        if (s.queued == syncs_) {                                                                    // the last upload may still be reading the pinned bytes
+            const int rc = spy_hip_sync(stream_);
+            if (rc != 0) { last_error_ = rc; return nullptr; }
+            ++syncs_;
+        }
         if (s.uploaded_cap < bytes) {
             spy_hip_host_free(s.uploaded);
             s.uploaded = nullptr; s.uploaded_cap = 0;
@@ -196,7 +200,7 @@ OperatorStatus HIPBackend::fetch(DataNode *node, const void *dev) {
         rc = spy_hip_download(node->tensor.data_ptr, dev, bytes, stream_);
         if (rc == 0) rc = spy_hip_take_error(&flag);
     }
-    ++syncs_;
+    if (rc == 0) ++syncs_;                                       // anything that failed may have failed before the stream was waited for
     if (rc != 0 || flag != 0) { last_error_ = rc != 0 ? rc : SPY_HIP_EINVAL; return OperatorStatus::Fail; }
     return OperatorStatus::Success;
 }

@@ -57,7 +57,7 @@ private:
     struct Staged { void *dev = nullptr; size_t bytes = 0; uint8_t *uploaded = nullptr; size_t uploaded_cap = 0, uploaded_bytes = 0; bool uploaded_valid = false; uint64_t queued = 0; };
     OperatorStatus fetch(DataNode *node, const void *dev);        // an IO result to its host vector, with the pass's error flag
     uint8_t *result_ = nullptr;                                   // pinned: a result of up to kResultLimit bytes behind 64 bytes that hold the error flag
-    uint64_t syncs_ = 1;                                          // synchronisations of the stream so far
+    uint64_t syncs_ = 1;                                          // synchronisations of the stream so far, those that succeeded
     std::unordered_map<const DataNode *, Staged> io_;             // IO node -> staging buffer
     OperatorStatus last_status_ = OperatorStatus::Success;
     int last_error_ = 0;

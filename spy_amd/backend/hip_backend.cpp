@@ -66,19 +66,25 @@ static spy_hip_tensor flat(const Tensor &t, const void *data) {
     return o;
 }
 
+constexpr size_t kResultLimit = 1u << 20;        // results of up to this size come through pinned memory
+constexpr size_t kStageBlock = 256u << 10;       // pinned memory that IO inputs take their copies from, as long as it lasts
+constexpr size_t kStageLarge = 64u << 10;        // inputs beyond this size get memory of their own
+
 HIPBackend::HIPBackend(const BackendFactory::BackendConfiguration &config) : Backend(BackendType::Device) {
     device_id_ = config.parse_or("device_id", 0);           // same key as the CUDA stub (backend/cuda/include/default_backend.h:38-40)
     last_error_ = spy_hip_init(device_id_);
     if (last_error_ == 0) last_error_ = spy_hip_stream_create(&stream_);
-    if (last_error_ != 0) last_status_ = OperatorStatus::Fail;
+    if (last_error_ != 0) { last_status_ = OperatorStatus::Fail; return; }
+    // The pinned memory of a single token's passes, here and not in the first of them.  Without it (nothing to pin) passes copy from and to pageable memory.
+    if (spy_hip_host_alloc(reinterpret_cast<void **>(&pinned_), 64 + kResultLimit + kStageBlock) != 0) pinned_ = nullptr;
 }
 
 HIPBackend::~HIPBackend() noexcept {
     spy_hip_sync(nullptr);
     for (auto &kv : pool_) for (void *p : kv.second) spy_hip_free(p);
     for (auto &kv : constants_) spy_hip_free(kv.second);
-    for (auto &kv : io_) { spy_hip_free(kv.second.dev); spy_hip_host_free(kv.second.uploaded); }
-    spy_hip_host_free(result_);
+    for (auto &kv : io_) { spy_hip_free(kv.second.dev); give_back(kv.second); }
+    spy_hip_host_free(pinned_);
     if (stream_) spy_hip_stream_destroy(stream_);
 }
 
@@ -134,6 +140,26 @@ bool HIPBackend::is_support(OperatorType t) const {
 
 void HIPBackend::sync() { spy_hip_sync(stream_); }
 
+void HIPBackend::give_back(Staged &s) {
+    if (s.uploaded_own) spy_hip_host_free(s.uploaded);           // a piece of the block stays unused: there are a handful of IO nodes
+    s.uploaded = nullptr; s.uploaded_cap = 0; s.uploaded_own = false;
+}
+
+// Pinned memory for an IO tensor's bytes: a piece of the block made by the constructor, or an allocation for large ones and once the block is used up
+bool HIPBackend::take_pinned(Staged &s, size_t bytes) {
+    give_back(s);
+    const size_t cap = bucket(bytes);
+    if (pinned_ && cap <= kStageLarge && stage_used_ + cap <= kStageBlock) {
+        s.uploaded = pinned_ + 64 + kResultLimit + stage_used_;
+        stage_used_ += cap;
+    } else {
+        if (spy_hip_host_alloc(reinterpret_cast<void **>(&s.uploaded), cap) != 0) { s.uploaded = nullptr; return false; }
+        s.uploaded_own = true;
+    }
+    s.uploaded_cap = cap;
+    return true;
+}
+
 // Device address of a node's data.  Dynamic / Cache tensors already hold device pointers (they
 // were handed out by alloc_memory and view arithmetic keeps them on the device).
 const void *HIPBackend::device_view(DataNode *node, bool is_output) {
@@ -168,12 +194,7 @@ const void *HIPBackend::device_view(DataNode *node, bool is_output) {
             if (rc != 0) { last_error_ = rc; return nullptr; }
             ++syncs_;
         }
-        if (s.uploaded_cap < bytes) {
-            spy_hip_host_free(s.uploaded);
-            s.uploaded = nullptr; s.uploaded_cap = 0;
-            if (spy_hip_host_alloc(reinterpret_cast<void **>(&s.uploaded), bucket(bytes)) != 0) return nullptr;
-            s.uploaded_cap = bucket(bytes);
-        }
+        if (s.uploaded_cap < bytes && !take_pinned(s, bytes)) return spy_hip_upload(s.dev, t.data_ptr, bytes, stream_) == 0 ? s.dev : nullptr;
         std::memcpy(s.uploaded, t.data_ptr, bytes);
         if (spy_hip_upload_pinned(s.dev, s.uploaded, bytes, stream_) != 0) return nullptr;
         s.queued = syncs_;
@@ -188,14 +209,12 @@ const void *HIPBackend::device_view(DataNode *node, bool is_output) {
 // A token's logits go through pinned memory, flag and all, in one launch and one synchronisation (55 -> 20 us for 128 KB); a prompt's are copied as
 // they are, which the copy engine does at the bus's rate.
 OperatorStatus HIPBackend::fetch(DataNode *node, const void *dev) {
-    constexpr size_t kResultLimit = 1u << 20;
     const size_t bytes = static_cast<size_t>(node->tensor.total_size());
     int rc = 0, flag = 0;
-    if (bytes > 0 && bytes <= kResultLimit) {
-        if (!result_ && spy_hip_host_alloc(reinterpret_cast<void **>(&result_), kResultLimit + 64) != 0) return OperatorStatus::Fail;
-        rc = spy_hip_download_pinned(result_ + 64, dev, bytes, reinterpret_cast<int *>(result_), stream_);
+    if (bytes > 0 && bytes <= kResultLimit && pinned_) {
+        rc = spy_hip_download_pinned(pinned_ + 64, dev, bytes, reinterpret_cast<int *>(pinned_), stream_);
         if (rc == 0) rc = spy_hip_sync(stream_);
-        if (rc == 0) { std::memcpy(node->tensor.data_ptr, result_ + 64, bytes); flag = *reinterpret_cast<const int *>(result_); }
+        if (rc == 0) { std::memcpy(node->tensor.data_ptr, pinned_ + 64, bytes); flag = *reinterpret_cast<const int *>(pinned_); }
     } else {
         rc = spy_hip_download(node->tensor.data_ptr, dev, bytes, stream_);
         if (rc == 0) rc = spy_hip_take_error(&flag);

@@ -54,9 +54,12 @@ private:
     // device copy of an IO tensor, and (up to 8 MiB) the host bytes it was last uploaded from: the positions and the mask of a
     // pass are read by one operator per layer, and uploading them again for each costs more than comparing them
     // (in pinned memory: the copy to the device is queued from it; it is written again only after a synchronisation since then)
-    struct Staged { void *dev = nullptr; size_t bytes = 0; uint8_t *uploaded = nullptr; size_t uploaded_cap = 0, uploaded_bytes = 0; bool uploaded_valid = false; uint64_t queued = 0; };
+    struct Staged { void *dev = nullptr; size_t bytes = 0; uint8_t *uploaded = nullptr; size_t uploaded_cap = 0, uploaded_bytes = 0; bool uploaded_valid = false, uploaded_own = false; uint64_t queued = 0; };
+    bool take_pinned(Staged &s, size_t bytes);
+    void give_back(Staged &s);
     OperatorStatus fetch(DataNode *node, const void *dev);        // an IO result to its host vector, with the pass's error flag
-    uint8_t *result_ = nullptr;                                   // pinned: a result of up to kResultLimit bytes behind 64 bytes that hold the error flag
+    uint8_t *pinned_ = nullptr;                                   // 64 bytes with the error flag of a result, a result of up to 1 MiB, the copies of small IO inputs
+    size_t stage_used_ = 0;                                       // bytes handed out of the last part
     uint64_t syncs_ = 1;                                          // synchronisations of the stream so far, those that succeeded
     std::unordered_map<const DataNode *, Staged> io_;             // IO node -> staging buffer
     OperatorStatus last_status_ = OperatorStatus::Success;

@@ -115,7 +115,9 @@ extern "C" int spy_hip_host_alloc(void **ptr, size_t bytes) {
     if (!ptr) return SPY_HIP_EINVAL;
     *ptr = nullptr;
     if (bytes == 0) return 0;
-    return (int)hipHostMalloc(ptr, bytes, hipHostMallocDefault);
+    const hipError_t e = hipHostMalloc(ptr, bytes, hipHostMallocDefault);
+    if (e != hipSuccess) { *ptr = nullptr; (void)hipGetLastError(); }       // a caller may go on without: the next launch does not report this
+    return (int)e;
 }
 extern "C" int spy_hip_host_free(void *ptr) { return ptr ? (int)hipHostFree(ptr) : 0; }
 

@@ -122,6 +122,30 @@ int main(int argc, char **argv) {
     } else if (what == "repeated") {
         for (int i = 0; i < 5; ++i) { p.run(be, static_cast<float>(i / 2)); NEED(p.holds(static_cast<float>(i / 2))); }
         NEED(be.last_status() == OperatorStatus::Success);
+    } else if (what == "first-pass") {               // a single token's pass: ids, positions and a mask row in, logits out
+        Pass ids(1), pos(1), mask(4352), logits(32000);
+        const int before = g_host_allocs;
+        for (Pass *q : {&ids, &pos, &mask}) { q->run(be, 5.0f); NEED(q->holds(5.0f)); }
+        NEED(g_host_allocs == before);
+        logits.run(be, 7.0f);                        // a large input has memory of its own
+        NEED(logits.holds(7.0f) && g_host_allocs == before + 1);
+    } else if (what == "many-inputs") {              // more than the block of the small ones holds, and one that grows
+        std::vector<std::unique_ptr<Pass>> ps;
+        for (int i = 0; i < 100; ++i) ps.push_back(std::make_unique<Pass>(n + i));
+        for (int r = 0; r < 3; ++r)
+            for (size_t i = 0; i < ps.size(); ++i) { ps[i]->run(be, static_cast<float>(i + 1000 * r)); NEED(ps[i]->holds(static_cast<float>(i + 1000 * r))); }
+        ps[0]->in.tensor.shape = Shape({n / 2 + 1, 1}, NumberType::FP32);
+        ps[0]->op.propagate();
+        ps[0]->run(be, 1.0f);
+        ps[0]->in.tensor.shape = Shape({n, 1}, NumberType::FP32);
+        ps[0]->op.propagate();
+        ps[0]->run(be, 3.0f);
+        NEED(ps[0]->holds(3.0f) && be.last_status() == OperatorStatus::Success);
+    } else if (what == "nothing-to-pin") {
+        g_fail_host_alloc = 1;
+        hip::HIPBackend other(config);
+        for (int i = 0; i < 4; ++i) { p.run(other, static_cast<float>(i)); NEED(p.holds(static_cast<float>(i))); }
+        NEED(other.last_status() == OperatorStatus::Success && other.last_error() == 0);
     } else { std::printf("no such scenario\n"); return 1; }
     NEED(g_overwritten == 0);
     std::printf("ok\n");

@@ -658,11 +658,13 @@ extern "C" int spy_hip_argmax(void *stream, const float *logits, int64_t n, int3
 // A single token's attention products (4096 x 128 and 128 x n_kv outputs) are launch and latency: R outputs share the activations and have their loads
 // on the way together, nothing is divided per output (64-bit divisions took longer than the products), and no launch converts the
 // activations: 8.7 + 2.5 -> 4.9 us each at 513 cached tokens and 32 heads.
-template <bool XF32, int R>
+// I: the index along the contraction; int64_t for rows of 2^30 elements and more only.
+template <bool XF32, int R, class I = int>
 __global__ __launch_bounds__(256) void matmul_f16_kernel(tdesc w, const uint8_t *__restrict__ x, int64_t x_nb1, int64_t x_nb2, int64_t x_nb3, tdesc d, int y0, int z0) {
     const int i01 = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * R, ne01 = (int)w.ne[1];
     if (i01 >= ne01) return;
-    const int lane = threadIdx.x & 63, i11 = y0 + (int)blockIdx.y, ne00 = (int)w.ne[0], ne02 = (int)w.ne[2];
+    const int lane = threadIdx.x & 63, i11 = y0 + (int)blockIdx.y, ne02 = (int)w.ne[2];
+    const I ne00 = (I)w.ne[0];
     int i02 = z0 + (int)blockIdx.z, i03 = 0;
     if (i02 >= ne02) { i03 = i02 / ne02; i02 -= i03 * ne02; }
     const uint16_t *wr[R];
@@ -672,8 +674,8 @@ __global__ __launch_bounds__(256) void matmul_f16_kernel(tdesc w, const uint8_t 
     float acc[R];
 #pragma unroll
     for (int j = 0; j < R; j++) acc[j] = 0.0f;
-    auto get = [&](int k) { return XF32 ? h2f(f2h(((const float *)xr)[k])) : h2f(((const uint16_t *)xr)[k]); };
-    int k = lane;
+    auto get = [&](I k) { return XF32 ? h2f(f2h(((const float *)xr)[k])) : h2f(((const uint16_t *)xr)[k]); };
+    I k = lane;
     for (; k + 192 < ne00; k += 256) {
         float xv[4];
         uint16_t wv[4][R];
@@ -781,13 +783,16 @@ static int own_matvec(hipStream_t st, int t0, const void *w, const float *x, flo
 template <bool XF32>
 static int matmul_f16_launch(hipStream_t st, const spy_hip_tensor *w, const uint8_t *x, int64_t x_nb1, int64_t x_nb2, int64_t x_nb3, const spy_hip_tensor *dst) {
     const int64_t ne11 = dst->ne[1], nz = w->ne[2] * w->ne[3];
-    SPY_CHECK_ARG(w->ne[0] > 0 && w->ne[0] < (1ll << 30) && w->ne[1] > 0 && w->ne[1] < (1ll << 30) && ne11 > 0 && ne11 < (1ll << 31) && nz > 0 && nz < (1ll << 31));
+    // an empty contraction gives zeros (f32 activations of no elements have been refused: there is nothing to convert)
+    SPY_CHECK_ARG((XF32 ? w->ne[0] > 0 : w->ne[0] >= 0) && w->ne[1] > 0 && w->ne[1] < (1ll << 30) && ne11 > 0 && ne11 < (1ll << 31) && nz > 0 && nz < (1ll << 31));
     const int64_t wgs = w->ne[1] * ne11 * nz / 4;
-    const int R = wgs >= 8 * 512 ? 8 : wgs >= 4 * 256 ? 4 : 1;
+    const bool wide = w->ne[0] >= (1ll << 30);
+    const int R = wide ? 1 : wgs >= 8 * 512 ? 8 : wgs >= 4 * 256 ? 4 : 1;
     for (int64_t z = 0; z < nz; z += 65535)
         for (int64_t y = 0; y < ne11; y += 65535) {
             const dim3 grid((unsigned)((w->ne[1] + 4 * R - 1) / (4 * R)), (unsigned)(ne11 - y < 65535 ? ne11 - y : 65535), (unsigned)(nz - z < 65535 ? nz - z : 65535));
-            if (R == 8) matmul_f16_kernel<XF32, 8><<<grid, dim3(256), 0, st>>>(mk(w), x, x_nb1, x_nb2, x_nb3, mk(dst), (int)y, (int)z);
+            if (wide) matmul_f16_kernel<XF32, 1, int64_t><<<grid, dim3(256), 0, st>>>(mk(w), x, x_nb1, x_nb2, x_nb3, mk(dst), (int)y, (int)z);
+            else if (R == 8) matmul_f16_kernel<XF32, 8><<<grid, dim3(256), 0, st>>>(mk(w), x, x_nb1, x_nb2, x_nb3, mk(dst), (int)y, (int)z);
             else if (R == 4) matmul_f16_kernel<XF32, 4><<<grid, dim3(256), 0, st>>>(mk(w), x, x_nb1, x_nb2, x_nb3, mk(dst), (int)y, (int)z);
             else matmul_f16_kernel<XF32, 1><<<grid, dim3(256), 0, st>>>(mk(w), x, x_nb1, x_nb2, x_nb3, mk(dst), (int)y, (int)z);
             const int rc = SPY_LAUNCH_RC();

@@ -22,3 +22,45 @@ def test_norm_rms_of_empty_rows_launches_nothing(exact, ne):
         assert L.spy_hip_op_norm_rms(None, B(H.tensor(4096, H.F32, ne)), B(H.tensor(8192, H.F32, [0, 7])), 1e-5) == H.EINVAL
     finally:
         L.spy_hip_set_exact_order(prev)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,T,batch", [(1, 1, 1), (5, 3, 2), (300, 1, 32), (1030, 15, 1)])
+def test_fp16_product_with_an_empty_contraction(M, T, batch):
+    """fp16 rows of no elements give zeros, one, four and eight outputs per wave; the same with f32 activations is refused."""
+    from tests.gpu_util import dev_empty, call
+    H.init(0)
+    L = H.load()
+    prev = L.spy_hip_set_exact_order(0)
+    try:
+        w, out = dev_empty(256, 0xFF), dev_empty(batch * T * M * 4 + 64, 0xFF)
+        tw, to = H.tensor(w, H.F16, [0, M, batch]), H.tensor(out, H.F32, [M, T, batch])
+        call(L.spy_hip_op_matmul, None, B(tw), B(H.tensor(w, H.F16, [0, T, batch])), B(to), None, 0)
+        got = out.download(np.uint32)
+        assert (got[:batch * T * M] == 0).all() and (got[batch * T * M:] == 0xFFFFFFFF).all()
+        assert L.spy_hip_op_matmul(None, B(tw), B(H.tensor(w, H.F32, [0, T, batch])), B(to), w.ptr, 256) == H.EINVAL
+    finally:
+        L.spy_hip_set_exact_order(prev)
+
+
+@pytest.mark.gpu
+def test_fp16_product_of_rows_beyond_32_bit_indices():
+    """One output over a contraction of 2^30 + 67 fp16 elements: zeros but for elements at both ends and around 2^30."""
+    from tests.gpu_util import dev_empty, call
+    H.init(0)
+    L = H.load()
+    prev = L.spy_hip_set_exact_order(0)
+    try:
+        K = (1 << 30) + 67
+        w, x, out = dev_empty(2 * K, 0), dev_empty(2 * K, 0x3C), dev_empty(64, 0xFF)          # x: 0x3C3C everywhere
+        at = [0, 63, 12345, (1 << 30) - 1, 1 << 30, K - 1]
+        vals = np.array([1, 2, 4, 8, 16, 32], np.float16)
+        for i, v in zip(at, vals):
+            b = np.array([v], np.float16)
+            call(L.spy_hip_upload, w.ptr + 2 * i, b.ctypes.data, 2, None)
+        call(L.spy_hip_op_matmul, None, B(H.tensor(w, H.F16, [K, 1])), B(H.tensor(x, H.F16, [K, 1])), B(H.tensor(out, H.F32, [1, 1])), None, 0)
+        got = out.download(np.float32)
+        assert got[0] == np.float32(63 * float(np.array([0x3C3C], np.uint16).view(np.float16)[0]))      # exact: 11 bits times 6
+        assert (got[1:].view(np.uint32) == 0xFFFFFFFF).all()
+    finally:
+        L.spy_hip_set_exact_order(prev)

@@ -1063,18 +1063,18 @@ int xo_dispatch(hipStream_t st, const xt_args &a, int nmat) {
 }   // namespace
 
 // ---- what exact_order.hip and the engine call -----------------------------------------------------------------------------------------
-// bytes of packed activations of T rows of K elements (0: K is not a multiple of 256)
+// bytes of packed activations of T rows of K elements (0: K is not a multiple of 256, or more groups of 16 rows than a grid's y takes)
 size_t spy_xgemm_pack_bytes(int64_t T, int64_t K) {
-    if (T <= 0 || K <= 0 || K % 256) return 0;
+    if (T <= 0 || T > 16 * 65535 || K <= 0 || K % 256) return 0;
     return (size_t)((T + 15) / 16 * (K / 128) * (XT_XB + XT_XD));
 }
 // shapes and alignments the kernels take: whole chunks, 16-byte-aligned weight rows, four outputs stored together
 bool spy_xgemm_ok(int wtype, const void *w, const float *dst, int64_t M, int64_t K, int64_t T, int64_t d_row) {
-    return (wtype == SPY_HIP_Q4_0 || wtype == SPY_HIP_Q8_0 || wtype == SPY_HIP_Q4_K || wtype == SPY_HIP_Q6_K) && T >= 2 && T < (1 << 20) && K > 0 && K % 256 == 0 && K <= (1 << 20) && M > 0 && M % 4 == 0 && M < (1 << 24) &&
+    return (wtype == SPY_HIP_Q4_0 || wtype == SPY_HIP_Q8_0 || wtype == SPY_HIP_Q4_K || wtype == SPY_HIP_Q6_K) && T >= 2 && T <= 16 * 65535 && K > 0 && K % 256 == 0 && K <= (1 << 20) && M > 0 && M % 4 == 0 && M < (1 << 24) &&
            ((uintptr_t)w & 15) == 0 && ((uintptr_t)dst & 15) == 0 && d_row % 4 == 0;
 }
 int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, int64_t K, void *pack) {
-    if (((uintptr_t)x & 15) || x_stride % 16 || ((uintptr_t)pack & 15) || !spy_xgemm_pack_bytes(T, K) || (T + 15) / 16 > 65535) return SPY_HIP_EINVAL;
+    if (((uintptr_t)x & 15) || x_stride % 16 || ((uintptr_t)pack & 15) || !spy_xgemm_pack_bytes(T, K)) return SPY_HIP_EINVAL;
     const int nst = (int)(K / 128), ncg = (int)((T + 15) / 16);
     uint8_t *xq = (uint8_t *)pack, *xd = xq + (int64_t)ncg * nst * XT_XB;
     xt_pack_kernel<<<dim3((unsigned)(K / 64), (unsigned)ncg), dim3(256), 0, st>>>((const uint8_t *)x, x_stride, (int)T, nst, xq, xd);
@@ -1082,7 +1082,7 @@ int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, 
 }
 // x [T][K] f32 -> NormRMS * w -> packed activations; own: sum of squares in this backend's own order
 int spy_xgemm_norm_pack(hipStream_t st, bool own, const float *x, const float *w, float eps, int64_t T, int64_t K, void *pack) {
-    if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)pack & 15) || !spy_xgemm_pack_bytes(T, K) || (T + 15) / 16 > 65535 || K > 8192) return SPY_HIP_EINVAL;
+    if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)pack & 15) || !spy_xgemm_pack_bytes(T, K) || K > 8192) return SPY_HIP_EINVAL;
     const int nst = (int)(K / 128), ncg = (int)((T + 15) / 16);
     uint8_t *xq = (uint8_t *)pack, *xd = xq + (int64_t)ncg * nst * XT_XB;
     const dim3 grid((unsigned)(ncg * 16));
@@ -1094,7 +1094,7 @@ int spy_xgemm_norm_pack(hipStream_t st, bool own, const float *x, const float *w
 }
 // gate, up [T][F] f32 -> up * silu(gate) -> packed activations; lut: the host's tables (spy_exact_luts), or null
 int spy_xgemm_silu_pack(hipStream_t st, const float *gate, const float *up, const float *lut, int64_t T, int64_t F, void *pack) {
-    if (((uintptr_t)gate & 15) || ((uintptr_t)up & 15) || ((uintptr_t)pack & 15) || !spy_xgemm_pack_bytes(T, F) || (T + 15) / 16 > 65535) return SPY_HIP_EINVAL;
+    if (((uintptr_t)gate & 15) || ((uintptr_t)up & 15) || ((uintptr_t)pack & 15) || !spy_xgemm_pack_bytes(T, F)) return SPY_HIP_EINVAL;
     const int nst = (int)(F / 128), ncg = (int)((T + 15) / 16);
     uint8_t *xq = (uint8_t *)pack, *xd = xq + (int64_t)ncg * nst * XT_XB;
     xt_silu_pack_kernel<<<dim3((unsigned)nst, (unsigned)ncg), dim3(256), 0, st>>>(gate, up, lut, (int)F, (int)T, nst, xq, xd);

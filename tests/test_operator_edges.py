@@ -64,3 +64,52 @@ def test_fp16_product_of_rows_beyond_32_bit_indices():
         assert (got[1:].view(np.uint32) == 0xFFFFFFFF).all()
     finally:
         L.spy_hip_set_exact_order(prev)
+
+
+MOST_ROWS = 16 * 65535                       # activation rows that one launch of the packed-activation kernels takes
+
+
+@pytest.mark.parametrize("order,wtype", [(0, H.Q4_K), (0, H.Q6_K), (1, H.Q4_K), (1, H.Q6_K)])
+def test_matmul_scratch_beyond_the_packed_rows(order, wtype):
+    """Beyond the rows that the packed-activation kernels take nothing is asked for but the Q8_0 activations of the kernels that run instead."""
+    L = H.load()
+    prev = L.spy_hip_set_exact_order(order)
+    try:
+        w = H.tensor(4096, wtype, [256, 4])
+        for T in (MOST_ROWS + 1, (1 << 20) - 1, 1 << 20):
+            assert L.spy_hip_op_matmul_scratch_size(B(w), B(H.tensor(4096, H.F32, [256, T]))) == T * 8 * 34
+        assert L.spy_hip_op_matmul_scratch_size(B(w), B(H.tensor(4096, H.F32, [256, MOST_ROWS]))) > MOST_ROWS * 8 * 34
+    finally:
+        L.spy_hip_set_exact_order(prev)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order,wtype", [(1, O.Q4_0), (1, O.Q4_K), (0, O.Q4_K), (0, O.Q6_K)])
+@pytest.mark.parametrize("T", [MOST_ROWS, MOST_ROWS + 1, (1 << 20) - 1])
+def test_matmul_of_about_a_million_rows(oracle, order, wtype, T):
+    """One row more than one launch of the packed-activation kernels takes, and the rest up to 2^20: another kernel, not an error.  The rows repeat, so every
+    output is known from the first 64; in the host's order with the oracle's bits."""
+    from tests.gpu_util import assert_close, call, dev, dev_empty
+    H.init(0)
+    L = H.load()
+    prev = L.spy_hip_set_exact_order(order)
+    try:
+        K, M, P = 256, 4, 64
+        rng = np.random.default_rng(T + wtype)
+        w = O.quantize(oracle, (rng.standard_normal((M, K)) * 0.02).astype(np.float32), wtype)
+        x = rng.standard_normal((P, K)).astype(np.float32)
+        want = O.matmul(oracle, w, wtype, M, K, x, nthread=4)
+        dw, dx, out = dev(w), dev(np.resize(x, (T, K))), dev_empty(T * M * 4 + 64, 0xFF)
+        tw, tx = H.tensor(dw, wtype, [K, M]), H.tensor(dx, H.F32, [K, T])
+        need = L.spy_hip_op_matmul_scratch_size(B(tw), B(tx))
+        scratch = dev_empty(need, 0xEE)
+        call(L.spy_hip_op_matmul, None, B(tw), B(tx), B(H.tensor(out, H.F32, [M, T])), scratch.ptr, need)
+        got = out.download(np.float32)
+        assert (got[T * M:].view(np.uint32) == 0xFFFFFFFF).all()
+        got = got[:T * M].reshape(T, M)
+        if order == 1:
+            assert np.array_equal(got.view(np.uint32), np.resize(want, (T, M)).view(np.uint32))
+        else:
+            assert_close(got, np.resize(want, (T, M)), "own order, %d rows" % T, tol=1e-5)
+    finally:
+        L.spy_hip_set_exact_order(prev)

@@ -95,10 +95,15 @@ const char *spy_hip_error_string(int code);
  * target_buffer_type (mat.cpp:32-42): (Q4_0|Q8_0, F32) quantizes x to Q8_0, (F16, F32) rounds x
  * to fp16; additionally (Q4_K|Q6_K, F32) -> Q8_0 activations, which the reference lacks.
  * `scratch` holds the converted activations (the reference allocates it in get_control_header,
- * mat.cpp:61-68); query its size with spy_hip_op_matmul_scratch_size.  While the host's summation
- * order is on (spy_hip_set_exact_order) that size also covers the fp16 operands from which the MatMul
- * of several rows runs fastest in that order; a buffer that holds only the
- * activations (rows * row size of the converted type) is accepted too and gives the same results.
+ * mat.cpp:61-68); query its size with spy_hip_op_matmul_scratch_size.  A buffer that holds only the activations
+ * (rows * row size of the converted type) is accepted too.  The queried size covers more where the MatMul of several
+ * rows runs fastest from activations laid out as fp16 (and, in the host's order of Q4_0 / Q8_0, from fp16 copies of
+ * both operands where that layout does not apply).  With the host's summation order on (spy_hip_set_exact_order), and
+ * for Q4_0 / Q8_0 in this backend's own order, a smaller buffer changes the time a call takes and no bit of its result.
+ * Q4_K / Q6_K in the own order with 8 rows and more: the kernel follows from the shape for every buffer that holds the
+ * packed activations of 16 rows (36 bytes per column; the rows then go through it in pieces); below that, which is
+ * possible up to 33 rows, other kernels run, and their results differ in the last bits (fp32 rounding).  In the own order
+ * the kernel depends on the number of rows as well, and so do the last bits of a row's result.
  * One contiguous f32 row against a plain quantized matrix (the weight products of a single-token pass) is
  * quantized inside the launch that multiplies it and leaves `scratch` untouched, in either summation order. */
 size_t spy_hip_op_matmul_scratch_size(const spy_hip_tensor *w, const spy_hip_tensor *x);
@@ -106,13 +111,13 @@ int spy_hip_op_matmul(void *stream, const spy_hip_tensor *w, const spy_hip_tenso
                       void *scratch, size_t scratch_bytes);
 /* MatMul with no allocation anywhere -- no counterpart in the reference, whose MatMul allocates its activation buffer
  * per node (mat.cpp:61-68).  For callers that cannot allocate: code under HIP graph capture, tight serving loops,
- * harnesses that forbid hipMalloc.  Same operator and same results as spy_hip_op_matmul; the converted activations go
+ * harnesses that forbid hipMalloc.  Same operator and same results as spy_hip_op_matmul with a buffer of the queried size (rows of up
+ * to 233016 columns; longer ones of Q4_K / Q6_K see above); the converted activations go
  * to a fixed array in device memory (spy_hip_op_matmul_noalloc_max_scratch() bytes, 8 MiB, held by every device the
  * library runs on until the process ends) instead of a caller buffer.  Returns SPY_HIP_ENOSPACE when the converted
  * activations (rows * row size of the converted type) exceed that.  All calls on a device share the array: calls that overlap on one
- * device (different streams or threads) race, and a replay of a graph that recorded such a call counts as a call.  While
- * the host's summation order is on, the fp16 operand copies of spy_hip_op_matmul_scratch_size go into the array as well
- * when they fit behind the activations, and are left out (same results) when they do not. */
+ * device (different streams or threads) race, and a replay of a graph that recorded such a call counts as a call.  What else
+ * spy_hip_op_matmul_scratch_size asks for goes into the array as far as it fits, with the same results. */
 size_t spy_hip_op_matmul_noalloc_max_scratch(void);
 int spy_hip_op_matmul_noalloc(void *stream, const spy_hip_tensor *w, const spy_hip_tensor *x, const spy_hip_tensor *dst);
 /* NormRMS -- OperatorNormRMSImpl::execute (non-linear.cpp:194-223); eps = NormRMSParam::eps */

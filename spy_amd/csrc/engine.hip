@@ -369,7 +369,7 @@ bool spy_xgemm_ok(int wtype, const void *w, const float *dst, int64_t M, int64_t
 int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, int64_t K, void *pack);
 int spy_xgemm_norm_pack(hipStream_t st, bool own, const float *x, const float *w, float eps, int64_t T, int64_t K, void *pack);
 int spy_xgemm_silu_pack(hipStream_t st, const float *gate, const float *up, const float *lut, int64_t T, int64_t F, void *pack);
-int spy_xgemm_own(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
+int spy_xgemm_own(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack, int64_t T_all = 0);
 bool spy_gemm_unsplit_shape(int64_t M, int64_t T);                                                                               // gemm.hip
 int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
 int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, float *out, const float *lut,

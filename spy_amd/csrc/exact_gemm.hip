@@ -68,6 +68,7 @@ struct xt_args {
     const float *resid;                            // added to the result (matrix 0 only), or null
     int64_t w_row, d_row;                          // bytes per weight row; elements between the outputs of two activation rows
     int M, tiles, nst, ncg, T;                     // rows and row tiles per matrix, stages (K / 128), groups of 16 activation rows, activation rows
+    int ncg_all;                                   // groups of the whole call of which this is a piece
     const uint8_t *xq, *xd;
 };
 
@@ -1035,12 +1036,15 @@ int xk_dispatch(hipStream_t st, const xt_args &a, int nmat) {
     }
 }
 
-// the own order of the K-quants; as in xt_dispatch
+// the own order of the K-quants; as in xt_dispatch.  xks_kernel adds the terms in another order than the tiles: the choice is that of the whole call, so that
+// a call in pieces has its bits
 template <int WT>
 int xko_dispatch(hipStream_t st, const xt_args &a, int nmat) {
+    xt_args all = a;
+    all.ncg = a.ncg_all;
     static const xt_cost k4[6] = {{16, 1, 94, 43}, {32, 2, 235, 74}, {64, 2, 250, 128}, {32, 4, 330, 128}, {64, 4, 355, 185}, {64, 8, 560, 355}},
                          k6[6] = {{16, 1, 110, 56}, {32, 2, 230, 110}, {64, 2, 310, 196}, {32, 4, 315, 161}, {64, 4, 390, 254}, {64, 8, 560, 396}};
-    switch (xt_pick(a, nmat, WT == SPY_HIP_Q4_K ? k4 : k6, 6)) {
+    switch (xt_pick(all, nmat, WT == SPY_HIP_Q4_K ? k4 : k6, 6)) {
     case 0: return xks_launch<WT>(st, a, nmat);
     case 1: return xk_launch<WT, true, 2, 2, 4>(st, a, nmat);
     case 2: return xk_launch<WT, true, 4, 2, 4>(st, a, nmat);
@@ -1070,7 +1074,7 @@ size_t spy_xgemm_pack_bytes(int64_t T, int64_t K) {
 }
 // shapes and alignments the kernels take: whole chunks, 16-byte-aligned weight rows, four outputs stored together
 bool spy_xgemm_ok(int wtype, const void *w, const float *dst, int64_t M, int64_t K, int64_t T, int64_t d_row) {
-    return (wtype == SPY_HIP_Q4_0 || wtype == SPY_HIP_Q8_0 || wtype == SPY_HIP_Q4_K || wtype == SPY_HIP_Q6_K) && T >= 2 && T <= 16 * 65535 && K > 0 && K % 256 == 0 && K <= (1 << 20) && M > 0 && M % 4 == 0 && M < (1 << 24) &&
+    return (wtype == SPY_HIP_Q4_0 || wtype == SPY_HIP_Q8_0 || wtype == SPY_HIP_Q4_K || wtype == SPY_HIP_Q6_K) && T >= 1 && T <= 16 * 65535 && K > 0 && K % 256 == 0 && K <= (1 << 20) && M > 0 && M % 4 == 0 && M < (1 << 24) &&
            ((uintptr_t)w & 15) == 0 && ((uintptr_t)dst & 15) == 0 && d_row % 4 == 0;
 }
 int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, int64_t K, void *pack) {
@@ -1109,7 +1113,7 @@ static int xt_fill(xt_args &a, int wtype, int nmat, const void *const *w, float 
         a.dst[i] = dst[i];
     }
     a.resid = resid; a.w_row = spy_row_size(wtype, K); a.d_row = d_row;
-    a.M = (int)M; a.nst = (int)(K / 128); a.ncg = (int)((T + 15) / 16); a.T = (int)T;
+    a.M = (int)M; a.nst = (int)(K / 128); a.ncg = a.ncg_all = (int)((T + 15) / 16); a.T = (int)T;
     a.xq = (const uint8_t *)pack; a.xd = a.xq + (int64_t)a.ncg * a.nst * XT_XB;
     return 0;
 }
@@ -1125,10 +1129,11 @@ int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *
     default: return xk_dispatch<SPY_HIP_Q6_K>(st, a, nmat);
     }
 }
-// the same in this backend's own order; Q4_0, Q4_K, Q6_K (Q8_0 unpacks more per block than Q4_0: 3 % slower than the tile kernel of gemm.hip at 22016 rows)
-int spy_xgemm_own(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack) {
+// the same in this backend's own order; T_all: rows of the whole call where it comes in pieces (0: this is all of it); Q4_0, Q4_K, Q6_K (Q8_0 unpacks more per block than Q4_0: 3 % slower than the tile kernel of gemm.hip at 22016 rows)
+int spy_xgemm_own(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack, int64_t T_all) {
     xt_args a;
     const int rc = xt_fill(a, wtype, nmat, w, dst, M, K, T, d_row, resid, pack);
     if (rc) return rc;
+    if (T_all > T) a.ncg_all = (int)((T_all + 15) / 16);
     return wtype == SPY_HIP_Q4_0 ? xo_dispatch(st, a, nmat) : wtype == SPY_HIP_Q4_K ? xko_dispatch<SPY_HIP_Q4_K>(st, a, nmat) : wtype == SPY_HIP_Q6_K ? xko_dispatch<SPY_HIP_Q6_K>(st, a, nmat) : SPY_HIP_EINVAL;
 }

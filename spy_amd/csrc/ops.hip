@@ -7,6 +7,8 @@
 
 #include <math.h>
 
+#include <algorithm>
+
 int *spy_hip_err_flag_ptr();
 
 // exact_order.hip: the same operators with every sum in the host backend's order (spy_hip_set_exact_order)
@@ -23,7 +25,7 @@ size_t spy_exact_pack_bytes(int64_t ne01, int64_t ne00, int64_t ne11);
 size_t spy_xgemm_pack_bytes(int64_t T, int64_t K);
 bool spy_xgemm_ok(int wtype, const void *w, const float *dst, int64_t M, int64_t K, int64_t T, int64_t d_row);
 int spy_xgemm_pack(hipStream_t st, const float *x, int64_t x_stride, int64_t T, int64_t K, void *pack);
-int spy_xgemm_own(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
+int spy_xgemm_own(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack, int64_t T_all = 0);
 int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
 
 struct tdesc {              // a tensor as the kernels see it
@@ -754,8 +756,9 @@ static bool xgemm_rows(int wtype, int64_t M, int64_t T) {
     if (spy_exact_on()) return T >= 3;
     return wtype == SPY_HIP_Q4_K || wtype == SPY_HIP_Q6_K ? T >= 8 : wtype == SPY_HIP_Q4_0 && spy_gemm_unsplit_shape(M, T);
 }
-// ... plus, while the exact summation order is on, room for the fp16 copies of both operands that its prompt-sized Q4_0 / Q8_0
-// MatMul runs from (a call with less than this, but the activations' part, runs the kernel that unpacks per tile: same results)
+// The activations' part, or what the kernels of exact_gemm.hip pack where they run.  In the host's order of Q4_0 / Q8_0 also room behind the activations
+// for the fp16 copies of both operands from which exact_gemm8p_kernel runs: K that is no multiple of 256, operands off the 16-byte grid.
+// With less (but the activations' part) the results are the same in that order; for K-quants in the own order see matmul_impl.
 extern "C" size_t spy_hip_op_matmul_scratch_size(const spy_hip_tensor *w, const spy_hip_tensor *x) {
     const size_t act = matmul_act_bytes(w, x);
     if (!act || x->type != SPY_HIP_F32 || mid_type(w->type, x->type) != SPY_HIP_Q8_0 || w->ne[2] != 1 || w->ne[3] != 1) return act;
@@ -802,8 +805,8 @@ static int matmul_f16_launch(hipStream_t st, const spy_hip_tensor *w, const uint
 }
 static int matmul_impl(void *stream, const spy_hip_tensor *w, const spy_hip_tensor *x, const spy_hip_tensor *dst, void *scratch, size_t scratch_bytes,
                        int skip_past, int klimit_past, bool own_kernels = false);
-// MatMul by the kernels of this backend's own order whatever the number of rows: the token loop's passes in that order, whose results do not depend on
-// how long a prompt is
+// MatMul without the kernels of exact_gemm.hip: the token loop's passes in this backend's own order.  The fused steps of such a pass leave Q8_0 blocks, which
+// the kernels of gemm.hip read, and the products between them that come through here stay with the same kernels.
 int spy_matmul_own(void *stream, const spy_hip_tensor *w, const spy_hip_tensor *x, const spy_hip_tensor *dst, void *scratch, size_t scratch_bytes) {
     return matmul_impl(stream, w, x, dst, scratch, scratch_bytes, -1, -1, true);
 }
@@ -844,18 +847,32 @@ static int matmul_impl(void *stream, const spy_hip_tensor *w, const spy_hip_tens
                                       : own_matvec(st, t0, w->data, (const float *)x->data, (float *)dst->data, ne01, ne00);
         if (rc != SPY_HIP_EUNSUPPORTED) return rc;
     }
-    // several rows: the kernels of exact_gemm.hip where they take the matrix and the scratch buffer holds the packed activations
+    // several rows: the kernels of exact_gemm.hip where they take the matrix and the scratch buffer holds the packed activations (K-quants in the own
+    // order: 16 rows of them)
     // (SPY_HIP_EXACT_TILED=u / 0, SPY_HIP_EXACT_SERIAL: tests of the other kernels)
     if (quant && t1 == SPY_HIP_F32 && xgemm_rows(t0, ne01, ne11) && !own_kernels && ne12 == 1 && ne13 == 1 && skip_past < 0 && klimit_past < 0 && x->nb[0] == 4 && x->nb[1] % 16 == 0 &&
         ((uintptr_t)x->data & 15) == 0 && dst->nb[1] % 16 == 0 && w->nb[0] == spy_type_size(t0) && w->nb[1] == spy_row_size(t0, ne00) &&
         spy_xgemm_ok(t0, w->data, (const float *)dst->data, ne01, ne00, ne11, dst->nb[1] / 4)) {
         const char *tiled = getenv("SPY_HIP_EXACT_TILED");
-        const size_t need = spy_xgemm_pack_bytes(ne11, ne00);
-        if (scratch && ((uintptr_t)scratch & 15) == 0 && scratch_bytes >= need && !(tiled && (*tiled == '0' || *tiled == 'u')) && !getenv("SPY_HIP_EXACT_SERIAL")) {
+        const size_t need = spy_xgemm_pack_bytes(ne11, ne00), group = spy_xgemm_pack_bytes(16, ne00);
+        // K-quants in the own order: in pieces of as many groups of 16 rows as the buffer holds, because the kernels further down add in another order (what a
+        // call gives would depend on the room it was given); in the host's order and for Q4_0 all kernels have the same bits
+        const bool pieces = !spy_exact_on() && t0 != SPY_HIP_Q4_0;
+        if (scratch && ((uintptr_t)scratch & 15) == 0 && scratch_bytes >= (pieces ? std::max(std::min(group, need), matmul_act_bytes(w, x)) : need) && !(tiled && (*tiled == '0' || *tiled == 'u')) && !getenv("SPY_HIP_EXACT_SERIAL")) {
             const void *wp = w->data;
             float *dp = (float *)dst->data;
+            if (!spy_exact_on()) {
+                const int64_t rows = scratch_bytes >= need ? ne11 : (int64_t)(scratch_bytes / group) * 16;
+                int rc = 0;
+                for (int64_t i = 0; i < ne11 && !rc; i += rows) {
+                    const int64_t n = ne11 - i < rows ? ne11 - i : rows;
+                    float *di = (float *)((uint8_t *)dp + i * dst->nb[1]);
+                    rc = spy_xgemm_pack(st, (const float *)((const uint8_t *)x->data + i * x->nb[1]), x->nb[1], n, ne00, scratch);
+                    if (!rc) rc = spy_xgemm_own(st, t0, 1, &wp, &di, ne01, ne00, n, dst->nb[1] / 4, nullptr, scratch, ne11);
+                }
+                return rc;
+            }
             const int rc = spy_xgemm_pack(st, (const float *)x->data, x->nb[1], ne11, ne00, scratch);
-            if (!rc && !spy_exact_on()) return spy_xgemm_own(st, t0, 1, &wp, &dp, ne01, ne00, ne11, dst->nb[1] / 4, nullptr, scratch);
             return rc ? rc : spy_xgemm(st, t0, 1, &wp, &dp, ne01, ne00, ne11, dst->nb[1] / 4, nullptr, scratch);
         }
     }

@@ -113,3 +113,39 @@ def test_matmul_of_about_a_million_rows(oracle, order, wtype, T):
             assert_close(got, np.resize(want, (T, M)), "own order, %d rows" % T, tol=1e-5)
     finally:
         L.spy_hip_set_exact_order(prev)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wtype,M,K,T", [(O.Q4_K, 36, 512, 40), (O.Q4_K, 4096, 512, 400), (O.Q4_K, 260, 11008, 400), (O.Q4_K, 1028, 256, 34), (O.Q4_K, 12288, 256, 129),
+                                         (O.Q6_K, 36, 512, 40), (O.Q6_K, 4096, 512, 400), (O.Q6_K, 260, 11008, 400), (O.Q6_K, 1028, 256, 49), (O.Q4_0, 4096, 1024, 400)])
+def test_own_order_result_does_not_depend_on_the_scratch_buffer(oracle, wtype, M, K, T):
+    """MatMul in this backend's own order with the queried buffer, with room for the activations as Q8_0 blocks only (the packed rows go through it in pieces: one group of
+    16, several, a last piece of one row), and from the fixed array of the entry point that allocates nothing: the same bits.  Too little is refused as before."""
+    from tests.gpu_util import assert_close, call, dev, dev_empty
+    H.init(0)
+    L = H.load()
+    prev = L.spy_hip_set_exact_order(0)
+    try:
+        rng = np.random.default_rng(M + K + T)
+        w = O.quantize(oracle, (rng.standard_normal((M, K)) * 0.02).astype(np.float32), wtype)
+        x = rng.standard_normal((T, K)).astype(np.float32)
+        want = O.matmul(oracle, w, wtype, M, K, x, nthread=8)
+        tw, tx, out = H.tensor(dev(w), wtype, [K, M]), H.tensor(dev(x), H.F32, [K, T]), dev_empty(T * M * 4 + 64, 0xFF)
+        to = H.tensor(out, H.F32, [M, T])
+        need, act, group = L.spy_hip_op_matmul_scratch_size(B(tw), B(tx)), T * K // 32 * 34, 36 * K
+        assert need == (T + 15) // 16 * group
+        scratch = dev_empty(need, 0xEE)
+        got = {}
+        for room in [need, act, max(act, group + 16), max(act, 2 * group + group // 2), need - 16, None]:
+            out.fill(0xFF)
+            if room is None: call(L.spy_hip_op_matmul_noalloc, None, B(tw), B(tx), B(to))
+            else: call(L.spy_hip_op_matmul, None, B(tw), B(tx), B(to), scratch.ptr, room)
+            r = out.download(np.float32)
+            assert (r[T * M:].view(np.uint32) == 0xFFFFFFFF).all(), "nothing is written beyond the outputs"
+            got[room] = r[:T * M]
+        assert_close(got[need].reshape(T, M), want, "own-order matmul type %d %dx%d T=%d" % (wtype, M, K, T), tol=1e-5)
+        for room, r in got.items():
+            assert np.array_equal(r.view(np.uint32), got[need].view(np.uint32)), (room, need)
+        assert L.spy_hip_op_matmul(None, B(tw), B(tx), B(to), scratch.ptr, act - 16) == H.ENOSPACE
+    finally:
+        L.spy_hip_set_exact_order(prev)

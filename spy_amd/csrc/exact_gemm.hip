@@ -37,12 +37,16 @@ typedef float xt_v16f __attribute__((ext_vector_type(16)));
 
 // 16 (4) bytes per lane from base + off to LDS bytes lds .. in lane order; base and lds are uniform over the wave.  Written as
 // instructions so that the compiler does not wait for them at the next LDS read; xt_wait_vm says when they have to be there.
+// (m0 among the clobbers keeps the compiler's own uses of it, if it has any, apart from these; it warns that the register is a reserved one.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void xt_dma16(const void *base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(off), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
 __device__ __forceinline__ void xt_dma4(const void *base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" :: "s"(lds), "v"(off), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" :: "s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 // at most N of the wave's requests are still on their way (they complete in order), and its LDS reads are done
 template <int N> __device__ __forceinline__ void xt_wait_vm() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(N) : "memory"); }
 

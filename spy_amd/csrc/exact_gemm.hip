@@ -989,22 +989,13 @@ int xks_launch(hipStream_t st, xt_args a, int nmat) {
     return SPY_LAUNCH_RC();
 }
 
-int xt_num_cu() {
-    static int n = 0;                              // the same value whoever writes it
-    if (!n) {
-        int dev = 0, v = 0;
-        n = hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0 ? v : 256;
-    }
-    return n;
-}
-
 // Which tile.  n workgroups per compute unit take about lat + (n - 1) * inc: figures in tenths of a microsecond for K = 4096, measured for
 // n = 1 .. 16 (whole workgroups count while they are few; everything scales with K).  Small tiles have the shorter chain, large ones unpack a
 // weight for more activation rows.
 // rest: what a workgroup of the ncg % groups groups that remain takes, 0 if it is a whole one.
 struct xt_cost { int rows, groups, lat, inc, rest = 0; };
 int xt_pick(const xt_args &a, int nmat, const xt_cost *c, int n) {
-    const int64_t cu = xt_num_cu();
+    const int64_t cu = spy_num_cu();
     int best = 0;
     int64_t least = 0;
     for (int i = 0; i < n; i++) {

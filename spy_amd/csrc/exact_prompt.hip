@@ -273,14 +273,6 @@ __global__ __launch_bounds__(64 * NW) void xp_softmax_kernel(const float *__rest
         __builtin_amdgcn_wave_barrier();
     }
 }
-int xp_num_cu() {
-    static int n = 0;                              // the same value whoever writes it
-    if (!n) {
-        int dev = 0, v = 0;
-        n = hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0 ? v : 256;
-    }
-    return n;
-}
 template <int R, int NW>
 int xp_softmax_launch(hipStream_t st, const float *S, uint16_t *P16, const float *lut, int T, int H, int P, int64_t s_row, int n_total, float scale, int ncu) {
     constexpr size_t lds = (XP_LUT + 4 + NW * (80 * R + 4)) * 4;
@@ -460,7 +452,7 @@ int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint1
     else if (one) xp_scores_kernel<false, true><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
     else xp_scores_kernel<false, false><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
     if (hipGetLastError() != hipSuccess) return SPY_HIP_EINVAL;
-    const int ncu = xp_num_cu(), rc = (int64_t)P + T <= 4096 ? xp_softmax_launch<16, 12>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
+    const int ncu = spy_num_cu(), rc = (int64_t)P + T <= 4096 ? xp_softmax_launch<16, 12>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
                                          : (int64_t)P + T <= 6144 ? xp_softmax_launch<24, 8>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
                                                                   : xp_softmax_launch<32, 4>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu);
     if (rc) return rc;

@@ -148,8 +148,7 @@ static int launch_wave_row_nr(hipStream_t st, const gemv_args &a, int T, size_t 
 // matrices beyond 8 rows per wave take more workgroups.
 template <int WT, int NITK>
 static int launch_wave_row_nitk(hipStream_t st, const gemv_args &a, int T) {
-    static int num_cu = 0;
-    if (!num_cu) { int dev = 0; hipDeviceProp_t prop; num_cu = (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess) ? prop.multiProcessorCount : 256; }
+    const int num_cu = spy_num_cu();
     const size_t lds = (size_t)T * staged_bytes(a.K);
     const int waves = WROW_THREADS / 64;
     const int64_t need = ((int64_t)a.M + (int64_t)num_cu * waves - 1) / ((int64_t)num_cu * waves);
@@ -271,23 +270,12 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_generic_kernel(const uint8_
     }
 }
 
-
-static int g_num_cu = 0;
-static int num_cu() {
-    if (!g_num_cu) {
-        int dev = 0; hipDeviceProp_t prop;
-        if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess) g_num_cu = prop.multiProcessorCount;
-        if (g_num_cu <= 0) g_num_cu = 256;
-    }
-    return g_num_cu;
-}
-
 // workgroups of `kern` that fit on the device at once (persistent kernels launch exactly that many)
 template <class Kern>
 static int resident_blocks(Kern kern, size_t lds) {
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, GEMV_THREADS, lds) != hipSuccess || per_cu < 1) per_cu = 1;
-    return per_cu * num_cu();
+    return per_cu * spy_num_cu();
 }
 
 template <int WT, int LPR, int NIT, int NT, bool DUMP>

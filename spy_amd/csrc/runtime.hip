@@ -6,6 +6,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -26,6 +27,18 @@ int *spy_hip_err_flag_ptr() {
 }
 int spy_static_scratch_setup(int device);    // ops.hip: address of the fixed scratch array on the current device
 int spy_exact_device_setup();                // exact_order.hip: the exp / silu tables of the current device
+
+// Compute units of the current device (256 where it does not say); asked once per device
+int spy_num_cu() {
+    static std::atomic<int> n[SPY_MAX_DEVICES];
+    int dev = -1, v = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= SPY_MAX_DEVICES) return 256;
+    const int have = n[dev].load(std::memory_order_relaxed);
+    if (have) return have;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
+    n[dev].store(v, std::memory_order_relaxed);
+    return v;
+}
 
 // A kernel's dynamic-LDS limit (hipFuncAttributeMaxDynamicSharedMemorySize) belongs to the kernel function on a device for the
 // whole process, whoever launches it: it is kept here per (device, kernel) and only ever raised, so that an engine or operator

@@ -15,3 +15,10 @@ def test_inline_assembly_names_the_m0_it_writes():
                 found += 1
                 assert m.group(1).rsplit(":", 1)[1].count('"m0"') == 1, (path, m.group(0))
     assert found >= 2
+
+
+def test_the_number_of_compute_units_is_kept_per_device():
+    """The launchers ask spy_num_cu (runtime.hip, one record per device) and keep no number of their own; an engine keeps that of its device (peaks.hip, the measured ceilings, asks on every call)."""
+    for path in sorted(glob.glob(os.path.join(ROOT, "spy_amd", "csrc", "*.hip")) + glob.glob(os.path.join(ROOT, "spy_amd", "csrc", "*.cuh"))):
+        if os.path.basename(path) not in ("runtime.hip", "engine.hip", "peaks.hip"):
+            assert not re.search("multiprocessorcount", open(path).read(), re.I), path

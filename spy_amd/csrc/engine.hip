@@ -497,18 +497,22 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
                  o_ids = take(T * 4), o_pos = take(T * 4), o_logits = take(head == HEAD_ALL ? V * T * 4 : V * 4), o_rt = take(T * hd * 4);
     const size_t act_q8 = (size_t)T * ((F > d ? F : d) / 32) * 34;
     const size_t act_f16 = sp_bytes / 2 > (size_t)d * T * 2 ? sp_bytes / 2 : (size_t)d * T * 2;
-    // exact order: room behind the activations for the packed fp16 operands of the largest MatMul (spy_exact_pack_bytes)
+    // exact order: room behind the activations for the fp16 copies of both operands (spy_exact_pack_bytes), where a product does not run from packed
+    // activations alone
     size_t pack = 0;
-    if (exact && T >= 16) {
-        const int64_t shapes[3][2] = {{d, d}, {F, d}, {d, F}};
-        for (auto &sh : shapes) { const size_t b = spy_exact_pack_bytes(sh[0], sh[1], T); pack = b > pack ? b : pack; }
-    }
-    const size_t xpack = exact && T >= 2 ? spy_xgemm_pack_bytes(T, F > d ? F : d) : 0;
+    if (exact && T >= 16)
+        for (const spy_hip_llama_layer &L : m->layers) {
+            const struct { const void *w; int t; int64_t M, K; } prod[7] = {{L.wq, L.t_wq, d, d}, {L.wk, L.t_wk, d, d}, {L.wv, L.t_wv, d, d}, {L.wo, L.t_wo, d, d},
+                                                                            {L.w_gate, L.t_gate, F, d}, {L.w_up, L.t_up, F, d}, {L.w_down, L.t_down, d, F}};
+            for (const auto &p : prod)
+                if ((p.t == SPY_HIP_Q4_0 || p.t == SPY_HIP_Q8_0) && !spy_xgemm_ok(p.t, p.w, nullptr, p.M, p.K, T, p.M)) pack = std::max(pack, spy_exact_pack_bytes(p.M, p.K, T));
+        }
+    const size_t packed = std::max(spy_xgemm_pack_bytes(T, d), spy_xgemm_pack_bytes(T, F)), xpack = exact && T >= 2 ? packed : 0;
     // own order, Q4_0 weights: where a product is large enough for gemm.hip not to split K, it runs from packed activations instead
     // (exact_gemm.hip: same bits, tiles that fill the chip better, wq | wk | wv in one launch)
     auto x_ok = [&](int t, const void *w, int64_t M, int64_t K) { return fuse_act && t == SPY_HIP_Q4_0 && d <= 8192 && K % 256 == 0 && spy_gemm_unsplit_shape(M, T) && spy_xgemm_ok(t, w, nullptr, M, K, T, M); };
     const bool any_x = fuse_act && (spy_gemm_unsplit_shape(d, T) || spy_gemm_unsplit_shape(F, T));
-    const size_t o_scr = take(std::max((act_q8 > act_f16 ? act_q8 : act_f16) + 256 + pack, std::max(xpack, any_x ? spy_xgemm_pack_bytes(T, F > d ? F : d) : 0)));
+    const size_t o_scr = take(std::max((act_q8 > act_f16 ? act_q8 : act_f16) + 256 + pack, std::max(xpack, any_x ? packed : 0)));
     const size_t scr_bytes = off - o_scr;
     RC_TRY(ops_workspace(m, st, off));
     uint8_t *B = m->ops_buf;

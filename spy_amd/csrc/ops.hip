@@ -757,7 +757,8 @@ static bool xgemm_rows(int wtype, int64_t M, int64_t T) {
     return wtype == SPY_HIP_Q4_K || wtype == SPY_HIP_Q6_K ? T >= 8 : wtype == SPY_HIP_Q4_0 && spy_gemm_unsplit_shape(M, T);
 }
 // The activations' part, or what the kernels of exact_gemm.hip pack where they run.  In the host's order of Q4_0 / Q8_0 also room behind the activations
-// for the fp16 copies of both operands from which exact_gemm8p_kernel runs: K that is no multiple of 256, operands off the 16-byte grid.
+// for the fp16 copies of both operands from which exact_gemm8p_kernel runs: K that is no multiple of 256, weights off the 16-byte grid (asked by shape: a
+// caller may size the buffer before its tensors have addresses).
 // With less (but the activations' part) the results are the same in that order; for K-quants in the own order see matmul_impl.
 extern "C" size_t spy_hip_op_matmul_scratch_size(const spy_hip_tensor *w, const spy_hip_tensor *x) {
     const size_t act = matmul_act_bytes(w, x);

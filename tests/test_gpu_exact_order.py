@@ -157,6 +157,33 @@ def test_tiled_matmul_bits(hip, oracle, wtype, M, K, T, monkeypatch):
         assert need > act + 2 * (M + T) * K, "the scratch size of the exact order covers the packed operands"
 
 
+@pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0])
+@pytest.mark.parametrize("M,K,T,off", [(160, 4224, 40, 0), (4096, 4224, 64, 0), (200, 384, 70, 0), (132, 4096, 130, 4), (96, 512, 17, 8)])
+def test_tiled_matmul_bits_where_activations_are_not_packed(hip, oracle, wtype, M, K, T, off):
+    """Contractions that are no multiple of 256 and weights off the 16-byte grid stay with the 64 x 64 tiles: from fp16 copies of both operands where the scratch buffer
+    has room for them, unpacking per tile where it holds the activations only, and one or the other from the fixed array of the entry point that allocates
+    nothing.  The oracle's bits each time."""
+    from tests.gpu_util import dev, dev_empty, call
+    rng = np.random.default_rng(5 * wtype + M + K + T)
+    w = O.quantize(oracle, (rng.standard_normal((M, K)) * 0.02).astype(np.float32), wtype)
+    x = (rng.standard_normal((T, K)) * rng.uniform(0.1, 30.0, (T, 1))).astype(np.float32)
+    want = O.matmul(oracle, w, wtype, M, K, x, nthread=8)
+    dw = dev(np.concatenate([np.zeros(off, np.uint8), w.view(np.uint8).reshape(-1)]))
+    tw, tx = hip.tensor(dw.ptr + off, wtype, [K, M]), hip.tensor(dev(x), hip.F32, [K, T])
+    L = hip.load()
+    need, act = L.spy_hip_op_matmul_scratch_size(B(tw), B(tx)), T * (K // 32) * 34
+    assert need > act + 2 * (M + T) * K, "room for the copies of both operands"
+    scratch, dd = dev_empty(need, 0xEE), dev_empty(T * M * 4 + 64, 0xFF)
+    td = hip.tensor(dd, hip.F32, [M, T])
+    for room in (need, act, None):
+        dd.fill(0xFF)
+        if room is None: call(L.spy_hip_op_matmul_noalloc, None, B(tw), B(tx), B(td))
+        else: call(L.spy_hip_op_matmul, None, B(tw), B(tx), B(td), scratch.ptr, room)
+        got = dd.download(np.float32)
+        _same_bits(got[:T * M].reshape(T, M), want, "tiled matmul type %d %dx%d T %d, scratch %s" % (wtype, M, K, T, room))
+        assert (got[T * M:].view(np.uint32) == 0xFFFFFFFF).all(), "nothing is written beyond the outputs"
+
+
 @pytest.mark.parametrize("T", [1, 2, 40])
 def test_q8_0_weights_of_any_byte(hip, oracle, T):
     """Weight bytes a quantizer never writes (-128): the host backend's sign / maddubs sequence

@@ -245,7 +245,7 @@ def main():
         ops_set = 2.0 * Tg * (4 * d_ * d_ + 3 * d_ * F_)
         tops = ops_set / us_set / 1e6
         gemm_roofline = {"summation_order": 0,
-                         "kernel": "gemm_q8act_kernel, the prompt GEMM of summation order 0 (NOT what the headline order's prompt runs: that is prompt_gemm_roofline): quantized GEMMs of one layer (%s weights x Q8_0 activations, int8 MFMA, per-block scales): 4 x %dx%d, 2 x %dx%d, 1 x %dx%d, %d activation rows"
+                         "kernel": "gemm_q8act_kernel, a prompt GEMM of summation order 0 (NOT what the headline order's prompt runs: that is prompt_gemm_roofline; order 0's own prompts run it for Q8_0, and xo_kernel for Q4_0 products of this size): quantized GEMMs of one layer (%s weights x Q8_0 activations, int8 MFMA, per-block scales): 4 x %dx%d, 2 x %dx%d, 1 x %dx%d, %d activation rows"
                                    % ({H.Q4_0: "Q4_0", H.Q8_0: "Q8_0", H.Q4_K: "Q4_K", H.Q6_K: "Q6_K"}[wt_g], d_, d_, F_, d_, d_, F_, Tg),
                          "bound": "mfma", "achieved": round(tops, 1), "peak": INT8_PEAK / 1e12, "unit": "TOP/s", "frac": round(tops * 1e12 / INT8_PEAK, 4),
                          "ops_per_set": ops_set, "us_per_set": round(us_set, 1)}
@@ -257,7 +257,7 @@ def main():
         log("prompt GEMMs of a layer, T = %d: %.1f us, %.0f TOP/s (%.1f%% of the int8 MFMA peak); its inner loop on register operands only: %.0f TOP/s (%.1f%%)"
             % (Tg, us_set, tops, 100 * tops * 1e12 / INT8_PEAK, ceil_tops.value, 100 * ceil_tops.value * 1e12 / INT8_PEAK))
         # The same seven products the way the prompt pass of summation order 1 runs them: spy_hip_op_matmul in the host backend's
-        # order = Q8_0 quantization of the f32 activations, both operands packed as fp16, exact_gemm8p_kernel (integer sums of
+        # order = xt_pack_kernel (f32 activations quantized to Q8_0 and laid out as fp16) and xt_kernel (integer sums of
         # four products from v_mfma_f32_16x16x4_4b_f16, one fma per accumulator and block on the vector units).
         gemm_roofline_o1 = None
         if cfg.wtype in (H.Q4_0, H.Q8_0):
@@ -281,7 +281,7 @@ def main():
                 us1 = ms.value * 1000.0 / n_set1
                 tops1 = ops_set / us1 / 1e6
                 gemm_roofline_o1 = {"summation_order": 1,
-                                    "kernel": "exact_gemm8p_kernel + xgp_pack_kernel x 2 + Q8_0 quantization, the prompt MatMul of summation order 1 (the headline's): the same seven products "
+                                    "kernel": "xt_pack_kernel + xt_kernel, the prompt MatMul of summation order 1 (the headline's): the same seven products "
                                               "through spy_hip_op_matmul in the host backend's order; integer sums of four products from v_mfma_f32_16x16x4_4b_f16 (fp16 matrix instructions), "
                                               "one fp32 fma per accumulator and block on the vector units",
                                     "bound": "mfma", "achieved": round(tops1, 1), "peak": INT8_PEAK / 1e12, "unit": "TOP/s", "frac": round(tops1 * 1e12 / INT8_PEAK, 4),

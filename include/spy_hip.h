@@ -173,8 +173,8 @@ int spy_hip_take_error(int *flag);   /* reads and clears the device error flag (
  * Dot<Q8_0,Q8_0> and Dot<FP16,FP16> (vec_dot.h:42-146, vec_util.h:75-81), libstdc++'s four-way std::reduce in
  * NormRMS and Softmax (non-linear.cpp:129-223) -- and take exp / silu from tables and the Rope angles from the
  * host's libm (lookup_table_impl/non-linear.h:39-47,131-139, non-linear.cpp:270-371), so that every operator
- * output equals the host backend's bit for bit.  A checking mode, about 12 x slower than the fused token
- * loop.  spy_hip_llama_forward / _forward_last / _decode_greedy follow it: every pass runs operator by operator
+ * output equals the host backend's bit for bit.  spy_hip_llama_forward / _forward_last / _decode_greedy follow it: a model
+ * that the passes of summation order 1 take runs those, any other operator by operator
  * (the prompt as one pass, the greedy loop with the argmax on the host).  With RopeParam::num_context > 0 the
  * rotations of all positions are kept in a device table and a position outside it raises the error flag of
  * spy_hip_take_error; with num_context == 0 Rope reads the positions back and synchronises the stream. */
@@ -329,7 +329,7 @@ int spy_hip_llama_forward_last(spy_hip_llama *m, void *stream, const int32_t *to
 int spy_hip_llama_decode_greedy(spy_hip_llama *m, void *stream, int32_t first_token, int32_t n_past, int32_t n_steps,
                                 int32_t *tokens_host, int32_t use_graph);
 /* Summation order of the model's passes: of the fused single-token pass, and of prompt passes (in order 1 they run
- * operator by operator through the exact-order kernels, in order 0 on the matrix cores).  1 (the default wherever the kernels take the model: 128-wide heads,
+ * through the exact-order kernels, in order 0 on the matrix cores).  1 (the default wherever the kernels take the model: 128-wide heads,
  * n_embd and n_ff multiples of 128): the host backend's -- the eight accumulators and hsum_float_8 of its quantized dots,
  * the 4 x 8 accumulators, tree and scalar tail of its fp16 dots (vec_dot.h:42-146), libstdc++'s four-way reduce in
  * NormRMS and Softmax (non-linear.cpp:129-223), exp / silu from the fp16-indexed tables and the RoPE angles from the

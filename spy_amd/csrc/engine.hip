@@ -2,8 +2,8 @@
 // (model/src/llm/model/llama.cpp:86-264 and plugins in the Spy tree) for a single new token as
 // six fused kernels per layer, greedy sampling on the device (greedy.h:20-25, cli.h:88-128), the
 // whole pass captured once as a HIP graph and replayed per token.  Passes over several tokens
-// (prompts) run operator by operator through the spy_hip_op_* entry points, exactly as the graph
-// lists them.
+// (prompts) run the graph's operators with what lies between two MatMuls in the kernels around them, or
+// operator by operator through the spy_hip_op_* entry points for the shapes those do not take.
 #define SPY_DECODE_COMMON_KERNELS
 #include "engine_types.cuh"
 #include "exact_decode.cuh"
@@ -331,7 +331,7 @@ static int enqueue_pass_any(spy_hip_llama *m, hipStream_t st, int mode) {
     return 0;
 }
 
-// ---- passes over several tokens: operator by operator --------------------------------------------
+// ---- passes over several tokens -----------------------------------------------------------------
 static spy_hip_tensor T2(int type, void *p, int64_t e0, int64_t e1) {
     spy_hip_tensor t;
     t.type = type; t.dim = 2; t.data = p;

@@ -810,7 +810,7 @@ __global__ __launch_bounds__(256, 3) void xks_kernel(xt_args a) {
 // (the arithmetic and the bits of gemm_q8act_kernel in gemm.hip).  The block dot of a 16 x 16 tile is one v_mfma_f32_16x16x32_f16, a float and exact,
 // and the scale products of four blocks are one 16x16x4_4b as above: 24 matrix-core cycles and four fmas (16 cycles) per tile and block, where
 // the int8 form takes a 35-cycle instruction, a 32-cycle one and two vector instructions per output of a 32 x 32 tile.
-// Matrix and vector cycles of these instructions add up here (counters: both together 70 % of the time with two or three waves per SIMD), which is
+// Matrix and vector cycles of these instructions add up here (counters at 1000 rows: vector 36 %, matrix 38 %, at once 13 % of the time), which is
 // why the cycles above are what counts; and the tiles fill the chip better than 128 x 128 ones.  Packing included, Q4_0, 4096 x 4096: 385 rows 66 -> 46 us,
 // 512 rows 68 -> 48, 600 rows 96 -> 64, 1000 rows 94 -> 75, 2048 rows 118 -> 117; 4096 x 11008: 512 rows 164 -> 112, 1000 rows 228 -> 184;
 // 22016 x 4096: 77 rows 85 -> 62, 320 rows 152 -> 131, 1000 rows 314 -> 302.

@@ -124,9 +124,9 @@ def test_packed_activation_matmul_bits(hip, oracle, wtype, M, K, T):
 @pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0, O.Q4_K, O.Q6_K])
 @pytest.mark.parametrize("M,K,T", [(96, 4096, 16), (200, 512, 70), (64, 128, 64), (64, 256, 64), (132, 11008, 33), (4096, 4096, 130)])
 def test_tiled_matmul_bits(hip, oracle, wtype, M, K, T, monkeypatch):
-    """Sixteen activation rows and more take the tiled kernel (64 x 64 outputs per workgroup, the eight accumulators
-    of every output in registers): the oracle's bits, with whole and partial tiles along both sides, and the same
-    bits as the row kernels give (SPY_HIP_EXACT_TILED=0)."""
+    """Sixteen activation rows and more: the kernels from packed activations (K = 128: the tiled kernel from fp16 copies of both operands), the tiled kernel
+    that unpacks per tile (SPY_HIP_EXACT_TILED=u, and a scratch buffer that holds the Q8_0 activations only; 64 x 64 outputs per workgroup, the eight accumulators
+    of every output in registers) and the row kernels (SPY_HIP_EXACT_TILED=0): the oracle's bits, with whole and partial tiles along both sides."""
     from tests.gpu_util import dev, dev_empty, call
     if K % 256 and wtype in (O.Q4_K, O.Q6_K):
         pytest.skip("K-quant rows are whole super-blocks")
@@ -139,7 +139,7 @@ def test_tiled_matmul_bits(hip, oracle, wtype, M, K, T, monkeypatch):
     L = hip.load()
     need = L.spy_hip_op_matmul_scratch_size(B(tw), B(tx))
     scratch = dev_empty(need, 0)
-    for tiled in ("1", "u", "0"):          # tiled kernel from packed operands, unpacking per tile, row kernels
+    for tiled in ("1", "u", "0"):          # the dispatch as it is, unpacking per tile, row kernels
         monkeypatch.setenv("SPY_HIP_EXACT_TILED", tiled)
         dd = dev_empty(T * M * 4, 0xFF)
         td = hip.tensor(dd, hip.F32, [M, T])

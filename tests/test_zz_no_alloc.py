@@ -66,10 +66,9 @@ def test_noalloc_matmul_fp16_weights_and_limit(hip, oracle):
 
 
 def test_noalloc_matmul_in_the_host_summation_order(hip, oracle):
-    """With the host backend's summation order on and 16 activation rows or more, the tiled exact MatMul runs from fp16 copies
-    of both operands placed behind the activations when the workspace has room.  Small shape: the copies fit the fixed array
-    (the packed kernel inside it); 7B-width shape: spy_hip_op_matmul_scratch_size exceeds the array while the activations
-    alone fit, and the call still succeeds (the kernel that unpacks per tile).  Both: the CPU oracle's bits."""
+    """With the host backend's summation order on, the queried size holds fp16 copies of both operands as well.  Small shape: it fits the fixed
+    array; 7B-width shape: it exceeds the array while the packed activations fit, and the call still succeeds.  Both: the CPU oracle's bits.  (The kernels that
+    run from the copies and without them: test_gpu_exact_order.py::test_tiled_matmul_bits_where_activations_are_not_packed.)"""
     from tests.gpu_util import dev, dev_empty, call
     L = hip.load()
     prev = L.spy_hip_set_exact_order(1)

@@ -507,6 +507,7 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
             for (const auto &p : prod)
                 if ((p.t == SPY_HIP_Q4_0 || p.t == SPY_HIP_Q8_0) && !spy_xgemm_ok(p.t, p.w, nullptr, p.M, p.K, T, p.M)) pack = std::max(pack, spy_exact_pack_bytes(p.M, p.K, T));
         }
+    // packed activations of either width: a width that is no multiple of 256 counts 0, and the other's may still be more than the Q8_0 blocks of both
     const size_t packed = std::max(spy_xgemm_pack_bytes(T, d), spy_xgemm_pack_bytes(T, F)), xpack = exact && T >= 2 ? packed : 0;
     // own order, Q4_0 weights: where a product is large enough for gemm.hip not to split K, it runs from packed activations instead
     // (exact_gemm.hip: same bits, tiles that fill the chip better, wq | wk | wv in one launch)

@@ -15,180 +15,149 @@
 #include "common.cuh"
 #include "exact_sum.cuh"
 
+#include <type_traits>
+
 namespace {
 
-typedef _Float16 xp_half2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ xp_half2 xp_pack(float a, float b) {
-    xp_half2 r;
-    r.x = __builtin_bit_cast(_Float16, f2h(a));
-    r.y = __builtin_bit_cast(_Float16, f2h(b));
-    return r;
+// ---------------------------------------------------------------- fma on the matrix cores
+// v_mfma_f32_16x16x1_4b_f32 is D_b[i][j] = fma(A_b[i], B_b[j], C_b[i][j]) for four blocks b of 16 x 16 outputs, one rounding, subnormals kept: the bits of
+// fmaf on 24-step chains of every kind of operand.  Where a term of the host's order is an outer product -- accumulator a of all (row, column)
+// pairs of a tile takes the product of their elements 32 c + a -- the four blocks are four of the 32 accumulators, and the chains of fmas run at twice
+// the rate of the vector units (74 against 39 Tfma/s measured).
+// Lane (g, j) = (lane / 16, lane % 16) supplies A_g[j] and B_g[j] and holds D_b[4 g + v][j] in register 4 b + v.
+typedef uint32_t xp_v4u __attribute__((ext_vector_type(4)));
+typedef float xp_v4f __attribute__((ext_vector_type(4)));
+typedef float xp_v16f __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ xp_v16f xp_mfma(float a, float b, xp_v16f c) { return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ xp_v16f xp_zero() {
+    const xp_v16f c = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    return c;
+}
+__device__ __forceinline__ void xp_widen(const uint4 w, float (&f)[8]) {
+    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        f[2 * i] = h2f((uint16_t)(u[i] & 0xFFFFu));
+        f[2 * i + 1] = h2f((uint16_t)(u[i] >> 16));
+    }
+}
+// FP16::block_reduce (vec_util.h:61-71) of accumulators 8 b + l, block b in registers 4 b .. 4 b + 3: its first two steps for one l
+__device__ __forceinline__ void xp_reduce8(const xp_v16f &s, float (&t)[4]) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) t[v] = (s[v] + s[8 + v]) + (s[4 + v] + s[12 + v]);
 }
 
 // ---------------------------------------------------------------- scores
-// One workgroup per (head, 128 query rows); a lane takes query rows t0 + lane and t0 + 64 + lane, their 2 x 128 q values
-// as packed fp16 pairs in registers.  A tile of 64 key rows is brought into LDS by the whole workgroup; every lane of a
-// wave reads the same key row -- LDS delivers that as a broadcast, but
-// at the cost of a full read, which is why a key row read serves two query rows per lane: with one, the kernel ran at the
-// LDS read rate (16 ds_read_b128 per 160 vector instructions).  A wave takes 16 of the 64 cached positions of a tile; the
-// scores go through LDS as well so that the rows of S are written in whole segments.
-#define XP_QT 128
+// One workgroup per (head, 64 query rows), a wave takes 16 of them: their q values as floats in registers, laid out as right operands.  A tile of
+// 64 key rows is brought into LDS by the whole workgroup.  Per 16 key rows and l = 0 .. 7 one chain of three matrix instructions (chunks of 32
+// elements while i + 32 < 128) gives accumulators l, 8 + l, 16 + l, 24 + l of the 16 x 16 scores; the vector units add them in the host's tree.  The
+// last 32 elements, added one by one, are a chain of 32 such instructions whose four blocks are the four groups of 16 key rows.
+// 2048 rows on 2048 positions, 32 heads: 1140 -> 597 us (the fmas on the vector units, two query rows per lane); 77 rows on 1000: 34.6 -> 20.4.  What bounds
+// it: matrix and vector instructions of this kind never run at once (counter SQ_VALU_MFMA_COEXEC_CYCLES: 0), so the 31 additions of the tree and the
+// widening of the operands (210 us) come on top of the fmas (348).
 #define XP_KSEG 512
-// fma(float(lower halves), c) and fma(float(upper halves), c) of two packed fp16 pairs, written out as instructions: left to
-// itself the compiler folds only one fp16 source into v_fma_mix_f32 and converts the loop-invariant q values to fp32 (once, which
-// doubles the registers they occupy, or inside the loop, which doubles the instructions)
-__device__ __forceinline__ float xp_fma_lo(uint32_t a, uint32_t b, float c) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,1,0]" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-__device__ __forceinline__ float xp_fma_hi(uint32_t a, uint32_t b, float c) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-
-// One key row (in LDS, 16 x 16 bytes) against the two query rows of a lane; the row is taken in its four chunks of 32 elements
-// so that only one chunk of it is in registers at a time.  A, B: the first / second query row takes part (else its score is not needed).
-template <bool A, bool B, int NB>
-__device__ __forceinline__ void xp_dot128_pair(const uint32_t (&qa)[64], const uint32_t (&qb)[NB], const uint4 *kr, float &sa, float &sb) {
-    float sum_a[32], sum_b[32];
-    // chunks of 32 elements while i + 32 < 128: accumulator l takes elements l, 32 + l, 64 + l
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        uint4 k4[4];
-#pragma unroll
-        for (int v = 0; v < 4; v++) k4[v] = kr[4 * c + v];
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const uint32_t kw[4] = {k4[v].x, k4[v].y, k4[v].z, k4[v].w};
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int l = 8 * v + 2 * i, qi = 16 * c + 4 * v + i;
-                if (A) {
-                    sum_a[l] = xp_fma_lo(kw[i], qa[qi], c == 0 ? 0.0f : sum_a[l]);
-                    sum_a[l + 1] = xp_fma_hi(kw[i], qa[qi], c == 0 ? 0.0f : sum_a[l + 1]);
-                }
-                if (B) {
-                    sum_b[l] = xp_fma_lo(kw[i], qb[qi], c == 0 ? 0.0f : sum_b[l]);
-                    sum_b[l + 1] = xp_fma_hi(kw[i], qb[qi], c == 0 ? 0.0f : sum_b[l + 1]);
-                }
-            }
-        }
-    }
-    // the last 32 elements one by one (their products are exact in fp32, so each step is one fma)
-    float tail_a = 0.0f, tail_b = 0.0f;
-    {
-        uint4 k4[4];
-#pragma unroll
-        for (int v = 0; v < 4; v++) k4[v] = kr[12 + v];
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const uint32_t kw[4] = {k4[v].x, k4[v].y, k4[v].z, k4[v].w};
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int qi = 48 + 4 * v + i;
-                if (A) { tail_a = xp_fma_lo(kw[i], qa[qi], tail_a); tail_a = xp_fma_hi(kw[i], qa[qi], tail_a); }
-                if (B) { tail_b = xp_fma_lo(kw[i], qb[qi], tail_b); tail_b = xp_fma_hi(kw[i], qb[qi], tail_b); }
-            }
-        }
-    }
-    // FP16::block_reduce (vec_util.h:61-71), then result = tail + that sum
-    auto reduce = [](float (&sum)[32]) {
-#pragma unroll
-        for (int l = 0; l < 8; l++) { sum[l] += sum[16 + l]; sum[8 + l] += sum[24 + l]; }
-#pragma unroll
-        for (int l = 0; l < 8; l++) sum[l] += sum[8 + l];
-        const float u0 = sum[0] + sum[4], u1 = sum[1] + sum[5], u2 = sum[2] + sum[6], u3 = sum[3] + sum[7];
-        return (u0 + u1) + (u2 + u3);
-    };
-    if (A) sa = tail_a + reduce(sum_a);
-    if (B) sb = tail_b + reduce(sum_b);
-}
-
-// ONE: 64 query rows per workgroup, one per lane (short passes: twice the waves per SIMD, half the granularity)
-template <bool F16Q, bool ONE>     // q: f32 [T][H * 128] as Rope leaves it, or already rounded to fp16 and laid out [H][T][128]
-__global__ __launch_bounds__(256, 2) void xp_scores_kernel(const void *__restrict__ q, const uint16_t *__restrict__ kc, float *__restrict__ S,
+template <bool F16Q>       // q: f32 [T][H * 128] as Rope leaves it, or already rounded to fp16 and laid out [H][T][128]
+__global__ __launch_bounds__(256, 3) void xp_scores_kernel(const void *__restrict__ q, const uint16_t *__restrict__ kc, float *__restrict__ S,
                                                            int T, int H, int P, int64_t s_row, int kseg) {
-    constexpr int QT = ONE ? 64 : XP_QT;
-    __shared__ float s_tile[QT][65];
-    __shared__ __align__(16) uint4 s_k[64][16];                  // 64 key rows of 256 bytes
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int QT = 64;
+    __shared__ __align__(16) uint4 s_k[2][64][17];               // 64 key rows of 256 bytes, 16 bytes apart
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, j = lane & 15;
     // The head is the fastest-running index of the grid: consecutive workgroups go to the eight XCDs in turn, and with the query tile
     // there an XCD would get tiles k and k + 8 of 16 only -- under the causal mask 24 to 10 units of work (68 % of the compute units
     // busy over the launch).  With the head there every XCD gets the same mix of tiles, and the key rows of its heads stay in its L2.
     const int t0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * QT, h = blockIdx.x;      // the longest rows first
     const int64_t d = (int64_t)H * 128;
     // the cached positions are dealt out in segments of kseg (a multiple of 64) over blockIdx.z, so that the workgroups are of similar length
-    // (one workgroup per 128 query rows would make the longest rows the critical path of the launch)
+    // (one workgroup per query tile would make the longest rows the critical path of the launch)
     const int kv_end = min(P + min(t0 + QT - 1, T - 1) + 1, ((int)blockIdx.z + 1) * kseg);       // cached positions that some row of the tile may see, within this segment
     if ((int)blockIdx.z * kseg >= kv_end) return;
-    uint32_t qa[64], qb[ONE ? 1 : 64];
+    const int tw = t0 + wave * 16, wave_end = tw < T ? P + min(tw + 15, T - 1) + 1 : 0;      // the wave's query rows, and the positions that some of them may see
+    float qm[3][8];                                              // elements 32 c + 8 g + l of query row j
+    uint4 qt[4];                                                 // elements 96 + 8 c + l, as fp16: widened for each tile, which costs less than the registers
+    const int t = min(tw + j, T - 1);
     if constexpr (F16Q) {
-        const uint4 *qp = (const uint4 *)((const uint16_t *)q + ((int64_t)h * T + min(t0 + lane, T - 1)) * 128), *qp2 = (const uint4 *)((const uint16_t *)q + ((int64_t)h * T + min(t0 + 64 + lane, T - 1)) * 128);
+        const uint4 *qp = (const uint4 *)((const uint16_t *)q + ((int64_t)h * T + t) * 128);
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const uint4 f = qp[i], f2 = qp2[i];
-            qa[4 * i] = f.x; qa[4 * i + 1] = f.y; qa[4 * i + 2] = f.z; qa[4 * i + 3] = f.w;
-            if constexpr (!ONE) { qb[4 * i] = f2.x; qb[4 * i + 1] = f2.y; qb[4 * i + 2] = f2.z; qb[4 * i + 3] = f2.w; }
-        }
+        for (int c = 0; c < 3; c++) xp_widen(qp[4 * c + g], qm[c]);
+#pragma unroll
+        for (int c = 0; c < 4; c++) qt[c] = qp[12 + c];
     } else {
-        const float4 *qp = (const float4 *)((const float *)q + (int64_t)min(t0 + lane, T - 1) * d + (int64_t)h * 128);
-        const float4 *qp2 = (const float4 *)((const float *)q + (int64_t)min(t0 + 64 + lane, T - 1) * d + (int64_t)h * 128);
+        const float *qp = (const float *)q + (int64_t)t * d + (int64_t)h * 128;
+        auto halves = [&](int at) -> uint4 {
+            const float4 x = *(const float4 *)(qp + at), y = *(const float4 *)(qp + at + 4);
+            auto pair = [](float a, float b) -> uint32_t { return (uint32_t)f2h(a) | ((uint32_t)f2h(b) << 16); };
+            return make_uint4(pair(x.x, x.y), pair(x.z, x.w), pair(y.x, y.y), pair(y.z, y.w));
+        };
 #pragma unroll
-        for (int i = 0; i < 32; i++) {
-            const float4 f = qp[i], f2 = qp2[i];
-            qa[2 * i] = __builtin_bit_cast(uint32_t, xp_pack(f.x, f.y));
-            qa[2 * i + 1] = __builtin_bit_cast(uint32_t, xp_pack(f.z, f.w));
-            if constexpr (!ONE) {
-                qb[2 * i] = __builtin_bit_cast(uint32_t, xp_pack(f2.x, f2.y));
-                qb[2 * i + 1] = __builtin_bit_cast(uint32_t, xp_pack(f2.z, f2.w));
-            }
-        }
+        for (int c = 0; c < 3; c++) xp_widen(halves(32 * c + 8 * g), qm[c]);
+#pragma unroll
+        for (int c = 0; c < 4; c++) qt[c] = halves(96 + 8 * c);
     }
-    const int kv_end_a = P + min(t0 + 63, T - 1) + 1;            // cached positions that some row of the tile's first half may see
     // staging: thread -> key row tid / 4 of the tile, 64 of its 256 bytes
     const int st_row = threadIdx.x >> 2, st_q = (threadIdx.x & 3) * 4;
-    uint4 kst0, kst1, kst2, kst3;
-#define XP_FETCH_K(kv_first) do { \
-        const uint4 *src_ = (const uint4 *)(kc + (int64_t)min((kv_first) + st_row, kv_end - 1) * d + (int64_t)h * 128) + st_q; \
-        kst0 = src_[0]; kst1 = src_[1]; kst2 = src_[2]; kst3 = src_[3]; } while (0)
-    for (int kv0 = (int)blockIdx.z * kseg; kv0 < kv_end; kv0 += 64) {
-        // (no key tile travelling in registers during the dots: with 2 x 64 registers of q values and 2 x 32 accumulators there is
-        // no room for it; the second workgroup of the compute unit covers the wait)
-        XP_FETCH_K(kv0);
-        s_k[st_row][st_q] = kst0; s_k[st_row][st_q + 1] = kst1; s_k[st_row][st_q + 2] = kst2; s_k[st_row][st_q + 3] = kst3;
-        __syncthreads();
-        const bool first_half = kv0 < kv_end_a;                   // else the whole key tile lies behind the mask of query rows t0 .. t0 + 63
-#pragma unroll 1
-        for (int j = 0; j < 16; j++) {
-            const int kvl = wave * 16 + j;
-            float sa = 0.0f, sb = 0.0f;
-            if (kv0 + kvl < kv_end) {
-                if constexpr (ONE) xp_dot128_pair<true, false, 64>(qa, qa, s_k[kvl], sa, sb);
-                else if (first_half) xp_dot128_pair<true, true, 64>(qa, qb, s_k[kvl], sa, sb);
-                else xp_dot128_pair<false, true, 64>(qa, qb, s_k[kvl], sa, sb);
-            }
-            s_tile[lane][kvl] = sa;
-            if constexpr (!ONE) s_tile[64 + lane][kvl] = sb;
-        }
-        __syncthreads();
-        {
-            constexpr int W = ONE ? 16 : 32;                      // scores per thread
-            const int row = threadIdx.x / (64 / W), seg = threadIdx.x % (64 / W);
-            if (t0 + row < T && (row >= 64 || first_half)) {
-                float4 *out = (float4 *)(S + ((int64_t)h * T + t0 + row) * s_row + kv0 + seg * W);
+    xp_v4u kst[4];
+    auto fetch = [&](int kv_first) {
+        const xp_v4u *src = (const xp_v4u *)(kc + (int64_t)min(kv_first + st_row, kv_end - 1) * d + (int64_t)h * 128) + st_q;
 #pragma unroll
-                for (int i = 0; i < W / 4; i++)
-                    out[i] = make_float4(s_tile[row][seg * W + 4 * i], s_tile[row][seg * W + 4 * i + 1], s_tile[row][seg * W + 4 * i + 2],
-                                         s_tile[row][seg * W + 4 * i + 3]);
-            }
+        for (int i = 0; i < 4; i++) kst[i] = src[i];
+    };
+    fetch((int)blockIdx.z * kseg);
+    int buf = 0;
+    for (int kv0 = (int)blockIdx.z * kseg; kv0 < kv_end; kv0 += 64, buf ^= 1) {
+        // (two buffers: a wave that writes this one is past the barrier of the tile before, which every wave reaches after its reads of this one)
+#pragma unroll
+        for (int i = 0; i < 4; i++) *(xp_v4u *)&s_k[buf][st_row][st_q + i] = kst[i];
+        __syncthreads();
+        if (kv0 + 64 < kv_end) fetch(kv0 + 64);
+        if (kv0 >= wave_end) continue;                            // the tile lies behind the mask of the wave's query rows
+        xp_v16f tail = xp_zero();
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            float a[8], b[8];
+            xp_widen(s_k[buf][lane][12 + c], a);
+            asm("" : "+v"(qt[c].x), "+v"(qt[c].y), "+v"(qt[c].z), "+v"(qt[c].w));      // (or the compiler widens them before the loop and keeps the floats)
+            xp_widen(qt[c], b);
+#pragma unroll
+            for (int l = 0; l < 8; l++) tail = xp_mfma(a[l], b[l], tail);
         }
-        // the next tile's key rows go into s_k at the top of the loop: every wave is past its reads of s_k once it has passed the
-        // barrier above, and the barrier after the writes orders them against the next reads
+        auto keys16 = [&](auto kt_c) {
+            constexpr int kt = decltype(kt_c)::value;
+            if (kv0 + 16 * kt >= wave_end) return;
+            float a[3][8];
+#pragma unroll
+            for (int c = 0; c < 3; c++) xp_widen(s_k[buf][16 * kt + j][4 * c + g], a[c]);
+            auto part = [&](int l, float (&r)[4]) {
+                xp_v16f s = xp_mfma(a[0][l], qm[0][l], xp_zero());
+                s = xp_mfma(a[1][l], qm[1][l], s);
+                s = xp_mfma(a[2][l], qm[2][l], s);
+                xp_reduce8(s, r);
+            };
+            float u[4][4], o[4];
+#pragma unroll
+            for (int l = 0; l < 4; l++) {
+                float x[4], y[4];
+                part(l, x);
+                __builtin_amdgcn_sched_barrier(0);
+                part(l + 4, y);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {                    // added here and now: eight chains waiting for their tree are 210 registers, this is 130
+                    u[l][v] = x[v] + y[v];
+                    asm volatile("" : "+v"(u[l][v]));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const float x = u[0][v] + u[1][v], y = u[2][v] + u[3][v];
+                o[v] = tail[4 * kt + v] + (x + y);
+            }
+            if (tw + j < T) *(float4 *)(S + ((int64_t)h * T + t) * s_row + kv0 + 16 * kt + 4 * g) = make_float4(o[0], o[1], o[2], o[3]);
+        };
+        keys16(std::integral_constant<int, 0>{});
+        keys16(std::integral_constant<int, 1>{});
+        keys16(std::integral_constant<int, 2>{});
+        keys16(std::integral_constant<int, 3>{});
     }
-#undef XP_FETCH_K
 }
 
 // ---------------------------------------------------------------- softmax
@@ -285,147 +254,107 @@ int xp_softmax_launch(hipStream_t st, const float *S, uint16_t *P16, const float
 }
 
 // ---------------------------------------------------------------- product with V^T
-// One workgroup per (head, 32 query rows, 32 of the 128 output elements); eight groups of 32 lanes, a group takes four
-// output elements.  Lane l of a group keeps accumulator l (cached positions 32c + l) of its 4 x 32 outputs, so a V value is
-// loaded once for 32 query rows; the probabilities of a chunk come through LDS, transposed to [position][row].
-// After the chunks the 32 accumulators of every output are added in the tree of FP16::block_reduce, spread over the lanes so
-// that lane l ends with the outputs of query row l, and the scalar tail of the host loop follows.
-#define XP_PT 32
-#define XP_SC 4            // chunks of 32 positions per stage
-__global__ __launch_bounds__(256, 2) void xp_pv_kernel(const uint16_t *__restrict__ P16, const uint16_t *__restrict__ vt, float *__restrict__ out,
+// One workgroup per (head, 32 query rows, 32 of the 128 output elements), a wave per 16 x 16 outputs: eight matrix instructions per chunk of 32 cached
+// positions, instruction l for accumulators l, 8 + l, 16 + l, 24 + l, so that lane (g, j) supplies positions 8 g .. 8 g + 7 of V^T row j and of the
+// probabilities of query row j: 16 bytes each, and every lane ends with all 32 accumulators of its four outputs.  Stages of two chunks go through LDS
+// (rows of 128 bytes, their 16-byte pieces exchanged by the row so that reads and writes meet no bank twice), requested one stage ahead.
+// 2048 rows on 2048 positions, 32 heads: 947 -> 557 us (the fmas on the vector units, a lane per accumulator); 77 rows on 1000: 26.5 -> 15.7.
+// What bounds it: 348 us of matrix instructions and, beside none of them, the two conversions each needs (about 90).  Straight from memory without LDS:
+// 705 us (the L2); two waves per SIMD instead of three: 609.
+typedef uint32_t xp_u4 __attribute__((ext_vector_type(4), aligned(2)));          // V^T rows of a caller's cache: no more alignment than an element's
+__global__ __launch_bounds__(256, 3) void xp_pv_kernel(const uint16_t *__restrict__ P16, const uint16_t *__restrict__ vt, float *__restrict__ out,
                                                        int T, int H, int P, int64_t p_row, int64_t C, int n_total) {
-    __shared__ __align__(16) uint16_t s_p[2][32 * XP_SC][40];  // [buffer][position in the stage][query row], rows of 80 bytes
-    const int g = threadIdx.x >> 5, l = threadIdx.x & 31;
-    const int t0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * XP_PT, h = blockIdx.x;      // head fastest: see xp_scores_kernel
-    const int dd0 = blockIdx.y * 32 + g * 4;
-    const int Lmax = P + min(t0 + XP_PT - 1, T - 1) + 1;
+    __shared__ __align__(16) xp_v4u s_v[2][32][8], s_p[2][32][8];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, j = lane & 15;
+    const int h = blockIdx.x, tb = ((int)gridDim.z - 1 - (int)blockIdx.z) * 32;      // head fastest: see xp_scores_kernel
+    const int t0 = tb + (wave >> 1) * 16, dd0 = (int)blockIdx.y * 32 + (wave & 1) * 16;
+    const int Lmax = P + min(tb + 31, T - 1) + 1;
     const int tail_start = (n_total - 1) / 32 * 32;
-    const int nchunk = min(tail_start, (Lmax + 31) & ~31) / 32;
-    const int nstage = (nchunk + XP_SC - 1) / XP_SC;
-    const uint16_t *vrow[4];
+    // whole chunks, and the one whose elements the host adds one by one (tail_start on, where a row of the tile reaches it)
+    const int nchunk = min(tail_start, (Lmax + 31) & ~31) / 32, nall = nchunk + (Lmax > tail_start ? 1 : 0);
+    // staging: thread -> row tid / 8 of either tile, 16 of the 128 bytes
+    const int st_row = threadIdx.x >> 3, st_i = threadIdx.x & 7, st_slot = st_i ^ ((st_row >> 1) & 7), st_pos = 8 * st_i;
+    const uint16_t *vsrc = vt + ((int64_t)h * 128 + blockIdx.y * 32 + st_row) * C, *psrc = P16 + ((int64_t)h * T + min(tb + st_row, T - 1)) * p_row;
+    xp_v16f acc[8];
 #pragma unroll
-    for (int j = 0; j < 4; j++) vrow[j] = vt + ((int64_t)h * 128 + dd0 + j) * C + l;
-    // staging of the probabilities: thread -> query row tid % 32, sixteen positions; neighbouring lanes write neighbouring
-    // query rows of one position, i.e. neighbouring LDS words (the other way round, 64 lanes would meet in four banks)
-    const int st_t = threadIdx.x & 31, st_k = (threadIdx.x >> 5) * 16;
-    const uint16_t *prow = P16 + ((int64_t)h * T + min(t0 + st_t, T - 1)) * p_row + st_k;
-    float acc[4][32];
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int i = 0; i < 32; i++) acc[j][i] = 0.0f;
-    uint4 pst[2];
-    uint16_t vn[XP_SC][4];
-    auto fetch = [&](int s) {
-        pst[0] = *(const uint4 *)(prow + 32 * XP_SC * s);
-        pst[1] = *(const uint4 *)(prow + 32 * XP_SC * s + 8);
-#pragma unroll
-        for (int c = 0; c < XP_SC; c++) {
-            const int pos = 32 * (XP_SC * s + c);
-#pragma unroll
-            for (int j = 0; j < 4; j++) vn[c][j] = pos + l < Lmax ? vrow[j][pos] : (uint16_t)0;      // past Lmax every probability is 0; the cache may hold anything there
-        }
+    for (int l = 0; l < 8; l++) acc[l] = xp_zero();
+    vsrc += st_pos;
+    psrc += st_pos;
+    xp_v4u vn, pn;
+    auto fetch = [&](int s) {                                       // the next stage, s; a second chunk that does not exist is the first one again
+        if (2 * s >= nall) return;
+        const int back = 2 * s + 2 > nall && st_pos >= 32 ? 32 : 0;
+        vn = *(const xp_u4 *)(vsrc - back);
+        pn = *(const xp_v4u *)(psrc - back);
+        vsrc += 64;
+        psrc += 64;
+        __builtin_amdgcn_sched_barrier(0);                          // (or the loads sink to where their data go into LDS)
     };
-    auto put = [&](int buf) {
-#pragma unroll
-        for (int v = 0; v < 2; v++) {
-            const uint32_t w[4] = {pst[v].x, pst[v].y, pst[v].z, pst[v].w};
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                s_p[buf][st_k + 8 * v + 2 * i][st_t] = (uint16_t)(w[i] & 0xFFFFu);
-                s_p[buf][st_k + 8 * v + 2 * i + 1][st_t] = (uint16_t)(w[i] >> 16);
-            }
-        }
-    };
-    if (nstage > 0) {
-        fetch(0);
-        put(0);
-    }
-    __syncthreads();
-    for (int s = 0; s < nstage; s++) {
-        const int buf = s & 1;
-        _Float16 vc[XP_SC][4];
-#pragma unroll
-        for (int c = 0; c < XP_SC; c++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) vc[c][j] = __builtin_bit_cast(_Float16, vn[c][j]);
-        if (s + 1 < nstage) fetch(s + 1);
-#pragma unroll
-        for (int c = 0; c < XP_SC; c++) {
-            if (XP_SC * s + c < nchunk) {
-                const uint4 *pp = (const uint4 *)&s_p[buf][32 * c + l][0];
-#pragma unroll
-                for (int qd = 0; qd < 4; qd++) {
-                    const uint4 w4 = pp[qd];
-                    const uint32_t w[4] = {w4.x, w4.y, w4.z, w4.w};
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const xp_half2 p2 = __builtin_bit_cast(xp_half2, w[i]);
-#pragma unroll
-                        for (int j = 0; j < 4; j++) {
-                            acc[j][8 * qd + 2 * i] = fmaf((float)vc[c][j], (float)p2.x, acc[j][8 * qd + 2 * i]);
-                            acc[j][8 * qd + 2 * i + 1] = fmaf((float)vc[c][j], (float)p2.y, acc[j][8 * qd + 2 * i + 1]);
-                        }
-                    }
-                }
-            }
-        }
-        if (s + 1 < nstage) put(buf ^ 1);
+    const int rd_v = (wave & 1) * 16 + j, rd_p = (wave >> 1) * 16 + j, sw = (j >> 1) & 7;
+    // a stage in buffer b (a wave that writes it is past the barrier of the stage before, which every wave reaches after its reads of it)
+    auto put = [&](int b) {
+        s_v[b][st_row][st_slot] = vn;
+        s_p[b][st_row][st_slot] = pn;
         __syncthreads();
-    }
-    // The tree: sum[l] += sum[l + 16], sum[l] += sum[l + 8], t_l = sum[l] + sum[l + 4], (t0 + t1) + (t2 + t3), where l is the lane.
-    // At each step a lane keeps the half of its query rows that matches its own lane bit and hands the other half to its
-    // partner, so 16 + 8 + 4 + 2 + 1 exchanges per output element leave lane l with the sum of query row l.
-    float res[4];
+    };
+    auto chunk = [&](int b, int c) {
+        const xp_v4u v = s_v[b][rd_v][(4 * c + g) ^ sw], p = s_p[b][rd_p][(4 * c + g) ^ sw];
+        float x[8], y[8];
+        xp_widen(make_uint4(v.x, v.y, v.z, v.w), x);
+        xp_widen(make_uint4(p.x, p.y, p.z, p.w), y);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        float a16[16], a8[8], a4[4], a2[2];
-        const bool b4 = l & 16, b3 = l & 8, b2 = l & 4, b0 = l & 1, b1 = l & 2;
+        for (int l = 0; l < 8; l++) acc[l] = xp_mfma(x[l], y[l], acc[l]);
+    };
+    xp_v4f tail = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto tail_chunk = [&](int b, int c) {                           // v_mfma_f32_16x16x4_f32: the fmas of its four elements one after the other, bit for bit
 #pragma unroll
-        for (int k = 0; k < 16; k++) {
-            const float keep = b4 ? acc[j][k + 16] : acc[j][k], send = b4 ? acc[j][k] : acc[j][k + 16];
-            a16[k] = keep + __shfl_xor(send, 16, SPY_WAVE);
+        for (int i = 0; i < 8; i++) {
+            const int slot = (4 * c + (i >> 1)) ^ sw, e = 4 * (i & 1) + g;          // lane (g, j): element 4 i + g of the chunk
+            tail = __builtin_amdgcn_mfma_f32_16x16x4f32(h2f(((const uint16_t *)&s_v[b][rd_v][slot])[e]), h2f(((const uint16_t *)&s_p[b][rd_p][slot])[e]), tail, 0, 0, 0);
         }
+    };
+    fetch(0);
+    const int nwhole = min(Lmax / 64, nchunk / 2);                  // stages of two chunks without a position past Lmax
+    int s = 0;
+    for (; s + 2 <= nwhole; s += 2) {
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const float keep = b3 ? a16[k + 8] : a16[k], send = b3 ? a16[k] : a16[k + 8];
-            a8[k] = keep + __shfl_xor(send, 8, SPY_WAVE);
-        }
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const float keep = b2 ? a8[k + 4] : a8[k], send = b2 ? a8[k] : a8[k + 4];
-            a4[k] = keep + __shfl_xor(send, 4, SPY_WAVE);
-        }
-        // query rows left: 4 per lane, their index = (l & 28) + k; the tree goes on with lane bit 0, then bit 1
-#pragma unroll
-        for (int k = 0; k < 2; k++) {
-            const float keep = b0 ? a4[2 * k + 1] : a4[2 * k], send = b0 ? a4[2 * k] : a4[2 * k + 1];
-            a2[k] = keep + __shfl_xor(send, 1, SPY_WAVE);
-        }
-        {
-            const float keep = b1 ? a2[1] : a2[0], send = b1 ? a2[0] : a2[1];
-            res[j] = keep + __shfl_xor(send, 2, SPY_WAVE);
+        for (int b = 0; b < 2; b++) {
+            put(b);
+            fetch(s + b + 1);
+            chunk(b, 0);
+            chunk(b, 1);
         }
     }
-    // lane l now holds query row t0 + l: rows were halved by lane bits 4, 3, 2 (index bits 4, 3, 2), then bit 0 chose index bit 0 and
-    // bit 1 index bit 1
-    const int t = t0 + l;
+    for (; 2 * s < nall; s++) {
+        const int left = Lmax - (64 * s + st_pos), b = s & 1;       // past Lmax every probability is 0, but the cache may hold anything
+#pragma unroll
+        for (int i = 0; i < 4; i++) vn[i] = left >= 2 * i + 2 ? vn[i] : left == 2 * i + 1 ? vn[i] & 0xFFFFu : 0u;
+        put(b);
+        fetch(s + 1);
+#pragma unroll 1
+        for (int c = 0; c < 2; c++)
+            if (2 * s + c < nchunk) chunk(b, c);
+            else if (2 * s + c < nall) tail_chunk(b, c);
+    }
+    // FP16::block_reduce: t_l from the four accumulators of instruction l, t_l + t_(l + 4), (u0 + u1) + (u2 + u3)
+    float u[4][4];
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+        float x[4], y[4];
+        xp_reduce8(acc[l], x);
+        xp_reduce8(acc[l + 4], y);
+#pragma unroll
+        for (int v = 0; v < 4; v++) u[l][v] = x[v] + y[v];
+    }
+    const int t = t0 + j;
     if (t >= T) return;
-    const int Lt = P + t + 1;                                      // positions row t sees
-    const int tail_end = min(n_total, Lt);
-    const uint16_t *pr = P16 + ((int64_t)h * T + t) * p_row;
-    float o4[4];
+    float o[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        float tail = 0.0f;
-        const uint16_t *vr = vt + ((int64_t)h * 128 + dd0 + j) * C;
-        for (int i = tail_start; i < tail_end; i++) {
-            const float pr_ = h2f(vr[i]) * h2f(pr[i]);
-            tail += pr_;
-        }
-        o4[j] = tail + res[j];
+    for (int v = 0; v < 4; v++) {
+        const float x = u[0][v] + u[1][v], y = u[2][v] + u[3][v];
+        o[v] = tail[v] + (x + y);
     }
-    *(float4 *)(out + (int64_t)t * H * 128 + (int64_t)h * 128 + dd0) = make_float4(o4[0], o4[1], o4[2], o4[3]);
+    *(float4 *)(out + (int64_t)t * H * 128 + (int64_t)h * 128 + dd0 + 4 * g) = make_float4(o[0], o[1], o[2], o[3]);
 }
 
 }   // namespace
@@ -442,21 +371,18 @@ int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint1
     const int64_t s_row = spy_exact_prompt_attn_row((int64_t)P + T);
     // segments of the cached positions: 512 long where that fills the chip, down to one key tile for short passes (77 tokens on 1000 cached ones
     // gave 96 workgroups: 114 us; one per 64 positions and 64 query rows 29)
-    const bool one = T <= 256;
-    const int tiles = (T + (one ? 64 : XP_QT) - 1) / (one ? 64 : XP_QT);
+    const int tiles = (T + 63) / 64;
     int kseg = XP_KSEG;
     while (kseg > 64 && (int64_t)H * tiles * ((P + T + kseg - 1) / kseg) < 1024) kseg >>= 1;
     const dim3 sgrid((unsigned)H, (unsigned)tiles, (unsigned)((P + T + kseg - 1) / kseg));
-    if (q_f16 && one) xp_scores_kernel<true, true><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
-    else if (q_f16) xp_scores_kernel<true, false><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
-    else if (one) xp_scores_kernel<false, true><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
-    else xp_scores_kernel<false, false><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
+    if (q_f16) xp_scores_kernel<true><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
+    else xp_scores_kernel<false><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
     if (hipGetLastError() != hipSuccess) return SPY_HIP_EINVAL;
     const int ncu = spy_num_cu(), rc = (int64_t)P + T <= 4096 ? xp_softmax_launch<16, 12>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
                                          : (int64_t)P + T <= 6144 ? xp_softmax_launch<24, 8>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
                                                                   : xp_softmax_launch<32, 4>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu);
     if (rc) return rc;
-    xp_pv_kernel<<<dim3((unsigned)H, 4, (unsigned)((T + XP_PT - 1) / XP_PT)), dim3(256), 0, st>>>(P16, vt, out, T, H, P, s_row, C, n_total);
+    xp_pv_kernel<<<dim3((unsigned)H, 4, (unsigned)((T + 31) / 32)), dim3(256), 0, st>>>(P16, vt, out, T, H, P, s_row, C, n_total);
     return SPY_LAUNCH_RC();
 }
 

@@ -287,6 +287,34 @@ def test_exact_prompt_attention_bits(hip, oracle, H_, past, T, n_ctx, cuts):
     assert L.spy_hip_prompt_attention_exact(None, dq.ptr, dk.ptr, dv.ptr, out.ptr, T, H_, hd, past, n_ctx, n_kv, scale, sc.ptr, 1024) == hip.ENOSPACE
 
 
+@pytest.mark.parametrize("H_,past,T,n_ctx,cuts", [
+    (2, 0, 16, 32, (0, 16)), (2, 0, 17, 32, (0, 17)), (1, 0, 32, 32, (0, 32)), (1, 0, 33, 64, (0, 33)),      # tiles of 16 and 32 query rows; all of the pass in the one-by-one tail
+    (1, 63, 65, 128, (0, 65)), (1, 64, 64, 128, (0, 64)), (1, 65, 64, 160, (0, 64)),       # key tiles of 64, stages of two chunks: an odd and an even number of whole ones
+    (2, 31, 34, 96, (0, 1, 34)), (1, 95, 2, 128, (0, 1, 2)), (1, 127, 130, 288, (0, 129, 130)),      # the tail as first and as second chunk of a stage; a piece that does not reach it
+])
+def test_exact_prompt_attention_tile_edges(hip, oracle, H_, past, T, n_ctx, cuts):
+    """The causal attention kernels at the edges of their tiles, bits as in test_exact_prompt_attention_bits."""
+    test_exact_prompt_attention_bits(hip, oracle, H_, past, T, n_ctx, cuts)
+
+
+def test_exact_prompt_attention_unaligned_v(hip):
+    """A V^T cache two bytes off the 16-byte grid gives the bits of an aligned one."""
+    from tests.gpu_util import dev, dev_empty, call
+    H_, T, past, n_ctx, hd = 2, 70, 90, 192, 128
+    rng = np.random.default_rng(5)
+    q, kc = rng.standard_normal((T, H_ * hd)).astype(np.float32), rng.standard_normal((n_ctx, H_ * hd)).astype(np.float16)
+    vc = rng.standard_normal(H_ * hd * n_ctx).astype(np.float16)
+    L = hip.load()
+    need = L.spy_hip_prompt_attention_exact_scratch_size(T, H_, past)
+    dq, dk, sc, outs = dev(q), dev(kc.view(np.uint16)), dev_empty(need, 0xFF), []
+    for off in (0, 1):
+        dv = dev(np.concatenate([np.zeros(off, np.float16), vc, np.zeros(8, np.float16)]).view(np.uint16))
+        out = dev_empty(T * H_ * hd * 4, 0xFF)
+        call(L.spy_hip_prompt_attention_exact, None, dq.ptr, dk.ptr, dv.ptr + 2 * off, out.ptr, T, H_, hd, past, n_ctx, past + T, 0.125, sc.ptr, need)
+        outs.append(out.download(np.float32))
+    _same_bits(outs[1], outs[0], "V^T cache at an odd element")
+
+
 @pytest.mark.parametrize("H_,past,T,n_ctx,spread", [
     (2, 4032, 64, 4096, 1.0),                 # the longest row of sixteen groups per lane, 1024 group sums
     (1, 5000, 40, 5056, 1.0), (1, 6130, 30, 6176, 1.0), (1, 8170, 22, 8192, 1.0),      # the wider forms and their edges (6144, 8192)

@@ -813,10 +813,12 @@ __global__ __launch_bounds__(256, 3) void xks_kernel(xt_args a) {
 // Matrix and vector cycles of these instructions add up here (counters at 1000 rows: vector 36 %, matrix 38 %, at once 13 % of the time), which is
 // why the cycles above are what counts; and the tiles fill the chip better than 128 x 128 ones.  Packing included, Q4_0, 4096 x 4096: 385 rows 66 -> 46 us,
 // 512 rows 68 -> 48, 600 rows 96 -> 64, 1000 rows 94 -> 75, 2048 rows 118 -> 117; 4096 x 11008: 512 rows 164 -> 112, 1000 rows 228 -> 184;
-// 22016 x 4096: 77 rows 85 -> 62, 320 rows 152 -> 131, 1000 rows 314 -> 302.
+// 22016 x 4096: 77 rows 85 -> 62, 320 rows 152 -> 131, 1000 rows 314 -> 297.
 // A wave takes RW groups of 16 weight rows and C groups of activation rows, so that an activation operand read from LDS serves RW instructions.
-// Weights: lane (q, r) reads blocks 2q and 2q + 1 of row r and chunk (contiguous over the four lanes of a row), and 4 x 4 exchanges between the
-// lane blocks (v_permlane16_swap, v_permlane32_swap) leave words q and 4 + q of every block in lane block q.
+// Weights: lane (q, r) reads blocks 2q and 2q + 1 of row r and chunk (contiguous over the four lanes of a row), brings words 2i and 2i + 1 of a block
+// into one dword, and 4 x 4 exchanges between the lane blocks (v_permlane16_swap, v_permlane32_swap) leave words 2q and 2q + 1 of every block in lane block q:
+// the sixteen neighbouring bytes that a lane's activation operand is in LDS.  (With words q and 4 + q, two 8-byte reads 16 bytes apart met in the same banks,
+// half of the LDS cycles: 4096 x 11008 x 1000 182 -> 166 us, 22016 x 4096 x 1000 307 -> 297, 4096 x 4096 x 1000 74 -> 71.)
 struct xo_raw { uint32_t w[9]; };
 __device__ __forceinline__ void xo_transpose(uint32_t (&r)[4]) {
     auto s16 = [](uint32_t &a, uint32_t &b) { auto v = __builtin_amdgcn_permlane16_swap(a, b, false, false); a = v[0]; b = v[1]; };
@@ -873,11 +875,14 @@ __global__ __launch_bounds__(64 * WV, OCC) void xo_kernel(xt_args a) {
         for (int w = 0; w < RW; w++) {
             const uint32_t *v = cur[w].w;
             dd[w] = (v[0] & 0xFFFFu) | (v[4] & 0xFFFF0000u);
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                wd[w][0][k] = __builtin_amdgcn_alignbit(v[k + 1], v[k], 16);
-                wd[w][1][k] = v[5 + k];
-            }
+            // dword i of a block: word 2i in the low nibbles, word 2i + 1 in the high ones (words 0..3 are the low nibbles of the block's four dwords, words 4..7 the high ones)
+            auto pair = [](uint32_t (&o)[4], uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+                constexpr uint32_t lo = 0x0F0F0F0Fu;
+                o[0] = (a & lo) | ((b << 4) & ~lo); o[1] = (c & lo) | ((d << 4) & ~lo);
+                o[2] = ((a >> 4) & lo) | (b & ~lo); o[3] = ((c >> 4) & lo) | (d & ~lo);
+            };
+            pair(wd[w][0], __builtin_amdgcn_alignbit(v[1], v[0], 16), __builtin_amdgcn_alignbit(v[2], v[1], 16), __builtin_amdgcn_alignbit(v[3], v[2], 16), __builtin_amdgcn_alignbit(v[4], v[3], 16));
+            pair(wd[w][1], v[5], v[6], v[7], v[8]);
             xo_transpose(wd[w][0]);
             xo_transpose(wd[w][1]);
         }
@@ -886,8 +891,8 @@ __global__ __launch_bounds__(64 * WV, OCC) void xo_kernel(xt_args a) {
     const xk_v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
     auto compute = [&](int s, auto par_c) {
         constexpr int par = decltype(par_c)::value;
-        const uint8_t *sx = smem + (s & 1) * XB + (q >> 1) * 256 + r * 16 + (q & 1) * 8, *sd = smem + (s & 1) * XB + C * XT_XB + lane * 4;
-        uint4 w[RW][4];                            // operands of the stage's four blocks: words q and 4 + q, elements 0, 2, 1, 3 each
+        const uint8_t *sx = smem + (s & 1) * XB + q * 256 + r * 16, *sd = smem + (s & 1) * XB + C * XT_XB + lane * 4;
+        uint4 w[RW][4];                            // operands of the stage's four blocks: words 2q and 2q + 1, elements 0, 2, 1, 3 each
         uint32_t dw[RW];
 #pragma unroll
         for (int g = 0; g < RW; g++) {
@@ -907,9 +912,7 @@ __global__ __launch_bounds__(64 * WV, OCC) void xo_kernel(xt_args a) {
         xk_v4f p[2][RW];
         xt_v16f D[RW];
         auto rd = [&](int j) {
-            const uint8_t *o = sx + (j >> 2) * XT_XB + (j & 3) * 1024;
-            const uint2 l = *(const uint2 *)o, h = *(const uint2 *)(o + 512);
-            xv[j % 3] = make_uint4(l.x, l.y, h.x, h.y);
+            xv[j % 3] = *(const uint4 *)(sx + (j >> 2) * XT_XB + (j & 3) * 1024);
         };
         dx[0] = *(const uint32_t *)sd;
         rd(0);

@@ -1,0 +1,157 @@
+// Attention of one token in the host backend's summation order where the cache is short: scores, softmax and P.V^T in one launch.
+// (In a source of its own: the kernels of a layer of the single-token pass about fill the instruction cache, and where they lie in it counts.)
+#include "exact_decode.cuh"
+#include "engine_types.cuh"
+
+// ---- scores, softmax and P.V^T of a short cache in one launch ------------------------------------------------------------
+// Up to XF_MAX cached tokens: the same 256 workgroups (head, 16 rows of V^T), each with all the scores of its head.  The eight
+// workgroups of a head read its keys eight times over, from the L2 of the one XCD that they share (head = workgroup index modulo n_head, n_head a
+// multiple of 8 in the models there are), and what that costs is less than the launch and the scores' way through memory that it saves:
+// the two launches 8.5 -> 4.3 us with 40 tokens, 10.1 -> 7.9 with 512.  Up to XF_MAX tokens the keys of a head fit LDS.
+// What bounds it: the chain launch, keys and V^T rows (one wait for both), dots, exponentials (a gather), running sum, walk.
+#define XF_NP (XF_MAX * 16 / XP_THREADS)   // 16-byte pieces of keys per thread
+static size_t xattn_short_lds(int n_ctx) { return (size_t)(n_ctx < XF_MAX ? n_ctx : XF_MAX) * 256 + 16 * 96 * 2; }      // the keys; later the rows of V^T (16 rows of cap + 32 .. 96 halfs)
+static __global__ __launch_bounds__(XP_THREADS) void xattn_short_kernel(const dev_state *st, int pos_imm, const uint16_t *__restrict__ q16, const uint16_t *kc, const uint16_t *vc,
+                                                                 float *__restrict__ scores, float *attn_out, const float *__restrict__ lut, int n_ctx, float scale) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    __shared__ __attribute__((aligned(16))) uint4 s_qh[16];
+    __shared__ __attribute__((aligned(16))) float s_t[XF_MAX], s_e[XF_MAX + 32], s_grp[(XF_MAX / 4 + 63) / 64 * 64];
+    __shared__ __attribute__((aligned(16))) uint16_t s_tail[8][32];
+    __shared__ float s_sum;
+    const int cap = n_ctx < XF_MAX ? n_ctx : XF_MAX;
+    const int n_head = (int)gridDim.x >> 3, hd_ = (int)blockIdx.x % n_head, dgrp = (int)blockIdx.x / n_head, d = n_head * 128;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int VS = (cap + 63) / 64 * 64 + 32;                         // as xattn_pv_vstride
+    uint4 *s_k = (uint4 *)smem;                                       // [token][16 pieces], rotated by 4 pieces per token against bank conflicts
+    uint16_t *s_v = (uint16_t *)smem;                                 // the rows of V^T, once the keys have been read
+    const uint16_t *vrow = vc + (size_t)(hd_ * 128 + dgrp * 16 + wave) * n_ctx;
+    // Keys first, then the rows of V^T.  What the first piece of either holds does not depend on the position, which is itself on its way: 64 keys and
+    // 512 elements of a row, as far as the cache goes; what lies behind the last token is not used.
+    xp_u4 kr[XF_NP], vb, vb1, qr;
+    auto key_piece = [&](int u, int n) {
+        const int c = min(tid + u * XP_THREADS, n * 16 - 1);
+        kr[u] = *(const xp_u4 *)(kc + (size_t)(c >> 4) * d + hd_ * 128 + (c & 15) * 8);
+    };
+    key_piece(0, cap);
+    if (tid < 16) qr = *(const xp_u4 *)(q16 + hd_ * 128 + tid * 8);
+    const int n_kv = min((st ? st->pos : pos_imm) + 1, cap), npiece = n_kv * 16, last_piece = (n_kv - 1) >> 3;
+    vb = *(const xp_u4 *)(vrow + (size_t)min(lane, n_ctx % 8 ? last_piece : n_ctx / 8 - 1) * 8);
+    if (last_piece >= 64) vb1 = *(const xp_u4 *)(vrow + (size_t)min(64 + lane, last_piece) * 8);
+#pragma unroll
+    for (int u = 1; u < XF_NP; u++) if (u * XP_THREADS < npiece) key_piece(u, n_kv);
+    if (tid < 16) *(xp_u4 *)&s_qh[tid] = qr;
+#pragma unroll
+    for (int u = 0; u < XF_NP; u++) {
+        const int c = tid + u * XP_THREADS, t = c >> 4;
+        if (c < npiece) *(xp_u4 *)&s_k[t * 16 + (((c & 15) + 4 * t) & 15)] = kr[u];
+    }
+    __syncthreads();
+    // four adjacent threads per key, thread `part` with accumulators 8 part .. 8 part + 7 (xattn_scores_kernel's form for few keys)
+    for (int base = 0; base < n_kv * 4; base += XP_THREADS) {
+        const int key = (base + tid) >> 2, part = tid & 3;
+        if (key >= n_kv) break;
+        const uint4 *kp = s_k + key * 16;
+        const int rot = 4 * key;
+        float sum[8];
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const uint4 kv = kp[(4 * i + part + rot) & 15], qv = s_qh[4 * i + part];
+            const uint32_t kw[4] = {kv.x, kv.y, kv.z, kv.w}, qw[4] = {qv.x, qv.y, qv.z, qv.w};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                sum[2 * e] = fmaf(h2f((uint16_t)(kw[e] & 0xFFFFu)), h2f((uint16_t)(qw[e] & 0xFFFFu)), i == 0 ? 0.0f : sum[2 * e]);
+                sum[2 * e + 1] = fmaf(h2f((uint16_t)(kw[e] >> 16)), h2f((uint16_t)(qw[e] >> 16)), i == 0 ? 0.0f : sum[2 * e + 1]);
+            }
+        }
+        // sum[0] += sum[2], sum[1] += sum[3]; sum[0] += sum[1] over the four threads, then the tree of FP16::block_reduce
+#pragma unroll
+        for (int l = 0; l < 8; l++) {
+            sum[l] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum[l]), 0x4E, 0xF, 0xF, true));        // quad_perm [2, 3, 0, 1]
+            sum[l] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum[l]), 0xB1, 0xF, 0xF, true));        // quad_perm [1, 0, 3, 2]
+        }
+        const float u0 = sum[0] + sum[4], u1 = sum[1] + sum[5], u2 = sum[2] + sum[6], u3 = sum[3] + sum[7];
+        const float v0 = u0 + u1, v1 = u2 + u3, simd = v0 + v1;
+        float tail = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint4 kv = kp[(12 + j + rot) & 15], qv = s_qh[12 + j];
+            const uint32_t kw[4] = {kv.x, kv.y, kv.z, kv.w}, qw[4] = {qv.x, qv.y, qv.z, qv.w};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                tail = fmaf(h2f((uint16_t)(kw[e] & 0xFFFFu)), h2f((uint16_t)(qw[e] & 0xFFFFu)), tail);
+                tail = fmaf(h2f((uint16_t)(kw[e] >> 16)), h2f((uint16_t)(qw[e] >> 16)), tail);
+            }
+        }
+        if (part == 0) {
+            s_t[key] = (tail + simd) * scale;
+            if (dgrp == 0) scores[(size_t)hd_ * n_ctx + key] = s_t[key];      // as the launch of its own leaves them
+        }
+    }
+    __syncthreads();
+    // the keys are dead: the rows of V^T take their place; the maximum, by every wave for itself; the exponentials
+    if (lane <= last_piece) *(xp_u4 *)(s_v + (size_t)wave * VS + lane * 8) = vb;
+    if (64 + lane <= last_piece) *(xp_u4 *)(s_v + (size_t)wave * VS + 512 + lane * 8) = vb1;
+    if (wave * 64 < n_kv) {
+        float mx = -INFINITY;
+        for (int j = lane; j < n_kv; j += 64) mx = fmaxf(mx, s_t[j]);
+        mx = wave_max(mx);
+        const float e = lut[f2h(s_t[min(tid, n_kv - 1)] - mx)];
+        s_e[tid] = tid < n_kv ? e : 0.0f;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        // std::reduce: groups of four added to one running sum (at most 144 of them: a plain chain; zeros behind the last one leave it as it is), then the last n % 4 elements
+        const int ngrp = n_kv / 4;
+#pragma unroll
+        for (int u = 0; u < (XF_MAX / 4 + 63) / 64; u++) {
+            const int g = lane + 64 * u;
+            const float4 v = g < ngrp ? *(const float4 *)(s_e + 4 * g) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const float v1 = v.x + v.y, v2 = v.z + v.w;
+            s_grp[g] = v1 + v2;
+        }
+        __builtin_amdgcn_wave_barrier();
+        float sum = 0.0f;
+        for (int g = 0; g < ngrp; g += 16) {
+            float4 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) v[u] = *(const float4 *)(s_grp + g + 4 * u);
+#pragma unroll
+            for (int u = 0; u < 4; u++) { sum = sum + v[u].x; sum = sum + v[u].y; sum = sum + v[u].z; sum = sum + v[u].w; }
+        }
+        for (int j = ngrp * 4; j < n_kv; j++) sum = sum + s_e[j];
+        if (lane == 0) s_sum = sum;
+    }
+    __syncthreads();
+    if (wave >= 8) return;
+    // P.V^T as in xattn_pv_kernel, the probabilities formed where they are used
+    const float inv = 1.0f / s_sum;
+    const int nfull = (n_kv - 1) / 32, ntail = n_kv - 32 * nfull, r16 = wave * 2 + (lane >> 5), cl = lane & 31;
+    const uint16_t *vr = s_v + (size_t)r16 * VS;
+    if (lane < 32) s_tail[wave][lane] = f2h(s_e[32 * nfull + lane] * inv);
+    float acc = 0.0f;
+    for (int i = 0; i < nfull; i++) acc = fmaf(h2f(vr[32 * i + cl]), h2f(f2h(s_e[32 * i + cl] * inv)), acc);
+    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc), __float_as_uint(acc), false, false);
+    acc = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+#define XP_ADD(CTRL) acc += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc), CTRL, 0xF, 0xF, true));
+    XP_ADD(0x128) XP_ADD(0x124) XP_ADD(0xB1) XP_ADD(0x4E)
+#undef XP_ADD
+    __builtin_amdgcn_wave_barrier();
+    float tail = 0.0f;
+    xp_u4 tv[4], tq[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) { tv[u] = *(const xp_u4 *)(vr + 32 * nfull + 8 * u); tq[u] = *(const xp_u4 *)&s_tail[wave][8 * u]; }
+#pragma unroll
+    for (int e = 0; e < 32; e++) {
+        const uint32_t wv = tv[e >> 3][(e >> 1) & 3], wq = tq[e >> 3][(e >> 1) & 3];
+        if (e < ntail) tail = fmaf(h2f((uint16_t)(e & 1 ? wv >> 16 : wv & 0xFFFFu)), h2f((uint16_t)(e & 1 ? wq >> 16 : wq & 0xFFFFu)), tail);
+    }
+    if (cl == 0) attn_out[hd_ * 128 + dgrp * 16 + r16] = tail + acc;
+}
+
+int spy_attn_short_prepare(int n_ctx) { return spy_raise_lds_limit((const void *)xattn_short_kernel, xattn_short_lds(n_ctx)); }
+// scores: [n_head][n_ctx], as the launch of xattn_scores_kernel leaves them
+int spy_attn_short(hipStream_t st, const dev_state *state, int pos_imm, const uint16_t *q16, const uint16_t *kc, const uint16_t *vc, float *scores, float *out,
+                   const float *lut, int n_head, int n_ctx, float scale) {
+    xattn_short_kernel<<<dim3((unsigned)(n_head * 8)), dim3(XP_THREADS), xattn_short_lds(n_ctx), st>>>(state, pos_imm, q16, kc, vc, scores, out, lut, n_ctx, scale);
+    return SPY_LAUNCH_RC();
+}

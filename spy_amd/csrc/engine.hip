@@ -35,6 +35,14 @@ int spy_exact_luts(const float **lut);           // exact_order.hip
 // exact-order switch is on (and the exact kernels take the model), else this backend's own
 static int pass_order(const spy_hip_llama *m) { return (m->exact_ok && (m->order == 1 || spy_exact_on())) ? 1 : 0; }
 static int enqueue_pass_any(spy_hip_llama *m, hipStream_t st, int mode);
+static void drop_graphs(spy_hip_llama *m) {
+    for (auto &kind : m->graphs)
+        for (auto &g : kind) {
+            if (g.exec) (void)hipGraphExecDestroy(g.exec);
+            if (g.graph) (void)hipGraphDestroy(g.graph);
+            g.exec = nullptr; g.graph = nullptr;
+        }
+}
 
 static int dalloc(spy_hip_llama *m, void **p, size_t bytes, bool zero) {
     HIP_TRY(hipMalloc(p, bytes));
@@ -46,10 +54,7 @@ static int dalloc(spy_hip_llama *m, void **p, size_t bytes, bool zero) {
 extern "C" int spy_hip_llama_destroy(spy_hip_llama *m) {
     if (!m) return 0;
     (void)hipDeviceSynchronize();
-    if (m->graph_exec) (void)hipGraphExecDestroy(m->graph_exec);
-    if (m->graph_n_exec) (void)hipGraphExecDestroy(m->graph_n_exec);
-    if (m->graph_n) (void)hipGraphDestroy(m->graph_n);
-    if (m->graph) (void)hipGraphDestroy(m->graph);
+    drop_graphs(m);
     if (m->own_stream) (void)hipStreamDestroy(m->own_stream);
     if (m->ev0) (void)hipEventDestroy(m->ev0);
     if (m->ev1) (void)hipEventDestroy(m->ev1);
@@ -153,6 +158,7 @@ extern "C" int spy_hip_llama_create(const spy_hip_llama_desc *desc, spy_hip_llam
         if (!rc) rc = spy_exact_luts(&m->lut);
         if (!rc) rc = spy_ensure_lds(m, (const void *)xattn_pv_kernel<0>, xattn_pv_lds(c.n_ctx));
         if (!rc) rc = spy_ensure_lds(m, (const void *)xattn_scores_kernel<0>, xattn_scores_lds(c.n_head));
+        if (!rc) rc = spy_attn_short_prepare(c.n_ctx);
         if (!rc) {
             m->exact_ok = true;
             m->order = 1;
@@ -222,9 +228,10 @@ static bool fused_ok(const spy_hip_llama *m) {
 
 static int enqueue_one(spy_hip_llama *m, hipStream_t st, int which, int il) {
     const spy_hip_llama_desc &c = m->desc;
-    if (pass_order(m) == 1 || (m->dry && m->order == 1)) {      // the host backend's summation order: six launches per layer
+    if (pass_order(m) == 1 || (m->dry && m->order == 1)) {      // the host backend's summation order: six launches per layer, five where the cache is short
+        const bool one_launch = m->kv_bound > 0 && m->kv_bound <= XF_MAX && !getenv("SPY_HIP_SCORES_GRID");
         if (which == K_SCORES) {
-            if (m->dry) return 0;
+            if (m->dry || one_launch) return 0;
             // one workgroup per compute unit; SPY_HIP_SCORES_GRID (tests) forces fewer, so that a workgroup's share of the tokens
             // takes several rounds of XS_TOK, as it would on a part with fewer compute units or a longer cache
             int sgrid = m->num_cu;
@@ -235,6 +242,8 @@ static int enqueue_one(spy_hip_llama *m, hipStream_t st, int which, int il) {
         }
         if (which == K_PV) {
             if (m->dry) return 0;
+            if (one_launch)
+                return spy_attn_short(st, m->st, m->pos_imm, m->q16, m->k_cache[il], m->v_cache[il], m->scores, m->attn_out, m->lut, c.n_head, c.n_ctx, 1.0f / sqrtf((float)m->hd));
             xattn_pv_kernel<0><<<dim3((unsigned)(c.n_head * 8)), dim3(XP_THREADS), xattn_pv_lds(c.n_ctx), st>>>(m->st, m->pos_imm, m->scores, m->v_cache[il], m->attn_out, m->lut, c.n_ctx, m->stamp_dbg);
             return SPY_LAUNCH_RC();
         }
@@ -300,8 +309,7 @@ extern "C" int spy_hip_llama_set_spin_limit(spy_hip_llama *m, uint32_t polls) {
     SPY_CHECK_ARG(m);
     m->spin_limit = polls;
     // captured graphs carry the old limit in their kernel arguments
-    if (m->graph_exec) { (void)hipGraphExecDestroy(m->graph_exec); m->graph_exec = nullptr; }
-    if (m->graph_n_exec) { (void)hipGraphExecDestroy(m->graph_n_exec); m->graph_n_exec = nullptr; }
+    drop_graphs(m);
     return 0;
 }
 
@@ -702,7 +710,10 @@ static int forward_any(spy_hip_llama *m, void *stream, const int32_t *tokens_hos
     if (n_token == 1 && fused_ok(m) && (!exact || m->exact_ok)) {
         dev_state h = {tokens_host[0], n_past, 0, 0};
         HIP_TRY(hipMemcpyAsync(m->st, &h, sizeof(h), hipMemcpyHostToDevice, st));
-        RC_TRY(enqueue_pass_any(m, st, PASS_LOGITS));
+        m->kv_bound = n_past + 1;
+        const int rc = enqueue_pass_any(m, st, PASS_LOGITS);
+        m->kv_bound = 0;
+        if (rc) return rc;
         if (logits_host) HIP_TRY(hipMemcpyAsync(logits_host, m->logits, (size_t)m->desc.n_vocab * 4, hipMemcpyDeviceToHost, st));
         return check_pass_error(m, st);
     }
@@ -761,35 +772,43 @@ extern "C" int spy_hip_llama_decode_greedy(spy_hip_llama *m, void *stream, int32
     dev_state h = {first_token, n_past, 0, 0};
     HIP_TRY(hipMemcpyAsync(m->st, &h, sizeof(h), hipMemcpyHostToDevice, st));
     HIP_TRY(hipStreamSynchronize(st));
-    if (use_graph && (!m->graph_exec || !m->graph_n_exec || m->graph_stream != st || m->graph_order != pass_order(m))) {
+    // Nothing in a pass depends on the host (token, position and step count live on the device) but the choice of its attention launches: passes that end
+    // at a short cache, and passes anywhere, are graphs of their own, captured when a run first needs them.
+    auto short_run = [&](int pos, int steps) { return pass_order(m) == 1 && pos + steps <= XF_MAX; };
+    if (use_graph) {
+        if (m->graph_stream != st || m->graph_order != pass_order(m)) drop_graphs(m);
         m->graph_order = pass_order(m);
-        if (m->graph_exec) { (void)hipGraphExecDestroy(m->graph_exec); m->graph_exec = nullptr; }
-        if (m->graph) { (void)hipGraphDestroy(m->graph); m->graph = nullptr; }
-        HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        const int rc = enqueue_pass_any(m, st, PASS_GREEDY);
-        hipError_t e = hipStreamEndCapture(st, &m->graph);
-        if (rc) return rc;
-        if (e != hipSuccess) return (int)e;
-        HIP_TRY(hipGraphInstantiate(&m->graph_exec, m->graph, nullptr, nullptr, 0));
         m->graph_stream = st;
-        // several passes as one graph: nothing in a pass depends on the host (token, position and step count live on the device)
-        if (m->graph_n_exec) { (void)hipGraphExecDestroy(m->graph_n_exec); m->graph_n_exec = nullptr; }
-        if (m->graph_n) { (void)hipGraphDestroy(m->graph_n); m->graph_n = nullptr; }
-        HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        int rcn = 0;
-        for (int i = 0; i < SPY_GRAPH_STEPS && !rcn; i++) rcn = enqueue_pass_any(m, st, PASS_GREEDY);
-        e = hipStreamEndCapture(st, &m->graph_n);
-        if (rcn) return rcn;
-        if (e != hipSuccess) return (int)e;
-        HIP_TRY(hipGraphInstantiate(&m->graph_n_exec, m->graph_n, nullptr, nullptr, 0));
+        const bool need[2] = {!short_run(n_past, n_steps), short_run(n_past, n_steps < SPY_GRAPH_STEPS ? 1 : SPY_GRAPH_STEPS)};
+        for (int kind = 0; kind < 2; kind++)
+            for (int many = 0; many < 2 && need[kind]; many++) {
+                auto &g = m->graphs[kind][many];
+                if (g.exec) continue;
+                if (g.graph) { (void)hipGraphDestroy(g.graph); g.graph = nullptr; }
+                m->kv_bound = kind ? XF_MAX : 0;
+                HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+                int rc = 0;
+                for (int i = 0; i < (many ? SPY_GRAPH_STEPS : 1) && !rc; i++) rc = enqueue_pass_any(m, st, PASS_GREEDY);
+                m->kv_bound = 0;
+                const hipError_t e = hipStreamEndCapture(st, &g.graph);
+                if (rc) return rc;
+                if (e != hipSuccess) return (int)e;
+                HIP_TRY(hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0));
+            }
     }
     RC_TRY(enqueue_embed(m, st));              // embedding of the first token; every step prepares the next one's
     HIP_TRY(hipEventRecord(m->ev0, st));
     for (int i = 0; i < n_steps;) {
-        if (use_graph && n_steps - i >= SPY_GRAPH_STEPS) { HIP_TRY(hipGraphLaunch(m->graph_n_exec, st)); i += SPY_GRAPH_STEPS; continue; }
-        if (use_graph) HIP_TRY(hipGraphLaunch(m->graph_exec, st));
-        else RC_TRY(enqueue_pass_any(m, st, PASS_GREEDY));
-        i++;
+        const int steps = use_graph && n_steps - i >= SPY_GRAPH_STEPS ? SPY_GRAPH_STEPS : 1;
+        const auto &kind = m->graphs[short_run(n_past + i, steps)];
+        if (use_graph) HIP_TRY(hipGraphLaunch(kind[steps > 1].exec, st));
+        else {
+            m->kv_bound = n_past + i + 1;
+            const int rc = enqueue_pass_any(m, st, PASS_GREEDY);
+            m->kv_bound = 0;
+            if (rc) return rc;
+        }
+        i += steps;
     }
     HIP_TRY(hipEventRecord(m->ev1, st));
     HIP_TRY(hipEventSynchronize(m->ev1));
@@ -991,6 +1010,8 @@ extern "C" int spy_hip_attn_decode(void *stream, int32_t order, const void *q16,
         if (n_ctx > 512 * XP_NP || xattn_pv_lds((int)n_ctx) > 160 * 1024 - 256 || xattn_scores_lds(n_head) > 160 * 1024) return SPY_HIP_EUNSUPPORTED;
         RC_TRY(spy_ensure_lds(&f.m, (const void *)xattn_pv_kernel<0>, xattn_pv_lds((int)n_ctx)));
         RC_TRY(spy_ensure_lds(&f.m, (const void *)xattn_scores_kernel<0>, xattn_scores_lds(n_head)));
+        RC_TRY(spy_attn_short_prepare((int)n_ctx));
+        f.m.kv_bound = n_kv;
     } else {
         if (pv_lds > 160 * 1024) return SPY_HIP_EUNSUPPORTED;
         RC_TRY(spy_ensure_lds(&f.m, (const void *)attn_pv_kernel, pv_lds));

@@ -30,9 +30,10 @@ struct spy_hip_llama {
     float theta_scale = 0.0f;
     // op-by-op path scratch (sized lazily for the largest chunk seen)
     uint8_t *ops_buf = nullptr; size_t ops_bytes = 0;
-    // graph of one single-token pass
-    hipGraph_t graph = nullptr; hipGraphExec_t graph_exec = nullptr; hipStream_t graph_stream = nullptr;
-    hipGraph_t graph_n = nullptr; hipGraphExec_t graph_n_exec = nullptr;   // SPY_GRAPH_STEPS passes in one graph
+    // graphs of single-token passes: [0] for any position, [1] for caches of up to XF_MAX tokens; one pass, SPY_GRAPH_STEPS passes
+    struct pass_graph { hipGraph_t graph = nullptr; hipGraphExec_t exec = nullptr; } graphs[2][2];
+    hipStream_t graph_stream = nullptr;
+    int kv_bound = 0;                                                      // the passes being enqueued see no more cached tokens than this (0: not known)
     int graph_order = -1;                                                  // summation order the graphs were captured with
     hipStream_t own_stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -71,6 +72,12 @@ static inline bool wave_ok(const spy_hip_llama *m) {
     const spy_hip_llama_desc &c = m->desc;
     return c.n_embd % 64 == 0 && c.n_embd <= 4096 && c.n_ff % 64 == 0 && c.n_ff <= 16384 && m->hd <= WGV_THREADS && m->hd % 2 == 0 && c.n_embd % 2 == 0;
 }
+
+// attn_short.hip: the attention of one token in order 1 over up to XF_MAX cached tokens, one launch
+#define XF_MAX 576
+int spy_attn_short_prepare(int n_ctx);
+int spy_attn_short(hipStream_t st, const dev_state *state, int pos_imm, const uint16_t *q16, const uint16_t *kc, const uint16_t *vc, float *scores, float *out,
+                   const float *lut, int n_head, int n_ctx, float scale);
 
 enum { K_QKV = 0, K_SCORES, K_PV, K_WO, K_GATEUP, K_DOWN, K_HEAD, K_COUNT };
 

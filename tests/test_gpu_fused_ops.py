@@ -215,6 +215,31 @@ def test_attn_decode(hip, oracle, order, n_kv):
     _check(do.download(np.float32), out.reshape(-1), "attention output, n_kv %d" % n_kv, order)
 
 
+@pytest.mark.parametrize("n_head", [32, 3])
+@pytest.mark.parametrize("n_kv,n_ctx", [(1, 8), (3, 8), (4, 8), (5, 64), (31, 32), (32, 32), (33, 40), (63, 64), (64, 64), (65, 72), (255, 256), (257, 264), (511, 512), (512, 512),
+                                        (513, 520), (575, 576), (576, 576), (576, 1024), (577, 584)])
+def test_attn_decode_short_cache(hip, n_head, n_kv, n_ctx, monkeypatch):
+    """Up to 576 cached tokens order 1 takes one launch: the bits of the two launches (which SPY_HIP_SCORES_GRID asks for), scores and outputs, at the edges of
+    its chunks, key tiles and row pieces; NaN behind the last token."""
+    from tests.gpu_util import dev, dev_empty, call
+    d = n_head * 128
+    rng = np.random.default_rng(n_kv * 7 + n_head)
+    q16 = (rng.standard_normal(d) * 1.5).astype(np.float16)
+    kc, vc = rng.standard_normal((n_ctx, d)).astype(np.float16), rng.standard_normal((d, n_ctx)).astype(np.float16)
+    kc[n_kv:] = np.nan; vc[:, n_kv:] = np.nan
+    dq, dk, dv = dev(q16.view(np.uint16)), dev(kc.view(np.uint16)), dev(vc.view(np.uint16))
+    res = []
+    for grid in (None, "256"):
+        monkeypatch.delenv("SPY_HIP_SCORES_GRID", raising=False) if grid is None else monkeypatch.setenv("SPY_HIP_SCORES_GRID", grid)
+        ds, do = dev_empty(n_head * n_ctx * 4, 0xEE), dev_empty(d * 4, 0xEE)
+        call(hip.load().spy_hip_attn_decode, None, 1, dq.ptr, dk.ptr, dv.ptr, n_head, n_kv, n_ctx, ds.ptr, do.ptr)
+        hip.sync()
+        res.append((ds.download(np.uint32).reshape(n_head, n_ctx).copy(), do.download(np.uint32).copy()))
+    assert np.array_equal(res[0][0], res[1][0]), "scores"
+    assert np.array_equal(res[0][1], res[1][1]), "outputs"
+    assert not np.isnan(res[0][1].view(np.float32)).any()
+
+
 @pytest.mark.parametrize("grid,n_kv", [(64, 4351), (7, 300), (100, 1900)])
 def test_attn_scores_in_several_rounds(hip, grid, n_kv, monkeypatch):
     """The score kernel of order 1 deals the cached tokens out over its workgroups and takes a workgroup's share in rounds of 18

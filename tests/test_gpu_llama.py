@@ -210,6 +210,32 @@ def test_fused_decode_real_widths_long_cache(order, n_ctx, positions):
     eng.close()
 
 
+def test_greedy_run_over_the_end_of_the_short_cache(monkeypatch):
+    """Tokens, logits and caches of greedy runs that begin on a cache short enough for the one-launch attention and end on a longer one, with and without
+    graphs, against the same runs on the two-launch attention throughout (SPY_HIP_SCORES_GRID)."""
+    from spy_amd import model as M
+    cfg = M.Config(n_layer=2, n_embd=512, n_head=4, n_ff=1024, n_vocab=512, n_ctx=640, wtype=O.Q4_0)
+    tensors = M.synth_model(cfg, seed=3)
+    prompt = np.random.default_rng(5).integers(0, cfg.n_vocab, 545).astype(np.int32)
+    runs = []
+    for grid in (None, "256"):
+        monkeypatch.delenv("SPY_HIP_SCORES_GRID", raising=False) if grid is None else monkeypatch.setenv("SPY_HIP_SCORES_GRID", grid)
+        eng = M.Engine(cfg, tensors, order=1)
+        eng.forward_last(prompt, 0)
+        out = []
+        for use_graph in (True, False, True):
+            for n_past, steps in ((545, 60), (562, 14), (568, 9), (575, 3), (100, 7), (545, 60)):
+                out.append(eng.decode_greedy(int(prompt[n_past % 64]), n_past, steps, use_graph=use_graph))
+                out.append(eng.read_buffer("logits", 0, np.uint32))
+        for n_past in (574, 575, 576):
+            out.append(eng.forward(prompt[:1], n_past).view(np.uint32))
+        out.append(eng.read_buffer("k_cache", 1, np.uint16))
+        runs.append(out)
+        eng.close()
+    for i, (a, b) in enumerate(zip(*runs)):
+        assert np.array_equal(a, b), i
+
+
 def test_model_wider_than_4096_takes_the_tiled_kernels():
     """n_embd = 5120 (the 13B width): the one-row-per-wave kernels stage 4096 activations per workgroup at most, so the fused
     single-token pass of such a model runs the 256-thread tiled kernels, in this backend's own summation order (the kernels of

@@ -11,8 +11,8 @@
 //   * The vector units do one fma per term; that is what bounds the kernel: 4096 x 4096 x 2048 is 1.34e8 wave-fmas = 255 us at the
 //     2.05 GHz the part holds under this load.
 //   * A weight word is used by exactly one wave, which unpacks it itself (0x6400 | n is the fp16 1024 + n) and applies it to C groups
-//     of 16 activation rows.  The accumulators of an output are split over AS waves (words 0..3 | 4..7, or pairs of words), which meet
-//     in hsum_float_8 at the end: few activation rows still give AS * rows / 16 waves, and a wave's chain is AS times shorter.
+//     of 16 activation rows.  The accumulators of an output are split over two waves (words 0..3 | 4..7), which meet in hsum_float_8 at the
+//     end: a wave's chain is half as long.
 //   * Weights (in chunks of eight blocks) and activations (in stages of four) go from memory straight into rings of LDS slots
 //     (global_load_lds), P stages ahead of their use, one workgroup barrier per stage.
 // Measured against what these kernels replaced (operands packed as fp16 once per call, 64 x 64 tiles), packing included:
@@ -76,10 +76,11 @@ struct xt_args {
     const uint8_t *xq, *xd;
 };
 
-// AS: waves that share the accumulators of a tile (2 or 4); RG: groups of 16 weight rows per workgroup; C: groups of 16 activation rows per
+// AS: waves that share the accumulators of a tile; RG: groups of 16 weight rows per workgroup; C: groups of 16 activation rows per
 // wave; NXS, NWC: LDS slots for stages and chunks (powers of two); P: stages requested ahead
-template <int WT, int AS, int RG, int C, int NXS, int P, int NWC>
+template <int WT, int C, int NXS, int P, int NWC>
 __device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
+    constexpr int AS = 2, RG = 2;
     constexpr int NT = 64 * AS * RG, ROWS = 16 * RG;
     constexpr int CU = xt_w<WT>::CU, UW = ROWS * CU, NI = (UW + NT - 1) / NT, NXI = C * 256 / NT;
     constexpr int XB = C * (XT_XB + 256), WB = (UW + 63) / 64 * 1024;
@@ -135,34 +136,29 @@ __device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
 #pragma unroll
         for (int i = 0; i < NACC; i++) acc[c][i] = 0.0f;
 
-    // Where a lane finds its operands.  AS == 2: word 4g + q of one block per matrix instruction.  AS == 4: lane block q holds word 2g + (q & 1)
-    // of block 2i + (q >> 1), so one instruction takes two blocks.  A Q4_0 block holds words 0..3 in the low nibbles and 4..7 in the
+    // Where a lane finds its operands: word 4g + q of one block per matrix instruction.  A Q4_0 block holds words 0..3 in the low nibbles and 4..7 in the
     // high nibbles of its four quant dwords (which start at byte 2: blocks at odd dword halves are read as two dwords).
     constexpr bool Q4 = WT == SPY_HIP_Q4_0;
     constexpr int PD = xt_w<WT>::PD, OD = Q4 ? 5 : 9, BB = xt_w<WT>::BB;
-    const int kbpar = q >> 1;
     const uint32_t wbase = (rg * 16 + r) * xt_w<WT>::CB +
-                           4 * (AS == 2 ? q + (Q4 ? 0 : 4 * g) : kbpar * OD + (q & 1) + (Q4 ? 2 * (g & 1) : 2 * g));
-    const uint32_t al = AS == 4 && kbpar ? 0 : 16;
-    const int sh = Q4 ? 4 * (AS == 2 ? g : g >> 1) : 0;
+                           4 * (q + (Q4 ? 0 : 4 * g));
+    const int sh = Q4 ? 4 * g : 0;
     const uint32_t dbase = (rg * 16 + r) * xt_w<WT>::CB + q * BB;
-    const uint32_t xbase = AS == 2 ? (2 * g + (q >> 1)) * 256 + r * 16 + (q & 1) * 8 : kbpar * 1024 + g * 256 + r * 16 + (q & 1) * 8;
+    const uint32_t xbase = (2 * g + (q >> 1)) * 256 + r * 16 + (q & 1) * 8;
     const uint32_t c64 = 0x64006400u;
 
     auto compute = [&](int s, auto par_c) {
         constexpr int par = decltype(par_c)::value;                 // which half of the chunk
         const uint8_t *sx = smem + (s & (NXS - 1)) * XB, *sw = smem + NXS * XB + ((s >> 1) & (NWC - 1)) * WB;
-        constexpr int NW = AS == 2 ? 4 : 2;                         // weight operands of the stage
+        constexpr int NW = 4;                                       // weight operands of the stage
         uint32_t wa[NW], wb[NW];
         {
             const uint32_t *b = (const uint32_t *)(sw + wbase);
             uint32_t v[NW];
 #pragma unroll
             for (int i = 0; i < 2; i++) {
-                if constexpr (AS == 2) {
-                    v[2 * i] = __builtin_amdgcn_alignbit(b[PD * (2 * par + i) + 1], b[PD * (2 * par + i)], 16);
-                    v[2 * i + 1] = b[PD * (2 * par + i) + OD];
-                } else v[i] = __builtin_amdgcn_alignbit(b[PD * (2 * par + i) + 1], b[PD * (2 * par + i)], al);
+                v[2 * i] = __builtin_amdgcn_alignbit(b[PD * (2 * par + i) + 1], b[PD * (2 * par + i)], 16);
+                v[2 * i + 1] = b[PD * (2 * par + i) + OD];
             }
 #pragma unroll
             for (int i = 0; i < NW; i++) {                          // elements 0, 2 and 1, 3 of the word
@@ -182,7 +178,7 @@ __device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
         // steps (activation group, weight operand), pipelined by hand: the activations of step j + 2 are read and the matrix instruction of step
         // j + 1 is issued before the fmas on the result of step j
         constexpr int NJ = C * NW;
-        auto rd = [&](int j) -> uint2 { return *(const uint2 *)(sx + (j / NW) * XT_XB + (j % NW) * (AS == 2 ? 1024 : 2048) + xbase); };
+        auto rd = [&](int j) -> uint2 { return *(const uint2 *)(sx + (j / NW) * XT_XB + (j % NW) * 1024 + xbase); };
         uint2 xv[3];
         xt_v16f p[2], D[2];
         uint32_t dx = *(const uint32_t *)sd, dxn = 0;
@@ -204,15 +200,8 @@ __device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
                 p[(j + 1) & 1] = xt_mfma(wa[i1], wb[i1], xv[(j + 1) % 3].x, xv[(j + 1) % 3].y);
             }
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (AS == 2) {
 #pragma unroll
-                for (int n = 0; n < 16; n++) acc[c][n] = fmaf(D[c & 1][4 * i + (n & 3)], p[j & 1][n], acc[c][n]);
-            } else {
-#pragma unroll
-                for (int b = 0; b < 2; b++)
-#pragma unroll
-                    for (int n = 0; n < 8; n++) acc[c][n] = fmaf(D[c & 1][4 * (2 * i + b) + (n & 3)], p[j & 1][8 * b + n], acc[c][n]);
-            }
+            for (int n = 0; n < 16; n++) acc[c][n] = fmaf(D[c & 1][4 * i + (n & 3)], p[j & 1][n], acc[c][n]);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -254,16 +243,8 @@ __device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             float rr[4];
-            if constexpr (AS == 2) {
 #pragma unroll
-                for (int k = 0; k < 4; k++) rr[k] = ex[(c * NACC + 4 * k + v) * 64 + lane] + acc[c][4 * k + v];
-            } else {
-#pragma unroll
-                for (int k = 0; k < 2; k++) {
-                    rr[k] = ex[((C + c) * NACC + 4 * k + v) * 64 + lane] + acc[c][4 * k + v];
-                    rr[2 + k] = ex[((2 * C + c) * NACC + 4 * k + v) * 64 + lane] + ex[(c * NACC + 4 * k + v) * 64 + lane];
-                }
-            }
+            for (int k = 0; k < 4; k++) rr[k] = ex[(c * NACC + 4 * k + v) * 64 + lane] + acc[c][4 * k + v];
             const float s0 = rr[0] + rr[2], s1 = rr[1] + rr[3];
             o[v] = s0 + s1;
         }
@@ -278,15 +259,174 @@ __device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
     }
 }
 
-template <int WT, int AS, int RG, int C, int NXS, int P, int NWC, int OCC>
-__global__ __launch_bounds__(64 * AS * RG, OCC) void xt_kernel(xt_args a) { xt_tile<WT, AS, RG, C, NXS, P, NWC>(a, (int)blockIdx.y * C); }
+template <int WT, int C, int NXS, int P, int NWC>
+__global__ __launch_bounds__(256, 3) void xt_kernel(xt_args a) { xt_tile<WT, C, NXS, P, NWC>(a, (int)blockIdx.y * C); }
 // Tiles of four activation groups and, behind them in the grid, one of the R groups that remain: the sums of groups that do not exist cost as much
 // as those of groups that do (22016 x 4096 Q4_0: 77 rows 98 -> 85 us, 140 rows 161 -> 135, 200 rows 224 -> 188, 900 rows 831 -> 796)
 template <int WT, int R>
 __global__ __launch_bounds__(256, 3) void xt_mixed_kernel(xt_args a) {
     const int full = a.ncg / 4;
-    if ((int)blockIdx.y < full) xt_tile<WT, 2, 2, 4, 2, 1, 2>(a, (int)blockIdx.y * 4);
-    else xt_tile<WT, 2, 2, R, R < 3 ? 4 : 2, R < 3 ? 2 : 1, 2>(a, full * 4);
+    if ((int)blockIdx.y < full) xt_tile<WT, 4, 2, 1, 2>(a, (int)blockIdx.y * 4);
+    else xt_tile<WT, R, R < 3 ? 4 : 2, R < 3 ? 2 : 1, 2>(a, full * 4);
+}
+
+// Few activation rows: one group of them and 16 weight rows per workgroup, the accumulators of the tile over its four waves (words 2g, 2g + 1 to wave g).
+// With a wave or two on a SIMD what bounds it is the chain barrier, LDS read, unpack, matrix instruction, fmas: it is walked once per chunk of eight
+// blocks, and the operands of the next chunk are read from LDS before the fmas of this one.  NS: LDS slots for chunks, all of them on their way: four where
+// a compute unit has one or two workgroups, whose weights come from memory (two: 20 % slower there); two, 24 KB, where it has more (four: up to
+// 20 % slower).  32 weight rows and eight waves per workgroup: 30 % slower with 4096.  From five workgroups on the tiles of 32 rows are faster.
+// Against one stage of four blocks per barrier, weights from memory, in us, packing of the activations (4 us) included: 8 rows, Q4_0 4096 x 4096 14.4 -> 12.1,
+// 4096 x 11008 30.6 -> 23.6, 12288 x 4096 21.0 -> 17.7, Q8_0 14.4 -> 12.5, 30.3 -> 24.3, 22.5 -> 20.8; 48 rows, Q4_0 4096 x 4096 21.2 -> 17.8, 4096 x 11008 47.5 -> 37.3.
+template <int WT, int NS>
+__global__ __launch_bounds__(256, 2) void xn_kernel(xt_args a) {
+    constexpr int NT = 256, ROWS = 16, CU = xt_w<WT>::CU, UW = ROWS * CU, NI = (UW + NT - 1) / NT, NXI = 2;
+    constexpr int XB = 2 * (XT_XB + 256), WB = (UW + 63) / 64 * 1024, NREQ = NXI + 1 + NI;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = wave, q = lane >> 4, r = lane & 15;
+    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS, cg = (int)blockIdx.y;
+    const int nch = a.nst / 2, M = a.M;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
+    // requests as in xt_tile: uniform bases that advance by a chunk, per-lane offsets that stay; waves 0 and 1 bring the scales of the chunk's stages (the others repeat them)
+    const uint8_t *bx = a.xq + (int64_t)cg * a.nst * XT_XB + wave * 1024, *bd = a.xd + ((int64_t)cg * a.nst + min(wave, 1)) * XT_XD, *bw = a.w[mat] + (int64_t)m0 * a.w_row;
+    uint32_t ow[NI];
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const int u = min(tid + i * NT, UW - 1);
+        ow[i] = (uint32_t)(min(m0 + u / CU, M - 1) - m0) * (uint32_t)a.w_row + (u % CU) * 16;
+    }
+    const bool spare = wave * 64 + (NI - 1) * NT >= UW;
+    const uint32_t lds_spare = __builtin_amdgcn_readfirstlane(lds0 + NS * (XB + WB));
+    const uint32_t l16 = lane * 16, l4 = lane * 4;
+    const uint32_t ldsx = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024), ldsd = __builtin_amdgcn_readfirstlane(lds0 + 2 * XT_XB + min(wave, 1) * 256),
+                   ldsw = __builtin_amdgcn_readfirstlane(lds0 + NS * XB + wave * 1024);
+    int is = 0;                                    // next chunk to request; past the last one it is requested again (same count of requests, slot unused)
+    auto issue = [&]() {
+        const uint32_t slot = is & (NS - 1);
+        const int adv = is + 1 < nch ? 1 : 0;
+#pragma unroll
+        for (int i = 0; i < NI; i++) xt_dma16(bw, ow[i], i == NI - 1 && spare ? lds_spare : ldsw + slot * WB + i * NT * 16);
+#pragma unroll
+        for (int i = 0; i < NXI; i++) xt_dma16(bx + i * NT * 16, l16, ldsx + slot * XB + i * NT * 16);
+        xt_dma4(bd, l4, ldsd + slot * XB);
+        bw += adv * xt_w<WT>::CB;
+        bx += adv * 2 * XT_XB;
+        bd += adv * 2 * XT_XD;
+        is++;
+    };
+#pragma unroll
+    for (int s = 0; s < NS; s++) issue();
+
+    float acc[8];                                  // [word 2g, 2g + 1][weight rows 4q .. 4q + 3], activation row r
+#pragma unroll
+    for (int i = 0; i < 8; i++) acc[i] = 0.0f;
+    // Where a lane finds its operands: lane block q holds word 2g + (q & 1) of block 2i + (q >> 1), so one instruction takes two blocks.  A Q4_0 block holds
+    // words 0..3 in the low nibbles and 4..7 in the high nibbles of its four quant dwords (which start at byte 2: blocks at odd dword halves are read as two dwords).
+    constexpr bool Q4 = WT == SPY_HIP_Q4_0;
+    constexpr int PD = xt_w<WT>::PD, OD = Q4 ? 5 : 9, BB = xt_w<WT>::BB;
+    const int odd = q >> 1;
+    const uint32_t wbase = r * xt_w<WT>::CB + 4 * (odd * OD + (q & 1) + (Q4 ? 2 * (g & 1) : 2 * g));
+    const uint32_t al = odd ? 0 : 16;
+    const int sh = Q4 ? 4 * (g >> 1) : 0;
+    const uint32_t dbase = r * xt_w<WT>::CB + q * BB, xbase = odd * 1024 + g * 256 + r * 16 + (q & 1) * 8;
+    const uint32_t c64 = 0x64006400u;
+    struct operands { uint32_t w0[4], w1[4], dw[2], dx[2]; uint2 x[4]; };
+    auto read = [&](int s, operands &o) {
+        const uint8_t *sx = smem + (s & (NS - 1)) * XB, *sw = smem + NS * XB + (s & (NS - 1)) * WB;
+        const uint32_t *b = (const uint32_t *)(sw + wbase);
+#pragma unroll
+        for (int i = 0; i < 4; i++) { o.w0[i] = b[PD * i]; o.w1[i] = b[PD * i + 1]; }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            o.dw[h] = *(const uint16_t *)(sw + dbase + h * 4 * BB);
+            o.dx[h] = *(const uint32_t *)(sx + 2 * XT_XB + h * 256 + lane * 4);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) o.x[i] = *(const uint2 *)(sx + i * 2048 + xbase);
+    };
+    auto compute = [&](const operands &o) {
+        uint32_t wa[4], wb[4], dw[2];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {                               // elements 0, 2 and 1, 3 of the word
+            const uint32_t v = __builtin_amdgcn_alignbit(o.w1[i], o.w0[i], al);
+            if constexpr (Q4) {
+                wa[i] = xt_sub(xt_and_or(v >> sh, 0x000F000Fu, c64), 0x64086408u);
+                wb[i] = xt_sub(xt_and_or(v >> (sh + 8), 0x000F000Fu, c64), 0x64086408u);
+            } else {
+                const uint32_t t = v ^ 0x80808080u;
+                wa[i] = xt_sub(xt_and_or(t, 0x00FF00FFu, c64), 0x64806480u);
+                wb[i] = xt_sub(xt_and_or(t >> 8, 0x00FF00FFu, c64), 0x64806480u);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) dw[h] = o.dw[h] == 0xFFFFu ? 0u : o.dw[h];         // conversion.h:39-41: the host's table has no entry for 0xFFFF
+        // the matrix instruction of step j + 1 before the fmas on the result of step j
+        xt_v16f p[2], D[2];
+        D[0] = xt_mfma(dw[0], 0u, o.dx[0], 0u);
+        p[0] = xt_mfma(wa[0], wb[0], o.x[0].x, o.x[0].y);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (j == 1) D[1] = xt_mfma(dw[1], 0u, o.dx[1], 0u);
+            if (j < 3) p[(j + 1) & 1] = xt_mfma(wa[j + 1], wb[j + 1], o.x[j + 1].x, o.x[j + 1].y);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int n = 0; n < 8; n++) acc[n] = fmaf(D[j >> 1][4 * (2 * (j & 1) + b) + (n & 3)], p[j & 1][8 * b + n], acc[n]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    operands A, B;
+    xt_wait_vm<(NS - 1) * NREQ>();
+    __builtin_amdgcn_s_barrier();
+    read(0, A);
+    auto body = [&](int s, operands &now, operands &next) {
+        xt_wait_vm<(NS - 2) * NREQ>();             // chunk s + 1 is there (the requests of the NS - 2 chunks after it may be on their way), and this wave has read chunk s
+        __builtin_amdgcn_s_barrier();
+        issue();                                   // chunk s + NS, where chunk s was
+        read(s + 1, next);                         // (past the last chunk: what the slot holds, not used)
+        __builtin_amdgcn_sched_barrier(0);
+        compute(now);
+    };
+    int s = 0;
+    for (; s + 2 <= nch; s += 2) { body(s, A, B); body(s + 1, B, A); }
+    if (s < nch) body(s, A, B);
+    xt_wait_vm<0>();
+    __builtin_amdgcn_s_barrier();
+    // hsum_float_8, as in xt_tile
+    float *ex = (float *)smem;
+    if (g > 0) {
+#pragma unroll
+        for (int n = 0; n < 8; n++) ex[((g - 1) * 8 + n) * 64 + lane] = acc[n];
+    }
+    __syncthreads();
+    if (g > 0) return;
+    const int row = m0 + 4 * q, t = cg * 16 + r;
+    float o[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        float rr[4];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            rr[k] = ex[(8 + 4 * k + v) * 64 + lane] + acc[4 * k + v];
+            rr[2 + k] = ex[(16 + 4 * k + v) * 64 + lane] + ex[(4 * k + v) * 64 + lane];
+        }
+        const float s0 = rr[0] + rr[2], s1 = rr[1] + rr[3];
+        o[v] = s0 + s1;
+    }
+    if (t < a.T && row + 3 < M) {
+        const int64_t at = (int64_t)t * a.d_row + row;
+        if (a.resid) { const float4 z = *(const float4 *)(a.resid + at); o[0] += z.x; o[1] += z.y; o[2] += z.z; o[3] += z.w; }
+        *(float4 *)(a.dst[mat] + at) = make_float4(o[0], o[1], o[2], o[3]);
+    }
+}
+template <int WT, int NS>
+int xn_launch(hipStream_t st, xt_args a, int nmat) {
+    constexpr size_t lds = NS * (2 * (XT_XB + 256) + (16 * xt_w<WT>::CU + 63) / 64 * 1024) + 1024;
+    static_assert(lds <= 64 * 1024 && lds >= 3 * 8 * 256, "no raised LDS limit; room for the exchange of the accumulators");
+    a.tiles = (a.M + 15) / 16;
+    xn_kernel<WT, NS><<<dim3((unsigned)(a.tiles * nmat), (unsigned)a.ncg), dim3(256), lds, st>>>(a);
+    return SPY_LAUNCH_RC();
 }
 
 // f32 rows -> packed activations: Quantizator<FP32,Q8_0>::transform (vec_convert.h:178-261), as quantize_q8_0_kernel, the quants as fp16.
@@ -430,21 +570,21 @@ __global__ __launch_bounds__(256) void xt_silu_pack_kernel(const float *__restri
     xt_store8(y, sub, xq + ((int64_t)cg * nst + blockIdx.x) * XT_XB + bl * 1024, xd + ((int64_t)cg * nst + blockIdx.x) * XT_XD + bl * 64, row);
 }
 
-template <int WT, int AS, int RG, int C, int NXS, int NWC> constexpr size_t xt_lds() {
-    constexpr size_t ring = NXS * C * (XT_XB + 256) + NWC * ((16 * RG * xt_w<WT>::CU + 63) / 64) * 1024 + 1024, ex = (size_t)RG * (AS - 1) * C * (32 / AS) * 256, lds = ring > ex ? ring : ex;
+template <int WT, int C, int NXS, int NWC> constexpr size_t xt_lds() {
+    constexpr size_t ring = NXS * C * (XT_XB + 256) + NWC * ((32 * xt_w<WT>::CU + 63) / 64) * 1024 + 1024, ex = (size_t)2 * C * 16 * 256, lds = ring > ex ? ring : ex;
     static_assert(lds <= 64 * 1024, "no raised LDS limit");
     return lds;
 }
-template <int WT, int AS, int RG, int C, int NXS, int P, int NWC, int OCC>
+template <int WT, int C, int NXS, int P, int NWC>
 int xt_launch(hipStream_t st, xt_args a, int nmat) {
-    a.tiles = (a.M + 16 * RG - 1) / (16 * RG);
-    xt_kernel<WT, AS, RG, C, NXS, P, NWC, OCC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * AS * RG), xt_lds<WT, AS, RG, C, NXS, NWC>(), st>>>(a);
+    a.tiles = (a.M + 31) / 32;
+    xt_kernel<WT, C, NXS, P, NWC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(256), xt_lds<WT, C, NXS, NWC>(), st>>>(a);
     return SPY_LAUNCH_RC();
 }
 template <int WT, int R>
 int xt_launch_mixed(hipStream_t st, xt_args a, int nmat) {
     a.tiles = (a.M + 31) / 32;
-    constexpr size_t l4 = xt_lds<WT, 2, 2, 4, 2, 2>(), lr = xt_lds<WT, 2, 2, R, R < 3 ? 4 : 2, 2>();
+    constexpr size_t l4 = xt_lds<WT, 4, 2, 2>(), lr = xt_lds<WT, R, R < 3 ? 4 : 2, 2>();
     xt_mixed_kernel<WT, R><<<dim3((unsigned)(a.tiles * nmat), (unsigned)(a.ncg / 4 + 1)), dim3(256), l4 > lr ? l4 : lr, st>>>(a);
     return SPY_LAUNCH_RC();
 }
@@ -1013,12 +1153,12 @@ int xt_dispatch(hipStream_t st, const xt_args &a, int nmat) {
     // the last one: tiles of four groups and one of what remains, where something remains
     static const int of_rest[4] = {0, 60, 100, 132};
     const int rest = a.ncg > 4 ? a.ncg % 4 : 0;
-    const xt_cost c[5] = {{16, 1, 86, 43}, {32, 1, 103, 56}, {32, 2, 173, 96}, {32, 4, 288, 165}, {32, 4, 288, 165, of_rest[rest]}};
+    const xt_cost c[5] = {{16, 1, 44, 44}, {32, 1, 106, 56}, {32, 2, 173, 96}, {32, 4, 288, 165}, {32, 4, 288, 165, of_rest[rest]}};
     switch (xt_pick(a, nmat, c, rest ? 5 : 4)) {
-    case 0: return xt_launch<WT, 4, 1, 1, 8, 6, 4, 2>(st, a, nmat);
-    case 1: return xt_launch<WT, 2, 2, 1, 4, 2, 2, 3>(st, a, nmat);
-    case 2: return xt_launch<WT, 2, 2, 2, 4, 2, 2, 3>(st, a, nmat);
-    case 3: return xt_launch<WT, 2, 2, 4, 2, 1, 2, 3>(st, a, nmat);
+    case 0: return (int64_t)(a.M + 15) / 16 * nmat * a.ncg <= 2 * spy_num_cu() ? xn_launch<WT, 4>(st, a, nmat) : xn_launch<WT, 2>(st, a, nmat);
+    case 1: return xt_launch<WT, 1, 4, 2, 2>(st, a, nmat);
+    case 2: return xt_launch<WT, 2, 4, 2, 2>(st, a, nmat);
+    case 3: return xt_launch<WT, 4, 2, 1, 2>(st, a, nmat);
     default: return rest == 1 ? xt_launch_mixed<WT, 1>(st, a, nmat) : rest == 2 ? xt_launch_mixed<WT, 2>(st, a, nmat) : xt_launch_mixed<WT, 3>(st, a, nmat);
     }
 }

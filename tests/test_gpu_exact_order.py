@@ -121,6 +121,13 @@ def test_packed_activation_matmul_bits(hip, oracle, wtype, M, K, T):
     assert (got[T * M:].view(np.uint32) == 0xFFFFFFFF).all(), "nothing is written beyond the outputs"
 
 
+@pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0])
+@pytest.mark.parametrize("M,K,T", [(12288, 256, 16), (12300, 768, 10), (8196, 512, 17), (4096, 256, 33), (4084, 1280, 48), (16, 512, 3), (28, 768, 32)])
+def test_narrow_matmul_bits(hip, oracle, wtype, M, K, T):
+    """Few activation rows, tiles of 16 x 16 with two and with four chunks on their way: one chunk (K = 256), odd and even numbers of them, partial tiles."""
+    test_packed_activation_matmul_bits(hip, oracle, wtype, M, K, T)
+
+
 @pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0, O.Q4_K, O.Q6_K])
 @pytest.mark.parametrize("M,K,T", [(96, 4096, 16), (200, 512, 70), (64, 128, 64), (64, 256, 64), (132, 11008, 33), (4096, 4096, 130)])
 def test_tiled_matmul_bits(hip, oracle, wtype, M, K, T, monkeypatch):

@@ -712,25 +712,32 @@ __device__ __forceinline__ void xk_unpack(const xk_raw<WT> &w, int q, uint4 (&o)
 // with sc on the weights' operand and the second sum, a contraction over sub-blocks, on v_mfma_f32_16x16x4_f32: 5 vector instructions per tile and
 // sub-block instead of 17 (Q4_K) and 9 (Q6_K).  4096 x 4096 x 1000, packing included: Q4_K 105 -> 87 us, Q6_K 112 -> 97; 22016 x 4096 x 1000: 557 -> 401
 // and 588 -> 449 (the 128 x 128 tiles of gemm.hip: 424 and 755).
-template <int WT, bool OWN, int RG, int C, int OCC>
-__global__ __launch_bounds__(64 * RG, OCC) void xk_kernel(xt_args a) {
+// KS (own order): that many sets of RG waves, each with its share of the super-blocks and activation stages of its own; their sums meet at the end.
+template <int WT, bool OWN, int RG, int C, int OCC, int KS = 1>
+__global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(xt_args a) {
     constexpr bool K4 = WT == SPY_HIP_Q4_K;
+    static_assert(KS == 1 || OWN, "the host's order is one chain over K");
     constexpr int NT = 64 * RG, ROWS = 16 * RG, NXI = C * 256 / NT, C2 = (C + 1) / 2;
     constexpr int XB = C * XT_XB + C2 * 1024;
     constexpr int NXS = 2;                         // stage s is worked on, stage s + 1 is on its way
     static_assert(NXI * NT == C * 256 && RG >= C2, "one request per thread and group, one wave per two groups' records");
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, r = lane & 15;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem_all[];
+    const int tid = threadIdx.x, lane = tid & 63, wg_wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, r = lane & 15;
+    const int ks = KS > 1 ? wg_wave / RG : 0, wave = KS > 1 ? wg_wave % RG : wg_wave;
     const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS, cg0 = (int)blockIdx.y * C;
-    const int nst = a.nst, ncg = a.ncg, M = a.M;
+    const int ncg = a.ncg, M = a.M;
+    // the set's super-blocks: sb0 .. sb0 + nsb - 1; every set takes part in as many steps as the longest
+    const int all = a.nst / 2, per = (all + KS - 1) / KS, sb0 = min(ks * per, all - 1), nsb = KS > 1 ? max(min(per, all - ks * per), 0) : all;
+    const int nst = 2 * nsb, nstep = 2 * per;
+    uint8_t *smem = smem_all + ks * (NXS * XB);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
     // activation stages into the ring, as in xt_kernel; one request brings the records of two groups
     const uint8_t *bx[NXI], *bd;
 #pragma unroll
-    for (int i = 0; i < NXI; i++) bx[i] = a.xq + (int64_t)min(cg0 + (i * NT + wave * 64) / 256, ncg - 1) * nst * XT_XB + (i * NT + wave * 64) % 256 * 16;
+    for (int i = 0; i < NXI; i++) bx[i] = a.xq + ((int64_t)min(cg0 + (i * NT + wave * 64) / 256, ncg - 1) * a.nst + 2 * sb0) * XT_XB + (i * NT + wave * 64) % 256 * 16;
     const int dc0 = min(cg0 + 2 * min(wave, C2 - 1), ncg - 1), dc1 = min(dc0 + 1, ncg - 1);
-    bd = a.xd + (int64_t)dc0 * nst * XT_XD;
-    const uint32_t l16 = lane * 16, ld = (lane & 31) * 16 + (lane >> 5) * (uint32_t)((dc1 - dc0) * nst * XT_XD);
+    bd = a.xd + ((int64_t)dc0 * a.nst + 2 * sb0) * XT_XD;
+    const uint32_t l16 = lane * 16, ld = (lane & 31) * 16 + (lane >> 5) * (uint32_t)((dc1 - dc0) * a.nst * XT_XD);
     const uint32_t ldsx = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024), ldsd = __builtin_amdgcn_readfirstlane(lds0 + C * XT_XB + min(wave, C2 - 1) * 1024);
     int is = 0;
     auto issue_x = [&]() {
@@ -743,7 +750,7 @@ __global__ __launch_bounds__(64 * RG, OCC) void xk_kernel(xt_args a) {
         is++;
     };
     const uint8_t *wr = a.w[mat] + (int64_t)min(m0 + wave * 16 + r, M - 1) * a.w_row;
-    xk_raw<WT> cur = xk_load<WT>(wr, 0, q);
+    xk_raw<WT> cur = xk_load<WT>(wr, sb0, q);
     issue_x();
 
     float acc[C][4];                               // rows 4q .. 4q + 3 of the wave's 16, activation row r of the group
@@ -753,7 +760,7 @@ __global__ __launch_bounds__(64 * RG, OCC) void xk_kernel(xt_args a) {
         for (int v = 0; v < 4; v++) acc[c][v] = 0.0f;
     float A[OWN ? C : 1][4];
     xk_v4f Bm[OWN && K4 ? C : 1];
-    float *tab = (float *)(smem + NXS * XB) + wave * (K4 ? (OWN ? 288 : 256) : 16);      // the wave's scales: Q4_K [sub-block][d * sc, dmin * m][row], Q6_K [row] d
+    float *tab = (float *)(smem_all + KS * NXS * XB) + wg_wave * (K4 ? (OWN ? 288 : 256) : 16);      // the wave's scales: Q4_K [sub-block][d * sc, dmin * m][row], Q6_K [row] d
     const xk_v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
     auto compute = [&](int s, auto par_c) {
         constexpr int par = decltype(par_c)::value;
@@ -838,19 +845,41 @@ __global__ __launch_bounds__(64 * RG, OCC) void xk_kernel(xt_args a) {
         xt_wait_vm<0>();
         __builtin_amdgcn_s_barrier();
     };
-    for (int s = 0; s < nst; s += 2) {
+    for (int s = 0; s < nstep; s += 2) {
+        const bool on = KS == 1 || s < nst;
         ready();
         if constexpr (OWN && K4) xk_put_scales_own(cur, tab, q, r);
         else xk_put_scales<WT>(cur, tab, q, r);         // the compiler's own wait for the super-block stands here, where nothing is on its way
-        const xk_raw<WT> nxt = xk_load<WT>(wr, min(s / 2 + 1, nst / 2 - 1), q);
+        // the activations of the next stage ahead of the weights of the next super-block, which come from memory: requests are served in order, and the
+        // own order's stages are shorter than what the weights take (11008 x 4096 x 128 Q4_K 51.5 -> 47.2 us, 16000 x 6144 x 200 142 -> 130)
         issue_x();
-        compute(s, std::integral_constant<int, 0>{});
+        __builtin_amdgcn_sched_barrier(0);
+        const xk_raw<WT> nxt = xk_load<WT>(wr, sb0 + max(min(s / 2 + 1, nsb - 1), 0), q);
+        if (on) compute(s, std::integral_constant<int, 0>{});
         ready();
         issue_x();
-        compute(s + 1, std::integral_constant<int, 1>{});
+        if (on) compute(s + 1, std::integral_constant<int, 1>{});
         cur = nxt;
     }
     xt_wait_vm<0>();
+    if constexpr (KS > 1) {                         // the sets' sums, in order
+        __builtin_amdgcn_s_barrier();
+        float *ex = (float *)smem_all;
+        if (ks > 0) {
+#pragma unroll
+            for (int c = 0; c < C; c++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) ex[(((ks - 1) * RG + wave) * C * 4 + c * 4 + v) * 64 + lane] = acc[c][v];
+        }
+        __syncthreads();
+        if (ks > 0) return;
+#pragma unroll
+        for (int k = 0; k < KS - 1; k++)
+#pragma unroll
+            for (int c = 0; c < C; c++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[c][v] += ex[((k * RG + wave) * C * 4 + c * 4 + v) * 64 + lane];
+    }
     const int row = m0 + wave * 16 + 4 * q;
     float *dst = a.dst[mat];
 #pragma unroll
@@ -1117,12 +1146,13 @@ int xo_launch(hipStream_t st, xt_args a, int nmat) {
     xo_kernel<RW, WV, C, OCC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * WV), lds, st>>>(a);
     return SPY_LAUNCH_RC();
 }
-template <int WT, bool OWN, int RG, int C, int OCC>
+template <int WT, bool OWN, int RG, int C, int OCC, int KS = 1>
 int xk_launch(hipStream_t st, xt_args a, int nmat) {
-    constexpr size_t lds = 2 * (C * XT_XB + (C + 1) / 2 * 1024) + RG * (OWN ? 1152 : 1024);
-    if (lds > 64 * 1024) { const int rc = spy_raise_lds_limit((const void *)xk_kernel<WT, OWN, RG, C, OCC>, lds); if (rc) return rc; }
+    constexpr size_t lds = KS * (2 * (C * XT_XB + (C + 1) / 2 * 1024) + RG * (OWN ? 1152 : 1024));
+    static_assert(lds <= 160 * 1024 && lds >= (size_t)(KS - 1) * RG * C * 1024, "");
+    if (lds > 64 * 1024) { const int rc = spy_raise_lds_limit((const void *)xk_kernel<WT, OWN, RG, C, OCC, KS>, lds); if (rc) return rc; }
     a.tiles = (a.M + 16 * RG - 1) / (16 * RG);
-    xk_kernel<WT, OWN, RG, C, OCC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * RG), lds, st>>>(a);
+    xk_kernel<WT, OWN, RG, C, OCC, KS><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * RG * KS), lds, st>>>(a);
     return SPY_LAUNCH_RC();
 }
 template <int WT>
@@ -1174,21 +1204,39 @@ int xk_dispatch(hipStream_t st, const xt_args &a, int nmat) {
     }
 }
 
-// the own order of the K-quants; as in xt_dispatch.  xks_kernel adds the terms in another order than the tiles: the choice is that of the whole call, so that
-// a call in pieces has its bits
+// the own order of the K-quants.  xks_kernel and the tiles that split K add the terms in other orders than the rest: the choice is that of the whole call, so
+// that a call in pieces has its bits
 template <int WT>
 int xko_dispatch(hipStream_t st, const xt_args &a, int nmat) {
-    xt_args all = a;
-    all.ncg = a.ncg_all;
-    static const xt_cost k4[6] = {{16, 1, 94, 43}, {32, 2, 235, 74}, {64, 2, 250, 128}, {32, 4, 330, 128}, {64, 4, 355, 185}, {64, 8, 560, 355}},
-                         k6[6] = {{16, 1, 110, 56}, {32, 2, 230, 110}, {64, 2, 310, 196}, {32, 4, 315, 161}, {64, 4, 390, 254}, {64, 8, 560, 396}};
-    switch (xt_pick(all, nmat, WT == SPY_HIP_Q4_K ? k4 : k6, 6)) {
+    // Times in tenths of a microsecond at K = 4096 with 1, 2, 3, 4 and 6 workgroups per compute unit, weights from memory.  The last three split K: where a matrix
+    // gives a compute unit one workgroup, the chain of its super-blocks is what it takes (8192 x 4096 x 64: Q4_K 35.6 -> 23.8 us, Q6_K 39.8 -> 28.0;
+    // 8192 x 11008 x 100: 104 -> 73 and 126 -> 108); with two and more the tiles without a split are faster.
+    struct tile { int rows, groups, t[5]; };
+    static const tile k4[9] = {{16, 1, {98, 122, 171, 220, 298}}, {32, 2, {263, 288, 325, 375, 530}}, {64, 2, {323, 365, 422, 586, 832}}, {32, 4, {324, 418, 463, 523, 966}},
+                               {64, 4, {379, 460, 624, 853, 1171}}, {64, 8, {521, 737, 1131, 1395, 2048}},
+                               {32, 2, {150, 279, 411, 542, 806}}, {32, 4, {199, 379, 559, 734, 1087}}, {64, 4, {305, 572, 838, 1107, 1637}}},
+                      k6[9] = {{16, 1, {113, 160, 206, 269, 364}}, {32, 2, {274, 332, 417, 509, 748}}, {64, 2, {366, 504, 692, 886, 1274}}, {32, 4, {324, 483, 561, 657, 1154}},
+                               {64, 4, {421, 625, 827, 1085, 1560}}, {64, 8, {591, 850, 1291, 1616, 2381}},
+                               {32, 2, {194, 369, 545, 720, 1067}}, {32, 4, {240, 458, 673, 887, 1312}}, {64, 4, {392, 751, 1116, 1475, 2187}}};
+    const int64_t cu = spy_num_cu();
+    int best = 0;
+    int64_t least = 0;
+    for (int i = 0; i < 9; i++) {
+        const tile &c = WT == SPY_HIP_Q4_K ? k4[i] : k6[i];
+        const int64_t wgs = (int64_t)((a.M + c.rows - 1) / c.rows) * nmat * ((a.ncg_all + c.groups - 1) / c.groups), n = (wgs + cu - 1) / cu;
+        const int64_t t = n <= 4 ? c.t[n - 1] : n == 5 ? (c.t[3] + c.t[4]) / 2 : c.t[4] * wgs / (6 * cu);
+        if (!i || t < least) { best = i; least = t; }
+    }
+    switch (best) {
     case 0: return xks_launch<WT>(st, a, nmat);
     case 1: return xk_launch<WT, true, 2, 2, 4>(st, a, nmat);
     case 2: return xk_launch<WT, true, 4, 2, 4>(st, a, nmat);
     case 3: return xk_launch<WT, true, 2, 4, 3>(st, a, nmat);
     case 4: return xk_launch<WT, true, 4, 4, 4>(st, a, nmat);
-    default: return xk_launch<WT, true, 4, 8, 2>(st, a, nmat);
+    case 5: return xk_launch<WT, true, 4, 8, 2>(st, a, nmat);
+    case 6: return xk_launch<WT, true, 2, 2, 2, 4>(st, a, nmat);
+    case 7: return xk_launch<WT, true, 2, 4, 2, 4>(st, a, nmat);
+    default: return xk_launch<WT, true, 4, 4, 2, 2>(st, a, nmat);
     }
 }
 

@@ -183,6 +183,14 @@ def test_matmul_operator_takes_the_packed_activation_kernels(hip, oracle, wtype,
         L.spy_hip_set_exact_order(prev)
 
 
+@pytest.mark.parametrize("wtype", [O.Q4_K, O.Q6_K])
+@pytest.mark.parametrize("M,K,T", [(4096, 256, 17), (8188, 768, 32), (8192, 1280, 50), (4100, 2816, 64), (11000, 512, 40), (11008, 4352, 48)])
+def test_matmul_operator_splits_k(hip, oracle, wtype, M, K, T, monkeypatch):
+    """The tiles of the own order whose sets of waves share K, one workgroup per compute unit: fewer super-blocks than sets (256, 768), numbers of
+    them that do not divide, partial tiles."""
+    test_matmul_operator_takes_the_packed_activation_kernels(hip, oracle, wtype, M, K, T, monkeypatch)
+
+
 @pytest.mark.parametrize("n_prompt", [129, 400])
 def test_own_order_prompt_from_packed_activations(hip, n_prompt, monkeypatch):
     """One layer of the 7B shape in this backend's own order: norm, activation and residual steps around the packed-activation MatMuls (from 129 tokens

@@ -592,16 +592,21 @@ int xt_launch_mixed(hipStream_t st, xt_args a, int nmat) {
 // ---- Q4_K / Q6_K ------------------------------------------------------------------------------------------------------------------------
 // These dots keep ONE accumulator per output and add one term per sub-block of 32 elements (the order this project defines; exact_order.hip):
 //   Q4_K:  acc = fma(d_x, d * float(sc * isum) - dmin * float(m * bsum), acc)       Q6_K:  acc = fma(d_x * d, float(sc0 * isum0 + sc1 * isum1), acc)
-// so the integer sums of a whole sub-block come from v_mfma_f32_16x16x32_f16 -- lane (q, r): elements 8q .. 8q + 7 of row r -- and the vector units
-// have 16 (Q4_K) or 8 (Q6_K) instructions per 16 x 16 tile and sub-block where the tile kernel of exact_order.hip had 64 and 56:
+// so the integer sums of a whole sub-block come from v_mfma_f32_16x16x32_f16 -- lane (q, r): elements 8q .. 8q + 7 of row r -- and the outer products of a
+// term (Q4_K dmin * m by bsum, Q6_K d by d_x) for two sub-blocks and two groups of activation rows from one instruction of four blocks (v_mfma_f32_16x16x1_4b_f32,
+// whose single product rounds once as the multiplication does, and v_mfma_f32_16x16x4_4b_f16, exact).  Left for the vector units are 12 (Q4_K) or 4 (Q6_K)
+// instructions per 16 x 16 tile and sub-block where the tile kernel of exact_order.hip had 64 and 56:
 //   * small integers are fp16 subnormals as they are (the bit pattern n is n * 2^-24): unpacking a pair of nibbles is one AND.  The factor
 //     2^24 goes into the weights' scale; every product and sum below is still exact.
 //   * d * sc, dmin * m and d_w * d_x have at most 22 significant bits: they are exact in fp32, so (d * sc) * isum rounds once, as d * (sc * isum) does.
 //   * Q6_K: q - 32 = l + 16 (h - 2) with the low four and the high two bits, and sc * l, 16 * sc * (h - 2) are exact in fp16: the scales of the
 //     two halves of a sub-block ride on the operands, and two matrix instructions leave sc0 * isum0 + sc1 * isum1 (below 2^24).
-// A wave takes 16 weight rows, which it reads straight into registers one super-block ahead, and C groups of 16 activation rows.
-// 4096 x 4096 x 2048, quantization and packing included: Q4_K 374 -> 162 us, Q6_K 346 -> 169; 77 rows 89 -> 28 and 89 -> 37.  The vector units bound both:
-// 592 (Q4_K: 512 of them the terms) and 484 (Q6_K) instructions per super-block of 16 rows x 4 groups, 4 cycles each.
+//   * Q6_K: the 2^24 stays out until the end: accumulators are multiples of 2^-72, so no sum below it is rounded otherwise.
+// A wave takes 16 weight rows, which it reads straight into registers half a super-block ahead, and C groups of 16 activation rows.
+// 4096 x 4096 x 2048, quantization and packing included: Q4_K 374 -> 150 us, Q6_K 346 -> 146; 77 rows 89 -> 28 and 89 -> 35.  Vector and matrix cycles bound both and
+// hardly overlap: per super-block of 16 rows x 8 groups 845 vector instructions (768 of them the terms) of 4 cycles beside 1536 matrix cycles (Q4_K), 440 beside 2560 (Q6_K).
+// The outer products on the matrix units and the halves of a super-block in turn (no second copy of it in registers) against 16 and 8 vector instructions
+// per tile and sub-block: 22016 x 4096 x 2048 Q4_K 767 -> 730 us, 4096 x 11008 x 2048 Q6_K 445 -> 394, 300 rows 197 -> 156.
 typedef _Float16 xk_h8 __attribute__((ext_vector_type(8)));
 typedef float xk_v4f __attribute__((ext_vector_type(4)));
 
@@ -640,6 +645,35 @@ __device__ __forceinline__ xk_raw<WT> xk_load(const uint8_t *row, int sb, int q)
         t.d = *(const uint16_t *)(p + 208);
     }
     return t;
+}
+// half H of a super-block, what stage H of its two takes, and of the first half the scales
+template <int H> __device__ __forceinline__ void xk_load_half(xk_raw<SPY_HIP_Q4_K> &t, const uint8_t *row, int sb, int q) {
+    const uint8_t *p = row + (int64_t)sb * 144;
+    if constexpr (H == 0) t.head = *(const uint4 *)p;
+#pragma unroll
+    for (int k = 2 * H; k < 2 * H + 2; k++) t.qs[k] = *(const uint2 *)(p + 16 + 32 * k + 8 * q);
+}
+template <int H> __device__ __forceinline__ void xk_load_half(xk_raw<SPY_HIP_Q6_K> &t, const uint8_t *row, int sb, int q) {
+    const uint8_t *p = row + (int64_t)sb * 210;
+#pragma unroll
+    for (int k = 2 * H; k < 2 * H + 2; k++) t.ql[k] = __builtin_bit_cast(uint2, *(const xk_u2 *)(p + 32 * k + 8 * q));
+    t.qh[H] = __builtin_bit_cast(uint2, *(const xk_u2 *)(p + 128 + 32 * H + 8 * q));
+    const uint2 sc = __builtin_bit_cast(uint2, *(const xk_u2 *)(p + 192 + 8 * H));
+    if constexpr (H == 0) { t.sc.x = sc.x; t.sc.y = sc.y; t.d = *(const uint16_t *)(p + 208); }
+    else { t.sc.z = sc.x; t.sc.w = sc.y; }
+}
+// the compiler's wait for half H stands where this does
+template <int H, int WT> __device__ __forceinline__ void xk_arrived(xk_raw<WT> &t) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (WT == SPY_HIP_Q4_K) {
+        asm volatile("" : "+v"(t.qs[2 * H].x), "+v"(t.qs[2 * H].y), "+v"(t.qs[2 * H + 1].x), "+v"(t.qs[2 * H + 1].y));
+        if constexpr (H == 0) asm volatile("" : "+v"(t.head.x), "+v"(t.head.y), "+v"(t.head.z), "+v"(t.head.w));
+    } else {
+        asm volatile("" : "+v"(t.ql[2 * H].x), "+v"(t.ql[2 * H].y), "+v"(t.ql[2 * H + 1].x), "+v"(t.ql[2 * H + 1].y), "+v"(t.qh[H].x), "+v"(t.qh[H].y));
+        if constexpr (H == 0) asm volatile("" : "+v"(t.sc.x), "+v"(t.sc.y), "+v"(t.d));
+        else asm volatile("" : "+v"(t.sc.z), "+v"(t.sc.w));
+    }
+#endif
 }
 __device__ __forceinline__ float xk_half(uint32_t h) { return h == 0xFFFFu ? 0.0f : h2f((uint16_t)h); }      // conversion.h:39-41
 // The scales of a super-block into the wave's table: lane (q, r) prepares those of row r, sub-blocks 2q and 2q + 1.
@@ -710,7 +744,7 @@ __device__ __forceinline__ void xk_unpack(const xk_raw<WT> &w, int q, uint4 (&o)
 // OWN: this backend's own order.  The terms of a super-block are added before its d and dmin are applied:
 //   acc = acc + d * (sum d_x * (sc * isum)) - dmin * (sum m * (d_x * bsum))
 // with sc on the weights' operand and the second sum, a contraction over sub-blocks, on v_mfma_f32_16x16x4_f32: 5 vector instructions per tile and
-// sub-block instead of 17 (Q4_K) and 9 (Q6_K).  4096 x 4096 x 1000, packing included: Q4_K 105 -> 87 us, Q6_K 112 -> 97; 22016 x 4096 x 1000: 557 -> 401
+// sub-block instead of 17 (Q4_K) and 9 (Q6_K) before the outer products of the host's order went to the matrix units.  4096 x 4096 x 1000, packing included: Q4_K 105 -> 87 us, Q6_K 112 -> 97; 22016 x 4096 x 1000: 557 -> 355
 // and 588 -> 449 (the 128 x 128 tiles of gemm.hip: 424 and 755).
 // KS (own order): that many sets of RG waves, each with its share of the super-blocks and activation stages of its own; their sums meet at the end.
 template <int WT, bool OWN, int RG, int C, int OCC, int KS = 1>
@@ -750,8 +784,10 @@ __global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(xt_args a) {
         is++;
     };
     const uint8_t *wr = a.w[mat] + (int64_t)min(m0 + wave * 16 + r, M - 1) * a.w_row;
-    xk_raw<WT> cur = xk_load<WT>(wr, sb0, q);
+    xk_raw<WT> cur;
+    xk_load_half<0>(cur, wr, sb0, q);
     issue_x();
+    uint32_t dd = 0;                               // Q6_K in the host's order: the row's d
 
     float acc[C][4];                               // rows 4q .. 4q + 3 of the wave's 16, activation row r of the group
 #pragma unroll
@@ -762,31 +798,26 @@ __global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(xt_args a) {
     xk_v4f Bm[OWN && K4 ? C : 1];
     float *tab = (float *)(smem_all + KS * NXS * XB) + wg_wave * (K4 ? (OWN ? 288 : 256) : 16);      // the wave's scales: Q4_K [sub-block][d * sc, dmin * m][row], Q6_K [row] d
     const xk_v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    auto compute = [&](int s, auto par_c) {
+    auto compute_own = [&](int s, auto par_c) {
         constexpr int par = decltype(par_c)::value;
         const uint8_t *sx = smem + (s & (NXS - 1)) * XB + q * 256 + r * 16, *sd = smem + (s & (NXS - 1)) * XB + C * XT_XB + r * 4;
         // steps (sub-block, activation group): operands of step j + 2 read and the matrix instruction of step j + 1 issued before the vector work of step j
         constexpr int NJ = 4 * C;
         uint4 w[2][K4 ? 1 : 2], xv[3];
         uint32_t dx[3];
-        float bs[3];
-        xk_v4f p[2], dsc[2], dm[2];
+        xk_v4f p[2];
         auto rd = [&](int j) {
             const int b = j / C, c = j % C;
             xv[j % 3] = *(const uint4 *)(sx + c * XT_XB + b * 1024);
             dx[j % 3] = *(const uint32_t *)(sd + c * XT_XD + b * 64);
-            if constexpr (K4 && !OWN) bs[j % 3] = *(const float *)(sd + c * XT_XD + 256 + b * 64);
         };
         auto weights = [&](auto b_c) {
             constexpr int b = decltype(b_c)::value;
             xk_unpack<WT, 4 * par + b>(cur, q, w[b & 1]);
-            if constexpr (K4 && OWN) {
+            if constexpr (K4) {
                 const uint32_t sc = ((const uint32_t *)tab)[(4 * par + b) * 16 + r];
                 uint4 &o = w[b & 1][0];
                 o = make_uint4(xk_pk_mul(o.x, sc), xk_pk_mul(o.y, sc), xk_pk_mul(o.z, sc), xk_pk_mul(o.w, sc));
-            } else if constexpr (K4) {
-                dsc[b & 1] = *(const xk_v4f *)(tab + (4 * par + b) * 32 + 4 * q);
-                dm[b & 1] = *(const xk_v4f *)(tab + (4 * par + b) * 32 + 16 + 4 * q);
             }
         };
         auto mm = [&](int j) {
@@ -794,7 +825,6 @@ __global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(xt_args a) {
             p[j & 1] = xk_mfma(w[b & 1][0], xv[j % 3], zero);
             if constexpr (!K4) p[j & 1] = xk_mfma(w[b & 1][1], xv[j % 3], p[j & 1]);
         };
-        if constexpr (!K4 && !OWN) dsc[0] = *(const xk_v4f *)(tab + 4 * q);
         rd(0);
         rd(1);
         weights(std::integral_constant<int, 0>{});
@@ -809,17 +839,11 @@ __global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(xt_args a) {
             __builtin_amdgcn_sched_barrier(0);
             const float x = h2f((uint16_t)dx[j % 3]);
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                if constexpr (OWN) A[c][v] = par == 0 && b == 0 ? x * p[j & 1][v] : fmaf(x, p[j & 1][v], A[c][v]);
-                else if constexpr (K4) {
-                    const float pos = dsc[b & 1][v] * p[j & 1][v], neg = dm[b & 1][v] * bs[j % 3];
-                    acc[c][v] = fmaf(x, pos - neg, acc[c][v]);
-                } else acc[c][v] = fmaf(x * dsc[0][v], p[j & 1][v], acc[c][v]);
-            }
+            for (int v = 0; v < 4; v++) A[c][v] = par == 0 && b == 0 ? x * p[j & 1][v] : fmaf(x, p[j & 1][v], A[c][v]);
             __builtin_amdgcn_sched_barrier(0);
         };
         [&]<int... J>(std::integer_sequence<int, J...>) { (step(std::integral_constant<int, J>{}), ...); }(std::make_integer_sequence<int, NJ>{});
-        if constexpr (OWN && K4) {                 // lane (q, r): sub-block q of the stage, row r of either side
+        if constexpr (K4) {                        // lane (q, r): sub-block q of the stage, row r of either side
             const float m = tab[128 + (4 * par + q) * 16 + r];
             const uint8_t *sq = sd + q * 64;
 #pragma unroll
@@ -828,7 +852,7 @@ __global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(xt_args a) {
                 Bm[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(m, xb, par == 0 ? zero : Bm[c], 0, 0, 0);
             }
         }
-        if constexpr (OWN && par == 1) {
+        if constexpr (par == 1) {
             const xk_v4f d = *(const xk_v4f *)(tab + (K4 ? 256 : 0) + 4 * q);
             xk_v4f dmin = zero;
             if constexpr (K4) dmin = *(const xk_v4f *)(tab + 272 + 4 * q);
@@ -841,6 +865,79 @@ __global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(xt_args a) {
                 }
         }
     };
+    auto compute_host = [&](int s, auto par_c) {
+        constexpr int par = decltype(par_c)::value;
+        const uint8_t *sx = smem + (s & (NXS - 1)) * XB + q * 256 + r * 16, *sd = smem + (s & (NXS - 1)) * XB + C * XT_XB + r * 4;
+        const uint8_t *so = sd + (q >> 1) * XT_XD + (q & 1) * 64;
+        // steps of four: sub-blocks 2h and 2h + 1 by activation groups 2g and 2g + 1, whose outer products come from one instruction of four blocks
+        constexpr int NJ = 4 * C;
+        static_assert(OWN || C % 2 == 0, "groups in pairs");
+        uint4 w[2][K4 ? 1 : 2], xv[3];
+        uint32_t dx[3];
+        xk_v4f p[2], dsc[2];
+        xt_v16f D;
+        auto rd = [&](int j) {
+            const int b = j / (2 * C) * 2 + (j & 1), c = j % (2 * C) / 4 * 2 + (j >> 1 & 1);
+            xv[j % 3] = *(const uint4 *)(sx + c * XT_XB + b * 1024);
+            if constexpr (K4) dx[j % 3] = *(const uint32_t *)(sd + c * XT_XD + b * 64);
+        };
+        float dm = 0.0f, bs = 0.0f;
+        uint32_t dxo = 0;
+        auto rd_outer = [&](int j) {               // lane (q, r): sub-block 2h + q % 2, group 2g + q / 2
+            const int h = j / (2 * C), g = j % (2 * C) / 4;
+            if constexpr (K4) bs = *(const float *)(so + 256 + 2 * g * XT_XD + h * 128);
+            else dxo = *(const uint32_t *)(so + 2 * g * XT_XD + h * 128);
+        };
+        auto outer = [&]() {
+            if constexpr (K4) D = __builtin_amdgcn_mfma_f32_16x16x1f32(dm, bs, xt_v16f{}, 0, 0, 0);
+            else D = xt_mfma(dd, 0u, dxo, 0u);
+        };
+        auto weights = [&](auto h_c) {
+            constexpr int h = decltype(h_c)::value;
+            xk_unpack<WT, 4 * par + 2 * h>(cur, q, w[0]);
+            xk_unpack<WT, 4 * par + 2 * h + 1>(cur, q, w[1]);
+            if constexpr (K4) {
+                dsc[0] = *(const xk_v4f *)(tab + (4 * par + 2 * h) * 32 + 4 * q);
+                dsc[1] = *(const xk_v4f *)(tab + (4 * par + 2 * h + 1) * 32 + 4 * q);
+                dm = tab[(4 * par + 2 * h + (q & 1)) * 32 + 16 + r];
+            }
+        };
+        auto mm = [&](int j) {
+            p[j & 1] = xk_mfma(w[j & 1][0], xv[j % 3], zero);
+            if constexpr (!K4) p[j & 1] = xk_mfma(w[j & 1][1], xv[j % 3], p[j & 1]);
+        };
+        rd(0);
+        rd_outer(0);
+        rd(1);
+        weights(std::integral_constant<int, 0>{});
+        mm(0);
+        outer();
+        auto step = [&](auto j_c) {
+            constexpr int j = decltype(j_c)::value, c = j % (2 * C) / 4 * 2 + (j >> 1 & 1);
+            const xk_v4f ds = dsc[j & 1];
+            if constexpr (j + 2 < NJ) rd(j + 2);
+            if constexpr ((j & 3) == 1 && j + 3 < NJ) rd_outer(j + 3);
+            if constexpr (j + 1 < NJ) {
+                if constexpr ((j + 1) % (2 * C) == 0) weights(std::integral_constant<int, (j + 1) / (2 * C)>{});
+                mm(j + 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            float x = 0.0f;
+            if constexpr (K4) x = h2f((uint16_t)dx[j % 3]);
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                if constexpr (K4) acc[c][v] = fmaf(x, ds[v] * p[j & 1][v] - D[4 * (j & 3) + v], acc[c][v]);
+                else acc[c][v] = fmaf(D[4 * (j & 3) + v], p[j & 1][v], acc[c][v]);
+            }
+            if constexpr ((j & 3) == 3 && j + 1 < NJ) outer();
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        [&]<int... J>(std::integer_sequence<int, J...>) { (step(std::integral_constant<int, J>{}), ...); }(std::make_integer_sequence<int, NJ>{});
+    };
+    auto compute = [&](int s, auto par_c) {
+        if constexpr (OWN) compute_own(s, par_c);
+        else compute_host(s, par_c);
+    };
     auto ready = [&]() {
         xt_wait_vm<0>();
         __builtin_amdgcn_s_barrier();
@@ -848,18 +945,23 @@ __global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(xt_args a) {
     for (int s = 0; s < nstep; s += 2) {
         const bool on = KS == 1 || s < nst;
         ready();
+        xk_arrived<0>(cur);                        // where nothing is on its way
         if constexpr (OWN && K4) xk_put_scales_own(cur, tab, q, r);
-        else xk_put_scales<WT>(cur, tab, q, r);         // the compiler's own wait for the super-block stands here, where nothing is on its way
-        // the activations of the next stage ahead of the weights of the next super-block, which come from memory: requests are served in order, and the
-        // own order's stages are shorter than what the weights take (11008 x 4096 x 128 Q4_K 51.5 -> 47.2 us, 16000 x 6144 x 200 142 -> 130)
+        else if constexpr (OWN || K4) xk_put_scales<WT>(cur, tab, q, r);
+        else dd = cur.d == 0xFFFFu ? 0u : cur.d;
+        // the activations of the next stage ahead of the weights, which come from memory: requests are served in order, and the
+        // own order's stages are shorter than what the weights take (11008 x 4096 x 128 Q4_K 51.5 -> 47.2 us, 16000 x 6144 x 200 142 -> 130).
+        // A half of a super-block is requested a stage ahead, into the registers of the one that has been unpacked.
         issue_x();
         __builtin_amdgcn_sched_barrier(0);
-        const xk_raw<WT> nxt = xk_load<WT>(wr, sb0 + max(min(s / 2 + 1, nsb - 1), 0), q);
+        xk_load_half<1>(cur, wr, sb0 + max(min(s / 2, nsb - 1), 0), q);
         if (on) compute(s, std::integral_constant<int, 0>{});
         ready();
+        xk_arrived<1>(cur);
         issue_x();
+        __builtin_amdgcn_sched_barrier(0);
+        xk_load_half<0>(cur, wr, sb0 + max(min(s / 2 + 1, nsb - 1), 0), q);
         if (on) compute(s + 1, std::integral_constant<int, 1>{});
-        cur = nxt;
     }
     xt_wait_vm<0>();
     if constexpr (KS > 1) {                         // the sets' sums, in order
@@ -879,6 +981,12 @@ __global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(xt_args a) {
             for (int c = 0; c < C; c++)
 #pragma unroll
                 for (int v = 0; v < 4; v++) acc[c][v] += ex[((k * RG + wave) * C * 4 + c * 4 + v) * 64 + lane];
+    }
+    if constexpr (!OWN && !K4) {                    // their operands were small integers times 2^-24
+#pragma unroll
+        for (int c = 0; c < C; c++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) acc[c][v] *= 16777216.0f;
     }
     const int row = m0 + wave * 16 + 4 * q;
     float *dst = a.dst[mat];
@@ -1192,14 +1300,28 @@ int xt_dispatch(hipStream_t st, const xt_args &a, int nmat) {
     default: return rest == 1 ? xt_launch_mixed<WT, 1>(st, a, nmat) : rest == 2 ? xt_launch_mixed<WT, 2>(st, a, nmat) : xt_launch_mixed<WT, 3>(st, a, nmat);
     }
 }
+// Tiles of the K-quants: times in tenths of a microsecond at K = 4096 with 1, 2, 3, 4 and 6 workgroups per compute unit, weights from memory
+struct xk_tile { int rows, groups, t[5]; };
+int xk_pick(const xt_args &a, int nmat, int ncg, const xk_tile *c, int n_tiles) {
+    const int64_t cu = spy_num_cu();
+    int best = 0;
+    int64_t least = 0;
+    for (int i = 0; i < n_tiles; i++) {
+        const int64_t wgs = (int64_t)((a.M + c[i].rows - 1) / c[i].rows) * nmat * ((ncg + c[i].groups - 1) / c[i].groups), n = (wgs + cu - 1) / cu;
+        const int64_t t = n <= 4 ? c[i].t[n - 1] : n == 5 ? (c[i].t[3] + c[i].t[4]) / 2 : c[i].t[4] * wgs / (6 * cu);
+        if (!i || t < least) { best = i; least = t; }
+    }
+    return best;
+}
 template <int WT>
 int xk_dispatch(hipStream_t st, const xt_args &a, int nmat) {
-    static const xt_cost k4[4] = {{16, 1, 94, 43}, {64, 2, 230, 132}, {64, 4, 360, 205}, {128, 8, 900, 660}},
-                         k6[4] = {{16, 1, 110, 56}, {64, 2, 330, 210}, {64, 4, 440, 260}, {128, 8, 940, 690}};
-    switch (xt_pick(a, nmat, WT == SPY_HIP_Q4_K ? k4 : k6, 4)) {
+    static const xk_tile k4[5] = {{16, 1, {99, 123, 171, 220, 297}}, {32, 2, {226, 264, 278, 319, 517}}, {64, 2, {273, 302, 407, 557, 899}}, {64, 4, {338, 467, 643, 815, 1176}}, {128, 8, {830, 1414, 2069, 2736, 4053}}},
+                         k6[5] = {{16, 1, {113, 160, 207, 269, 364}}, {32, 2, {240, 267, 354, 460, 702}}, {64, 2, {305, 455, 635, 832, 1210}}, {64, 4, {357, 526, 756, 987, 1443}}, {128, 8, {827, 1403, 2101, 2768, 4116}}};
+    switch (xk_pick(a, nmat, a.ncg, WT == SPY_HIP_Q4_K ? k4 : k6, 5)) {
     case 0: return xks_launch<WT>(st, a, nmat);
-    case 1: return xk_launch<WT, false, 4, 2, 4>(st, a, nmat);
-    case 2: return xk_launch<WT, false, 4, 4, 4>(st, a, nmat);
+    case 1: return xk_launch<WT, false, 2, 2, 4>(st, a, nmat);
+    case 2: return xk_launch<WT, false, 4, 2, 4>(st, a, nmat);
+    case 3: return xk_launch<WT, false, 4, 4, 4>(st, a, nmat);
     default: return xk_launch<WT, false, 8, 8, 4>(st, a, nmat);
     }
 }
@@ -1208,26 +1330,11 @@ int xk_dispatch(hipStream_t st, const xt_args &a, int nmat) {
 // that a call in pieces has its bits
 template <int WT>
 int xko_dispatch(hipStream_t st, const xt_args &a, int nmat) {
-    // Times in tenths of a microsecond at K = 4096 with 1, 2, 3, 4 and 6 workgroups per compute unit, weights from memory.  The last three split K: where a matrix
-    // gives a compute unit one workgroup, the chain of its super-blocks is what it takes (8192 x 4096 x 64: Q4_K 35.6 -> 23.8 us, Q6_K 39.8 -> 28.0;
-    // 8192 x 11008 x 100: 104 -> 73 and 126 -> 108); with two and more the tiles without a split are faster.
-    struct tile { int rows, groups, t[5]; };
-    static const tile k4[9] = {{16, 1, {98, 122, 171, 220, 298}}, {32, 2, {263, 288, 325, 375, 530}}, {64, 2, {323, 365, 422, 586, 832}}, {32, 4, {324, 418, 463, 523, 966}},
-                               {64, 4, {379, 460, 624, 853, 1171}}, {64, 8, {521, 737, 1131, 1395, 2048}},
-                               {32, 2, {150, 279, 411, 542, 806}}, {32, 4, {199, 379, 559, 734, 1087}}, {64, 4, {305, 572, 838, 1107, 1637}}},
-                      k6[9] = {{16, 1, {113, 160, 206, 269, 364}}, {32, 2, {274, 332, 417, 509, 748}}, {64, 2, {366, 504, 692, 886, 1274}}, {32, 4, {324, 483, 561, 657, 1154}},
-                               {64, 4, {421, 625, 827, 1085, 1560}}, {64, 8, {591, 850, 1291, 1616, 2381}},
-                               {32, 2, {194, 369, 545, 720, 1067}}, {32, 4, {240, 458, 673, 887, 1312}}, {64, 4, {392, 751, 1116, 1475, 2187}}};
-    const int64_t cu = spy_num_cu();
-    int best = 0;
-    int64_t least = 0;
-    for (int i = 0; i < 9; i++) {
-        const tile &c = WT == SPY_HIP_Q4_K ? k4[i] : k6[i];
-        const int64_t wgs = (int64_t)((a.M + c.rows - 1) / c.rows) * nmat * ((a.ncg_all + c.groups - 1) / c.groups), n = (wgs + cu - 1) / cu;
-        const int64_t t = n <= 4 ? c.t[n - 1] : n == 5 ? (c.t[3] + c.t[4]) / 2 : c.t[4] * wgs / (6 * cu);
-        if (!i || t < least) { best = i; least = t; }
-    }
-    switch (best) {
+    // The last three split K: where a matrix gives a compute unit one workgroup, the chain of its super-blocks is what it takes (8192 x 4096 x 64: Q4_K
+    // 35.6 -> 22.6 us, Q6_K 39.8 -> 25.2; 8192 x 11008 x 100: 104 -> 69 and 126 -> 92); with two and more the tiles without a split are faster.
+    static const xk_tile k4[9] = {{16, 1, {99, 123, 171, 219, 298}}, {32, 2, {246, 271, 286, 323, 513}}, {64, 2, {287, 320, 405, 556, 802}}, {32, 4, {303, 382, 421, 482, 902}}, {64, 4, {331, 420, 569, 770, 1071}}, {64, 8, {497, 706, 1082, 1333, 1960}}, {32, 2, {148, 259, 380, 499, 736}}, {32, 4, {186, 340, 498, 654, 964}}, {64, 4, {278, 516, 754, 995, 1466}}},
+                         k6[9] = {{16, 1, {113, 160, 206, 269, 364}}, {32, 2, {247, 286, 369, 468, 703}}, {64, 2, {316, 468, 643, 841, 1223}}, {32, 4, {295, 408, 480, 586, 1052}}, {64, 4, {354, 532, 762, 1001, 1447}}, {64, 8, {524, 764, 1159, 1473, 2173}}, {32, 2, {174, 317, 462, 606, 892}}, {32, 4, {211, 394, 579, 758, 1122}}, {64, 4, {344, 639, 930, 1230, 1814}}};
+    switch (xk_pick(a, nmat, a.ncg_all, WT == SPY_HIP_Q4_K ? k4 : k6, 9)) {
     case 0: return xks_launch<WT>(st, a, nmat);
     case 1: return xk_launch<WT, true, 2, 2, 4>(st, a, nmat);
     case 2: return xk_launch<WT, true, 4, 2, 4>(st, a, nmat);

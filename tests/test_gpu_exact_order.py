@@ -128,6 +128,30 @@ def test_narrow_matmul_bits(hip, oracle, wtype, M, K, T):
     test_packed_activation_matmul_bits(hip, oracle, wtype, M, K, T)
 
 
+@pytest.mark.parametrize("wtype", [O.Q4_K, O.Q6_K])
+@pytest.mark.parametrize("M,K,T", [(11000, 256, 40), (8192, 768, 70), (4100, 512, 150), (4096, 1280, 300)])
+def test_k_quant_tiles_with_scales_of_any_size(hip, oracle, wtype, M, K, T):
+    """The tiles of several groups from packed activations, whose outer products and scaled operands come from matrix instructions: block scales down to fp16's subnormals
+    and up to its largest numbers, any quants, activation rows whose scales are as small and as large.  The oracle's bits."""
+    from tests.gpu_util import dev, dev_empty, call
+    rng = np.random.default_rng(11 * wtype + M + K + T)
+    size, at = (144, (0, 2)) if wtype == O.Q4_K else (210, (208,))
+    w = rng.integers(0, 256, (M * K // 256, size), dtype=np.uint8)
+    for o in at:
+        d = np.ldexp(rng.uniform(0.5, 1.0, len(w)), rng.integers(-24, 16, len(w))).astype(np.float16)
+        d[rng.random(len(w)) < 0.05] = 0.0
+        w[:, o:o + 2] = (d * rng.choice([-1, 1], len(w)).astype(np.float16)).view(np.uint8).reshape(-1, 2)
+    w = w.reshape(-1)
+    x = (rng.standard_normal((T, K)) * np.ldexp(1.0, rng.integers(-16, 16, (T, 1)))).astype(np.float32)
+    want = O.matmul(oracle, w, wtype, M, K, x, nthread=8)
+    dw, dx, dd = dev(w), dev(x), dev_empty(T * M * 4, 0xFF)
+    tw, tx, td = hip.tensor(dw, wtype, [K, M]), hip.tensor(dx, hip.F32, [K, T]), hip.tensor(dd, hip.F32, [M, T])
+    need = hip.load().spy_hip_op_matmul_scratch_size(B(tw), B(tx))
+    scratch = dev_empty(need, 0xEE)
+    call(hip.load().spy_hip_op_matmul, None, B(tw), B(tx), B(td), scratch.ptr, need)
+    _same_bits(dd.download(np.float32).reshape(T, M), want, "matmul type %d %dx%d T %d, scales of any size" % (wtype, M, K, T))
+
+
 @pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0, O.Q4_K, O.Q6_K])
 @pytest.mark.parametrize("M,K,T", [(96, 4096, 16), (200, 512, 70), (64, 128, 64), (64, 256, 64), (132, 11008, 33), (4096, 4096, 130)])
 def test_tiled_matmul_bits(hip, oracle, wtype, M, K, T, monkeypatch):

@@ -1087,34 +1087,45 @@ __global__ __launch_bounds__(256, 3) void xks_kernel(xt_args a) {
 // (the arithmetic and the bits of gemm_q8act_kernel in gemm.hip).  The block dot of a 16 x 16 tile is one v_mfma_f32_16x16x32_f16, a float and exact,
 // and the scale products of four blocks are one 16x16x4_4b as above: 24 matrix-core cycles and four fmas (16 cycles) per tile and block, where
 // the int8 form takes a 35-cycle instruction, a 32-cycle one and two vector instructions per output of a 32 x 32 tile.
-// Matrix and vector cycles of these instructions add up here (counters at 1000 rows: vector 36 %, matrix 38 %, at once 13 % of the time), which is
-// why the cycles above are what counts; and the tiles fill the chip better than 128 x 128 ones.  Packing included, Q4_0, 4096 x 4096: 385 rows 66 -> 46 us,
-// 512 rows 68 -> 48, 600 rows 96 -> 64, 1000 rows 94 -> 75, 2048 rows 118 -> 117; 4096 x 11008: 512 rows 164 -> 112, 1000 rows 228 -> 184;
-// 22016 x 4096: 77 rows 85 -> 62, 320 rows 152 -> 131, 1000 rows 314 -> 297.
-// A wave takes RW groups of 16 weight rows and C groups of activation rows, so that an activation operand read from LDS serves RW instructions.
+// Matrix and vector cycles of these instructions hardly overlap (counters of 16 x 16 tiles at 1000 rows: vector 36 %, matrix 38 %, at once 13 % of the time), which is
+// why the cycles above are what counts; and the tiles fill the chip better than 128 x 128 ones.  Packing included, Q4_0, 4096 x 4096: 385 rows 66 -> 42 us,
+// 512 rows 68 -> 45, 1000 rows 94 -> 68, 2048 rows 118 -> 108; 4096 x 11008: 1000 rows 228 -> 162; 22016 x 4096: 77 rows 85 -> 56, 1000 rows 314 -> 272.
+// Two kernels of one arithmetic.  xo_kernel, for few workgroups: four waves of 16 rows by four activation groups, in tiles of 16 x 16.
 // Weights: lane (q, r) reads blocks 2q and 2q + 1 of row r and chunk (contiguous over the four lanes of a row), brings words 2i and 2i + 1 of a block
 // into one dword, and 4 x 4 exchanges between the lane blocks (v_permlane16_swap, v_permlane32_swap) leave words 2q and 2q + 1 of every block in lane block q:
 // the sixteen neighbouring bytes that a lane's activation operand is in LDS.  (With words q and 4 + q, two 8-byte reads 16 bytes apart met in the same banks,
 // half of the LDS cycles: 4096 x 11008 x 1000 182 -> 166 us, 22016 x 4096 x 1000 307 -> 297, 4096 x 4096 x 1000 74 -> 71.)
-struct xo_raw { uint32_t w[9]; };
+typedef float xo_v32f __attribute__((ext_vector_type(32)));
+__device__ __forceinline__ xt_v16f xo_mfma(const uint4 &a, const uint4 &b, const xt_v16f &c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(xk_h8, a), __builtin_bit_cast(xk_h8, b), c, 0, 0, 0);
+}
+// eight quants of two words, low and high nibbles, as fp16 less 8: elements 0, 2, 1, 3 of either
+__device__ __forceinline__ uint4 xo_unpack(uint32_t v) {
+    const uint32_t u = v >> 8, c64 = 0x64006400u;
+    return make_uint4(xt_sub(xt_and_or(v, 0x000F000Fu, c64), 0x64086408u), xt_sub(xt_and_or(u, 0x000F000Fu, c64), 0x64086408u),
+                      xk_pk_fma(xt_and_or(v, 0x00F000F0u, c64), 0x2C002C00u, 0xD480D480u), xk_pk_fma(xt_and_or(u, 0x00F000F0u, c64), 0x2C002C00u, 0xD480D480u));        // (1024 + 16 n) / 16 - 72
+}
+// products of two blocks' scales, 32 x 32 each: lane (h, r) brings those of block h and row r
+__device__ __forceinline__ xo_v32f xo_scales(uint32_t a, uint32_t b) {
+    return __builtin_amdgcn_mfma_f32_32x32x4f16(__builtin_bit_cast(xt_h4, make_uint2(a, 0u)), __builtin_bit_cast(xt_h4, make_uint2(b, 0u)), xo_v32f{}, 0, 0, 0);
+}
 __device__ __forceinline__ void xo_transpose(uint32_t (&r)[4]) {
     auto s16 = [](uint32_t &a, uint32_t &b) { auto v = __builtin_amdgcn_permlane16_swap(a, b, false, false); a = v[0]; b = v[1]; };
     auto s32 = [](uint32_t &a, uint32_t &b) { auto v = __builtin_amdgcn_permlane32_swap(a, b, false, false); a = v[0]; b = v[1]; };
     s16(r[0], r[1]); s16(r[2], r[3]);
     s32(r[0], r[2]); s32(r[1], r[3]);
 }
-template <int RW, int WV, int C, int OCC>
-__global__ __launch_bounds__(64 * WV, OCC) void xo_kernel(xt_args a) {
-    constexpr int NT = 64 * WV, ROWS = 16 * RW * WV, NXI = C * 256 / NT, C2 = (C + 1) / 2, XB = C * XT_XB + C2 * 1024, NDW = 9, CB = xt_w<SPY_HIP_Q4_0>::CB;
-    static_assert(NXI * NT == C * 256 && WV >= C2, "one request per thread and group, one wave per two groups' records");
+constexpr int XO_C = 4;
+__global__ __launch_bounds__(256, 3) void xo_kernel(xt_args a) {
+    constexpr int C = XO_C, NT = 256, ROWS = 64, C2 = C / 2, XB = C * XT_XB + C2 * 1024, NDW = 9, CB = xt_w<SPY_HIP_Q4_0>::CB;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, r = lane & 15;
     const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS, cg0 = (int)blockIdx.y * C;
     const int nst = a.nst, ncg = a.ncg, M = a.M;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
-    const uint8_t *bx[NXI], *bd;
+    const uint8_t *bx[C], *bd;
 #pragma unroll
-    for (int i = 0; i < NXI; i++) bx[i] = a.xq + (int64_t)min(cg0 + (i * NT + wave * 64) / 256, ncg - 1) * nst * XT_XB + (i * NT + wave * 64) % 256 * 16;
+    for (int i = 0; i < C; i++) bx[i] = a.xq + (int64_t)min(cg0 + i, ncg - 1) * nst * XT_XB + wave * 1024;
     const int dc0 = min(cg0 + 2 * min(wave, C2 - 1), ncg - 1), dc1 = min(dc0 + 1, ncg - 1);
     bd = a.xd + (int64_t)dc0 * nst * XT_XD;
     const uint32_t l16 = lane * 16, ld = (lane & 31) * 16 + (lane >> 5) * (uint32_t)((dc1 - dc0) * nst * XT_XD);
@@ -1124,95 +1135,70 @@ __global__ __launch_bounds__(64 * WV, OCC) void xo_kernel(xt_args a) {
         const uint32_t o = (is & 1) * XB;
         const int adv = is + 1 < nst ? 1 : 0;
 #pragma unroll
-        for (int i = 0; i < NXI; i++) { xt_dma16(bx[i], l16, ldsx + o + i * NT * 16); bx[i] += adv * XT_XB; }
+        for (int i = 0; i < C; i++) { xt_dma16(bx[i], l16, ldsx + o + i * NT * 16); bx[i] += adv * XT_XB; }
         xt_dma16(bd, ld, ldsd + o);
         bd += adv * XT_XD;
         is++;
     };
-    const uint8_t *wr[RW];
-#pragma unroll
-    for (int w = 0; w < RW; w++) wr[w] = a.w[mat] + (int64_t)min(m0 + (wave * RW + w) * 16 + r, M - 1) * a.w_row + q * (NDW * 4);
-    auto load_w = [&](xo_raw (&t)[RW], int chunk) {
-#pragma unroll
-        for (int w = 0; w < RW; w++) __builtin_memcpy(t[w].w, __builtin_assume_aligned(wr[w] + (int64_t)chunk * CB, 4), NDW * 4);
-    };
-    xo_raw cur[RW];
-    load_w(cur, 0);
+    const uint8_t *wr = a.w[mat] + (int64_t)min(m0 + wave * 16 + r, M - 1) * a.w_row + q * (NDW * 4);
+    uint32_t cur[NDW];
+    auto load_w = [&](int chunk) { __builtin_memcpy(cur, __builtin_assume_aligned(wr + (int64_t)chunk * CB, 4), NDW * 4); };
+    load_w(0);
     issue_x();
-    float acc[RW][C][4];
+    float acc[C][4];
 #pragma unroll
-    for (int w = 0; w < RW; w++)
+    for (int c = 0; c < C; c++)
 #pragma unroll
-        for (int c = 0; c < C; c++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) acc[w][c][v] = 0.0f;
-    uint32_t wd[RW][2][4], dd[RW];                 // [row group][even, odd blocks][block of that kind]; the lane's two scales
+        for (int v = 0; v < 4; v++) acc[c][v] = 0.0f;
+    uint32_t wd[2][4], dd;                         // [even, odd blocks][block of that kind]; the lane's two scales
     auto spread = [&]() {
-#pragma unroll
-        for (int w = 0; w < RW; w++) {
-            const uint32_t *v = cur[w].w;
-            dd[w] = (v[0] & 0xFFFFu) | (v[4] & 0xFFFF0000u);
-            // dword i of a block: word 2i in the low nibbles, word 2i + 1 in the high ones (words 0..3 are the low nibbles of the block's four dwords, words 4..7 the high ones)
-            auto pair = [](uint32_t (&o)[4], uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
-                constexpr uint32_t lo = 0x0F0F0F0Fu;
-                o[0] = (a & lo) | ((b << 4) & ~lo); o[1] = (c & lo) | ((d << 4) & ~lo);
-                o[2] = ((a >> 4) & lo) | (b & ~lo); o[3] = ((c >> 4) & lo) | (d & ~lo);
-            };
-            pair(wd[w][0], __builtin_amdgcn_alignbit(v[1], v[0], 16), __builtin_amdgcn_alignbit(v[2], v[1], 16), __builtin_amdgcn_alignbit(v[3], v[2], 16), __builtin_amdgcn_alignbit(v[4], v[3], 16));
-            pair(wd[w][1], v[5], v[6], v[7], v[8]);
-            xo_transpose(wd[w][0]);
-            xo_transpose(wd[w][1]);
-        }
+        const uint32_t *v = cur;
+        dd = (v[0] & 0xFFFFu) | (v[4] & 0xFFFF0000u);
+        // dword i of a block: word 2i in the low nibbles, word 2i + 1 in the high ones (words 0..3 are the low nibbles of the block's four dwords, words 4..7 the high ones)
+        auto pair = [](uint32_t (&o)[4], uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+            constexpr uint32_t lo = 0x0F0F0F0Fu;
+            o[0] = (a & lo) | ((b << 4) & ~lo); o[1] = (c & lo) | ((d << 4) & ~lo);
+            o[2] = ((a >> 4) & lo) | (b & ~lo); o[3] = ((c >> 4) & lo) | (d & ~lo);
+        };
+        pair(wd[0], __builtin_amdgcn_alignbit(v[1], v[0], 16), __builtin_amdgcn_alignbit(v[2], v[1], 16), __builtin_amdgcn_alignbit(v[3], v[2], 16), __builtin_amdgcn_alignbit(v[4], v[3], 16));
+        pair(wd[1], v[5], v[6], v[7], v[8]);
+        xo_transpose(wd[0]);
+        xo_transpose(wd[1]);
     };
-    const uint32_t c64 = 0x64006400u;
     const xk_v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
     auto compute = [&](int s, auto par_c) {
         constexpr int par = decltype(par_c)::value;
         const uint8_t *sx = smem + (s & 1) * XB + q * 256 + r * 16, *sd = smem + (s & 1) * XB + C * XT_XB + lane * 4;
-        uint4 w[RW][4];                            // operands of the stage's four blocks: words 2q and 2q + 1, elements 0, 2, 1, 3 each
-        uint32_t dw[RW];
+        uint4 w[4];                                // operands of the stage's four blocks: words 2q and 2q + 1, elements 0, 2, 1, 3 each
+        // lane (kb, r): the scale of block 4 par + kb, which lane block 2 par + kb / 2 holds
+        const uint32_t d2 = (uint32_t)__builtin_amdgcn_ds_bpermute(((2 * par + (q >> 1)) * 16 + r) * 4, (int)dd), dw = (q & 1) ? d2 >> 16 : d2 & 0xFFFFu;
 #pragma unroll
-        for (int g = 0; g < RW; g++) {
-            // lane (kb, r): the scale of block 4 par + kb, which lane block 2 par + kb / 2 holds
-            const uint32_t d2 = (uint32_t)__builtin_amdgcn_ds_bpermute(((2 * par + (q >> 1)) * 16 + r) * 4, (int)dd[g]);
-            dw[g] = (q & 1) ? d2 >> 16 : d2 & 0xFFFFu;
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const uint32_t v = wd[g][b & 1][2 * par + (b >> 1)], u = v >> 8;
-                w[g][b] = make_uint4(xt_sub(xt_and_or(v, 0x000F000Fu, c64), 0x64086408u), xt_sub(xt_and_or(u, 0x000F000Fu, c64), 0x64086408u),
-                                     xk_pk_fma(xt_and_or(v, 0x00F000F0u, c64), 0x2C002C00u, 0xD480D480u), xk_pk_fma(xt_and_or(u, 0x00F000F0u, c64), 0x2C002C00u, 0xD480D480u));   // (1024 + 16 n) / 16 - 72
-            }
-        }
+        for (int b = 0; b < 4; b++) w[b] = xo_unpack(wd[b & 1][2 * par + (b >> 1)]);
         constexpr int NJ = 4 * C;                  // steps (activation group, block)
         uint4 xv[3];
         uint32_t dx[2];
-        xk_v4f p[2][RW];
-        xt_v16f D[RW];
+        xk_v4f p[2];
+        xt_v16f D;
         auto rd = [&](int j) {
             xv[j % 3] = *(const uint4 *)(sx + (j >> 2) * XT_XB + (j & 3) * 1024);
         };
         dx[0] = *(const uint32_t *)sd;
         rd(0);
         rd(1);
-#pragma unroll
-        for (int g = 0; g < RW; g++) p[0][g] = xk_mfma(w[g][0], xv[0], zero);
-#pragma unroll
-        for (int g = 0; g < RW; g++) D[g] = xt_mfma(dw[g], 0u, dx[0], 0u);
+        p[0] = xk_mfma(w[0], xv[0], zero);
+        D = xt_mfma(dw, 0u, dx[0], 0u);
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
             const int c = j >> 2, b = j & 3;
             if (j + 2 < NJ) rd(j + 2);
             if (b == 1 && c + 1 < C) dx[(c + 1) & 1] = *(const uint32_t *)(sd + (c + 1) * XT_XD);
             // one matrix instruction, then the four fmas that run beside it
+            if (j + 1 < NJ) p[(j + 1) & 1] = xk_mfma(w[(j + 1) & 3], xv[(j + 1) % 3], zero);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int g = 0; g < RW; g++) {
-                if (j + 1 < NJ) p[(j + 1) & 1][g] = xk_mfma(w[g][(j + 1) & 3], xv[(j + 1) % 3], zero);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int v = 0; v < 4; v++) acc[g][c][v] = fmaf(D[g][4 * b + v], p[j & 1][g][v], acc[g][c][v]);
-                if (b == 3 && c + 1 < C) D[g] = xt_mfma(dw[g], 0u, dx[(c + 1) & 1], 0u);
-                __builtin_amdgcn_sched_barrier(0);
-            }
+            for (int v = 0; v < 4; v++) acc[c][v] = fmaf(D[4 * b + v], p[j & 1][v], acc[c][v]);
+            if (b == 3 && c + 1 < C) D = xt_mfma(dw, 0u, dx[(c + 1) & 1], 0u);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
     auto ready = [&]() {
@@ -1222,8 +1208,142 @@ __global__ __launch_bounds__(64 * WV, OCC) void xo_kernel(xt_args a) {
     for (int s = 0; s < nst; s += 2) {
         ready();
         spread();                                  // the compiler's own wait for the chunk stands here, where nothing is on its way
-        load_w(cur, min(s / 2 + 1, nst / 2 - 1));
         issue_x();
+        load_w(min(s / 2 + 1, nst / 2 - 1));
+        compute(s, std::integral_constant<int, 0>{});
+        ready();
+        issue_x();
+        compute(s + 1, std::integral_constant<int, 1>{});
+    }
+    xt_wait_vm<0>();
+    float *dst = a.dst[mat];
+    const int row = m0 + wave * 16 + 4 * q;
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int t = (cg0 + c) * 16 + r;
+        if (t < a.T && row + 3 < M) {
+            const int64_t at = (int64_t)t * a.d_row + row;
+            float4 o = make_float4(acc[c][0], acc[c][1], acc[c][2], acc[c][3]);
+            if (a.resid) { const float4 z = *(const float4 *)(a.resid + at); o.x += z.x; o.y += z.y; o.z += z.z; o.w += z.w; }
+            *(float4 *)(dst + at) = o;
+        }
+    }
+}
+// The same for many activation rows: four waves of 32 rows by four pairs of activation groups, in tiles of 32 x 32.  An operand read from LDS serves twice the
+// arithmetic of a 16 x 16 tile's, and the compiler may order the matrix and vector instructions of a tile, which with 16 x 16 it did worse than by hand.
+// On registers alone this form takes 19.4 ns per 16 x 16 x 32 and SIMD (two waves; the clock falls under these instructions) and the other 23.2; here it is
+// 23.8, for 100 instructions of unpacking beside 256 fmas and 1536 matrix cycles.  Packing included, two row groups of 16 per wave before: 22016 x 4096 x 1000
+// 308 -> 272 us, 12288 x 4096 x 1000 167 -> 151, 4096 x 11008 x 1000 171 -> 162, 4096 x 4096 x 1000 73 -> 68.
+// (Two pairs per wave: 340 us at 22016 x 4096 x 1000; three: 311.)
+constexpr int XO_CP = 4;
+__global__ __launch_bounds__(256, 2) void xo32_kernel(xt_args a) {
+    constexpr int CP = XO_CP, NT = 256, ROWS = 128, C = 2 * CP, XB = C * XT_XB + CP * 1024, NDW = 18, CB = xt_w<SPY_HIP_Q4_0>::CB;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, r = lane & 31;
+    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS, cg0 = (int)blockIdx.y * C;
+    const int nst = a.nst, ncg = a.ncg, M = a.M;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
+    const uint8_t *bx[C], *bd;
+#pragma unroll
+    for (int i = 0; i < C; i++) bx[i] = a.xq + (int64_t)min(cg0 + i, ncg - 1) * nst * XT_XB + wave * 1024;
+    const int dc0 = min(cg0 + 2 * min(wave, CP - 1), ncg - 1), dc1 = min(dc0 + 1, ncg - 1);
+    bd = a.xd + (int64_t)dc0 * nst * XT_XD;
+    const uint32_t l16 = lane * 16, ld = r * 16 + h * (uint32_t)((dc1 - dc0) * nst * XT_XD);
+    const uint32_t ldsx = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024), ldsd = __builtin_amdgcn_readfirstlane(lds0 + C * XT_XB + min(wave, CP - 1) * 1024);
+    int is = 0;
+    auto issue_x = [&]() {
+        const uint32_t o = (is & 1) * XB;
+        const int adv = is + 1 < nst ? 1 : 0;
+#pragma unroll
+        for (int i = 0; i < C; i++) { xt_dma16(bx[i], l16, ldsx + o + i * NT * 16); bx[i] += adv * XT_XB; }
+        xt_dma16(bd, ld, ldsd + o);
+        bd += adv * XT_XD;
+        is++;
+    };
+    // lane (h, r): blocks 4h .. 4h + 3 of row r and chunk
+    const uint8_t *wr = a.w[mat] + (int64_t)min(m0 + wave * 32 + r, M - 1) * a.w_row + h * (NDW * 4);
+    uint32_t cur[NDW];
+    auto load_w = [&](int chunk) { __builtin_memcpy(cur, __builtin_assume_aligned(wr + (int64_t)chunk * CB, 4), NDW * 4); };
+    load_w(0);
+    issue_x();
+    float acc[CP][16];
+#pragma unroll
+    for (int c = 0; c < CP; c++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[c][v] = 0.0f;
+    uint32_t wd[2][4][2], dd[2][2];                // [stage of the chunk][block][words 4h, 4h + 1 | 4h + 2, 4h + 3]; [stage][block pair] scales
+    auto swap = [](uint32_t &x, uint32_t &y) { auto v = __builtin_amdgcn_permlane32_swap(x, y, false, false); x = v[0]; y = v[1]; };
+    auto spread = [&]() {
+        constexpr uint32_t lo = 0x0F0F0F0Fu;
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            uint32_t v[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int k = b * 9 / 2 + i;                                    // the block's quants start at byte 18 b + 2
+                v[i] = b & 1 ? cur[k + 1] : __builtin_amdgcn_alignbit(cur[k + 1], cur[k], 16);
+            }
+            // words 0 .. 3 are the low nibbles of the block's four dwords, 4 .. 7 the high ones: the lanes below keep the low ones of theirs and take those of the others
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                uint32_t l = (v[2 * i] & lo) | ((v[2 * i + 1] << 4) & ~lo), u = ((v[2 * i] >> 4) & lo) | (v[2 * i + 1] & ~lo);
+                swap(l, u);
+                wd[0][b][i] = l;
+                wd[1][b][i] = u;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            uint32_t x = (cur[9 * k] & 0xFFFFu) | (cur[9 * k + 4] & 0xFFFF0000u), y = x;
+            swap(x, y);
+            dd[0][k] = h ? x >> 16 : x & 0xFFFFu;
+            dd[1][k] = h ? y >> 16 : y & 0xFFFFu;
+        }
+    };
+    auto compute = [&](int s, auto par_c) {
+        constexpr int par = decltype(par_c)::value;
+        const uint8_t *sx = smem + (s & 1) * XB + (r >> 4) * XT_XB + h * 512 + (r & 15) * 16, *sd = smem + (s & 1) * XB + C * XT_XB + (r >> 4) * XT_XD + h * 64 + (r & 15) * 4;
+        uint4 w[4][2];
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) w[b][i] = xo_unpack(wd[par][b][i]);
+        constexpr int NJ = 4 * CP;                 // steps (activation pair, block)
+        uint4 xv[3][2];
+        uint32_t dx[2];
+        xt_v16f p[2];
+        xo_v32f D;
+        auto rd = [&](int j) {
+            xv[j % 3][0] = *(const uint4 *)(sx + (j >> 2) * 2 * XT_XB + (j & 3) * 1024);
+            xv[j % 3][1] = *(const uint4 *)(sx + (j >> 2) * 2 * XT_XB + (j & 3) * 1024 + 256);
+        };
+        auto rd_d = [&](int k) { dx[k & 1] = *(const uint32_t *)(sd + (k >> 1) * 2 * XT_XD + (k & 1) * 128); };        // k: (activation pair, block pair)
+        auto mm = [&](int j) { p[j & 1] = xo_mfma(w[j & 3][1], xv[j % 3][1], xo_mfma(w[j & 3][0], xv[j % 3][0], xt_v16f{})); };
+        rd_d(0);
+        rd(0);
+        rd_d(1);
+        rd(1);
+        mm(0);
+        D = xo_scales(dd[par][0], dx[0]);
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            if (j + 2 < NJ) rd(j + 2);
+            if ((j & 1) == 0 && j / 2 + 2 < NJ / 2) rd_d(j / 2 + 2);
+            if (j + 1 < NJ) mm(j + 1);
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[j >> 2][v] = fmaf(D[16 * (j & 1) + v], p[j & 1][v], acc[j >> 2][v]);
+            if ((j & 1) && j + 1 < NJ) D = xo_scales(dd[par][(j + 1) >> 1 & 1], dx[(j + 1) >> 1 & 1]);
+        }
+    };
+    auto ready = [&]() {
+        xt_wait_vm<0>();
+        __builtin_amdgcn_s_barrier();
+    };
+    for (int s = 0; s < nst; s += 2) {
+        ready();
+        spread();                                  // the compiler's own wait for the chunk stands here, where nothing is on its way
+        issue_x();
+        load_w(min(s / 2 + 1, nst / 2 - 1));
         compute(s, std::integral_constant<int, 0>{});
         ready();
         issue_x();
@@ -1232,26 +1352,33 @@ __global__ __launch_bounds__(64 * WV, OCC) void xo_kernel(xt_args a) {
     xt_wait_vm<0>();
     float *dst = a.dst[mat];
 #pragma unroll
-    for (int g = 0; g < RW; g++) {
-        const int row = m0 + (wave * RW + g) * 16 + 4 * q;
+    for (int c = 0; c < CP; c++) {
+        const int t = (cg0 + 2 * c) * 16 + r;
 #pragma unroll
-        for (int c = 0; c < C; c++) {
-            const int t = (cg0 + c) * 16 + r;
+        for (int g = 0; g < 4; g++) {
+            const int row = m0 + wave * 32 + 8 * g + 4 * h;
             if (t < a.T && row + 3 < M) {
                 const int64_t at = (int64_t)t * a.d_row + row;
-                float4 o = make_float4(acc[g][c][0], acc[g][c][1], acc[g][c][2], acc[g][c][3]);
+                float4 o = make_float4(acc[c][4 * g], acc[c][4 * g + 1], acc[c][4 * g + 2], acc[c][4 * g + 3]);
                 if (a.resid) { const float4 z = *(const float4 *)(a.resid + at); o.x += z.x; o.y += z.y; o.z += z.z; o.w += z.w; }
                 *(float4 *)(dst + at) = o;
             }
         }
     }
 }
-template <int RW, int WV, int C, int OCC>
+int xo32_launch(hipStream_t st, xt_args a, int nmat) {
+    constexpr size_t lds = 2 * (2 * XO_CP * XT_XB + XO_CP * 1024);
+    const int rc = spy_raise_lds_limit((const void *)xo32_kernel, lds);
+    if (rc) return rc;
+    a.tiles = (a.M + 127) / 128;
+    xo32_kernel<<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + 2 * XO_CP - 1) / (2 * XO_CP))), dim3(256), lds, st>>>(a);
+    return SPY_LAUNCH_RC();
+}
 int xo_launch(hipStream_t st, xt_args a, int nmat) {
-    constexpr size_t lds = 2 * (C * XT_XB + (C + 1) / 2 * 1024);
-    if (lds > 64 * 1024) { const int rc = spy_raise_lds_limit((const void *)xo_kernel<RW, WV, C, OCC>, lds); if (rc) return rc; }
-    a.tiles = (a.M + 16 * RW * WV - 1) / (16 * RW * WV);
-    xo_kernel<RW, WV, C, OCC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * WV), lds, st>>>(a);
+    constexpr size_t lds = 2 * (XO_C * XT_XB + XO_C / 2 * 1024);
+    static_assert(lds <= 64 * 1024, "");
+    a.tiles = (a.M + 63) / 64;
+    xo_kernel<<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + XO_C - 1) / XO_C)), dim3(256), lds, st>>>(a);
     return SPY_LAUNCH_RC();
 }
 template <int WT, bool OWN, int RG, int C, int OCC, int KS = 1>
@@ -1300,7 +1427,7 @@ int xt_dispatch(hipStream_t st, const xt_args &a, int nmat) {
     default: return rest == 1 ? xt_launch_mixed<WT, 1>(st, a, nmat) : rest == 2 ? xt_launch_mixed<WT, 2>(st, a, nmat) : xt_launch_mixed<WT, 3>(st, a, nmat);
     }
 }
-// Tiles of the K-quants: times in tenths of a microsecond at K = 4096 with 1, 2, 3, 4 and 6 workgroups per compute unit, weights from memory
+// Tiles of the K-quants, and of Q4_0 in the own order: times in tenths of a microsecond at K = 4096 with 1, 2, 3, 4 and 6 workgroups per compute unit, weights from memory
 struct xk_tile { int rows, groups, t[5]; };
 int xk_pick(const xt_args &a, int nmat, int ncg, const xk_tile *c, int n_tiles) {
     const int64_t cu = spy_num_cu();
@@ -1348,13 +1475,9 @@ int xko_dispatch(hipStream_t st, const xt_args &a, int nmat) {
 }
 
 int xo_dispatch(hipStream_t st, const xt_args &a, int nmat) {
-    // as in xt_dispatch: measured with one workgroup per CU and with the chip full
-    static const xt_cost c4[3] = {{64, 4, 290, 155}, {128, 4, 400, 275}, {128, 8, 600, 490}};
-    switch (xt_pick(a, nmat, c4, 3)) {
-    case 0: return xo_launch<1, 4, 4, 3>(st, a, nmat);
-    case 1: return xo_launch<2, 4, 4, 3>(st, a, nmat);
-    default: return xo_launch<2, 4, 8, 2>(st, a, nmat);
-    }
+    // tiles of 128 rows by four groups (two of 32 x 32 per wave) were the better ones nowhere: 8192 x 4096 x 500 69.1 us, these two 68.9 and 66.2
+    static const xk_tile c[2] = {{64, 4, {342, 383, 515, 650, 949}}, {128, 8, {607, 990, 1472, 1933, 2895}}};
+    return xk_pick(a, nmat, a.ncg, c, 2) == 0 ? xo_launch(st, a, nmat) : xo32_launch(st, a, nmat);
 }
 
 }   // namespace

@@ -191,6 +191,12 @@ def test_matmul_operator_splits_k(hip, oracle, wtype, M, K, T, monkeypatch):
     test_matmul_operator_takes_the_packed_activation_kernels(hip, oracle, wtype, M, K, T, monkeypatch)
 
 
+@pytest.mark.parametrize("M,K,T", [(8100, 768, 985), (16300, 256, 485), (12284, 512, 970)])
+def test_matmul_operator_tiles_of_32(hip, oracle, M, K, T, monkeypatch):
+    """Q4_0 in the own order from many activation rows, tiles of 32 x 32: one chunk, odd and even numbers of them, an odd number of activation groups, partial tiles."""
+    test_matmul_operator_takes_the_packed_activation_kernels(hip, oracle, O.Q4_0, M, K, T, monkeypatch)
+
+
 @pytest.mark.parametrize("n_prompt", [129, 400])
 def test_own_order_prompt_from_packed_activations(hip, n_prompt, monkeypatch):
     """One layer of the 7B shape in this backend's own order: norm, activation and residual steps around the packed-activation MatMuls (from 129 tokens

@@ -113,19 +113,20 @@ __global__ __launch_bounds__(64) void rope_store_kernel(const float *__restrict_
     }
 }
 
-// v: f32 [T][d] -> V^T cache: fp16 vc[col * n_ctx + t] for t < T (vc points at the pass's first position); 64 x 64 tiles through LDS
+// v: f32 [T][d] -> V^T cache: fp16 vc[col * n_ctx + t] for t < T (vc points at the pass's first position); 64 x 64 tiles through LDS, a thread's
+// sixteen elements all on their way at once (one after the other: 77 rows of 4096 8.3 -> 4.9 us, 1000 rows 11.4 -> 6.3, 2048 rows 14 -> 10, the time of a copy)
 __global__ __launch_bounds__(256) void vt_store_kernel(const float *__restrict__ v, uint16_t *__restrict__ vc, int T, int d, int64_t n_ctx) {
     __shared__ uint16_t tile[64][66];
-    const int t0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
-    for (int i = threadIdx.x; i < 64 * 64; i += 256) {
-        const int tt = i >> 6, cc = i & 63;
-        tile[tt][cc] = (t0 + tt < T && c0 + cc < d) ? f2h(v[(size_t)(t0 + tt) * d + c0 + cc]) : (uint16_t)0;
-    }
+    const int t0 = blockIdx.x * 64, c0 = blockIdx.y * 64, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float x[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) x[k] = v[(size_t)min(t0 + wave + 4 * k, T - 1) * d + min(c0 + lane, d - 1)];
+#pragma unroll
+    for (int k = 0; k < 16; k++) tile[wave + 4 * k][lane] = f2h(x[k]);
     __syncthreads();
-    for (int i = threadIdx.x; i < 64 * 64; i += 256) {
-        const int cc = i >> 6, tt = i & 63;
-        if (t0 + tt < T && c0 + cc < d) vc[(size_t)(c0 + cc) * n_ctx + t0 + tt] = tile[tt][cc];
-    }
+#pragma unroll
+    for (int k = 0; k < 16; k++)
+        if (t0 + lane < T && c0 + wave + 4 * k < d) vc[(size_t)(c0 + wave + 4 * k) * n_ctx + t0 + lane] = tile[lane][wave + 4 * k];
 }
 
 int spy_rope_table_launch(hipStream_t st, float *table, int past, int T, int hd, float freq_base, float freq_scale, float mscale) {

@@ -94,6 +94,10 @@ __device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
 
     // what a wave requests: uniform bases that advance, per-lane offsets that stay.  Row groups and activation groups past the end
     // repeat the last one.
+    // The last request of a chunk covers it with the first waves only; the others repeat the first wave's, the same bytes to the same place.  (With a spare
+    // kilobyte for what they repeat a compute unit had room for two workgroups of the Q8_0 tile instead of three: 22016 x 4096 x 512 474 -> 448 us,
+    // 4096 x 4096 x 2048 347 -> 326, 12288 x 4096 x 100 69.7 -> 61.8.)
+    const int wl = wave * 64 + (NI - 1) * NT >= UW ? 0 : wave;
     const uint8_t *bx[NXI], *bd, *bw = a.w[mat] + (int64_t)m0 * a.w_row;
     uint32_t ow[NI];
 #pragma unroll
@@ -101,15 +105,12 @@ __device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
     bd = a.xd + (int64_t)min(cg0 + min(wave, C - 1), ncg - 1) * nst * XT_XD;
 #pragma unroll
     for (int i = 0; i < NI; i++) {
-        const int u = min(tid + i * NT, UW - 1);
+        const int u = min((i == NI - 1 ? wl * 64 + lane : tid) + i * NT, UW - 1);
         ow[i] = (uint32_t)(min(m0 + u / CU, M - 1) - m0) * (uint32_t)a.w_row + (u % CU) * 16;
     }
-    // (the last request of a chunk covers it with the first waves only: the others put what they repeat into the spare kilobyte after the rings)
-    const bool spare = wave * 64 + (NI - 1) * NT >= UW;
-    const uint32_t lds_spare = __builtin_amdgcn_readfirstlane(lds0 + NXS * XB + NWC * WB);
     const uint32_t l16 = lane * 16, l4 = lane * 4;
     const uint32_t ldsx = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024), ldsd = __builtin_amdgcn_readfirstlane(lds0 + C * XT_XB + min(wave, C - 1) * 256),
-                   ldsw = __builtin_amdgcn_readfirstlane(lds0 + NXS * XB + wave * 1024);
+                   ldsw = __builtin_amdgcn_readfirstlane(lds0 + NXS * XB + wave * 1024), ldswl = __builtin_amdgcn_readfirstlane(lds0 + NXS * XB + wl * 1024);
     int is = 0;                                    // next stage to request; past the last one it is requested again (same count of requests, slot unused)
     auto issue_x = [&]() {
         const uint32_t o = (is & (NXS - 1)) * XB;
@@ -121,9 +122,9 @@ __device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
         is++;
     };
     auto issue_w = [&]() {
-        const uint32_t o = ldsw + ((is >> 1) & (NWC - 1)) * WB;
+        const uint32_t o = ((is >> 1) & (NWC - 1)) * WB;
 #pragma unroll
-        for (int i = 0; i < NI; i++) xt_dma16(bw, ow[i], i == NI - 1 && spare ? lds_spare : o + i * NT * 16);
+        for (int i = 0; i < NI; i++) xt_dma16(bw, ow[i], (i == NI - 1 ? ldswl : ldsw) + o + i * NT * 16);
         bw += is + 2 < nst ? xt_w<WT>::CB : 0;
     };
 #pragma unroll
@@ -574,7 +575,7 @@ __global__ __launch_bounds__(256) void xt_silu_pack_kernel(const float *__restri
 }
 
 template <int WT, int C, int NXS, int NWC> constexpr size_t xt_lds() {
-    constexpr size_t ring = NXS * C * (XT_XB + 256) + NWC * ((32 * xt_w<WT>::CU + 63) / 64) * 1024 + 1024, ex = (size_t)2 * C * 16 * 256, lds = ring > ex ? ring : ex;
+    constexpr size_t ring = NXS * C * (XT_XB + 256) + NWC * ((32 * xt_w<WT>::CU + 63) / 64) * 1024, ex = (size_t)2 * C * 16 * 256, lds = ring > ex ? ring : ex;
     static_assert(lds <= 64 * 1024, "no raised LDS limit");
     return lds;
 }

@@ -605,6 +605,26 @@ def test_engine_prompt_attention_kernels_have_the_oracle_bits(hip, n_prompt, n_f
         eng.close()
 
 
+@pytest.mark.parametrize("n_prompt", [150, 160])
+def test_engine_prompt_with_gates_of_any_size(hip, n_prompt):
+    """A prompt long enough for the SiLU kernel that keeps part of the host's table in LDS, gates from 2^-14 to beyond 32, zeros among them, a ragged last group of rows:
+    the oracle's bits."""
+    from spy_amd import model as M
+    from tests.model_util import OracleModel
+    cfg = M.Config(n_layer=1, n_embd=256, n_head=2, n_ff=11008, n_vocab=512, n_ctx=256, wtype=O.Q4_0)
+    tensors = M.synth_model(cfg, seed=7)
+    name = next(k for k in tensors if "ffn_gate" in k)
+    w = tensors[name].copy().reshape(cfg.n_ff, -1, 18)
+    d = np.ascontiguousarray(w[:, :, :2]).view(np.float16)[:, :, 0].astype(np.float32) * np.ldexp(1.0, np.arange(cfg.n_ff) % 21 - 12).astype(np.float32)[:, None]
+    d[5::50] = 0.0
+    w[:, :, :2] = d.astype(np.float16)[:, :, None].view(np.uint8)
+    tensors[name] = np.ascontiguousarray(w).reshape(-1)
+    prompt = np.random.default_rng(n_prompt).integers(0, cfg.n_vocab, n_prompt).astype(np.int32)
+    eng = M.Engine(cfg, tensors)
+    _same_bits(eng.forward(prompt, 0), OracleModel(cfg, tensors).forward(prompt, 0), "%d tokens, gates of any size" % n_prompt)
+    eng.close()
+
+
 def test_prompt_attention_kernels_at_the_7b_width(hip, monkeypatch):
     """One layer of the 7B shape, 700 tokens on top of 300: the attention kernels against the operator path, bit for bit."""
     from spy_amd import model as M

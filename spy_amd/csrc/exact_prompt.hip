@@ -168,6 +168,8 @@ __global__ __launch_bounds__(256, 3) void xp_scores_kernel(const void *__restric
 // The exponentials: a gather of 64 table entries from memory takes about 64 cycles of the compute unit, so the part of the table that is not zero lies in
 // LDS: arguments are <= 0 (or NaN), and exp is 0 from -104 on.  The sum of a row goes through xg_segment_sum: 2 us instead of a chain of up to
 // 1024 additions.  2048 rows of 2049 .. 4096 positions and 32 heads (1.2 GB): 462 -> 306 us; 2048 rows of 1 .. 2048: 193 -> 152.
+// A row of a wave is a chain of latencies, so waves are what counts: with half the registers and group sums for rows of up to 2048 positions a workgroup has 16
+// instead of 12 (2048 rows of 1 .. 2048 positions 155 -> 123 us, 1000 rows 66 -> 50, 512 rows 29 -> 21).  The next row's scores requested a row ahead: 160 instead of 123.
 #define XP_LUT 0x5680      // fp16 -104.0 without its sign
 #define XP_SM_R 32         // groups per lane: rows of up to 8192 positions
 template <int R, int NW>
@@ -378,7 +380,8 @@ int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint1
     if (q_f16) xp_scores_kernel<true><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
     else xp_scores_kernel<false><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
     if (hipGetLastError() != hipSuccess) return SPY_HIP_EINVAL;
-    const int ncu = spy_num_cu(), rc = (int64_t)P + T <= 4096 ? xp_softmax_launch<16, 12>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
+    const int ncu = spy_num_cu(), rc = (int64_t)P + T <= 2048 ? xp_softmax_launch<8, 16>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
+                                         : (int64_t)P + T <= 4096 ? xp_softmax_launch<16, 12>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
                                          : (int64_t)P + T <= 6144 ? xp_softmax_launch<24, 8>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
                                                                   : xp_softmax_launch<32, 4>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu);
     if (rc) return rc;

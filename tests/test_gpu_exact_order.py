@@ -381,6 +381,12 @@ def test_exact_prompt_softmax_forms(hip, oracle, H_, past, T, n_ctx, spread):
     _same_bits(out.download(np.float32).reshape(T, d), want, "attention H %d past %d T %d spread %g" % (H_, past, T, spread))
 
 
+@pytest.mark.parametrize("H_,past,T,n_ctx", [(2, 2000, 48, 2048), (2, 2001, 48, 2080), (3, 1970, 41, 2016)])
+def test_exact_prompt_softmax_of_eight_groups(hip, oracle, H_, past, T, n_ctx):
+    """Rows up to and across 2048 positions, the longest of eight groups of four per lane."""
+    test_exact_prompt_softmax_forms(hip, oracle, H_, past, T, n_ctx, 1.0)
+
+
 def test_norm_softmax_silu_rope_bits(hip, oracle):
     from tests.gpu_util import dev, dev_empty, call
     L = hip.load()

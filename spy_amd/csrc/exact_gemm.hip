@@ -1462,7 +1462,10 @@ int xt_dispatch(hipStream_t st, const xt_args &a, int nmat) {
     // the last one: tiles of four groups and one of what remains, where something remains
     static const int of_rest[4] = {0, 60, 100, 132};
     const int rest = a.ncg > 4 ? a.ncg % 4 : 0;
-    const xt_cost c[5] = {{16, 1, 44, 44}, {32, 1, 106, 56}, {32, 2, 173, 96}, {32, 4, 288, 165}, {32, 4, 288, 165, of_rest[rest]}};
+    // Q8_0's first two tiles have room for four workgroups on a compute unit, and its chunks are larger: 4096 x 11008 x 150 100.5 -> 93.1 us, 4096 x 4096 x 150 42.2 -> 39.4,
+    // 12288 x 4096 x 180 116 -> 108 with its own increments.  98 for the third: 22016 x 4096 x 128 goes to the fourth, Q8_0 142 -> 128, Q4_0 129 -> 122.
+    constexpr bool Q8 = WT == SPY_HIP_Q8_0;
+    const xt_cost c[5] = {{16, 1, 44, Q8 ? 50 : 44}, {32, 1, 106, Q8 ? 64 : 56}, {32, 2, 173, 98}, {32, 4, 288, 165}, {32, 4, 288, 165, of_rest[rest]}};
     switch (xt_pick(a, nmat, c, rest ? 5 : 4)) {
     case 0: return (int64_t)(a.M + 15) / 16 * nmat * a.ncg <= 2 * spy_num_cu() ? xn_launch<WT, 4>(st, a, nmat) : xn_launch<WT, 2>(st, a, nmat);
     case 1: return xt_launch<WT, 1, 4, 2, 2>(st, a, nmat);

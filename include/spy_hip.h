@@ -252,7 +252,8 @@ int spy_hip_rope_kvwrite(void *stream, int32_t order, int32_t wtype, int32_t wty
                          void *q16, void *k_cache, void *v_cache, void *xq_dump);
 /* attn_score, Softmax, KQV of one token over n_kv cached tokens, all heads (MatMul(K view, q) -> Softmax(mask 0, scale
  * 1/sqrt(128)) -> MatMul(V^T view, P); mat.cpp:71-146, vec_dot.h:117-146, non-linear.cpp:129-180): two launches (scores;
- * softmax + P.V^T), or one with order 1 and up to 576 cached tokens.  scores: scratch f32 [n_head][n_ctx]; out: f32 [n_head * 128]. */
+ * softmax + P.V^T), or one with order 1 and up to 576 cached tokens.  k_cache: fp16 rows of n_head * 128, n_kv of them are read; v_cache: fp16 rows of n_ctx
+ * (a multiple of 8), n_head * 128 of them, of each the first n_kv elements rounded up to whole 16-byte pieces.  scores: scratch f32 [n_head][n_ctx]; out: f32 [n_head * 128]. */
 int spy_hip_attn_decode(void *stream, int32_t order, const void *q16, const void *k_cache, const void *v_cache, int32_t n_head, int32_t n_kv,
                         int64_t n_ctx, float *scores, float *out);
 /* One matrix x vector launch with its prologue and epilogue: normw != NULL, resid == NULL: RMSNorm * weight -> Q8_0 -> M rows

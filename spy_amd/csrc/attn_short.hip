@@ -2,6 +2,7 @@
 // (In a source of its own: the kernels of a layer of the single-token pass about fill the instruction cache, and where they lie in it counts.)
 #include "exact_decode.cuh"
 #include "engine_types.cuh"
+#include "attn_reach.h"
 
 // ---- scores, softmax and P.V^T of a short cache in one launch ------------------------------------------------------------
 // Up to XF_MAX cached tokens: the same 256 workgroups (head, 16 rows of V^T), each with all the scores of its head.  The eight
@@ -25,18 +26,19 @@ static __global__ __launch_bounds__(XP_THREADS) void xattn_short_kernel(const de
     uint4 *s_k = (uint4 *)smem;                                       // [token][16 pieces], rotated by 4 pieces per token against bank conflicts
     uint16_t *s_v = (uint16_t *)smem;                                 // the rows of V^T, once the keys have been read
     const uint16_t *vrow = vc + (size_t)(hd_ * 128 + dgrp * 16 + wave) * n_ctx;
-    // Keys first, then the rows of V^T.  What the first piece of either holds does not depend on the position, which is itself on its way: 64 keys and
-    // 512 elements of a row, as far as the cache goes; what lies behind the last token is not used.
+    // Keys first, then the rows of V^T.  Where the position is on its way itself (st), the first piece of either does not wait for it: 64 keys and 512 elements
+    // of a row, as far as the cache goes; what lies behind the last token is not used.  Where it is a number, nothing behind the last token is asked for (attn_reach.h).
     xp_u4 kr[XF_NP], vb, vb1, qr;
     auto key_piece = [&](int u, int n) {
-        const int c = min(tid + u * XP_THREADS, n * 16 - 1);
+        const int c = xf_piece(tid + u * XP_THREADS, n * 16);
         kr[u] = *(const xp_u4 *)(kc + (size_t)(c >> 4) * d + hd_ * 128 + (c & 15) * 8);
     };
-    key_piece(0, cap);
+    const int keys0 = xf_keys_before(st != nullptr, pos_imm, cap);
+    key_piece(0, keys0);
     if (tid < 16) qr = *(const xp_u4 *)(q16 + hd_ * 128 + tid * 8);
-    const int n_kv = min((st ? st->pos : pos_imm) + 1, cap), npiece = n_kv * 16, last_piece = (n_kv - 1) >> 3;
-    vb = *(const xp_u4 *)(vrow + (size_t)min(lane, n_ctx % 8 ? last_piece : n_ctx / 8 - 1) * 8);
-    if (last_piece >= 64) vb1 = *(const xp_u4 *)(vrow + (size_t)min(64 + lane, last_piece) * 8);
+    const int n_kv = st ? min(st->pos + 1, cap) : keys0, npiece = n_kv * 16, last_piece = (n_kv - 1) >> 3;
+    vb = *(const xp_u4 *)(vrow + (size_t)xf_piece(lane, xf_row_pieces_before(st != nullptr, pos_imm, n_ctx)) * 8);
+    if (last_piece >= 64) vb1 = *(const xp_u4 *)(vrow + (size_t)xf_piece(64 + lane, last_piece + 1) * 8);
 #pragma unroll
     for (int u = 1; u < XF_NP; u++) if (u * XP_THREADS < npiece) key_piece(u, n_kv);
     if (tid < 16) *(xp_u4 *)&s_qh[tid] = qr;

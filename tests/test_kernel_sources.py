@@ -2,6 +2,7 @@
 import glob
 import os
 import re
+import subprocess
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -22,3 +23,14 @@ def test_the_number_of_compute_units_is_kept_per_device():
     for path in sorted(glob.glob(os.path.join(ROOT, "spy_amd", "csrc", "*.hip")) + glob.glob(os.path.join(ROOT, "spy_amd", "csrc", "*.cuh"))):
         if os.path.basename(path) not in ("runtime.hip", "engine.hip", "peaks.hip"):
             assert not re.search("multiprocessorcount", open(path).read(), re.I), path
+
+
+def test_single_token_attention_reads_no_keys_behind_the_last_one(tmp_path):
+    """What the one-launch attention of order 1 requests before it knows the position lies within n_kv keys and the 16-byte piece of a V^T row that holds the last
+    token where the position is a number (spy_hip_attn_decode, a caller's caches), and within n_ctx where it is in device memory (the engine's)."""
+    out = str(tmp_path / "attn_reach")
+    subprocess.check_call(["g++", "-O1", "-std=c++20", "-o", out, os.path.join(ROOT, "tests", "host", "attn_reach.cpp")])
+    r = subprocess.run([out], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr
+    kernel = open(os.path.join(ROOT, "spy_amd", "csrc", "attn_short.hip")).read()
+    assert kernel.count("xf_keys_before(st != nullptr") == 1 and kernel.count("xf_row_pieces_before(st != nullptr") == 1 and kernel.count("key_piece(0, keys0)") == 1

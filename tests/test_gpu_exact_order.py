@@ -346,6 +346,24 @@ def test_exact_prompt_attention_unaligned_v(hip):
     _same_bits(outs[1], outs[0], "V^T cache at an odd element")
 
 
+def test_exact_prompt_attention_wants_its_probabilities_on_the_16_byte_grid(hip):
+    """The library's own entry behind spy_hip_prompt_attention_exact: the product reads the probabilities in 16-byte pieces, so a place for them 8 bytes off that
+    grid is refused, as it is for the other operands; one on the grid is taken."""
+    from tests.gpu_util import dev, dev_empty
+    H_, T, past, n_ctx, hd = 1, 20, 12, 64, 128
+    rng = np.random.default_rng(2)
+    dq, dk, dv = (dev(rng.standard_normal((r, c)).astype(t)) for r, c, t in ((T, H_ * hd, np.float32), (n_ctx, H_ * hd, np.float16), (H_ * hd, n_ctx, np.float16)))
+    L = hip.load()
+    need = L.spy_hip_prompt_attention_exact_scratch_size(T, H_, past)
+    S, P16, out, lut = dev_empty(need, 0), dev_empty(need + 16, 0), dev_empty(T * H_ * hd * 4, 0), C.c_void_p()
+    assert getattr(L, "_Z14spy_exact_lutsPPKf")(C.byref(lut)) == 0
+    attn = getattr(L, "_Z21spy_exact_prompt_attnP12ihipStream_tPKvbPKtS4_PfPtS5_PKfiiilif")
+    attn.argtypes = [C.c_void_p, C.c_void_p, C.c_bool] + [C.c_void_p] * 6 + [C.c_int] * 3 + [C.c_int64, C.c_int, C.c_float]
+    arg = lambda off: (None, dq.ptr, False, dk.ptr, dv.ptr, S.ptr, P16.ptr + off, out.ptr, lut, T, H_, past, n_ctx, past + T, 0.125)
+    assert attn(*arg(8)) == hip.EINVAL and attn(*arg(0)) == 0
+    hip.sync()
+
+
 @pytest.mark.parametrize("H_,past,T,n_ctx,spread", [
     (2, 4032, 64, 4096, 1.0),                 # the longest row of sixteen groups per lane, 1024 group sums
     (1, 5000, 40, 5056, 1.0), (1, 6130, 30, 6176, 1.0), (1, 8170, 22, 8192, 1.0),      # the wider forms and their edges (6144, 8192)

@@ -64,6 +64,14 @@ extern "C" int spy_hip_llama_destroy(spy_hip_llama *m) {
     return 0;
 }
 
+// SPY_HIP_SCORES_GRID (tests): read when an engine is made, so that its eager passes and its captured graphs launch the same kernels
+static int scores_grid_wanted(int num_cu) {
+    const char *e = getenv("SPY_HIP_SCORES_GRID");
+    if (!e) return 0;
+    const int v = atoi(e);
+    return v >= 1 && v <= num_cu ? v : num_cu;
+}
+
 extern "C" int spy_hip_llama_create(const spy_hip_llama_desc *desc, spy_hip_llama **out) {
     SPY_CHECK_ARG(desc && out && desc->layers);
     *out = nullptr;
@@ -100,6 +108,7 @@ extern "C" int spy_hip_llama_create(const spy_hip_llama_desc *desc, spy_hip_llam
     {
         int dev = 0; hipDeviceProp_t prop;
         if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0) m->num_cu = prop.multiProcessorCount;
+        m->scores_grid = scores_grid_wanted(m->num_cu);
     }
     m->theta_scale = powf(c.rope_freq_base, -2.0f / (float)m->hd);      // non-linear.cpp:282, host libm like the reference
     const size_t d = c.n_embd, C = c.n_ctx;
@@ -229,13 +238,12 @@ static bool fused_ok(const spy_hip_llama *m) {
 static int enqueue_one(spy_hip_llama *m, hipStream_t st, int which, int il) {
     const spy_hip_llama_desc &c = m->desc;
     if (pass_order(m) == 1 || (m->dry && m->order == 1)) {      // the host backend's summation order: six launches per layer, five where the cache is short
-        const bool one_launch = m->kv_bound > 0 && m->kv_bound <= XF_MAX && !getenv("SPY_HIP_SCORES_GRID");
+        const bool one_launch = m->kv_bound > 0 && m->kv_bound <= XF_MAX && !m->scores_grid;
         if (which == K_SCORES) {
             if (m->dry || one_launch) return 0;
-            // one workgroup per compute unit; SPY_HIP_SCORES_GRID (tests) forces fewer, so that a workgroup's share of the tokens
-            // takes several rounds of XS_TOK, as it would on a part with fewer compute units or a longer cache
-            int sgrid = m->num_cu;
-            if (const char *e = getenv("SPY_HIP_SCORES_GRID")) { const int v = atoi(e); if (v >= 1 && v <= m->num_cu) sgrid = v; }
+            // one workgroup per compute unit; tests have fewer, so that a workgroup's share of the tokens takes several rounds of
+            // XS_TOK, as it would on a part with fewer compute units or a longer cache
+            const int sgrid = m->scores_grid ? m->scores_grid : m->num_cu;
             xattn_scores_kernel<0><<<dim3((unsigned)sgrid), dim3(XS_THREADS), xattn_scores_lds(c.n_head), st>>>(
                 m->st, m->pos_imm, m->q16, m->k_cache[il], m->scores, c.n_head, c.n_ctx, 1.0f / sqrtf((float)m->hd));   // SoftmaxParam::scale (attention.cpp:113)
             return SPY_LAUNCH_RC();
@@ -909,6 +917,7 @@ struct family_ctx {
         if (kq && (n_embd % 256 != 0 || n_ff % 256 != 0)) return SPY_HIP_EINVAL;
         int dev = 0; hipDeviceProp_t prop;
         if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0) m.num_cu = prop.multiProcessorCount;
+        m.scores_grid = scores_grid_wanted(m.num_cu);
         if (order == 1) {
             if (n_embd % 128 != 0 || n_ff % 128 != 0) return SPY_HIP_EUNSUPPORTED;
             RC_TRY(spy_exact_luts(&m.lut));

@@ -27,6 +27,7 @@ struct spy_hip_llama {
     int32_t *tokens_out = nullptr;
     int max_out = 0;
     int num_cu = 256;
+    int scores_grid = 0;                        // tests (SPY_HIP_SCORES_GRID when the engine is made): workgroups of order 1's score kernel, and no one-launch attention; 0: as the product does
     float theta_scale = 0.0f;
     // op-by-op path scratch (sized lazily for the largest chunk seen)
     uint8_t *ops_buf = nullptr; size_t ops_bytes = 0;

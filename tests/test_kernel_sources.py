@@ -34,3 +34,13 @@ def test_single_token_attention_reads_no_keys_behind_the_last_one(tmp_path):
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr
     kernel = open(os.path.join(ROOT, "spy_amd", "csrc", "attn_short.hip")).read()
     assert kernel.count("xf_keys_before(st != nullptr") == 1 and kernel.count("xf_row_pieces_before(st != nullptr") == 1 and kernel.count("key_piece(0, keys0)") == 1
+
+
+def test_launches_of_a_single_token_pass_read_no_environment():
+    """What enqueues the kernels of a single-token pass, eagerly or into a graph that outlives the call, asks the engine and not the environment: a variable set
+    after a capture would change eager passes but not replays."""
+    engine = open(os.path.join(ROOT, "spy_amd", "csrc", "engine.hip")).read()
+    body = engine[engine.index("static int enqueue_one("):engine.index("// ---- passes over several tokens")]
+    assert "xattn_scores_kernel" in body and "spy_attn_short" in body and "static int enqueue_pass_any(" in body
+    for name, text in [("engine.hip", body)] + [(n, open(os.path.join(ROOT, "spy_amd", "csrc", n)).read()) for n in ("exact_launch.cuh", "decode_launch.cuh", "attn_short.hip")]:
+        assert "getenv" not in text, name

@@ -1463,7 +1463,11 @@ int xt_dispatch(hipStream_t st, const xt_args &a, int nmat) {
     static const int of_rest[4] = {0, 60, 100, 132};
     const int rest = a.ncg > 4 ? a.ncg % 4 : 0;
     // Q8_0's first two tiles have room for four workgroups on a compute unit, and its chunks are larger: 4096 x 11008 x 150 100.5 -> 93.1 us, 4096 x 4096 x 150 42.2 -> 39.4,
-    // 12288 x 4096 x 180 116 -> 108 with its own increments.  98 for the third: 22016 x 4096 x 128 goes to the fourth, Q8_0 142 -> 128, Q4_0 129 -> 122.
+    // 12288 x 4096 x 180 116 -> 108 with its own increments.
+    // The third tile's increment: another workgroup on a compute unit that has 8 to 16 takes 95 .. 96 on the scale of the fourth's 165, in either type; but beyond six the
+    // rule counts parts of workgroups, where the third is in truth still rounded up (22016 x 4096 x 128, 10.75 of them: 130.7 us, the line between ten and twelve says 125).  Every tile timed
+    // at 322 shapes (4096 .. 32000 x 4096 and 4096 x 11008 by 4 .. 512 rows, both types): the choice is 0.12 % slower than the best tile in the mean with 97 or 98, 0.28 % with 96
+    // (fourth against third tile: 22016 x 4096 x 128 Q4_0 124 / 132 us, Q8_0 132 / 145; 11008 x 4096 x 256 Q8_0 127 / 142), 0.49 % with 100 (4096 x 11008 x 100 Q4_0: third tile 73.4, mixed fourth 85.1).
     constexpr bool Q8 = WT == SPY_HIP_Q8_0;
     const xt_cost c[5] = {{16, 1, 44, Q8 ? 50 : 44}, {32, 1, 106, Q8 ? 64 : 56}, {32, 2, 173, 98}, {32, 4, 288, 165}, {32, 4, 288, 165, of_rest[rest]}};
     switch (xt_pick(a, nmat, c, rest ? 5 : 4)) {

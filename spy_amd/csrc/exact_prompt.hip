@@ -10,6 +10,8 @@
 //     call): the host's fp16 dot runs its 32 accumulators over whole chunks of 32 elements while i + 32 < n and adds
 //     the last 1..32 elements one by one, and the softmax sum adds the last n % 4 terms one by one.  A call may therefore
 //     be cut into chunks of query rows without moving a rounding.
+// An infinite or NaN V element is added in by every row that sees its token.  The host also multiplies it with the masked zeros of the rows before it in the same
+// pass, which makes their sums NaN; here they keep their finite sums, but for those that share its tile of 32 rows.
 // Values that cannot occur are not looked after: the fp16 caches are written by this library's float -> half
 // conversion, which never produces the pattern 0xFFFF that the host's conversion table maps to 0 (conversion.h:39-41).
 #include "common.cuh"

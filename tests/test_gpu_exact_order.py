@@ -346,6 +346,82 @@ def test_exact_prompt_attention_unaligned_v(hip):
     _same_bits(outs[1], outs[0], "V^T cache at an odd element")
 
 
+def _special_attention_case(kind, H_, past, T, n_ctx):
+    """q, K cache, V^T cache with values that end chains of fma differently when one of them flushes, reorders or leaves out: fp16 subnormals everywhere, scores of
+    minus infinity, infinities and NaN in cached values that every query row sees (the host's Softmax stops at a row whose largest score or sum is none, so
+    those are not among them)."""
+    hd, n_kv, d = 128, past + T, H_ * 128
+    rng = np.random.default_rng(past * 1000 + T)
+    q = rng.standard_normal((T, H_, hd)).astype(np.float32)
+    kc, vc = np.zeros((n_ctx, d), np.float16), np.full((d, n_ctx), np.nan, np.float16)
+    kc[:n_kv] = rng.standard_normal((n_kv, d)).astype(np.float16)
+    vc[:, :n_kv] = rng.standard_normal((d, n_kv)).astype(np.float16)
+    if kind == "subnormal":
+        tiny = lambda shape: (rng.integers(-1023, 1024, shape) * 2.0 ** -24)
+        q = np.where(rng.random(q.shape) < 0.5, tiny(q.shape), q * 300).astype(np.float32)
+        kc[:n_kv] = np.where(rng.random((n_kv, d)) < 0.5, tiny((n_kv, d)), kc[:n_kv].astype(np.float32) * 3).astype(np.float16)
+        vc[:, :n_kv] = np.where(rng.random((d, n_kv)) < 0.7, tiny((d, n_kv)), vc[:, :n_kv].astype(np.float32)).astype(np.float16)
+    elif kind == "minus infinity":                                  # elements 5 (accumulators) and 101 (scalar tail) of a head, queries positive there
+        q[:, :, [5, 101]] = np.abs(q[:, :, [5, 101]]) + 0.25
+        kc[1:n_kv:3, 5::hd] = -np.inf
+        kc[2:n_kv:7, 101::hd] = -np.inf
+    else:                                                           # cached values, most of them multiplied by an ordinary probability, some by 0
+        q[(np.arange(T)[:, None] + np.arange(H_)) % 2 == 1] *= 40
+        for r, value in ((0, np.inf), (17, -np.inf), (40, np.nan), (66, np.inf), (66, -np.inf), (127, np.inf)):
+            vc[r::hd, rng.integers(0, past + 1)] = value
+    return q, kc, vc
+
+
+def _oracle_attention(oracle, q, kc, vc, past, T, n_ctx, scale):
+    H_, hd, n_kv = q.shape[1], 128, past + T
+    d = H_ * hd
+    mask = np.where(np.arange(n_ctx)[None, :] <= (np.arange(T)[:, None] + past), 0.0, -np.inf).astype(np.float32)
+    S_o, P_o, O_o = np.zeros((H_, T, n_kv), np.float32), np.zeros((H_, T, n_kv), np.float32), np.zeros((H_, T, hd), np.float32)
+    assert oracle.spy_o_matmul(B(O.tensor(kc.view(np.uint16), O.F16, [hd, n_kv, H_], nb=[2, 2 * d, 2 * hd])),
+                               B(O.tensor(q, O.F32, [hd, T, H_], nb=[4, 4 * d, 4 * hd])), B(O.tensor(S_o, O.F32, [n_kv, T, H_])), 4) == 0
+    assert oracle.spy_o_softmax(B(O.tensor(S_o, O.F32, [n_kv, T, H_])), B(O.tensor(mask, O.I32, [n_ctx, T])), B(O.tensor(P_o, O.F32, [n_kv, T, H_])), scale) == 0
+    assert oracle.spy_o_matmul(B(O.tensor(vc.view(np.uint16), O.F16, [n_kv, hd, H_], nb=[2, 2 * n_ctx, 2 * n_ctx * hd])),
+                               B(O.tensor(P_o, O.F32, [n_kv, T, H_])), B(O.tensor(O_o, O.F32, [hd, T, H_])), 4) == 0
+    return np.ascontiguousarray(O_o.transpose(1, 0, 2)).reshape(T, d)
+
+
+def _same_bits_or_both_nan(got, want, what):
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan), "%s: NaN in %d outputs, expected in %d, %d places differ" % (what, np.isnan(got).sum(), nan.sum(), (np.isnan(got) != nan).sum())
+    _same_bits(np.where(nan, 0, got), np.where(nan, 0, want), what)
+
+
+@pytest.mark.parametrize("kind", ["subnormal", "minus infinity", "cached infinities and NaN"])
+@pytest.mark.parametrize("H_,past,T,n_ctx", [(2, 70, 40, 128), (1, 32, 65, 128), (2, 300, 17, 320), (1, 2040, 20, 2080)])
+def test_exact_prompt_attention_of_special_values(hip, oracle, kind, H_, past, T, n_ctx):
+    """The causal attention kernels, whose fmas are matrix instructions, against the oracle's bits (NaN: in the same places)."""
+    from tests.gpu_util import dev, dev_empty, call
+    q, kc, vc = _special_attention_case(kind, H_, past, T, n_ctx)
+    scale = float(1.0 / np.sqrt(128))
+    want = _oracle_attention(oracle, q, kc, vc, past, T, n_ctx, scale)
+    assert kind != "cached infinities and NaN" or (np.isnan(want).any() and np.isinf(want).any())
+    L = hip.load()
+    need = L.spy_hip_prompt_attention_exact_scratch_size(T, H_, past)
+    dq, dk, dv, sc, out = dev(q), dev(kc.view(np.uint16)), dev(vc.view(np.uint16)), dev_empty(need, 0xFF), dev_empty(want.nbytes, 0xEE)
+    call(L.spy_hip_prompt_attention_exact, None, dq.ptr, dk.ptr, dv.ptr, out.ptr, T, H_, 128, past, n_ctx, past + T, scale, sc.ptr, need)
+    _same_bits_or_both_nan(out.download(np.float32).reshape(want.shape), want, "%s, %d on %d" % (kind, T, past))
+
+
+@pytest.mark.parametrize("kind", ["subnormal", "minus infinity", "cached infinities and NaN"])
+@pytest.mark.parametrize("n_kv,n_ctx", [(33, 64), (300, 320), (576, 576), (577, 640), (1300, 1344)])
+def test_single_token_attention_of_special_values(hip, oracle, kind, n_kv, n_ctx):
+    """One token in order 1, one launch up to 576 cached tokens and two beyond, against the oracle's bits (NaN: in the same places)."""
+    from tests.gpu_util import dev, dev_empty, call
+    H_ = 3
+    q, kc, vc = _special_attention_case(kind, H_, n_kv - 1, 1, n_ctx)
+    q16 = q.astype(np.float16)
+    want = _oracle_attention(oracle, q16.astype(np.float32), kc, vc, n_kv - 1, 1, n_ctx, float(np.float32(1.0) / np.sqrt(np.float32(128))))
+    dq, dk, dv = dev(q16.view(np.uint16)), dev(kc.view(np.uint16)), dev(vc.view(np.uint16))
+    ds, do = dev_empty(H_ * n_ctx * 4, 0xEE), dev_empty(H_ * 128 * 4, 0xEE)
+    call(hip.load().spy_hip_attn_decode, None, 1, dq.ptr, dk.ptr, dv.ptr, H_, n_kv, n_ctx, ds.ptr, do.ptr)
+    _same_bits_or_both_nan(do.download(np.float32), want.reshape(-1), "%s, %d cached" % (kind, n_kv))
+
+
 def test_exact_prompt_attention_wants_its_probabilities_on_the_16_byte_grid(hip):
     """The library's own entry behind spy_hip_prompt_attention_exact: the product reads the probabilities in 16-byte pieces, so a place for them 8 bytes off that
     grid is refused, as it is for the other operands; one on the grid is taken."""

@@ -56,34 +56,14 @@ static __global__ __launch_bounds__(XP_THREADS) void xattn_short_kernel(const de
         const int rot = 4 * key;
         float sum[8];
 #pragma unroll
-        for (int i = 0; i < 3; i++) {
-            const uint4 kv = kp[(4 * i + part + rot) & 15], qv = s_qh[4 * i + part];
-            const uint32_t kw[4] = {kv.x, kv.y, kv.z, kv.w}, qw[4] = {qv.x, qv.y, qv.z, qv.w};
+        for (int l = 0; l < 8; l++) sum[l] = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                sum[2 * e] = fmaf(h2f((uint16_t)(kw[e] & 0xFFFFu)), h2f((uint16_t)(qw[e] & 0xFFFFu)), i == 0 ? 0.0f : sum[2 * e]);
-                sum[2 * e + 1] = fmaf(h2f((uint16_t)(kw[e] >> 16)), h2f((uint16_t)(qw[e] >> 16)), i == 0 ? 0.0f : sum[2 * e + 1]);
-            }
-        }
-        // sum[0] += sum[2], sum[1] += sum[3]; sum[0] += sum[1] over the four threads, then the tree of FP16::block_reduce
-#pragma unroll
-        for (int l = 0; l < 8; l++) {
-            sum[l] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum[l]), 0x4E, 0xF, 0xF, true));        // quad_perm [2, 3, 0, 1]
-            sum[l] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum[l]), 0xB1, 0xF, 0xF, true));        // quad_perm [1, 0, 3, 2]
-        }
-        const float u0 = sum[0] + sum[4], u1 = sum[1] + sum[5], u2 = sum[2] + sum[6], u3 = sum[3] + sum[7];
-        const float v0 = u0 + u1, v1 = u2 + u3, simd = v0 + v1;
+        for (int i = 0; i < 3; i++) xa_fma8(sum, kp[(4 * i + part + rot) & 15], s_qh[4 * i + part]);
+        xa_quad(sum);
+        const float simd = xa_tree8(sum);
         float tail = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint4 kv = kp[(12 + j + rot) & 15], qv = s_qh[12 + j];
-            const uint32_t kw[4] = {kv.x, kv.y, kv.z, kv.w}, qw[4] = {qv.x, qv.y, qv.z, qv.w};
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                tail = fmaf(h2f((uint16_t)(kw[e] & 0xFFFFu)), h2f((uint16_t)(qw[e] & 0xFFFFu)), tail);
-                tail = fmaf(h2f((uint16_t)(kw[e] >> 16)), h2f((uint16_t)(qw[e] >> 16)), tail);
-            }
-        }
+        for (int j = 0; j < 4; j++) tail = xa_tail8(tail, kp[(12 + j + rot) & 15], s_qh[12 + j]);
         if (part == 0) {
             s_t[key] = (tail + simd) * scale;
             if (dgrp == 0) scores[(size_t)hd_ * n_ctx + key] = s_t[key];      // as the launch of its own leaves them
@@ -107,9 +87,7 @@ static __global__ __launch_bounds__(XP_THREADS) void xattn_short_kernel(const de
 #pragma unroll
         for (int u = 0; u < (XF_MAX / 4 + 63) / 64; u++) {
             const int g = lane + 64 * u;
-            const float4 v = g < ngrp ? *(const float4 *)(s_e + 4 * g) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            const float v1 = v.x + v.y, v2 = v.z + v.w;
-            s_grp[g] = v1 + v2;
+            s_grp[g] = xa_group(g < ngrp ? *(const float4 *)(s_e + 4 * g) : make_float4(0.0f, 0.0f, 0.0f, 0.0f));
         }
         __builtin_amdgcn_wave_barrier();
         float sum = 0.0f;
@@ -132,21 +110,13 @@ static __global__ __launch_bounds__(XP_THREADS) void xattn_short_kernel(const de
     if (lane < 32) s_tail[wave][lane] = f2h(s_e[32 * nfull + lane] * inv);
     float acc = 0.0f;
     for (int i = 0; i < nfull; i++) acc = fmaf(h2f(vr[32 * i + cl]), h2f(f2h(s_e[32 * i + cl] * inv)), acc);
-    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc), __float_as_uint(acc), false, false);
-    acc = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-#define XP_ADD(CTRL) acc += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc), CTRL, 0xF, 0xF, true));
-    XP_ADD(0x128) XP_ADD(0x124) XP_ADD(0xB1) XP_ADD(0x4E)
-#undef XP_ADD
+    acc = xa_tree32(acc);
     __builtin_amdgcn_wave_barrier();
     float tail = 0.0f;
     xp_u4 tv[4], tq[4];
 #pragma unroll
     for (int u = 0; u < 4; u++) { tv[u] = *(const xp_u4 *)(vr + 32 * nfull + 8 * u); tq[u] = *(const xp_u4 *)&s_tail[wave][8 * u]; }
-#pragma unroll
-    for (int e = 0; e < 32; e++) {
-        const uint32_t wv = tv[e >> 3][(e >> 1) & 3], wq = tq[e >> 3][(e >> 1) & 3];
-        if (e < ntail) tail = fmaf(h2f((uint16_t)(e & 1 ? wv >> 16 : wv & 0xFFFFu)), h2f((uint16_t)(e & 1 ? wq >> 16 : wq & 0xFFFFu)), tail);
-    }
+    XA_TAIL32(tail, tv, tq, ntail)
     if (cl == 0) attn_out[hd_ * 128 + dgrp * 16 + r16] = tail + acc;
 }
 

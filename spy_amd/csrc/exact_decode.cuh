@@ -471,6 +471,63 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(xg_args a) {
 // scalar tail over elements 96..127 (a product of two fp16 values is exact in fp32, so `tail += a * b` is the fma it is
 // written as here), result = tail + simd.  Stored: t = dot * scale (mask 0, then * scale: non-linear.cpp:141-150).
 typedef uint32_t xp_u4 __attribute__((ext_vector_type(4)));
+// ---- what the attention kernels of one token (the two below, attn_short.hip) share: the order of Dot<FP16,FP16> lies here and nowhere else.  A product of two fp16
+// values is exact in fp32, so `sum + a * b` is the fma it is written as.
+// eight elements of a key or query, packed in four words, onto the eight accumulators l of one (chunk, j)
+static __device__ __forceinline__ void xa_fma8(float (&sum)[8], const uint4 kv, const uint4 qv) {
+    const uint32_t kw[4] = {kv.x, kv.y, kv.z, kv.w}, qw[4] = {qv.x, qv.y, qv.z, qv.w};
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        sum[2 * e] = fmaf(h2f((uint16_t)(kw[e] & 0xFFFFu)), h2f((uint16_t)(qw[e] & 0xFFFFu)), sum[2 * e]);
+        sum[2 * e + 1] = fmaf(h2f((uint16_t)(kw[e] >> 16)), h2f((uint16_t)(qw[e] >> 16)), sum[2 * e + 1]);
+    }
+}
+// eight elements of the scalar tail, one after the other
+static __device__ __forceinline__ float xa_tail8(float tail, const uint4 kv, const uint4 qv) {
+    const uint32_t kw[4] = {kv.x, kv.y, kv.z, kv.w}, qw[4] = {qv.x, qv.y, qv.z, qv.w};
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        tail = fmaf(h2f((uint16_t)(kw[e] & 0xFFFFu)), h2f((uint16_t)(qw[e] & 0xFFFFu)), tail);
+        tail = fmaf(h2f((uint16_t)(kw[e] >> 16)), h2f((uint16_t)(qw[e] >> 16)), tail);
+    }
+    return tail;
+}
+// first two steps of FP16::block_reduce where four adjacent lanes hold j = 0 .. 3: sum[0] += sum[2], sum[1] += sum[3]; sum[0] += sum[1]
+static __device__ __forceinline__ void xa_quad(float (&sum)[8]) {
+#pragma unroll
+    for (int l = 0; l < 8; l++) {
+        sum[l] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum[l]), 0x4E, 0xF, 0xF, true));        // quad_perm [2, 3, 0, 1]
+        sum[l] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum[l]), 0xB1, 0xF, 0xF, true));        // quad_perm [1, 0, 3, 2]
+    }
+}
+// its last three
+static __device__ __forceinline__ float xa_tree8(const float (&sum)[8]) {
+    const float u0 = sum[0] + sum[4], u1 = sum[1] + sum[5], u2 = sum[2] + sum[6], u3 = sum[3] + sum[7];
+    const float v0 = u0 + u1, v1 = u2 + u3;
+    return v0 + v1;
+}
+// a group of four of std::reduce's running sum
+static __device__ __forceinline__ float xa_group(const float4 v) {
+    const float v1 = v.x + v.y, v2 = v.z + v.w;
+    return v1 + v2;
+}
+// block_reduce of 32 accumulators 8 j + l that 32 lanes hold: sum[0] += sum[2], sum[1] += sum[3] (lane ^ 16); sum[0] += sum[1] (^ 8); t_l = sum[0][l] + sum[0][l + 4] (^ 4);
+// t_0 + t_1, t_2 + t_3 (^ 1); (t_0 + t_1) + (t_2 + t_3) (^ 2); inside a row of 16 as rotations where the values are periodic already
+static __device__ __forceinline__ float xa_tree32(float acc) {
+    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc), __float_as_uint(acc), false, false);
+    acc = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+#define XP_ADD(CTRL) acc += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc), CTRL, 0xF, 0xF, true));
+    XP_ADD(0x128) XP_ADD(0x124) XP_ADD(0xB1) XP_ADD(0x4E)
+#undef XP_ADD
+    return acc;
+}
+// the scalar tail of P.V^T: the first ntail of 32 elements tv . tq onto tail, one after the other.  A macro because the steps stay branches that way: in a function the
+// compiler makes them selections, which doubles the chain.
+#define XA_TAIL32(tail, tv, tq, ntail) \
+    _Pragma("unroll") for (int e = 0; e < 32; e++) { \
+        const uint32_t wv = tv[e >> 3][(e >> 1) & 3], wq = tq[e >> 3][(e >> 1) & 3]; \
+        if (e < ntail) tail = fmaf(h2f((uint16_t)(e & 1 ? wv >> 16 : wv & 0xFFFFu)), h2f((uint16_t)(e & 1 ? wq >> 16 : wq & 0xFFFFu)), tail); \
+    }
 #define XS_THREADS 1024
 #define XS_TOK 18
 #define XS_NLD 9                                        // pieces per thread requested together: 1024 x 9 x 16 bytes = 18 tokens of 32 heads
@@ -538,40 +595,18 @@ __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_stat
 #pragma unroll
                 for (int j = 0; j < NJ; j++) {
                     const int jj = part + j * SP;
-                    const uint4 kv = kp[(4 * i + jj + rot) & 15], qv = qp[4 * i + jj];
-                    const uint32_t kw[4] = {kv.x, kv.y, kv.z, kv.w}, qw[4] = {qv.x, qv.y, qv.z, qv.w};
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        sum[j][2 * e] = fmaf(h2f((uint16_t)(kw[e] & 0xFFFFu)), h2f((uint16_t)(qw[e] & 0xFFFFu)), sum[j][2 * e]);
-                        sum[j][2 * e + 1] = fmaf(h2f((uint16_t)(kw[e] >> 16)), h2f((uint16_t)(qw[e] >> 16)), sum[j][2 * e + 1]);
-                    }
+                    xa_fma8(sum[j], kp[(4 * i + jj + rot) & 15], qp[4 * i + jj]);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
-            auto other = [](float v, auto ctrl) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xF, 0xF, true)); };
-            // sum[0] += sum[2], sum[1] += sum[3]; sum[0] += sum[1]
+            if constexpr (SP == 1) {
 #pragma unroll
-            for (int l = 0; l < 8; l++) {
-                if constexpr (SP == 1) { sum[0][l] += sum[2][l]; sum[1][l] += sum[3][l]; sum[0][l] += sum[1][l]; }
-                else {
-                    sum[0][l] += other(sum[0][l], std::integral_constant<int, 0x4E>{});        // quad_perm [2, 3, 0, 1]
-                    sum[0][l] += other(sum[0][l], std::integral_constant<int, 0xB1>{});             // quad_perm [1, 0, 3, 2]
-                }
-            }
-            const float u0 = sum[0][0] + sum[0][4], u1 = sum[0][1] + sum[0][5], u2 = sum[0][2] + sum[0][6], u3 = sum[0][3] + sum[0][7];
-            const float v0 = u0 + u1, v1 = u2 + u3;
-            const float simd = v0 + v1;
+                for (int l = 0; l < 8; l++) { sum[0][l] += sum[2][l]; sum[1][l] += sum[3][l]; sum[0][l] += sum[1][l]; }
+            } else xa_quad(sum[0]);
+            const float simd = xa_tree8(sum[0]);
             float tail = 0.0f;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint4 kv = kp[(12 + j + rot) & 15], qv = qp[12 + j];
-                const uint32_t kw[4] = {kv.x, kv.y, kv.z, kv.w}, qw[4] = {qv.x, qv.y, qv.z, qv.w};
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    tail = fmaf(h2f((uint16_t)(kw[e] & 0xFFFFu)), h2f((uint16_t)(qw[e] & 0xFFFFu)), tail);
-                    tail = fmaf(h2f((uint16_t)(kw[e] >> 16)), h2f((uint16_t)(qw[e] >> 16)), tail);
-                }
-            }
+            for (int j = 0; j < 4; j++) tail = xa_tail8(tail, kp[(12 + j + rot) & 15], qp[12 + j]);
             if (part == 0) scores[(size_t)hh * n_ctx + t0 + tt] = (tail + simd) * scale;
         }
     };
@@ -676,9 +711,7 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
     for (int u = 0; u < 2; u++) {
         const int g = tid + u * XP_THREADS;
         if (g < ngrp) {
-            const float4 v = *(const float4 *)(s_e + 4 * g);
-            const float v1 = v.x + v.y, v2 = v.z + v.w;
-            s_grp[xg_seg_at(g)] = v1 + v2;
+            s_grp[xg_seg_at(g)] = xa_group(*(const float4 *)(s_e + 4 * g));
         }
     }
     if (tid < 32) for (int g = ngrp + tid; g < ((ngrp + 31) & ~31); g += 32) s_grp[xg_seg_at(g)] = 0.0f;
@@ -749,21 +782,9 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
         }
         for (; i < nfull; i++) acc = fmaf((float)vr[32 * i], (float)pr[32 * i], acc);
         XSTAMP(dbg, 6);
-        // sum[0] += sum[2], sum[1] += sum[3] (lane ^ 16); sum[0] += sum[1] (^ 8); t_l = sum[0][l] + sum[0][l + 4] (^ 4); t_0 + t_1, t_2 + t_3 (^ 1);
-        // (t_0 + t_1) + (t_2 + t_3) (^ 2); inside a row of 16 as rotations where the values are periodic already
-        const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc), __float_as_uint(acc), false, false);
-        acc = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-#define XP_ADD(CTRL) acc += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc), CTRL, 0xF, 0xF, true));
-        XP_ADD(0x128) XP_ADD(0x124) XP_ADD(0xB1) XP_ADD(0x4E)
-#undef XP_ADD
-        // the scalar tail: elements 32 nfull .. n_kv - 1, one after the other (a product of two fp16 values is exact in fp32: the fma is
-        // `tail + v * p`)
+        acc = xa_tree32(acc);
         float tail = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 32; e++) {
-            const uint32_t wv = tv[e >> 3][(e >> 1) & 3], wq = tq[e >> 3][(e >> 1) & 3];
-            if (e < ntail) tail = fmaf(h2f((uint16_t)(e & 1 ? wv >> 16 : wv & 0xFFFFu)), h2f((uint16_t)(e & 1 ? wq >> 16 : wq & 0xFFFFu)), tail);
-        }
+        XA_TAIL32(tail, tv, tq, ntail)                               // elements 32 nfull .. n_kv - 1
         if (cl == 0) attn_out[hd_ * 128 + dgrp * 16 + r16] = tail + acc;
         XSTAMP(dbg, 7);
     }

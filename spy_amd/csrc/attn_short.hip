@@ -12,6 +12,8 @@
 // What bounds it: the chain launch, keys and V^T rows (one wait for both), dots, exponentials (a gather), running sum, walk.
 #define XF_NP (XF_MAX * 16 / XP_THREADS)   // 16-byte pieces of keys per thread
 static size_t xattn_short_lds(int n_ctx) { return (size_t)(n_ctx < XF_MAX ? n_ctx : XF_MAX) * 256 + 16 * 96 * 2; }      // the keys; later the rows of V^T (16 rows of cap + 32 .. 96 halfs)
+// IN_STATE: the position is st->pos, else pos_imm (decided when the kernel is compiled: asked in the kernel it cost the engine's launches 0.15 of 5 us)
+template <bool IN_STATE>
 static __global__ __launch_bounds__(XP_THREADS) void xattn_short_kernel(const dev_state *st, int pos_imm, const uint16_t *__restrict__ q16, const uint16_t *kc, const uint16_t *vc,
                                                                  float *__restrict__ scores, float *attn_out, const float *__restrict__ lut, int n_ctx, float scale) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -26,18 +28,18 @@ static __global__ __launch_bounds__(XP_THREADS) void xattn_short_kernel(const de
     uint4 *s_k = (uint4 *)smem;                                       // [token][16 pieces], rotated by 4 pieces per token against bank conflicts
     uint16_t *s_v = (uint16_t *)smem;                                 // the rows of V^T, once the keys have been read
     const uint16_t *vrow = vc + (size_t)(hd_ * 128 + dgrp * 16 + wave) * n_ctx;
-    // Keys first, then the rows of V^T.  Where the position is on its way itself (st), the first piece of either does not wait for it: 64 keys and 512 elements
+    // Keys first, then the rows of V^T.  Where the position is on its way itself, the first piece of either does not wait for it: 64 keys and 512 elements
     // of a row, as far as the cache goes; what lies behind the last token is not used.  Where it is a number, nothing behind the last token is asked for (attn_reach.h).
     xp_u4 kr[XF_NP], vb, vb1, qr;
     auto key_piece = [&](int u, int n) {
         const int c = xf_piece(tid + u * XP_THREADS, n * 16);
         kr[u] = *(const xp_u4 *)(kc + (size_t)(c >> 4) * d + hd_ * 128 + (c & 15) * 8);
     };
-    const int keys0 = xf_keys_before(st != nullptr, pos_imm, cap);
+    const int keys0 = xf_keys_before(IN_STATE, pos_imm, cap);
     key_piece(0, keys0);
     if (tid < 16) qr = *(const xp_u4 *)(q16 + hd_ * 128 + tid * 8);
-    const int n_kv = st ? min(st->pos + 1, cap) : keys0, npiece = n_kv * 16, last_piece = (n_kv - 1) >> 3;
-    vb = *(const xp_u4 *)(vrow + (size_t)xf_piece(lane, xf_row_pieces_before(st != nullptr, pos_imm, n_ctx)) * 8);
+    const int n_kv = IN_STATE ? min(st->pos + 1, cap) : keys0, npiece = n_kv * 16, last_piece = (n_kv - 1) >> 3;
+    vb = *(const xp_u4 *)(vrow + (size_t)xf_piece(lane, xf_row_pieces_before(IN_STATE, pos_imm, n_ctx)) * 8);
     if (last_piece >= 64) vb1 = *(const xp_u4 *)(vrow + (size_t)xf_piece(64 + lane, last_piece + 1) * 8);
 #pragma unroll
     for (int u = 1; u < XF_NP; u++) if (u * XP_THREADS < npiece) key_piece(u, n_kv);
@@ -120,10 +122,15 @@ static __global__ __launch_bounds__(XP_THREADS) void xattn_short_kernel(const de
     if (cl == 0) attn_out[hd_ * 128 + dgrp * 16 + r16] = tail + acc;
 }
 
-int spy_attn_short_prepare(int n_ctx) { return spy_raise_lds_limit((const void *)xattn_short_kernel, xattn_short_lds(n_ctx)); }
+int spy_attn_short_prepare(int n_ctx) {
+    const int rc = spy_raise_lds_limit((const void *)xattn_short_kernel<true>, xattn_short_lds(n_ctx));
+    return rc ? rc : spy_raise_lds_limit((const void *)xattn_short_kernel<false>, xattn_short_lds(n_ctx));
+}
 // scores: [n_head][n_ctx], as the launch of xattn_scores_kernel leaves them
 int spy_attn_short(hipStream_t st, const dev_state *state, int pos_imm, const uint16_t *q16, const uint16_t *kc, const uint16_t *vc, float *scores, float *out,
                    const float *lut, int n_head, int n_ctx, float scale) {
-    xattn_short_kernel<<<dim3((unsigned)(n_head * 8)), dim3(XP_THREADS), xattn_short_lds(n_ctx), st>>>(state, pos_imm, q16, kc, vc, scores, out, lut, n_ctx, scale);
+    const dim3 grid((unsigned)(n_head * 8)), block(XP_THREADS);
+    if (state) xattn_short_kernel<true><<<grid, block, xattn_short_lds(n_ctx), st>>>(state, pos_imm, q16, kc, vc, scores, out, lut, n_ctx, scale);
+    else xattn_short_kernel<false><<<grid, block, xattn_short_lds(n_ctx), st>>>(state, pos_imm, q16, kc, vc, scores, out, lut, n_ctx, scale);
     return SPY_LAUNCH_RC();
 }

@@ -33,7 +33,7 @@ def test_single_token_attention_reads_no_keys_behind_the_last_one(tmp_path):
     r = subprocess.run([out], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr
     kernel = open(os.path.join(ROOT, "spy_amd", "csrc", "attn_short.hip")).read()
-    assert kernel.count("xf_keys_before(st != nullptr") == 1 and kernel.count("xf_row_pieces_before(st != nullptr") == 1 and kernel.count("key_piece(0, keys0)") == 1
+    assert kernel.count("xf_keys_before(IN_STATE") == 1 and kernel.count("xf_row_pieces_before(IN_STATE") == 1 and kernel.count("if (state) xattn_short_kernel<true>") == 1 and kernel.count("key_piece(0, keys0)") == 1
 
 
 def test_launches_of_a_single_token_pass_read_no_environment():

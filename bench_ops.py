@@ -272,7 +272,7 @@ def main():
                 kv = 2 * n_kv * cfg.n_embd * 2
                 if mode == "host_order":
                     s_us, p_us = eng.kernel_time_us("scores", args.reps), eng.kernel_time_us("pv", args.reps)
-                    us, nb, label = s_us + p_us, kv, "host summation order: `xattn_scores_kernel` %.2f + `xattn_pv_kernel` %.2f" % (s_us, p_us)
+                    us, nb, label = s_us + p_us, kv, "host summation order: " + ("`xattn_scores_kernel` %.2f + `xattn_pv_kernel` %.2f" % (s_us, p_us) if s_us else "`xattn_short_kernel`")
                 elif split:
                     s_us, p_us = eng.kernel_time_us("scores", args.reps), eng.kernel_time_us("pv", args.reps)
                     us, nb, label = s_us + p_us, kv, "`attn_scores_kernel` %.2f + `attn_pv_kernel` %.2f" % (s_us, p_us)

@@ -34,7 +34,7 @@ int spy_exact_luts(const float **lut);           // exact_order.hip
 // summation order of the next single-token pass: the host backend's when the engine is set to it or the library-wide
 // exact-order switch is on (and the exact kernels take the model), else this backend's own
 static int pass_order(const spy_hip_llama *m) { return (m->exact_ok && (m->order == 1 || spy_exact_on())) ? 1 : 0; }
-static int enqueue_pass_any(spy_hip_llama *m, hipStream_t st, int mode);
+static int enqueue_pass_any(spy_hip_llama *m, hipStream_t st, int mode, int kv_bound);
 static void drop_graphs(spy_hip_llama *m) {
     for (auto &kind : m->graphs)
         for (auto &g : kind) {
@@ -148,7 +148,7 @@ extern "C" int spy_hip_llama_create(const spy_hip_llama_desc *desc, spy_hip_llam
             m->attn_fused = ok;
         }
     }
-    if (!rc && fused_ok(m)) { m->dry = true; rc = enqueue_pass_any(m, m->own_stream, PASS_GREEDY); m->dry = false; }   // sizes the persistent grids
+    if (!rc && fused_ok(m)) { m->dry = true; rc = enqueue_pass_any(m, m->own_stream, PASS_GREEDY, 0); m->dry = false; }   // sizes the persistent grids
     // the host backend's summation order: cos / sin of every position from the host's libm (theta_0 = pos, theta_{k+1} =
     // theta_k * theta_scale in fp32, non-linear.cpp:304-309), the exp / silu tables, shapes the kernels take
     if (!rc && fused_ok(m) && m->wave && m->hd == 128 && c.n_embd % 128 == 0 && c.n_ff % 128 == 0 && c.n_ff <= 16384 &&
@@ -171,7 +171,7 @@ extern "C" int spy_hip_llama_create(const spy_hip_llama_desc *desc, spy_hip_llam
         if (!rc) {
             m->exact_ok = true;
             m->order = 1;
-            m->dry = true; rc = enqueue_pass_any(m, m->own_stream, PASS_GREEDY); m->dry = false;
+            m->dry = true; rc = enqueue_pass_any(m, m->own_stream, PASS_GREEDY, 0); m->dry = false;
             if (rc == SPY_HIP_EUNSUPPORTED) { rc = 0; m->exact_ok = false; m->order = 0; }
             const char *env = getenv("SPY_HIP_ORDER");                       // "own": this backend's own summation order by default
             if (env && env[0] == 'o') m->order = 0;
@@ -235,10 +235,12 @@ static bool fused_ok(const spy_hip_llama *m) {
     return true;
 }
 
-static int enqueue_one(spy_hip_llama *m, hipStream_t st, int which, int il) {
+// order 1: one launch for the attention of passes that see no more than kv_bound cached tokens (0: not known)
+static bool attn_one_launch(const spy_hip_llama *m, int kv_bound) { return kv_bound > 0 && kv_bound <= XF_MAX && !m->scores_grid; }
+static int enqueue_one(spy_hip_llama *m, hipStream_t st, int which, int il, int kv_bound) {
     const spy_hip_llama_desc &c = m->desc;
     if (pass_order(m) == 1 || (m->dry && m->order == 1)) {      // the host backend's summation order: six launches per layer, five where the cache is short
-        const bool one_launch = m->kv_bound > 0 && m->kv_bound <= XF_MAX && !m->scores_grid;
+        const bool one_launch = attn_one_launch(m, kv_bound);
         if (which == K_SCORES) {
             if (m->dry || one_launch) return 0;
             // one workgroup per compute unit; tests have fewer, so that a workgroup's share of the tokens takes several rounds of
@@ -330,8 +332,8 @@ static int enqueue_embed(spy_hip_llama *m, hipStream_t st) {
 
 // One single-token pass.  PASS_LOGITS: embedding, layers, head (spy_hip_llama_forward).  PASS_GREEDY: layers, head, and one
 // launch that samples, advances the position and prepares the next pass's embedding and RoPE table -- the first pass of a
-// greedy run is preceded by enqueue_embed.
-static int enqueue_pass_any(spy_hip_llama *m, hipStream_t st, int mode) {
+// greedy run is preceded by enqueue_embed.  kv_bound: as in enqueue_one.
+static int enqueue_pass_any(spy_hip_llama *m, hipStream_t st, int mode, int kv_bound) {
     const spy_hip_llama_desc &c = m->desc;
     auto sample = [&](bool embed_next) {
         sample_advance_kernel<<<dim3(1), dim3(1024), 0, st>>>(m->st, m->logits, c.n_vocab, m->tokens_out, m->max_out,
@@ -341,8 +343,8 @@ static int enqueue_pass_any(spy_hip_llama *m, hipStream_t st, int mode) {
     };
     if (mode == PASS_LOGITS && !m->dry) RC_TRY(enqueue_embed(m, st));
     for (int il = 0; il < c.n_layer; il++)
-        for (int k = K_QKV; k <= K_DOWN; k++) RC_TRY(enqueue_one(m, st, k, il));
-    RC_TRY(enqueue_one(m, st, K_HEAD, 0));
+        for (int k = K_QKV; k <= K_DOWN; k++) RC_TRY(enqueue_one(m, st, k, il, kv_bound));
+    RC_TRY(enqueue_one(m, st, K_HEAD, 0, kv_bound));
     if (mode == PASS_GREEDY && !m->dry) RC_TRY(sample(true));
     return 0;
 }
@@ -718,10 +720,7 @@ static int forward_any(spy_hip_llama *m, void *stream, const int32_t *tokens_hos
     if (n_token == 1 && fused_ok(m) && (!exact || m->exact_ok)) {
         dev_state h = {tokens_host[0], n_past, 0, 0};
         HIP_TRY(hipMemcpyAsync(m->st, &h, sizeof(h), hipMemcpyHostToDevice, st));
-        m->kv_bound = n_past + 1;
-        const int rc = enqueue_pass_any(m, st, PASS_LOGITS);
-        m->kv_bound = 0;
-        if (rc) return rc;
+        RC_TRY(enqueue_pass_any(m, st, PASS_LOGITS, n_past + 1));
         if (logits_host) HIP_TRY(hipMemcpyAsync(logits_host, m->logits, (size_t)m->desc.n_vocab * 4, hipMemcpyDeviceToHost, st));
         return check_pass_error(m, st);
     }
@@ -793,11 +792,9 @@ extern "C" int spy_hip_llama_decode_greedy(spy_hip_llama *m, void *stream, int32
                 auto &g = m->graphs[kind][many];
                 if (g.exec) continue;
                 if (g.graph) { (void)hipGraphDestroy(g.graph); g.graph = nullptr; }
-                m->kv_bound = kind ? XF_MAX : 0;
                 HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
                 int rc = 0;
-                for (int i = 0; i < (many ? SPY_GRAPH_STEPS : 1) && !rc; i++) rc = enqueue_pass_any(m, st, PASS_GREEDY);
-                m->kv_bound = 0;
+                for (int i = 0; i < (many ? SPY_GRAPH_STEPS : 1) && !rc; i++) rc = enqueue_pass_any(m, st, PASS_GREEDY, kind ? XF_MAX : 0);
                 const hipError_t e = hipStreamEndCapture(st, &g.graph);
                 if (rc) return rc;
                 if (e != hipSuccess) return (int)e;
@@ -810,12 +807,7 @@ extern "C" int spy_hip_llama_decode_greedy(spy_hip_llama *m, void *stream, int32
         const int steps = use_graph && n_steps - i >= SPY_GRAPH_STEPS ? SPY_GRAPH_STEPS : 1;
         const auto &kind = m->graphs[short_run(n_past + i, steps)];
         if (use_graph) HIP_TRY(hipGraphLaunch(kind[steps > 1].exec, st));
-        else {
-            m->kv_bound = n_past + i + 1;
-            const int rc = enqueue_pass_any(m, st, PASS_GREEDY);
-            m->kv_bound = 0;
-            if (rc) return rc;
-        }
+        else RC_TRY(enqueue_pass_any(m, st, PASS_GREEDY, n_past + i + 1));
         i += steps;
     }
     HIP_TRY(hipEventRecord(m->ev1, st));
@@ -831,7 +823,8 @@ extern "C" int spy_hip_llama_decode_greedy(spy_hip_llama *m, void *stream, int32
 // Average duration of ONE kernel of the single-token pass, measured with HIP events on the stream it
 // is launched on: the kernel is launched for layer 0, 1, .. n_layer-1 (different weights and
 // caches every launch, so nothing is served from a cache that the token loop would not have),
-// `reps` times over.  The position used is the one left by the last pass.  which: "qkv", "scores",
+// `reps` times over.  The position used is the one left by the last pass, and the launches are those of a
+// pass there: 0 for "scores" where "pv" is the whole attention.  which: "qkv", "scores",
 // "pv", "wo", "gate_up", "down", "head".
 extern "C" int spy_hip_llama_kernel_time(spy_hip_llama *m, void *stream, const char *which, int32_t reps, float *us_per_launch) {
     SPY_CHECK_ARG(m && which && reps > 0 && us_per_launch);
@@ -841,7 +834,12 @@ extern "C" int spy_hip_llama_kernel_time(spy_hip_llama *m, void *stream, const c
     for (int i = 0; i < K_COUNT; i++) if (!strcmp(which, names[i])) k = i;
     SPY_CHECK_ARG(k >= 0);
     hipStream_t st = stream ? (hipStream_t)stream : m->own_stream;
-    auto once = [&](int il) { return enqueue_one(m, st, k, il); };
+    dev_state h;
+    HIP_TRY(hipMemcpyAsync(&h, m->st, sizeof(h), hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    const int kv_bound = h.pos + 1;
+    if (k == K_SCORES && pass_order(m) == 1 && attn_one_launch(m, kv_bound)) { *us_per_launch = 0.0f; return 0; }
+    auto once = [&](int il) { return enqueue_one(m, st, k, il, kv_bound); };
     for (int il = 0; il < m->desc.n_layer; il++) RC_TRY(once(il));           // warm-up
     HIP_TRY(hipEventRecord(m->ev0, st));
     for (int r = 0; r < reps; r++)
@@ -972,14 +970,14 @@ extern "C" int spy_hip_gemv_fused(void *stream, int32_t order, int32_t wtype, co
         RC_TRY(f.init(order, (int)K, (int)(K / 128), (int)K, (int)M, 8, wtype));
         f.m.desc.w_out = w; f.m.desc.out_norm = normw; f.m.desc.eps = eps;
         f.m.x = (float *)x; f.m.logits = out; f.m.q8_dump = (uint8_t *)xq_dump;
-        return enqueue_one(&f.m, (hipStream_t)stream, K_HEAD, 0);
+        return enqueue_one(&f.m, (hipStream_t)stream, K_HEAD, 0, 0);
     }
     if (!normw && resid) {                       // KQV_linear + Add, ffn_down + Add: Q8_0(x) -> rows of w -> + resid
         SPY_CHECK_ARG(M % 128 == 0);
         RC_TRY(f.init(order, (int)M, (int)(M / 128), (int)K, 1, 8, wtype));
         f.m.layers[0].w_down = w;
         f.m.hbuf = (float *)x; f.m.x1 = (float *)resid; f.m.x = out; f.m.q8_dump = (uint8_t *)xq_dump;
-        return enqueue_one(&f.m, (hipStream_t)stream, K_DOWN, 0);
+        return enqueue_one(&f.m, (hipStream_t)stream, K_DOWN, 0, 0);
     }
     return SPY_HIP_EUNSUPPORTED;
 }
@@ -991,7 +989,7 @@ extern "C" int spy_hip_ffn_gate_up_silu(void *stream, int32_t order, int32_t wty
     RC_TRY(f.init(order, (int)K, (int)(K / 128), (int)F, 1, 8, wtype));
     f.m.layers[0].w_gate = w_gate; f.m.layers[0].w_up = w_up; f.m.layers[0].ffn_norm = normw; f.m.desc.eps = eps;
     f.m.x1 = (float *)x; f.m.hbuf = out; f.m.q8_dump = (uint8_t *)xq_dump;
-    return enqueue_one(&f.m, (hipStream_t)stream, K_GATEUP, 0);
+    return enqueue_one(&f.m, (hipStream_t)stream, K_GATEUP, 0, 0);
 }
 
 extern "C" int spy_hip_rope_kvwrite(void *stream, int32_t order, int32_t wtype, int32_t wtype_v, const void *wq, const void *wk, const void *wv, const float *x,
@@ -1006,7 +1004,7 @@ extern "C" int spy_hip_rope_kvwrite(void *stream, int32_t order, int32_t wtype, 
     f.m.desc.eps = eps;
     f.m.x = (float *)x; f.m.q16 = (uint16_t *)q16; f.m.k_cache[0] = (uint16_t *)k_cache; f.m.v_cache[0] = (uint16_t *)v_cache;
     f.m.rope_cs = (float *)rope_cs; f.m.rope_tab = (float *)rope_cs; f.m.rope_row0 = pos; f.m.pos_imm = pos; f.m.q8_dump = (uint8_t *)xq_dump;
-    return enqueue_one(&f.m, (hipStream_t)stream, K_QKV, 0);
+    return enqueue_one(&f.m, (hipStream_t)stream, K_QKV, 0, 0);
 }
 
 extern "C" int spy_hip_attn_decode(void *stream, int32_t order, const void *q16, const void *k_cache, const void *v_cache, int32_t n_head, int32_t n_kv,
@@ -1020,13 +1018,12 @@ extern "C" int spy_hip_attn_decode(void *stream, int32_t order, const void *q16,
         RC_TRY(spy_ensure_lds(&f.m, (const void *)xattn_pv_kernel<0>, xattn_pv_lds((int)n_ctx)));
         RC_TRY(spy_ensure_lds(&f.m, (const void *)xattn_scores_kernel<0>, xattn_scores_lds(n_head)));
         RC_TRY(spy_attn_short_prepare((int)n_ctx));
-        f.m.kv_bound = n_kv;
     } else {
         if (pv_lds > 160 * 1024) return SPY_HIP_EUNSUPPORTED;
         RC_TRY(spy_ensure_lds(&f.m, (const void *)attn_pv_kernel, pv_lds));
     }
     f.m.q16 = (uint16_t *)q16; f.m.k_cache[0] = (uint16_t *)k_cache; f.m.v_cache[0] = (uint16_t *)v_cache;
     f.m.scores = scores; f.m.attn_out = out; f.m.pos_imm = n_kv - 1;
-    RC_TRY(enqueue_one(&f.m, (hipStream_t)stream, K_SCORES, 0));
-    return enqueue_one(&f.m, (hipStream_t)stream, K_PV, 0);
+    RC_TRY(enqueue_one(&f.m, (hipStream_t)stream, K_SCORES, 0, n_kv));
+    return enqueue_one(&f.m, (hipStream_t)stream, K_PV, 0, n_kv);
 }

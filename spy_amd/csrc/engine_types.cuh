@@ -34,7 +34,6 @@ struct spy_hip_llama {
     // graphs of single-token passes: [0] for any position, [1] for caches of up to XF_MAX tokens; one pass, SPY_GRAPH_STEPS passes
     struct pass_graph { hipGraph_t graph = nullptr; hipGraphExec_t exec = nullptr; } graphs[2][2];
     hipStream_t graph_stream = nullptr;
-    int kv_bound = 0;                                                      // the passes being enqueued see no more cached tokens than this (0: not known)
     int graph_order = -1;                                                  // summation order the graphs were captured with
     hipStream_t own_stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;

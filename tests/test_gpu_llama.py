@@ -236,6 +236,28 @@ def test_greedy_run_over_the_end_of_the_short_cache(monkeypatch):
         assert np.array_equal(a, b), i
 
 
+def test_kernel_times_are_those_of_the_launches_of_a_pass():
+    """spy_hip_llama_kernel_time times what a pass at the engine's position launches: up to 576 cached tokens in order 1 the attention is "pv" and nothing else; a run
+    across that length does not change what is launched before and behind it."""
+    from spy_amd import model as M
+    cfg = M.Config(n_layer=2, n_embd=512, n_head=4, n_ff=1024, n_vocab=512, n_ctx=640, wtype=O.Q4_0)
+    eng = M.Engine(cfg, M.synth_model(cfg, seed=3), order=1)
+    tok = np.array([5], np.int32)
+    for n_past, short in ((40, True), (575, True), (576, False), (8, True)):
+        eng.forward(tok, n_past, want_logits=False)
+        s, p = eng.kernel_time_us("scores", 1), eng.kernel_time_us("pv", 1)
+        assert p > 0 and (s == 0) == short, (n_past, s, p)
+    eng.decode_greedy(5, 570, 5, use_graph=True)                 # leaves position 575
+    assert eng.kernel_time_us("scores", 1) == 0
+    eng.decode_greedy(5, 570, 6, use_graph=True)
+    assert eng.kernel_time_us("scores", 1) > 0
+    eng.set_order(0)
+    eng.forward(tok, 40, want_logits=False)
+    assert eng.kernel_time_us("pv", 1) > 0
+    eng.close()
+
+
+
 def test_model_wider_than_4096_takes_the_tiled_kernels():
     """n_embd = 5120 (the 13B width): the one-row-per-wave kernels stage 4096 activations per workgroup at most, so the fused
     single-token pass of such a model runs the 256-thread tiled kernels, in this backend's own summation order (the kernels of

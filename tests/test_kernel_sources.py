@@ -44,3 +44,12 @@ def test_launches_of_a_single_token_pass_read_no_environment():
     assert "xattn_scores_kernel" in body and "spy_attn_short" in body and "static int enqueue_pass_any(" in body
     for name, text in [("engine.hip", body)] + [(n, open(os.path.join(ROOT, "spy_amd", "csrc", n)).read()) for n in ("exact_launch.cuh", "decode_launch.cuh", "attn_short.hip")]:
         assert "getenv" not in text, name
+
+
+def test_launches_of_a_single_token_pass_depend_on_no_state_of_an_earlier_call():
+    """How many cached tokens a pass sees chooses its attention kernels: an argument of what enqueues them, not a field of the engine that a call which fails half-way
+    would leave behind for the next one."""
+    types = open(os.path.join(ROOT, "spy_amd", "csrc", "engine_types.cuh")).read()
+    engine = open(os.path.join(ROOT, "spy_amd", "csrc", "engine.hip")).read()
+    assert "kv_bound" not in types and "->kv_bound" not in engine and ".kv_bound" not in engine
+    assert "static int enqueue_one(spy_hip_llama *m, hipStream_t st, int which, int il, int kv_bound)" in engine

@@ -353,8 +353,8 @@ int spy_hip_llama_buffer(spy_hip_llama *m, const char *name, int32_t layer, void
 int spy_hip_llama_timing(spy_hip_llama *m, float *ms_per_pass, int32_t *n_pass);
 /* average duration (microseconds) of one kernel of the single-token pass, HIP events around
  * reps x n_layer launches that walk the layers (fresh weights / caches every launch); which:
- * "qkv", "scores", "pv", "wo", "gate_up", "down", "head".  Uses the position of the last pass and the launches of
- * a pass there: 0 for "scores" where "pv" is the whole attention (order 1, up to 576 cached tokens). */
+ * "qkv", "scores", "pv", "wo", "gate_up", "down", "head".  Uses the position that the last pass left (the cache's
+ * last one where that is past it; "qkv" writes its slots) and the launches of a pass there: 0 for "scores" where "pv" is the whole attention (order 1, up to 576 cached tokens). */
 int spy_hip_llama_kernel_time(spy_hip_llama *m, void *stream, const char *which, int32_t reps, float *us_per_launch);
 /* How single-token passes are launched, as a bit mask (negative: error).
  * bit 1 (value 2): the attention part of a layer (qkv, scores, softmax + KQV) is ONE launch whose

@@ -823,7 +823,7 @@ extern "C" int spy_hip_llama_decode_greedy(spy_hip_llama *m, void *stream, int32
 // Average duration of ONE kernel of the single-token pass, measured with HIP events on the stream it
 // is launched on: the kernel is launched for layer 0, 1, .. n_layer-1 (different weights and
 // caches every launch, so nothing is served from a cache that the token loop would not have),
-// `reps` times over.  The position used is the one left by the last pass, and the launches are those of a
+// `reps` times over.  The position used is the one left by the last pass (the last slot where that is past the cache), and the launches are those of a
 // pass there: 0 for "scores" where "pv" is the whole attention.  which: "qkv", "scores",
 // "pv", "wo", "gate_up", "down", "head".
 extern "C" int spy_hip_llama_kernel_time(spy_hip_llama *m, void *stream, const char *which, int32_t reps, float *us_per_launch) {
@@ -837,6 +837,11 @@ extern "C" int spy_hip_llama_kernel_time(spy_hip_llama *m, void *stream, const c
     dev_state h;
     HIP_TRY(hipMemcpyAsync(&h, m->st, sizeof(h), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
+    if (h.pos >= m->desc.n_ctx) {                // a greedy run that filled the cache leaves the position behind its last slot: "qkv" would write there, "scores" and "pv" read
+        h.pos = m->desc.n_ctx - 1;
+        HIP_TRY(hipMemcpyAsync(m->st, &h, sizeof(h), hipMemcpyHostToDevice, st));
+        HIP_TRY(hipStreamSynchronize(st));
+    }
     const int kv_bound = h.pos + 1;
     if (k == K_SCORES && pass_order(m) == 1 && attn_one_launch(m, kv_bound)) { *us_per_launch = 0.0f; return 0; }
     auto once = [&](int il) { return enqueue_one(m, st, k, il, kv_bound); };

@@ -257,6 +257,24 @@ def test_kernel_times_are_those_of_the_launches_of_a_pass():
     eng.close()
 
 
+@pytest.mark.parametrize("order", [0, 1])
+def test_kernel_times_on_a_full_cache(order):
+    """After a greedy run that fills the cache the kernels are timed at its last position: nothing else in the caches changes (a position behind it
+    is the first slot of the next row of V^T)."""
+    from spy_amd import model as M
+    cfg = M.Config(n_layer=2, n_embd=512, n_head=4, n_ff=1024, n_vocab=512, n_ctx=64, wtype=O.Q4_0)
+    eng = M.Engine(cfg, M.synth_model(cfg, seed=3), order=order)
+    caches = lambda: [eng.read_buffer("k_cache", il, np.uint16).reshape(64, 512)[:63] for il in (0, 1)] + [eng.read_buffer("v_cache", il, np.uint16).reshape(512, 64)[:, :63] for il in (0, 1)]
+    eng.decode_greedy(5, 0, 64, use_graph=True)
+    want = caches()
+    for which in ("qkv", "scores", "pv", "wo", "gate_up", "down", "head"):
+        eng.kernel_time_us(which, 1)
+        for a, b in zip(want, caches()):
+            assert np.array_equal(a, b), which
+    eng.close()
+
+
+
 
 def test_model_wider_than_4096_takes_the_tiled_kernels():
     """n_embd = 5120 (the 13B width): the one-row-per-wave kernels stage 4096 activations per workgroup at most, so the fused

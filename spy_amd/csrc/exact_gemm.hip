@@ -19,6 +19,7 @@
 // 4096 x 4096 Q4_0: 16 rows 80 -> 15 us, 77 rows 104 -> 28, 512 rows 137 -> 88, 2048 rows 400 -> 313; 8 rows (one launch per row) 36 -> 15.
 #include "common.cuh"
 #include "exact_sum.cuh"
+#include "gemm_tiles.h"
 
 #include <type_traits>
 #include <utility>
@@ -275,7 +276,7 @@ __global__ __launch_bounds__(256, 3) void xt_mixed_kernel(xt_args a) {
 // With a wave or two on a SIMD what bounds it is the chain barrier, LDS read, unpack, matrix instruction, fmas: it is walked once per chunk of eight
 // blocks, and the operands of the next chunk are read from LDS before the fmas of this one.  NS: LDS slots for chunks, all of them on their way: four where
 // a compute unit has one or two workgroups, whose weights come from memory (two: 20 % slower there); two, 24 KB, where it has more (four: up to
-// 20 % slower).  32 weight rows and eight waves per workgroup: 30 % slower with 4096.  From five workgroups on the tiles of 32 rows are faster.
+// 20 % slower).  32 weight rows and eight waves per workgroup: 30 % slower with 4096.  From four workgroups on a compute unit the tiles of 32 rows are faster (xt_choose).
 // Against one stage of four blocks per barrier, weights from memory, in us, packing of the activations (4 us) included: 8 rows, Q4_0 4096 x 4096 14.4 -> 12.1,
 // 4096 x 11008 30.6 -> 23.6, 12288 x 4096 21.0 -> 17.7, Q8_0 14.4 -> 12.5, 30.3 -> 24.3, 22.5 -> 20.8; 48 rows, Q4_0 4096 x 4096 21.2 -> 17.8, 4096 x 11008 47.5 -> 37.3.
 template <int WT, int NS>
@@ -1441,61 +1442,22 @@ int xks_launch(hipStream_t st, xt_args a, int nmat) {
     return SPY_LAUNCH_RC();
 }
 
-// Which tile.  n workgroups per compute unit take about lat + (n - 1) * inc: figures in tenths of a microsecond for K = 4096, measured for
-// n = 1 .. 16 (whole workgroups count while they are few; everything scales with K).  Small tiles have the shorter chain, large ones unpack a
-// weight for more activation rows.
-// rest: what a workgroup of the ncg % groups groups that remain takes, 0 if it is a whole one.
-struct xt_cost { int rows, groups, lat, inc, rest = 0; };
-int xt_pick(const xt_args &a, int nmat, const xt_cost *c, int n) {
-    const int64_t cu = spy_num_cu();
-    int best = 0;
-    int64_t least = 0;
-    for (int i = 0; i < n; i++) {
-        const int64_t tiles = (int64_t)((a.M + c[i].rows - 1) / c[i].rows) * nmat, wgs = tiles * (c[i].rest ? a.ncg / c[i].groups : (a.ncg + c[i].groups - 1) / c[i].groups);
-        const int64_t t = c[i].lat + (wgs <= 6 * cu && !c[i].rest ? (wgs + cu - 1) / cu * 10 - 10 : 10 * wgs / cu - 10) * c[i].inc / 10 + tiles * c[i].rest / cu;
-        if (!i || t < least) { best = i; least = t; }
-    }
-    return best;
-}
 template <int WT>
 int xt_dispatch(hipStream_t st, const xt_args &a, int nmat) {
-    // the last one: tiles of four groups and one of what remains, where something remains
-    static const int of_rest[4] = {0, 60, 100, 132};
-    const int rest = a.ncg > 4 ? a.ncg % 4 : 0;
-    // Q8_0's first two tiles have room for four workgroups on a compute unit, and its chunks are larger: 4096 x 11008 x 150 100.5 -> 93.1 us, 4096 x 4096 x 150 42.2 -> 39.4,
-    // 12288 x 4096 x 180 116 -> 108 with its own increments.
-    // The third tile's increment: another workgroup on a compute unit that has 8 to 16 takes 95 .. 96 on the scale of the fourth's 165, in either type; but beyond six the
-    // rule counts parts of workgroups, where the third is in truth still rounded up (22016 x 4096 x 128, 10.75 of them: 130.7 us, the line between ten and twelve says 125).  Every tile timed
-    // at 322 shapes (4096 .. 32000 x 4096 and 4096 x 11008 by 4 .. 512 rows, both types): the choice is 0.12 % slower than the best tile in the mean with 97 or 98, 0.28 % with 96
-    // (fourth against third tile: 22016 x 4096 x 128 Q4_0 124 / 132 us, Q8_0 132 / 145; 11008 x 4096 x 256 Q8_0 127 / 142), 0.49 % with 100 (4096 x 11008 x 100 Q4_0: third tile 73.4, mixed fourth 85.1).
-    constexpr bool Q8 = WT == SPY_HIP_Q8_0;
-    const xt_cost c[5] = {{16, 1, 44, Q8 ? 50 : 44}, {32, 1, 106, Q8 ? 64 : 56}, {32, 2, 173, 98}, {32, 4, 288, 165}, {32, 4, 288, 165, of_rest[rest]}};
-    switch (xt_pick(a, nmat, c, rest ? 5 : 4)) {
-    case 0: return (int64_t)(a.M + 15) / 16 * nmat * a.ncg <= 2 * spy_num_cu() ? xn_launch<WT, 4>(st, a, nmat) : xn_launch<WT, 2>(st, a, nmat);
-    case 1: return xt_launch<WT, 1, 4, 2, 2>(st, a, nmat);
-    case 2: return xt_launch<WT, 2, 4, 2, 2>(st, a, nmat);
-    case 3: return xt_launch<WT, 4, 2, 1, 2>(st, a, nmat);
-    default: return rest == 1 ? xt_launch_mixed<WT, 1>(st, a, nmat) : rest == 2 ? xt_launch_mixed<WT, 2>(st, a, nmat) : xt_launch_mixed<WT, 3>(st, a, nmat);
+    switch (xt_choose(WT == SPY_HIP_Q8_0, a.M, nmat, a.ncg, spy_num_cu())) {
+    case XT_N4: return xn_launch<WT, 4>(st, a, nmat);
+    case XT_N2: return xn_launch<WT, 2>(st, a, nmat);
+    case XT_1: return xt_launch<WT, 1, 4, 2, 2>(st, a, nmat);
+    case XT_2: return xt_launch<WT, 2, 4, 2, 2>(st, a, nmat);
+    case XT_4: return xt_launch<WT, 4, 2, 1, 2>(st, a, nmat);
+    case XT_MIXED + 1: return xt_launch_mixed<WT, 1>(st, a, nmat);
+    case XT_MIXED + 2: return xt_launch_mixed<WT, 2>(st, a, nmat);
+    default: return xt_launch_mixed<WT, 3>(st, a, nmat);
     }
-}
-// Tiles of the K-quants, and of Q4_0 in the own order: times in tenths of a microsecond at K = 4096 with 1, 2, 3, 4 and 6 workgroups per compute unit, weights from memory
-struct xk_tile { int rows, groups, t[5]; };
-int xk_pick(const xt_args &a, int nmat, int ncg, const xk_tile *c, int n_tiles) {
-    const int64_t cu = spy_num_cu();
-    int best = 0;
-    int64_t least = 0;
-    for (int i = 0; i < n_tiles; i++) {
-        const int64_t wgs = (int64_t)((a.M + c[i].rows - 1) / c[i].rows) * nmat * ((ncg + c[i].groups - 1) / c[i].groups), n = (wgs + cu - 1) / cu;
-        const int64_t t = n <= 4 ? c[i].t[n - 1] : n == 5 ? (c[i].t[3] + c[i].t[4]) / 2 : c[i].t[4] * wgs / (6 * cu);
-        if (!i || t < least) { best = i; least = t; }
-    }
-    return best;
 }
 template <int WT>
 int xk_dispatch(hipStream_t st, const xt_args &a, int nmat) {
-    static const xk_tile k4[5] = {{16, 1, {99, 123, 171, 220, 297}}, {32, 2, {226, 264, 278, 319, 517}}, {64, 2, {273, 302, 407, 557, 899}}, {64, 4, {338, 467, 643, 815, 1176}}, {128, 8, {830, 1414, 2069, 2736, 4053}}},
-                         k6[5] = {{16, 1, {113, 160, 207, 269, 364}}, {32, 2, {240, 267, 354, 460, 702}}, {64, 2, {305, 455, 635, 832, 1210}}, {64, 4, {357, 526, 756, 987, 1443}}, {128, 8, {827, 1403, 2101, 2768, 4116}}};
-    switch (xk_pick(a, nmat, a.ncg, WT == SPY_HIP_Q4_K ? k4 : k6, 5)) {
+    switch (xk_choose(WT == SPY_HIP_Q4_K, a.M, nmat, a.ncg, spy_num_cu())) {
     case 0: return xks_launch<WT>(st, a, nmat);
     case 1: return xk_launch<WT, false, 2, 2, 4>(st, a, nmat);
     case 2: return xk_launch<WT, false, 4, 2, 4>(st, a, nmat);
@@ -1508,11 +1470,7 @@ int xk_dispatch(hipStream_t st, const xt_args &a, int nmat) {
 // that a call in pieces has its bits
 template <int WT>
 int xko_dispatch(hipStream_t st, const xt_args &a, int nmat) {
-    // The last three split K: where a matrix gives a compute unit one workgroup, the chain of its super-blocks is what it takes (8192 x 4096 x 64: Q4_K
-    // 35.6 -> 22.6 us, Q6_K 39.8 -> 25.2; 8192 x 11008 x 100: 104 -> 69 and 126 -> 92); with two and more the tiles without a split are faster.
-    static const xk_tile k4[9] = {{16, 1, {99, 123, 171, 219, 298}}, {32, 2, {246, 271, 286, 323, 513}}, {64, 2, {287, 320, 405, 556, 802}}, {32, 4, {303, 382, 421, 482, 902}}, {64, 4, {331, 420, 569, 770, 1071}}, {64, 8, {497, 706, 1082, 1333, 1960}}, {32, 2, {148, 259, 380, 499, 736}}, {32, 4, {186, 340, 498, 654, 964}}, {64, 4, {278, 516, 754, 995, 1466}}},
-                         k6[9] = {{16, 1, {113, 160, 206, 269, 364}}, {32, 2, {247, 286, 369, 468, 703}}, {64, 2, {316, 468, 643, 841, 1223}}, {32, 4, {295, 408, 480, 586, 1052}}, {64, 4, {354, 532, 762, 1001, 1447}}, {64, 8, {524, 764, 1159, 1473, 2173}}, {32, 2, {174, 317, 462, 606, 892}}, {32, 4, {211, 394, 579, 758, 1122}}, {64, 4, {344, 639, 930, 1230, 1814}}};
-    switch (xk_pick(a, nmat, a.ncg_all, WT == SPY_HIP_Q4_K ? k4 : k6, 9)) {
+    switch (xko_choose(WT == SPY_HIP_Q4_K, a.M, nmat, a.ncg_all, spy_num_cu())) {
     case 0: return xks_launch<WT>(st, a, nmat);
     case 1: return xk_launch<WT, true, 2, 2, 4>(st, a, nmat);
     case 2: return xk_launch<WT, true, 4, 2, 4>(st, a, nmat);
@@ -1526,9 +1484,7 @@ int xko_dispatch(hipStream_t st, const xt_args &a, int nmat) {
 }
 
 int xo_dispatch(hipStream_t st, const xt_args &a, int nmat) {
-    // tiles of 128 rows by four groups (two of 32 x 32 per wave) were the better ones nowhere: 8192 x 4096 x 500 69.1 us, these two 68.9 and 66.2
-    static const xk_tile c[2] = {{64, 4, {342, 383, 515, 650, 949}}, {128, 8, {607, 990, 1472, 1933, 2895}}};
-    return xk_pick(a, nmat, a.ncg, c, 2) == 0 ? xo_launch(st, a, nmat) : xo32_launch(st, a, nmat);
+    return xo_choose(a.M, nmat, a.ncg, spy_num_cu()) == 0 ? xo_launch(st, a, nmat) : xo32_launch(st, a, nmat);
 }
 
 }   // namespace

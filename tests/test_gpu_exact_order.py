@@ -91,11 +91,18 @@ def test_single_row_matmul_takes_the_two_phase_kernel(hip, oracle, wtype, M, K, 
             assert (scratch.download(np.uint8) == 0xEE).all(), "the single-row route does not use the scratch buffer"
 
 
+# (test_kernel_sources.py: which tiles of the dispatch these reach on 256 compute units)
+PACKED_SHAPES = [(4, 256, 3), (20, 512, 4), (4096, 256, 15), (100, 1280, 16), (36, 4096, 17), (12288, 256, 33), (4100, 512, 48), (8192, 256, 100), (4096, 768, 257), (8192, 256, 1025),
+                 (12300, 768, 10), (8196, 512, 17), (12700, 768, 17), (14988, 512, 49), (3556, 256, 66), (2724, 768, 81), (2372, 512, 102)]
+NARROW_SHAPES = [(12288, 256, 16), (12284, 768, 10), (8196, 512, 10), (4096, 256, 33), (4084, 1280, 48), (16, 512, 3), (28, 768, 32)]
+ANY_SCALE_SHAPES = [(11000, 256, 40), (8192, 768, 70), (4100, 512, 150), (4096, 1280, 300), (24604, 256, 17), (8196, 512, 1000), (12300, 256, 2025)]
+
+
 @pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0, O.Q4_K, O.Q6_K])
-@pytest.mark.parametrize("M,K,T", [(4, 256, 3), (20, 512, 4), (4096, 256, 15), (100, 1280, 16), (36, 4096, 17), (12288, 256, 33), (4100, 512, 48), (8192, 256, 100), (4096, 768, 257), (8192, 256, 1025)])
+@pytest.mark.parametrize("M,K,T", PACKED_SHAPES)
 def test_packed_activation_matmul_bits(hip, oracle, wtype, M, K, T):
-    """Three rows and more against rows of whole super-blocks: the kernels that unpack a weight once per wave (exact_gemm.hip), in every tile
-    the dispatch has, with partial tiles on both sides, the shortest contraction and scales down to fp16 subnormals."""
+    """Three rows and more against rows of whole super-blocks: the kernels that unpack a weight once per wave (exact_gemm.hip), for Q4_0 and Q8_0 in every tile
+    the dispatch has (test_kernel_sources.py asks it), with partial tiles on both sides, the shortest contraction and scales down to fp16 subnormals."""
     from tests.gpu_util import dev, dev_empty, call
     rng = np.random.default_rng(11 * wtype + M + K + T)
     w = O.quantize(oracle, (rng.standard_normal((M, K)) * 0.02).astype(np.float32), wtype)
@@ -122,16 +129,16 @@ def test_packed_activation_matmul_bits(hip, oracle, wtype, M, K, T):
 
 
 @pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0])
-@pytest.mark.parametrize("M,K,T", [(12288, 256, 16), (12300, 768, 10), (8196, 512, 17), (4096, 256, 33), (4084, 1280, 48), (16, 512, 3), (28, 768, 32)])
+@pytest.mark.parametrize("M,K,T", NARROW_SHAPES)
 def test_narrow_matmul_bits(hip, oracle, wtype, M, K, T):
     """Few activation rows, tiles of 16 x 16 with two and with four chunks on their way: one chunk (K = 256), odd and even numbers of them, partial tiles."""
     test_packed_activation_matmul_bits(hip, oracle, wtype, M, K, T)
 
 
 @pytest.mark.parametrize("wtype", [O.Q4_K, O.Q6_K])
-@pytest.mark.parametrize("M,K,T", [(11000, 256, 40), (8192, 768, 70), (4100, 512, 150), (4096, 1280, 300)])
+@pytest.mark.parametrize("M,K,T", ANY_SCALE_SHAPES)
 def test_k_quant_tiles_with_scales_of_any_size(hip, oracle, wtype, M, K, T):
-    """The tiles of several groups from packed activations, whose outer products and scaled operands come from matrix instructions: block scales down to fp16's subnormals
+    """Every tile of several groups from packed activations, whose outer products and scaled operands come from matrix instructions: block scales down to fp16's subnormals
     and up to its largest numbers, any quants, activation rows whose scales are as small and as large.  The oracle's bits."""
     from tests.gpu_util import dev, dev_empty, call
     rng = np.random.default_rng(11 * wtype + M + K + T)

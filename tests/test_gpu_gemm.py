@@ -153,8 +153,15 @@ def test_op_matmul_prompt_sizes(hip, oracle):
     assert_close(dO.download(np.float32).reshape(O_want.shape), O_want, "KQV T=40", tol=1e-5)
 
 
-@pytest.mark.parametrize("wtype,M,K,T", [(O.Q4_0, 16356, 256, 65), (O.Q4_0, 8164, 512, 129), (O.Q4_0, 4068, 768, 400), (O.Q4_0, 2020, 256, 1025), (O.Q4_0, 11008, 4096, 130),
-                                         (O.Q4_K, 36, 512, 8), (O.Q4_K, 4100, 256, 130), (O.Q4_K, 12300, 256, 70), (O.Q4_K, 8200, 512, 650), (O.Q4_K, 11012, 256, 40), (O.Q6_K, 36, 512, 9), (O.Q6_K, 4100, 256, 130), (O.Q6_K, 12300, 256, 70), (O.Q6_K, 8200, 512, 650)])
+# (test_kernel_sources.py: which tiles of the dispatch these reach on 256 compute units)
+OWN_SHAPES = [(O.Q4_0, 16356, 256, 65), (O.Q4_0, 8164, 512, 129), (O.Q4_0, 4068, 768, 400), (O.Q4_0, 2020, 256, 1025), (O.Q4_0, 11008, 4096, 130),
+              (O.Q4_K, 36, 512, 8), (O.Q4_K, 4100, 256, 130), (O.Q4_K, 12300, 256, 70), (O.Q4_K, 8200, 512, 650), (O.Q4_K, 11012, 256, 40), (O.Q4_K, 16396, 512, 17), (O.Q4_K, 3604, 768, 513), (O.Q4_K, 28892, 256, 70),
+              (O.Q6_K, 36, 512, 9), (O.Q6_K, 4100, 256, 130), (O.Q6_K, 12300, 256, 70), (O.Q6_K, 8200, 512, 650), (O.Q6_K, 8236, 768, 17), (O.Q6_K, 16396, 512, 33)]
+SPLIT_SHAPES = [(4096, 256, 17), (8188, 768, 32), (8192, 1280, 50), (4100, 2816, 64), (11000, 512, 40), (11008, 4352, 48), (8188, 256, 30), (8188, 256, 40), (8188, 256, 100)]
+TILES_OF_32_SHAPES = [(8100, 768, 985), (16300, 256, 485), (12284, 512, 970)]
+
+
+@pytest.mark.parametrize("wtype,M,K,T", OWN_SHAPES)
 def test_matmul_operator_takes_the_packed_activation_kernels(hip, oracle, wtype, M, K, T, monkeypatch):
     """MatMul in this backend's own order from packed activations, with partial tiles on both sides: within fp32 rounding of the oracle,
     and for Q4_0 the bits of the tile kernel, which adds an output's blocks in the same sequence."""
@@ -184,14 +191,14 @@ def test_matmul_operator_takes_the_packed_activation_kernels(hip, oracle, wtype,
 
 
 @pytest.mark.parametrize("wtype", [O.Q4_K, O.Q6_K])
-@pytest.mark.parametrize("M,K,T", [(4096, 256, 17), (8188, 768, 32), (8192, 1280, 50), (4100, 2816, 64), (11000, 512, 40), (11008, 4352, 48)])
+@pytest.mark.parametrize("M,K,T", SPLIT_SHAPES)
 def test_matmul_operator_splits_k(hip, oracle, wtype, M, K, T, monkeypatch):
-    """The tiles of the own order whose sets of waves share K, one workgroup per compute unit: fewer super-blocks than sets (256, 768), numbers of
-    them that do not divide, partial tiles."""
+    """The tiles of the own order whose sets of waves share K, one workgroup per compute unit: fewer super-blocks than sets (256: all but one without any; 768), numbers of
+    them that do not divide, partial tiles (and, 4096 x 256 x 17, the kernel for fewer workgroups)."""
     test_matmul_operator_takes_the_packed_activation_kernels(hip, oracle, wtype, M, K, T, monkeypatch)
 
 
-@pytest.mark.parametrize("M,K,T", [(8100, 768, 985), (16300, 256, 485), (12284, 512, 970)])
+@pytest.mark.parametrize("M,K,T", TILES_OF_32_SHAPES)
 def test_matmul_operator_tiles_of_32(hip, oracle, M, K, T, monkeypatch):
     """Q4_0 in the own order from many activation rows, tiles of 32 x 32: one chunk, odd and even numbers of them, an odd number of activation groups, partial tiles."""
     test_matmul_operator_takes_the_packed_activation_kernels(hip, oracle, O.Q4_0, M, K, T, monkeypatch)

@@ -53,3 +53,37 @@ def test_launches_of_a_single_token_pass_depend_on_no_state_of_an_earlier_call()
     engine = open(os.path.join(ROOT, "spy_amd", "csrc", "engine.hip")).read()
     assert "kv_bound" not in types and "->kv_bound" not in engine and ".kv_bound" not in engine
     assert "static int enqueue_one(spy_hip_llama *m, hipStream_t st, int which, int il, int kv_bound)" in engine
+
+
+def test_shapes_of_the_packed_activation_tests_reach_every_tile(tmp_path):
+    """The tile choice (gemm_tiles.h, on 256 compute units) for the shapes of the GPU tests: every tile there is runs on a matrix with a remainder on both sides, and the
+    tests named for one kernel run that one."""
+    from tests import oracle_lib as O
+    from tests import test_gpu_exact_order as E, test_gpu_gemm as G
+    out = str(tmp_path / "gemm_tiles")
+    subprocess.check_call(["g++", "-O1", "-std=c++20", "-o", out, os.path.join(ROOT, "tests", "host", "gemm_tiles.cpp")])
+
+    def tiles(which, flag, shapes):
+        text = "".join("%s %d %d %d 256\n" % (which, flag, M, T) for M, K, T in shapes)
+        got = [int(v) for v in subprocess.run([out], input=text, capture_output=True, text=True, check=True).stdout.split()]
+        assert len(got) == len(shapes)
+        return got
+
+    def ragged(which, flag, shapes, rows=16):
+        return {t for t, (M, K, T) in zip(tiles(which, flag, shapes), shapes) if M % rows and T % 16}
+
+    for q8 in (0, 1):
+        assert ragged("t", q8, E.PACKED_SHAPES + E.NARROW_SHAPES, 32) == set(range(8))
+        assert set(tiles("t", q8, E.NARROW_SHAPES)) == {0, 1}, "xn_kernel with four and with two slots, and nothing else"
+        assert {1} == {t for t, (M, K, T) in zip(tiles("t", q8, E.NARROW_SHAPES), E.NARROW_SHAPES) if M in (12284, 8196)}, "... two slots: remainders, odd numbers of chunks"
+    for q4 in (0, 1):
+        assert ragged("k", q4, E.PACKED_SHAPES + E.ANY_SCALE_SHAPES) == set(range(5))
+        assert set(tiles("k", q4, E.ANY_SCALE_SHAPES)) == {1, 2, 3, 4}
+        assert [t for t, (M, K, T) in zip(tiles("k", q4, E.ANY_SCALE_SHAPES), E.ANY_SCALE_SHAPES) if M % 128 and (T + 15) // 16 % 8 and t == 4], "128 rows x 8 groups, part of either"
+        own = [s[1:] for s in G.OWN_SHAPES if s[0] == (O.Q4_K if q4 else O.Q6_K)]
+        assert ragged("o", q4, own + G.SPLIT_SHAPES, 32) == set(range(9)) - (set() if q4 else {2})       # (64 rows x 2 groups of Q6_K: chosen for no shape there is up to 36000 rows by 4096)
+        split = list(zip(tiles("o", q4, G.SPLIT_SHAPES), G.SPLIT_SHAPES))
+        assert {t for t, (M, K, T) in split if K == 256} >= {6, 7, 8}, "one super-block for all sets"
+        assert {t for t, _ in split} == {0, 6, 7, 8}
+    own = [s[1:] for s in G.OWN_SHAPES if s[0] == O.Q4_0]
+    assert set(tiles("q", 0, own)) == {0} and set(tiles("q", 0, G.TILES_OF_32_SHAPES)) == {1}

@@ -8,11 +8,12 @@
 // Up to XF_MAX cached tokens: the same 256 workgroups (head, 16 rows of V^T), each with all the scores of its head.  The eight
 // workgroups of a head read its keys eight times over, from the L2 of the one XCD that they share (head = workgroup index modulo n_head, n_head a
 // multiple of 8 in the models there are), and what that costs is less than the launch and the scores' way through memory that it saves:
-// the two launches 8.5 -> 4.3 us with 40 tokens, 10.1 -> 7.9 with 512.  Up to XF_MAX tokens the keys of a head fit LDS.
+// one layer's after the other, the two launches 8.4 -> 4.7 or 5.4 us (by process) with 40 tokens, 9.9 -> 7.0 with 300, 10.6 -> 9.2 with 512, 11.0 -> 10.4 with 576; kernel times
+// in a pass 10.3 -> 4.9 with 8 .. 40 tokens, 12.0 -> 10.5 with 512 .. 535.  Up to XF_MAX tokens the keys of a head fit LDS.  n_ctx is a multiple of 8 (16-byte pieces of a V^T row).
 // What bounds it: the chain launch, keys and V^T rows (one wait for both), dots, exponentials (a gather), running sum, walk.
 #define XF_NP (XF_MAX * 16 / XP_THREADS)   // 16-byte pieces of keys per thread
 static size_t xattn_short_lds(int n_ctx) { return (size_t)(n_ctx < XF_MAX ? n_ctx : XF_MAX) * 256 + 16 * 96 * 2; }      // the keys; later the rows of V^T (16 rows of cap + 32 .. 96 halfs)
-// IN_STATE: the position is st->pos, else pos_imm (decided when the kernel is compiled: asked in the kernel it cost the engine's launches 0.15 of 5 us)
+// IN_STATE: the position is st->pos, else pos_imm (decided when the kernel is compiled: asked in the kernel it cost the engine's launches 0.1 of 5 us)
 template <bool IN_STATE>
 static __global__ __launch_bounds__(XP_THREADS) void xattn_short_kernel(const dev_state *st, int pos_imm, const uint16_t *__restrict__ q16, const uint16_t *kc, const uint16_t *vc,
                                                                  float *__restrict__ scores, float *attn_out, const float *__restrict__ lut, int n_ctx, float scale) {

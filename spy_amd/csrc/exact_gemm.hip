@@ -1133,8 +1133,8 @@ __global__ __launch_bounds__(256, 3) void xks_kernel(xt_args a) {
 // and the scale products of four blocks are one 16x16x4_4b as above: 24 matrix-core cycles and four fmas (16 cycles) per tile and block, where
 // the int8 form takes a 35-cycle instruction, a 32-cycle one and two vector instructions per output of a 32 x 32 tile.
 // Matrix and vector cycles of these instructions hardly overlap (counters of 16 x 16 tiles at 1000 rows: vector 36 %, matrix 38 %, at once 13 % of the time), which is
-// why the cycles above are what counts; and the tiles fill the chip better than 128 x 128 ones.  Packing included, Q4_0, 4096 x 4096: 385 rows 66 -> 42 us,
-// 512 rows 68 -> 45, 1000 rows 94 -> 68, 2048 rows 118 -> 108; 4096 x 11008: 1000 rows 228 -> 162; 22016 x 4096: 77 rows 85 -> 56, 1000 rows 314 -> 272.
+// why the cycles above are what counts; and the tiles fill the chip better than 128 x 128 ones.  Packing included, weights from memory, Q4_0, 4096 x 4096: 385 rows 90 -> 40 us,
+// 512 rows 92 -> 41, 1000 rows 95 -> 68, 2048 rows 117 -> 109; 4096 x 11008: 1000 rows 232 -> 165; 22016 x 4096: 77 rows 90 -> 54, 1000 rows 312 -> 278.
 // Two kernels of one arithmetic.  xo_kernel, for few workgroups: four waves of 16 rows by four activation groups, in tiles of 16 x 16.
 // Weights: lane (q, r) reads blocks 2q and 2q + 1 of row r and chunk (contiguous over the four lanes of a row), brings words 2i and 2i + 1 of a block
 // into one dword, and 4 x 4 exchanges between the lane blocks (v_permlane16_swap, v_permlane32_swap) leave words 2q and 2q + 1 of every block in lane block q:
@@ -1277,8 +1277,8 @@ __global__ __launch_bounds__(256, 3) void xo_kernel(xt_args a) {
 // The same for many activation rows: four waves of 32 rows by four pairs of activation groups, in tiles of 32 x 32.  An operand read from LDS serves twice the
 // arithmetic of a 16 x 16 tile's, and the compiler may order the matrix and vector instructions of a tile, which with 16 x 16 it did worse than by hand.
 // On registers alone this form takes 19.4 ns per 16 x 16 x 32 and SIMD (two waves; the clock falls under these instructions) and the other 23.2; here it is
-// 23.8, for 100 instructions of unpacking beside 256 fmas and 1536 matrix cycles.  Packing included, two row groups of 16 per wave before: 22016 x 4096 x 1000
-// 308 -> 272 us, 12288 x 4096 x 1000 167 -> 151, 4096 x 11008 x 1000 171 -> 162, 4096 x 4096 x 1000 73 -> 68.
+// 23.8, for 100 instructions of unpacking beside 256 fmas and 1536 matrix cycles.  Packing included, weights from memory, against two row groups of 16 per wave
+// (with the operand reads in one bank that xo_kernel had then): 22016 x 4096 x 1000 310 -> 278 us, 12288 x 4096 x 1000 168 -> 151, 4096 x 11008 x 1000 188 -> 165, 4096 x 4096 x 1000 78 -> 68.
 // (Two pairs per wave: 340 us at 22016 x 4096 x 1000; three: 311.)
 constexpr int XO_CP = 4;
 __global__ __launch_bounds__(256, 2) void xo32_kernel(xt_args a) {

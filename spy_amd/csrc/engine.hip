@@ -152,7 +152,7 @@ extern "C" int spy_hip_llama_create(const spy_hip_llama_desc *desc, spy_hip_llam
     // the host backend's summation order: cos / sin of every position from the host's libm (theta_0 = pos, theta_{k+1} =
     // theta_k * theta_scale in fp32, non-linear.cpp:304-309), the exp / silu tables, shapes the kernels take
     if (!rc && fused_ok(m) && m->wave && m->hd == 128 && c.n_embd % 128 == 0 && c.n_ff % 128 == 0 && c.n_ff <= 16384 &&
-        c.n_ctx <= 512 * XP_NP && xattn_pv_lds(c.n_ctx) <= 160 * 1024 - 256 && xattn_scores_lds(c.n_head) <= 160 * 1024) {
+        c.n_ctx <= XA_MAX_CTX && c.n_head <= XA_MAX_HEAD) {
         std::vector<float> tab((size_t)c.n_ctx * m->hd);
         for (int pos = 0; pos < c.n_ctx; pos++) {
             float theta = (float)pos;
@@ -166,7 +166,6 @@ extern "C" int spy_hip_llama_create(const spy_hip_llama_desc *desc, spy_hip_llam
         if (!rc) rc = (int)hipMemcpy(m->rope_tab, tab.data(), tab.size() * 4, hipMemcpyHostToDevice);
         if (!rc) rc = spy_exact_luts(&m->lut);
         if (!rc) rc = spy_ensure_lds(m, (const void *)xattn_pv_kernel<0>, xattn_pv_lds(c.n_ctx));
-        if (!rc) rc = spy_ensure_lds(m, (const void *)xattn_scores_kernel<0>, xattn_scores_lds(c.n_head));
         if (!rc) rc = spy_attn_short_prepare(c.n_ctx);
         if (!rc) {
             m->exact_ok = true;
@@ -243,10 +242,10 @@ static int enqueue_one(spy_hip_llama *m, hipStream_t st, int which, int il, int 
         const bool one_launch = attn_one_launch(m, kv_bound);
         if (which == K_SCORES) {
             if (m->dry || one_launch) return 0;
-            // one workgroup per compute unit; tests have fewer, so that a workgroup's share of the tokens takes several rounds of
-            // XS_TOK, as it would on a part with fewer compute units or a longer cache
+            // one workgroup per compute unit; tests have fewer, so that a wave's share of the tokens takes more units than it has in flight, as it would
+            // on a part with fewer compute units or a longer cache
             const int sgrid = m->scores_grid ? m->scores_grid : m->num_cu;
-            xattn_scores_kernel<0><<<dim3((unsigned)sgrid), dim3(XS_THREADS), xattn_scores_lds(c.n_head), st>>>(
+            xattn_scores_kernel<0><<<dim3((unsigned)max(sgrid, (c.n_head + 15) / 16)), dim3(XS_THREADS), 0, st>>>(
                 m->st, m->pos_imm, m->q16, m->k_cache[il], m->scores, c.n_head, c.n_ctx, 1.0f / sqrtf((float)m->hd));   // SoftmaxParam::scale (attention.cpp:113)
             return SPY_LAUNCH_RC();
         }
@@ -1019,9 +1018,8 @@ extern "C" int spy_hip_attn_decode(void *stream, int32_t order, const void *q16,
     RC_TRY(f.init(order, n_head * 128, n_head, n_head * 128, 1, n_ctx, SPY_HIP_Q4_0));
     const size_t pv_lds = (size_t)n_ctx * 6 + 16;
     if (order == 1) {
-        if (n_ctx > 512 * XP_NP || xattn_pv_lds((int)n_ctx) > 160 * 1024 - 256 || xattn_scores_lds(n_head) > 160 * 1024) return SPY_HIP_EUNSUPPORTED;
+        if (n_ctx > XA_MAX_CTX || n_head > XA_MAX_HEAD) return SPY_HIP_EUNSUPPORTED;
         RC_TRY(spy_ensure_lds(&f.m, (const void *)xattn_pv_kernel<0>, xattn_pv_lds((int)n_ctx)));
-        RC_TRY(spy_ensure_lds(&f.m, (const void *)xattn_scores_kernel<0>, xattn_scores_lds(n_head)));
         RC_TRY(spy_attn_short_prepare((int)n_ctx));
     } else {
         if (pv_lds > 160 * 1024) return SPY_HIP_EUNSUPPORTED;

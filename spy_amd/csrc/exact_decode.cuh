@@ -463,13 +463,8 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(xg_args a) {
 }
 
 // ---- attention scores in the order of Dot<FP16,FP16> -------------------------------------------------------------------
-// The cached tokens are dealt out evenly over the workgroups (one per compute unit): workgroup b takes tokens
-// b * tpw .. (b + 1) * tpw - 1, tpw = ceil(n_kv / workgroups), all heads, in rounds of XS_TOK tokens.  The keys of a round
-// (8 KiB per token, [head][128] fp16) are read coalesced, XS_NLD 16-byte pieces per thread all requested at once and a
-// round ahead of their use, and laid into LDS; then ONE thread per (token, head) key walks the dot exactly as vec_dot.h:124-145 does for n = 128:
-// accumulators sum[j][l] over the chunks i = 0, 32, 64 (i + 32 < n), the reduction tree of FP16::block_reduce, then the
-// scalar tail over elements 96..127 (a product of two fp16 values is exact in fp32, so `tail += a * b` is the fma it is
-// written as here), result = tail + simd.  Stored: t = dot * scale (mask 0, then * scale: non-linear.cpp:141-150).
+// result = tail + simd as vec_dot.h:124-145 has it for n = 128: accumulators sum[j][l] over the chunks i = 0, 32, 64 (i + 32 < n), the reduction tree of
+// FP16::block_reduce, then the scalar tail over elements 96..127.  Stored: t = dot * scale (mask 0, then * scale: non-linear.cpp:141-150).
 typedef uint32_t xp_u4 __attribute__((ext_vector_type(4)));
 // ---- what the attention kernels of one token (the two below, attn_short.hip) share: the order of Dot<FP16,FP16> lies here and nowhere else.  A product of two fp16
 // values is exact in fp32, so `sum + a * b` is the fma it is written as.
@@ -528,109 +523,64 @@ static __device__ __forceinline__ float xa_tree32(float acc) {
         const uint32_t wv = tv[e >> 3][(e >> 1) & 3], wq = tq[e >> 3][(e >> 1) & 3]; \
         if (e < ntail) tail = fmaf(h2f((uint16_t)(e & 1 ? wv >> 16 : wv & 0xFFFFu)), h2f((uint16_t)(e & 1 ? wq >> 16 : wq & 0xFFFFu)), tail); \
     }
+#define XA_MAX_CTX 4736                                 // longest cache, most heads of the attention kernels of one token
+#define XA_MAX_HEAD 33
 #define XS_THREADS 1024
-#define XS_TOK 18
-#define XS_NLD 9                                        // pieces per thread requested together: 1024 x 9 x 16 bytes = 18 tokens of 32 heads
-static inline size_t xattn_scores_lds(int n_head) { return (size_t)(XS_TOK + 1) * n_head * 16 * 16; }
-// kc is not a restrict pointer on purpose: the loads of the next round must stay where they are written, ahead of the
-// barrier and the dots of the current round, so that they are in flight meanwhile.
+#define XS_NU 3                                         // units of a wave in flight (2 and 4: the same)
+// A unit is the keys of 16 heads of one token (4 KiB in a row), four adjacent lanes per key: lane `part` has the 16 bytes of accumulators (part, l) of every
+// chunk, straight from memory, and its head's part of q in registers.  The tail goes down the four lanes, eight elements each.  The tokens are dealt out evenly over the
+// workgroups of a head group, a workgroup's over its waves, so that it writes neighbouring scores.
+// What bounds it: the keys at 5.5 TB/s behind launch, position and first wait (4100 tokens: 33.6 MB in 8.5 us).  Through LDS, one thread per key, the dots began when the last
+// key of a round was there and then took 1.6 us: 4100 tokens 10.0 -> 8.5 us, 3000 7.9 -> 6.8, 2060 6.8 -> 5.7, 1100 5.2 -> 4.6, 600 4.4 -> 3.9; here a wave's
+// dots follow its own keys, and what is left after the last ones is one chain of 32 fmas.
+// kc is not a restrict pointer on purpose: the loads must stay where they are written, ahead of the dots of the units before.
 template <int DUMMY>
 __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_state *st, int pos_imm, const uint16_t *__restrict__ q16, const uint16_t *kc,
                                                                   float *__restrict__ scores, int n_head, int n_ctx, float scale) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), part = lane & 3;
+    const int ng = (n_head + 15) >> 4, nb = (int)gridDim.x / ng, tb = (int)blockIdx.x / ng, hg = (int)blockIdx.x - tb * ng;
     const int n_kv = (st ? st->pos : pos_imm) + 1;
-    const int tpw = (n_kv + (int)gridDim.x - 1) / (int)gridDim.x;
-    const int t_begin = blockIdx.x * tpw, t_end = min(n_kv, t_begin + tpw);
-    if (t_begin >= t_end) return;
-    const int d = n_head * 128, tid = threadIdx.x;
-    uint4 *s_k = (uint4 *)smem;                         // [XS_TOK][n_head][16 chunks of 16 bytes], chunk index rotated per key against bank conflicts
-    uint4 *s_qh = s_k + XS_TOK * n_head * 16;           // [n_head][16]
-    const int per_tok = n_head * 16;                    // 16-byte pieces per token
-    // the pieces in flight
-    xp_u4 kr[XS_NLD];
-    // piece u of a thread: token and place in it; the quotient by multiplication with 2^32 / per_tok rounded up, exact for the few thousand pieces there are
-    const uint32_t inv = 0xFFFFFFFFu / (uint32_t)per_tok + 1u;
-    auto pieces = [&](auto f) {
-        int c0 = tid;
-        asm volatile("" : "+v"(c0));                     // worked out again each time: kept over the dots they would not fit the registers
+    const int tpw = (n_kv + nb - 1) / nb, t_end = min(n_kv, (tb + 1) * tpw);
+    int t = tb * tpw + wave;
+    if (tb >= nb || t >= t_end) return;
+    const int hh = hg * 16 + (lane >> 2), h = min(hh, n_head - 1);
+    const size_t d = (size_t)n_head * 128;
+    const uint16_t *qp = q16 + h * 128 + part * 8, *kp = kc + h * 128 + part * 8;
+    uint4 q[4];
+    xp_u4 k[XS_NU][4];
 #pragma unroll
-        for (int u = 0; u < XS_NLD; u++) {
-            const int c = c0 + u * XS_THREADS, tt = (int)__umulhi((uint32_t)c, inv);
-            f(u, tt, c - tt * per_tok);
-        }
+    for (int i = 0; i < 4; i++) q[i] = *(const uint4 *)(qp + 32 * i);
+    auto request = [&](int u, int tt) {
+        if (tt >= t_end) return;
+#pragma unroll
+        for (int i = 0; i < 4; i++) k[u][i] = *(const xp_u4 *)(kp + (size_t)tt * d + 32 * i);
     };
-    auto request = [&](int t0, int nt, int tb) {
-        pieces([&](int u, int tt, int rem) {
-            if (u < 5 || tb * per_tok + 5 * XS_THREADS < nt * per_tok) kr[u] = *(const xp_u4 *)(kc + (size_t)(t0 + min(tb + tt, nt - 1)) * d + rem * 8);
-        });
-    };
-    // a workgroup with few keys: at most four pieces per thread, four threads per key
-    const int nt_all = t_end - t_begin;
-    const bool few = nt_all * n_head * 4 <= XS_THREADS && nt_all <= XS_TOK;
-    auto lay = [&](int nt, int tb) {
-        pieces([&](int u, int tt, int rem) {
-            const int t = tb + tt, hh = rem >> 4, ch = rem & 15;
-            if (t < nt) *(xp_u4 *)&s_k[(t * n_head + hh) * 16 + ((ch + t + 8 * (hh & 1)) & 15)] = kr[u];
-        });
-    };
-    // SP = 1: one thread walks a key; 4, where the workgroup's keys leave threads for it: four adjacent threads, thread `part` with the accumulators of
-    // j = part (one thread alone takes 1.6 us for its 128 elements).  No form between them: the kernels of a layer together fill the 64 KB
-    // instruction cache, and what does not fit costs every kernel 0.5 to 1 us.
-    auto dots = [&](auto sp, int t0, int nt) {
-        constexpr int SP = decltype(sp)::value, NJ = 4 / SP;
-        for (int base = 0; base < nt * n_head * SP; base += XS_THREADS) {
-            const int w = base + tid, key = w / SP, part = w % SP;
-            if (key >= nt * n_head) break;
-            const int hh = key / nt, tt = key - hh * nt;
-            const uint4 *kp = s_k + (tt * n_head + hh) * 16, *qp = s_qh + hh * 16;
-            const int rot = tt + 8 * (hh & 1);
-            float sum[NJ][8];
 #pragma unroll
-            for (int j = 0; j < NJ; j++)
+    for (int u = 0; u < XS_NU; u++) request(u, t + 16 * u);
+    for (; t < t_end; t += 16 * XS_NU) {
 #pragma unroll
-                for (int l = 0; l < 8; l++) sum[j][l] = 0.0f;
+        for (int u = 0; u < XS_NU; u++) {
+            const int tt = t + 16 * u;
+            if (tt >= t_end) break;
+            uint4 kv[4];
 #pragma unroll
-            for (int i = 0; i < 3; i++) {                // chunks of 32 elements = 4 x 16 bytes
-                __builtin_amdgcn_sched_barrier(0);      // one chunk's LDS reads at a time: the next round's keys occupy registers meanwhile
+            for (int i = 0; i < 4; i++) kv[i] = make_uint4(k[u][i].x, k[u][i].y, k[u][i].z, k[u][i].w);
+            float sum[8];
 #pragma unroll
-                for (int j = 0; j < NJ; j++) {
-                    const int jj = part + j * SP;
-                    xa_fma8(sum[j], kp[(4 * i + jj + rot) & 15], qp[4 * i + jj]);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (SP == 1) {
+            for (int l = 0; l < 8; l++) sum[l] = 0.0f;
 #pragma unroll
-                for (int l = 0; l < 8; l++) { sum[0][l] += sum[2][l]; sum[1][l] += sum[3][l]; sum[0][l] += sum[1][l]; }
-            } else xa_quad(sum[0]);
-            const float simd = xa_tree8(sum[0]);
+            for (int i = 0; i < 3; i++) xa_fma8(sum, kv[i], q[i]);
+            xa_quad(sum);
+            const float simd = xa_tree8(sum);
             float tail = 0.0f;
 #pragma unroll
-            for (int j = 0; j < 4; j++) tail = xa_tail8(tail, kp[(12 + j + rot) & 15], qp[12 + j]);
-            if (part == 0) scores[(size_t)hh * n_ctx + t0 + tt] = (tail + simd) * scale;
+            for (int j = 0; j < 4; j++) {
+                if (j) tail = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(tail), 0x90, 0xF, 0xF, true));      // quad_perm [0, 0, 1, 2]
+                tail = xa_tail8(tail, kv[3], q[3]);
+            }
+            if (part == 3 && hh < n_head) scores[(size_t)h * n_ctx + tt] = (tail + simd) * scale;
+            request(u, tt + 16 * XS_NU);
         }
-    };
-    constexpr int TB = XS_NLD * XS_THREADS;              // pieces per request of the workgroup
-    if (few) pieces([&](int u, int tt, int rem) { if (u < 4 && u * XS_THREADS < nt_all * per_tok) kr[u] = *(const xp_u4 *)(kc + (size_t)(t_begin + min(tt, nt_all - 1)) * d + rem * 8); });
-    else request(t_begin, min(XS_TOK, nt_all), 0);
-    for (int c = tid; c < per_tok; c += XS_THREADS) s_qh[c] = *(const uint4 *)(q16 + c * 8);
-    if (few) {
-        pieces([&](int u, int tt, int rem) {
-            const int hh = rem >> 4, ch = rem & 15;
-            if (u < 4 && tt < nt_all) *(xp_u4 *)&s_k[(tt * n_head + hh) * 16 + ((ch + tt + 8 * (hh & 1)) & 15)] = kr[u];
-        });
-        __syncthreads();
-        dots(std::integral_constant<int, 4>{}, t_begin, nt_all);
-        return;
-    }
-    for (int t0 = t_begin; t0 < t_end; t0 += XS_TOK) {
-        const int nt = min(XS_TOK, t_end - t0);
-        if (t0 != t_begin) __syncthreads();             // the previous round's keys have been read
-        lay(nt, 0);                                     // the first batch of the round was requested a round ahead
-        for (int tb = TB / per_tok; tb < nt; tb += TB / per_tok) { request(t0, nt, tb); lay(nt, tb); }
-        if (t0 + XS_TOK < t_end) request(t0 + XS_TOK, min(XS_TOK, t_end - t0 - XS_TOK), 0);
-        __syncthreads();
-        dots(std::integral_constant<int, 1>{}, t0, nt);
     }
 }
 

@@ -242,10 +242,9 @@ def test_attn_decode_short_cache(hip, n_head, n_kv, n_ctx, monkeypatch):
 
 @pytest.mark.parametrize("grid,n_kv", [(64, 4351), (7, 300), (100, 1900)])
 def test_attn_scores_in_several_rounds(hip, grid, n_kv, monkeypatch):
-    """The score kernel of order 1 deals the cached tokens out over its workgroups and takes a workgroup's share in rounds of 18
-    tokens, the next round's keys requested while the current round is multiplied.  With one workgroup per compute unit of this
-    part a share never exceeds one round at the supported cache lengths; SPY_HIP_SCORES_GRID forces fewer workgroups, so that the
-    rounds (full ones, a short last one, workgroups without tokens) are exercised: same bits as the one-round launch."""
+    """The score kernel of order 1 deals the cached tokens out over its workgroups and waves, three tokens of a wave in flight.  With one workgroup per
+    compute unit of this part a wave has no more than three at the supported cache lengths; SPY_HIP_SCORES_GRID forces fewer workgroups, so that later
+    requests (full rounds, a short last one, workgroups without tokens) are exercised: same bits as the one-round launch."""
     from tests.gpu_util import dev, dev_empty, call
     H_, hd, n_ctx = 32, 128, 4352
     d = H_ * hd
@@ -266,6 +265,25 @@ def test_attn_scores_in_several_rounds(hip, grid, n_kv, monkeypatch):
         res.append((ds.download(np.uint32).reshape(H_, n_ctx)[:, :n_kv].copy(), do.download(np.uint32).copy()))
     assert np.array_equal(res[0][0], res[1][0]), "scores differ between one round and %d workgroups" % grid
     assert np.array_equal(res[0][1], res[1][1])
+
+
+@pytest.mark.parametrize("n_head,n_kv", [(1, 577), (16, 593), (17, 1033), (31, 700)])
+def test_attn_decode_head_groups(hip, oracle, n_head, n_kv):
+    """Scores are formed for groups of 16 heads: full ones, a last one of one or 15 heads, one head alone."""
+    from tests.gpu_util import dev, dev_empty, call
+    hd, n_ctx, d = 128, 1040, n_head * 128
+    rng = np.random.default_rng(n_head)
+    q16, kc, vc = rng.standard_normal(d).astype(np.float16), rng.standard_normal((n_ctx, d)).astype(np.float16), rng.standard_normal((d, n_ctx)).astype(np.float16)
+    S = np.zeros((n_head, 1, n_kv), np.float32)
+    assert oracle.spy_o_matmul(B(O.tensor(kc.view(np.uint16), O.F16, [hd, n_kv, n_head], nb=[2, 2 * d, 2 * hd])),
+                               B(O.tensor(q16.astype(np.float32), O.F32, [hd, 1, n_head], nb=[4, 4 * d, 4 * hd])), B(O.tensor(S, O.F32, [n_kv, 1, n_head])), 8) == 0
+    dq, dk, dv = dev(q16.view(np.uint16)), dev(kc.view(np.uint16)), dev(vc.view(np.uint16))
+    ds, do = dev_empty((n_head * n_ctx + 64) * 4, 0xEE), dev_empty(d * 4, 0xEE)
+    call(hip.load().spy_hip_attn_decode, None, 1, dq.ptr, dk.ptr, dv.ptr, n_head, n_kv, n_ctx, ds.ptr, do.ptr)
+    got = ds.download(np.uint32)
+    want = (S[:, 0, :] * (np.float32(1.0) / np.sqrt(np.float32(hd)))).astype(np.float32)
+    assert np.array_equal(got[:n_head * n_ctx].reshape(n_head, n_ctx)[:, :n_kv], want.view(np.uint32))
+    assert (got[:n_head * n_ctx].reshape(n_head, n_ctx)[:, n_kv:] == 0xEEEEEEEE).all() and (got[n_head * n_ctx:] == 0xEEEEEEEE).all()
 
 
 def _running_sum_ref(t):

@@ -348,7 +348,16 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(xg_args a) {
         if (EPI == EPI_QKV && r == 2) load_tile<WTV, 64, NITK>(tv, row_ptr(r), npair, lane);
         else load_tile<WT, 64, NITK>(t[r % RING], row_ptr(r), npair, lane);
     };
+    // What the epilogue needs from memory is requested ahead where that pays: the residual of rows of several slabs with the activations (11008 columns Q4_0 9.7 -> 9.5 us,
+    // Q6_K 11.85 -> 11.78; rows of one slab: 5.1 both ways, Q8_0 6.1 -> 6.3), the rotation of a pair ahead of the rows (qkv 10.82 -> 10.75; behind them 10.95).
+    constexpr bool RS_AHEAD = EPI == EPI_RESID && NITK > 1;
+    float rs = 0.0f;
+    if constexpr (RS_AHEAD) { if (a.resid) rs = a.resid[min((int)blockIdx.x * XG_WAVES + tid / NCH % XG_WAVES, a.M - 1)]; }
+    const int pos = EPI != EPI_QKV ? 0 : a.st ? a.st->pos : a.pos_imm;
+    float2 cs = make_float2(0.0f, 0.0f);
     auto issue_first = [&]() {
+        if constexpr (EPI == EPI_QKV)
+            cs = *(const float2 *)(a.rope_tab + (size_t)(pos - a.rope_row0) * a.hd + (2 * ((int)blockIdx.x * XG_WAVES + tid / (2 * NCH) % XG_WAVES)) % a.d % a.hd);
         if constexpr (!NORM) __builtin_amdgcn_s_barrier();      // x of every wave ahead of every wave's rows in the compute unit's memory queue
 #pragma unroll
         for (int r = 0; r < NROW; r++) if (r < DEPTH && r >= PRE) {
@@ -377,6 +386,9 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(xg_args a) {
     static_assert(NITK == 1 || NROW == 1, "rows longer than one slab are walked one row per wave");
     act_frag<1> af, av;
     int n8[16];
+    // gate|up: the SiLU table's answers are awaited after the last step only (Q4_0 15.38 -> 15.08 us, Q4_K 14.26 -> 13.86; Q8_0 has no registers left for it: 21.3 -> 21.5)
+    constexpr bool LATE = EPI == EPI_GATEUP && WT != SPY_HIP_Q8_0;
+    float up[LATE ? NSTEP : 1], sl[LATE ? NSTEP : 1];
 #pragma unroll
     for (int step = 0; step < NSTEPS; step++) {
         const int r0 = EPI == EPI_QKV ? 2 * step : step * RPS;                  // first row of the step
@@ -436,19 +448,19 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(xg_args a) {
         const int ogw = (int)blockIdx.x * XG_WAVES + ow;
         if constexpr (EPI == EPI_RESID || EPI == EPI_STORE) {
             const int u = (ogw + step * NW) * RPS + oj;
-            if (owner && u < a.M) a.out[u] = (EPI == EPI_RESID && a.resid) ? acc + a.resid[u] : acc;       // Add(KQV_linear, x) / Add(ffn_out, ffn_input); no resid: the MatMul alone
+            if (owner && u < a.M) a.out[u] = (EPI == EPI_RESID && a.resid) ? acc + (RS_AHEAD ? rs : a.resid[u]) : acc;       // Add(KQV_linear, x) / Add(ffn_out, ffn_input); no resid: the MatMul alone
         } else if constexpr (EPI == EPI_GATEUP) {
-            const float up = __shfl_xor(acc, nch, SPY_WAVE);                   // the row after (up_i) sits nch lanes further
+            const float u = __shfl_xor(acc, nch, SPY_WAVE);                    // the row after (up_i) sits nch lanes further
             const int i = ogw + step * NW;
-            if (owner && oj == 0 && i < a.M) a.out[i] = up * a.lut[65536 + f2h(acc)];             // Mul(ffn_up, Silu(ffn_gate)) (ffn.cpp:24-35, non-linear.cpp:11-14)
+            if constexpr (LATE) {
+                up[step] = u;
+                if (owner && oj == 0 && i < a.M) sl[step] = a.lut[65536 + f2h(acc)];
+            } else if (owner && oj == 0 && i < a.M) a.out[i] = u * a.lut[65536 + f2h(acc)];       // Mul(ffn_up, Silu(ffn_gate)) (ffn.cpp:24-35, non-linear.cpp:11-14)
         } else {
-            const int pos = a.st ? a.st->pos : a.pos_imm;
-            const float *rt = a.rope_tab + (size_t)(pos - a.rope_row0) * a.hd;
             if (step == 0) {
                 const float x1 = __shfl_xor(acc, nch, SPY_WAVE);
                 if (owner && oj == 0 && ogw < a.d) {
-                    const int row = (2 * ogw) % a.d, k2 = row % a.hd;
-                    const float c = rt[k2], sn = rt[k2 + 1];
+                    const float c = cs.x, sn = cs.y;
                     // (x0, x1) -> (x0*c - x1*s, x0*s + x1*c), every product rounded (non-linear.cpp:349-364)
                     const float pa_ = acc * c, pb_ = x1 * sn, pc_ = acc * sn, pd_ = x1 * c;
                     const uint32_t pr = (uint32_t)f2h(pa_ - pb_) | ((uint32_t)f2h(pc_ + pd_) << 16);
@@ -458,6 +470,14 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(xg_args a) {
             } else {
                 if (owner && ogw < a.d) a.vc[(size_t)ogw * a.n_ctx + pos] = f2h(acc);                 // VCache_cpy: [d][C] column pos
             }
+        }
+    }
+    if constexpr (LATE) {
+        const bool owner = tid < XG_WAVES * 2 * NCH && tid % (2 * NCH) == 0;
+#pragma unroll
+        for (int step = 0; step < NSTEP; step++) {
+            const int i = (int)blockIdx.x * XG_WAVES + tid / (2 * NCH) + step * NW;
+            if (owner && i < a.M) a.out[i] = up[step] * sl[step];
         }
     }
 }

@@ -19,6 +19,7 @@
 #pragma once
 
 #include "decode_kernels.cuh"
+#include "exact_exp.cuh"
 #include "exact_sum.cuh"
 
 #define XG_THREADS 1024
@@ -605,154 +606,233 @@ __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_stat
 }
 
 // ---- softmax + P.V^T in the host order ---------------------------------------------------------------------------------
-// One 1024-thread workgroup per (head, 16 rows of V^T); wave w streams row w into registers (16-byte pieces, all requested
-// before the softmax's serial sum so that the row arrives while that sum is walked).
-// Softmax (non-linear.cpp:129-180): m = max t; e = exp_table[fp16(t - m)]; sum = std::reduce(e) = groups of four added to
+// One 1024-thread workgroup per (head, 16 rows of V^T).  Waves 0..7 do the softmax and then the product, waves 8..15 bring two rows of V^T each into LDS meanwhile.
+// Softmax (non-linear.cpp:129-180): m = max t; e = exp_table[fp16(t - m)] (exact_exp.cuh); sum = std::reduce(e) = groups of four added to
 // one running sum, then the last n % 4 elements; p = e * (1 / sum), rounded to fp16 for the product (mat.cpp:37).
 // P.V^T (vec_dot.h:124-145 with n = n_kv): output row r has 4 x 8 accumulators, accumulator (j, l) adds elements
-// 32 i + 8 j + l for every chunk with 32 i + 32 < n_kv.  The 16 waves lay their rows into LDS; then 32 lanes hold the
-// accumulators of one row (two rows per wave, the 16 rows in waves 0..7) and read V^T and P from LDS; tree; scalar tail (the
+// 32 i + 8 j + l for every chunk with 32 i + 32 < n_kv.  32 lanes hold the accumulators of one row (two rows per wave); tree; scalar tail (the
 // last 1..32 elements, by the lane of accumulator 0).
+// Rows and probabilities lie in LDS by accumulator, not by token, so that a lane reads the elements of eight of its steps at once: a wave's 128-bit read costs the
+// compute unit 4 clocks, a 16-bit one 2.7 (measured), and the walk took 2 us of them, 0.6 now.  The rows are turned on the way: a lane
+// asks for the same octet of eight chunks, which 32 byte permutes turn into eight octets of one accumulator each.
+// What bounds it: from 3500 tokens or so on the rows (16 per compute unit at 24 B/ns, then 0.6 us to write them to LDS and 0.6 to walk them), below the softmax's
+// chain of latencies.  The waves of the softmax meet on counters in LDS: at a workgroup barrier they would wait until the other eight have
+// asked for all their rows, which takes as long as the rows take to come.  All 16 waves taking part in both, with the table's gathers in the same memory
+// queue as the rows: 4100 tokens 12.7 us, 4000 12.7, 3000 11.5, 2060 9.4, 1500 9.2, 600 7.5; now 10.2, 9.9, 8.8, 8.2, 7.9, 6.7.  With this layout and
+// list but all waves in both: 11.5, -, 9.3, 8.5, 8.1, 6.8.  Scores asked for before the position is known: 10.7, 10.4, 9.2, 8.3, 8.0, 6.8.
 #define XP_THREADS 1024
-#define XP_NP 10                           // 16-byte pieces per lane of a V^T row: n_ctx <= 5120
-#define XP_NS 5                            // scores per thread: n_ctx <= 5120
-static inline int xattn_pv_vstride(int n_ctx) { return ((n_ctx + 63) / 64) * 64 + 32; }        // halfs between rows in LDS: = 64 bytes mod 128, the two rows of a wave on different banks
-static inline size_t xattn_pv_lds(int n_ctx) {
-    const size_t p_bytes = (size_t)((n_ctx + 32 + 7) & ~7) * 2, v_bytes = (size_t)16 * xattn_pv_vstride(n_ctx) * 2 + 1024;      // + the walk's read-ahead
-    const size_t soft = (size_t)n_ctx * 4 + (size_t)(n_ctx / 4 + 31) / 32 * 160;                  // t / e and the group sums live where the rows go later
-    return p_bytes + (v_bytes > soft ? v_bytes : soft);
+#define XP_NP 10                           // 16-byte pieces per lane of a V^T row
+#define XP_NG 3                            // groups of four scores per thread of the softmax
+// Where an element lies in LDS: chunk c, accumulator a at [c & 1][4 (a & 7) + (a >> 3)][c >> 1], the last index
+// xattn_pv_sa long, an odd number of 16-byte pieces (32 lanes, 16 at a time, on banks of their own); up to XP_LAY tokens, those behind them as they come.
+#define XP_LAY 4608
+static __host__ __device__ inline int xattn_pv_sa(int n_ctx) { return (((n_ctx < XP_LAY ? n_ctx : XP_LAY) + 511) / 512 * 8) | 8; }
+static __host__ __device__ inline int xattn_pv_row(int n_ctx) { return 64 * xattn_pv_sa(n_ctx) + (n_ctx > XP_LAY ? XA_MAX_CTX - XP_LAY : 0) + 32; }       // halfs of a row: laid out, behind XP_LAY, its last chunk
+// what the softmax works in: group sums, the list of exact_exp.cuh; behind the rows, or over the last of them where LDS is full
+#define XP_LDS (160 * 1024 - 256)
+static __host__ __device__ inline int xattn_pv_soft(int n_ctx) { return (n_ctx / 4 + 31) / 32 * 160 + XE_WORDS * 4; }
+static __host__ __device__ inline int xattn_pv_soft_at(int n_ctx) {
+    const int end = 17 * xattn_pv_row(n_ctx) * 2, at = XP_LDS - xattn_pv_soft(n_ctx);
+    return end < at ? end : at & ~15;
 }
+static inline size_t xattn_pv_lds(int n_ctx) {
+    const int end = 17 * xattn_pv_row(n_ctx) * 2, soft = xattn_pv_soft_at(n_ctx) + xattn_pv_soft(n_ctx);
+    return end > soft ? end : soft;
+}
+// arrival and wait of waves of one workgroup on a counter in LDS (all of them resident, and none waits before it has arrived)
+static __device__ __forceinline__ void xp_arrive(uint32_t *c) { if ((threadIdx.x & 63) == 0) __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP); }
+static __device__ __forceinline__ void xp_await(uint32_t *c, uint32_t n) { while (__hip_atomic_load(c, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < n) __builtin_amdgcn_s_sleep(1); }
 template <int DUMMY>
 __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *st, int pos_imm, const float *__restrict__ scores, const uint16_t *vc,
                                                               float *attn_out, const float *__restrict__ lut, int n_ctx, long long *dbg) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    __shared__ float s_red[16];
+    __shared__ float s_red[8], s_rem[4];
     __shared__ float s_sum;
+    __shared__ uint32_t s_cnt[3];
     XSTAMP(dbg, 0);
     const int n_kv = (st ? st->pos : pos_imm) + 1;
     const int hd_ = blockIdx.x >> 3, dgrp = blockIdx.x & 7;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int VS = ((n_ctx + 63) / 64) * 64 + 32;
-    uint16_t *s_p = (uint16_t *)smem;                                 // n_ctx + 32 halfs: the probabilities as fp16
-    uint8_t *region = smem + (size_t)((n_ctx + 32 + 7) & ~7) * 2;
-    float *s_e = (float *)region;                                     // n_ctx floats: e (softmax phase)
-    float *s_grp = s_e + n_ctx;                                       // n_ctx / 4 group sums
-    uint16_t *s_v = (uint16_t *)region;                               // 16 rows x VS halfs (product phase)
-    const float *srow = scores + (size_t)hd_ * n_ctx;
-    const uint16_t *vrow = vc + (size_t)(hd_ * 128 + dgrp * 16 + wave) * n_ctx;
-    // ---- softmax: scores -> registers, maximum ----
-    float sreg[XP_NS];
+    const int SA = xattn_pv_sa(n_ctx), RS = xattn_pv_row(n_ctx), REST = RS - 64 * SA - 32;
+    uint16_t *s_p = (uint16_t *)smem, *s_v = s_p + RS;                // the probabilities as fp16, 16 rows of V^T
+    float *s_grp = (float *)(smem + xattn_pv_soft_at(n_ctx));
+    uint32_t *s_code = (uint32_t *)(s_grp + (n_ctx / 4 + 31) / 32 * 40);
+    const int last_piece = (n_kv - 1) >> 3, nfull = (n_kv - 1) / 32;  // chunks with 32 i + 32 < n_kv
+    const int ngrp = n_kv / 4, nall = (n_kv + 3) / 4;
+    if (tid < 3) s_cnt[tid] = 0;
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+    f4 v[XP_NG];
+    xp_u4 cd = {0, 0, 0, 0};
+    if (wave < 8) {
+        const float *srow = scores + (size_t)hd_ * n_ctx;
 #pragma unroll
-    for (int u = 0; u < XP_NS; u++) sreg[u] = srow[min(tid + u * XP_THREADS, n_ctx - 1)];
-    // The V^T rows: nothing beyond the last cached token is asked for.  Rows of up to 1024 tokens are on their way beside the scores; the
-    // pieces of longer ones would stand before the table gathers in the memory queue (4096 tokens 13.9 -> 14.1 us with four of eight ahead).  From 3072
-    // tokens on, two pieces of a row follow right behind the gathers (4096 tokens 13.8 -> 12.7 us, 3000 11.65 -> 11.55; 2500 10.6 -> 11.2:
-    // there the stream is shorter than what the wait for their issue costs).
-    // vc is not a restrict pointer on purpose: the loads must stay where they are written.
-    xp_u4 vb[XP_NP];
-    const int last_piece = (n_kv - 1) >> 3;
-    auto load_row = [&](int from, int to) {
-#pragma unroll
-        for (int i = 0; i < XP_NP; i++) if (i >= from && i < to && i * 64 <= last_piece) vb[i] = *(const xp_u4 *)(vrow + (size_t)min(i * 64 + lane, last_piece) * 8);
-    };
-    const bool early = n_kv <= 1024, ahead = n_kv > 3072;
-    if (early) load_row(0, 2);
-    float mx = -INFINITY;
-#pragma unroll
-    for (int u = 0; u < XP_NS; u++) if (tid + u * XP_THREADS < n_kv) mx = fmaxf(mx, sreg[u]);
-    mx = wave_max(mx);
-    if (lane == 0) s_red[wave] = mx;
-    __syncthreads();
-    mx = s_red[0];
-#pragma unroll
-    for (int w = 1; w < 16; w++) mx = fmaxf(mx, s_red[w]);
-    XSTAMP(dbg, 1);
-    // exponentials from the table (a gather of 64 entries takes 64 cycles: only where there are scores)
-#pragma unroll
-    for (int u = 0; u < XP_NS; u++) if (wave * 64 + u * XP_THREADS < n_kv) sreg[u] = lut[f2h(sreg[u] - mx)];
-    if (ahead) load_row(0, 2);
-#pragma unroll
-    for (int u = 0; u < XP_NS; u++) { const int j = tid + u * XP_THREADS; if (j < n_kv) s_e[j] = sreg[u]; }
-    __syncthreads();
-    XSTAMP(dbg, 2);
-    const int ngrp = n_kv / 4;
-    static_assert(XP_NS * XP_THREADS / 4 <= 2 * XP_THREADS, "two group sums per thread");
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-        const int g = tid + u * XP_THREADS;
-        if (g < ngrp) {
-            s_grp[xg_seg_at(g)] = xa_group(*(const float4 *)(s_e + 4 * g));
+        for (int u = 0; u < XP_NG; u++) {
+            const int g = min(tid + 512 * u, nall - 1);
+            if (512 * u < nall) {
+                if (4 * g + 3 < n_ctx) v[u] = *(const f4 *)(srow + 4 * g);
+                else v[u] = f4{srow[4 * g], srow[min(4 * g + 1, n_ctx - 1)], srow[min(4 * g + 2, n_ctx - 1)], srow[n_ctx - 1]};
+            }
         }
-    }
-    if (tid < 32) for (int g = ngrp + tid; g < ((ngrp + 31) & ~31); g += 32) s_grp[xg_seg_at(g)] = 0.0f;
-    __syncthreads();
-    XSTAMP(dbg, 3);
-    // Longer rows are requested now, by every wave but the one that walks the sum (a wave that asks for its whole row sits in the issue stage
-    // until the memory queue has room, i.e. for most of the row's transfer time): they arrive while the sum is walked.
-    auto rest = [&]() {
-        if (!early && !ahead) load_row(0, 2);
-        if (!early) load_row(2, XP_NP);
-    };
-    if (wave != 0) rest();
-    else {
-        float init = xg_segment_sum<2>(s_grp, ngrp);
-        for (int j = ngrp * 4; j < n_kv; j++) init = init + s_e[j];
-        if (lane == 0) s_sum = init;
-        rest();
+        if (tid < XE_WORDS / 4) cd = ((const xp_u4 *)(lut + XE_AT))[tid];
     }
     __syncthreads();
-    XSTAMP(dbg, 4);
-    const float inv = 1.0f / s_sum;
+    if (wave < 8) {
+        // ---- softmax ----
+        if (tid < XE_WORDS / 4) ((xp_u4 *)s_code)[tid] = cd;
+        float mx = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < XP_NS; u++) { const int j = tid + u * XP_THREADS; if (j < n_kv) s_p[j] = f2h(sreg[u] * inv); }
-    // ---- the rows into LDS (s_e / s_grp are dead: every thread passed the barrier after the sum) ----
-    {
-        uint16_t *dst = s_v + (size_t)wave * VS + lane * 8;
+        for (int u = 0; u < XP_NG; u++)
+            if (512 * u < nall) {
+                const int j = 4 * (tid + 512 * u);
 #pragma unroll
-        for (int i = 0; i < XP_NP; i++) if (i * 64 + lane <= last_piece) *(xp_u4 *)(dst + i * 512) = vb[i];
+                for (int i = 0; i < 4; i++) if (j + i < n_kv) mx = fmaxf(mx, v[u][i]);
+            }
+        mx = wave_max(mx);
+        if (lane == 0) s_red[wave] = mx;
+        xp_arrive(s_cnt);
+        xp_await(s_cnt, 8);
+        mx = s_red[0];
+#pragma unroll
+        for (int w = 1; w < 8; w++) mx = fmaxf(mx, s_red[w]);
+        XSTAMP(dbg, 1);
+#pragma unroll
+        for (int u = 0; u < XP_NG; u++) {
+            const int g = tid + 512 * u;
+            if (512 * u + 64 * wave < nall) {
+                float e[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    bool ask;
+                    e[i] = xe_exp(f2h(mx - v[u][i]), s_code, ask);
+                    if (__any(ask)) e[i] = ask ? lut[f2h(v[u][i] - mx)] : e[i];
+                }
+                v[u] = f4{e[0], e[1], e[2], e[3]};
+                if (g < ngrp) s_grp[xg_seg_at(g)] = xa_group(make_float4(e[0], e[1], e[2], e[3]));
+                else if (g < ((ngrp + 31) & ~31)) s_grp[xg_seg_at(g)] = 0.0f;
+                if (g == ngrp) { s_rem[0] = e[0]; s_rem[1] = e[1]; s_rem[2] = e[2]; }
+            } else if (g >= ngrp && g < ((ngrp + 31) & ~31)) s_grp[xg_seg_at(g)] = 0.0f;
+        }
+        xp_arrive(s_cnt + 1);
+        if (wave == 0) {
+            xp_await(s_cnt + 1, 8);
+            XSTAMP(dbg, 3);
+            float sum = xg_segment_sum<2>(s_grp, ngrp);
+            for (int j = ngrp * 4; j < n_kv; j++) sum = sum + s_rem[j & 3];
+            if (lane == 0) s_sum = sum;
+            xp_arrive(s_cnt + 2);
+        }
+        xp_await(s_cnt + 2, 1);
+        XSTAMP(dbg, 4);
+        const float inv = 1.0f / s_sum;
+#pragma unroll
+        for (int u = 0; u < XP_NG; u++) {
+            const int g = tid + 512 * u;
+            if (g < nall) {                                          // (of the last group also what lies behind the last token: not used)
+                uint16_t p[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) p[i] = f2h(v[u][i] * inv);
+                const uint2 pp = make_uint2(p[0] | ((uint32_t)p[1] << 16), p[2] | ((uint32_t)p[3] << 16));
+                if (g < XP_LAY / 4) {
+                    uint16_t *at = s_p + (((g >> 3) & 1) * 32 + ((g >> 1) & 3) + 16 * (g & 1)) * SA + (g >> 4);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) at[4 * i * SA] = p[i];
+                } else *(uint2 *)(s_p + 64 * SA + 4 * g - XP_LAY) = pp;
+                if (g >= 8 * nfull) *(uint2 *)(s_p + 64 * SA + REST + 4 * (g - 8 * nfull)) = pp;
+            }
+        }
+    } else {
+        // ---- two rows of V^T from memory to their places; nothing beyond the last cached token is asked for ----
+        // vc is not a restrict pointer on purpose: the loads must stay where they are written.
+        const uint16_t *vrow = vc + (size_t)(hd_ * 128 + dgrp * 16 + 2 * (wave - 8)) * n_ctx;
+        xp_u4 vb[2][XP_NP], vt[2];
+        const int u = lane >> 3, par = (lane >> 2) & 1, o = lane & 3;
+        const int walked = 4 * nfull;                                 // pieces of whole chunks; the last chunk, 1 .. 32 elements, goes apart
+        const bool mine = 64 * u + 4 * par < walked;
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            vt[r] = *(const xp_u4 *)(vrow + (size_t)r * n_ctx + (size_t)min(4 * nfull + o, last_piece) * 8);
+#pragma unroll
+            for (int i = 8; i < XP_NP; i++) if (64 * i < walked) vb[r][i] = *(const xp_u4 *)(vrow + (size_t)r * n_ctx + (size_t)min(64 * i + lane, walked - 1) * 8);
+        }
+        if (mine) {
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+#pragma unroll
+                for (int i = 0; i < 8; i++) vb[r][i] = *(const xp_u4 *)(vrow + (size_t)r * n_ctx + (size_t)min(64 * u + 8 * i + (lane & 7), walked - 1) * 8);
+        }
+        if (RS * 2 * (2 * (wave - 8) + 3) > xattn_pv_soft_at(n_ctx)) xp_await(s_cnt + 2, 1);       // the softmax works where these rows go
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            uint16_t *row = s_v + (size_t)(2 * (wave - 8) + r) * RS;
+            if (mine) {
+                uint16_t *dst = row + (par * 32 + o) * SA + 8 * u;
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    xp_u4 w;
+#pragma unroll
+                    for (int k = 0; k < 4; k++) w[k] = __builtin_amdgcn_perm(vb[r][2 * k + 1][e >> 1], vb[r][2 * k][e >> 1], e & 1 ? 0x07060302u : 0x05040100u);
+                    *(xp_u4 *)(dst + 4 * e * SA) = w;
+                }
+            }
+            if (512 + lane < walked) {
+                const int c = 128 + (lane >> 2);
+#pragma unroll
+                for (int e = 0; e < 8; e++) row[((c & 1) * 32 + 4 * e + o) * SA + (c >> 1)] = (uint16_t)(vb[r][8][e >> 1] >> (16 * (e & 1)));
+            }
+            if (576 + lane < walked) *(xp_u4 *)(row + 64 * SA + lane * 8) = vb[r][9];
+            if (lane < 4) *(xp_u4 *)(row + 64 * SA + REST + lane * 8) = vt[r];
+        }
     }
     __syncthreads();
     XSTAMP(dbg, 5);
     // ---- P . V^T ----
-    // One lane per accumulator: each step is two 16-bit LDS reads and one fma that takes the fp16 operands as they are; a
-    // wave issues an instruction every 2.6 ns or so whatever the other waves do, so the walk is spread over eight waves.
     if (wave < 8) {
-        const int nfull = (n_kv - 1) / 32;                            // chunks with 32 i + 32 < n_kv
-        const int r16 = wave * 2 + (lane >> 5), cl = lane & 31;       // row of the 16 and accumulator 8 j + l
-        const _Float16 *vr = (const _Float16 *)s_v + (size_t)r16 * VS + cl, *pr = (const _Float16 *)s_p + cl;
+        const int r16 = wave * 2 + (lane >> 5), cl = lane & 31, acl = 8 * (cl & 3) + (cl >> 2);       // row of the 16, place and accumulator 8 j + l
+        const uint16_t *vr = s_v + (size_t)r16 * RS;
+        const uint16_t *v0 = vr + cl * SA, *v1 = v0 + 32 * SA, *p0 = s_p + cl * SA, *p1 = p0 + 32 * SA;
         float acc = 0.0f;
         const int ntail = n_kv - 32 * nfull;                          // 1 .. 32
         // operands of the scalar tail, requested ahead of the walk (the 32 lanes of a row read the same addresses)
         xp_u4 tv[4], tq[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) { tv[u] = *(const xp_u4 *)(vr - cl + 32 * nfull + 8 * u); tq[u] = *(const xp_u4 *)(pr - cl + 32 * nfull + 8 * u); }
-        _Float16 va[8], pa[8], vb[8], pb[8];
-        auto ld = [&](_Float16 (&v)[8], _Float16 (&q)[8], int i) {   // up to 16 chunks beyond nfull are read and not used: the next row, or the slack after the last
+        for (int u = 0; u < 4; u++) { tv[u] = *(const xp_u4 *)(vr + 64 * SA + REST + 8 * u); tq[u] = *(const xp_u4 *)(s_p + 64 * SA + REST + 8 * u); }
+        struct chunks16 { xp_u4 v0, v1, p0, p1; };
+        auto ld = [&](chunks16 &x, int g) { x.v0 = *(const xp_u4 *)(v0 + 8 * g); x.v1 = *(const xp_u4 *)(v1 + 8 * g); x.p0 = *(const xp_u4 *)(p0 + 8 * g); x.p1 = *(const xp_u4 *)(p1 + 8 * g); };
+        auto run = [&](const chunks16 &x, int n) {
 #pragma unroll
-            for (int u = 0; u < 8; u++) { v[u] = vr[32 * (i + u)]; q[u] = pr[32 * (i + u)]; }
-        };
-        auto run = [&](const _Float16 (&v)[8], const _Float16 (&q)[8]) {
-#pragma unroll
-            for (int u = 0; u < 8; u++) acc = fmaf((float)v[u], (float)q[u], acc);
-        };
-        int i = 0;
-        const int n16 = nfull - nfull % 16;
-        if (n16) {
-            ld(va, pa, 0);
-            for (; i < n16; i += 16) {
-                ld(vb, pb, i + 8);
-                __builtin_amdgcn_sched_barrier(0);
-                run(va, pa);
-                __builtin_amdgcn_sched_barrier(0);
-                ld(va, pa, i + 16);
-                __builtin_amdgcn_sched_barrier(0);
-                run(vb, pb);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int c = 0; c < 16; c++) {
+                const xp_u4 &v = c & 1 ? x.v1 : x.v0, &p = c & 1 ? x.p1 : x.p0;
+                const int k = c >> 1;
+                const uint32_t vw = v[k >> 1], pw = p[k >> 1];
+                if (c < n) acc = fmaf(h2f((uint16_t)(k & 1 ? vw >> 16 : vw & 0xFFFFu)), h2f((uint16_t)(k & 1 ? pw >> 16 : pw & 0xFFFFu)), acc);
             }
+        };
+        const int nlay = min(nfull, XP_LAY / 32), ng = nlay / 16, glast = SA / 8 - 1;
+        chunks16 A, B;
+        ld(A, 0);
+        int g = 0;
+        for (; g + 2 <= ng; g += 2) {
+            ld(B, g + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            run(A, 16);
+            __builtin_amdgcn_sched_barrier(0);
+            ld(A, min(g + 2, glast));
+            __builtin_amdgcn_sched_barrier(0);
+            run(B, 16);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        for (; i < nfull; i++) acc = fmaf((float)vr[32 * i], (float)pr[32 * i], acc);
+        if (g < ng) { run(A, 16); g++; ld(A, min(g, glast)); }
+        run(A, nlay - 16 * g);
+        for (int c = nlay; c < nfull; c++) acc = fmaf(h2f(vr[64 * SA + 32 * c - XP_LAY + acl]), h2f(s_p[64 * SA + 32 * c - XP_LAY + acl]), acc);
         XSTAMP(dbg, 6);
-        acc = xa_tree32(acc);
+        // block_reduce of the 32 accumulators (xa_tree32's sums) at these places: a ^ 16 and a ^ 8 are lanes ^ 2 and ^ 1, a ^ 4 lane ^ 16, a ^ 1 and a ^ 2 lanes ^ 4 and ^ 8,
+        // which a mirror reaches where the four or eight lanes of a group agree
+#define XP_ADD(CTRL) acc += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc), CTRL, 0xF, 0xF, true));
+        XP_ADD(0x4E) XP_ADD(0xB1)
+        const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc), __float_as_uint(acc), false, false);
+        acc = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+        XP_ADD(0x141) XP_ADD(0x140)
+#undef XP_ADD
         float tail = 0.0f;
         XA_TAIL32(tail, tv, tq, ntail)                               // elements 32 nfull .. n_kv - 1
         if (cl == 0) attn_out[hd_ * 128 + dgrp * 16 + r16] = tail + acc;

@@ -12,6 +12,7 @@
 // angles come from the host's libm, and the outputs are the host backend's bit for bit.  The token loop
 // issues the prompt passes of a model in the host's order through these kernels as well (a thread-local
 // scope, spy_exact_thread_scope); its single-token passes have fused kernels of their own.
+#include "exact_exp.cuh"
 #include "common.cuh"
 
 #include <math.h>
@@ -40,7 +41,7 @@ __device__ __forceinline__ uint8_t *xat(const xdesc &t, int64_t i0, int64_t i1, 
 int g_exact = -1;          // -1: not decided yet (environment), 0 / 1
 // Per-device state, set up once per device and kept until the process ends (never freed, never replaced: a stream of
 // another thread may still read it), guarded by one mutex:
-//   lut    exp table [65536], then silu table [65536]; built by spy_exact_device_setup, which spy_hip_init calls
+//   lut    exp table [65536], then silu table [65536], then the list of exact_exp.cuh; built by spy_exact_device_setup, which spy_hip_init calls
 //   rope   the Rope tables (cos / sin of every position of a context) by parameter set; built by spy_hip_rope_prepare, or by
 //          the first exact-order Rope call with a new parameter set where that call is allowed to allocate (not under capture)
 #define XO_MAX_DEVICES 64
@@ -72,12 +73,23 @@ float host_h2f(uint16_t h) {
 
 // The reference's tables (lookup_table_impl/non-linear.h:39-47,131-139): entry k holds the function of
 // float(half k), evaluated by the host's libm in fp32; the loop stops before k = 0xFFFF, which stays 0.
+// Behind them the list of exact_exp.cuh.
+__global__ __launch_bounds__(64) void xe_code_kernel(const float *__restrict__ lut, uint32_t *__restrict__ codes) {
+    const uint32_t w = blockIdx.x * 64 + threadIdx.x;
+    if (w >= XE_WORDS) return;
+    uint32_t word = 0;
+    for (uint32_t i = 0; i < 16; i++) {
+        const uint32_t hx = w * 16 + i, off = hx <= XE_MAX ? __float_as_uint(lut[0x8000 + hx]) - __float_as_uint(xe_near(hx)) + 1 : 3;
+        word |= (off < 3 ? off : 3) << (2 * i);
+    }
+    codes[w] = word;
+}
 int device_luts(const float **lut) {
     const int dev = current_device();
     if (dev < 0) return SPY_HIP_EINVAL;
     std::lock_guard<std::mutex> lock(g_mu);
     if (g_dev[dev].lut) { *lut = g_dev[dev].lut; return 0; }
-    std::vector<float> h(2 * 65536, 0.0f);
+    std::vector<float> h(XE_AT + XE_WORDS, 0.0f);
     for (uint32_t k = 0; k < 0xFFFFu; k++) {
         const float v = host_h2f((uint16_t)k);
         h[k] = expf(v);
@@ -87,6 +99,11 @@ int device_luts(const float **lut) {
     hipError_t e = hipMalloc((void **)&d, h.size() * sizeof(float));
     if (e != hipSuccess) return (int)e;
     e = hipMemcpy(d, h.data(), h.size() * sizeof(float), hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        xe_code_kernel<<<dim3((XE_WORDS + 63) / 64), dim3(64)>>>(d, (uint32_t *)d + XE_AT);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) { (void)hipFree(d); return (int)e; }
     g_dev[dev].lut = d;
     *lut = d;

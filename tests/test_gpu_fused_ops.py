@@ -215,6 +215,37 @@ def test_attn_decode(hip, oracle, order, n_kv):
     _check(do.download(np.float32), out.reshape(-1), "attention output, n_kv %d" % n_kv, order)
 
 
+@pytest.mark.parametrize("n_kv,n_ctx", [(600, 600), (2048, 2048), (2049, 2056), (3584, 3584), (3585, 3592), (4097, 4352), (4128, 4352), (4129, 4352), (4608, 4608), (4609, 4616), (4640, 4736),
+                                        (4641, 4736), (4736, 4736)])
+def test_attn_decode_places_of_the_rows(hip, oracle, n_kv, n_ctx):
+    """Softmax and product at the edges of where a row of V^T lies in LDS: units of 512 tokens, 64 accumulator rows of an odd number of pieces, the group sums over the last
+    rows from 3592 tokens on, chunks 128 .. 143, those behind them; scores that spread over more than 104 (exp 0) and down to -inf, NaN behind the last token."""
+    from tests.gpu_util import dev, dev_empty, call
+    H_, hd = 2, 128
+    d = H_ * hd
+    rng = np.random.default_rng(n_kv)
+    q16 = (rng.standard_normal(d) * 30).astype(np.float16)
+    q16[hd:] /= np.float16(20)
+    kc, vc = np.full((n_ctx, d), np.nan, np.float16), np.full((d, n_ctx), np.nan, np.float16)
+    kc[:n_kv] = rng.standard_normal((n_kv, d)); vc[:, :n_kv] = rng.standard_normal((d, n_kv))
+    kc[5::97, 3] = -np.sign(q16[3]) * np.float16(np.inf)
+    kc[n_kv:] = np.nan
+    S = np.zeros((H_, 1, n_kv), np.float32)
+    P, out, mask = np.zeros_like(S), np.zeros((H_, 1, hd), np.float32), np.zeros((1, n_ctx), np.float32)
+    assert oracle.spy_o_matmul(B(O.tensor(kc.view(np.uint16), O.F16, [hd, n_kv, H_], nb=[2, 2 * d, 2 * hd])),
+                               B(O.tensor(q16.astype(np.float32), O.F32, [hd, 1, H_], nb=[4, 4 * d, 4 * hd])), B(O.tensor(S, O.F32, [n_kv, 1, H_])), 8) == 0
+    assert np.isneginf(S[0]).any() and not np.isnan(S).any()
+    assert oracle.spy_o_softmax(B(O.tensor(S, O.F32, [n_kv, 1, H_])), B(O.tensor(mask, O.F32, [n_ctx, 1])), B(O.tensor(P, O.F32, [n_kv, 1, H_])),
+                                float(np.float32(1.0) / np.sqrt(np.float32(hd)))) == 0
+    assert oracle.spy_o_matmul(B(O.tensor(vc.view(np.uint16), O.F16, [n_kv, hd, H_], nb=[2, 2 * n_ctx, 2 * n_ctx * hd])),
+                               B(O.tensor(P, O.F32, [n_kv, 1, H_])), B(O.tensor(out, O.F32, [hd, 1, H_])), 8) == 0
+    dq, dk, dv = dev(q16.view(np.uint16)), dev(kc.view(np.uint16)), dev(vc.view(np.uint16))
+    ds, do = dev_empty(H_ * n_ctx * 4, 0xEE), dev_empty(d * 4, 0xEE)
+    call(hip.load().spy_hip_attn_decode, None, 1, dq.ptr, dk.ptr, dv.ptr, H_, n_kv, n_ctx, ds.ptr, do.ptr)
+    got = do.download(np.uint32)
+    assert np.array_equal(got, out.reshape(-1).view(np.uint32)), "%d of %d differ" % (int((got != out.reshape(-1).view(np.uint32)).sum()), d)
+
+
 @pytest.mark.parametrize("n_head", [32, 3])
 @pytest.mark.parametrize("n_kv,n_ctx", [(1, 8), (3, 8), (4, 8), (5, 64), (31, 32), (32, 32), (33, 40), (63, 64), (64, 64), (65, 72), (255, 256), (257, 264), (511, 512), (512, 512),
                                         (513, 520), (575, 576), (576, 576), (576, 1024), (577, 584)])

@@ -245,7 +245,7 @@ static int enqueue_one(spy_hip_llama *m, hipStream_t st, int which, int il, int 
             // one workgroup per compute unit; tests have fewer, so that a wave's share of the tokens takes more units than it has in flight, as it would
             // on a part with fewer compute units or a longer cache
             const int sgrid = m->scores_grid ? m->scores_grid : m->num_cu;
-            xattn_scores_kernel<0><<<dim3((unsigned)max(sgrid, (c.n_head + 15) / 16)), dim3(XS_THREADS), 0, st>>>(
+            xattn_scores_kernel<0><<<dim3((unsigned)max(sgrid & ~7, 8)), dim3(XS_THREADS), 0, st>>>(
                 m->st, m->pos_imm, m->q16, m->k_cache[il], m->scores, c.n_head, c.n_ctx, 1.0f / sqrtf((float)m->hd));   // SoftmaxParam::scale (attention.cpp:113)
             return SPY_LAUNCH_RC();
         }
@@ -253,7 +253,7 @@ static int enqueue_one(spy_hip_llama *m, hipStream_t st, int which, int il, int 
             if (m->dry) return 0;
             if (one_launch)
                 return spy_attn_short(st, m->st, m->pos_imm, m->q16, m->k_cache[il], m->v_cache[il], m->scores, m->attn_out, m->lut, c.n_head, c.n_ctx, 1.0f / sqrtf((float)m->hd));
-            xattn_pv_kernel<0><<<dim3((unsigned)(c.n_head * 8)), dim3(XP_THREADS), xattn_pv_lds(c.n_ctx), st>>>(m->st, m->pos_imm, m->scores, m->v_cache[il], m->attn_out, m->lut, c.n_ctx, m->stamp_dbg);
+            xattn_pv_kernel<0><<<dim3((unsigned)c.n_head, 8), dim3(XP_THREADS), xattn_pv_lds(c.n_ctx), st>>>(m->st, m->pos_imm, m->scores, m->v_cache[il], m->attn_out, m->lut, c.n_ctx, m->stamp_dbg);
             return SPY_LAUNCH_RC();
         }
         const spy_hip_llama_layer &Lx = m->layers[which == K_HEAD ? 0 : il];

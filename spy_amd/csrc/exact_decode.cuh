@@ -548,23 +548,26 @@ static __device__ __forceinline__ float xa_tree32(float acc) {
 #define XA_MAX_HEAD 33
 #define XS_THREADS 1024
 #define XS_NU 3                                         // units of a wave in flight (2 and 4: the same)
-// A unit is the keys of 16 heads of one token (4 KiB in a row), four adjacent lanes per key: lane `part` has the 16 bytes of accumulators (part, l) of every
-// chunk, straight from memory, and its head's part of q in registers.  The tail goes down the four lanes, eight elements each.  The tokens are dealt out evenly over the
-// workgroups of a head group, a workgroup's over its waves, so that it writes neighbouring scores.
-// What bounds it: the keys at 5.5 TB/s behind launch, position and first wait (4100 tokens: 33.6 MB in 8.5 us).  Through LDS, one thread per key, the dots began when the last
-// key of a round was there and then took 1.6 us: 4100 tokens 10.0 -> 8.5 us, 3000 7.9 -> 6.8, 2060 6.8 -> 5.7, 1100 5.2 -> 4.6, 600 4.4 -> 3.9; here a wave's
+// A unit is 16 keys, four adjacent lanes per key: lane `part` has the 16 bytes of accumulators (part, l) of every chunk, straight from memory, and its head's part of q
+// in registers.  The tail goes down the four lanes, eight elements each.  The heads are dealt out over eight groups (heads g, g + 8, ...), a unit has one, two, four or eight
+// of them and tokens to match; workgroup b takes group b modulo 8, so that a head's keys are read and its scores written by one XCD, the one that reads
+// them next where the cache is long (in a pass 4100 tokens 8.58 -> 8.26 us against units of 16 heads of one token, 2060 5.62 -> 5.17, 1000 and 600 the same).  A group's tokens are
+// dealt out evenly over its workgroups, a workgroup's over its waves.
+// What bounds it: the keys at 5.5 TB/s behind launch, position and first wait (4100 tokens: 33.6 MB in 8.05 us).  Through LDS, one thread per key, the dots began when the last
+// key of a round was there and then took 1.6 us: 4100 tokens 9.9, 2060 6.7, 1000 and 600 4.83 us (now 4.75); here a wave's
 // dots follow its own keys, and what is left after the last ones is one chain of 32 fmas.
 // kc is not a restrict pointer on purpose: the loads must stay where they are written, ahead of the dots of the units before.
 template <int DUMMY>
 __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_state *st, int pos_imm, const uint16_t *__restrict__ q16, const uint16_t *kc,
                                                                   float *__restrict__ scores, int n_head, int n_ctx, float scale) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), part = lane & 3;
-    const int ng = (n_head + 15) >> 4, nb = (int)gridDim.x / ng, tb = (int)blockIdx.x / ng, hg = (int)blockIdx.x - tb * ng;
+    const int hs = n_head > 32 ? 3 : n_head > 16 ? 2 : n_head > 8 ? 1 : 0, nt = 16 >> hs;       // log2 of a unit's heads, its tokens
+    const int nb = (int)gridDim.x >> 3, tb = (int)blockIdx.x >> 3, hg = (int)blockIdx.x & 7;
     const int n_kv = (st ? st->pos : pos_imm) + 1;
-    const int tpw = (n_kv + nb - 1) / nb, t_end = min(n_kv, (tb + 1) * tpw);
-    int t = tb * tpw + wave;
+    const int tpw = ((n_kv + nb - 1) / nb + nt - 1) & -nt, t_end = min(n_kv, (tb + 1) * tpw);
+    int t = tb * tpw + wave * nt;
     if (tb >= nb || t >= t_end) return;
-    const int hh = hg * 16 + (lane >> 2), h = min(hh, n_head - 1);
+    const int hh = hg + 8 * ((lane >> 2) & ((1 << hs) - 1)), h = min(hh, n_head - 1), dt = lane >> (2 + hs);
     const size_t d = (size_t)n_head * 128;
     const uint16_t *qp = q16 + h * 128 + part * 8, *kp = kc + h * 128 + part * 8;
     uint4 q[4];
@@ -574,14 +577,14 @@ __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_stat
     auto request = [&](int u, int tt) {
         if (tt >= t_end) return;
 #pragma unroll
-        for (int i = 0; i < 4; i++) k[u][i] = *(const xp_u4 *)(kp + (size_t)tt * d + 32 * i);
+        for (int i = 0; i < 4; i++) k[u][i] = *(const xp_u4 *)(kp + (size_t)min(tt + dt, t_end - 1) * d + 32 * i);
     };
 #pragma unroll
-    for (int u = 0; u < XS_NU; u++) request(u, t + 16 * u);
-    for (; t < t_end; t += 16 * XS_NU) {
+    for (int u = 0; u < XS_NU; u++) request(u, t + 16 * nt * u);
+    for (; t < t_end; t += 16 * nt * XS_NU) {
 #pragma unroll
         for (int u = 0; u < XS_NU; u++) {
-            const int tt = t + 16 * u;
+            const int tt = t + 16 * nt * u;
             if (tt >= t_end) break;
             uint4 kv[4];
 #pragma unroll
@@ -599,14 +602,15 @@ __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_stat
                 if (j) tail = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(tail), 0x90, 0xF, 0xF, true));      // quad_perm [0, 0, 1, 2]
                 tail = xa_tail8(tail, kv[3], q[3]);
             }
-            if (part == 3 && hh < n_head) scores[(size_t)h * n_ctx + tt] = (tail + simd) * scale;
-            request(u, tt + 16 * XS_NU);
+            if (part == 3 && hh < n_head && tt + dt < t_end) scores[(size_t)h * n_ctx + tt + dt] = (tail + simd) * scale;
+            request(u, tt + 16 * nt * XS_NU);
         }
     }
 }
 
 // ---- softmax + P.V^T in the host order ---------------------------------------------------------------------------------
-// One 1024-thread workgroup per (head, 16 rows of V^T).  Waves 0..7 do the softmax and then the product, waves 8..15 bring two rows of V^T each into LDS meanwhile.
+// One 1024-thread workgroup per (head, 16 rows of V^T), the head first in the grid, so that the eight of a head are on one XCD, the one that wrote its scores
+// (4100 tokens 10.04 -> 9.81 us in a pass, 2060 8.46 -> 8.11, 1000 and 600 the same).  Waves 0..7 do the softmax and then the product, waves 8..15 bring two rows of V^T each into LDS meanwhile.
 // Softmax (non-linear.cpp:129-180): m = max t; e = exp_table[fp16(t - m)] (exact_exp.cuh); sum = std::reduce(e) = groups of four added to
 // one running sum, then the last n % 4 elements; p = e * (1 / sum), rounded to fp16 for the product (mat.cpp:37).
 // P.V^T (vec_dot.h:124-145 with n = n_kv): output row r has 4 x 8 accumulators, accumulator (j, l) adds elements
@@ -618,8 +622,9 @@ __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_stat
 // What bounds it: from 3500 tokens or so on the rows (16 per compute unit at 24 B/ns, then 0.6 us to write them to LDS and 0.6 to walk them), below the softmax's
 // chain of latencies.  The waves of the softmax meet on counters in LDS: at a workgroup barrier they would wait until the other eight have
 // asked for all their rows, which takes as long as the rows take to come.  All 16 waves taking part in both, with the table's gathers in the same memory
-// queue as the rows: 4100 tokens 12.7 us, 4000 12.7, 3000 11.5, 2060 9.4, 1500 9.2, 600 7.5; now 10.2, 9.9, 8.8, 8.2, 7.9, 6.7.  With this layout and
-// list but all waves in both: 11.5, -, 9.3, 8.5, 8.1, 6.8.  Scores asked for before the position is known: 10.7, 10.4, 9.2, 8.3, 8.0, 6.8.
+// queue as the rows: in a pass 4100 tokens 13.6 us, 2060 11.1, 1000 9.5, 600 8.1; now 9.8, 8.1, 7.0, 6.6.  One launch after the other (scores and list in the L2), before
+// arguments came in registers: 4100 tokens 12.7 us, 3000 11.5, 2060 9.4, 600 7.5; this 10.2, 8.8, 8.2, 6.7; this layout and list but all waves in both: 11.5, 9.3, 8.5, 6.8; scores asked
+// for before the position is known: 10.7, 9.2, 8.3, 6.8.
 #define XP_THREADS 1024
 #define XP_NP 10                           // 16-byte pieces per lane of a V^T row
 #define XP_NG 3                            // groups of four scores per thread of the softmax
@@ -651,7 +656,7 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
     __shared__ uint32_t s_cnt[3];
     XSTAMP(dbg, 0);
     const int n_kv = (st ? st->pos : pos_imm) + 1;
-    const int hd_ = blockIdx.x >> 3, dgrp = blockIdx.x & 7;
+    const int hd_ = blockIdx.x, dgrp = blockIdx.y;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int SA = xattn_pv_sa(n_ctx), RS = xattn_pv_row(n_ctx), REST = RS - 64 * SA - 32;
     uint16_t *s_p = (uint16_t *)smem, *s_v = s_p + RS;                // the probabilities as fp16, 16 rows of V^T
@@ -670,7 +675,7 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
             const int g = min(tid + 512 * u, nall - 1);
             if (512 * u < nall) {
                 if (4 * g + 3 < n_ctx) v[u] = *(const f4 *)(srow + 4 * g);
-                else v[u] = f4{srow[4 * g], srow[min(4 * g + 1, n_ctx - 1)], srow[min(4 * g + 2, n_ctx - 1)], srow[n_ctx - 1]};
+                else v[u] = f4{srow[4 * g], srow[min(4 * g + 1, n_ctx - 1)], srow[min(4 * g + 2, n_ctx - 1)], 0.0f};
             }
         }
         if (tid < XE_WORDS / 4) cd = ((const xp_u4 *)(lut + XE_AT))[tid];
@@ -683,9 +688,10 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
 #pragma unroll
         for (int u = 0; u < XP_NG; u++)
             if (512 * u < nall) {
-                const int j = 4 * (tid + 512 * u);
+                const int left = n_kv - 4 * min(tid + 512 * u, nall - 1);          // behind the last token: -inf, which leaves 0
 #pragma unroll
-                for (int i = 0; i < 4; i++) if (j + i < n_kv) mx = fmaxf(mx, v[u][i]);
+                for (int i = 1; i < 4; i++) v[u][i] = i < left ? v[u][i] : -INFINITY;
+                mx = fmaxf(fmaxf(fmaxf(mx, v[u][0]), fmaxf(v[u][1], v[u][2])), v[u][3]);
             }
         mx = wave_max(mx);
         if (lane == 0) s_red[wave] = mx;
@@ -700,11 +706,16 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
             const int g = tid + 512 * u;
             if (512 * u + 64 * wave < nall) {
                 float e[4];
+                bool any = false;
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     bool ask;
                     e[i] = xe_exp(f2h(mx - v[u][i]), s_code, ask);
-                    if (__any(ask)) e[i] = ask ? lut[f2h(v[u][i] - mx)] : e[i];
+                    any |= ask;
+                }
+                if (__any(any)) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) e[i] = lut[f2h(v[u][i] - mx)];
                 }
                 v[u] = f4{e[0], e[1], e[2], e[3]};
                 if (g < ngrp) s_grp[xg_seg_at(g)] = xa_group(make_float4(e[0], e[1], e[2], e[3]));
@@ -716,7 +727,11 @@ __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *s
         if (wave == 0) {
             xp_await(s_cnt + 1, 8);
             XSTAMP(dbg, 3);
-            float sum = xg_segment_sum<2>(s_grp, ngrp);
+            float sum = xg_segment_sum<1>(s_grp, min(ngrp, 1024));
+            for (int g = 1024; g < ngrp; g += 4) {                   // zeros behind the last group leave the sum as it is
+                const float4 t = *(const float4 *)(s_grp + xg_seg_at(g));
+                sum = sum + t.x; sum = sum + t.y; sum = sum + t.z; sum = sum + t.w;
+            }
             for (int j = ngrp * 4; j < n_kv; j++) sum = sum + s_rem[j & 3];
             if (lane == 0) s_sum = sum;
             xp_arrive(s_cnt + 2);

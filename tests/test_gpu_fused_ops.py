@@ -298,9 +298,9 @@ def test_attn_scores_in_several_rounds(hip, grid, n_kv, monkeypatch):
     assert np.array_equal(res[0][1], res[1][1])
 
 
-@pytest.mark.parametrize("n_head,n_kv", [(1, 577), (16, 593), (17, 1033), (31, 700)])
+@pytest.mark.parametrize("n_head,n_kv", [(1, 577), (8, 581), (9, 594), (16, 593), (17, 1033), (31, 700)])
 def test_attn_decode_head_groups(hip, oracle, n_head, n_kv):
-    """Scores are formed for groups of 16 heads: full ones, a last one of one or 15 heads, one head alone."""
+    """Scores are formed for eight groups of heads, one, two or four heads of as many tokens at a time: full groups, groups that lack a head, groups without one."""
     from tests.gpu_util import dev, dev_empty, call
     hd, n_ctx, d = 128, 1040, n_head * 128
     rng = np.random.default_rng(n_head)

@@ -83,6 +83,8 @@ struct fused_args {
     uint8_t *q8_dump;              // tests: workgroup 0 of a one-row-per-wave launch writes its staged activations here as native Q8_0 blocks
 };
 
+// what the first requests of a launch need goes ahead of the rest: the first 14 dwords of a kernel's arguments come in registers (Makefile)
+#define WGV_ARGS(a) (a).x_in, (a).normw, (a).W0, (a).W1, (a).W2, (a).resid, (a).K, (a).M, (a)
 enum { EPI_QKV = 0, EPI_RESID = 1, EPI_GATEUP = 2, EPI_STORE = 3 };
 
 // Prologue: EPI_RESID stages the plain f32 input, every other epilogue the RMS-normalised, weighted
@@ -202,7 +204,9 @@ static __device__ __forceinline__ void wgv_stage(const float4 (&xv)[NITK], const
 #define WGV_DEPTH 3             // rows per wave requested ahead of their use
 #endif
 template <int WT, int NITK, int NR, int EPI, int WTV = WT>      // WTV: type of W2 (the v rows of EPI_QKV)
-__global__ __launch_bounds__(WGV_THREADS) void wave_gemv_kernel(fused_args a) {
+__global__ __launch_bounds__(WGV_THREADS) void wave_gemv_kernel(const float *x_in, const float *normw, const uint8_t *W0, const uint8_t *W1, const uint8_t *W2, const float *resid, int K_, int M,
+                                                                fused_args a) {
+    a.x_in = x_in; a.normw = normw; a.W0 = W0; a.W1 = W1; a.W2 = W2; a.resid = resid; a.K = K_; a.M = M;
     constexpr bool NORM = (EPI != EPI_RESID);
     constexpr int NB = EPI == EPI_QKV ? 3 : (EPI == EPI_GATEUP ? 2 * NR : NR);
     constexpr int DEPTH = EPI == EPI_QKV ? WGV_DEPTH_QKV : WGV_DEPTH;
@@ -358,6 +362,7 @@ struct attn_layer_args {
     long long *dbg;               // measurement builds only: wall-clock stamps (10 ns units) of workgroups 0 and 100
 #endif
 };
+#define ATL_ARGS(a) (a).x_in, (a).normw, (a).wq, (a).wk, (a).wv, (a).st, (a).d, (a).n_ctx, (a)
 #ifdef ATL_STAMPS
 #define ATL_STAMP(i) do { if (a.dbg && tid == 0) { if (blockIdx.x == 0 || blockIdx.x == 100) a.dbg[(blockIdx.x ? 64 : 0) + (i)] = wall_clock64(); \
                                                     if ((i) == 0 || (i) == 3 || (i) == 5 || (i) == 8) a.dbg[128 + blockIdx.x * 8 + ((i) == 0 ? 0 : (i) == 3 ? 1 : (i) == 5 ? 2 : 3)] = wall_clock64(); \
@@ -367,7 +372,9 @@ struct attn_layer_args {
 #endif
 
 template <int WT, int WTV>        // types of wq / wk and of wv
-__global__ __launch_bounds__(ATL_THREADS, 4) void attn_layer_kernel(attn_layer_args a) {
+__global__ __launch_bounds__(ATL_THREADS, 4) void attn_layer_kernel(const float *x_in, const float *normw, const uint8_t *wq_, const uint8_t *wk_, const uint8_t *wv_, dev_state *st, int d_, int n_ctx_,
+                                                                    attn_layer_args a) {
+    a.x_in = x_in; a.normw = normw; a.wq = wq_; a.wk = wk_; a.wv = wv_; a.st = st; a.d = d_; a.n_ctx = n_ctx_;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     __shared__ float s_red[16];
     __shared__ int s_ok;

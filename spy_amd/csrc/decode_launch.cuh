@@ -62,7 +62,7 @@ static int launch_wave(spy_hip_llama *m, hipStream_t st, const fused_args &a) {
     if (m->dry) return 0;
     const int units = EPI == EPI_QKV ? a.d : (EPI == EPI_GATEUP ? a.M / 2 : a.M);       // one per wave and step
     const int grid = (units + WGV_WAVES * NR - 1) / (WGV_WAVES * NR);
-    kern<<<dim3((unsigned)grid), dim3(WGV_THREADS), lds, st>>>(a);
+    kern<<<dim3((unsigned)grid), dim3(WGV_THREADS), lds, st>>>(WGV_ARGS(a));
     return SPY_LAUNCH_RC();
 }
 // rows (head) and row pairs (gate|up) per wave.  The kernel keeps a ring of DEPTH + 1 rows in registers; 8 rows per wave give
@@ -98,7 +98,7 @@ static int launch_wave_plain(hipStream_t st, const fused_args &a) {
     const size_t lds = staged_bytes(a.K);
     auto kern = wave_gemv_kernel<WT, NITK, NR, EPI_RESID, WT>;
     RC_TRY(spy_raise_lds_limit((const void *)kern, lds));
-    kern<<<dim3((unsigned)((a.M + WGV_WAVES * NR - 1) / (WGV_WAVES * NR))), dim3(WGV_THREADS), lds, st>>>(a);
+    kern<<<dim3((unsigned)((a.M + WGV_WAVES * NR - 1) / (WGV_WAVES * NR))), dim3(WGV_THREADS), lds, st>>>(WGV_ARGS(a));
     return SPY_LAUNCH_RC();
 }
 template <int WT>
@@ -148,7 +148,7 @@ static int launch_attn_layer_tv(spy_hip_llama *m, hipStream_t st, int il, bool p
 #ifdef ATL_STAMPS
     a.dbg = m->stamp_dbg;
 #endif
-    kern<<<dim3((unsigned)(c.n_head * ATL_GPH)), dim3(ATL_THREADS), lds, st>>>(a);
+    kern<<<dim3((unsigned)(c.n_head * ATL_GPH)), dim3(ATL_THREADS), lds, st>>>(ATL_ARGS(a));
     return SPY_LAUNCH_RC();
 }
 

@@ -42,6 +42,8 @@ struct xg_args {
     int pos_imm, rope_row0;                // st == nullptr: the position as a number; first position of rope_tab
     long long *dbg;                        // measurement builds (-DXDBG_STAMPS): wall-clock stamps of workgroup 0
 };
+// what the first requests of a launch need goes ahead of the rest: the first 14 dwords of a kernel's arguments come in registers (Makefile)
+#define XG_ARGS(a) (a).x_in, (a).normw, (a).W0, (a).W1, (a).W2, (a).st, (a).K, (a).M, (a)
 #ifdef XDBG_STAMPS
 #define XSTAMP(dbg, i) do { if ((dbg) && blockIdx.x == 0 && threadIdx.x == 0) (dbg)[i] = wall_clock64(); } while (0)
 #else
@@ -298,7 +300,10 @@ static __device__ __forceinline__ float xg_hsum8(float acc) {
 // A step's rows of all 16 waves form one batch: phase 1 (all waves) -> barrier -> phase 2 (the first lanes, one per
 // accumulator) -> barrier, per slab of 4096 elements of K; the accumulators stay in their lanes from slab to slab.
 template <int WT, int NITK, int RPS, int NSTEP, int EPI, int WTV = WT>
-__global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(xg_args a) {
+__global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, const float *normw, const uint8_t *W0, const uint8_t *W1, const uint8_t *W2, const dev_state *st, int K_, int M,
+                                                           xg_args a) {
+    a.x_in = x_in; a.normw = normw; a.W0 = W0; a.W1 = W1; a.W2 = W2; a.st = st; a.K = K_; a.M = M;
+    if constexpr (EPI == EPI_QKV) a.d = M;
     constexpr bool NORM = (EPI != EPI_RESID);
     constexpr int NCH = xg_traits<WT>::NCH, NCHV = xg_traits<WTV>::NCH;
     constexpr int NROW = EPI == EPI_QKV ? 3 : RPS * NSTEP;                  // rows per wave
@@ -310,11 +315,11 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(xg_args a) {
     const int K = a.K, npair = K / 64;
     const size_t RB = (size_t)spy_row_size(WT, K);
 
-    // row index (within its matrix) and base of the wave's row r (0 .. NROW-1); rows beyond the matrix re-read a valid row and are dropped in the epilogue
+    // row index (within its matrix) and base of the wave's row r (0 .. NROW-1); rows beyond the matrix re-read the last one and are dropped in the epilogue
     auto row_of = [&](int r, bool &valid) -> int {
-        if constexpr (EPI == EPI_QKV) { valid = gw < a.d; const int j = gw % a.d; return r == 2 ? j : ((2 * j) % a.d) + r; }
-        else if constexpr (EPI == EPI_GATEUP) { const int u = gw + (r >> 1) * NW; valid = u < a.M; return valid ? u : gw % a.M; }
-        else { const int u = (gw + (r / RPS) * NW) * RPS + (r % RPS); valid = u < a.M; return valid ? u : u % a.M; }
+        if constexpr (EPI == EPI_QKV) { valid = gw < a.d; const int j = min(gw, a.d - 1); return r == 2 ? j : 2 * j - (2 * j < a.d ? 0 : a.d) + r; }
+        else if constexpr (EPI == EPI_GATEUP) { const int u = gw + (r >> 1) * NW; valid = u < a.M; return min(u, a.M - 1); }
+        else { const int u = (gw + (r / RPS) * NW) * RPS + (r % RPS); valid = u < a.M; return min(u, a.M - 1); }
     };
     auto row_ptr = [&](int r) -> const uint8_t * {
         bool v; int i = row_of(r, v);
@@ -323,7 +328,7 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(xg_args a) {
 #endif
         if constexpr (EPI == EPI_QKV) {
             if (r == 2) return a.W2 + (size_t)i * spy_row_size(WTV, K);
-            return (2 * (gw % a.d) < a.d ? a.W0 : a.W1) + (size_t)i * RB;
+            return (2 * gw < a.d ? a.W0 : a.W1) + (size_t)i * RB;
         } else if constexpr (EPI == EPI_GATEUP) return ((r & 1) ? a.W1 : a.W0) + (size_t)i * RB;
         else return a.W0 + (size_t)i * RB;
     };
@@ -358,7 +363,7 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(xg_args a) {
     float2 cs = make_float2(0.0f, 0.0f);
     auto issue_first = [&]() {
         if constexpr (EPI == EPI_QKV)
-            cs = *(const float2 *)(a.rope_tab + (size_t)(pos - a.rope_row0) * a.hd + (2 * ((int)blockIdx.x * XG_WAVES + tid / (2 * NCH) % XG_WAVES)) % a.d % a.hd);
+            cs = *(const float2 *)(a.rope_tab + (size_t)(pos - a.rope_row0) * a.hd + ((2 * ((int)blockIdx.x * XG_WAVES + tid / (2 * NCH) % XG_WAVES)) & (a.hd - 1)));      // heads are 128 wide
         if constexpr (!NORM) __builtin_amdgcn_s_barrier();      // x of every wave ahead of every wave's rows in the compute unit's memory queue
 #pragma unroll
         for (int r = 0; r < NROW; r++) if (r < DEPTH && r >= PRE) {

@@ -76,11 +76,22 @@ struct xt_args {
     int ncg_all;                                   // groups of the whole call of which this is a piece
     const uint8_t *xq, *xd;
 };
+// What the first requests of a launch need, ahead of the rest: the first 14 dwords of a kernel's arguments come in registers (Makefile).
+#define XT_PARAMS const uint8_t *w0_, const uint8_t *w1_, const uint8_t *w2_, const uint8_t *xq_, const uint8_t *xd_, int64_t w_row_, int tiles_, int nst_, xt_args a
+#define XT_HOT const xt_hot hot = {w0_, w1_, w2_, xq_, xd_, w_row_, tiles_, nst_}
+#define XT_ARGS(a) (a).w[0], (a).w[1], (a).w[2], (a).xq, (a).xd, (a).w_row, (a).tiles, (a).nst, (a)
+struct xt_hot {
+    const uint8_t *w0, *w1, *w2, *xq, *xd;
+    int64_t w_row;
+    int tiles, nst;
+    __device__ __forceinline__ int mat(int b) const { return (b >= tiles ? 1 : 0) + (b >= 2 * tiles ? 1 : 0); }      // matrix of a workgroup
+    __device__ __forceinline__ const uint8_t *w(int m) const { return m == 0 ? w0 : m == 1 ? w1 : w2; }
+};
 
 // AS: waves that share the accumulators of a tile; RG: groups of 16 weight rows per workgroup; C: groups of 16 activation rows per
 // wave; NXS, NWC: LDS slots for stages and chunks (powers of two); P: stages requested ahead
 template <int WT, int C, int NXS, int P, int NWC>
-__device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
+__device__ __forceinline__ void xt_tile(const xt_hot &hot, const xt_args &a, int cg0) {
     constexpr int AS = 2, RG = 2;
     constexpr int NT = 64 * AS * RG, ROWS = 16 * RG;
     constexpr int CU = xt_w<WT>::CU, UW = ROWS * CU, NI = (UW + NT - 1) / NT, NXI = C * 256 / NT;
@@ -89,8 +100,8 @@ __device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = wave % AS, rg = wave / AS, q = lane >> 4, r = lane & 15;
-    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS;
-    const int nst = a.nst, ncg = a.ncg, M = a.M;
+    const int mat = hot.mat((int)blockIdx.x), m0 = ((int)blockIdx.x - mat * hot.tiles) * ROWS;
+    const int nst = hot.nst, ncg = a.ncg, M = a.M;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
 
     // what a wave requests: uniform bases that advance, per-lane offsets that stay.  Row groups and activation groups past the end
@@ -99,15 +110,15 @@ __device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
     // kilobyte for what they repeat a compute unit had room for two workgroups of the Q8_0 tile instead of three: 22016 x 4096 x 512 474 -> 448 us,
     // 4096 x 4096 x 2048 347 -> 326, 12288 x 4096 x 100 69.7 -> 61.8.)
     const int wl = wave * 64 + (NI - 1) * NT >= UW ? 0 : wave;
-    const uint8_t *bx[NXI], *bd, *bw = a.w[mat] + (int64_t)m0 * a.w_row;
+    const uint8_t *bx[NXI], *bd, *bw = hot.w(mat) + (int64_t)m0 * hot.w_row;
     uint32_t ow[NI];
 #pragma unroll
-    for (int i = 0; i < NXI; i++) bx[i] = a.xq + (int64_t)min(cg0 + (i * NT + wave * 64) / 256, ncg - 1) * nst * XT_XB + (i * NT + wave * 64) % 256 * 16;
-    bd = a.xd + (int64_t)min(cg0 + min(wave, C - 1), ncg - 1) * nst * XT_XD;
+    for (int i = 0; i < NXI; i++) bx[i] = hot.xq + (int64_t)min(cg0 + (i * NT + wave * 64) / 256, ncg - 1) * nst * XT_XB + (i * NT + wave * 64) % 256 * 16;
+    bd = hot.xd + (int64_t)min(cg0 + min(wave, C - 1), ncg - 1) * nst * XT_XD;
 #pragma unroll
     for (int i = 0; i < NI; i++) {
         const int u = min((i == NI - 1 ? wl * 64 + lane : tid) + i * NT, UW - 1);
-        ow[i] = (uint32_t)(min(m0 + u / CU, M - 1) - m0) * (uint32_t)a.w_row + (u % CU) * 16;
+        ow[i] = (uint32_t)(min(m0 + u / CU, M - 1) - m0) * (uint32_t)hot.w_row + (u % CU) * 16;
     }
     const uint32_t l16 = lane * 16, l4 = lane * 4;
     const uint32_t ldsx = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024), ldsd = __builtin_amdgcn_readfirstlane(lds0 + C * XT_XB + min(wave, C - 1) * 256),
@@ -262,14 +273,15 @@ __device__ __forceinline__ void xt_tile(const xt_args &a, int cg0) {
 }
 
 template <int WT, int C, int NXS, int P, int NWC>
-__global__ __launch_bounds__(256, 3) void xt_kernel(xt_args a) { xt_tile<WT, C, NXS, P, NWC>(a, (int)blockIdx.y * C); }
+__global__ __launch_bounds__(256, 3) void xt_kernel(XT_PARAMS) { XT_HOT; xt_tile<WT, C, NXS, P, NWC>(hot, a, (int)blockIdx.y * C); }
 // Tiles of four activation groups and, behind them in the grid, one of the R groups that remain: the sums of groups that do not exist cost as much
 // as those of groups that do (22016 x 4096 Q4_0: 77 rows 98 -> 85 us, 140 rows 161 -> 135, 200 rows 224 -> 188, 900 rows 831 -> 796)
 template <int WT, int R>
-__global__ __launch_bounds__(256, 3) void xt_mixed_kernel(xt_args a) {
+__global__ __launch_bounds__(256, 3) void xt_mixed_kernel(XT_PARAMS) {
+    XT_HOT;
     const int full = a.ncg / 4;
-    if ((int)blockIdx.y < full) xt_tile<WT, 4, 2, 1, 2>(a, (int)blockIdx.y * 4);
-    else xt_tile<WT, R, R < 3 ? 4 : 2, R < 3 ? 2 : 1, 2>(a, full * 4);
+    if ((int)blockIdx.y < full) xt_tile<WT, 4, 2, 1, 2>(hot, a, (int)blockIdx.y * 4);
+    else xt_tile<WT, R, R < 3 ? 4 : 2, R < 3 ? 2 : 1, 2>(hot, a, full * 4);
 }
 
 // Few activation rows: one group of them and 16 weight rows per workgroup, the accumulators of the tile over its four waves (words 2g, 2g + 1 to wave g).
@@ -280,22 +292,23 @@ __global__ __launch_bounds__(256, 3) void xt_mixed_kernel(xt_args a) {
 // Against one stage of four blocks per barrier, weights from memory, in us, packing of the activations (4 us) included: 8 rows, Q4_0 4096 x 4096 14.4 -> 12.1,
 // 4096 x 11008 30.6 -> 23.6, 12288 x 4096 21.0 -> 17.7, Q8_0 14.4 -> 12.5, 30.3 -> 24.3, 22.5 -> 20.8; 48 rows, Q4_0 4096 x 4096 21.2 -> 17.8, 4096 x 11008 47.5 -> 37.3.
 template <int WT, int NS>
-__global__ __launch_bounds__(256, 2) void xn_kernel(xt_args a) {
+__global__ __launch_bounds__(256, 2) void xn_kernel(XT_PARAMS) {
+    XT_HOT;
     constexpr int NT = 256, ROWS = 16, CU = xt_w<WT>::CU, UW = ROWS * CU, NI = (UW + NT - 1) / NT, NXI = 2;
     constexpr int XB = 2 * (XT_XB + 256), WB = (UW + 63) / 64 * 1024, NREQ = NXI + 1 + NI;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = wave, q = lane >> 4, r = lane & 15;
-    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS, cg = (int)blockIdx.y;
-    const int nch = a.nst / 2, M = a.M;
+    const int mat = hot.mat((int)blockIdx.x), m0 = ((int)blockIdx.x - mat * hot.tiles) * ROWS, cg = (int)blockIdx.y;
+    const int nch = hot.nst / 2, M = a.M;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
     // requests as in xt_tile: uniform bases that advance by a chunk, per-lane offsets that stay; waves 0 and 1 bring the scales of the chunk's stages (the others repeat them)
-    const uint8_t *bx = a.xq + (int64_t)cg * a.nst * XT_XB + wave * 1024, *bd = a.xd + ((int64_t)cg * a.nst + min(wave, 1)) * XT_XD, *bw = a.w[mat] + (int64_t)m0 * a.w_row;
+    const uint8_t *bx = hot.xq + (int64_t)cg * hot.nst * XT_XB + wave * 1024, *bd = hot.xd + ((int64_t)cg * hot.nst + min(wave, 1)) * XT_XD, *bw = hot.w(mat) + (int64_t)m0 * hot.w_row;
     uint32_t ow[NI];
 #pragma unroll
     for (int i = 0; i < NI; i++) {
         const int u = min(tid + i * NT, UW - 1);
-        ow[i] = (uint32_t)(min(m0 + u / CU, M - 1) - m0) * (uint32_t)a.w_row + (u % CU) * 16;
+        ow[i] = (uint32_t)(min(m0 + u / CU, M - 1) - m0) * (uint32_t)hot.w_row + (u % CU) * 16;
     }
     const bool spare = wave * 64 + (NI - 1) * NT >= UW;
     const uint32_t lds_spare = __builtin_amdgcn_readfirstlane(lds0 + NS * (XB + WB));
@@ -427,7 +440,7 @@ int xn_launch(hipStream_t st, xt_args a, int nmat) {
     constexpr size_t lds = NS * (2 * (XT_XB + 256) + (16 * xt_w<WT>::CU + 63) / 64 * 1024) + 1024;
     static_assert(lds <= 64 * 1024 && lds >= 3 * 8 * 256, "no raised LDS limit; room for the exchange of the accumulators");
     a.tiles = (a.M + 15) / 16;
-    xn_kernel<WT, NS><<<dim3((unsigned)(a.tiles * nmat), (unsigned)a.ncg), dim3(256), lds, st>>>(a);
+    xn_kernel<WT, NS><<<dim3((unsigned)(a.tiles * nmat), (unsigned)a.ncg), dim3(256), lds, st>>>(XT_ARGS(a));
     return SPY_LAUNCH_RC();
 }
 
@@ -623,14 +636,14 @@ template <int WT, int C, int NXS, int NWC> constexpr size_t xt_lds() {
 template <int WT, int C, int NXS, int P, int NWC>
 int xt_launch(hipStream_t st, xt_args a, int nmat) {
     a.tiles = (a.M + 31) / 32;
-    xt_kernel<WT, C, NXS, P, NWC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(256), xt_lds<WT, C, NXS, NWC>(), st>>>(a);
+    xt_kernel<WT, C, NXS, P, NWC><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(256), xt_lds<WT, C, NXS, NWC>(), st>>>(XT_ARGS(a));
     return SPY_LAUNCH_RC();
 }
 template <int WT, int R>
 int xt_launch_mixed(hipStream_t st, xt_args a, int nmat) {
     a.tiles = (a.M + 31) / 32;
     constexpr size_t l4 = xt_lds<WT, 4, 2, 2>(), lr = xt_lds<WT, R, R < 3 ? 4 : 2, 2>();
-    xt_mixed_kernel<WT, R><<<dim3((unsigned)(a.tiles * nmat), (unsigned)(a.ncg / 4 + 1)), dim3(256), l4 > lr ? l4 : lr, st>>>(a);
+    xt_mixed_kernel<WT, R><<<dim3((unsigned)(a.tiles * nmat), (unsigned)(a.ncg / 4 + 1)), dim3(256), l4 > lr ? l4 : lr, st>>>(XT_ARGS(a));
     return SPY_LAUNCH_RC();
 }
 
@@ -793,7 +806,8 @@ __device__ __forceinline__ void xk_unpack(const xk_raw<WT> &w, int q, uint4 (&o)
 // and 588 -> 449 (the 128 x 128 tiles of gemm.hip: 424 and 755).
 // KS (own order): that many sets of RG waves, each with its share of the super-blocks and activation stages of its own; their sums meet at the end.
 template <int WT, bool OWN, int RG, int C, int OCC, int KS = 1>
-__global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(xt_args a) {
+__global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(XT_PARAMS) {
+    XT_HOT;
     constexpr bool K4 = WT == SPY_HIP_Q4_K;
     static_assert(KS == 1 || OWN, "the host's order is one chain over K");
     constexpr int NT = 64 * RG, ROWS = 16 * RG, NXI = C * 256 / NT, C2 = (C + 1) / 2;
@@ -803,20 +817,20 @@ __global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(xt_args a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem_all[];
     const int tid = threadIdx.x, lane = tid & 63, wg_wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, r = lane & 15;
     const int ks = KS > 1 ? wg_wave / RG : 0, wave = KS > 1 ? wg_wave % RG : wg_wave;
-    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS, cg0 = (int)blockIdx.y * C;
+    const int mat = hot.mat((int)blockIdx.x), m0 = ((int)blockIdx.x - mat * hot.tiles) * ROWS, cg0 = (int)blockIdx.y * C;
     const int ncg = a.ncg, M = a.M;
     // the set's super-blocks: sb0 .. sb0 + nsb - 1; every set takes part in as many steps as the longest
-    const int all = a.nst / 2, per = (all + KS - 1) / KS, sb0 = min(ks * per, all - 1), nsb = KS > 1 ? max(min(per, all - ks * per), 0) : all;
+    const int all = hot.nst / 2, per = (all + KS - 1) / KS, sb0 = min(ks * per, all - 1), nsb = KS > 1 ? max(min(per, all - ks * per), 0) : all;
     const int nst = 2 * nsb, nstep = 2 * per;
     uint8_t *smem = smem_all + ks * (NXS * XB);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
     // activation stages into the ring, as in xt_kernel; one request brings the records of two groups
     const uint8_t *bx[NXI], *bd;
 #pragma unroll
-    for (int i = 0; i < NXI; i++) bx[i] = a.xq + ((int64_t)min(cg0 + (i * NT + wave * 64) / 256, ncg - 1) * a.nst + 2 * sb0) * XT_XB + (i * NT + wave * 64) % 256 * 16;
+    for (int i = 0; i < NXI; i++) bx[i] = hot.xq + ((int64_t)min(cg0 + (i * NT + wave * 64) / 256, ncg - 1) * hot.nst + 2 * sb0) * XT_XB + (i * NT + wave * 64) % 256 * 16;
     const int dc0 = min(cg0 + 2 * min(wave, C2 - 1), ncg - 1), dc1 = min(dc0 + 1, ncg - 1);
-    bd = a.xd + ((int64_t)dc0 * a.nst + 2 * sb0) * XT_XD;
-    const uint32_t l16 = lane * 16, ld = (lane & 31) * 16 + (lane >> 5) * (uint32_t)((dc1 - dc0) * a.nst * XT_XD);
+    bd = hot.xd + ((int64_t)dc0 * hot.nst + 2 * sb0) * XT_XD;
+    const uint32_t l16 = lane * 16, ld = (lane & 31) * 16 + (lane >> 5) * (uint32_t)((dc1 - dc0) * hot.nst * XT_XD);
     const uint32_t ldsx = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024), ldsd = __builtin_amdgcn_readfirstlane(lds0 + C * XT_XB + min(wave, C2 - 1) * 1024);
     int is = 0;
     auto issue_x = [&]() {
@@ -828,7 +842,7 @@ __global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(xt_args a) {
         bd += adv * XT_XD;
         is++;
     };
-    const uint8_t *wr = a.w[mat] + (int64_t)min(m0 + wave * 16 + r, M - 1) * a.w_row;
+    const uint8_t *wr = hot.w(mat) + (int64_t)min(m0 + wave * 16 + r, M - 1) * hot.w_row;
     xk_raw<WT> cur;
     xk_load_half<0>(cur, wr, sb0, q);
     issue_x();
@@ -1050,15 +1064,16 @@ __global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(xt_args a) {
 // the fma per sub-block; the terms are independent, so each round the waves leave the terms of four super-blocks in LDS and then every wave
 // walks a quarter of the outputs through their 32 fmas.  (16 rows of a 4096 x 4096 Q4_K matrix: 20 us as a chain in one wave, 10 here.)
 template <int WT>
-__global__ __launch_bounds__(256, 3) void xks_kernel(xt_args a) {
+__global__ __launch_bounds__(256, 3) void xks_kernel(XT_PARAMS) {
+    XT_HOT;
     constexpr bool K4 = WT == SPY_HIP_Q4_K;
     __shared__ __align__(16) float s_t[32][4][64];                  // [sub-block of the round][row 4q + v][lane]
     __shared__ __align__(16) float s_tab[4][K4 ? 256 : 16];
     __shared__ float s_x[32][16], s_d[4][16];                       // d_x of the round's sub-blocks; Q6_K: d of its super-blocks
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, r = lane & 15;
-    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * 16, cg = (int)blockIdx.y, nsb = a.nst / 2;
-    const uint8_t *wr = a.w[mat] + (int64_t)min(m0 + r, a.M - 1) * a.w_row;
-    const uint8_t *xq = a.xq + (int64_t)cg * a.nst * XT_XB + q * 256 + r * 16, *xd = a.xd + (int64_t)cg * a.nst * XT_XD;
+    const int mat = hot.mat((int)blockIdx.x), m0 = ((int)blockIdx.x - mat * hot.tiles) * 16, cg = (int)blockIdx.y, nsb = hot.nst / 2;
+    const uint8_t *wr = hot.w(mat) + (int64_t)min(m0 + r, a.M - 1) * hot.w_row;
+    const uint8_t *xq = hot.xq + (int64_t)cg * hot.nst * XT_XB + q * 256 + r * 16, *xd = hot.xd + (int64_t)cg * hot.nst * XT_XD;
     xk_raw<WT> cur = xk_load<WT>(wr, min(wave, nsb - 1), q), nxt;
     uint4 xv[8], xn[8];
     uint32_t dx[2], dn[2];
@@ -1161,18 +1176,19 @@ __device__ __forceinline__ void xo_transpose(uint32_t (&r)[4]) {
     s32(r[0], r[2]); s32(r[1], r[3]);
 }
 constexpr int XO_C = 4;
-__global__ __launch_bounds__(256, 3) void xo_kernel(xt_args a) {
+__global__ __launch_bounds__(256, 3) void xo_kernel(XT_PARAMS) {
+    XT_HOT;
     constexpr int C = XO_C, NT = 256, ROWS = 64, C2 = C / 2, XB = C * XT_XB + C2 * 1024, NDW = 9, CB = xt_w<SPY_HIP_Q4_0>::CB;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, r = lane & 15;
-    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS, cg0 = (int)blockIdx.y * C;
-    const int nst = a.nst, ncg = a.ncg, M = a.M;
+    const int mat = hot.mat((int)blockIdx.x), m0 = ((int)blockIdx.x - mat * hot.tiles) * ROWS, cg0 = (int)blockIdx.y * C;
+    const int nst = hot.nst, ncg = a.ncg, M = a.M;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
     const uint8_t *bx[C], *bd;
 #pragma unroll
-    for (int i = 0; i < C; i++) bx[i] = a.xq + (int64_t)min(cg0 + i, ncg - 1) * nst * XT_XB + wave * 1024;
+    for (int i = 0; i < C; i++) bx[i] = hot.xq + (int64_t)min(cg0 + i, ncg - 1) * nst * XT_XB + wave * 1024;
     const int dc0 = min(cg0 + 2 * min(wave, C2 - 1), ncg - 1), dc1 = min(dc0 + 1, ncg - 1);
-    bd = a.xd + (int64_t)dc0 * nst * XT_XD;
+    bd = hot.xd + (int64_t)dc0 * nst * XT_XD;
     const uint32_t l16 = lane * 16, ld = (lane & 31) * 16 + (lane >> 5) * (uint32_t)((dc1 - dc0) * nst * XT_XD);
     const uint32_t ldsx = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024), ldsd = __builtin_amdgcn_readfirstlane(lds0 + C * XT_XB + min(wave, C2 - 1) * 1024);
     int is = 0;
@@ -1185,7 +1201,7 @@ __global__ __launch_bounds__(256, 3) void xo_kernel(xt_args a) {
         bd += adv * XT_XD;
         is++;
     };
-    const uint8_t *wr = a.w[mat] + (int64_t)min(m0 + wave * 16 + r, M - 1) * a.w_row + q * (NDW * 4);
+    const uint8_t *wr = hot.w(mat) + (int64_t)min(m0 + wave * 16 + r, M - 1) * hot.w_row + q * (NDW * 4);
     uint32_t cur[NDW];
     auto load_w = [&](int chunk) { __builtin_memcpy(cur, __builtin_assume_aligned(wr + (int64_t)chunk * CB, 4), NDW * 4); };
     load_w(0);
@@ -1281,18 +1297,19 @@ __global__ __launch_bounds__(256, 3) void xo_kernel(xt_args a) {
 // (with the operand reads in one bank that xo_kernel had then): 22016 x 4096 x 1000 310 -> 278 us, 12288 x 4096 x 1000 168 -> 151, 4096 x 11008 x 1000 188 -> 165, 4096 x 4096 x 1000 78 -> 68.
 // (Two pairs per wave: 340 us at 22016 x 4096 x 1000; three: 311.)
 constexpr int XO_CP = 4;
-__global__ __launch_bounds__(256, 2) void xo32_kernel(xt_args a) {
+__global__ __launch_bounds__(256, 2) void xo32_kernel(XT_PARAMS) {
+    XT_HOT;
     constexpr int CP = XO_CP, NT = 256, ROWS = 128, C = 2 * CP, XB = C * XT_XB + CP * 1024, NDW = 18, CB = xt_w<SPY_HIP_Q4_0>::CB;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, r = lane & 31;
-    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS, cg0 = (int)blockIdx.y * C;
-    const int nst = a.nst, ncg = a.ncg, M = a.M;
+    const int mat = hot.mat((int)blockIdx.x), m0 = ((int)blockIdx.x - mat * hot.tiles) * ROWS, cg0 = (int)blockIdx.y * C;
+    const int nst = hot.nst, ncg = a.ncg, M = a.M;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
     const uint8_t *bx[C], *bd;
 #pragma unroll
-    for (int i = 0; i < C; i++) bx[i] = a.xq + (int64_t)min(cg0 + i, ncg - 1) * nst * XT_XB + wave * 1024;
+    for (int i = 0; i < C; i++) bx[i] = hot.xq + (int64_t)min(cg0 + i, ncg - 1) * nst * XT_XB + wave * 1024;
     const int dc0 = min(cg0 + 2 * min(wave, CP - 1), ncg - 1), dc1 = min(dc0 + 1, ncg - 1);
-    bd = a.xd + (int64_t)dc0 * nst * XT_XD;
+    bd = hot.xd + (int64_t)dc0 * nst * XT_XD;
     const uint32_t l16 = lane * 16, ld = r * 16 + h * (uint32_t)((dc1 - dc0) * nst * XT_XD);
     const uint32_t ldsx = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024), ldsd = __builtin_amdgcn_readfirstlane(lds0 + C * XT_XB + min(wave, CP - 1) * 1024);
     int is = 0;
@@ -1306,7 +1323,7 @@ __global__ __launch_bounds__(256, 2) void xo32_kernel(xt_args a) {
         is++;
     };
     // lane (h, r): blocks 4h .. 4h + 3 of row r and chunk
-    const uint8_t *wr = a.w[mat] + (int64_t)min(m0 + wave * 32 + r, M - 1) * a.w_row + h * (NDW * 4);
+    const uint8_t *wr = hot.w(mat) + (int64_t)min(m0 + wave * 32 + r, M - 1) * hot.w_row + h * (NDW * 4);
     uint32_t cur[NDW];
     auto load_w = [&](int chunk) { __builtin_memcpy(cur, __builtin_assume_aligned(wr + (int64_t)chunk * CB, 4), NDW * 4); };
     load_w(0);
@@ -1416,14 +1433,14 @@ int xo32_launch(hipStream_t st, xt_args a, int nmat) {
     const int rc = spy_raise_lds_limit((const void *)xo32_kernel, lds);
     if (rc) return rc;
     a.tiles = (a.M + 127) / 128;
-    xo32_kernel<<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + 2 * XO_CP - 1) / (2 * XO_CP))), dim3(256), lds, st>>>(a);
+    xo32_kernel<<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + 2 * XO_CP - 1) / (2 * XO_CP))), dim3(256), lds, st>>>(XT_ARGS(a));
     return SPY_LAUNCH_RC();
 }
 int xo_launch(hipStream_t st, xt_args a, int nmat) {
     constexpr size_t lds = 2 * (XO_C * XT_XB + XO_C / 2 * 1024);
     static_assert(lds <= 64 * 1024, "");
     a.tiles = (a.M + 63) / 64;
-    xo_kernel<<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + XO_C - 1) / XO_C)), dim3(256), lds, st>>>(a);
+    xo_kernel<<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + XO_C - 1) / XO_C)), dim3(256), lds, st>>>(XT_ARGS(a));
     return SPY_LAUNCH_RC();
 }
 template <int WT, bool OWN, int RG, int C, int OCC, int KS = 1>
@@ -1432,13 +1449,13 @@ int xk_launch(hipStream_t st, xt_args a, int nmat) {
     static_assert(lds <= 160 * 1024 && lds >= (size_t)(KS - 1) * RG * C * 1024, "");
     if (lds > 64 * 1024) { const int rc = spy_raise_lds_limit((const void *)xk_kernel<WT, OWN, RG, C, OCC, KS>, lds); if (rc) return rc; }
     a.tiles = (a.M + 16 * RG - 1) / (16 * RG);
-    xk_kernel<WT, OWN, RG, C, OCC, KS><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * RG * KS), lds, st>>>(a);
+    xk_kernel<WT, OWN, RG, C, OCC, KS><<<dim3((unsigned)(a.tiles * nmat), (unsigned)((a.ncg + C - 1) / C)), dim3(64 * RG * KS), lds, st>>>(XT_ARGS(a));
     return SPY_LAUNCH_RC();
 }
 template <int WT>
 int xks_launch(hipStream_t st, xt_args a, int nmat) {
     a.tiles = (a.M + 15) / 16;
-    xks_kernel<WT><<<dim3((unsigned)(a.tiles * nmat), (unsigned)a.ncg), dim3(256), 0, st>>>(a);
+    xks_kernel<WT><<<dim3((unsigned)(a.tiles * nmat), (unsigned)a.ncg), dim3(256), 0, st>>>(XT_ARGS(a));
     return SPY_LAUNCH_RC();
 }
 

@@ -17,7 +17,7 @@ static int launch_xg(spy_hip_llama *m, hipStream_t st, const xg_args &a, int uni
     RC_TRY(spy_ensure_lds(m, (const void *)kern, lds));
     if (m->dry) return 0;
     const int per_wg = XG_WAVES * (EPI == EPI_QKV ? 1 : (EPI == EPI_GATEUP ? NSTEP : RPS * NSTEP));     // units (QKV: waves, GATEUP: pairs, else rows) per workgroup
-    kern<<<dim3((unsigned)((units + per_wg - 1) / per_wg)), dim3(XG_THREADS), lds, st>>>(a);
+    kern<<<dim3((unsigned)((units + per_wg - 1) / per_wg)), dim3(XG_THREADS), lds, st>>>(XG_ARGS(a));
     return SPY_LAUNCH_RC();
 }
 
@@ -51,7 +51,7 @@ static int launch_xg_plain(hipStream_t st, const xg_args &a) {
     if (lds > 160 * 1024) return SPY_HIP_EUNSUPPORTED;
     auto kern = xgemv_kernel<WT, NITK, 1, 1, EPI_RESID, WT>;
     RC_TRY(spy_raise_lds_limit((const void *)kern, lds));
-    kern<<<dim3((unsigned)((a.M + XG_WAVES - 1) / XG_WAVES)), dim3(XG_THREADS), lds, st>>>(a);
+    kern<<<dim3((unsigned)((a.M + XG_WAVES - 1) / XG_WAVES)), dim3(XG_THREADS), lds, st>>>(XG_ARGS(a));
     return SPY_LAUNCH_RC();
 }
 // the LDS limits of these launches for every row length they take, raised ahead (spy_hip_init): an operator call then finds them

@@ -84,7 +84,8 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_kernel(gemv_args a) {
 #define WROW_DEPTH 3
 #define WROW_T 4
 template <int WT, int NITK, int NR>
-__global__ __launch_bounds__(WROW_THREADS) void wave_row_kernel(gemv_args a, int T) {
+__global__ __launch_bounds__(WROW_THREADS) void wave_row_kernel(const uint8_t *W, const uint8_t *xq, float *dst, const float *residual, int M, int K_, int T, gemv_args a) {
+    a.W = W; a.xq = xq; a.dst = dst; a.residual = residual; a.M = M; a.K = K_;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int NW = (int)gridDim.x * (WROW_THREADS / 64), gw = (int)blockIdx.x * (WROW_THREADS / 64) + wave;
@@ -139,7 +140,7 @@ template <int WT, int NITK, int NR>
 static int launch_wave_row_nr(hipStream_t st, const gemv_args &a, int T, size_t lds, int grid) {
     auto kern = wave_row_kernel<WT, NITK, NR>;
     { const int rc_ = spy_raise_lds_limit((const void *)kern, lds); if (rc_) return rc_; }
-    kern<<<dim3((unsigned)grid), dim3(WROW_THREADS), lds, st>>>(a, T);
+    kern<<<dim3((unsigned)grid), dim3(WROW_THREADS), lds, st>>>(a.W, a.xq, a.dst, a.residual, a.M, a.K, T, a);
     return SPY_LAUNCH_RC();
 }
 

@@ -527,6 +527,24 @@ static __device__ __forceinline__ float xa_tree8(const float (&sum)[8]) {
     const float v0 = u0 + u1, v1 = u2 + u3;
     return v0 + v1;
 }
+// Dot<FP16,FP16> of a key and its query by four adjacent lanes: lane `part` has elements 32 i + 8 part .. + 7 of either in piece i; the tail goes down the four lanes, eight
+// elements each, so that the result is in the lane of part 3
+static __device__ __forceinline__ float xa_dot4(const uint4 (&kv)[4], const uint4 (&q)[4]) {
+    float sum[8];
+#pragma unroll
+    for (int l = 0; l < 8; l++) sum[l] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 3; i++) xa_fma8(sum, kv[i], q[i]);
+    xa_quad(sum);
+    const float simd = xa_tree8(sum);
+    float tail = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if (j) tail = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(tail), 0x90, 0xF, 0xF, true));      // quad_perm [0, 0, 1, 2]
+        tail = xa_tail8(tail, kv[3], q[3]);
+    }
+    return tail + simd;
+}
 // a group of four of std::reduce's running sum
 static __device__ __forceinline__ float xa_group(const float4 v) {
     const float v1 = v.x + v.y, v2 = v.z + v.w;
@@ -594,20 +612,8 @@ __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_stat
             uint4 kv[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) kv[i] = make_uint4(k[u][i].x, k[u][i].y, k[u][i].z, k[u][i].w);
-            float sum[8];
-#pragma unroll
-            for (int l = 0; l < 8; l++) sum[l] = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 3; i++) xa_fma8(sum, kv[i], q[i]);
-            xa_quad(sum);
-            const float simd = xa_tree8(sum);
-            float tail = 0.0f;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if (j) tail = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(tail), 0x90, 0xF, 0xF, true));      // quad_perm [0, 0, 1, 2]
-                tail = xa_tail8(tail, kv[3], q[3]);
-            }
-            if (part == 3 && hh < n_head && tt + dt < t_end) scores[(size_t)h * n_ctx + tt + dt] = (tail + simd) * scale;
+            const float dot = xa_dot4(kv, q);
+            if (part == 3 && hh < n_head && tt + dt < t_end) scores[(size_t)h * n_ctx + tt + dt] = dot * scale;
             request(u, tt + 16 * nt * XS_NU);
         }
     }

@@ -152,8 +152,10 @@ static __device__ __forceinline__ void xg_dump_q8(const int8_t *s_q, const int2 
 
 // ---- phase 1: a lane's block pair of one weight row -> partial sums and scale products in LDS -------------------------
 // x[0..3]: the 64 int8 activations of the pair (16 bytes each), mm / mm2: their {scale bits, sum q} (see load_act_frag),
-// n8[i] = -8 * (sum of the four bytes of activation dword i): folds the -8 of the Q4_0 nibbles into the accumulator
-// input of v_dot4, so that each partial sum is sum (n - 8) * q exactly as sub_epi8 / maddubs / madd form it.
+// n8[i] = -8 * (sum of the four bytes of activation dword i): folds the -8 of the low Q4_0 nibbles into the accumulator
+// input of v_dot4, so that each partial sum is sum (n - 8) * q exactly as sub_epi8 / maddubs / madd form it.  High nibbles stay where they are: with their sign bit turned
+// they are 16 (n - 8) as signed bytes, one instruction instead of two, and accumulators 0..3 are walked times 16, which moves no rounding (every term is a
+// multiple of 2^-48 below 2^56 or not finite).  down 9.22 -> 8.50 us, qkv 10.73 -> 10.50, gate|up 14.8 -> 14.6.
 // slot: this row's LDS record; pl: the pair's index within the slab (= lane).
 template <int WT>
 static __device__ __forceinline__ void xg_phase1(const uint32_t *w, const act_frag<1> &f, const int (&n8)[16], int p, int pl, float *slot) {
@@ -172,9 +174,9 @@ static __device__ __forceinline__ void xg_phase1(const uint32_t *w, const act_fr
             for (int k = 0; k < 4; k++) {
                 // accumulators 4..7: low nibbles against elements 0..15; 0..3: high nibbles against 16..31 (vec_dot.h:62-78)
                 pa[4 + k] = __builtin_amdgcn_sdot4((int)(a[k] & 0x0F0F0F0Fu), xa[k], n8[k], false);
-                pa[k]     = __builtin_amdgcn_sdot4((int)((a[k] >> 4) & 0x0F0F0F0Fu), xb[k], n8[4 + k], false);
+                pa[k]     = __builtin_amdgcn_sdot4((int)((a[k] & 0xF0F0F0F0u) ^ 0x80808080u), xb[k], 0, false);
                 pb[4 + k] = __builtin_amdgcn_sdot4((int)(w[5 + k] & 0x0F0F0F0Fu), xc[k], n8[8 + k], false);
-                pb[k]     = __builtin_amdgcn_sdot4((int)((w[5 + k] >> 4) & 0x0F0F0F0Fu), xd[k], n8[12 + k], false);
+                pb[k]     = __builtin_amdgcn_sdot4((int)((w[5 + k] & 0xF0F0F0F0u) ^ 0x80808080u), xd[k], 0, false);
             }
         } else {
             sA = h2f((uint16_t)(w[0] & 0xFFFFu)) * __int_as_float(mm.x); sB = h2f((uint16_t)(w[8] >> 16)) * __int_as_float(mm.z);
@@ -447,7 +449,10 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
             }
         }
         // epilogue of the step: the lanes that walked accumulator 0 of a row hold its total after the tree
-        if (nch == 8) acc = xg_hsum8(acc);
+        if (nch == 8) {
+            if constexpr (WT == SPY_HIP_Q4_0) acc *= tid & 4 ? 1.0f : 0.0625f;    // accumulators 0..3 were walked times 16 (xg_phase1)
+            acc = xg_hsum8(acc);
+        }
         const bool owner = tid < chains && (tid % nch) == 0;
         const int slot_i = tid / nch;                                         // = wave_of_row * rows + j
         const int ow = slot_i / rows, oj = slot_i % rows;                      // the wave that owned the row and its index in the step

@@ -30,6 +30,8 @@ template <int WT> struct xg_traits { static constexpr int NCH = (WT == SPY_HIP_Q
 // floats of LDS per row slot: NCH rows of partials (+4: bank skew between the rows) and the row of scale products (+4: skew between slots)
 static __host__ __device__ constexpr int xg_slot_floats(int nch) { return nch * (XG_NBS + 4) + XG_NBS + 4; }
 
+#define XG_LDS_PAD 64                       // what xg_chain reads past the last row
+
 struct xg_args {
     const uint8_t *W0, *W1, *W2;
     int M, K;                              // output elements (RESID / STORE: rows of W0; GATEUP: rows of W0 = rows of W1; QKV: n_embd), contraction length
@@ -249,39 +251,42 @@ static __device__ __forceinline__ void xg_phase1(const uint32_t *w, const act_fr
 }
 
 // ---- phase 2: one lane walks one accumulator over the blocks of a slab ------------------------------------------------
-template <int NCH>
 static __device__ __forceinline__ float xg_chain(const float *P, const float *D, int nblk, float acc) {
-    // nblk % 4 == 0.  Eight blocks per group; the 128-bit reads of a group are requested two groups (sixteen dependent fmas,
-    // about the latency of an LDS read under load) before its fmas: three register sets in rotation, no copies.  Reads beyond
-    // nblk stay inside the row's 128 + 4 floats and are not used.
+    // Eight blocks per group (an odd four at the end of a row has zeros behind it, which leave a sum that started at +0 as it is).  The 128-bit reads of a group are
+    // requested two groups (sixteen dependent fmas, about the latency of an LDS read under load) before its fmas: three register sets in rotation, no copies.  Reads
+    // beyond the last group are not used.
     // (Taking the scale products, which the eight lanes of a row share, from one lane per quad through DPP broadcasts cut the LDS
     // traffic but measured slower: 1.25 instead of 0.8 us per 128 blocks.)
+    const int ng = (nblk + 7) >> 3;
     float4 p0[2], p1[2], p2[2], d0[2], d1[2], d2[2];
-    auto ld = [&](float4 (&p)[2], float4 (&d)[2], int b) {
+    auto ld = [&](float4 (&p)[2], float4 (&d)[2], int g) {
 #pragma unroll
-        for (int u = 0; u < 2; u++) { p[u] = *(const float4 *)(P + min(b + 4 * u, XG_NBS - 4)); d[u] = *(const float4 *)(D + min(b + 4 * u, XG_NBS - 4)); }
+        for (int u = 0; u < 2; u++) { p[u] = *(const float4 *)(P + 8 * g + 4 * u); d[u] = *(const float4 *)(D + 8 * g + 4 * u); }
     };
-    auto run = [&](const float4 (&p)[2], const float4 (&d)[2], int b) {
+    auto run = [&](const float4 (&p)[2], const float4 (&d)[2]) {
 #pragma unroll
-        for (int u = 0; u < 2; u++)
-            if (b + 4 * u < nblk) { acc = fmaf(d[u].x, p[u].x, acc); acc = fmaf(d[u].y, p[u].y, acc); acc = fmaf(d[u].z, p[u].z, acc); acc = fmaf(d[u].w, p[u].w, acc); }
+        for (int u = 0; u < 2; u++) { acc = fmaf(d[u].x, p[u].x, acc); acc = fmaf(d[u].y, p[u].y, acc); acc = fmaf(d[u].z, p[u].z, acc); acc = fmaf(d[u].w, p[u].w, acc); }
     };
     ld(p0, d0, 0);
-    ld(p1, d1, 8);
-    for (int b = 0; b < nblk; b += 24) {
-        ld(p2, d2, b + 16);
+    ld(p1, d1, 1);
+    int g = 0;
+#pragma unroll 1
+    for (; g + 3 <= ng; g += 3) {
+        ld(p2, d2, g + 2);
         __builtin_amdgcn_sched_barrier(0);
-        run(p0, d0, b);
+        run(p0, d0);
         __builtin_amdgcn_sched_barrier(0);
-        ld(p0, d0, b + 24);
+        ld(p0, d0, g + 3);
         __builtin_amdgcn_sched_barrier(0);
-        run(p1, d1, b + 8);
+        run(p1, d1);
         __builtin_amdgcn_sched_barrier(0);
-        ld(p1, d1, b + 32);
+        ld(p1, d1, g + 4);
         __builtin_amdgcn_sched_barrier(0);
-        run(p2, d2, b + 16);
+        run(p2, d2);
         __builtin_amdgcn_sched_barrier(0);
     }
+    if (g < ng) run(p0, d0);
+    if (g + 1 < ng) run(p1, d1);
     return acc;
 }
 
@@ -433,6 +438,8 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
                     if (p < npair) {
                         if (vstep) { if constexpr (WTV != WT) xg_phase1<WTV>(tv.w[it], av, n8, p, lane, slot); else xg_phase1<WTV>(tv.w[it], af, n8, p, lane, slot); }
                         else xg_phase1<WT>(t[r % RING].w[it], af, n8, p, lane, slot);
+                    } else if (p < ((npair + 3) & ~3)) {                      // xg_chain's odd four blocks
+                        for (int l = 0; l <= nch; l++) *(float2 *)(slot + l * (XG_NBS + 4) + 2 * lane) = make_float2(0.0f, 0.0f);
                     }
                 }
                 XSTAMP(a.dbg, 18 + 3 * (step * NITK + it));
@@ -441,8 +448,7 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
                 if (tid < chains) {
                     const int slot_i = tid / nch, l = tid % nch;
                     const float *slot = s_part + (size_t)slot_i * SLOTF;
-                    if (nch == 8) acc = xg_chain<8>(slot + l * (XG_NBS + 4), slot + nch * (XG_NBS + 4), nblk, acc);
-                    else acc = xg_chain<1>(slot + l * (XG_NBS + 4), slot + nch * (XG_NBS + 4), nblk, acc);
+                    acc = xg_chain(slot + l * (XG_NBS + 4), slot + nch * (XG_NBS + 4), nblk, acc);
                 }
                 XSTAMP(a.dbg, 20 + 3 * (step * NITK + it));
                 __syncthreads();

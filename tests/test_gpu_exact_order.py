@@ -98,6 +98,26 @@ NARROW_SHAPES = [(12288, 256, 16), (12284, 768, 10), (8196, 512, 10), (4096, 256
 ANY_SCALE_SHAPES = [(11000, 256, 40), (8192, 768, 70), (4100, 512, 150), (4096, 1280, 300), (24604, 256, 17), (8196, 512, 1000), (12300, 256, 2025)]
 
 
+@pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0])
+@pytest.mark.parametrize("K", [384, 896, 4224, 8064, 12160])
+def test_single_row_matmul_ends_in_half_a_group(hip, oracle, wtype, K):
+    """The walk takes eight blocks at a time: rows and slabs that end in four, whose zeros lie in LDS that held something else before.  Activations of one sign, so that no sum hides
+    what it should not have added."""
+    from tests.gpu_util import dev, dev_empty, call
+    M = 37
+    rng = np.random.default_rng(K + wtype)
+    w = O.quantize(oracle, (rng.standard_normal((M, K)) * 0.02).astype(np.float32), wtype)
+    x = np.abs(rng.standard_normal((1, K)) * 3.0).astype(np.float32)
+    want = O.matmul(oracle, w, wtype, M, K, x, nthread=8)[0]
+    dw, dx, do = dev(w), dev(x), dev_empty(M * 4, 0xEE)
+    L = hip.load()
+    tw, tx, to = hip.tensor(dw.ptr, wtype, [K, M]), hip.tensor(dx.ptr, O.F32, [K, 1]), hip.tensor(do.ptr, O.F32, [M, 1])
+    need = L.spy_hip_op_matmul_scratch_size(B(tw), B(tx))
+    sc = dev_empty(max(need, 1), 0xEE)
+    call(L.spy_hip_op_matmul, None, B(tw), B(tx), B(to), sc.ptr, need)
+    assert np.array_equal(do.download(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0, O.Q4_K, O.Q6_K])
 @pytest.mark.parametrize("M,K,T", PACKED_SHAPES)
 def test_packed_activation_matmul_bits(hip, oracle, wtype, M, K, T):

@@ -175,18 +175,18 @@ static __device__ __forceinline__ void xg_phase1(const uint32_t *w, const act_fr
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 // accumulators 4..7: low nibbles against elements 0..15; 0..3: high nibbles against 16..31 (vec_dot.h:62-78)
-                pa[4 + k] = __builtin_amdgcn_sdot4((int)(a[k] & 0x0F0F0F0Fu), xa[k], n8[k], false);
-                pa[k]     = __builtin_amdgcn_sdot4((int)((a[k] & 0xF0F0F0F0u) ^ 0x80808080u), xb[k], 0, false);
-                pb[4 + k] = __builtin_amdgcn_sdot4((int)(w[5 + k] & 0x0F0F0F0Fu), xc[k], n8[8 + k], false);
-                pb[k]     = __builtin_amdgcn_sdot4((int)((w[5 + k] & 0xF0F0F0F0u) ^ 0x80808080u), xd[k], 0, false);
+                pa[4 + k] = __builtin_amdgcn_sdot4((int)(a[k] & 0x0F0F0F0Fu), xa[k], n8[k], true);
+                pa[k]     = __builtin_amdgcn_sdot4((int)((a[k] & 0xF0F0F0F0u) ^ 0x80808080u), xb[k], 0, true);
+                pb[4 + k] = __builtin_amdgcn_sdot4((int)(w[5 + k] & 0x0F0F0F0Fu), xc[k], n8[8 + k], true);
+                pb[k]     = __builtin_amdgcn_sdot4((int)((w[5 + k] & 0xF0F0F0F0u) ^ 0x80808080u), xd[k], 0, true);
             }
         } else {
             sA = h2f((uint16_t)(w[0] & 0xFFFFu)) * __int_as_float(mm.x); sB = h2f((uint16_t)(w[8] >> 16)) * __int_as_float(mm.z);
             const int xa[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w}, xb[8] = {x2.x, x2.y, x2.z, x2.w, x3.x, x3.y, x3.z, x3.w};
 #pragma unroll
             for (int l = 0; l < 8; l++) {               // accumulator l: elements 4l..4l+3 (vec_util.h:126-132)
-                pa[l] = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_alignbit(w[l + 1], w[l], 16), xa[l], 0, false);
-                pb[l] = __builtin_amdgcn_sdot4((int)w[9 + l], xb[l], 0, false);
+                pa[l] = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_alignbit(w[l + 1], w[l], 16), xa[l], 0, true);
+                pb[l] = __builtin_amdgcn_sdot4((int)w[9 + l], xb[l], 0, true);
             }
         }
 #pragma unroll

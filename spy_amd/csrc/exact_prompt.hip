@@ -15,6 +15,7 @@
 // Values that cannot occur are not looked after: the fp16 caches are written by this library's float -> half
 // conversion, which never produces the pattern 0xFFFF that the host's conversion table maps to 0 (conversion.h:39-41).
 #include "common.cuh"
+#include "exact_exp.cuh"
 #include "exact_sum.cuh"
 
 #include <type_traits>
@@ -167,20 +168,25 @@ __global__ __launch_bounds__(256, 3) void xp_scores_kernel(const void *__restric
 // lane keeps its share of the row in registers (groups of four consecutive elements, the unit of the host's sum), so the row is read once
 // and written once.  The probabilities leave as fp16 (the first step of the KQV MatMul, mat.cpp:37), followed by zeros up to the end of the
 // 32-row tile's last chunk, which the product kernel reads.
-// The exponentials: a gather of 64 table entries from memory takes about 64 cycles of the compute unit, so the part of the table that is not zero lies in
+// The exponentials: a gather of 64 table entries from memory takes about 64 cycles of the compute unit, so for many rows the part of the table that is not zero lies in
 // LDS: arguments are <= 0 (or NaN), and exp is 0 from -104 on.  The sum of a row goes through xg_segment_sum: 2 us instead of a chain of up to
 // 1024 additions.  2048 rows of 2049 .. 4096 positions and 32 heads (1.2 GB): 462 -> 306 us; 2048 rows of 1 .. 2048: 193 -> 152.
 // A row of a wave is a chain of latencies, so waves are what counts: with half the registers and group sums for rows of up to 2048 positions a workgroup has 16
 // instead of 12 (2048 rows of 1 .. 2048 positions 155 -> 123 us, 1000 rows 66 -> 50, 512 rows 29 -> 21).  The next row's scores requested a row ahead: 160 instead of 123.
-#define XP_LUT 0x5680      // fp16 -104.0 without its sign
+// LIST: few rows, where bringing 88 KB of table to every compute unit is most of the time: the exponentials are worked out (exact_exp.cuh), which is 5.5 KB and about twice the vector
+// instructions (32 heads, table -> list: 8 rows 7.2 -> 5.0 us, 33 6.9 -> 5.0, 200 on 100 positions 11.9 -> 9.7, 512 22.6 -> 20.5, 1000 45.3 -> 46.1, 2048 118 -> 123; rows of up to 4096 positions:
+// 2048 301 -> 303).
+#define XP_LUT XE_MAX
+#define XP_LIST_ROWS 24576
 #define XP_SM_R 32         // groups per lane: rows of up to 8192 positions
-template <int R, int NW>
-__global__ __launch_bounds__(64 * NW) void xp_softmax_kernel(const float *__restrict__ S, uint16_t *__restrict__ P16, const float *__restrict__ lut, int T, int H, int P,
+template <int R, int NW, int OCC, bool LIST>
+__global__ __launch_bounds__(64 * NW, OCC) void xp_softmax_kernel(const float *__restrict__ S, uint16_t *__restrict__ P16, const float *__restrict__ lut, int T, int H, int P,
                                                              int64_t s_row, int n_total, float scale) {
-    extern __shared__ __align__(16) float s_mem[];               // table, then per wave 64 R padded group sums and 4 floats
+    constexpr int TAB = LIST ? XE_WORDS : XP_LUT + 4;
+    extern __shared__ __align__(16) float s_mem[];               // table or list, then per wave 64 R padded group sums and 4 floats
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    float *s_grp = s_mem + XP_LUT + 4 + wave * (80 * R + 4), *s_rem = s_grp + 80 * R;
-    for (int i = threadIdx.x; i <= XP_LUT / 4; i += 64 * NW) ((float4 *)s_mem)[i] = ((const float4 *)(lut + 0x8000))[i];
+    float *s_grp = s_mem + TAB + wave * (80 * R + 4), *s_rem = s_grp + 80 * R;
+    for (int i = threadIdx.x; i < TAB / 4; i += 64 * NW) ((float4 *)s_mem)[i] = ((const float4 *)(lut + (LIST ? XE_AT : 0x8000)))[i];
     __syncthreads();
     const int rows = T * H;
     for (int id = (int)blockIdx.x * NW + wave; id < rows; id += (int)gridDim.x * NW) {
@@ -214,14 +220,18 @@ __global__ __launch_bounds__(64 * NW) void xp_softmax_kernel(const float *__rest
             if (64 * r < ng_row) {
                 float e[4] = {v[r].x, v[r].y, v[r].z, v[r].w};
                 uint32_t hx[4];
+                bool ask[4];
 #pragma unroll
                 for (int k = 0; k < 4; k++) hx[k] = f2h(mx - e[k]);          // the argument without its sign
 #pragma unroll
-                for (int k = 0; k < 4; k++) e[k] = s_mem[min(hx[k], (uint32_t)XP_LUT)];      // entry XP_LUT: 0, exp of everything below
-                if (__any(max(max(hx[0], hx[1]), max(hx[2], hx[3])) > 0x7C00u)) {            // a NaN somewhere
+                for (int k = 0; k < 4; k++) {
+                    if constexpr (LIST) e[k] = xe_exp(hx[k], (const uint32_t *)s_mem, ask[k]);
+                    else { e[k] = s_mem[min(hx[k], (uint32_t)XP_LUT)]; ask[k] = hx[k] > 0x7C00u; }      // entry XP_LUT: 0, exp of everything below
+                }
+                if (__any(ask[0] || ask[1] || ask[2] || ask[3])) {           // a NaN somewhere
                     const float w[4] = {v[r].x, v[r].y, v[r].z, v[r].w};
 #pragma unroll
-                    for (int k = 0; k < 4; k++) if (hx[k] > 0x7C00u && 4 * (lane + 64 * r) + k < L) e[k] = lut[f2h(w[k] - mx)];
+                    for (int k = 0; k < 4; k++) if (ask[k] && 4 * (lane + 64 * r) + k < L) e[k] = lut[f2h(w[k] - mx)];
                 }
                 v[r] = make_float4(e[0], e[1], e[2], e[3]);
                 const int g = lane + 64 * r;
@@ -246,14 +256,15 @@ __global__ __launch_bounds__(64 * NW) void xp_softmax_kernel(const float *__rest
         __builtin_amdgcn_wave_barrier();
     }
 }
-template <int R, int NW>
+template <int R, int NW, int OCC, bool LIST>
 int xp_softmax_launch(hipStream_t st, const float *S, uint16_t *P16, const float *lut, int T, int H, int P, int64_t s_row, int n_total, float scale, int ncu) {
-    constexpr size_t lds = (XP_LUT + 4 + NW * (80 * R + 4)) * 4;
-    static_assert(lds <= 160 * 1024, "");
-    const int rc = spy_raise_lds_limit((const void *)xp_softmax_kernel<R, NW>, lds);
+    constexpr size_t lds = ((LIST ? XE_WORDS : XP_LUT + 4) + NW * (80 * R + 4)) * 4;
+    constexpr int WGS = OCC * 4 / NW;                            // workgroups on a compute unit
+    static_assert(lds * WGS <= 160 * 1024, "");
+    const int rc = spy_raise_lds_limit((const void *)xp_softmax_kernel<R, NW, OCC, LIST>, lds);
     if (rc) return rc;
-    const int64_t need = ((int64_t)T * H + NW - 1) / NW;
-    xp_softmax_kernel<R, NW><<<dim3((unsigned)(need < ncu ? need : ncu)), dim3(64 * NW), lds, st>>>(S, P16, lut, T, H, P, s_row, n_total, scale);
+    const int64_t need = ((int64_t)T * H + NW - 1) / NW, most = (int64_t)ncu * WGS;
+    xp_softmax_kernel<R, NW, OCC, LIST><<<dim3((unsigned)(need < most ? need : most)), dim3(64 * NW), lds, st>>>(S, P16, lut, T, H, P, s_row, n_total, scale);
     return SPY_LAUNCH_RC();
 }
 
@@ -382,10 +393,13 @@ int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint1
     if (q_f16) xp_scores_kernel<true><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
     else xp_scores_kernel<false><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
     if (hipGetLastError() != hipSuccess) return SPY_HIP_EINVAL;
-    const int ncu = spy_num_cu(), rc = (int64_t)P + T <= 2048 ? xp_softmax_launch<8, 16>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
-                                         : (int64_t)P + T <= 4096 ? xp_softmax_launch<16, 12>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
-                                         : (int64_t)P + T <= 6144 ? xp_softmax_launch<24, 8>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
-                                                                  : xp_softmax_launch<32, 4>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu);
+    const int64_t n_kv = (int64_t)P + T;
+    const int ncu = spy_num_cu();
+    const bool few = (int64_t)T * H <= XP_LIST_ROWS;
+#define XP_SOFTMAX(...) xp_softmax_launch<__VA_ARGS__>(st, S, P16, lut, T, H, P, s_row, n_total, scale, ncu)
+    const int rc = n_kv <= 2048 ? (few ? XP_SOFTMAX(8, 4, 5, true) : XP_SOFTMAX(8, 16, 4, false)) : n_kv <= 4096 ? (few ? XP_SOFTMAX(16, 4, 3, true) : XP_SOFTMAX(16, 12, 3, false))
+                 : n_kv <= 6144 ? XP_SOFTMAX(24, 8, 2, false) : XP_SOFTMAX(32, 4, 1, false);
+#undef XP_SOFTMAX
     if (rc) return rc;
     xp_pv_kernel<<<dim3((unsigned)H, 4, (unsigned)((T + 31) / 32)), dim3(256), 0, st>>>(P16, vt, out, T, H, P, s_row, C, n_total);
     return SPY_LAUNCH_RC();

@@ -841,3 +841,31 @@ def test_llama2_7b_greedy_32_tokens_identical(wtype):
         eng.close()
     finally:
         H.load().spy_hip_set_exact_order(prev)
+
+
+@pytest.mark.parametrize("past", [0, 2048])
+def test_prompt_softmax_worked_out_and_from_the_table(hip, past):
+    """Up to 24 576 rows the prompt's softmax works its exponentials out, beyond it reads them from the table: a row has the same bits either way, also with scores
+    that spread over more than 104, with -inf among them and with NaN."""
+    from tests.gpu_util import dev, dev_empty, call
+    H_, hd, T = 32, 128, 768
+    d, n = H_ * hd, past + T + 1
+    n_ctx = (n + 31) // 32 * 32
+    rng = np.random.default_rng(past)
+    q = rng.standard_normal((T + 1, d)).astype(np.float32)
+    q[::5] *= 25.0
+    q[7] = np.nan
+    kc, vt = rng.standard_normal((n_ctx, d)).astype(np.float16), rng.standard_normal((d, n_ctx)).astype(np.float16)
+    kc[3, 5::128] = np.inf                                  # score +inf or -inf of token 3, by the sign of q's element
+    L = hip.load()
+    dq, dk, dv = dev(q), dev(kc.view(np.uint16)), dev(vt.view(np.uint16))
+    res = []
+    for t in (T, T + 1):
+        need = L.spy_hip_prompt_attention_exact_scratch_size(t, H_, past)
+        sc, do = dev_empty(need, 0xEE), dev_empty(t * d * 4, 0xEE)
+        call(L.spy_hip_prompt_attention_exact, None, dq.ptr, dk.ptr, dv.ptr, do.ptr, t, H_, hd, past, n_ctx, n, C.c_float(1.0 / np.sqrt(np.float32(hd))), sc.ptr, need)
+        hip.sync()
+        res.append(do.download(np.uint32).reshape(t, d)[:T].copy())
+    assert np.array_equal(res[0], res[1])
+    f = res[0].view(np.float32)
+    assert np.isfinite(f).any() and np.isnan(f[7]).all()

@@ -391,6 +391,8 @@ bool spy_gemm_unsplit_shape(int64_t M, int64_t T);                              
 int spy_xgemm(hipStream_t st, int wtype, int nmat, const void *const *w, float *const *dst, int64_t M, int64_t K, int64_t T, int64_t d_row, const float *resid, const void *pack);
 int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, float *out, const float *lut,
                           int T, int H, int P, int64_t C, int n_total, float scale);                                        // exact_prompt.hip
+int spy_exact_prompt_attn_pack(hipStream_t st, const uint16_t *q16, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, void *pack, const float *lut,
+                               int T, int H, int P, int64_t C, int n_total, float scale);                                   // exact_prompt.hip
 
 // KQ mask of a pass over tokens P .. P + T - 1 (llama.cpp:248-263): row i allows the cached positions j <= P + i
 __global__ __launch_bounds__(256) void causal_mask_kernel(float *__restrict__ mask, int C, int P) {
@@ -415,7 +417,7 @@ static int ops_workspace(spy_hip_llama *m, hipStream_t st, size_t bytes) {
     return 0;
 }
 
-// A prompt pass in the host's order with what lies between two MatMuls in the kernels around them, 13 launches per layer instead of 42:
+// A prompt pass in the host's order with what lies between two MatMuls in the kernels around them, 12 launches per layer instead of 42:
 // norm and activation end in the next MatMul's packed activations (quantized once for wq | wk | wv and for gate | up, which are one launch
 // each where their types allow), Rope stores q as fp16 and k into its cache rows, the residual additions are the products' epilogues.  Each
 // step is the arithmetic of the operator it replaces, so the bits are those of forward_ops with the exact order on.
@@ -436,12 +438,12 @@ static int forward_exact(spy_hip_llama *m, hipStream_t st, const int32_t *tokens
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off += (bytes + 255) & ~(size_t)255; return o; };
     const size_t sp = (size_t)spy_exact_prompt_attn_row((int64_t)P + T) * T * H;
-    const size_t o_x = take(d * T * 4), o_t1 = take(d * T * 4), o_q = take(d * T * 4), o_k = take(d * T * 4), o_v = take(d * T * 4), o_o2 = take(d * T * 4), o_q16 = take(d * T * 2),
+    const size_t o_x = take(d * T * 4), o_t1 = take(d * T * 4), o_q = take(d * T * 4), o_k = take(d * T * 4), o_v = take(d * T * 4), o_q16 = take(d * T * 2),
                  o_up = take(F * T * 4), o_gate = take(F * T * 4), o_S = take(sp * 4), o_P = take(sp * 2), o_ids = take(T * 4), o_xn = take(d * 4),
                  o_logits = take(head == HEAD_ALL ? V * T * 4 : V * 4), o_pack = take(spy_xgemm_pack_bytes(T, F > d ? F : d));
     RC_TRY(ops_workspace(m, st, off));
     uint8_t *B = m->ops_buf;
-    float *x = (float *)(B + o_x), *t1 = (float *)(B + o_t1), *q = (float *)(B + o_q), *k = (float *)(B + o_k), *v = (float *)(B + o_v), *o2 = (float *)(B + o_o2),
+    float *x = (float *)(B + o_x), *t1 = (float *)(B + o_t1), *q = (float *)(B + o_q), *k = (float *)(B + o_k), *v = (float *)(B + o_v),
           *up = (float *)(B + o_up), *gate = (float *)(B + o_gate), *lg = (float *)(B + o_logits), *xn = (float *)(B + o_xn);
     uint16_t *q16 = (uint16_t *)(B + o_q16);
     int32_t *ids = (int32_t *)(B + o_ids);
@@ -461,8 +463,7 @@ static int forward_exact(spy_hip_llama *m, hipStream_t st, const int32_t *tokens
         if (together == 2) RC_TRY(spy_xgemm(st, L.t_wv, 1, w3 + 2, d3 + 2, d, d, T, d, nullptr, pack));
         RC_TRY(spy_rope_store_launch(st, q, k, m->rope_tab + (size_t)P * hd, q16, m->k_cache[il] + d * P, T, (int)H, (int)hd));
         RC_TRY(spy_vt_store_launch(st, v, m->v_cache[il] + P, T, (int)d, C));
-        RC_TRY(spy_exact_prompt_attn(st, q16, true, m->k_cache[il], m->v_cache[il], (float *)(B + o_S), (uint16_t *)(B + o_P), o2, m->lut, T, (int)H, P, C, n_total, scale));
-        RC_TRY(spy_xgemm_pack(st, o2, 4 * d, T, d, pack));
+        RC_TRY(spy_exact_prompt_attn_pack(st, q16, m->k_cache[il], m->v_cache[il], (float *)(B + o_S), (uint16_t *)(B + o_P), pack, m->lut, T, (int)H, P, C, n_total, scale));
         RC_TRY(spy_xgemm(st, L.t_wo, 1, &L.wo, &t1, d, d, T, d, x, pack));                     // KQV_linear + Add
         RC_TRY(spy_xgemm_norm_pack(st, false, t1, L.ffn_norm, c.eps, T, d, pack));
         const void *w2[2] = {L.w_up, L.w_gate};

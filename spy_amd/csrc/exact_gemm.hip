@@ -20,6 +20,7 @@
 #include "common.cuh"
 #include "exact_sum.cuh"
 #include "gemm_tiles.h"
+#include "xt_pack.cuh"
 
 #include <type_traits>
 #include <utility>
@@ -29,12 +30,6 @@ namespace {
 typedef _Float16 xt_h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 xt_h4 __attribute__((ext_vector_type(4)));
 typedef float xt_v16f __attribute__((ext_vector_type(16)));
-
-// Layout of packed activations, per group of 16 rows and stage of four Q8_0 blocks: XT_XB bytes of quants
-//   [block][word pair g][row][word of the pair][4 x fp16: elements 0, 2, 1, 3 of the word]
-// and one record of XT_XD bytes: scales [block][row], fp16 in the lower half of a dword, then the sums of the quants [block][row], fp32
-#define XT_XB 4096
-#define XT_XD 512
 
 // 16 (4) bytes per lane from base + off to LDS bytes lds .. in lane order; base and lds are uniform over the wave.  Written as
 // instructions so that the compiler does not wait for them at the next LDS read; xt_wait_vm says when they have to be there.
@@ -444,33 +439,13 @@ int xn_launch(hipStream_t st, xt_args a, int nmat) {
     return SPY_LAUNCH_RC();
 }
 
-// f32 rows -> packed activations: Quantizator<FP32,Q8_0>::transform (vec_convert.h:178-261), as quantize_q8_0_kernel, the quants as fp16.
-// Rows past T become zeros.  8 lanes per block; a workgroup takes 16 rows and two blocks.
+// f32 rows -> packed activations.  Rows past T become zeros.  8 lanes per block; a workgroup takes 16 rows and two blocks.
 __global__ __launch_bounds__(256) void xt_pack_kernel(const uint8_t *__restrict__ x, int64_t x_stride, int T, int nst, uint8_t *__restrict__ xq, uint8_t *__restrict__ xd) {
     const int tid = threadIdx.x, e = tid & 7, c = (tid >> 3) & 15, b = (int)blockIdx.x * 2 + (tid >> 7), cg = blockIdx.y;
     const int t = cg * 16 + c;
     float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (t < T) v = *(const float4 *)(x + (int64_t)t * x_stride + (b * 32 + e * 4) * 4);
-    float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-    amax = fmaxf(amax, __shfl_xor(amax, 1, SPY_WAVE));
-    amax = fmaxf(amax, __shfl_xor(amax, 2, SPY_WAVE));
-    amax = fmaxf(amax, __shfl_xor(amax, 4, SPY_WAVE));
-    const float d = amax / 127.0f, id = (amax != 0.0f) ? 127.0f / amax : 0.0f;
-    int qv[4] = {(int)rintf(v.x * id), (int)rintf(v.y * id), (int)rintf(v.z * id), (int)rintf(v.w * id)};
-    uint32_t h[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) { qv[i] = qv[i] < -128 ? -128 : (qv[i] > 127 ? 127 : qv[i]); h[i] = __builtin_bit_cast(uint16_t, (_Float16)(float)qv[i]); }
-    uint8_t *o = xq + ((int64_t)cg * nst + (b >> 2)) * XT_XB + (b & 3) * 1024 + (e >> 1) * 256 + c * 16 + (e & 1) * 8;
-    *(uint2 *)o = make_uint2(h[0] | (h[2] << 16), h[1] | (h[3] << 16));
-    int sum = (qv[0] + qv[1]) + (qv[2] + qv[3]);
-    sum += __shfl_xor(sum, 1, SPY_WAVE);
-    sum += __shfl_xor(sum, 2, SPY_WAVE);
-    sum += __shfl_xor(sum, 4, SPY_WAVE);
-    if (e == 0) {
-        uint32_t *rec = (uint32_t *)(xd + ((int64_t)cg * nst + (b >> 2)) * XT_XD + (b & 3) * 64 + c * 4);
-        rec[0] = f2h(d);
-        rec[64] = __float_as_uint((float)sum);
-    }
+    xt_store4(v, cg, nst, b, c, e, xq, xd);
 }
 
 // ---- producers: the operators in front of a MatMul, ending in its packed activations, in the host's order ---------------------------------

@@ -17,6 +17,7 @@
 #include "common.cuh"
 #include "exact_exp.cuh"
 #include "exact_sum.cuh"
+#include "xt_pack.cuh"
 
 #include <type_traits>
 
@@ -277,8 +278,12 @@ int xp_softmax_launch(hipStream_t st, const float *S, uint16_t *P16, const float
 // What bounds it: 348 us of matrix instructions and, beside none of them, the two conversions each needs (about 90).  Straight from memory without LDS:
 // 705 us (the L2); two waves per SIMD instead of three: 609.
 typedef uint32_t xp_u4 __attribute__((ext_vector_type(4), aligned(2)));          // V^T rows of a caller's cache: no more alignment than an element's
+// PACK: the outputs leave as the packed activations of the MatMul that follows (xt_pack.cuh) instead of as floats: the 32 outputs of a row that a workgroup forms
+// are one Q8_0 block.  A launch less, and the outputs do not go through memory: 8 rows 3.5 + 2.6 -> 4.4 us, 33 4.7 + 4.7 -> 5.1,
+// 77 on 1000 positions 16.6 + 4.9 -> 17.5, 512 19.2 + 5.4 -> 21.6, 2048 215 + 10.2 -> 224.
+template <bool PACK>
 __global__ __launch_bounds__(256, 3) void xp_pv_kernel(const uint16_t *__restrict__ P16, const uint16_t *__restrict__ vt, float *__restrict__ out,
-                                                       int T, int H, int P, int64_t p_row, int64_t C, int n_total) {
+                                                       int T, int H, int P, int64_t p_row, int64_t C, int n_total, uint8_t *__restrict__ pack) {
     __shared__ __align__(16) xp_v4u s_v[2][32][8], s_p[2][32][8];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, j = lane & 15;
     const int h = blockIdx.x, tb = ((int)gridDim.z - 1 - (int)blockIdx.z) * 32;      // head fastest: see xp_scores_kernel
@@ -362,27 +367,37 @@ __global__ __launch_bounds__(256, 3) void xp_pv_kernel(const uint16_t *__restric
         for (int v = 0; v < 4; v++) u[l][v] = x[v] + y[v];
     }
     const int t = t0 + j;
-    if (t >= T) return;
+    if (!PACK && t >= T) return;
     float o[4];
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         const float x = u[0][v] + u[1][v], y = u[2][v] + u[3][v];
         o[v] = tail[v] + (x + y);
     }
-    *(float4 *)(out + (int64_t)t * H * 128 + (int64_t)h * 128 + dd0 + 4 * g) = make_float4(o[0], o[1], o[2], o[3]);
+    if constexpr (PACK) {
+        // the 32 x 32 outputs through LDS (rows of 36 floats) to eight lanes per row; rows past T are zeros
+        static_assert(32 * 36 * 4 <= sizeof(s_v), "");
+        float *s_o = (float *)s_v;
+        const float4 z = t < T ? make_float4(o[0], o[1], o[2], o[3]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        __syncthreads();
+        *(float4 *)(s_o + ((wave >> 1) * 16 + j) * 36 + (wave & 1) * 16 + 4 * g) = z;
+        __syncthreads();
+        const int c = threadIdx.x >> 3, e = threadIdx.x & 7, ncg = (T + 15) / 16, cg = tb / 16 + (c >> 4);
+        if (cg < ncg) xt_store4(*(const float4 *)(s_o + c * 36 + 4 * e), cg, H, h * 4 + (int)blockIdx.y, c & 15, e, pack, pack + (int64_t)ncg * H * XT_XB);
+    } else *(float4 *)(out + (int64_t)t * H * 128 + (int64_t)h * 128 + dd0 + 4 * g) = make_float4(o[0], o[1], o[2], o[3]);
 }
 
 }   // namespace
 
-// q: after Rope, fp32 [T][H][128], or (q_f16) fp16 [H][T][128]; kc: fp16 [position][H][128]; vt: fp16 [H * 128][C]; out: fp32 [T][H][128];
+// q: after Rope, fp32 [T][H][128], or (q_f16) fp16 [H][T][128]; kc: fp16 [position][H][128]; vt: fp16 [H * 128][C]; out: fp32 [T][H][128], or pack: the outputs as packed activations;
 // S: H * T * s_row floats and P16: H * T * s_row halves of scratch, s_row = spy_exact_prompt_attn_row(P + T)
 int64_t spy_exact_prompt_attn_row(int64_t n_kv) { return (n_kv + 127) & ~(int64_t)127; }
 
-int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, float *out, const float *lut,
-                          int T, int H, int P, int64_t C, int n_total, float scale) {
+static int prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, float *out, const float *lut,
+                          int T, int H, int P, int64_t C, int n_total, float scale, void *pack) {
     if (T <= 0 || H <= 0 || H > 65535 || P < 0 || (int64_t)P + T > C || n_total < P + T || n_total > C || C % 32) return SPY_HIP_EINVAL;
     if ((int64_t)P + T > 256 * XP_SM_R) return SPY_HIP_EUNSUPPORTED;      // the softmax kernel keeps a row in the registers of a wave
-    if (((uintptr_t)q & 15) || ((uintptr_t)kc & 15) || ((uintptr_t)S & 15) || ((uintptr_t)P16 & 15) || ((uintptr_t)out & 15)) return SPY_HIP_EINVAL;
+    if (((uintptr_t)q & 15) || ((uintptr_t)kc & 15) || ((uintptr_t)S & 15) || ((uintptr_t)P16 & 15) || ((uintptr_t)out & 15) || ((uintptr_t)pack & 15)) return SPY_HIP_EINVAL;
     const int64_t s_row = spy_exact_prompt_attn_row((int64_t)P + T);
     // segments of the cached positions: 512 long where that fills the chip, down to one key tile for short passes (77 tokens on 1000 cached ones
     // gave 96 workgroups: 114 us; one per 64 positions and 64 query rows 29)
@@ -401,8 +416,21 @@ int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint1
                  : n_kv <= 6144 ? XP_SOFTMAX(24, 8, 2, false) : XP_SOFTMAX(32, 4, 1, false);
 #undef XP_SOFTMAX
     if (rc) return rc;
-    xp_pv_kernel<<<dim3((unsigned)H, 4, (unsigned)((T + 31) / 32)), dim3(256), 0, st>>>(P16, vt, out, T, H, P, s_row, C, n_total);
+    const dim3 pgrid((unsigned)H, 4, (unsigned)((T + 31) / 32));
+    if (pack) xp_pv_kernel<true><<<pgrid, dim3(256), 0, st>>>(P16, vt, nullptr, T, H, P, s_row, C, n_total, (uint8_t *)pack);
+    else xp_pv_kernel<false><<<pgrid, dim3(256), 0, st>>>(P16, vt, out, T, H, P, s_row, C, n_total, nullptr);
     return SPY_LAUNCH_RC();
+}
+
+int spy_exact_prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, float *out, const float *lut,
+                          int T, int H, int P, int64_t C, int n_total, float scale) {
+    return prompt_attn(st, q, q_f16, kc, vt, S, P16, out, lut, T, H, P, C, n_total, scale, nullptr);
+}
+// q: fp16 [H][T][128]; the outputs as packed activations: spy_xgemm_pack_bytes(T, 128 H) bytes
+int spy_exact_prompt_attn_pack(hipStream_t st, const uint16_t *q16, const uint16_t *kc, const uint16_t *vt, float *S, uint16_t *P16, void *pack, const float *lut,
+                               int T, int H, int P, int64_t C, int n_total, float scale) {
+    if (!pack || H % 2) return SPY_HIP_EINVAL;
+    return prompt_attn(st, q16, true, kc, vt, S, P16, nullptr, lut, T, H, P, C, n_total, scale, pack);
 }
 
 int spy_exact_luts(const float **lut);           // exact_order.hip

@@ -869,3 +869,32 @@ def test_prompt_softmax_worked_out_and_from_the_table(hip, past):
     assert np.array_equal(res[0], res[1])
     f = res[0].view(np.float32)
     assert np.isfinite(f).any() and np.isnan(f[7]).all()
+
+
+@pytest.mark.parametrize("H_,past,T", [(2, 0, 2), (2, 5, 16), (4, 0, 17), (2, 96, 32), (6, 40, 33), (2, 0, 49)])
+def test_prompt_attention_leaves_packed_activations(hip, H_, past, T):
+    """The prompt's product hands its outputs to the next MatMul as packed activations: the bytes that packing its fp32 outputs gives, rows of zeros up to a whole group of
+    16 among them, at the edges of its 32-row tiles and of the groups."""
+    from tests.gpu_util import dev, dev_empty
+    hd, n = 128, past + T
+    d, n_ctx = H_ * hd, (n + 31) // 32 * 32
+    rng = np.random.default_rng(T)
+    q16, kc, vt = rng.standard_normal((H_, T, hd)).astype(np.float16), rng.standard_normal((n_ctx, d)).astype(np.float16), rng.standard_normal((d, n_ctx)).astype(np.float16)
+    vt[:hd // 4] = 0                                        # a block of zeros: scale 0
+    L = hip.load()
+    plain, packed, pack, luts = (getattr(L, s) for s in ("_Z21spy_exact_prompt_attnP12ihipStream_tPKvbPKtS4_PfPtS5_PKfiiilif", "_Z26spy_exact_prompt_attn_packP12ihipStream_tPKtS2_S2_PfPtPvPKfiiilif",
+                                                        "_Z14spy_xgemm_packP12ihipStream_tPKflllPv", "_Z14spy_exact_lutsPPKf"))
+    lut = C.c_void_p()
+    assert luts(C.byref(lut)) == 0
+    s_row, nbytes = (n + 127) // 128 * 128, (T + 15) // 16 * (d // 128) * (4096 + 512)
+    dq, dk, dv = dev(q16.view(np.uint16)), dev(kc.view(np.uint16)), dev(vt.view(np.uint16))
+    S, P, o, p0, p1 = dev_empty(H_ * T * s_row * 4, 0xEE), dev_empty(H_ * T * s_row * 2, 0xEE), dev_empty(T * d * 4, 0xEE), dev_empty(nbytes + 64, 0xEE), dev_empty(nbytes + 64, 0xEE)
+    i32, i64, vp, f32 = C.c_int, C.c_int64, C.c_void_p, C.c_float
+    tail = (i32(T), i32(H_), i32(past), i64(n_ctx), i32(n), f32(0.0883883461))
+    assert plain(None, vp(dq.ptr), C.c_bool(True), vp(dk.ptr), vp(dv.ptr), vp(S.ptr), vp(P.ptr), vp(o.ptr), lut, *tail) == 0
+    assert pack(None, vp(o.ptr), i64(4 * d), i64(T), i64(d), vp(p0.ptr)) == 0
+    assert packed(None, vp(dq.ptr), vp(dk.ptr), vp(dv.ptr), vp(S.ptr), vp(P.ptr), vp(p1.ptr), lut, *tail) == 0
+    hip.sync()
+    a, b = p0.download(np.uint32), p1.download(np.uint32)
+    assert np.array_equal(a, b)
+    assert (b[-16:] == 0xEEEEEEEE).all()

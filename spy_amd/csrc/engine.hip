@@ -370,8 +370,7 @@ int spy_matmul_own(void *stream, const spy_hip_tensor *w, const spy_hip_tensor *
 int spy_norm_mul_q8_launch(hipStream_t st, const float *x, int64_t x_stride, const float *w, float eps, void *y, int64_t nrow, int64_t K);   // prompt_fused.hip
 int spy_silu_mul_q8_launch(hipStream_t st, const float *gate, const float *up, void *y, int64_t nrow, int64_t F);                           // prompt_fused.hip
 int spy_rope_table_launch(hipStream_t st, float *table, int past, int T, int hd, float freq_base, float freq_scale, float mscale);       // prompt_fused.hip
-int spy_rope_store_launch(hipStream_t st, const float *q, const float *k, const float *table, uint16_t *q16, uint16_t *kc, int T, int H, int hd);
-int spy_vt_store_launch(hipStream_t st, const float *v, uint16_t *vc, int T, int d, int64_t n_ctx);
+int spy_qkv_store_launch(hipStream_t st, const float *q, const float *k, const float *v, const float *table, uint16_t *q16, uint16_t *kc, uint16_t *vc, int T, int H, int hd, int64_t n_ctx);
 int spy_prompt_attn_launch(hipStream_t st, const uint16_t *q16, const uint16_t *k_cache, const uint16_t *v_cache, float *out,
                            int T, int H, int hd, int past, int64_t n_ctx, float scale);                                       // prompt_attn.hip
 int spy_gemm_q8act_pair(hipStream_t st, int wtype, const void *w1, const void *w2, const void *xq, float *dst1, float *dst2,
@@ -417,7 +416,7 @@ static int ops_workspace(spy_hip_llama *m, hipStream_t st, size_t bytes) {
     return 0;
 }
 
-// A prompt pass in the host's order with what lies between two MatMuls in the kernels around them, 12 launches per layer instead of 42:
+// A prompt pass in the host's order with what lies between two MatMuls in the kernels around them, 11 launches per layer instead of 42:
 // norm and activation end in the next MatMul's packed activations (quantized once for wq | wk | wv and for gate | up, which are one launch
 // each where their types allow), Rope stores q as fp16 and k into its cache rows, the residual additions are the products' epilogues.  Each
 // step is the arithmetic of the operator it replaces, so the bits are those of forward_ops with the exact order on.
@@ -461,8 +460,7 @@ static int forward_exact(spy_hip_llama *m, hipStream_t st, const int32_t *tokens
         const int together = L.t_wv == L.t_wq ? 3 : 2;
         RC_TRY(spy_xgemm(st, L.t_wq, together, w3, d3, d, d, T, d, nullptr, pack));
         if (together == 2) RC_TRY(spy_xgemm(st, L.t_wv, 1, w3 + 2, d3 + 2, d, d, T, d, nullptr, pack));
-        RC_TRY(spy_rope_store_launch(st, q, k, m->rope_tab + (size_t)P * hd, q16, m->k_cache[il] + d * P, T, (int)H, (int)hd));
-        RC_TRY(spy_vt_store_launch(st, v, m->v_cache[il] + P, T, (int)d, C));
+        RC_TRY(spy_qkv_store_launch(st, q, k, v, m->rope_tab + (size_t)P * hd, q16, m->k_cache[il] + d * P, m->v_cache[il] + P, T, (int)H, (int)hd, C));
         RC_TRY(spy_exact_prompt_attn_pack(st, q16, m->k_cache[il], m->v_cache[il], (float *)(B + o_S), (uint16_t *)(B + o_P), pack, m->lut, T, (int)H, P, C, n_total, scale));
         RC_TRY(spy_xgemm(st, L.t_wo, 1, &L.wo, &t1, d, d, T, d, x, pack));                     // KQV_linear + Add
         RC_TRY(spy_xgemm_norm_pack(st, false, t1, L.ffn_norm, c.eps, T, d, pack));
@@ -592,8 +590,7 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
         }
         spy_hip_tensor t_qp;
         if (fuse_act) {           // Rope(q), Rope(k), the fp16 conversion of q and both cache writes in two kernels (prompt_fused.hip)
-            RC_TRY(spy_rope_store_launch(st, q, k, rope_tab, (uint16_t *)xn, (uint16_t *)m->k_cache[il] + d * P, T, (int)H, (int)hd));
-            RC_TRY(spy_vt_store_launch(st, v, (uint16_t *)m->v_cache[il] + P, T, (int)d, C));
+            RC_TRY(spy_qkv_store_launch(st, q, k, v, rope_tab, (uint16_t *)xn, (uint16_t *)m->k_cache[il] + d * P, (uint16_t *)m->v_cache[il] + P, T, (int)H, (int)hd, C));
             t_qp = T3s(SPY_HIP_F16, xn, hd, T, H, 2, 2 * hd, 2 * hd * T);
         } else {
             spy_hip_tensor t_q3 = T3s(SPY_HIP_F32, q, hd, H, T, 4, 4 * hd, 4 * d), t_k3 = T3s(SPY_HIP_F32, k, hd, H, T, 4, 4 * hd, 4 * d);

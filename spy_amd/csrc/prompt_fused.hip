@@ -98,35 +98,38 @@ __global__ __launch_bounds__(64) void rope_table_kernel(float2 *__restrict__ tab
     }
 }
 
-// grid (T, H); q, k: f32 [T][H * hd]; q16: fp16 [H][T][hd]; kc: K cache row of the pass's first token, fp16 [T][H * hd]
-__global__ __launch_bounds__(64) void rope_store_kernel(const float *__restrict__ q, const float *__restrict__ k, const float2 *__restrict__ table,
-                                                        uint16_t *__restrict__ q16, uint16_t *__restrict__ kc, int T, int H, int hd) {
-    const int t = blockIdx.x, h = blockIdx.y, npair = hd / 2;
-    const size_t row = ((size_t)t * H + h) * hd;
-    for (int p = threadIdx.x; p < npair; p += 64) {
-        const float2 cs = table[(size_t)t * npair + p];
-        const float2 a = *(const float2 *)(q + row + 2 * p), b = *(const float2 *)(k + row + 2 * p);
-        const float q0 = a.x * cs.x - a.y * cs.y, q1 = a.x * cs.y + a.y * cs.x;
-        const float k0 = b.x * cs.x - b.y * cs.y, k1 = b.x * cs.y + b.y * cs.x;
-        *(uint32_t *)(q16 + ((size_t)h * T + t) * hd + 2 * p) = (uint32_t)f2h(q0) | ((uint32_t)f2h(q1) << 16);
-        *(uint32_t *)(kc + row + 2 * p) = (uint32_t)f2h(k0) | ((uint32_t)f2h(k1) << 16);
-    }
-}
-
-// v: f32 [T][d] -> V^T cache: fp16 vc[col * n_ctx + t] for t < T (vc points at the pass's first position); 64 x 64 tiles through LDS, a thread's
-// sixteen elements all on their way at once (one after the other: 77 rows of 4096 8.3 -> 4.9 us, 1000 rows 11.4 -> 6.3, 2048 rows 14 -> 10, the time of a copy)
-__global__ __launch_bounds__(256) void vt_store_kernel(const float *__restrict__ v, uint16_t *__restrict__ vc, int T, int d, int64_t n_ctx) {
+// The first nv workgroups: v: f32 [T][d] -> V^T cache: fp16 vc[col * n_ctx + t] for t < T (vc points at the pass's first position); 64 x 64 tiles through LDS, a thread's
+// sixteen elements all on their way at once (one after the other: 77 rows of 4096 8.3 -> 4.9 us, 1000 rows 11.4 -> 6.3, 2048 rows 14 -> 10, the time of a copy).
+// Behind them, a wave per (token, head): q, k: f32 [T][H * hd]; q16: fp16 [H][T][hd]; kc: K cache row of the pass's first token, fp16 [T][H * hd].
+// One launch for both, us: 8 rows of 4096 4.8 + 4.6 -> 4.4, 77 5.2 + 4.8 -> 5.5, 512 5.2 + 5.9 -> 7.9, 1000 6.4 + 10.5 -> 14.6, 2048 10.9 + 17.0 -> 25.4.
+__global__ __launch_bounds__(256) void qkv_store_kernel(const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v, const float2 *__restrict__ table,
+                                                        uint16_t *__restrict__ q16, uint16_t *__restrict__ kc, uint16_t *__restrict__ vc, int T, int H, int hd, int64_t n_ctx, int nv) {
     __shared__ uint16_t tile[64][66];
-    const int t0 = blockIdx.x * 64, c0 = blockIdx.y * 64, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), d = H * hd;
+    if ((int)blockIdx.x >= nv) {
+        const int u = ((int)blockIdx.x - nv) * 4 + wave, h = u / T, t = u - h * T, npair = hd / 2;
+        if (h >= H) return;
+        const size_t row = ((size_t)t * H + h) * hd;
+        for (int p = lane; p < npair; p += 64) {
+            const float2 cs = table[(size_t)t * npair + p];
+            const float2 a = *(const float2 *)(q + row + 2 * p), b = *(const float2 *)(k + row + 2 * p);
+            const float q0 = a.x * cs.x - a.y * cs.y, q1 = a.x * cs.y + a.y * cs.x;
+            const float k0 = b.x * cs.x - b.y * cs.y, k1 = b.x * cs.y + b.y * cs.x;
+            *(uint32_t *)(q16 + ((size_t)h * T + t) * hd + 2 * p) = (uint32_t)f2h(q0) | ((uint32_t)f2h(q1) << 16);
+            *(uint32_t *)(kc + row + 2 * p) = (uint32_t)f2h(k0) | ((uint32_t)f2h(k1) << 16);
+        }
+        return;
+    }
+    const int nt = (T + 63) / 64, t0 = (int)blockIdx.x % nt * 64, c0 = (int)blockIdx.x / nt * 64;
     float x[16];
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = v[(size_t)min(t0 + wave + 4 * k, T - 1) * d + min(c0 + lane, d - 1)];
+    for (int i = 0; i < 16; i++) x[i] = v[(size_t)min(t0 + wave + 4 * i, T - 1) * d + min(c0 + lane, d - 1)];
 #pragma unroll
-    for (int k = 0; k < 16; k++) tile[wave + 4 * k][lane] = f2h(x[k]);
+    for (int i = 0; i < 16; i++) tile[wave + 4 * i][lane] = f2h(x[i]);
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++)
-        if (t0 + lane < T && c0 + wave + 4 * k < d) vc[(size_t)(c0 + wave + 4 * k) * n_ctx + t0 + lane] = tile[lane][wave + 4 * k];
+    for (int i = 0; i < 16; i++)
+        if (t0 + lane < T && c0 + wave + 4 * i < d) vc[(size_t)(c0 + wave + 4 * i) * n_ctx + t0 + lane] = tile[lane][wave + 4 * i];
 }
 
 int spy_rope_table_launch(hipStream_t st, float *table, int past, int T, int hd, float freq_base, float freq_scale, float mscale) {
@@ -136,15 +139,11 @@ int spy_rope_table_launch(hipStream_t st, float *table, int past, int T, int hd,
     return SPY_LAUNCH_RC();
 }
 
-int spy_rope_store_launch(hipStream_t st, const float *q, const float *k, const float *table, uint16_t *q16, uint16_t *kc, int T, int H, int hd) {
-    SPY_CHECK_ARG(q && k && table && q16 && kc && T > 0 && H > 0 && H < 65536 && hd > 0 && hd % 2 == 0);
+int spy_qkv_store_launch(hipStream_t st, const float *q, const float *k, const float *v, const float *table, uint16_t *q16, uint16_t *kc, uint16_t *vc, int T, int H, int hd, int64_t n_ctx) {
+    SPY_CHECK_ARG(q && k && v && table && q16 && kc && vc && T > 0 && H > 0 && H < 65536 && hd > 0 && hd % 2 == 0 && n_ctx >= T);
     SPY_CHECK_ARG(((uintptr_t)q % 8) == 0 && ((uintptr_t)k % 8) == 0 && ((uintptr_t)table % 8) == 0 && ((uintptr_t)q16 % 4) == 0 && ((uintptr_t)kc % 4) == 0);
-    rope_store_kernel<<<dim3((unsigned)T, (unsigned)H), dim3(64), 0, st>>>(q, k, (const float2 *)table, q16, kc, T, H, hd);
-    return SPY_LAUNCH_RC();
-}
-
-int spy_vt_store_launch(hipStream_t st, const float *v, uint16_t *vc, int T, int d, int64_t n_ctx) {
-    SPY_CHECK_ARG(v && vc && T > 0 && d > 0 && n_ctx >= T && (d + 63) / 64 < 65536);
-    vt_store_kernel<<<dim3((unsigned)((T + 63) / 64), (unsigned)((d + 63) / 64)), dim3(256), 0, st>>>(v, vc, T, d, n_ctx);
+    const int64_t nv = (int64_t)((T + 63) / 64) * (((int64_t)H * hd + 63) / 64), wgs = nv + ((int64_t)T * H + 3) / 4;
+    SPY_CHECK_ARG((int64_t)H * hd < (1ll << 31) && (int64_t)T * H < (1ll << 31) && wgs < (1ll << 31));
+    qkv_store_kernel<<<dim3((unsigned)wgs), dim3(256), 0, st>>>(q, k, v, (const float2 *)table, q16, kc, vc, T, H, hd, n_ctx, (int)nv);
     return SPY_LAUNCH_RC();
 }

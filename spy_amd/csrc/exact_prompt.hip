@@ -55,13 +55,14 @@ __device__ __forceinline__ void xp_reduce8(const xp_v16f &s, float (&t)[4]) {
 // One workgroup per (head, 64 query rows), a wave takes 16 of them: their q values as floats in registers, laid out as right operands.  A tile of
 // 64 key rows is brought into LDS by the whole workgroup.  Per 16 key rows and l = 0 .. 7 one chain of three matrix instructions (chunks of 32
 // elements while i + 32 < 128) gives accumulators l, 8 + l, 16 + l, 24 + l of the 16 x 16 scores; the vector units add them in the host's tree.  The
-// last 32 elements, added one by one, are a chain of 32 such instructions whose four blocks are the four groups of 16 key rows.
-// 2048 rows on 2048 positions, 32 heads: 1140 -> 597 us (the fmas on the vector units, two query rows per lane); 77 rows on 1000: 34.6 -> 20.4.  What bounds
+// last 32 elements, added one by one, are a chain of eight v_mfma_f32_16x16x4_f32, which do the fmas of their four elements one after the other, bit for bit: a lane's
+// eight elements of q stay in registers.  (As 32 of the former, whose four blocks were the four groups of 16 keys, they were widened for every tile, at 168 registers and three
+// workgroups on a compute unit: 2048 rows on 2048 positions, 32 heads, 645 us; three workgroups 601, four 588; 2048 rows alone 238 -> 218.)  What bounds
 // it: matrix and vector instructions of this kind never run at once (counter SQ_VALU_MFMA_COEXEC_CYCLES: 0), so the 31 additions of the tree and the
-// widening of the operands (210 us) come on top of the fmas (348).
+// widening of the keys come on top of the fmas (348 us).  A last tile of few rows with its keys dealt out over the waves: nothing (77 rows on 1000 16.4 us).
 #define XP_KSEG 512
 template <bool F16Q>       // q: f32 [T][H * 128] as Rope leaves it, or already rounded to fp16 and laid out [H][T][128]
-__global__ __launch_bounds__(256, 3) void xp_scores_kernel(const void *__restrict__ q, const uint16_t *__restrict__ kc, float *__restrict__ S,
+__global__ __launch_bounds__(256, 4) void xp_scores_kernel(const void *__restrict__ q, const uint16_t *__restrict__ kc, float *__restrict__ S,
                                                            int T, int H, int P, int64_t s_row, int kseg) {
     constexpr int QT = 64;
     __shared__ __align__(16) uint4 s_k[2][64][17];               // 64 key rows of 256 bytes, 16 bytes apart
@@ -76,15 +77,14 @@ __global__ __launch_bounds__(256, 3) void xp_scores_kernel(const void *__restric
     const int kv_end = min(P + min(t0 + QT - 1, T - 1) + 1, ((int)blockIdx.z + 1) * kseg);       // cached positions that some row of the tile may see, within this segment
     if ((int)blockIdx.z * kseg >= kv_end) return;
     const int tw = t0 + wave * 16, wave_end = tw < T ? P + min(tw + 15, T - 1) + 1 : 0;      // the wave's query rows, and the positions that some of them may see
-    float qm[3][8];                                              // elements 32 c + 8 g + l of query row j
-    uint4 qt[4];                                                 // elements 96 + 8 c + l, as fp16: widened for each tile, which costs less than the registers
+    float qm[3][8], qt[8];                                       // elements 32 c + 8 g + l and 96 + 4 l + g of query row j
     const int t = min(tw + j, T - 1);
     if constexpr (F16Q) {
         const uint4 *qp = (const uint4 *)((const uint16_t *)q + ((int64_t)h * T + t) * 128);
 #pragma unroll
         for (int c = 0; c < 3; c++) xp_widen(qp[4 * c + g], qm[c]);
 #pragma unroll
-        for (int c = 0; c < 4; c++) qt[c] = qp[12 + c];
+        for (int l = 0; l < 8; l++) qt[l] = h2f(((const uint16_t *)qp)[96 + 4 * l + g]);
     } else {
         const float *qp = (const float *)q + (int64_t)t * d + (int64_t)h * 128;
         auto halves = [&](int at) -> uint4 {
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(256, 3) void xp_scores_kernel(const void *__restric
 #pragma unroll
         for (int c = 0; c < 3; c++) xp_widen(halves(32 * c + 8 * g), qm[c]);
 #pragma unroll
-        for (int c = 0; c < 4; c++) qt[c] = halves(96 + 8 * c);
+        for (int l = 0; l < 8; l++) qt[l] = h2f(f2h(qp[96 + 4 * l + g]));
     }
     // staging: thread -> key row tid / 4 of the tile, 64 of its 256 bytes
     const int st_row = threadIdx.x >> 2, st_q = (threadIdx.x & 3) * 4;
@@ -114,19 +114,12 @@ __global__ __launch_bounds__(256, 3) void xp_scores_kernel(const void *__restric
         __syncthreads();
         if (kv0 + 64 < kv_end) fetch(kv0 + 64);
         if (kv0 >= wave_end) continue;                            // the tile lies behind the mask of the wave's query rows
-        xp_v16f tail = xp_zero();
+#pragma unroll 1
+        for (int kt = 0; kt < 4; kt++) {
+            if (kv0 + 16 * kt >= wave_end) break;
+            xp_v4f tail = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            float a[8], b[8];
-            xp_widen(s_k[buf][lane][12 + c], a);
-            asm("" : "+v"(qt[c].x), "+v"(qt[c].y), "+v"(qt[c].z), "+v"(qt[c].w));      // (or the compiler widens them before the loop and keeps the floats)
-            xp_widen(qt[c], b);
-#pragma unroll
-            for (int l = 0; l < 8; l++) tail = xp_mfma(a[l], b[l], tail);
-        }
-        auto keys16 = [&](auto kt_c) {
-            constexpr int kt = decltype(kt_c)::value;
-            if (kv0 + 16 * kt >= wave_end) return;
+            for (int l = 0; l < 8; l++) tail = __builtin_amdgcn_mfma_f32_16x16x4f32(h2f(((const uint16_t *)s_k[buf][16 * kt + j])[96 + 4 * l + g]), qt[l], tail, 0, 0, 0);
             float a[3][8];
 #pragma unroll
             for (int c = 0; c < 3; c++) xp_widen(s_k[buf][16 * kt + j][4 * c + g], a[c]);
@@ -153,14 +146,10 @@ __global__ __launch_bounds__(256, 3) void xp_scores_kernel(const void *__restric
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const float x = u[0][v] + u[1][v], y = u[2][v] + u[3][v];
-                o[v] = tail[4 * kt + v] + (x + y);
+                o[v] = tail[v] + (x + y);
             }
             if (tw + j < T) *(float4 *)(S + ((int64_t)h * T + t) * s_row + kv0 + 16 * kt + 4 * g) = make_float4(o[0], o[1], o[2], o[3]);
-        };
-        keys16(std::integral_constant<int, 0>{});
-        keys16(std::integral_constant<int, 1>{});
-        keys16(std::integral_constant<int, 2>{});
-        keys16(std::integral_constant<int, 3>{});
+        }
     }
 }
 
@@ -399,11 +388,11 @@ static int prompt_attn(hipStream_t st, const void *q, bool q_f16, const uint16_t
     if ((int64_t)P + T > 256 * XP_SM_R) return SPY_HIP_EUNSUPPORTED;      // the softmax kernel keeps a row in the registers of a wave
     if (((uintptr_t)q & 15) || ((uintptr_t)kc & 15) || ((uintptr_t)S & 15) || ((uintptr_t)P16 & 15) || ((uintptr_t)out & 15) || ((uintptr_t)pack & 15)) return SPY_HIP_EINVAL;
     const int64_t s_row = spy_exact_prompt_attn_row((int64_t)P + T);
-    // segments of the cached positions: 512 long where that fills the chip, down to one key tile for short passes (77 tokens on 1000 cached ones
-    // gave 96 workgroups: 114 us; one per 64 positions and 64 query rows 29)
+    // segments of the cached positions: 512 long where that gives every compute unit its four workgroups three times over, down to one key tile for short passes (512 rows
+    // with 1024 workgroups asked for 28.8 us, 2048 22.0, 3072 21.6, 4096 22.0; 1000 rows 75.8, 66.4, 62.0, 62.2; 77 rows on 1000 positions 16.4 with any)
     const int tiles = (T + 63) / 64;
     int kseg = XP_KSEG;
-    while (kseg > 64 && (int64_t)H * tiles * ((P + T + kseg - 1) / kseg) < 1024) kseg >>= 1;
+    while (kseg > 64 && (int64_t)H * tiles * ((P + T + kseg - 1) / kseg) < 3072) kseg >>= 1;
     const dim3 sgrid((unsigned)H, (unsigned)tiles, (unsigned)((P + T + kseg - 1) / kseg));
     if (q_f16) xp_scores_kernel<true><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);
     else xp_scores_kernel<false><<<sgrid, dim3(256), 0, st>>>(q, kc, S, T, H, P, s_row, kseg);

@@ -86,7 +86,7 @@ int spy_silu_mul_q8_launch(hipStream_t st, const float *gate, const float *up, v
 // sinf of theta * freq_scale, times the attention factor).  Per layer one kernel then rotates q and k
 // and stores them where the next operators read them: q as fp16 [head][token][hd] (the conversion the
 // score product applies to its right operand, mat.cpp:37) and k as fp16 into the K cache rows of the
-// pass (the Copy of view.cpp:83-227); a second kernel transposes v into the V^T cache.
+// pass (the Copy of view.cpp:83-227); the same launch transposes v into the V^T cache.
 __global__ __launch_bounds__(64) void rope_table_kernel(float2 *__restrict__ table, int past, int npair, float theta_scale, float freq_scale, float mscale) {
     const int t = blockIdx.x;
     const float p = (float)(past + t);

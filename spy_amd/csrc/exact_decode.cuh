@@ -302,8 +302,8 @@ static __device__ __forceinline__ float xg_hsum8(float acc) {
 // ---- the kernel --------------------------------------------------------------------------------------------------------
 // 1024 threads; wave w of the grid (gw) owns, per step, RPS rows:
 //   EPI_RESID / EPI_STORE : rows gw * RPS + j + k * NW * RPS                              (NSTEP steps)
-//   EPI_GATEUP            : RPS = 2: row i = gw + k * NW of W0 (gate) and of W1 (up)      (NSTEP steps)
-//   EPI_QKV               : step 0: rows 2 gw, 2 gw + 1 of [W0; W1] (a RoPE pair), step 1: row gw of W2
+//   EPI_GATEUP            : rows i = gw + k * NW of W0 (gate) and of W1 (up), RPS / 2 pairs a step      (NSTEP steps)
+//   EPI_QKV               : step 0: rows 2 gw, 2 gw + 1 of [W0; W1] (a RoPE pair), step 1 (K-quants: step 0): row gw of W2
 // A step's rows of all 16 waves form one batch: phase 1 (all waves) -> barrier -> phase 2 (the first lanes, one per
 // accumulator) -> barrier, per slab of 4096 elements of K; the accumulators stay in their lanes from slab to slab.
 template <int WT, int NITK, int RPS, int NSTEP, int EPI, int WTV = WT>
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
     }
     // Rows requested ahead of their use.  A wave waits in the issue stage while the memory queue is full, i.e. while the stream runs, and the barriers
     // of the norm wait for every wave: 2 rows of each of 16 waves (73 KB of Q4_0, 3.3 us of the stream) about cover the norm's sum.  qkv with 2 of 3
-    // rows 10.4 us (all 3: 11.0; 1: 11.8), gate|up Q4_0 with 3 of 6 14.5 us (2: 15.1; 4: 15.3), Q4_K 13.0 (14.1; 14.3), Q8_0, whose rows are twice as long, with 2 19.8 us (3: 20.9;
+    // rows 10.4 us (all 3: 11.0; 1: 11.8), gate|up Q4_0 with 3 of 6 14.5 us (2: 15.1; 4: 15.3), Q4_K (in three steps) 13.0 (14.1; 14.3), Q8_0, whose rows are twice as long, with 2 19.8 us (3: 20.9;
     // 1: 22.3).  gate|up asks for its first row (37 KB, which the queue takes at once) right behind the activations (Q4_0 14.9 us without, Q8_0 20.4); with less to
     // stream after the norm the other kernels lose by it (two rows ahead of it: 20 us and more).
     constexpr int DEPTH = EPI == EPI_GATEUP ? (WT == SPY_HIP_Q8_0 ? 2 : 3) : NROW < 2 ? NROW : 2, PRE = EPI == EPI_GATEUP ? 1 : 0;
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
     float2 cs = make_float2(0.0f, 0.0f);
     auto issue_first = [&]() {
         if constexpr (EPI == EPI_QKV)
-            cs = *(const float2 *)(a.rope_tab + (size_t)(pos - a.rope_row0) * a.hd + ((2 * ((int)blockIdx.x * XG_WAVES + tid / (2 * NCH) % XG_WAVES)) & (a.hd - 1)));      // heads are 128 wide
+            cs = *(const float2 *)(a.rope_tab + (size_t)(pos - a.rope_row0) * a.hd + ((2 * ((int)blockIdx.x * XG_WAVES + tid / ((NCH == 1 && NCHV == 1 ? 3 : 2) * NCH) % XG_WAVES)) & (a.hd - 1)));      // heads are 128 wide
         if constexpr (!NORM) __builtin_amdgcn_s_barrier();      // x of every wave ahead of every wave's rows in the compute unit's memory queue
 #pragma unroll
         for (int r = 0; r < NROW; r++) if (r < DEPTH && r >= PRE) {
@@ -395,7 +395,10 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
     if (a.q8_dump && blockIdx.x == 0) xg_dump_q8(s_q, s_meta, K, a.q8_dump);
     staged_act act; act.q = s_q; act.meta = s_meta;
 
-    constexpr int NSTEPS = EPI == EPI_QKV ? 2 : NSTEP;
+    // K-quant rows have one accumulator and small slots: all rows of a wave lie in LDS side by side and are walked together, once, instead of one walk (0.5 us) and two
+    // barriers per step.  In a pass gate|up Q4_K 12.99 -> 11.76 us, qkv Q4_K with Q6_K 11.07 -> 10.22; the head (8 rows) is the same either way and keeps its two steps.
+    constexpr bool ONE = EPI == EPI_QKV && NCH == 1 && NCHV == 1;
+    constexpr int NSTEPS = EPI == EPI_QKV ? (ONE ? 1 : 2) : NSTEP;
     static_assert(NITK == 1 || NROW == 1, "rows longer than one slab are walked one row per wave");
     act_frag<1> af, av;
     int n8[16];
@@ -405,9 +408,8 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
 #pragma unroll
     for (int step = 0; step < NSTEPS; step++) {
         const int r0 = EPI == EPI_QKV ? 2 * step : step * RPS;                  // first row of the step
-        const int rows = EPI == EPI_QKV ? 2 - step : RPS;
-        const bool vstep = EPI == EPI_QKV && step == 1;
-        const int nch = vstep ? NCHV : NCH;
+        const int rows = EPI == EPI_QKV ? (ONE ? 3 : 2 - step) : RPS;
+        const int nch = EPI == EPI_QKV && step == 1 ? NCHV : NCH;
         const int chains = XG_WAVES * rows * nch;
         float acc = 0.0f;
 #pragma unroll
@@ -429,14 +431,14 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
                     }
                 }
                 if (it + 1 < NITK) load_slab<WT, 64, NITK>(t[0], row_ptr(0), npair, lane, it + 1);
-                if constexpr (WTV != WT) { if (vstep && p < npair) load_act_frag<WTV, 1>(av, act, npair, p); }
+                if constexpr (WTV != WT) { if ((ONE || step == 1) && p < npair) load_act_frag<WTV, 1>(av, act, npair, p); }
 #pragma unroll
                 for (int j = 0; j < rows; j++) {
                     const int r = r0 + j;
                     if (it == 0 && r + DEPTH < NROW) issue(r + DEPTH);            // its ring slot held row r - 1, multiplied in the previous step
                     float *slot = s_part + (size_t)(wave * rows + j) * SLOTF;
                     if (p < npair) {
-                        if (vstep) { if constexpr (WTV != WT) xg_phase1<WTV>(tv.w[it], av, n8, p, lane, slot); else xg_phase1<WTV>(tv.w[it], af, n8, p, lane, slot); }
+                        if (EPI == EPI_QKV && r == 2) { if constexpr (WTV != WT) xg_phase1<WTV>(tv.w[it], av, n8, p, lane, slot); else xg_phase1<WTV>(tv.w[it], af, n8, p, lane, slot); }
                         else xg_phase1<WT>(t[r % RING].w[it], af, n8, p, lane, slot);
                     } else if (p < ((npair + 3) & ~3)) {                      // xg_chain's odd four blocks
                         for (int l = 0; l <= nch; l++) *(float2 *)(slot + l * (XG_NBS + 4) + 2 * lane) = make_float2(0.0f, 0.0f);
@@ -451,7 +453,7 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
                     acc = xg_chain(slot + l * (XG_NBS + 4), slot + nch * (XG_NBS + 4), nblk, acc);
                 }
                 XSTAMP(a.dbg, 20 + 3 * (step * NITK + it));
-                __syncthreads();
+                if (step + 1 < NSTEPS || it + 1 < NITK) __syncthreads();       // nothing is written behind the last walk
             }
         }
         // epilogue of the step: the lanes that walked accumulator 0 of a row hold its total after the tree
@@ -468,14 +470,14 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
             if (owner && u < a.M) a.out[u] = (EPI == EPI_RESID && a.resid) ? acc + (RS_AHEAD ? rs : a.resid[u]) : acc;       // Add(KQV_linear, x) / Add(ffn_out, ffn_input); no resid: the MatMul alone
         } else if constexpr (EPI == EPI_GATEUP) {
             const float u = __shfl_xor(acc, nch, SPY_WAVE);                    // the row after (up_i) sits nch lanes further
-            const int i = ogw + step * NW;
+            const int i = ogw + (step * (RPS / 2) + (oj >> 1)) * NW;
             if constexpr (LATE) {
                 up[step] = u;
-                if (owner && oj == 0 && i < a.M) sl[step] = a.lut[65536 + f2h(acc)];
-            } else if (owner && oj == 0 && i < a.M) a.out[i] = u * a.lut[65536 + f2h(acc)];       // Mul(ffn_up, Silu(ffn_gate)) (ffn.cpp:24-35, non-linear.cpp:11-14)
+                if (owner && (oj & 1) == 0 && i < a.M) sl[step] = a.lut[65536 + f2h(acc)];
+            } else if (owner && (oj & 1) == 0 && i < a.M) a.out[i] = u * a.lut[65536 + f2h(acc)];       // Mul(ffn_up, Silu(ffn_gate)) (ffn.cpp:24-35, non-linear.cpp:11-14)
         } else {
             if (step == 0) {
-                const float x1 = __shfl_xor(acc, nch, SPY_WAVE);
+                const float x1 = ONE ? __shfl_down(acc, 1, SPY_WAVE) : __shfl_xor(acc, nch, SPY_WAVE);      // (ONE: 48 lanes of one wave)
                 if (owner && oj == 0 && ogw < a.d) {
                     const float c = cs.x, sn = cs.y;
                     // (x0, x1) -> (x0*c - x1*s, x0*s + x1*c), every product rounded (non-linear.cpp:349-364)
@@ -484,16 +486,17 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
                     if (2 * ogw < a.d) ((uint32_t *)a.q16)[ogw] = pr;                                  // attn_score rounds Q to fp16 (mat.cpp:37)
                     else ((uint32_t *)(a.kc + (size_t)pos * a.d))[ogw - a.d / 2] = pr;                 // KCache_cpy: [token][head][hd]
                 }
-            } else {
+            }
+            if (ONE ? oj == 2 : step == 1) {
                 if (owner && ogw < a.d) a.vc[(size_t)ogw * a.n_ctx + pos] = f2h(acc);                 // VCache_cpy: [d][C] column pos
             }
         }
     }
     if constexpr (LATE) {
-        const bool owner = tid < XG_WAVES * 2 * NCH && tid % (2 * NCH) == 0;
+        const bool owner = tid < XG_WAVES * RPS * NCH && tid % (2 * NCH) == 0;
 #pragma unroll
         for (int step = 0; step < NSTEP; step++) {
-            const int i = (int)blockIdx.x * XG_WAVES + tid / (2 * NCH) + step * NW;
+            const int i = (int)blockIdx.x * XG_WAVES + tid / (RPS * NCH) + (step * (RPS / 2) + tid / (2 * NCH) % (RPS / 2)) * NW;
             if (owner && i < a.M) a.out[i] = up[step] * sl[step];
         }
     }

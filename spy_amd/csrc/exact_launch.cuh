@@ -10,24 +10,24 @@
 template <int WT, int NITK, int RPS, int NSTEP, int EPI, int WTV = WT>
 static int launch_xg(spy_hip_llama *m, hipStream_t st, const xg_args &a, int units) {
     constexpr int NCH = xg_traits<WT>::NCH, NCHV = xg_traits<WTV>::NCH;
-    constexpr int rows_max = EPI == EPI_QKV ? 2 : RPS;
+    constexpr int rows_max = EPI == EPI_QKV ? (NCH == 1 && NCHV == 1 ? 3 : 2) : RPS;
     const size_t lds = ((staged_bytes(a.K) + 15) & ~(size_t)15) + (size_t)XG_WAVES * rows_max * xg_slot_floats(NCH > NCHV ? NCH : NCHV) * 4 + XG_LDS_PAD;
     if (lds > 160 * 1024) return SPY_HIP_EUNSUPPORTED;
     auto kern = xgemv_kernel<WT, NITK, RPS, NSTEP, EPI, WTV>;
     RC_TRY(spy_ensure_lds(m, (const void *)kern, lds));
     if (m->dry) return 0;
-    const int per_wg = XG_WAVES * (EPI == EPI_QKV ? 1 : (EPI == EPI_GATEUP ? NSTEP : RPS * NSTEP));     // units (QKV: waves, GATEUP: pairs, else rows) per workgroup
+    const int per_wg = XG_WAVES * (EPI == EPI_QKV ? 1 : (EPI == EPI_GATEUP ? RPS / 2 * NSTEP : RPS * NSTEP));     // units (QKV: waves, GATEUP: pairs, else rows) per workgroup
     kern<<<dim3((unsigned)((units + per_wg - 1) / per_wg)), dim3(XG_THREADS), lds, st>>>(XG_ARGS(a));
     return SPY_LAUNCH_RC();
 }
 
 // rows per wave of the output head and pairs per wave of gate|up, as wave_rows in decode_launch.cuh
-// Q4_0 / Q8_0: 2 rows per wave and step (32 row slots of 4.6 KB fill LDS); K-quant rows have one accumulator and small slots: 4
+// Q4_0 / Q8_0: 2 rows per wave and step (32 row slots of 4.6 KB fill LDS); K-quant rows have one accumulator and small slots: head 4, gate|up all 6
 template <int WT> struct xg_rows {
     static constexpr bool KQ = WT == SPY_HIP_Q4_K || WT == SPY_HIP_Q6_K;
     static constexpr int HEAD_RPS = KQ ? 4 : 2;
-    static constexpr int HEAD_STEPS = WT == SPY_HIP_Q4_0 ? 4 : 2;                               // 8 rows per wave (Q8_0: 4: its rows are twice as wide)
-    static constexpr int GATEUP_STEPS = 3;
+    static constexpr int HEAD_STEPS = KQ ? 2 : WT == SPY_HIP_Q4_0 ? 4 : 2;                               // 8 rows per wave (Q8_0: 4: its rows are twice as wide)
+    static constexpr int GATEUP_RPS = KQ ? 6 : 2, GATEUP_STEPS = KQ ? 1 : 3;
 };
 
 template <int WT>
@@ -115,7 +115,7 @@ static int enqueue_exact(spy_hip_llama *m, hipStream_t st, int which, int il) {
         return xg_resid<WT>(m, st, a);
     case K_GATEUP:
         a.W0 = (const uint8_t *)L.w_gate; a.W1 = (const uint8_t *)L.w_up; a.M = F; a.K = d; a.x_in = m->x1; a.normw = L.ffn_norm; a.out = m->hbuf;
-        return launch_xg<WT, 1, 2, xg_rows<WT>::GATEUP_STEPS, EPI_GATEUP>(m, st, a, F);
+        return launch_xg<WT, 1, xg_rows<WT>::GATEUP_RPS, xg_rows<WT>::GATEUP_STEPS, EPI_GATEUP>(m, st, a, F);
     case K_DOWN:
         a.W0 = (const uint8_t *)L.w_down; a.M = d; a.K = F; a.x_in = m->hbuf; a.resid = m->x1; a.out = m->x;
         return xg_resid<WT>(m, st, a);

@@ -131,6 +131,26 @@ def test_ffn_gate_up_silu(hip, oracle, order, wtype):
     _check(do.download(np.float32), want, "up * silu(gate), type %d" % wtype, order)
 
 
+@pytest.mark.parametrize("wtype", [O.Q4_K, O.Q6_K, O.Q4_0])
+@pytest.mark.parametrize("F,K", [(256, 256), (512, 1280), (768, 4096), (1280, 768)])
+def test_gate_up_rows_over_the_waves(hip, oracle, wtype, F, K):
+    """three pairs of a wave, 16 pairs per workgroup apart: all three there in every wave (768), the third missing in some; rows of few and of all lanes"""
+    from tests.gpu_util import dev, dev_empty, call
+    rng = np.random.default_rng(wtype * 5 + F + K)
+    wg, wu = (O.quantize(oracle, (rng.standard_normal((F, K)) * 0.05).astype(np.float32), wtype) for _ in range(2))
+    x = (rng.standard_normal(K) * 2.0).astype(np.float32)
+    nw = (1.0 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    xn = _norm_mul(oracle, x, nw)
+    g, u = (O.matmul(oracle, w, wtype, F, K, xn[None, :], nthread=8)[0] for w in (wg, wu))
+    sg = np.zeros_like(g)
+    assert oracle.spy_o_silu(B(O.tensor(g, O.F32, [F, 1])), B(O.tensor(sg, O.F32, [F, 1]))) == 0
+    dg, du, dx, dn, do = dev(wg), dev(wu), dev(x), dev(nw), dev_empty(F * 4 + 64, 0xEE)
+    call(hip.load().spy_hip_ffn_gate_up_silu, None, 1, wtype, dg.ptr, du.ptr, dx.ptr, dn.ptr, EPS, do.ptr, F, K, None)
+    got = do.download(np.float32)
+    _check(got[:F], u * sg, "up * silu(gate), type %d, %d rows" % (wtype, F), 1)
+    assert (got[F:].view(np.uint32) == 0xEEEEEEEE).all()
+
+
 def _rope_table(oracle, pos, hd, n_ctx):
     """cos, sin per pair of position pos, through the oracle's Rope on unit vectors (1, 0): the host libm's values"""
     unit = np.zeros(hd, np.float32); unit[0::2] = 1.0
@@ -142,7 +162,7 @@ def _rope_table(oracle, pos, hd, n_ctx):
 
 
 @pytest.mark.parametrize("order", [1, 0])
-@pytest.mark.parametrize("wtype,wtype_v,pos", [(O.Q4_0, 0, 0), (O.Q4_0, 0, 4100), (O.Q8_0, 0, 517), (O.Q4_K, O.Q6_K, 33), (O.Q6_K, 0, 1000)])
+@pytest.mark.parametrize("wtype,wtype_v,pos", [(O.Q4_0, 0, 0), (O.Q4_0, 0, 4100), (O.Q8_0, 0, 517), (O.Q4_K, O.Q6_K, 33), (O.Q4_K, 0, 66), (O.Q6_K, 0, 1000)])
 def test_rope_kvwrite(hip, oracle, order, wtype, wtype_v, pos):
     """attn_norm, Q/K/V_project, Rope, fp16 Q, KV-cache copies of one token at d = 4096, 32 heads"""
     from tests.gpu_util import dev, dev_empty, call

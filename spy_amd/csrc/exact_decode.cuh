@@ -29,6 +29,9 @@
 template <int WT> struct xg_traits { static constexpr int NCH = (WT == SPY_HIP_Q4_0 || WT == SPY_HIP_Q8_0) ? 8 : 1; };
 // floats of LDS per row slot: NCH rows of partials (+4: bank skew between the rows) and the row of scale products (+4: skew between slots)
 static __host__ __device__ constexpr int xg_slot_floats(int nch) { return nch * (XG_NBS + 4) + XG_NBS + 4; }
+// K-quant rows of several slabs: slots of their own for every slab, so that the waves that do not walk go on to the next one (11008 columns Q6_K 11.17 -> 10.48 us in a pass);
+// two slots of eight accumulators per wave do not fit next to 11008 staged elements
+static __host__ __device__ constexpr bool xg_slabs(int nch, int nitk) { return nch == 1 && nitk > 1; }
 
 #define XG_LDS_PAD 64                       // what xg_chain reads past the last row
 
@@ -305,7 +308,7 @@ static __device__ __forceinline__ float xg_hsum8(float acc) {
 //   EPI_GATEUP            : rows i = gw + k * NW of W0 (gate) and of W1 (up), RPS / 2 pairs a step      (NSTEP steps)
 //   EPI_QKV               : step 0: rows 2 gw, 2 gw + 1 of [W0; W1] (a RoPE pair), step 1 (K-quants: step 0): row gw of W2
 // A step's rows of all 16 waves form one batch: phase 1 (all waves) -> barrier -> phase 2 (the first lanes, one per
-// accumulator) -> barrier, per slab of 4096 elements of K; the accumulators stay in their lanes from slab to slab.
+// accumulator) -> barrier (none where every slab has slots of its own), per slab of 4096 elements of K; the accumulators stay in their lanes from slab to slab.
 template <int WT, int NITK, int RPS, int NSTEP, int EPI, int WTV = WT>
 __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, const float *normw, const uint8_t *W0, const uint8_t *W1, const uint8_t *W2, const dev_state *st, int K_, int M,
                                                            xg_args a) {
@@ -375,7 +378,7 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
 #pragma unroll
         for (int r = 0; r < NROW; r++) if (r < DEPTH && r >= PRE) {
             // a row of several slabs: the first one ahead of the quantization, whose barrier waits for the issue, the next ones a slab ahead of their use
-            // (11008 columns: Q4_0 11.8 -> 10.2 us, Q6_K 14.0 -> 11.9; two slabs ahead 10.9 and 13.0)
+            // (11008 columns: Q4_0 11.8 -> 10.2 us, Q6_K 14.0 -> 11.9; two slabs ahead 10.9 and 13.0; with slots per slab Q6_K 10.48, two ahead 12.1, all 13.1)
             if constexpr (NITK > 1) load_slab<WT, 64, NITK>(t[0], row_ptr(0), npair, lane, 0);
             else issue(r);
         }
@@ -399,6 +402,7 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
     // barriers per step.  In a pass gate|up Q4_K 12.99 -> 11.76 us, qkv Q4_K with Q6_K 11.07 -> 10.22; the head (8 rows) is the same either way and keeps its two steps.
     constexpr bool ONE = EPI == EPI_QKV && NCH == 1 && NCHV == 1;
     constexpr int NSTEPS = EPI == EPI_QKV ? (ONE ? 1 : 2) : NSTEP;
+    constexpr bool SLABS = xg_slabs(NCH, NITK);
     static_assert(NITK == 1 || NROW == 1, "rows longer than one slab are walked one row per wave");
     act_frag<1> af, av;
     int n8[16];
@@ -436,7 +440,7 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
                 for (int j = 0; j < rows; j++) {
                     const int r = r0 + j;
                     if (it == 0 && r + DEPTH < NROW) issue(r + DEPTH);            // its ring slot held row r - 1, multiplied in the previous step
-                    float *slot = s_part + (size_t)(wave * rows + j) * SLOTF;
+                    float *slot = s_part + (size_t)((SLABS ? it * XG_WAVES : 0) + wave * rows + j) * SLOTF;
                     if (p < npair) {
                         if (EPI == EPI_QKV && r == 2) { if constexpr (WTV != WT) xg_phase1<WTV>(tv.w[it], av, n8, p, lane, slot); else xg_phase1<WTV>(tv.w[it], af, n8, p, lane, slot); }
                         else xg_phase1<WT>(t[r % RING].w[it], af, n8, p, lane, slot);
@@ -449,11 +453,11 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
                 XSTAMP(a.dbg, 19 + 3 * (step * NITK + it));
                 if (tid < chains) {
                     const int slot_i = tid / nch, l = tid % nch;
-                    const float *slot = s_part + (size_t)slot_i * SLOTF;
+                    const float *slot = s_part + (size_t)((SLABS ? it * XG_WAVES : 0) + slot_i) * SLOTF;
                     acc = xg_chain(slot + l * (XG_NBS + 4), slot + nch * (XG_NBS + 4), nblk, acc);
                 }
                 XSTAMP(a.dbg, 20 + 3 * (step * NITK + it));
-                if (step + 1 < NSTEPS || it + 1 < NITK) __syncthreads();       // nothing is written behind the last walk
+                if (step + 1 < NSTEPS || (!SLABS && it + 1 < NITK)) __syncthreads();       // nothing is written behind the last walk
             }
         }
         // epilogue of the step: the lanes that walked accumulator 0 of a row hold its total after the tree

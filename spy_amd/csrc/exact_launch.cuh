@@ -11,7 +11,7 @@ template <int WT, int NITK, int RPS, int NSTEP, int EPI, int WTV = WT>
 static int launch_xg(spy_hip_llama *m, hipStream_t st, const xg_args &a, int units) {
     constexpr int NCH = xg_traits<WT>::NCH, NCHV = xg_traits<WTV>::NCH;
     constexpr int rows_max = EPI == EPI_QKV ? (NCH == 1 && NCHV == 1 ? 3 : 2) : RPS;
-    const size_t lds = ((staged_bytes(a.K) + 15) & ~(size_t)15) + (size_t)XG_WAVES * rows_max * xg_slot_floats(NCH > NCHV ? NCH : NCHV) * 4 + XG_LDS_PAD;
+    const size_t lds = ((staged_bytes(a.K) + 15) & ~(size_t)15) + (size_t)XG_WAVES * rows_max * (xg_slabs(NCH, NITK) ? NITK : 1) * xg_slot_floats(NCH > NCHV ? NCH : NCHV) * 4 + XG_LDS_PAD;
     if (lds > 160 * 1024) return SPY_HIP_EUNSUPPORTED;
     auto kern = xgemv_kernel<WT, NITK, RPS, NSTEP, EPI, WTV>;
     RC_TRY(spy_ensure_lds(m, (const void *)kern, lds));
@@ -47,7 +47,7 @@ static int xg_resid(spy_hip_llama *m, hipStream_t st, const xg_args &a) {
 template <int WT, int NITK>
 static int launch_xg_plain(hipStream_t st, const xg_args &a) {
     constexpr int NCH = xg_traits<WT>::NCH;
-    const size_t lds = ((staged_bytes(a.K) + 15) & ~(size_t)15) + (size_t)XG_WAVES * xg_slot_floats(NCH) * 4 + XG_LDS_PAD;
+    const size_t lds = ((staged_bytes(a.K) + 15) & ~(size_t)15) + (size_t)XG_WAVES * (xg_slabs(NCH, NITK) ? NITK : 1) * xg_slot_floats(NCH) * 4 + XG_LDS_PAD;
     if (lds > 160 * 1024) return SPY_HIP_EUNSUPPORTED;
     auto kern = xgemv_kernel<WT, NITK, 1, 1, EPI_RESID, WT>;
     RC_TRY(spy_raise_lds_limit((const void *)kern, lds));
@@ -59,7 +59,7 @@ static int launch_xg_plain(hipStream_t st, const xg_args &a) {
 template <int WT, int NITK>
 static int xg_plain_prepare_one() {
     constexpr int NCH = xg_traits<WT>::NCH;
-    const size_t lds = ((staged_bytes(4096 * NITK) + 15) & ~(size_t)15) + (size_t)XG_WAVES * xg_slot_floats(NCH) * 4 + XG_LDS_PAD;
+    const size_t lds = ((staged_bytes(4096 * NITK) + 15) & ~(size_t)15) + (size_t)XG_WAVES * (xg_slabs(NCH, NITK) ? NITK : 1) * xg_slot_floats(NCH) * 4 + XG_LDS_PAD;
     return lds > 160 * 1024 ? 0 : spy_raise_lds_limit((const void *)xgemv_kernel<WT, NITK, 1, 1, EPI_RESID, WT>, lds);
 }
 template <int WT>

@@ -179,6 +179,25 @@ def test_k_quant_tiles_with_scales_of_any_size(hip, oracle, wtype, M, K, T):
     _same_bits(dd.download(np.float32).reshape(T, M), want, "matmul type %d %dx%d T %d, scales of any size" % (wtype, M, K, T))
 
 
+@pytest.mark.parametrize("wtype", [O.Q4_K, O.Q6_K])
+@pytest.mark.parametrize("K", [4352, 7936, 8448, 12288])
+def test_single_row_matmul_of_several_slabs(hip, oracle, wtype, K):
+    """K-quant rows of two and three slabs, each in slots of its own: a last slab of one super-block, of nearly all and of all lanes"""
+    from tests.gpu_util import dev, dev_empty, call
+    M = 53
+    rng = np.random.default_rng(K + wtype)
+    w = O.quantize(oracle, (rng.standard_normal((M, K)) * 0.02).astype(np.float32), wtype)
+    x = (rng.standard_normal((1, K)) * 3.0).astype(np.float32)
+    want = O.matmul(oracle, w, wtype, M, K, x, nthread=8)[0]
+    dw, dx, do = dev(w), dev(x), dev_empty(M * 4, 0xEE)
+    L = hip.load()
+    tw, tx, to = hip.tensor(dw.ptr, wtype, [K, M]), hip.tensor(dx.ptr, O.F32, [K, 1]), hip.tensor(do.ptr, O.F32, [M, 1])
+    need = L.spy_hip_op_matmul_scratch_size(B(tw), B(tx))
+    sc = dev_empty(max(need, 1), 0xEE)
+    call(L.spy_hip_op_matmul, None, B(tw), B(tx), B(to), sc.ptr, need)
+    assert np.array_equal(do.download(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0, O.Q4_K, O.Q6_K])
 @pytest.mark.parametrize("M,K,T", [(96, 4096, 16), (200, 512, 70), (64, 128, 64), (64, 256, 64), (132, 11008, 33), (4096, 4096, 130)])
 def test_tiled_matmul_bits(hip, oracle, wtype, M, K, T, monkeypatch):

@@ -353,8 +353,8 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
     }
     // Rows requested ahead of their use.  A wave waits in the issue stage while the memory queue is full, i.e. while the stream runs, and the barriers
     // of the norm wait for every wave: 2 rows of each of 16 waves (73 KB of Q4_0, 3.3 us of the stream) about cover the norm's sum.  qkv with 2 of 3
-    // rows 10.4 us (all 3: 11.0; 1: 11.8), gate|up Q4_0 with 3 of 6 14.5 us (2: 15.1; 4: 15.3), Q4_K (in three steps) 13.0 (14.1; 14.3), Q8_0, whose rows are twice as long, with 2 19.8 us (3: 20.9;
-    // 1: 22.3).  gate|up asks for its first row (37 KB, which the queue takes at once) right behind the activations (Q4_0 14.9 us without, Q8_0 20.4); with less to
+    // rows 10.4 us (all 3: 11.0; 1: 11.8), gate|up Q4_0 with 3 of 6 14.5 us (2: 15.1; 4: 15.3), Q4_K 11.8 (12.6; 12.35), Q8_0, whose rows are twice as long, with 2 19.8 us (3: 20.9;
+    // 1: 22.3).  gate|up asks for its first row (37 KB, which the queue takes at once) right behind the activations (Q4_0 14.9 us without, Q8_0 20.4; two rows ahead of it: Q4_K 13.05); with less to
     // stream after the norm the other kernels lose by it (two rows ahead of it: 20 us and more).
     constexpr int DEPTH = EPI == EPI_GATEUP ? (WT == SPY_HIP_Q8_0 ? 2 : 3) : NROW < 2 ? NROW : 2, PRE = EPI == EPI_GATEUP ? 1 : 0;
     constexpr int RING = NROW < DEPTH + 1 ? NROW : DEPTH + 1;

@@ -174,7 +174,7 @@ def main():
         count = {k: (1 if k == "head" else cfg.n_layer) for k in per_kernel}
         if order == 1:
             names = {"qkv": "xgemv_kernel<%s, qkv> (RMSNorm in std::reduce order, Q8_0, wq|wk|wv as 8-accumulator walks, RoPE, cache write)" % tn[tt("attn_q")],
-                     "scores": "xattn_scores_kernel (Dot<FP16,FP16> order, one thread per key)", "pv": "xattn_pv_kernel (softmax with std::reduce sum, P.V^T in Dot<FP16,FP16> order)",
+                     "scores": "xattn_scores_kernel (Dot<FP16,FP16> order, four lanes per key)", "pv": "xattn_pv_kernel (softmax with std::reduce sum, P.V^T in Dot<FP16,FP16> order)",
                      "wo": "xgemv_kernel<%s, wo + residual>" % tn[tt("attn_output")], "gate_up": "xgemv_kernel<%s, gate|up + SiLU table>" % tn[tt("ffn_gate")],
                      "down": "xgemv_kernel<%s, down + residual>" % tn[tt("ffn_down")], "head": "xgemv_kernel<%s, output head>" % tn[cfg.t_out]}
         else:

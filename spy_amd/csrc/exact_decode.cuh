@@ -7,7 +7,7 @@
 //   * fp16 dots (vec_dot.h:117-146): 4 x 8 accumulators over chunks of 32 while i + 32 < n, the reduction tree, then
 //     the scalar tail;
 //   * NormRMS and Softmax sums (non-linear.cpp:129-223): libstdc++'s groups of four added to ONE running sum;
-//   * exp and silu from the two fp16-indexed tables filled by the host's libm, the RoPE angles from a host table.
+//   * exp and silu as the two fp16-indexed tables filled by the host's libm have them (exp in the attention worked out: exact_exp.cuh), the RoPE angles from a host table.
 //
 // How a serial sum is made fast.  The integer block dots stay where they are (64 lanes x v_dot4, one block pair per
 // lane, weights read once, coalesced).  What changes is what follows them: instead of scaling and adding its blocks in
@@ -15,7 +15,7 @@
 // LDS, transposed, and after a workgroup barrier ONE lane per accumulator walks its row of LDS block after block:
 // 8 lanes per output element, 64 lanes = 8 output elements per wave, fed by 128-bit LDS reads.  The walk is a chain of
 // dependent fmas (about 4 ns each on this part, whatever else the compute unit does), so a 4096-wide row costs about
-// 0.6 us of latency per batch of rows; batches are as large as LDS allows (32 rows of 128 blocks).
+// 0.6 us of latency per batch of rows; batches are as large as LDS allows (32 rows of 128 blocks; of K-quants all rows).
 #pragma once
 
 #include "decode_kernels.cuh"

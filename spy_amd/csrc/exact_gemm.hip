@@ -71,7 +71,10 @@ struct xt_args {
     int ncg_all;                                   // groups of the whole call of which this is a piece
     const uint8_t *xq, *xd;
 };
-// What the first requests of a launch need, ahead of the rest: the first 14 dwords of a kernel's arguments come in registers (Makefile).
+// What the first requests of a launch need, ahead of the rest: the first 14 dwords of a kernel's arguments come in registers (Makefile).  K-quant tiles 1 % faster by it
+// (4096 x 11008 x 100 Q4_K 71.3 -> 69.8 us, 8192 x 4096 x 17 25.5 -> 25.1).  Not xks_kernel and xn_kernel, the short ones: at two workgroups per compute unit
+// 4096 x 4096 x 17 Q4_K 15.5 us without, 17.1 with, 8192 x 4096 x 8 16.7 and 17.9, 5120 x 5120 x 8 17.5 and 18.4; 4096 x 11008 x 17 Q6_K 48.9 and 50.2; xn_kernel 4096 x 11008 x 8 Q4_0
+// 23.3 and 24.0; 1024 x 1024 of any type 0.1 more of 7.
 #define XT_PARAMS const uint8_t *w0_, const uint8_t *w1_, const uint8_t *w2_, const uint8_t *xq_, const uint8_t *xd_, int64_t w_row_, int tiles_, int nst_, xt_args a
 #define XT_HOT const xt_hot hot = {w0_, w1_, w2_, xq_, xd_, w_row_, tiles_, nst_}
 #define XT_ARGS(a) (a).w[0], (a).w[1], (a).w[2], (a).xq, (a).xd, (a).w_row, (a).tiles, (a).nst, (a)
@@ -287,23 +290,22 @@ __global__ __launch_bounds__(256, 3) void xt_mixed_kernel(XT_PARAMS) {
 // Against one stage of four blocks per barrier, weights from memory, in us, packing of the activations (4 us) included: 8 rows, Q4_0 4096 x 4096 14.4 -> 12.1,
 // 4096 x 11008 30.6 -> 23.6, 12288 x 4096 21.0 -> 17.7, Q8_0 14.4 -> 12.5, 30.3 -> 24.3, 22.5 -> 20.8; 48 rows, Q4_0 4096 x 4096 21.2 -> 17.8, 4096 x 11008 47.5 -> 37.3.
 template <int WT, int NS>
-__global__ __launch_bounds__(256, 2) void xn_kernel(XT_PARAMS) {
-    XT_HOT;
+__global__ __launch_bounds__(256, 2) void xn_kernel(xt_args a) {
     constexpr int NT = 256, ROWS = 16, CU = xt_w<WT>::CU, UW = ROWS * CU, NI = (UW + NT - 1) / NT, NXI = 2;
     constexpr int XB = 2 * (XT_XB + 256), WB = (UW + 63) / 64 * 1024, NREQ = NXI + 1 + NI;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = wave, q = lane >> 4, r = lane & 15;
-    const int mat = hot.mat((int)blockIdx.x), m0 = ((int)blockIdx.x - mat * hot.tiles) * ROWS, cg = (int)blockIdx.y;
-    const int nch = hot.nst / 2, M = a.M;
+    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * ROWS, cg = (int)blockIdx.y;
+    const int nch = a.nst / 2, M = a.M;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)smem;
     // requests as in xt_tile: uniform bases that advance by a chunk, per-lane offsets that stay; waves 0 and 1 bring the scales of the chunk's stages (the others repeat them)
-    const uint8_t *bx = hot.xq + (int64_t)cg * hot.nst * XT_XB + wave * 1024, *bd = hot.xd + ((int64_t)cg * hot.nst + min(wave, 1)) * XT_XD, *bw = hot.w(mat) + (int64_t)m0 * hot.w_row;
+    const uint8_t *bx = a.xq + (int64_t)cg * a.nst * XT_XB + wave * 1024, *bd = a.xd + ((int64_t)cg * a.nst + min(wave, 1)) * XT_XD, *bw = a.w[mat] + (int64_t)m0 * a.w_row;
     uint32_t ow[NI];
 #pragma unroll
     for (int i = 0; i < NI; i++) {
         const int u = min(tid + i * NT, UW - 1);
-        ow[i] = (uint32_t)(min(m0 + u / CU, M - 1) - m0) * (uint32_t)hot.w_row + (u % CU) * 16;
+        ow[i] = (uint32_t)(min(m0 + u / CU, M - 1) - m0) * (uint32_t)a.w_row + (u % CU) * 16;
     }
     const bool spare = wave * 64 + (NI - 1) * NT >= UW;
     const uint32_t lds_spare = __builtin_amdgcn_readfirstlane(lds0 + NS * (XB + WB));
@@ -435,7 +437,7 @@ int xn_launch(hipStream_t st, xt_args a, int nmat) {
     constexpr size_t lds = NS * (2 * (XT_XB + 256) + (16 * xt_w<WT>::CU + 63) / 64 * 1024) + 1024;
     static_assert(lds <= 64 * 1024 && lds >= 3 * 8 * 256, "no raised LDS limit; room for the exchange of the accumulators");
     a.tiles = (a.M + 15) / 16;
-    xn_kernel<WT, NS><<<dim3((unsigned)(a.tiles * nmat), (unsigned)a.ncg), dim3(256), lds, st>>>(XT_ARGS(a));
+    xn_kernel<WT, NS><<<dim3((unsigned)(a.tiles * nmat), (unsigned)a.ncg), dim3(256), lds, st>>>(a);
     return SPY_LAUNCH_RC();
 }
 
@@ -1039,16 +1041,15 @@ __global__ __launch_bounds__(64 * RG * KS, OCC) void xk_kernel(XT_PARAMS) {
 // the fma per sub-block; the terms are independent, so each round the waves leave the terms of four super-blocks in LDS and then every wave
 // walks a quarter of the outputs through their 32 fmas.  (16 rows of a 4096 x 4096 Q4_K matrix: 20 us as a chain in one wave, 10 here.)
 template <int WT>
-__global__ __launch_bounds__(256, 3) void xks_kernel(XT_PARAMS) {
-    XT_HOT;
+__global__ __launch_bounds__(256, 3) void xks_kernel(xt_args a) {
     constexpr bool K4 = WT == SPY_HIP_Q4_K;
     __shared__ __align__(16) float s_t[32][4][64];                  // [sub-block of the round][row 4q + v][lane]
     __shared__ __align__(16) float s_tab[4][K4 ? 256 : 16];
     __shared__ float s_x[32][16], s_d[4][16];                       // d_x of the round's sub-blocks; Q6_K: d of its super-blocks
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, r = lane & 15;
-    const int mat = hot.mat((int)blockIdx.x), m0 = ((int)blockIdx.x - mat * hot.tiles) * 16, cg = (int)blockIdx.y, nsb = hot.nst / 2;
-    const uint8_t *wr = hot.w(mat) + (int64_t)min(m0 + r, a.M - 1) * hot.w_row;
-    const uint8_t *xq = hot.xq + (int64_t)cg * hot.nst * XT_XB + q * 256 + r * 16, *xd = hot.xd + (int64_t)cg * hot.nst * XT_XD;
+    const int mat = (int)blockIdx.x / a.tiles, m0 = ((int)blockIdx.x - mat * a.tiles) * 16, cg = (int)blockIdx.y, nsb = a.nst / 2;
+    const uint8_t *wr = a.w[mat] + (int64_t)min(m0 + r, a.M - 1) * a.w_row;
+    const uint8_t *xq = a.xq + (int64_t)cg * a.nst * XT_XB + q * 256 + r * 16, *xd = a.xd + (int64_t)cg * a.nst * XT_XD;
     xk_raw<WT> cur = xk_load<WT>(wr, min(wave, nsb - 1), q), nxt;
     uint4 xv[8], xn[8];
     uint32_t dx[2], dn[2];
@@ -1430,7 +1431,7 @@ int xk_launch(hipStream_t st, xt_args a, int nmat) {
 template <int WT>
 int xks_launch(hipStream_t st, xt_args a, int nmat) {
     a.tiles = (a.M + 15) / 16;
-    xks_kernel<WT><<<dim3((unsigned)(a.tiles * nmat), (unsigned)a.ncg), dim3(256), 0, st>>>(XT_ARGS(a));
+    xks_kernel<WT><<<dim3((unsigned)(a.tiles * nmat), (unsigned)a.ncg), dim3(256), 0, st>>>(a);
     return SPY_LAUNCH_RC();
 }
 

@@ -19,6 +19,7 @@
 #pragma once
 
 #include "decode_kernels.cuh"
+#include "attn_reach.h"
 #include "exact_exp.cuh"
 #include "exact_sum.cuh"
 
@@ -586,13 +587,15 @@ static __device__ __forceinline__ float xa_tree32(float acc) {
         if (e < ntail) tail = fmaf(h2f((uint16_t)(e & 1 ? wv >> 16 : wv & 0xFFFFu)), h2f((uint16_t)(e & 1 ? wq >> 16 : wq & 0xFFFFu)), tail); \
     }
 #define XA_MAX_CTX 4736                                 // longest cache, most heads of the attention kernels of one token
-#define XA_MAX_HEAD 33
+#define XA_MAX_HEAD 32
 #define XS_THREADS 1024
 #define XS_NU 3                                         // units of a wave in flight (2 and 4: the same)
 // A unit is 16 keys, four adjacent lanes per key: lane `part` has the 16 bytes of accumulators (part, l) of every chunk, straight from memory, and its head's part of q
-// in registers.  The tail goes down the four lanes, eight elements each.  The heads are dealt out over eight groups (heads g, g + 8, ...), a unit has one, two, four or eight
-// of them and tokens to match; workgroup b takes group b modulo 8, so that a head's keys are read and its scores written by one XCD, the one that reads
-// them next where the cache is long (in a pass 4100 tokens 8.58 -> 8.26 us against units of 16 heads of one token, 2060 5.62 -> 5.17, 1000 and 600 the same).  A group's tokens are
+// in registers.  The tail goes down the four lanes, eight elements each.  The heads are dealt out over eight groups (heads g, g + 8, ...), a unit has one, two or four
+// of its group's and tokens to match (attn_reach.h); workgroup b takes group b modulo 8, so that a head's keys are read and its scores written by one XCD, the one that reads
+// them next where the cache is long (in a pass 4100 tokens 8.58 -> 8.26 us against units of 16 heads of one token, 2060 5.62 -> 5.17, 1000 and 600 the same).  A place without a head
+// repeats the group's first and a group without heads has no work (24 heads, with units of the largest group's size and the last head in such places: scores and product of
+// 4100 tokens 16.1 us, now 15.1, 2060 11.9 and 11.3; 17 heads 15.0 and 14.5).  A group's tokens are
 // dealt out evenly over its workgroups, a workgroup's over its waves.
 // What bounds it: the keys at 5.5 TB/s behind launch, position and first wait (4100 tokens: 33.6 MB in 8.05 us).  Through LDS, one thread per key, the dots began when the last
 // key of a round was there and then took 1.6 us: 4100 tokens 9.9, 2060 6.7, 1000 and 600 4.83 us (now 4.75); here a wave's
@@ -602,13 +605,14 @@ template <int DUMMY>
 __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_state *st, int pos_imm, const uint16_t *__restrict__ q16, const uint16_t *kc,
                                                                   float *__restrict__ scores, int n_head, int n_ctx, float scale) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), part = lane & 3;
-    const int hs = n_head > 32 ? 3 : n_head > 16 ? 2 : n_head > 8 ? 1 : 0, nt = 16 >> hs;       // log2 of a unit's heads, its tokens
     const int nb = (int)gridDim.x >> 3, tb = (int)blockIdx.x >> 3, hg = (int)blockIdx.x & 7;
+    if (hg >= n_head) return;
+    const int hs = xs_log2(n_head, hg), nt = 16 >> hs;
     const int n_kv = (st ? st->pos : pos_imm) + 1;
-    const int tpw = ((n_kv + nb - 1) / nb + nt - 1) & -nt, t_end = min(n_kv, (tb + 1) * tpw);
+    const int tpw = xs_share(n_kv, nb, nt), t_end = min(n_kv, (tb + 1) * tpw);
     int t = tb * tpw + wave * nt;
     if (tb >= nb || t >= t_end) return;
-    const int hh = hg + 8 * ((lane >> 2) & ((1 << hs) - 1)), h = min(hh, n_head - 1), dt = lane >> (2 + hs);
+    const int slot = (lane >> 2) & ((1 << hs) - 1), h = xs_head(n_head, hg, slot), dt = lane >> (2 + hs);
     const size_t d = (size_t)n_head * 128;
     const uint16_t *qp = q16 + h * 128 + part * 8, *kp = kc + h * 128 + part * 8;
     uint4 q[4];
@@ -631,7 +635,7 @@ __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_stat
 #pragma unroll
             for (int i = 0; i < 4; i++) kv[i] = make_uint4(k[u][i].x, k[u][i].y, k[u][i].z, k[u][i].w);
             const float dot = xa_dot4(kv, q);
-            if (part == 3 && hh < n_head && tt + dt < t_end) scores[(size_t)h * n_ctx + tt + dt] = dot * scale;
+            if (part == 3 && hg + 8 * slot < n_head && tt + dt < t_end) scores[(size_t)h * n_ctx + tt + dt] = dot * scale;
             request(u, tt + 16 * nt * XS_NU);
         }
     }

@@ -1,6 +1,7 @@
-// What xattn_short_kernel asks of the caches before it knows the position, walked with the functions it uses (attn_reach.h) over every thread, length
-// and context up to the largest the kernel takes.  Prints "ok", or the first request outside the caches (exit status 1).
+// What the attention kernels of one token ask of the caches, walked with the functions they use (attn_reach.h): xattn_short_kernel before it knows the position, over every
+// thread, length and context up to the largest the kernel takes; xattn_scores_kernel over every number of heads.  Prints "ok", or the first request that is not as it should be (exit status 1).
 #include <cstdio>
+#include <vector>
 
 #include "../../spy_amd/csrc/attn_reach.h"
 
@@ -21,6 +22,26 @@ int main() {
                     if (xf_piece(c, keys * 16) != c) { std::printf("n_kv %d of %d: piece %d\n", n_kv, n_ctx, c); return 1; }
                 for (int c = 0; c <= (n_kv - 1) / 8 && c < 64; c++)
                     if (xf_piece(c, pieces) != c) { std::printf("n_kv %d of %d: row piece %d\n", n_kv, n_ctx, c); return 1; }
+            }
+    // every key of every head once, by a workgroup of its head's group; nothing else is read but a key of the group's own
+    for (int n_head = 1; n_head <= 32; n_head++)
+        for (int nb : {1, 2, 13, 32})
+            for (int n_kv : {1, 3, 16, 17, 300, 577, 1900, 4736}) {
+                std::vector<int> seen((size_t)n_head * n_kv);
+                for (int b = 0; b < 8 * nb; b++) {
+                    const int g = b & 7, tb = b >> 3;
+                    if (g >= n_head) continue;
+                    const int nh = (n_head - g + 7) / 8, hs = xs_log2(n_head, g), nt = 16 >> hs;
+                    if (nh > 1 << hs || (hs && nh <= 1 << (hs - 1))) { std::printf("%d heads, group %d: %d heads in units of %d\n", n_head, g, nh, 1 << hs); return 1; }
+                    const int tpw = xs_share(n_kv, nb, nt);
+                    for (int t = tb * tpw; t < n_kv && t < (tb + 1) * tpw; t += nt)
+                        for (int key = 0; key < 16; key++) {
+                            const int slot = key & ((1 << hs) - 1), h = xs_head(n_head, g, slot), tt = t + (key >> hs);
+                            if (h % 8 != g || h >= n_head) { std::printf("%d heads, group %d: reads head %d\n", n_head, g, h); return 1; }
+                            if (slot < nh && tt < n_kv && tt < (tb + 1) * tpw) seen[(size_t)h * n_kv + tt]++;
+                        }
+                }
+                for (int s : seen) if (s != 1) { std::printf("%d heads, %d tokens, %d workgroups a group: a key %d times\n", n_head, n_kv, nb, s); return 1; }
             }
     std::puts("ok");
     return 0;

@@ -291,34 +291,51 @@ def test_attn_decode_short_cache(hip, n_head, n_kv, n_ctx, monkeypatch):
     assert not np.isnan(res[0][1].view(np.float32)).any()
 
 
-@pytest.mark.parametrize("grid,n_kv", [(64, 4351), (7, 300), (100, 1900)])
-def test_attn_scores_in_several_rounds(hip, grid, n_kv, monkeypatch):
-    """The score kernel of order 1 deals the cached tokens out over its workgroups and waves, three tokens of a wave in flight.  With one workgroup per
-    compute unit of this part a wave has no more than three at the supported cache lengths; SPY_HIP_SCORES_GRID forces fewer workgroups, so that later
-    requests (full rounds, a short last one, workgroups without tokens) are exercised: same bits as the one-round launch."""
+def _scores_geometry(grid, n_head, n_kv):
+    """(units of the busiest wave, workgroups of a head group without tokens) of xattn_scores_kernel, of the group with the fewest tokens per unit: units of 16 keys, 16 waves"""
+    nb, heads = max(grid // 8, 1), (n_head + 7) // 8
+    nt = 16 if heads == 1 else 8 if heads == 2 else 4
+    tpw = (-(-n_kv // nb) + nt - 1) // nt * nt
+    return -(-min(tpw, n_kv) // (16 * nt)), nb - -(-n_kv // tpw)
+
+
+@pytest.mark.parametrize("grid,n_head,n_kv,units,empty", [(64, 32, 4351, 9, 0), (7, 32, 300, 5, 0), (100, 32, 1900, 3, 0), (16, 32, 1900, 15, 0), (8, 12, 1201, 10, 0), (8, 5, 1030, 5, 0), (256, 32, 577, 1, 3),
+                                                          (256, 17, 4736, 3, 0), (64, 24, 4097, 9, 0), (96, 32, 2306, 4, 0), (256, 8, 577, 1, 13)])
+def test_attn_scores_in_several_rounds(hip, oracle, grid, n_head, n_kv, units, empty, monkeypatch):
+    """The score kernel of order 1 deals the cached tokens of a head group out over its workgroups and waves, three units of 16 keys of a wave in flight.  With one workgroup per
+    compute unit of this part a wave has no more than three at the supported cache lengths; SPY_HIP_SCORES_GRID (rounded down to a multiple of eight, eight at least) forces fewer
+    workgroups, so that later requests are exercised: full rounds, a short last one, also units and workgroups with fewer tokens than the others and workgroups without tokens."""
     from tests.gpu_util import dev, dev_empty, call
-    H_, hd, n_ctx = 32, 128, 4352
-    d = H_ * hd
+    assert _scores_geometry(grid, n_head, n_kv) == (units, empty)
+    hd, n_ctx = 128, (n_kv + 63) // 64 * 64
+    d = n_head * hd
     rng = np.random.default_rng(grid * 10000 + n_kv)
     q16 = (rng.standard_normal(d) * 1.5).astype(np.float16)
-    kc = np.zeros((n_ctx, d), np.float16); kc[:n_kv] = rng.standard_normal((n_kv, d)).astype(np.float16)
-    vc = np.zeros((d, n_ctx), np.float16); vc[:, :n_kv] = rng.standard_normal((d, n_kv)).astype(np.float16)
+    kc, vc = np.full((n_ctx, d), np.nan, np.float16), np.full((d, n_ctx), np.nan, np.float16)
+    kc[:n_kv] = rng.standard_normal((n_kv, d)); vc[:, :n_kv] = rng.standard_normal((d, n_kv))
+    S = np.zeros((n_head, 1, n_kv), np.float32)
+    assert oracle.spy_o_matmul(B(O.tensor(kc.view(np.uint16), O.F16, [hd, n_kv, n_head], nb=[2, 2 * d, 2 * hd])),
+                               B(O.tensor(q16.astype(np.float32), O.F32, [hd, 1, n_head], nb=[4, 4 * d, 4 * hd])), B(O.tensor(S, O.F32, [n_kv, 1, n_head])), 8) == 0
+    want = (S[:, 0, :] * (np.float32(1.0) / np.sqrt(np.float32(hd)))).astype(np.float32)
     dq, dk, dv = dev(q16.view(np.uint16)), dev(kc.view(np.uint16)), dev(vc.view(np.uint16))
-    res = []
+    outs = []
     for g in (None, grid):
         if g is None:
             monkeypatch.delenv("SPY_HIP_SCORES_GRID", raising=False)
         else:
             monkeypatch.setenv("SPY_HIP_SCORES_GRID", str(g))
-        ds, do = dev_empty(H_ * n_ctx * 4, 0xEE), dev_empty(d * 4, 0xEE)
-        call(hip.load().spy_hip_attn_decode, None, 1, dq.ptr, dk.ptr, dv.ptr, H_, n_kv, n_ctx, ds.ptr, do.ptr)
+        ds, do = dev_empty((n_head * n_ctx + 64) * 4, 0xEE), dev_empty(d * 4, 0xEE)
+        call(hip.load().spy_hip_attn_decode, None, 1, dq.ptr, dk.ptr, dv.ptr, n_head, n_kv, n_ctx, ds.ptr, do.ptr)
         hip.sync()
-        res.append((ds.download(np.uint32).reshape(H_, n_ctx)[:, :n_kv].copy(), do.download(np.uint32).copy()))
-    assert np.array_equal(res[0][0], res[1][0]), "scores differ between one round and %d workgroups" % grid
-    assert np.array_equal(res[0][1], res[1][1])
+        got = ds.download(np.uint32)
+        rows = got[:n_head * n_ctx].reshape(n_head, n_ctx)
+        assert np.array_equal(rows[:, :n_kv], want.view(np.uint32)), "scores, %s workgroups" % g
+        assert (rows[:, n_kv:] == 0xEEEEEEEE).all() and (got[n_head * n_ctx:] == 0xEEEEEEEE).all()
+        outs.append(do.download(np.uint32).copy())
+    assert np.array_equal(outs[0], outs[1])
 
 
-@pytest.mark.parametrize("n_head,n_kv", [(1, 577), (8, 581), (9, 594), (16, 593), (17, 1033), (31, 700)])
+@pytest.mark.parametrize("n_head,n_kv", [(1, 577), (5, 601), (8, 581), (9, 594), (16, 593), (17, 1033), (20, 700), (24, 1001), (31, 700)])
 def test_attn_decode_head_groups(hip, oracle, n_head, n_kv):
     """Scores are formed for eight groups of heads, one, two or four heads of as many tokens at a time: full groups, groups that lack a head, groups without one."""
     from tests.gpu_util import dev, dev_empty, call

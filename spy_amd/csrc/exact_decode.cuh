@@ -405,6 +405,7 @@ __global__ __launch_bounds__(XG_THREADS) void xgemv_kernel(const float *x_in, co
     constexpr int NSTEPS = EPI == EPI_QKV ? (ONE ? 1 : 2) : NSTEP;
     constexpr bool SLABS = xg_slabs(NCH, NITK);
     static_assert(NITK == 1 || NROW == 1, "rows longer than one slab are walked one row per wave");
+    static_assert(WT == WTV || (NCH == 1 && NCHV == 1), "n8 and the factor 16 of Q4_0's high nibbles follow WT in every step");
     act_frag<1> af, av;
     int n8[16];
     // gate|up: the SiLU table's answers are awaited after the last step only (Q4_0 15.38 -> 15.08 us, Q4_K 14.26 -> 13.86; Q8_0 has no registers left for it: 21.3 -> 21.5)

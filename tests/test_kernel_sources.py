@@ -91,3 +91,22 @@ def test_shapes_of_the_packed_activation_tests_reach_every_tile(tmp_path):
         assert {t for t, _ in split} == {0, 6, 7, 8}
     own = [s[1:] for s in G.OWN_SHAPES if s[0] == O.Q4_0]
     assert set(tiles("q", 0, own)) == {0} and set(tiles("q", 0, G.TILES_OF_32_SHAPES)) == {1}
+
+
+def test_single_token_qkv_pairs_q4_0_and_q8_0_with_themselves_only(tmp_path):
+    """The kernel undoes the factor 16 of Q4_0's high nibbles, and sums the activations that fold its -8, by the type of wq and wk: with another type of wv beside it, it does not compile."""
+    import shutil
+    from concurrent.futures import ThreadPoolExecutor
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+    def compiles(pair):
+        src = tmp_path / ("%d_%d.hip" % pair)
+        src.write_text('#include "%s/spy_amd/csrc/exact_decode.cuh"\nauto kernel = xgemv_kernel<%d, 1, 2, 1, EPI_QKV, %d>;\n' % (ROOT, pair[0], pair[1]))
+        r = subprocess.run([hipcc, "--offload-arch=gfx950", "-std=c++20", "--cuda-device-only", "-fsyntax-only", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", str(src)],
+                           capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0 or "follow WT in every step" in r.stderr, r.stderr
+        return r.returncode == 0
+
+    from spy_amd._lib import Q4_0, Q4_K, Q6_K, Q8_0
+    with ThreadPoolExecutor(4) as pool:
+        assert list(pool.map(compiles, [(Q4_0, Q4_0), (Q4_K, Q6_K), (Q8_0, Q4_0), (Q4_0, Q8_0), (Q4_0, Q6_K)])) == [True, True, False, False, False]

@@ -678,8 +678,13 @@ static inline size_t xattn_pv_lds(int n_ctx) {
     const int end = 17 * xattn_pv_row(n_ctx) * 2, soft = xattn_pv_soft_at(n_ctx) + xattn_pv_soft(n_ctx);
     return end > soft ? end : soft;
 }
-// arrival and wait of waves of one workgroup on a counter in LDS (all of them resident, and none waits before it has arrived)
-static __device__ __forceinline__ void xp_arrive(uint32_t *c) { if ((threadIdx.x & 63) == 0) __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP); }
+// Arrival and wait of waves of one workgroup on a counter in LDS (all of them resident, and none waits before it has arrived).  Every lane's stores lie before the count, so every lane
+// has the release; the count itself, by one of them, needs none of its own.
+static __device__ __forceinline__ void xp_arrive(uint32_t *c) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    if ((threadIdx.x & 63) == 0) __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 static __device__ __forceinline__ void xp_await(uint32_t *c, uint32_t n) { while (__hip_atomic_load(c, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < n) __builtin_amdgcn_s_sleep(1); }
 template <int DUMMY>
 __global__ __launch_bounds__(XP_THREADS) void xattn_pv_kernel(const dev_state *st, int pos_imm, const float *__restrict__ scores, const uint16_t *vc,

@@ -110,3 +110,14 @@ def test_single_token_qkv_pairs_q4_0_and_q8_0_with_themselves_only(tmp_path):
     from spy_amd._lib import Q4_0, Q4_K, Q6_K, Q8_0
     with ThreadPoolExecutor(4) as pool:
         assert list(pool.map(compiles, [(Q4_0, Q4_0), (Q4_K, Q6_K), (Q8_0, Q4_0), (Q4_0, Q8_0), (Q4_0, Q6_K)])) == [True, True, False, False, False]
+
+
+def test_a_wave_releases_what_all_its_lanes_wrote_before_it_is_counted():
+    """Waves of the single-token softmax meet on counters in LDS: one lane counts its wave, but what the others wait for was written by all 64, so the release is
+    theirs too and stands ahead of the branch."""
+    kernel = open(os.path.join(ROOT, "spy_amd", "csrc", "exact_decode.cuh")).read()
+    body = re.search(r"void xp_arrive\(uint32_t \*c\) \{(.*?)\n\}", kernel, re.S).group(1)
+    fence, barrier, branch, count = (body.index(x) for x in ('__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup")', "__builtin_amdgcn_wave_barrier()", "if (", "__hip_atomic_fetch_add(c"))
+    assert fence < barrier < branch < count
+    await_ = re.search(r"void xp_await\(.*?\n", kernel).group(0)
+    assert "__ATOMIC_ACQUIRE" in await_ and "if (" not in await_

@@ -12,9 +12,9 @@ constexpr int xf_row_pieces_before(bool in_state, int pos_imm, int n_ctx) { retu
 // piece c of `pieces` there are: the last one where c is none of them
 constexpr int xf_piece(int c, int pieces) { return c < pieces ? c : pieces - 1; }
 
-// Which keys xattn_scores_kernel (exact_decode.cuh) reads.  Head group g of eight has heads g, g + 8, ...; a unit of a wave is 16 keys: one, two or four heads (as many as hold the
-// group's, four at most with 32 heads) of 16, 8 or 4 tokens.
-constexpr int xs_log2(int n_head, int g) { return (n_head - g - 1) >> 3 < 2 ? (n_head - g - 1) >> 3 : 2; }         // log2 of the heads of a unit; g < n_head
+// Which keys xattn_scores_kernel (exact_decode.cuh) reads.  Head group g of eight has heads g, g + 8, ...; a unit of a wave is 16 keys: one, two or four heads (as many as the largest
+// group has, four at most with 32 heads) of 16, 8 or 4 tokens.
+constexpr int xs_log2(int n_head) { return n_head > 16 ? 2 : n_head > 8 ? 1 : 0; }                                // log2 of the heads of a unit
 constexpr int xs_head(int n_head, int g, int slot) { return g + 8 * slot < n_head ? g + 8 * slot : g; }           // head of place `slot` in a unit: the group's first where it has none
 // tokens of a workgroup where nb share n_kv, a multiple of the nt of a unit
 constexpr int xs_share(int n_kv, int nb, int nt) { return ((n_kv + nb - 1) / nb + nt - 1) & -nt; }

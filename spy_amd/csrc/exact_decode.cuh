@@ -595,8 +595,8 @@ static __device__ __forceinline__ float xa_tree32(float acc) {
 // in registers.  The tail goes down the four lanes, eight elements each.  The heads are dealt out over eight groups (heads g, g + 8, ...), a unit has one, two or four
 // of its group's and tokens to match (attn_reach.h); workgroup b takes group b modulo 8, so that a head's keys are read and its scores written by one XCD, the one that reads
 // them next where the cache is long (in a pass 4100 tokens 8.58 -> 8.26 us against units of 16 heads of one token, 2060 5.62 -> 5.17, 1000 and 600 the same).  A place without a head
-// repeats the group's first and a group without heads has no work (24 heads, with units of the largest group's size and the last head in such places: scores and product of
-// 4100 tokens 16.1 us, now 15.1, 2060 11.9 and 11.3; 17 heads 15.0 and 14.5).  A group's tokens are
+// repeats the group's first and a group without heads has no work (with the last head in such places: 24 heads, scores and product of 4100 tokens 16.1 us, now 15.1, 2060 11.9 and
+// 11.3).  A group's tokens are
 // dealt out evenly over its workgroups, a workgroup's over its waves.
 // What bounds it: the keys at 5.5 TB/s behind launch, position and first wait (4100 tokens: 33.6 MB in 8.05 us).  Through LDS, one thread per key, the dots began when the last
 // key of a round was there and then took 1.6 us: 4100 tokens 9.9, 2060 6.7, 1000 and 600 4.83 us (now 4.75); here a wave's
@@ -608,7 +608,7 @@ __global__ __launch_bounds__(XS_THREADS) void xattn_scores_kernel(const dev_stat
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), part = lane & 3;
     const int nb = (int)gridDim.x >> 3, tb = (int)blockIdx.x >> 3, hg = (int)blockIdx.x & 7;
     if (hg >= n_head) return;
-    const int hs = xs_log2(n_head, hg), nt = 16 >> hs;
+    const int hs = xs_log2(n_head), nt = 16 >> hs;
     const int n_kv = (st ? st->pos : pos_imm) + 1;
     const int tpw = xs_share(n_kv, nb, nt), t_end = min(n_kv, (tb + 1) * tpw);
     int t = tb * tpw + wave * nt;

@@ -31,8 +31,8 @@ int main() {
                 for (int b = 0; b < 8 * nb; b++) {
                     const int g = b & 7, tb = b >> 3;
                     if (g >= n_head) continue;
-                    const int nh = (n_head - g + 7) / 8, hs = xs_log2(n_head, g), nt = 16 >> hs;
-                    if (nh > 1 << hs || (hs && nh <= 1 << (hs - 1))) { std::printf("%d heads, group %d: %d heads in units of %d\n", n_head, g, nh, 1 << hs); return 1; }
+                    const int nh = (n_head - g + 7) / 8, hs = xs_log2(n_head), nt = 16 >> hs;
+                    if (nh > 1 << hs) { std::printf("%d heads, group %d: %d heads in units of %d\n", n_head, g, nh, 1 << hs); return 1; }
                     const int tpw = xs_share(n_kv, nb, nt);
                     for (int t = tb * tpw; t < n_kv && t < (tb + 1) * tpw; t += nt)
                         for (int key = 0; key < 16; key++) {

@@ -37,7 +37,7 @@ def test_single_token_attention_reads_no_keys_behind_the_last_one(tmp_path):
     # ... and the score kernel: each head's keys by its own group, no work for a group without heads
     kernel = open(os.path.join(ROOT, "spy_amd", "csrc", "exact_decode.cuh")).read()
     kernel = kernel[kernel.index("void xattn_scores_kernel("):kernel.index("// ---- softmax + P.V^T in the host order")]
-    assert [kernel.count(f) for f in ("xs_log2(n_head, hg)", "xs_share(n_kv, nb, nt)", "xs_head(n_head, hg, slot)", "if (hg >= n_head) return;", "hg + 8 * slot < n_head")] == [1] * 5
+    assert [kernel.count(f) for f in ("xs_log2(n_head)", "xs_share(n_kv, nb, nt)", "xs_head(n_head, hg, slot)", "if (hg >= n_head) return;", "hg + 8 * slot < n_head")] == [1] * 5
 
 
 def test_launches_of_a_single_token_pass_read_no_environment():

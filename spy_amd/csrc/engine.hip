@@ -589,7 +589,7 @@ static int forward_ops(spy_hip_llama *m, hipStream_t st, const int32_t *tokens_h
             RC_TRY(mm(L.wv, L.t_wv, d, d, &t_xn, &t_v));
         }
         spy_hip_tensor t_qp;
-        if (fuse_act) {           // Rope(q), Rope(k), the fp16 conversion of q and both cache writes in two kernels (prompt_fused.hip)
+        if (fuse_act) {           // Rope(q), Rope(k), the fp16 conversion of q and both cache writes in one launch (prompt_fused.hip)
             RC_TRY(spy_qkv_store_launch(st, q, k, v, rope_tab, (uint16_t *)xn, (uint16_t *)m->k_cache[il] + d * P, (uint16_t *)m->v_cache[il] + P, T, (int)H, (int)hd, C));
             t_qp = T3s(SPY_HIP_F16, xn, hd, T, H, 2, 2 * hd, 2 * hd * T);
         } else {

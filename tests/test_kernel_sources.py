@@ -121,3 +121,12 @@ def test_a_wave_releases_what_all_its_lanes_wrote_before_it_is_counted():
     assert fence < barrier < branch < count
     await_ = re.search(r"void xp_await\(.*?\n", kernel).group(0)
     assert "__ATOMIC_ACQUIRE" in await_ and "if (" not in await_
+
+
+def test_objects_are_remade_when_the_flags_change():
+    """Flags lie in the Makefile, so every object depends on it, and on every header there is."""
+    csrc = os.path.join(ROOT, "spy_amd", "csrc")
+    sources = {os.path.basename(p) for p in glob.glob(os.path.join(csrc, "*.hip"))}
+    for changed in ["Makefile"] + [os.path.basename(p) for p in glob.glob(os.path.join(csrc, "*.cuh")) + glob.glob(os.path.join(csrc, "*.h"))]:
+        r = subprocess.run(["make", "-C", csrc, "-n", "-W", changed], capture_output=True, text=True, check=True, timeout=60)
+        assert set(re.findall(r" -c (\S+\.hip) ", r.stdout)) == sources, changed

@@ -238,6 +238,10 @@ int spy_hip_block_dots(void *stream, int wtype, const void *w, const void *xq, i
  * -> *out, bit for bit; chunked = 0: one chain of additions, 1: the chunked form the gate|up kernel of order 1 uses
  * (integer increments per 64-term chunk inside a binade, the chain only where the sum crosses a power of two). */
 int spy_hip_running_sum_f32(void *stream, const float *terms, int64_t n, int32_t chunked, float *out);
+/* The exponential that Softmax of the host backend takes (lookup_table_impl/non-linear.h:39-47: expf of the host's libm by the bits of an fp16
+ * value) for n fp16 values not above 0, or NaN: a score minus its row's maximum.  worked_out = 0: from the device's copy of the
+ * table; 1: worked out and put right to the same bits by a list, as the attention kernels of order 1 do. */
+int spy_hip_exp_f16(void *stream, const void *x, int64_t n, int32_t worked_out, float *out);
 /* RMSNorm * weight -> Q8_0: OperatorNormRMSImpl::execute + the Mul node + Quantizator<FP32,Q8_0>::transform
  * (non-linear.cpp:194-223, basic.cpp:15-50, vec_convert.h:178-261) as the fused kernels stage their activations;
  * normw == NULL: the quantization alone.  yq: K/32 native Q8_0 blocks. */

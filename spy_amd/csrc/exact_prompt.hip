@@ -443,3 +443,25 @@ extern "C" int spy_hip_prompt_attention_exact(void *stream, const float *q, cons
     uint16_t *P16 = (uint16_t *)((uint8_t *)scratch + need / 6 * 4);
     return spy_exact_prompt_attn((hipStream_t)stream, q, false, (const uint16_t *)k_cache, (const uint16_t *)v_cache, S, P16, out, lut, T, H, past, n_ctx, n_total, scale);
 }
+
+// xe_exp argument by argument (exact_exp.cuh), the list in LDS as the attention kernels have it
+__global__ __launch_bounds__(256) void exp_f16_kernel(const uint16_t *__restrict__ x, int64_t n, int worked_out, const float *__restrict__ lut, float *__restrict__ out) {
+    __shared__ __align__(16) uint32_t s_code[XE_WORDS];
+    for (int i = threadIdx.x; i < XE_WORDS / 4; i += 256) ((uint4 *)s_code)[i] = ((const uint4 *)(lut + XE_AT))[i];
+    __syncthreads();
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        bool ask = true;
+        float e = 0.0f;
+        if (worked_out) e = xe_exp((uint32_t)x[i] ^ 0x8000u, s_code, ask);
+        out[i] = ask ? lut[x[i]] : e;
+    }
+}
+extern "C" int spy_hip_exp_f16(void *stream, const void *x, int64_t n, int32_t worked_out, float *out) {
+    SPY_CHECK_ARG(x && out && n > 0 && (worked_out == 0 || worked_out == 1) && ((uintptr_t)x % 2) == 0 && ((uintptr_t)out % 4) == 0);
+    const float *lut = nullptr;
+    const int rc = spy_exact_luts(&lut);
+    if (rc) return rc;
+    const int64_t need = (n + 255) / 256;
+    exp_f16_kernel<<<dim3((unsigned)(need < 1024 ? need : 1024)), dim3(256), 0, (hipStream_t)stream>>>((const uint16_t *)x, n, worked_out, lut, out);
+    return SPY_LAUNCH_RC();
+}

@@ -917,3 +917,85 @@ def test_prompt_attention_leaves_packed_activations(hip, H_, past, T):
     a, b = p0.download(np.uint32), p1.download(np.uint32)
     assert np.array_equal(a, b)
     assert (b[-16:] == 0xEEEEEEEE).all()
+
+
+def test_exponentials_worked_out_for_every_argument(hip):
+    """Attention works its exponentials out and puts them right to the host's by a list: every fp16 value not above 0, and every NaN, against the table, and the table against the
+    host's expf."""
+    from tests.gpu_util import dev, dev_empty, call
+    x = np.concatenate([np.arange(0x8000, 0x10000), np.arange(0x7C01, 0x8000), [0]]).astype(np.uint16)
+    dx, res = dev(x), []
+    for worked_out in (0, 1):
+        do = dev_empty(x.size * 4 + 64, 0xEE)
+        call(hip.load().spy_hip_exp_f16, None, dx.ptr, x.size, worked_out, do.ptr)
+        got = do.download(np.uint32)
+        assert (got[x.size:] == 0xEEEEEEEE).all()
+        res.append(got[:x.size])
+    assert np.array_equal(res[0], res[1])
+    expf = C.CDLL("libm.so.6").expf
+    expf.restype, expf.argtypes = C.c_float, [C.c_float]
+    f = x.view(np.float16).astype(np.float32)
+    number = ~np.isnan(f)
+    want = np.array([expf(v) for v in f[number]], np.float32)
+    assert np.array_equal(res[0][number], want.view(np.uint32))
+    assert np.isnan(res[0][~number & (x != 0xFFFF)].view(np.float32)).all()                  # 0xFFFF: the host's table has 0 there (its loop ends before)
+
+
+@pytest.mark.parametrize("share", [1.0, 0.02])
+def test_exponentials_that_only_the_table_can_tell(hip, share):
+    """A correction of more than one ulp does not fit the list: such an argument has code 3 and asks the table.  This libm has none, so the code is set for all arguments, or for one
+    in fifty: attention of short and of long caches and of prompts gives the same bits."""
+    from tests.gpu_util import dev, dev_empty, call
+    H_, hd = 4, 128
+    d = H_ * hd
+    rng = np.random.default_rng(7)
+    L = hip.load()
+    lut = C.c_void_p()
+    assert getattr(L, "_Z14spy_exact_lutsPPKf")(C.byref(lut)) == 0
+    at, words = lut.value + 2 * 65536 * 4, 1388                                               # XE_AT, XE_WORDS
+    x = np.arange(0x8000, 0x8000 + words * 16).astype(np.uint16)
+
+    def run():
+        out = []
+        dx, do = dev(x), dev_empty(x.size * 4, 0xEE)
+        call(L.spy_hip_exp_f16, None, dx.ptr, x.size, 1, do.ptr)
+        out.append(do.download(np.uint32))
+        r = np.random.default_rng(11)
+        for n_kv in (300, 1000, 4700):
+            n_ctx = (n_kv + 63) // 64 * 64
+            q, kc, vc = (r.standard_normal(d) * 12).astype(np.float16), r.standard_normal((n_ctx, d)).astype(np.float16), r.standard_normal((d, n_ctx)).astype(np.float16)
+            dq, dk, dv = dev(q.view(np.uint16)), dev(kc.view(np.uint16)), dev(vc.view(np.uint16))
+            ds, do = dev_empty(H_ * n_ctx * 4, 0xEE), dev_empty(d * 4, 0xEE)
+            call(L.spy_hip_attn_decode, None, 1, dq.ptr, dk.ptr, dv.ptr, H_, n_kv, n_ctx, ds.ptr, do.ptr)
+            out.append(do.download(np.uint32))
+        for past, T in ((0, 130), (2100, 20)):
+            n_ctx = (past + T + 31) // 32 * 32
+            q, kc, vc = (r.standard_normal((T, d)) * 12).astype(np.float32), r.standard_normal((n_ctx, d)).astype(np.float16), r.standard_normal((d, n_ctx)).astype(np.float16)
+            dq, dk, dv = dev(q), dev(kc.view(np.uint16)), dev(vc.view(np.uint16))
+            need = L.spy_hip_prompt_attention_exact_scratch_size(T, H_, past)
+            sc, do = dev_empty(need, 0xEE), dev_empty(T * d * 4, 0xEE)
+            call(L.spy_hip_prompt_attention_exact, None, dq.ptr, dk.ptr, dv.ptr, do.ptr, T, H_, hd, past, n_ctx, past + T, C.c_float(1.0 / np.sqrt(np.float32(hd))), sc.ptr, need)
+            out.append(do.download(np.uint32))
+        hip.sync()
+        return out
+
+    def put(codes):
+        hip.check(L.spy_hip_upload(at, codes.ctypes.data, codes.nbytes, None))
+        hip.sync()
+
+    codes = np.empty(words, np.uint32)
+    hip.check(L.spy_hip_download(codes.ctypes.data, at, codes.nbytes, None))
+    want = run()
+    assert all(np.isfinite(w.view(np.float32)).all() for w in want)
+    three = np.zeros(words, np.uint32)
+    for i in range(16):
+        three |= np.where(rng.random(words) < share, np.uint32(3 << (2 * i)), np.uint32(0)).astype(np.uint32)
+    assert ((codes | three) != codes).any()
+    try:
+        put(codes | three)
+        got = run()
+    finally:
+        put(codes)
+    for g, w in zip(got, want):
+        assert np.array_equal(g, w)
+    assert all(np.array_equal(g, w) for g, w in zip(run(), want))

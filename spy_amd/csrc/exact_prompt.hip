@@ -56,8 +56,8 @@ __device__ __forceinline__ void xp_reduce8(const xp_v16f &s, float (&t)[4]) {
 // 64 key rows is brought into LDS by the whole workgroup.  Per 16 key rows and l = 0 .. 7 one chain of three matrix instructions (chunks of 32
 // elements while i + 32 < 128) gives accumulators l, 8 + l, 16 + l, 24 + l of the 16 x 16 scores; the vector units add them in the host's tree.  The
 // last 32 elements, added one by one, are a chain of eight v_mfma_f32_16x16x4_f32, which do the fmas of their four elements one after the other, bit for bit: a lane's
-// eight elements of q stay in registers.  (As 32 of the former, whose four blocks were the four groups of 16 keys, they were widened for every tile, at 168 registers and three
-// workgroups on a compute unit: 2048 rows on 2048 positions, 32 heads, 645 us; three workgroups 601, four 588; 2048 rows alone 238 -> 218.)  What bounds
+// eight elements of q stay in registers.  (As 32 of the former, whose four blocks were the four groups of 16 keys, they were widened for every tile; 125 registers then, 113 now, four workgroups on a
+// compute unit either way.  Both in one run, 32 heads: 2048 rows on 2048 positions 670 -> 632 us, 2048 rows 231 -> 220, 77 rows on 1000 positions 20.7 -> 19.4.)  What bounds
 // it: matrix and vector instructions of this kind never run at once (counter SQ_VALU_MFMA_COEXEC_CYCLES: 0), so the 31 additions of the tree and the
 // widening of the keys come on top of the fmas (348 us).  A last tile of few rows with its keys dealt out over the waves: nothing (77 rows on 1000 16.4 us).
 #define XP_KSEG 512
@@ -166,6 +166,8 @@ __global__ __launch_bounds__(256, 4) void xp_scores_kernel(const void *__restric
 // LIST: few rows, where bringing 88 KB of table to every compute unit is most of the time: the exponentials are worked out (exact_exp.cuh), which is 5.5 KB and about twice the vector
 // instructions (32 heads, table -> list: 8 rows 7.2 -> 5.0 us, 33 6.9 -> 5.0, 200 on 100 positions 11.9 -> 9.7, 512 22.6 -> 20.5, 1000 45.3 -> 46.1, 2048 118 -> 123; rows of up to 4096 positions:
 // 2048 301 -> 303).
+// (Five and three waves per SIMD of four-wave workgroups leave the list's form 2 and 5 registers short, 12 and 24 bytes of scratch a lane; the table's form of rows of up to 4096
+// positions is as short.)
 #define XP_LUT XE_MAX
 #define XP_LIST_ROWS 24576
 #define XP_SM_R 32         // groups per lane: rows of up to 8192 positions
@@ -270,6 +272,7 @@ typedef uint32_t xp_u4 __attribute__((ext_vector_type(4), aligned(2)));         
 // PACK: the outputs leave as the packed activations of the MatMul that follows (xt_pack.cuh) instead of as floats: the 32 outputs of a row that a workgroup forms
 // are one Q8_0 block.  A launch less, and the outputs do not go through memory: 8 rows 3.5 + 2.6 -> 4.4 us, 33 4.7 + 4.7 -> 5.1,
 // 77 on 1000 positions 16.6 + 4.9 -> 17.5, 512 19.2 + 5.4 -> 21.6, 2048 215 + 10.2 -> 224.
+// (With packing three registers do not fit, 16 bytes of scratch a lane, written before the loop and read behind it: in those times.)
 template <bool PACK>
 __global__ __launch_bounds__(256, 3) void xp_pv_kernel(const uint16_t *__restrict__ P16, const uint16_t *__restrict__ vt, float *__restrict__ out,
                                                        int T, int H, int P, int64_t p_row, int64_t C, int n_total, uint8_t *__restrict__ pack) {
